@@ -105,7 +105,8 @@ struct LayerPlan {
 }  // namespace
 
 struct ksh_gemma4 {
-    std::vector<float> host_logits;   // decode_token_sampled's read-back
+    std::vector<float> host_logits;   // a whole row read back, where the device cannot narrow it down (no min-p filter)
+    ksh::SampleScratch sample;
     ksh_ctx *ctx = nullptr;
     ksh_gemma4_cfg c{};
     ksh_gemma4_globals g{};
@@ -153,6 +154,54 @@ struct ksh_gemma4 {
 namespace {
 
 using namespace ksh;
+
+// The ids of `rows` rows of logits that the stream is about to hold: greedy ids where temperature (may be null) is below
+// 1e-6, else sample_softcap_min_p's draw, on the entries that can survive its filter (launch_sample_candidates).  Waits
+// for the stream.
+int draw_ids(ksh_gemma4 *m, ksh_buf *logits, ksh_buf *best_ids, int rows, const float *temperature, const float *min_p, const uint32_t *seed,
+             uint32_t *next_ids)
+{
+    const int n = m->c.vocab;
+    SampleRow params[kSampleMaxRows] = {};
+    bool any = false, narrowed[kSampleMaxRows] = {};
+    for (int i = 0; i < rows; i++) {
+        if (!temperature || temperature[i] < 1e-6f) continue;
+        any = true;
+        narrowed[i] = sample_row_params(temperature[i], min_p[i], &params[i]);
+    }
+    if (!any) {
+        float ids[kSampleMaxRows];
+        if (ksh_buffer_read(m->ctx, best_ids, 0, ids, (size_t)rows * 4, 1)) return 1;
+        for (int i = 0; i < rows; i++) next_ids[i] = (uint32_t)ids[i];
+        return 0;
+    }
+    const float *dev = (const float *)ksh_buffer_device_ptr(logits);
+    if (launch_sample_candidates(m->sample, dev, n, rows, m->c.softcap, (const float *)ksh_buffer_device_ptr(best_ids), params,
+                                 (hipStream_t)ksh_stream(m->ctx)) ||
+        ksh_synchronize(m->ctx))
+        return 1;
+    std::vector<SampleCand> longer;
+    for (int i = 0; i < rows; i++) {
+        SampleHead &h = m->sample.heads[i];
+        next_ids[i] = h.best_id;
+        if (!temperature || temperature[i] < 1e-6f) continue;
+        if (narrowed[i]) {
+            SampleCand *cand = h.cand;
+            if (h.count > (uint32_t)kSampleInline) {
+                longer.resize(h.count);
+                KSH_HIP(hipMemcpy(longer.data(), (const SampleCand *)m->sample.joined + (size_t)i * n, (size_t)h.count * sizeof(SampleCand), hipMemcpyDeviceToHost));
+                cand = longer.data();
+            }
+            if (sample_from_candidates(cand, h.count, h.sum, (size_t)n, m->c.softcap, temperature[i], min_p[i], seed[i], &next_ids[i])) continue;
+        }
+        std::vector<float> &row = m->host_logits;   // (kept: a megabyte at the real vocabulary)
+        row.resize((size_t)n);
+        if (ksh_buffer_read(m->ctx, logits, (size_t)i * n * 4, row.data(), row.size() * 4, 0) ||
+            ksh_sample_softcap_min_p(row.data(), row.size(), m->c.softcap, temperature[i], min_p[i], seed[i], &next_ids[i]))
+            return 1;
+    }
+    return 0;
+}
 
 constexpr int kAttendPartitions = 16;
 constexpr int kShortPartitions = 8;     // sliding-window layers: the o-projection merges the partitions
@@ -962,17 +1011,15 @@ int ksh_gemma4_generate_until(ksh_gemma4 *m, const uint32_t *prompt, int n_promp
 }
 
 // GemmaPrimModel::decode_token_sampled (gemma_prim.rs:1614-1635): one token with logits; below a temperature of 1e-6
-// the device argmax decides, else the logits are read back and the host sampler draws (gemma_prim.rs:1239-1261).
+// the device argmax decides, else the host sampler draws (gemma_prim.rs:1239-1261) from what the device has narrowed the
+// logits down to.
 int ksh_gemma4_decode_token_sampled(ksh_gemma4 *m, uint32_t token, float temperature, float min_p, uint32_t seed, int use_graph,
                                     uint32_t *next_id)
 {
     if (!m || !next_id) return set_error("ksh_gemma4_decode_token_sampled: bad arguments");
     if (temperature < 1e-6f) return ksh_gemma4_forward_token(m, token, 1, use_graph, next_id);
     if (ksh_gemma4_forward_token(m, token, 1, use_graph, nullptr)) return 1;
-    std::vector<float> &logits = m->host_logits;   // (kept: a megabyte at the real vocabulary, every token)
-    logits.resize((size_t)m->c.vocab);
-    if (ksh_buffer_read(m->ctx, m->logits, 0, logits.data(), logits.size() * 4, 1)) return 1;
-    return ksh_sample_softcap_min_p(logits.data(), logits.size(), m->c.softcap, temperature, min_p, seed, next_id);
+    return draw_ids(m, m->logits, m->tok, 1, &temperature, &min_p, &seed, next_id);
 }
 
 // GemmaPrimModel::prefill_chunk (gemma_prim.rs:1305-1315): the tokens go through without logits, then one
@@ -1321,19 +1368,7 @@ int ksh_gemma4_decode_round(ksh_gemma4 *m, ksh_kvpool *pool, const int32_t *slot
         if (tokens[i] >= (uint32_t)m->c.vocab) return set_error("token id %u is outside the vocabulary", tokens[i]);
     }
     if (forward_decode_round4(m, pool, slots, tokens, n)) return 1;
-    float ids[kRoundMax];
-    if (ksh_buffer_read(m->ctx, m->r_next, 0, ids, (size_t)n * 4, 1)) return 1;
-    for (int i = 0; i < n; i++) {
-        next_ids[i] = (uint32_t)ids[i];
-        if (temperature && temperature[i] >= 1e-6f) {   // decode_token_sampled's other branch (gemma_prim.rs:1614-1635)
-            std::vector<float> &logits = m->host_logits;
-            logits.resize((size_t)m->c.vocab);
-            if (ksh_buffer_read(m->ctx, m->r_logits, (size_t)i * m->c.vocab * 4, logits.data(), logits.size() * 4, 0) ||
-                ksh_sample_softcap_min_p(logits.data(), logits.size(), m->c.softcap, temperature[i], min_p[i], seed[i], &next_ids[i]))
-                return 1;
-        }
-    }
-    return 0;
+    return draw_ids(m, m->r_logits, m->r_next, n, temperature, min_p, seed, next_ids);
 }
 
 ksh_buf *ksh_gemma4_round_logits(ksh_gemma4 *m) { return m ? m->r_logits : nullptr; }

@@ -85,6 +85,33 @@ struct DecodeTail {
     const uint8_t *embd; int dtype; int64_t n_rows; int n; float scale; float *x_out;
 };
 int launch_decode_tail(const ksh_kernel &k_argmax, const float *logits, DecodeTail t, hipStream_t st);
+
+// The sampled decode step (sample_device.hip, sample.cpp): the entries of a row of logits that can survive its min-p
+// filter are gathered on the device, the reference's arithmetic runs on those on the host.
+constexpr int kSampleMaxRows = 16, kSampleInline = 126;
+struct SampleRow {
+    float temperature;   // 0: a greedy row
+    float below;         // candidates lie at most this far below the best soft-capped logit
+};
+struct SampleCand { uint32_t id; float logit; };
+struct SampleHead {
+    uint32_t count, best_id;   // candidates (more than kSampleInline: all of them are in the device list), the argmax
+    float sum, pad;            // sum over the vocabulary of exp((y - best) / temperature)
+    SampleCand cand[kSampleInline];   // in no particular order
+};
+struct SampleScratch {
+    void *lists = nullptr, *joined = nullptr;   // device
+    SampleHead *heads = nullptr;                // pinned host memory
+    int rows = 0, n = 0;
+    ~SampleScratch();
+};
+int launch_sample_candidates(SampleScratch &s, const float *logits, int n, int rows, float cap, const float *best_ids, const SampleRow *params,
+                             hipStream_t st);
+// false: the row takes the whole vocabulary (no min-p filter)
+bool sample_row_params(float temperature, float min_p, SampleRow *out);
+// one draw; false: the logits are not finite and the row takes the whole vocabulary
+bool sample_from_candidates(SampleCand *cand, size_t count, float sum, size_t n, float cap, float temperature, float min_p, uint32_t seed,
+                            uint32_t *out);
 }  // namespace ksh
 
 // a pool's identity for whoever caches things per pool (HIP graphs captured over its buffers): unlike its address,

@@ -5,6 +5,7 @@
 // operation for operation on f32 logits (the reference reads them as f16): the
 // same pass structure, the same f32 accumulators, the same splitmix32 draw, so
 // that a seed picks the same id.
+#include <algorithm>
 #include <cmath>
 #include <vector>
 
@@ -23,6 +24,62 @@ uint32_t splitmix32(uint32_t &state)
 }
 
 }  // namespace
+
+namespace ksh {
+
+bool sample_row_params(float temperature, float min_p, SampleRow *out)
+{
+    if (!(min_p > 0.0f) || !(temperature >= 1e-6f) || !std::isfinite(temperature)) return false;
+    // An entry survives when exp((y - best) / temperature) >= min_p.  The margin is far above what the device's and the
+    // host's tanh and exp can differ by (an ulp or two of y, of the order of 1e-5 at a soft cap of 30); entries inside
+    // it that do not survive are dropped by the exact comparison below.
+    out->temperature = temperature;
+    out->below = std::fmax(-temperature * std::log(min_p), 0.0f) * 1.001f + 1e-3f + 1e-3f * temperature;
+    return true;
+}
+
+// ksh_sample_softcap_min_p below on the entries that can survive its filter.  The rest of the vocabulary takes part in
+// the result through the denominator alone, which scales every probability and the draw alike.
+bool sample_from_candidates(SampleCand *cand, size_t count, float sum, size_t n, float cap, float temperature, float min_p, uint32_t seed,
+                            uint32_t *out)
+{
+    if (!count || !std::isfinite(sum)) return false;
+    std::sort(cand, cand + count, [](const SampleCand &a, const SampleCand &b) { return a.id < b.id; });
+    uint32_t best_i = 0;
+    float best_v = -INFINITY;
+    for (size_t i = 0; i < count; i++) {
+        const float x = cand[i].logit;
+        const float y = cap > 0.0f ? cap * std::tanh(x / cap) : x;
+        cand[i].logit = y;
+        if (y > best_v) { best_v = y; best_i = cand[i].id; }
+    }
+    *out = best_i;
+    const float inv = 1.0f / std::fmax(sum, 1e-30f);
+    float p_max = 0.0f;
+    for (size_t i = 0; i < count; i++) {
+        const float x = std::exp((cand[i].logit - best_v) / temperature) * inv;
+        cand[i].logit = x;
+        if (x > p_max) p_max = x;
+    }
+    const float threshold = p_max * std::fmax(min_p, 0.0f);
+    float filtered = 0.0f;
+    for (size_t i = 0; i < count; i++) {
+        if (cand[i].logit < threshold) cand[i].logit = 0.0f;
+        else filtered += cand[i].logit;
+    }
+    if (filtered <= 1e-9f) return true;
+    uint32_t rng = seed | 1u;
+    const float r = ((float)splitmix32(rng) / 4294967296.0f) * filtered;
+    float cdf = 0.0f;
+    for (size_t i = 0; i < count; i++) {
+        cdf += cand[i].logit;
+        if (r < cdf) { *out = cand[i].id; return true; }
+    }
+    *out = (uint32_t)(n - 1);
+    return true;
+}
+
+}  // namespace ksh
 
 extern "C" int ksh_sample_softcap_min_p(const float *logits, size_t n, float cap, float temperature, float min_p, uint32_t seed,
                                         uint32_t *out)

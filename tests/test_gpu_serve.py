@@ -259,3 +259,25 @@ def test_destroying_a_busy_scheduler_frees_its_slots(ctx, model):
     assert pool.active_batch() == []
     m.bind_slot(None, 0)
     pool.close()
+
+
+@pytest.mark.parametrize("temperature,min_p", [(0.3, 0.05), (1.0, 0.5), (2.5, 0.001), (50.0, 0.9), (1.0, 1.5), (1.0, 0.0)])
+def test_draws_from_the_narrowed_logits_are_the_host_samplers(ctx, model, temperature, min_p):
+    """The device keeps only what can survive the min-p filter (few entries; more than a record holds; all of them; a
+    filter above 1; no filter): the draw is the host sampler's on the whole row, for the single step and for a round."""
+    m, cfg = model
+    (p,) = prompts_of(cfg, (5,), 706)
+    m.bind_slot(None, 0)
+    m.reset()
+    m.prefill_chunk(p[:-1])
+    for seed in range(3, 60, 7):
+        m.bind_slot(None, 4)
+        got = m.decode_token_sampled(p[-1], temperature, min_p, seed)
+        assert got == hip.sample_softcap_min_p(m.logits(), cfg["softcap"], temperature, min_p, seed)
+    pool = make_pool(ctx, cfg, 4)
+    slots = [pool.alloc() for _ in range(4)]
+    temps, seeds = [temperature, 0.0, temperature, 2 * temperature], [11, 12, 13, 14]
+    got = m.decode_round(pool, slots, p[:4], temps, [min_p] * 4, seeds)
+    rows = m.round_logits(4)
+    assert got == [hip.sample_softcap_min_p(rows[i], cfg["softcap"], temps[i], min_p, seeds[i]) for i in range(4)]
+    pool.close()
