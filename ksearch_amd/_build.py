@@ -9,6 +9,7 @@ import concurrent.futures as cf
 import os
 import subprocess
 import sys
+import sysconfig
 
 HERE = os.path.dirname(os.path.abspath(__file__))
 CSRC = os.path.join(HERE, "csrc")
@@ -63,9 +64,24 @@ def _link(objs: list[str], path: str) -> str:
     return path
 
 
+ENCODE_SRC = os.path.join(HERE, "pyext", "encode.c")
+ENCODE_PATH = os.path.join(LIBDIR, "_encode.so")
+
+
+def _build_encode() -> None:
+    """The binding's per-operator call as a CPython extension (host code; it gets the library's function by address)."""
+    tmp = ENCODE_PATH + ".tmp"
+    cmd = ["gcc", "-O2", "-Wall", "-shared", "-fPIC", "-I" + sysconfig.get_paths()["include"], ENCODE_SRC, "-o", tmp]
+    r = subprocess.run(cmd, capture_output=True, text=True)
+    if r.returncode:
+        raise RuntimeError(f"gcc failed on encode.c:\n{r.stderr}")
+    os.replace(tmp, ENCODE_PATH)
+
+
 def build(jobs: int = 8) -> str:
     """Compiles every source and links the library, then the timeline build beside it."""
     os.makedirs(OBJDIR, exist_ok=True)
+    _build_encode()
     srcs = sources()
     with cf.ThreadPoolExecutor(max_workers=jobs) as ex:
         objs = list(ex.map(_compile, srcs))

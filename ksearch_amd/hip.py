@@ -11,12 +11,15 @@ from __future__ import annotations
 
 import ctypes as C
 import enum
+import importlib.machinery
+import importlib.util
 import os
 
 import numpy as np
 
 _HERE = os.path.dirname(os.path.abspath(__file__))
 LIB_PATH = os.path.join(_HERE, "lib", "libksearch_hip.so")
+ENCODE_PATH = os.path.join(_HERE, "lib", "_encode.so")    # ksh_encode without ctypes in between (pyext/encode.c)
 
 
 class KshError(RuntimeError):
@@ -24,6 +27,7 @@ class KshError(RuntimeError):
 
 
 class DType(enum.IntEnum):          # crates/ksearch_ir/src/lib.rs:17-27
+    __hash__ = int.__hash__         # (members are keys of every operator's kernel lookup; Enum's own hash is a Python call)
     F32 = 0
     F16 = 1
     Q4K = 2
@@ -35,6 +39,7 @@ class DType(enum.IntEnum):          # crates/ksearch_ir/src/lib.rs:17-27
 
 
 class Kind(enum.IntEnum):           # enum ksh_kind
+    __hash__ = int.__hash__
     MATVEC = 1
     MATVEC_BATCH = 2
     MATVEC_QKV = 3
@@ -249,19 +254,25 @@ SYMBOLS = {
 }
 
 _lib = None
+_encode = None      # pyext/encode.c's encode(ctx, kernel, inputs, in_offs, outputs, out_offs) -> ksh_encode's code
 
 
 def lib() -> C.CDLL:
     """Loads the prebuilt library; never builds and never falls back."""
-    global _lib
+    global _lib, _encode
     if _lib is None:
-        if not os.path.exists(LIB_PATH):
-            raise KshError(f"{LIB_PATH} is missing: build it with `python -c 'import __graft_entry__ as g; g.build()'`")
+        for path in (LIB_PATH, ENCODE_PATH):
+            if not os.path.exists(path):
+                raise KshError(f"{path} is missing: build it with `python -c 'import __graft_entry__ as g; g.build()'`")
         L = C.CDLL(LIB_PATH)
         for name, (res, args) in SYMBOLS.items():
             fn = getattr(L, name)
             fn.restype, fn.argtypes = res, args
-        _lib = L
+        loader = importlib.machinery.ExtensionFileLoader("ksearch_amd._encode", ENCODE_PATH)
+        ext = importlib.util.module_from_spec(importlib.util.spec_from_loader(loader.name, loader))
+        loader.exec_module(ext)
+        ext.setup(C.cast(L.ksh_encode, C.c_void_p).value)
+        _lib, _encode = L, ext.encode
     return _lib
 
 
@@ -467,8 +478,9 @@ class Context:
         return Kernel(h.value)
 
     def encode_offsets_multi(self, kernel: Kernel, inputs, in_offs, outputs, out_offs) -> None:
-        _check(lib().ksh_encode(self.h, kernel.h, _bufs(inputs), _offs(in_offs, len(inputs)), len(inputs),
-                                _bufs(outputs), _offs(out_offs, len(outputs)), len(outputs)))
+        h = self.h
+        if _encode(h.value if h else None, kernel.h, inputs, in_offs, outputs, out_offs):
+            _check(1)
 
     def encode_multi(self, kernel: Kernel, inputs, outputs) -> None:
         self.encode_offsets_multi(kernel, inputs, None, outputs, None)
@@ -545,8 +557,7 @@ class Eng:
         self.cache: dict = {}
 
     def _k(self, ctx: Context, kind, dims=(), dtypes=(), params=(), sched=None) -> Kernel:
-        key = (int(kind), tuple(dims), tuple(int(d) for d in dtypes), tuple(params),
-               tuple(sorted(sched.items())) if isinstance(sched, dict) else None)
+        key = (kind, dims, dtypes, params, tuple(sorted(sched.items())) if isinstance(sched, dict) else None)
         k = self.cache.get(key)
         if k is None:
             k = ctx.compile(make_desc(kind, dims, dtypes, params, sched))
@@ -555,7 +566,7 @@ class Eng:
 
     # :137-160
     def matvec_wd(self, ctx, rows, cols, wdt, w, x, y, sched=None):
-        self.matvec_wd_at(ctx, rows, cols, wdt, w, x, 0, y, 0, sched)
+        ctx.encode_offsets_multi(self._k(ctx, Kind.MATVEC, (rows, cols), (wdt, DType.F32), (), sched), [w, x], None, [y], None)
 
     def matvec_wd_at(self, ctx, rows, cols, wdt, w, x, x_off, y, y_off, sched=None):
         k = self._k(ctx, Kind.MATVEC, (rows, cols), (wdt, DType.F32), (), sched)
