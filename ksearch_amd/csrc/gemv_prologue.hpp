@@ -200,7 +200,8 @@ struct StageRegs {
 // KIND: the prologue kind when the kernel is built for one (-1: read from the descriptor at run time).  With it and a
 // row length known at compile time the front of the kernel is a straight run of loads with constant offsets; with
 // neither it is a chain of compare-and-branch pairs, one per possible float4, in front of the first weight load.
-template <int NT, bool kMerge = false, int KMAX = kStageX, int KIND = -1>
+// H: the vectors (x, norm weights, residual, x_out) are half buffers; the partitions of kMergeParts stay f32.
+template <int NT, bool kMerge = false, int KMAX = kStageX, int KIND = -1, bool H = false>
 __device__ __forceinline__ void stage_fetch(const Prologue &pr_in, int cols, StageRegs &s)
 {
     Prologue pr = pr_in;
@@ -238,25 +239,25 @@ __device__ __forceinline__ void stage_fetch(const Prologue &pr_in, int cols, Sta
 #pragma unroll
     for (int k = 0; k < KX; k++) {
         const int i = tid + k * NT;
-        if (wbase + k * NT < n4) s.x[k] = ldg_f4(pr.x, i);
+        if (wbase + k * NT < n4) s.x[k] = act_ld4<H>(pr.x, i);
     }
     if (pr.kind == kPlain) return;
 #pragma unroll
     for (int k = 0; k < KP; k++) {
         const int i = tid + k * NT;
-        if (wbase + k * NT < n4) s.wn[k] = ldg_f4(pr.w_norm, i);
+        if (wbase + k * NT < n4) s.wn[k] = act_ld4<H>(pr.w_norm, i);
     }
     if (pr.kind != kAddThenRms) return;
 #pragma unroll
     for (int k = 0; k < KP; k++) {
         const int i = tid + k * NT;
-        if (wbase + k * NT < n4) { s.wp[k] = ldg_f4(pr.w_post, i); s.rs[k] = ldg_f4(pr.res, i); }
+        if (wbase + k * NT < n4) { s.wp[k] = act_ld4<H>(pr.w_post, i); s.rs[k] = act_ld4<H>(pr.res, i); }
     }
 }
 
 // Every thread must call this (it contains barriers); the LDS image is complete
 // after the caller's next __syncthreads().
-template <int XF, int NT, bool kMerge = false, int KMAX = kStageX, int KIND = -1>
+template <int XF, int NT, bool kMerge = false, int KMAX = kStageX, int KIND = -1, bool H = false>
 __device__ __forceinline__ void stage_finish(const Prologue &pr_in, uint8_t *lds, int cols, StageRegs &s)
 {
     Prologue pr = pr_in;
@@ -293,7 +294,7 @@ __device__ __forceinline__ void stage_finish(const Prologue &pr_in, uint8_t *lds
     }
     if (pr.kind == kPlain) {
         if (KMAX >= kStageX && n4 > NT * kStageX) {
-            for (int i = tid; i < n4; i += NT) store_x4<XF>(lds, cols, i, ldg_f4(pr.x, i));
+            for (int i = tid; i < n4; i += NT) store_x4<XF>(lds, cols, i, act_ld4<H>(pr.x, i));
             return;
         }
 #pragma unroll
@@ -358,7 +359,7 @@ __device__ __forceinline__ void stage_finish(const Prologue &pr_in, uint8_t *lds
                 v[k].y = (r.y + v[k].y * inv * w.y) * sc;
                 v[k].z = (r.z + v[k].z * inv * w.z) * sc;
                 v[k].w = (r.w + v[k].w * inv * w.w) * sc;
-                if (blockIdx.x == 0) stg_f4(pr.x_out, i, v[k]);
+                if (blockIdx.x == 0) act_st4<H>(pr.x_out, i, v[k]);
             }
         }
         const float ss2 = (sc * sc) * fmaf(inv * inv, acc[3], fmaf(2.0f * inv, acc[2], acc[1]));

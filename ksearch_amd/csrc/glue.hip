@@ -43,26 +43,63 @@ __global__ void fill_zero_kernel(uint4 *p, size_t n16, uint8_t *tail, size_t nta
 }
 
 // y = (x * rsqrt(mean(x^2) + eps)) * w  (+ residual)  (* scale)
-__global__ __launch_bounds__(kNormThreads) void rmsnorm_kernel(const float *__restrict__ x,
-                                                               const float *__restrict__ w,
-                                                               const float *res, float *y, int n, float eps,
+// PER: elements a thread holds (n <= 256 * PER).  Every input is requested before the first is used and x is read once:
+// with the two passes as loops over memory a row of 2048 was sixteen round trips, one behind the other (8.2 us for one
+// row of half values in a trace, 6.5 with this).  A thread's elements are added in the same order as there.  H: half buffers.
+template <int PER, bool H>
+__global__ __launch_bounds__(kNormThreads) void rmsnorm_kernel(const float *x, const float *__restrict__ w, const float *res, float *y, int n, float eps,
                                                                int has_res, int has_scale, float scale)
 {
     __shared__ float red[4];
     // rows form (rmsnorm_rows / rmsnorm_add_rows / rmsnorm_add_scale_rows, crates/ksearch_kernels/src/lib.rs:1478-1560):
     // one workgroup per row of a [rows, n] matrix, the weight shared
-    x += (size_t)blockIdx.x * n;
-    y += (size_t)blockIdx.x * n;
-    if (has_res) res += (size_t)blockIdx.x * n;
+    const size_t row = (size_t)blockIdx.x * n;
+    float xv[PER], wv[PER], rv[PER];
+#pragma unroll
+    for (int u = 0; u < PER; u++) {
+        const int i = threadIdx.x + u * kNormThreads;
+        xv[u] = i < n ? act_ld<H>(x, row + i) : 0.f;
+    }
+#pragma unroll
+    for (int u = 0; u < PER; u++) {
+        const int i = threadIdx.x + u * kNormThreads;
+        wv[u] = i < n ? act_ld<H>(w, i) : 0.f;
+        rv[u] = has_res && i < n ? act_ld<H>(res, row + i) : 0.f;
+    }
     float ss = 0.f;
-    for (int i = threadIdx.x; i < n; i += kNormThreads) ss += x[i] * x[i];
+#pragma unroll
+    for (int u = 0; u < PER; u++) ss += xv[u] * xv[u];
+    ss = block_sum_256(ss, red);
+    const float inv = 1.0f / sqrtf(ss / (float)n + eps);
+#pragma unroll
+    for (int u = 0; u < PER; u++) {
+        const int i = threadIdx.x + u * kNormThreads;
+        float v = xv[u] * inv * wv[u];
+        if (has_res) v = v + rv[u];
+        if (has_scale) v = scale * v;
+        if (i < n) act_st<H>(y, row + i, v);
+    }
+}
+
+// rows that do not fit a workgroup's registers
+template <bool H>
+__global__ __launch_bounds__(kNormThreads) void rmsnorm_long_kernel(const float *x, const float *__restrict__ w, const float *res, float *y, int n, float eps,
+                                                                    int has_res, int has_scale, float scale)
+{
+    __shared__ float red[4];
+    const size_t row = (size_t)blockIdx.x * n;
+    float ss = 0.f;
+    for (int i = threadIdx.x; i < n; i += kNormThreads) {
+        const float v = act_ld<H>(x, row + i);
+        ss += v * v;
+    }
     ss = block_sum_256(ss, red);
     const float inv = 1.0f / sqrtf(ss / (float)n + eps);
     for (int i = threadIdx.x; i < n; i += kNormThreads) {
-        float v = x[i] * inv * w[i];
-        if (has_res) v = v + res[i];
+        float v = act_ld<H>(x, row + i) * inv * act_ld<H>(w, i);
+        if (has_res) v = v + act_ld<H>(res, row + i);
         if (has_scale) v = scale * v;
-        y[i] = v;
+        act_st<H>(y, row + i, v);
     }
 }
 
@@ -108,7 +145,8 @@ __global__ __launch_bounds__(256) void quantize_q40_kernel(const float *__restri
 // (rms*w, RoPE, f32 out); blocks n_q..n_q+n_kv-1 do K (rms*w, RoPE, Q4_0) and
 // V (rms without weight, Q4_0) of one kv head.  RoPE pairs (i, i+hd/2) with
 // the row cos[0..hd/2) || sin[0..hd/2).  hd is 128, 256 or 512.
-template <int HD>
+// H: q, k, v, the norm weights and q_out are half buffers.
+template <int HD, bool H>
 __global__ __launch_bounds__(64) void per_head_qkv_q40_kernel(
     const float *q, const float *__restrict__ qw, const float *__restrict__ rope,
     const float *__restrict__ k, const float *__restrict__ kw, const float *__restrict__ v,
@@ -120,10 +158,7 @@ __global__ __launch_bounds__(64) void per_head_qkv_q40_kernel(
     // batch form (rmsnorm_per_head_qkv_q40_batch, crates/ksearch_kernels/src/lib.rs:1750): blockIdx.y is the token
     // of a chunk of consecutive positions; its q / k / v rows, rope row and cache rows follow the first token's
     const int tok = blockIdx.y;
-    q += (size_t)tok * n_q * HD;
-    k += (size_t)tok * n_kv * HD;
-    v += (size_t)tok * n_kv * HD;
-    q_out += (size_t)tok * n_q * HD;
+    const size_t q0 = (size_t)tok * n_q * HD, kv0 = (size_t)tok * n_kv * HD;
     if (slot_ids) {
         // tokens of different sequences (one decode step for several KV slots): token i has its own record
         // meta[4 i .. ] with its position in [3], and appends to slot slot_ids[i] of caches laid out
@@ -151,7 +186,8 @@ __global__ __launch_bounds__(64) void per_head_qkv_q40_kernel(
     const int head = blockIdx.x;
     const bool is_q = head < n_q;
     const int h = is_q ? head : head - n_q;
-    const float *x = (is_q ? q : k) + (size_t)h * HD;
+    const float *x = is_q ? q : k;
+    const size_t x0 = (is_q ? q0 : kv0) + (size_t)h * HD;
     const float *w = is_q ? qw : kw;
 
     // lane owns elements lane + 64*j: consecutive lanes hold consecutive
@@ -160,14 +196,14 @@ __global__ __launch_bounds__(64) void per_head_qkv_q40_kernel(
     float ss = 0.f;
 #pragma unroll
     for (int j = 0; j < PER; j++) {
-        xv[j] = x[lane + 64 * j];
+        xv[j] = act_ld<H>(x, x0 + lane + 64 * j);
         ss += xv[j] * xv[j];
     }
     ss = wave_sum(ss);
     const float inv = 1.0f / sqrtf(ss / (float)HD + eps);
     float nv[PER];
 #pragma unroll
-    for (int j = 0; j < PER; j++) nv[j] = xv[j] * inv * w[lane + 64 * j];
+    for (int j = 0; j < PER; j++) nv[j] = xv[j] * inv * act_ld<H>(w, lane + 64 * j);
     // RoPE: element e < HALF pairs with e + HALF, i.e. register j with j + PER/2
     float ro[PER];
 #pragma unroll
@@ -180,7 +216,7 @@ __global__ __launch_bounds__(64) void per_head_qkv_q40_kernel(
     }
     if (is_q) {
 #pragma unroll
-        for (int j = 0; j < PER; j++) q_out[(size_t)h * HD + lane + 64 * j] = ro[j];
+        for (int j = 0; j < PER; j++) act_st<H>(q_out, q0 + (size_t)h * HD + lane + 64 * j, ro[j]);
         return;
     }
     uint8_t *krow = k_out + (size_t)h * (HD / 32) * 18;
@@ -188,11 +224,10 @@ __global__ __launch_bounds__(64) void per_head_qkv_q40_kernel(
 #pragma unroll
     for (int j = 0; j < PER; j++) pack_q40_group(ro[j], lane & 31, krow + (size_t)(2 * j + (lane >> 5)) * 18, true);
 
-    const float *vx = v + (size_t)h * HD;
     float vs = 0.f;
 #pragma unroll
     for (int j = 0; j < PER; j++) {
-        xv[j] = vx[lane + 64 * j];
+        xv[j] = act_ld<H>(v, kv0 + (size_t)h * HD + lane + 64 * j);
         vs += xv[j] * xv[j];
     }
     vs = wave_sum(vs);
@@ -404,10 +439,13 @@ int done(const char *what)
     return e == hipSuccess ? 0 : hip_fail(e, what);
 }
 
+template <bool H>
 int launch_rmsnorm(const ksh_kernel &k, const LaunchArgs &a, hipStream_t st)
 {
     const int n = (int)k.desc.dims[0], has_res = (int)k.desc.dims[1], has_scale = (int)k.desc.dims[2];
-    hipLaunchKernelGGL(rmsnorm_kernel, dim3((unsigned)max((int64_t)1, k.desc.dims[3])), dim3(kNormThreads), 0, st, (const float *)a.in[0],
+    auto *kernel = n <= 2 * kNormThreads ? rmsnorm_kernel<2, H> : n <= 8 * kNormThreads ? rmsnorm_kernel<8, H>
+                   : n <= 24 * kNormThreads ? rmsnorm_kernel<24, H> : rmsnorm_long_kernel<H>;
+    hipLaunchKernelGGL(kernel, dim3((unsigned)max((int64_t)1, k.desc.dims[3])), dim3(kNormThreads), 0, st, (const float *)a.in[0],
                        (const float *)a.in[1], has_res ? (const float *)a.in[2] : nullptr, (float *)a.out[0], n,
                        k.desc.params[0], has_res, has_scale, k.desc.params[1]);
     return done("rmsnorm launch");
@@ -422,12 +460,13 @@ int launch_rmsnorm_add_then(const ksh_kernel &k, const LaunchArgs &a, hipStream_
     return done("rmsnorm_add_then_rmsnorm launch");
 }
 
+template <bool H>
 int launch_per_head(const ksh_kernel &k, const LaunchArgs &a, hipStream_t st)
 {
     const int n_q = (int)k.desc.dims[0], n_kv = (int)k.desc.dims[1], hd = (int)k.desc.dims[2];
     const dim3 grid(n_q + n_kv, (unsigned)max((int64_t)1, k.desc.dims[4])), block(64);
 #define KSH_PH(HD)                                                                                           \
-    hipLaunchKernelGGL((per_head_qkv_q40_kernel<HD>), grid, block, 0, st, (const float *)a.in[0],            \
+    hipLaunchKernelGGL((per_head_qkv_q40_kernel<HD, H>), grid, block, 0, st, (const float *)a.in[0],            \
                        (const float *)a.in[1], (const float *)a.in[2], (const float *)a.in[3],               \
                        (const float *)a.in[4], (const float *)a.in[5], (float *)a.out[0], (uint8_t *)a.out[1], \
                        (uint8_t *)a.out[2], n_q, n_kv, k.desc.params[0],                                      \
@@ -577,7 +616,8 @@ int bind_rmsnorm(ksh_kernel &k)
         k.out_align[0] = 4;
         set_launch(k, (uint32_t)rows, 1, 1, kNormThreads, 16);
         set_name(k, "rmsnorm%s%s%s", has_res ? "_add" : "", k.desc.dims[2] ? "_scale" : "", rows > 1 ? "_rows" : "");
-        k.launch = launch_rmsnorm;
+        k.launch = launch_rmsnorm<false>;
+        k.launch_half = launch_rmsnorm<true>;
         return 0;
     }
     // the reference stages the residual stream in threadgroup memory and
@@ -628,7 +668,8 @@ int bind_per_head_qkv_q40(ksh_kernel &k)
     k.out_bytes[1] = k.out_bytes[2] = kvb; k.out_align[1] = k.out_align[2] = 2;
     set_launch(k, (uint32_t)(n_q + n_kv), (uint32_t)n_tok, 1, 64, 0);
     set_name(k, "rmsnorm_per_head_qkv_q40_hd%d%s", (int)hd, n_slots ? "_slots" : n_tok > 1 ? "_batch" : "");
-    k.launch = launch_per_head;
+    k.launch = launch_per_head<false>;
+    k.launch_half = launch_per_head<true>;
     return 0;
 }
 

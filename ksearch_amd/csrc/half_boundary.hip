@@ -7,7 +7,9 @@
 // half, everything else keeps its type -- packed weights and caches, and the buffers the reference keeps in f32
 // (the rope table :33-56, the meta record :637, token ids, split-KV partials, the argmax index).
 //
-// Mechanics: the handle wraps the f32 handle of the same descriptor.  One launch widens all half inputs into f32
+// Mechanics: the handle wraps the f32 handle of the same descriptor.  Where that handle's kernel is also built over half
+// buffers (ksh_kernel::launch_half: the Q4_K GEMV family, RMSNorm, per-head norm + append, split-KV attention), it is
+// that one launch.  Otherwise one launch widens all half inputs into f32
 // staging that belongs to the handle, the f32 kernel runs on the staging, one launch narrows the results
 // (round to nearest even, what the reference's kernels do when they store a half).  Arithmetic is therefore the
 // f32 path's, bit for bit, on the widened inputs.  The decode loops inside the library keep f32 activations and do
@@ -83,6 +85,8 @@ int launch_half(const ksh_kernel &k, const LaunchArgs &a, hipStream_t st)
     if (in.launch(in, b, st)) return 1;
     return convert<false>(narrow, st);
 }
+
+int launch_half_native(const ksh_kernel &k, const LaunchArgs &a, hipStream_t st) { return k.inner->launch_half(*k.inner, a, st); }
 
 // Which bindings of a kind are activations: one letter per binding, 'A' activation (half at this boundary),
 // anything else keeps its type ('W' packed bytes, 'F' f32: meta, rope, token ids, partials, indices).
@@ -176,11 +180,11 @@ int bind_half_boundary(ksh_kernel &k, const ksh_kernel &inner)
         k.out_align[i] = 2;
         k.stage_out[i] = take(inner.out_bytes[i]);
     }
-    k.scratch_bytes = off;
+    k.scratch_bytes = inner.launch_half ? 0 : off;
     char name[sizeof(k.info.name)];
     snprintf(name, sizeof(name), "%.58s_f16", inner.info.name);
     memcpy(k.info.name, name, sizeof(name));
-    k.launch = launch_half;
+    k.launch = inner.launch_half ? launch_half_native : launch_half;
     return 0;
 }
 

@@ -93,6 +93,44 @@ __device__ __forceinline__ void stg_f4(float *p, size_t i, float4 v)
 }
 __device__ __forceinline__ void stg_f32(float *p, size_t i, float v) { ((KSH_GLOBAL float *)p)[i] = v; }
 
+// Activations as the caller's buffers hold them: f32, or half (H) at any 2-byte aligned address, widened on the way in
+// and rounded to nearest even on the way out.
+// (Pinned on the way to the conversion: where the value is a product, one instruction would multiply and round to half in
+// one step, which is another rounding and loses a zero's sign.)
+typedef _Float16 h16x4_a2_t __attribute__((ext_vector_type(4), aligned(2)));
+__device__ __forceinline__ _Float16 half_rn(float v)
+{
+    asm volatile("" : "+v"(v));
+    return (_Float16)v;
+}
+template <bool H>
+__device__ __forceinline__ float4 act_ld4(const float *p, size_t i)
+{
+    if (!H) return ldg_f4(p, i);
+    const h16x4_a2_t v = *(const KSH_GLOBAL h16x4_a2_t *)((const KSH_GLOBAL char *)p + 8 * i);
+    return make_float4((float)v.x, (float)v.y, (float)v.z, (float)v.w);
+}
+template <bool H>
+__device__ __forceinline__ void act_st4(float *p, size_t i, float4 v)
+{
+    if (!H) return stg_f4(p, i, v);
+    h16x4_a2_t w;
+    w.x = half_rn(v.x); w.y = half_rn(v.y); w.z = half_rn(v.z); w.w = half_rn(v.w);
+    *(KSH_GLOBAL h16x4_a2_t *)((KSH_GLOBAL char *)p + 8 * i) = w;
+}
+template <bool H>
+__device__ __forceinline__ float act_ld(const float *p, size_t i)
+{
+    if (!H) return p[i];
+    return (float)((const _Float16 *)p)[i];
+}
+template <bool H>
+__device__ __forceinline__ void act_st(float *p, size_t i, float v)
+{
+    if (!H) ((KSH_GLOBAL float *)p)[i] = v;
+    else ((KSH_GLOBAL _Float16 *)p)[i] = half_rn(v);
+}
+
 constexpr int kWave = 64;
 
 // A zero the compiler cannot see through, in a vector register.  Added to the index of a load whose address is the

@@ -56,6 +56,8 @@ struct ksh_kernel {
     size_t scratch_bytes = 0;
     void *scratch = nullptr;
     int (*launch)(const ksh_kernel &, const ksh::LaunchArgs &, hipStream_t) = nullptr;
+    // the same launch taking half buffers for its activations as they are, where the kernel is built for them
+    int (*launch_half)(const ksh_kernel &, const ksh::LaunchArgs &, hipStream_t) = nullptr;
     // a handle with half activations at the boundary (half_boundary.hip): the f32 handle it wraps, which bindings are
     // half, and where their f32 staging lies in `scratch`
     const ksh_kernel *inner = nullptr;

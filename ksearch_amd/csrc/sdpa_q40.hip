@@ -185,26 +185,43 @@ __global__ __launch_bounds__(kThreads) void sdpa_part_kernel(SdpaParams p)
     }
 }
 
-// grid = (n_q, n_slots); lower.rs:5897-6087
+// grid = (n_q, n_slots); lower.rs:5897-6087.  H: the result is a half buffer.  The partitions are folded in order, but
+// requested eight at a time: one by one their loads were sixteen round trips, one behind the other (8.5 us for 8 heads of
+// 256 in 16 partitions; 5.2 so).
+template <bool H>
 __global__ __launch_bounds__(kThreads) void sdpa_reduce_kernel(const float *tmp, float *out, int n_q, int hd, int nwg)
 {
+    constexpr int B = 8;
     const int head = blockIdx.x, slot = blockIdx.y, tid = threadIdx.x;
     const float *base = tmp + ((size_t)slot * n_q + head) * nwg * (size_t)(hd + 2);
+    const int d0 = min(tid, hd - 1), d1 = min(tid + kThreads, hd - 1);
+    const bool wide = hd > kThreads;
     float m = -1.0e30f, l = 0.f, O0 = 0.f, O1 = 0.f;
-    for (int pt = 0; pt < nwg; pt++) {
-        const float *rec = base + (size_t)pt * (hd + 2);
-        const float mp = rec[0], lp = rec[1];
-        const float m2 = fmaxf(m, mp);
-        const float a = __expf(m - m2), b = __expf(mp - m2);
-        l = l * a + lp * b;
-        m = m2;
-        if (tid < hd) O0 = O0 * a + rec[2 + tid] * b;
-        if (tid + kThreads < hd) O1 = O1 * a + rec[2 + tid + kThreads] * b;
+    for (int p0 = 0; p0 < nwg; p0 += B) {
+        float mp[B], lp[B], v0[B], v1[B];
+#pragma unroll
+        for (int u = 0; u < B; u++) {
+            const float *rec = base + (size_t)min(p0 + u, nwg - 1) * (hd + 2);
+            mp[u] = rec[0];
+            lp[u] = rec[1];
+            v0[u] = rec[2 + d0];
+            v1[u] = wide ? rec[2 + d1] : 0.f;
+        }
+#pragma unroll
+        for (int u = 0; u < B; u++) {
+            if (p0 + u >= nwg) break;
+            const float m2 = fmaxf(m, mp[u]);
+            const float a = __expf(m - m2), b = __expf(mp[u] - m2);
+            l = l * a + lp[u] * b;
+            m = m2;
+            O0 = O0 * a + v0[u] * b;
+            O1 = O1 * a + v1[u] * b;
+        }
     }
     const float inv_l = 1.0f / l;
-    float *o = out + ((size_t)slot * n_q + head) * hd;
-    if (tid < hd) o[tid] = O0 * inv_l;
-    if (tid + kThreads < hd) o[tid + kThreads] = O1 * inv_l;
+    const size_t o = ((size_t)slot * n_q + head) * hd;
+    if (tid < hd) act_st<H>(out, o + tid, O0 * inv_l);
+    if (tid + kThreads < hd) act_st<H>(out, o + tid + kThreads, O1 * inv_l);
 }
 
 size_t part_lds_bytes(int groups, int hd)
@@ -259,10 +276,11 @@ int launch_mwg_part(const ksh_kernel &k, const LaunchArgs &a, hipStream_t st)
     return done("sdpa_mwg_part launch");
 }
 
+template <bool H>
 int launch_mwg_reduce(const ksh_kernel &k, const LaunchArgs &a, hipStream_t st)
 {
     const int n_q = (int)k.desc.dims[0], hd = (int)k.desc.dims[1], nwg = (int)k.desc.dims[2];
-    hipLaunchKernelGGL(sdpa_reduce_kernel, dim3(n_q, 1), dim3(kThreads), 0, st, (const float *)a.in[0],
+    hipLaunchKernelGGL(sdpa_reduce_kernel<H>, dim3(n_q, 1), dim3(kThreads), 0, st, (const float *)a.in[0],
                        (float *)a.out[0], n_q, hd, nwg);
     return done("sdpa_mwg_reduce launch");
 }
@@ -279,7 +297,7 @@ int launch_slots(const ksh_kernel &k, const LaunchArgs &a, hipStream_t st)
     p.nwg = k.variant;
     launch_part(p, n_slots, st);
     if (done("sdpa_slots part launch")) return 1;
-    hipLaunchKernelGGL(sdpa_reduce_kernel, dim3(p.n_q, n_slots), dim3(kThreads), 0, st, p.tmp, p.out, p.n_q, p.hd,
+    hipLaunchKernelGGL(sdpa_reduce_kernel<false>, dim3(p.n_q, n_slots), dim3(kThreads), 0, st, p.tmp, p.out, p.n_q, p.hd,
                        p.nwg);
     return done("sdpa_slots reduce launch");
 }
@@ -312,7 +330,7 @@ int launch_batch(const ksh_kernel &k, const LaunchArgs &a, hipStream_t st)
     p.kv_shared = 1;
     launch_part(p, n_tok, st);
     if (done("sdpa_batch part launch")) return 1;
-    hipLaunchKernelGGL(sdpa_reduce_kernel, dim3(p.n_q, n_tok), dim3(kThreads), 0, st, p.tmp, p.out, p.n_q, p.hd, p.nwg);
+    hipLaunchKernelGGL(sdpa_reduce_kernel<false>, dim3(p.n_q, n_tok), dim3(kThreads), 0, st, p.tmp, p.out, p.n_q, p.hd, p.nwg);
     return done("sdpa_batch reduce launch");
 }
 
@@ -342,7 +360,8 @@ int bind_sdpa(ksh_kernel &k)
         k.out_bytes[0] = (size_t)n_q * hd * 4; k.out_align[0] = 4;
         set_launch(k, (uint32_t)n_q, 1, 1, kThreads, 0);
         set_name(k, "sdpa_mwg_reduce_hd%d_nwg%d", (int)hd, (int)nwg);
-        k.launch = launch_mwg_reduce;
+        k.launch = launch_mwg_reduce<false>;
+        k.launch_half = launch_mwg_reduce<true>;
         return 0;
     }
     if (k.desc.dtypes[0] != KSH_Q40) return set_error("sdpa: kv dtype %d is not built (Q4_0 is)", k.desc.dtypes[0]);

@@ -68,7 +68,7 @@ struct LaneParams {
     int groups;   // q heads this workgroup handles: (n_q / n_kv) / hsplit
     int hsplit;   // workgroups that share a kv head's rows, each with its own q heads
     int balance;  // the launch's nwg * n_slots partitions are dealt to the slots by length (kModeMerge, several slots)
-    int rope_row; // fused: `rope` is the current position's row of the table, not the table
+    int rope_row; // fused: `rope` is the current position's row of the table, not the table; otherwise: q is a half buffer
     int kv_shared; // every slot attends the same cache (a chunk of prompt tokens, one meta record and one q per token)
     int no_append; // fused: the step's K / V row is in the cache already (a layer that reuses another layer's cache): q is normed and
                    // roped as usual, nothing is appended, every attended row comes from the cache
@@ -718,7 +718,9 @@ __global__ __launch_bounds__(NW * 64) void sdpa_lanes_kernel(LaneParams p_in)
 #pragma unroll
         for (int h = 0; h < GP; h++) {
             const float *qh = qg + (size_t)min(h, groups - 1) * HD + 32 * b + 4 * w;
-            const float4 a = *reinterpret_cast<const float4 *>(qh), d = *reinterpret_cast<const float4 *>(qh + 16);
+            const size_t i4 = (((size_t)slot * p.n_q + head0 + min(h, groups - 1)) * HD + 32 * b + 4 * w) / 4;
+            const float4 a = p.rope_row ? act_ld4<true>(p.q, i4) : *reinterpret_cast<const float4 *>(qh);
+            const float4 d = p.rope_row ? act_ld4<true>(p.q, i4 + 4) : *reinterpret_cast<const float4 *>(qh + 16);
             const float sc = h < groups ? p.scale : 0.f;
             qv[h][0] = a.x * sc; qv[h][1] = a.y * sc; qv[h][2] = a.z * sc; qv[h][3] = a.w * sc;
             qv[h][4] = d.x * sc; qv[h][5] = d.y * sc; qv[h][6] = d.z * sc; qv[h][7] = d.w * sc;
@@ -1548,11 +1550,11 @@ int launch_inst(const LaneParams &p, int n_slots, hipStream_t st)
     return e == hipSuccess ? 0 : hip_fail(e, "sdpa (register form) launch");
 }
 
-// which launches take the instances for one or two q heads per workgroup: the fused decode step at heads of 256 and 512
+// which launches take the instances for one or two q heads per workgroup: at heads of 256 and 512 the fused decode step,
+// and split-KV partials with one head per workgroup
 bool lanes_few_heads(int fused, int mode, int groups, int hd)
 {
-    (void)mode;
-    return fused && (hd == 256 || hd == 512) && groups <= 2;
+    return (hd == 256 || hd == 512) && (fused ? groups <= 2 : mode == kModePart && groups == 1);
 }
 
 int launch_lanes(const LaneParams &p, int hd, int nw, int n_slots, hipStream_t st)
@@ -1560,7 +1562,11 @@ int launch_lanes(const LaneParams &p, int hd, int nw, int n_slots, hipStream_t s
     // the decode step with one or two q heads per workgroup (heads of 256): instances of their own
     if (lanes_few_heads(p.fused, p.mode, p.groups, hd) && (nw == 4 || nw == 8)) {
         const dim3 grid(p.nwg, p.n_kv * p.hsplit, n_slots);
-        if (hd == 512 && p.groups == 1 && nw == 8) hipLaunchKernelGGL((sdpa_lanes_kernel<512, 1, 8, true>), grid, dim3(512), (lanes_lds_bytes<512, 1, 8>()), st, p);
+        if (!p.fused && hd == 512 && nw == 8) hipLaunchKernelGGL((sdpa_lanes_kernel<512, 1, 8, false>), grid, dim3(512), (lanes_lds_bytes<512, 1, 8>()), st, p);
+        else if (!p.fused && hd == 512) hipLaunchKernelGGL((sdpa_lanes_kernel<512, 1, 4, false>), grid, dim3(256), (lanes_lds_bytes<512, 1, 4>()), st, p);
+        else if (!p.fused && nw == 8) hipLaunchKernelGGL((sdpa_lanes_kernel<256, 1, 8, false>), grid, dim3(512), (lanes_lds_bytes<256, 1, 8>()), st, p);
+        else if (!p.fused) hipLaunchKernelGGL((sdpa_lanes_kernel<256, 1, 4, false>), grid, dim3(256), (lanes_lds_bytes<256, 1, 4>()), st, p);
+        else if (hd == 512 && p.groups == 1 && nw == 8) hipLaunchKernelGGL((sdpa_lanes_kernel<512, 1, 8, true>), grid, dim3(512), (lanes_lds_bytes<512, 1, 8>()), st, p);
         else if (hd == 512 && p.groups == 1) hipLaunchKernelGGL((sdpa_lanes_kernel<512, 1, 4, true>), grid, dim3(256), (lanes_lds_bytes<512, 1, 4>()), st, p);
         else if (hd == 512 && nw == 8) hipLaunchKernelGGL((sdpa_lanes_kernel<512, 2, 8, true>), grid, dim3(512), (lanes_lds_bytes<512, 2, 8>()), st, p);
         else if (hd == 512) hipLaunchKernelGGL((sdpa_lanes_kernel<512, 2, 4, true>), grid, dim3(256), (lanes_lds_bytes<512, 2, 4>()), st, p);
@@ -1604,7 +1610,8 @@ LaneParams base_params(const ksh_kernel &k)
 // to derive the table itself.
 bool balanced_slots(int n_slots, int nwg) { return n_slots > 1 && n_slots <= 16 && nwg >= 2 && nwg <= 64; }
 
-// variant: nwg | NW << 16 | hsplit << 24
+// variant: nwg | NW << 16 | hsplit << 24.  H: q is a half buffer (split-KV partials)
+template <bool H = false>
 int launch_bound(const ksh_kernel &k, const LaunchArgs &a, hipStream_t st)
 {
     LaneParams p = base_params(k);
@@ -1656,6 +1663,7 @@ int launch_bound(const ksh_kernel &k, const LaunchArgs &a, hipStream_t st)
         p.tmp = (float *)a.out[0];
         p.scale = k.desc.params[0];
         p.mode = kModePart;
+        p.rope_row = H;
         break;
     case KSH_SDPA_SLOTS:
         n_slots = (int)k.desc.dims[4];
@@ -1787,7 +1795,7 @@ int bind_sdpa_lanes(ksh_kernel &k, int nwg, int n_slots)
         k.info.sched.lds_tile = 32;
         k.info.sched.unroll = 1;
         k.variant = nwg | (0xFD << 16) | (1 << 24);
-        k.launch = launch_bound;
+        k.launch = launch_bound<>;
         return 0;
     }
     if (k.desc.sched.vec == 2 || (k.desc.sched.vec == 0 && mfma_fits && !batch_fits)) {
@@ -1812,7 +1820,7 @@ int bind_sdpa_lanes(ksh_kernel &k, int nwg, int n_slots)
         k.info.sched.lds_tile = tile;
         k.info.sched.unroll = 1;
         k.variant = nwg | ((tile == 32 ? 0xFF : 0xFE) << 16) | (1 << 24);
-        k.launch = launch_bound;
+        k.launch = launch_bound<>;
         return 0;
     }
     int nw = k.desc.sched.nsg ? (int)k.desc.sched.nsg : 0;
@@ -1826,6 +1834,7 @@ int bind_sdpa_lanes(ksh_kernel &k, int nwg, int n_slots)
     // heads of 512, merging, 16 partitions, eight waves: one head per workgroup 8.3 / 9.6 / 15.2 us at 320 / 1000 / 3000
     // rows against 8.9 / 10.9 / 17.3 with two)
     int hsplit = k.desc.sched.unroll ? (int)k.desc.sched.unroll
+                 : k.desc.kind == KSH_SDPA_MWG_PART && (hd == 256 || hd == 512) ? total_groups   // (a partition of a few dozen rows: one head per workgroup, 5.6 us against 9.7 for 8 heads of 256, 700 rows, 16 partitions)
                  : k.desc.kind != KSH_ATTEND_DECODE || total_groups < 4 ? 1
                  : k.desc.dims[5] || hd == 512 ? total_groups : (total_groups % 2 == 0 ? total_groups / 2 : 1);
     // heads of 512: at most four per workgroup (the fold's LDS)
@@ -1836,6 +1845,7 @@ int bind_sdpa_lanes(ksh_kernel &k, int nwg, int n_slots)
     // the unmerged decode step with one head per workgroup: four waves (eight row groups to fold instead of sixteen; in
     // cfg4's loop 1207-1210 against 1194-1197 tok/s with eight, per launch 4.1 against 4.7 us at 64 rows, equal at 300 - 600)
     if (!k.desc.sched.nsg && k.desc.kind == KSH_ATTEND_DECODE && k.desc.dims[5] != 0 && wg_groups == 1 && hd == 256) nw = 4;
+    if (!k.desc.sched.nsg && k.desc.kind == KSH_SDPA_MWG_PART && wg_groups == 1) nw = hd == 256 ? 4 : 8;
     // heads of 512, one per workgroup, merging: eight waves at every partition length (16 row groups of 32 lanes)
     if (!k.desc.sched.nsg && k.desc.kind == KSH_ATTEND_DECODE && k.desc.dims[5] == 0 && wg_groups == 1 && hd == 512) nw = 8;
     const size_t lds = lanes_lds(hd, wg_groups, nw, k.desc.kind == KSH_ATTEND_DECODE && lanes_few_heads(1, k.desc.dims[5] ? kModeSplitPart : kModeMerge, wg_groups, hd));
@@ -1853,7 +1863,8 @@ int bind_sdpa_lanes(ksh_kernel &k, int nwg, int n_slots)
     k.info.sched.lds_tile = 0;
     k.info.sched.unroll = (uint32_t)hsplit;
     k.variant = nwg | (nw << 16) | (hsplit << 24);
-    k.launch = launch_bound;
+    k.launch = launch_bound<>;
+    if (k.desc.kind == KSH_SDPA_MWG_PART) k.launch_half = launch_bound<true>;
     return 0;
 }
 
