@@ -47,10 +47,30 @@ __device__ uint32_t f32_to_f16_ref(float value)
     return sign | (half_exp << 10) | (half_mant >> 13);
 }
 
+// The codes clamp(nearest_int(iscale * (x - mn)), 0, 15) of a sub-block, as floats.  Where every product is known to stay
+// below 2^22 in magnitude, the magic addition rounds and subtracting the constant again leaves the rounded value itself:
+// two additions and a median instead of the integer detour (mask, subtract, clamp, convert).  `lo` and `hi` bound x.
+__device__ __forceinline__ void grid_codes(const float (&x)[32], float iscale, float mn, float lo, float hi, float (&lf)[32])
+{
+    constexpr float magic = 12582912.0f;
+    const float reach = fabsf(iscale) * fmaxf(fabsf(lo - mn), fabsf(hi - mn));
+    if (reach < 4000000.0f) {
+#pragma unroll
+        for (int i = 0; i < 32; i++) lf[i] = __builtin_amdgcn_fmed3f((iscale * (x[i] - mn) + magic) - magic, 0.0f, 15.0f);
+    } else {
+        // (also where the reach is not a number: the host routine's integers, whatever they are)
+#pragma unroll
+        for (int i = 0; i < 32; i++) lf[i] = (float)clampi(nearest_int(iscale * (x[i] - mn)), 0, 15);
+    }
+}
+
 // gguf_impl.rs:811-901 with nmax=15, rmin=-1, rdelta=0.1, nstep=20, squared error.  One thread runs one 32-element
 // sub-block with every array in registers (the loops over the elements are unrolled; the sums run in the host
-// routine's order, element after element, so every rounding is the host's).  L: the 32 codes, one per byte.
-__device__ __forceinline__ float make_qkx2_quants(const float (&x)[32], const float (&weights)[32], uint32_t (&L)[8], float *the_min)
+// routine's order, element after element, so every rounding is the host's).
+// Bound: the vector ALU -- 22 passes over the elements, 11 instructions an element for a candidate's codes and sums and 6
+// for its error (24 with integer codes packed and unpacked between the two: 200 us for 16.8M weights, 130 so).
+// The codes of the chosen candidate are not kept: *code_iscale and *code_min name the grid that makes them again (*flat: all 0).
+__device__ __forceinline__ float make_qkx2_quants(const float (&x)[32], const float (&weights)[32], float *the_min, float *code_iscale, float *code_min, bool *flat)
 {
     constexpr int n = 32, nmax = 15, nstep = 20;
     const float rmin = -1.0f, rdelta = 0.1f;
@@ -63,23 +83,25 @@ __device__ __forceinline__ float make_qkx2_quants(const float (&x)[32], const fl
         sum_w += w;
         sum_x += w * x[i];
     }
+    const float lo = mn;
     if (mn > 0.0f) mn = 0.0f;
+    *flat = mx == mn;
     if (mx == mn) {
-#pragma unroll
-        for (int i = 0; i < 8; i++) L[i] = 0;
+        *code_iscale = 0.0f;
+        *code_min = mn;
         *the_min = -mn;
         return 0.0f;
     }
     float iscale = (float)nmax / (mx - mn);
     float scale = 1.0f / iscale;
     float best_error = 0.0f;
-#pragma unroll
-    for (int i = 0; i < 8; i++) L[i] = 0;
+    *code_iscale = iscale;
+    *code_min = mn;
+    float lf[32];
+    grid_codes(x, iscale, mn, lo, mx, lf);
 #pragma unroll
     for (int i = 0; i < n; i++) {
-        const int l = clampi(nearest_int(iscale * (x[i] - mn)), 0, nmax);
-        L[i >> 2] |= (uint32_t)l << (8 * (i & 3));
-        float diff = scale * (float)l + mn - x[i];
+        float diff = scale * lf[i] + mn - x[i];
         diff = diff * diff;
         best_error += weights[i] * diff;
     }
@@ -87,17 +109,13 @@ __device__ __forceinline__ float make_qkx2_quants(const float (&x)[32], const fl
     for (int is = 0; is <= nstep; is++) {
         iscale = (rmin + rdelta * (float)is + (float)nmax) / (mx - mn);
         float sum_l = 0.0f, sum_l2 = 0.0f, sum_xl = 0.0f;
-        uint32_t Laux[8];
-#pragma unroll
-        for (int i = 0; i < 8; i++) Laux[i] = 0;
+        grid_codes(x, iscale, mn, lo, mx, lf);
 #pragma unroll
         for (int i = 0; i < n; i++) {
-            const int l = clampi(nearest_int(iscale * (x[i] - mn)), 0, nmax);
-            Laux[i >> 2] |= (uint32_t)l << (8 * (i & 3));
-            const float w = weights[i], lf = (float)l;
-            sum_l += w * lf;
-            sum_l2 += w * lf * lf;
-            sum_xl += w * lf * x[i];
+            const float wl = weights[i] * lf[i];
+            sum_l += wl;
+            sum_l2 += wl * lf[i];
+            sum_xl += wl * x[i];
         }
         const float D = sum_w * sum_l2 - sum_l * sum_l;
         if (D > 0.0f) {
@@ -110,13 +128,13 @@ __device__ __forceinline__ float make_qkx2_quants(const float (&x)[32], const fl
             float cur_error = 0.0f;
 #pragma unroll
             for (int i = 0; i < n; i++) {
-                float diff = this_scale * (float)((Laux[i >> 2] >> (8 * (i & 3))) & 0xFFu) + this_min - x[i];
+                float diff = this_scale * lf[i] + this_min - x[i];
                 diff = diff * diff;
                 cur_error += weights[i] * diff;
             }
             if (cur_error < best_error) {
-#pragma unroll
-                for (int i = 0; i < 8; i++) L[i] = Laux[i];
+                *code_iscale = iscale;
+                *code_min = mn;
                 best_error = cur_error;
                 scale = this_scale;
                 mn = this_min;
@@ -155,8 +173,9 @@ __global__ __launch_bounds__(64) void quantize_q4k_kernel(const float *__restric
 #pragma unroll
     for (int i = 0; i < 32; i++) weights[i] = av_x + fabsf(x[i]);
     uint32_t L[8];
-    float mymin;
-    const float myscale = make_qkx2_quants(x, weights, L, &mymin);
+    float mymin, code_iscale, code_min;
+    bool flat;
+    const float myscale = make_qkx2_quants(x, weights, &mymin, &code_iscale, &code_min, &flat);
     float max_scale = 0.0f, max_min = 0.0f;
 #pragma unroll
     for (int k = 0; k < 8; k++) {
@@ -173,10 +192,14 @@ __global__ __launch_bounds__(64) void quantize_q4k_kernel(const float *__restric
     // the sub-block's final codes against the scale and minimum as they will be unpacked (get_scale_min_k4 returns ls, lm)
     const float d = half_bits_to_f32(db), dmin = half_bits_to_f32(mb);
     const float dj = d * (float)ls;
-    if (dj != 0.0f) {
-        const float dm = dmin * (float)lm;
 #pragma unroll
-        for (int i = 0; i < 8; i++) L[i] = 0;
+    for (int i = 0; i < 8; i++) L[i] = 0;
+    if (dj == 0.0f) {
+        // the scale came out as zero: the search's own codes stay
+#pragma unroll
+        for (int i = 0; i < 32; i++) L[i >> 2] |= (flat ? 0u : (uint32_t)clampi(nearest_int(code_iscale * (x[i] - code_min)), 0, 15)) << (8 * (i & 3));
+    } else {
+        const float dm = dmin * (float)lm;
 #pragma unroll
         for (int i = 0; i < 32; i++) L[i >> 2] |= (uint32_t)clampi(nearest_int((x[i] + dm) / dj), 0, 15) << (8 * (i & 3));
     }

@@ -42,6 +42,20 @@ def test_quantize_q4k_matches_host_routine_bytes(ctx, eng):
     assert np.all(back[256:512] == 0.0) and np.abs(back[:1024] - sig).max() < 0.35
 
 
+@pytest.mark.parametrize("shift,std,outlier", [(-5.0, 1.0, 0), (-1.0, 1e-7, 0), (3.0, 1e-3, 0), (0.0, 1e-30, 0), (0.0, 1e18, 0), (0.0, 0.02, 40.0),
+                                               (-0.5, 1e-6, 1e6), (0.0, 1e-40, 0)])
+def test_quantize_q4k_edges_of_the_scale_search(ctx, eng, shift, std, outlier):
+    """Blocks where a candidate's grid leaves the range in which codes are rounded as floats (nearly constant values, one
+    outlier), values of one sign, and scales that round to zero: the host routine's bytes."""
+    x = shift + synth.normal_f32(256 * 40, 404) * np.float32(std)
+    if outlier:
+        x[7::97] *= np.float32(outlier)
+    x = x.astype(np.float32)
+    dst = ctx.buffer_empty_bytes(x.size // 256 * 144)
+    eng.quantize_k(ctx, DType.Q4K, x.size, ctx.buffer_f32(x), dst)
+    assert np.array_equal(ctx.read_bytes(dst, x.size // 256 * 144), oracle.quantize_q4k(x))
+
+
 def test_quantize_q6k_matches_host_routine_bytes(ctx, eng):
     x = np.concatenate([synth.normal_f32(256 * 200, 402, std=0.02), np.zeros(256, np.float32),
                         synth.normal_f32(256 * 10, 403, std=5.0)])

@@ -244,3 +244,31 @@ def test_half_boundary_sizes_and_refusals(ctx):
     # the prompt pass's own forms of the GEMM (producers inside the preparation) take f32 rows only
     with pytest.raises(hip.KshError):
         ctx.compile(hip.make_desc(Kind.MATVEC_BATCH, (256, 2048, 32, 0, 0, 1), (DType.Q4K, DType.F16), (1e-6,)))
+
+
+@pytest.mark.parametrize("n,res,scale,rows", [(96, 0, 0, 1), (512, 1, 1, 3), (513, 1, 0, 2), (2048, 0, 0, 1), (2050, 1, 1, 2), (6144, 1, 0, 1),
+                                              (6400, 1, 1, 2)])
+def test_rmsnorm_half_every_row_length(ctx, n, res, scale, rows):
+    """The instances by row length (2, 8 and 24 elements per thread, rows read twice), rows that do not divide among the
+    threads."""
+    x, r = halfed(synth.normal_f32(n * rows, 770)), halfed(synth.normal_f32(n * rows, 771))
+    w, eps = halfed(1.0 + 0.1 * synth.normal_f32(n, 772)), 1e-6
+    (y,) = both(ctx, Kind.RMSNORM, (n, res, scale, rows), (), (eps, 0.5), [(x, "A"), (w, "A")] + ([(r, "A")] if res else []), [(n * rows, "A")])
+    for i in range(rows):
+        s = slice(i * n, (i + 1) * n)
+        want = oracle.rmsnorm(x[s], w, eps, res=r[s] if res else None, **({"scale": 0.5} if scale else {}))
+        assert rel_err(y[s], want.astype(np.float16).astype(np.float32)).max() <= BAR
+
+
+@pytest.mark.parametrize("n_q,n_kv,hd,nwg,tlen", [(8, 1, 256, 16, 700), (8, 1, 512, 5, 301), (4, 2, 128, 9, 77), (2, 2, 256, 1, 30)])
+def test_split_kv_partials_and_merge_half(ctx, n_q, n_kv, hd, nwg, tlen):
+    """Half q into split-KV partials (one head per workgroup at heads of 256 and 512), half result of the merge; partition
+    counts around the merge's eight at a time."""
+    max_t, scale = 768, 1.0 / np.sqrt(hd)
+    kk, vv = synth.q40_blocks(max_t * n_kv * hd // 32, 780), synth.q40_blocks(max_t * n_kv * hd // 32, 781)
+    q, meta = halfed(synth.normal_f32(n_q * hd, 782)), np.array([tlen, 3, 0, 0], np.float32)
+    (tmp,) = both(ctx, Kind.SDPA_MWG_PART, (n_q, n_kv, hd, max_t, nwg), (DType.Q40,), (scale,),
+                  [(q, "A"), (kk, "W"), (vv, "W"), (meta, "F")], [(n_q * nwg * (hd + 2), "F")])
+    (o,) = both(ctx, Kind.SDPA_MWG_REDUCE, (n_q, hd, nwg), (), (), [(tmp, "F")], [(n_q * hd, "A")])
+    want = oracle.sdpa(q, kk, vv, n_q, n_kv, hd, tlen, 3, scale).astype(np.float16).astype(np.float32)
+    assert rel_err(o, want).max() <= BAR
