@@ -989,6 +989,13 @@ __device__ __forceinline__ int mfma_k_elem(int s, int kq)
     return 4 * kq + byte + ((s >> 1) & 1) * 16;      //    nibble: lo lo hi hi lo lo hi hi
 }
 
+// Bytes from one K row of a tile to the next in LDS.  A row of 512 is 288 bytes, and sixteen lanes reading the same place
+// of sixteen rows met in eight of the 64 banks; 16 bytes of padding put them in sixteen
+// (952 prompt tokens behind 2048: 875 -> 833 us).  Rows of 256
+// (144 bytes) are spread as they are.
+template <int HD>
+constexpr int mfma_k_pitch() { return HD / 32 * 18 + (HD == 512 ? 16 : 0); }
+
 // HDV < HD (heads of 512 as two halves of 256): the workgroups of blockIdx.y = 2 * kvh + half both work out the scores
 // and the softmax over all HD dimensions (the same numbers twice) and each takes P.V for its HDV dimensions of V,
 // whose accumulators are what limits the head size a wave can hold.
@@ -1009,7 +1016,8 @@ __global__ __launch_bounds__(kMfmaRound / TR * 64, TR == 32 ? 2 : 1) void sdpa_m
     static_assert(HD % HDV == 0 && (HDV == HD || TR == 32), "V halves come with tiles of 32 rows");
     touch_lane_params(p_in);   // every kernel argument in one round trip
     KSH_STAMP_BEGIN
-    constexpr int NW = kMfmaRound / TR, NT = NW * 64, NB = HD / 32, ROWB = NB * 18, TILEB = TR * ROWB;
+    constexpr int NW = kMfmaRound / TR, NT = NW * 64, NB = HD / 32, ROWB = NB * 18, TILEB = TR * mfma_k_pitch<HD>();
+    constexpr int KPITCH = mfma_k_pitch<HD>();                             // bytes from one K row of the tile to the next in LDS
     constexpr int NBV = HDV / 32, ROWBV = NBV * 18, TILEBV = TR * ROWBV;   // this workgroup's share of a V row
     constexpr int STRIP = TILEB + TILEBV + TR * NB * 4 + TR * NBV * 4;     // K bytes, V bytes, K scales, V scales
     constexpr int PIECES = TR * ROWB / 16, PIECESV = TR * ROWBV / 16;      // 128-bit pieces of a tile
@@ -1019,8 +1027,10 @@ __global__ __launch_bounds__(kMfmaRound / TR * 64, TR == 32 ? 2 : 1) void sdpa_m
     const uint32_t odd_mask = 0u - (uint32_t)(q4 & 1);     // all ones in the lane groups whose accumulator rows are heads 4..7
     uint32_t nib_mask = 0x03C003C0u, nib_one = 0x4C004C00u;  // a nibble's place in an f16 mantissa; 16.0 twice
     asm volatile("" : "+v"(nib_mask), "+v"(nib_one));
-    // the two parts of x = p * dv: hi lanes keep x cut to 11 bits, lo lanes what the cut left over
-    const uint32_t keep = is_lo ? 0xFFFFFFFFu : 0xFFFFE000u, drop = is_lo ? 0xFFFFE000u : 0u;
+    // the two parts of x = p * dv: hi lanes x cut to 11 bits, which the conversion (towards zero) does by itself, lo lanes
+    // what the cut left over: x less nothing, or less its upper bits (two operations per value where a select took three:
+    // the same launch 833 -> 825 us)
+    const uint32_t drop = is_lo ? 0xFFFFE000u : 0u;
     uint8_t *strip = lds_raw + (size_t)wave * STRIP;
     uint8_t *kraw = strip, *vraw = strip + TILEB;
     float *ksc = reinterpret_cast<float *>(strip + TILEB + TILEBV), *vsc = ksc + TR * NB;
@@ -1166,7 +1176,7 @@ __global__ __launch_bounds__(kMfmaRound / TR * 64, TR == 32 ? 2 : 1) void sdpa_m
         for (int u = 0; u < NPC; u++) {
             const int idx = lane + 64 * u;
             if (idx < PIECES) {
-                *reinterpret_cast<u32x4_t *>(kraw + idx * 16) = kpre[u];
+                *reinterpret_cast<u32x4_t *>(kraw + (idx / (ROWB / 16)) * KPITCH + (idx % (ROWB / 16)) * 16) = kpre[u];
                 if (HDV == HD) *reinterpret_cast<u32x4_t *>(vraw + idx * 16) = vpre[u];
             }
         }
@@ -1182,7 +1192,7 @@ __global__ __launch_bounds__(kMfmaRound / TR * 64, TR == 32 ? 2 : 1) void sdpa_m
 #pragma unroll
         for (int u = 0; u < TR * NB / 64; u++) {
             const int idx = lane + 64 * u, b = idx / TR, row = idx % TR;      // tables are [block][row]
-            const uint32_t kb = *reinterpret_cast<const uint16_t *>(kraw + row * ROWB + 18 * b);
+            const uint32_t kb = *reinterpret_cast<const uint16_t *>(kraw + row * KPITCH + 18 * b);
             ksc[idx] = row < nvalid ? half_bits_to_f32(kb) : 0.f;
             if (HDV == HD) {
                 const uint32_t vb = *reinterpret_cast<const uint16_t *>(vraw + row * ROWBV + 18 * b);
@@ -1208,7 +1218,7 @@ __global__ __launch_bounds__(kMfmaRound / TR * 64, TR == 32 ? 2 : 1) void sdpa_m
                 for (int b = 0; b < NB; b++) {
                     const float4 dk4 = *reinterpret_cast<const float4 *>(ksc + b * TR + 4 * q4);
                     const float dk[4] = {dk4.x, dk4.y, dk4.z, dk4.w};
-                    const uint8_t *src = kraw + col * ROWB + 18 * b + 2 + 4 * q4;
+                    const uint8_t *src = kraw + col * KPITCH + 18 * b + 2 + 4 * q4;
                     const uint32_t d = (uint32_t)*reinterpret_cast<const uint16_t *>(src) |
                                        ((uint32_t)*reinterpret_cast<const uint16_t *>(src + 2) << 16);
                     const f4v c = __builtin_amdgcn_mfma_f32_16x16x32_f16(nibbles_f16(d, nib_mask, nib_one), qop[b], f4v{0.f, 0.f, 0.f, 0.f}, 0, 0, 0);
@@ -1275,8 +1285,7 @@ __global__ __launch_bounds__(kMfmaRound / TR * 64, TR == 32 ? 2 : 1) void sdpa_m
                 uint32_t pa[2], vlo[2], vhi[2];
 #pragma unroll
                 for (int i = 0; i < 2; i++) {
-                    const float y0 = as_f32(as_u32(x[2 * i]) & keep) - as_f32(as_u32(x[2 * i]) & drop);
-                    const float y1 = as_f32(as_u32(x[2 * i + 1]) & keep) - as_f32(as_u32(x[2 * i + 1]) & drop);
+                    const float y0 = x[2 * i] - as_f32(as_u32(x[2 * i]) & drop), y1 = x[2 * i + 1] - as_f32(as_u32(x[2 * i + 1]) & drop);
                     pa[i] = __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_pkrtz(y0, y1));
                     tsum += x[2 * i] + x[2 * i + 1];
                     const int ra = 4 * q4 + 2 * i;
@@ -1305,7 +1314,7 @@ __global__ __launch_bounds__(kMfmaRound / TR * 64, TR == 32 ? 2 : 1) void sdpa_m
                     const float4 dk4 = *reinterpret_cast<const float4 *>(ksc + b * TR + 16 * t + 4 * q4);   // rows 4*q4 .. +3
                     const float dk[4] = {dk4.x, dk4.y, dk4.z, dk4.w};
                     // A operand: row (16t + lane % 16), bytes 4*q4 .. 4*q4+3 of block b (2-byte aligned)
-                    const uint8_t *src = kraw + (16 * t + col) * ROWB + 18 * b + 2 + 4 * q4;
+                    const uint8_t *src = kraw + (16 * t + col) * KPITCH + 18 * b + 2 + 4 * q4;
                     const uint32_t d = (uint32_t)*reinterpret_cast<const uint16_t *>(src) |
                                        ((uint32_t)*reinterpret_cast<const uint16_t *>(src + 2) << 16);
                     const f4v c = __builtin_amdgcn_mfma_f32_16x16x32_f16(nibbles_f16(d, nib_mask, nib_one), qop[b], f4v{0.f, 0.f, 0.f, 0.f}, 0, 0, 0);
@@ -1370,8 +1379,7 @@ __global__ __launch_bounds__(kMfmaRound / TR * 64, TR == 32 ? 2 : 1) void sdpa_m
                 for (int i = 0; i < NS; i += 2) {
                     // (the conversion is exact for the hi part and cuts the lo part to 11 of its 13 bits)
                     const float x0 = pr[i] * dv[i], x1 = pr[i + 1] * dv[i + 1];
-                    const float y0 = as_f32(as_u32(x0) & keep) - as_f32(as_u32(x0) & drop);
-                    const float y1 = as_f32(as_u32(x1) & keep) - as_f32(as_u32(x1) & drop);
+                    const float y0 = x0 - as_f32(as_u32(x0) & drop), y1 = x1 - as_f32(as_u32(x1) & drop);
                     pa[i / 2] = __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_pkrtz(y0, y1));
                     tsum += x0 + x1;
                 }
@@ -1524,7 +1532,7 @@ template <int HD, int TR, int HDV = HD, bool PVX = false>
 constexpr size_t mfma_lds_bytes()
 {
     constexpr size_t waves = kMfmaRound / TR;
-    constexpr size_t strip = (size_t)TR * (HD / 32 * 18) + (size_t)TR * (HDV / 32 * 18) + (size_t)TR * (HD / 32) * 4 + (size_t)TR * (HDV / 32) * 4;
+    constexpr size_t strip = (size_t)TR * mfma_k_pitch<HD>() + (size_t)TR * (HDV / 32 * 18) + (size_t)TR * (HD / 32) * 4 + (size_t)TR * (HDV / 32) * 4;
     constexpr size_t qshare = (size_t)(HD / 32) * 64 * (16 + 4);                 // the shared q operands and sums
     constexpr size_t fold = waves * 8 * HDV * 4 + waves * 8 * 2 * 4;
     constexpr size_t qsum = (size_t)(HD / 32) * 64 * 4;
