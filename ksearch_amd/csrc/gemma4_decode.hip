@@ -458,8 +458,8 @@ int write_token(ksh_gemma4 *m, uint32_t token)
 }
 
 // gemma_prim.rs:33-56: per position cos[0..hd/2) || sin[0..hd/2); pairs past `angles` are the identity
-// prefill_chunk's chunk length (gemma_prim.rs:16)
-constexpr int kChunk4 = 1024;
+// (a prompt's passes: prefill_pass_tokens)
+constexpr int kChunk4 = kPrefillPass;
 constexpr int kChunkPartitions4 = 8;
 constexpr int kPartsRows4 = 4;      // room for the unfolded partial sums of a hidden-wide projection: this many chunks of rows
 
@@ -1023,7 +1023,7 @@ int ksh_gemma4_decode_token_sampled(ksh_gemma4 *m, uint32_t token, float tempera
 }
 
 // GemmaPrimModel::prefill_chunk (gemma_prim.rs:1305-1315): the tokens go through without logits, then one
-// synchronisation.  Chunks of up to 256 tokens go through the batched layer pass (forward_prefill_chunk,
+// synchronisation.  Chunks of up to 2048 tokens go through the batched layer pass (forward_prefill_chunk,
 // gemma_prim.rs:1317-1607), a chunk of one token through the decode step; use_graph & 2 feeds every token through
 // the decode step instead (use_graph & 1: from its captured graph).
 int ksh_gemma4_prefill_chunk(ksh_gemma4 *m, const uint32_t *tokens, int n, int use_graph)
@@ -1033,7 +1033,7 @@ int ksh_gemma4_prefill_chunk(ksh_gemma4 *m, const uint32_t *tokens, int n, int u
     for (int i = 0; i < n; i++)
         if (tokens[i] >= (uint32_t)m->c.vocab) return set_error("token id %u is outside the vocabulary", tokens[i]);
     for (int i = 0; i < n;) {
-        const int t = (use_graph & 2) ? 1 : std::min(kChunk4, n - i);
+        const int t = (use_graph & 2) ? 1 : prefill_pass_tokens(n - i);
         if (t == 1) {
             if (write_token(m, tokens[i])) return 1;
             if (run_token(m, false, (use_graph & 1) != 0)) return 1;

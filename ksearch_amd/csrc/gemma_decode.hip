@@ -358,8 +358,9 @@ bool span_fits(const ksh_gemma *m, int remaining)
     return (m->pos < m->short_context) == (m->pos + kSpan - 1 < m->short_context);
 }
 
-// prefill_chunk's chunk length (gemma_prim.rs:16)
-constexpr int kChunk = 1024;
+// A prompt goes through in passes of kChunk tokens while it has as many, then of half that, then the rest
+// (prefill_pass_tokens)
+constexpr int kChunk = kPrefillPass;
 constexpr int kPartsRows = 4;          // room for the unfolded partial sums of a hidden-wide projection: this many chunks of rows
 constexpr int kChunkPartitions = 8;   // partitions per token of the batched attention (its tmp buffer is sized for this)
 
@@ -685,8 +686,8 @@ int ksh_gemma_prefill_chunk(ksh_gemma *m, const uint32_t *tokens, int n)
     for (int i = 0; i < n; i++)
         if (tokens[i] >= (uint32_t)m->c.vocab) return set_error("token id %u is outside the vocabulary", tokens[i]);
     // gemma_prim.rs:1305-1315: chunks of PREFILL_CHUNK, a remainder of one token through the decode step
-    for (int i = 0; i < n; i += kChunk) {
-        const int t = std::min(kChunk, n - i);
+    for (int i = 0, t = 0; i < n; i += t) {
+        t = prefill_pass_tokens(n - i);
         if (t == 1) {
             if (write_token(m, tokens[i]) || run_token(m, false, false)) return 1;
         } else if (forward_prefill_chunk(m, tokens + i, t)) {

@@ -24,6 +24,16 @@ int hip_fail(hipError_t e, const char *what);
         if (_e != hipSuccess) return ::ksh::hip_fail(_e, #expr); \
     } while (0)
 
+// Tokens of one pass of a prompt through the layers (the reference's chunk length counts in the hundreds,
+// gemma_prim.rs:16): 2048 while the prompt has as many left, then 1024, then the rest.  At 1024 rows a hidden-wide
+// projection is 192 workgroups (1536 x 12288) and a quarter of the compute units has none; at 2048 a second workgroup
+// shares half of them (3000 prompt tokens of the checkpoints' layout: 66.0 -> 61.4 ms).
+constexpr int kPrefillPass = 2048;
+inline int prefill_pass_tokens(int left)
+{
+    return left >= kPrefillPass ? kPrefillPass : left >= kPrefillPass / 2 ? kPrefillPass / 2 : left;
+}
+
 constexpr int kMaxIn = 8;
 constexpr int kMaxOut = 4;
 

@@ -1426,12 +1426,12 @@ constexpr int kSkinnyMaxBatch = 64;
 // (bf16, cfg2: 33.7 us against 40.3 with 64-token tiles; f32, prompts of 256 / 1024 / 4000 tokens through cfg4's
 // model: 5.05 / 14.1 / 67.7 ms with this rule, 5.07 / 14.25 / 68.0 with 64-token tiles throughout, 5.3 / 14.9 / 72.7
 // with 128-token tiles from 65 tokens on).
-int mm_tile_tokens(const ksh_kernel_desc &d, int64_t ks)
+int mm_tile_tokens(const ksh_kernel_desc &d, int64_t batch, int64_t ks)
 {
     if (d.dtypes[0] == KSH_Q6K) return 128;
     const int64_t row_tiles = (d.dims[0] + BN - 1) / BN + (d.dims[3] + BN - 1) / BN + (d.dims[4] + BN - 1) / BN;
     const int64_t fill = d.dtypes[1] == KSH_F32 ? 512 : 256;
-    return d.dims[2] <= 64 || ((d.dims[2] + BM - 1) / BM) * row_tiles * ks < fill ? 64 : 128;
+    return batch <= 64 || ((batch + BM - 1) / BM) * row_tiles * ks < fill ? 64 : 128;
 }
 
 int launch_mul_mm(const ksh_kernel &k, const LaunchArgs &a, hipStream_t st)
@@ -1488,7 +1488,7 @@ int launch_mul_mm(const ksh_kernel &k, const LaunchArgs &a, hipStream_t st)
         const hipError_t e2 = hipGetLastError();
         return e2 == hipSuccess ? 0 : hip_fail(e2, "mul_mm (small batch) launch");
     }
-    const int tm = mm_tile_tokens(k.desc, k.variant >= 2 ? k.variant >> 1 : 1);
+    const int tm = mm_tile_tokens(k.desc, batch, k.variant >= 2 ? k.variant >> 1 : 1);
     const dim3 grid((batch + tm - 1) / tm, (rows + BN - 1) / BN + (rows1 + BN - 1) / BN + (rows2 + BN - 1) / BN);
     p.Xf = Xf; p.SxA = SxA; p.Xf_lo = Xf_lo; p.inv_s = inv_s;
     p.ksplit = 0; p.Y_parts = nullptr;
@@ -1606,8 +1606,11 @@ int bind_matvec_batch(ksh_kernel &k)
         ks = k.desc.sched.k_split;
         if (nsb % ks) return set_error("matvec_batch: k_split=%lld does not divide the %lld superblocks of a row", (long long)ks, (long long)nsb);
     } else {
-        // (a slice of one superblock is all prologue; the workgroups are counted with the token tile they will have)
-        auto workgroups = [&](int64_t s) { const int64_t tm_s = mm_tile_tokens(k.desc, s); return ((batch + tm_s - 1) / tm_s) * row_tiles * s; };
+        // (a slice of one superblock is all prologue; the workgroups are counted with the token tile they will have, and
+        // f32 rows of more than half a prompt pass as that many: how a row's sum is cut does not depend on which pass of its
+        // prompt the row is in)
+        const int64_t counted = f32x ? std::min<int64_t>(batch, kPrefillPass / 2) : batch;
+        auto workgroups = [&](int64_t s) { const int64_t tm_s = mm_tile_tokens(k.desc, counted, s); return ((counted + tm_s - 1) / tm_s) * row_tiles * s; };
         while (nsb % (ks * 2) == 0 && nsb / (ks * 2) >= 2 && workgroups(ks * 2) <= 256) ks *= 2;
     }
     const bool z_form = unfolded || ks > 1;
@@ -1619,7 +1622,7 @@ int bind_matvec_batch(ksh_kernel &k)
         k.out_bytes[0] = (size_t)ks * batch * rows_all * 4; k.out_align[0] = 16;
         k.info.n_outputs = 1 + keep;
     }
-    const int tm = mm_tile_tokens(k.desc, ks);
+    const int tm = mm_tile_tokens(k.desc, batch, ks);
     set_launch(k, (uint32_t)((batch + tm - 1) / tm), (uint32_t)row_tiles, z_form ? (uint32_t)ks : 1, kThreadsMM,
                (uint32_t)(tm == 64 ? kLdsBytes64 : kLdsBytes));
     k.info.sched.tg = kThreadsMM; k.info.sched.nsg = kThreadsMM / 64; k.info.sched.nr0 = BN; k.info.sched.k_split = (uint32_t)ks; k.info.sched.lds_tile = KS;

@@ -228,7 +228,7 @@ int bind_ple_ops(ksh_kernel &k)
     switch (k.desc.kind) {
     case KSH_RMSNORM_PER_HEAD: {
         const int64_t n_heads = d[0], hd = d[1], mode = d[2], max_seq = d[3];
-        if (n_heads <= 0 || n_heads > 65535) return set_error("rmsnorm_per_head: n_heads=%lld", (long long)n_heads);
+        if (n_heads <= 0 || n_heads > (1 << 20)) return set_error("rmsnorm_per_head: n_heads=%lld", (long long)n_heads);
         if (hd != 64 && hd != 128 && hd != 256 && hd != 512)
             return set_error("rmsnorm_per_head: hd=%lld is not built (64, 128, 256, 512 are)", (long long)hd);
         if (mode < 0 || mode > 2) return set_error("rmsnorm_per_head: dims[2]=%lld (0 norm only, 1 rope row, 2 rope table + meta)", (long long)mode);

@@ -244,6 +244,31 @@ def test_prefill_long_prompt_takes_two_chunks(ctx):
     cpu.close()
 
 
+@pytest.mark.parametrize("n_prompt", [2048, 3074])
+def test_prefill_passes_of_2048_are_those_of_1024(ctx, n_prompt):
+    """A pass of 2048 tokens cuts every row's sums as passes of 1024 do (K slices included: the k | v and o projections of
+    this shape have them): the caches are the same bytes as after calls of 1024."""
+    cfg = dict(n_layers=2, hidden=512, ffn=2048, n_q=4, n_kv=1, hd=256, vocab=4096, max_seq=3200,
+               eps=1e-6, softcap=30.0, rope_theta=10000.0, attn_scale=1.0 / 16.0)
+    w = synth.gemma_weights(cfg, 762, oracle.quantize_q4k, synth.chunked(oracle.quantize_q6k), std=0.05)
+    gpu = hip.Gemma(ctx, cfg, w)
+    toks = np.random.default_rng(763).integers(0, cfg["vocab"], n_prompt)
+    row = cfg["hd"] // 32 * 18
+
+    def caches():
+        return [ctx.read_bytes(hip.Buffer(ctx, hip.lib().ksh_gemma_kv(gpu.h, l, w_), owned=False), row * n_prompt, 0)
+                for l in range(cfg["n_layers"]) for w_ in (0, 1)]
+
+    gpu.prefill_chunk(toks)
+    whole = caches()
+    gpu.reset()
+    for i in range(0, n_prompt, 1024):
+        gpu.prefill_chunk(toks[i:i + 1024])
+    for a, b in zip(whole, caches()):
+        assert np.array_equal(a, b)
+    gpu.close()
+
+
 def test_prefill_in_two_calls_and_serial_prefill_agree(ctx, small_model):
     """A prompt fed as 40 + 1 + 23 tokens (a single token goes through the decode step) leaves the same cache as one
     call, and generate() gives the same continuation with batched and with token-by-token prefill unless a Q4_0 flip
