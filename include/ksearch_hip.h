@@ -81,6 +81,8 @@ enum ksh_kind {
      * dims[6] = 1: the tile's K slices stay unfolded -- out[0] is then f32[slices][batch][rows + rows1 + rows2]
      *   (slices = info.grid[2] = info.sched.k_split, the matrices' columns side by side) for a reader that adds them
      *   itself; out[1] = x_new with prologue 2.
+     * dims[6] = 2 (F32 activations): the rows are several prompts', each summed as in a launch of its own -- one more
+     *   input, the last, f32[batch]: the tokens of that launch (more than 64), whose K slices the row's sums are cut into.
      * dims[7] = the slices (info.grid[2]) of the GEMM whose unfolded result this one's X is (with a prologue;
      *   prologue 3 then reads gate | up from that one buffer and takes no `up` operand).  The sums are added in the
      *   fold's order, so a chain of GEMMs gives the same numbers with and without its folds.
@@ -237,7 +239,10 @@ enum ksh_kind {
      * 0, -, window}: token i attends tlen_i = min(tlen0 + i, window) rows from start_i = tlen0 + i - tlen_i.
      * dims: n_q, n_kv, hd, max_t, n_tok, nwg (0 = default; sched.k_split sets it too).  Heads of 256 in chunks of
      * more than 16 tokens run on the matrix cores and are fastest with one partition per token (nwg = 1).
-     * in: q[n_tok, n_q*hd], K, V, meta   out: tmp f32[n_tok*n_q*nwg*(hd+2)], o[n_tok, n_q*hd] */
+     * in: q[n_tok, n_q*hd], K, V, meta   out: tmp f32[n_tok*n_q*nwg*(hd+2)], o[n_tok, n_q*hd]
+     * dims[6] = slots in the K / V pools, dims[7] = bytes from one slot to the next (as KSH_SDPA_SLOTS): the tokens
+     * belong to several prompts; meta is then f32[n_tok][4] (token i attends meta[4 i] rows from meta[4 i + 1] on) and a
+     * 5th input f32[n_tok] names each token's slot (more than 16 tokens, heads of 256 or 512) */
     KSH_SDPA_BATCH = 29,
     /* The activations of a decode round (up to 16 rows, one per decoding sequence), prepared once for every GEMM
      * that reads them.  No counterpart in the reference, whose round is one decode step per request

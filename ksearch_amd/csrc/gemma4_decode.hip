@@ -137,7 +137,8 @@ struct ksh_gemma4 {
     ksh_buf *c_tok = nullptr, *c_x = nullptr, *c_x2 = nullptr, *c_y = nullptr, *c_q = nullptr, *c_k = nullptr, *c_v = nullptr, *c_o = nullptr,
             *c_g = nullptr, *c_u = nullptr, *c_ff = nullptr, *c_tmp = nullptr, *c_meta_full = nullptr, *c_meta_swa = nullptr,
             *c_po = nullptr, *c_pg = nullptr,   // unfolded partial sums of the o and the gate | up projection of a chunk
-            *c_ple_tok = nullptr, *c_ple_tmp = nullptr, *c_ple_ctx = nullptr, *c_ple_u = nullptr;
+            *c_ple_tok = nullptr, *c_ple_tmp = nullptr, *c_ple_ctx = nullptr, *c_ple_u = nullptr,
+            *c_tab = nullptr;                   // a pass over several slots: ids, slots, attended ranges per token
     // decode rounds over several KV slots (allocated at the first round): the per-token table (ids, slots, attended
     // ranges of the two layer kinds), the logits of every token of the round, the greedy ids
     ksh_buf *r_tab = nullptr, *r_logits = nullptr, *r_next = nullptr, *r_xp = nullptr, *r_xp2 = nullptr;   // (r_xp, r_xp2: a round's prepared GEMM operands)
@@ -461,6 +462,7 @@ int write_token(ksh_gemma4 *m, uint32_t token)
 // (a prompt's passes: prefill_pass_tokens)
 constexpr int kChunk4 = kPrefillPass;
 constexpr int kChunkPartitions4 = 8;
+constexpr int kSmallPass = 64;      // tokens up to which a GEMM of one matrix takes the small-batch form
 constexpr int kPartsRows4 = 4;      // room for the unfolded partial sums of a hidden-wide projection: this many chunks of rows
 
 int chunk_buffers4(ksh_gemma4 *m)
@@ -471,7 +473,7 @@ int chunk_buffers4(ksh_gemma4 *m)
     size_t max_ff = 0;
     for (const ksh_gemma4_layer &L : m->layers) max_ff = std::max(max_ff, (size_t)L.ffn);
     const size_t pt = (size_t)c.n_layers * c.ple_dim;
-    if (alloc(m, T * 4, &m->c_tok) || alloc(m, T * c.hidden * 4, &m->c_x) || alloc(m, T * c.hidden * 4, &m->c_x2) ||
+    if (alloc(m, T * 4, &m->c_tok) || alloc(m, T * 11 * 4, &m->c_tab) || alloc(m, T * c.hidden * 4, &m->c_x) || alloc(m, T * c.hidden * 4, &m->c_x2) ||
         alloc(m, T * c.hidden * 4, &m->c_y) || alloc(m, T * qd * 4, &m->c_q) || alloc(m, T * kvd * 4, &m->c_k) ||
         alloc(m, T * kvd * 4, &m->c_v) || alloc(m, T * qd * 4, &m->c_o) || alloc(m, T * max_ff * 4, &m->c_g) ||
         alloc(m, T * max_ff * 4, &m->c_u) || alloc(m, T * max_ff * 4, &m->c_ff) ||
@@ -484,56 +486,119 @@ int chunk_buffers4(ksh_gemma4 *m)
     return 0;
 }
 
+// A pass over the prompts of several pool slots: each one's tokens behind its slot's sequence length.
+struct JointPass {
+    struct Part {
+        int32_t slot;
+        const uint32_t *tokens;
+        int n;
+    };
+    ksh_kvpool *pool = nullptr;
+    std::vector<Part> parts;
+    std::vector<int> alone;      // the distinct (rounded) lengths of the passes these tokens would take alone
+    int max_batch = 0, pool_hd = 0;
+};
+
 // forward_prefill_chunk (gemma_prim.rs:1317-1607) for 2 <= t <= kChunk4 validated tokens: every layer as matrices
 // of t rows, with the layer kinds' own head sizes, rope tables and windows, cache-reading layers attending over their
 // source layer's rows, and the per-layer-embedding block.  The GEMMs run on the batch rounded up to 32 rows.
-int forward_prefill_chunk4(ksh_gemma4 *m, const uint32_t *tokens, int t)
+// joint: the t tokens are several slots' (`tokens` is not used, the model's own position is neither read nor moved):
+// the rows go through the same matrices together, and each carries its slot, its position and its attended range to
+// the append and the attention launch, and the length of the pass it would have had to the GEMMs, which cut its sums
+// accordingly (dims[6] = 2): a prompt's caches do not depend on what else arrived.  Sixteen prompts of 66 to 199 tokens
+// took sixteen passes that left most of the chip idle and converted the weights sixteen times; with their answers of ten
+// tokens 146 ms, in joint passes 82.
+int forward_prefill_chunk4(ksh_gemma4 *m, const uint32_t *tokens, int t, const JointPass *joint = nullptr)
 {
     const ksh_gemma4_cfg &c = m->c;
     if (chunk_buffers4(m)) return 1;
-    const int64_t h = c.hidden, tp = (t + 31) / 32 * 32, pt = (int64_t)c.n_layers * c.ple_dim;
-    float ids[kChunk4];
-    for (int i = 0; i < t; i++) ids[i] = (float)tokens[i];
-    if (ksh_synchronize(m->ctx)) return 1;                                   // c_tok may still be read by the previous chunk
-    if (ksh_buffer_write(m->ctx, m->c_tok, 0, ids, (size_t)t * 4, 1)) return 1;
+    // (joint passes in steps of 128 rows: their lengths are sums of many, and every length binds kernels of its own)
+    const int64_t step = joint ? 128 : 32, h = c.hidden, tp = (t + step - 1) / step * step, pt = (int64_t)c.n_layers * c.ple_dim;
+    const int tab_n = (t + 3) / 4 * 4;      // the table's fields: ids | slots | full-attention records | sliding-window records | pass alone
+    const size_t o_slots = (size_t)tab_n * 4, o_full = (size_t)tab_n * 8, o_swa = (size_t)tab_n * 24, o_alone = (size_t)tab_n * 40;
+    const int64_t slot_stride = joint ? (int64_t)c.max_seq * c.n_kv * (joint->pool_hd / 32) * 18 : 0;
+    ksh_buf *ids_buf = joint ? m->c_tab : m->c_tok;
+    if (ksh_synchronize(m->ctx)) return 1;                                   // the ids may still be read by the previous chunk
     hipStream_t st = (hipStream_t)ksh_stream(m->ctx);
-    hipLaunchKernelGGL(chunk_begin4_kernel, dim3(1), dim3(64), 0, st, (const float *)ksh_buffer_device_ptr(m->meta_full),
-                       (float *)ksh_buffer_device_ptr(m->c_meta_full), (float *)ksh_buffer_device_ptr(m->c_meta_swa), c.max_seq, c.sliding_window);
-    if (hipGetLastError() != hipSuccess) return set_error("chunk_begin launch failed");
+    if (joint) {
+        std::vector<float> tab((size_t)tab_n * 10 + (size_t)tp, 0.f);
+        int row = 0;
+        for (const JointPass::Part &part : joint->parts) {
+            const int pos0 = ksh_kvpool_seq_len(joint->pool, part.slot);
+            for (int i = 0, alone = 0, pass_end = 0; i < part.n; i++, row++) {
+                if (i == pass_end) { alone = prefill_pass_tokens(part.n - i); pass_end += alone; }
+                tab[(size_t)10 * tab_n + row] = (float)((alone + 31) / 32 * 32);
+                const int pos = pos0 + i, kv_len = pos + 1, start = kv_len > c.sliding_window ? kv_len - c.sliding_window : 0;
+                tab[row] = (float)part.tokens[i];
+                tab[(size_t)tab_n + row] = (float)part.slot;
+                float *full = &tab[(size_t)2 * tab_n + 4 * (size_t)row], *swa = &tab[(size_t)6 * tab_n + 4 * (size_t)row];
+                full[0] = (float)kv_len; full[3] = (float)pos;
+                swa[0] = (float)(kv_len - start); swa[1] = (float)start; swa[2] = (float)c.sliding_window; swa[3] = (float)pos;
+            }
+        }
+        if (ksh_buffer_write(m->ctx, m->c_tab, 0, tab.data(), tab.size() * 4, 1)) return 1;
+    } else {
+        float ids[kChunk4];
+        for (int i = 0; i < t; i++) ids[i] = (float)tokens[i];
+        if (ksh_buffer_write(m->ctx, m->c_tok, 0, ids, (size_t)t * 4, 1)) return 1;
+        hipLaunchKernelGGL(chunk_begin4_kernel, dim3(1), dim3(64), 0, st, (const float *)ksh_buffer_device_ptr(m->meta_full),
+                           (float *)ksh_buffer_device_ptr(m->c_meta_full), (float *)ksh_buffer_device_ptr(m->c_meta_swa), c.max_seq, c.sliding_window);
+        if (hipGetLastError() != hipSuccess) return set_error("chunk_begin launch failed");
+    }
     int n = 0;
     ksh_kernel *k = nullptr, *k_norm = nullptr, *k_add = nullptr, *k_add_then = nullptr;
-    auto mm = [&](int dt, int64_t rows, int64_t cols, ksh_buf *w, ksh_buf *x, ksh_buf *y) {
+    // one GEMM of the pass: dims = rows, cols, tp[, rows1, rows2[, prologue[, unfolded, slices of X]]]
+    auto gemm = [&](int dt, std::initializer_list<int64_t> dims, std::initializer_list<ksh_buf *> ins, std::initializer_list<ksh_buf *> outs) -> int {
+        ksh_kernel_desc d{};
+        d.kind = KSH_MATVEC_BATCH;
+        int nd = 0;
+        for (int64_t v : dims) d.dims[nd++] = v;
+        d.dtypes[0] = dt; d.dtypes[1] = d.dtypes[2] = KSH_F32;
+        if (d.dims[5]) d.params[0] = c.eps;
+        ksh_buf *ib[kMaxIn], *ob[kMaxOut];
+        size_t io[kMaxIn] = {};
+        int ni = 0, no = 0;
+        for (ksh_buf *b : ins) ib[ni++] = b;
+        for (ksh_buf *b : outs) ob[no++] = b;
+        if (joint) {
+            // K slices as the prompts would have alone: the launch's own (workgroups per slice) where all have the same and
+            // the launch could do with the workgroups, else each row's
+            int lo = 1 << 30, hi = 0;
+            for (int len : joint->alone) { const int ks = matvec_batch_slices(d, len); lo = std::min(lo, ks); hi = std::max(hi, ks); }
+            if (hi == 1 || (lo == hi && matvec_batch_slices(d, (int)tp) > 1)) {
+                d.sched.k_split = (uint32_t)hi;
+            } else {
+                d.dims[6] = 2;
+                ib[ni] = m->c_tab;
+                io[ni++] = o_alone;
+            }
+        }
         ksh_kernel *kk = nullptr;
-        return get(m, KSH_MATVEC_BATCH, {rows, cols, tp}, {dt, KSH_F32, KSH_F32}, {}, &kk) || enc(m, kk, {w, x}, {y}, n);
+        n += 1;
+        return ksh_kernel_get(m->ctx, &d, &kk) || ksh_encode(m->ctx, kk, ib, io, ni, ob, nullptr, no);
     };
+    auto mm = [&](int dt, int64_t rows, int64_t cols, ksh_buf *w, ksh_buf *x, ksh_buf *y) { return gemm(dt, {rows, cols, tp}, {w, x}, {y}); };
     // matrices of one dtype over the same rows (q | k | v, gate | up) are one launch of the tile over one preparation
     // of the rows
     auto mm2 = [&](int dt, int64_t rows, int64_t cols, ksh_buf *w0, ksh_buf *w1, ksh_buf *x, ksh_buf *y0, ksh_buf *y1) {
-        ksh_kernel *kk = nullptr;
-        return get(m, KSH_MATVEC_BATCH, {rows, cols, tp, rows}, {dt, KSH_F32, KSH_F32}, {}, &kk) || enc(m, kk, {w0, x, w1}, {y0, y1}, n);
+        return gemm(dt, {rows, cols, tp, rows}, {w0, x, w1}, {y0, y1});
     };
     auto mm3 = [&](int dt, int64_t rows0, int64_t rows12, int64_t cols, ksh_buf *w0, ksh_buf *w1, ksh_buf *w2, ksh_buf *x, ksh_buf *y0, ksh_buf *y1,
                    ksh_buf *y2) {
-        ksh_kernel *kk = nullptr;
-        return get(m, KSH_MATVEC_BATCH, {rows0, cols, tp, rows12, rows12}, {dt, KSH_F32, KSH_F32}, {}, &kk) ||
-               enc(m, kk, {w0, x, w1, w2}, {y0, y1, y2}, n);
+        return gemm(dt, {rows0, cols, tp, rows12, rows12}, {w0, x, w1, w2}, {y0, y1, y2});
     };
     const bool merged = true;
     // ... with the rows' producers inside the GEMMs' preparations (dims[5]: the attention norm in q | k | v's,
     // add-then-norm in gate | up's, gelu(gate) * up in the down projection's)
     const bool inside = merged && h % 512 == 0 && h <= 8192;
-    auto mm_pro = [&](int dt, std::initializer_list<int64_t> dims, std::initializer_list<ksh_buf *> ins, std::initializer_list<ksh_buf *> outs) {
-        ksh_kernel *kk = nullptr;
-        return get(m, KSH_MATVEC_BATCH, dims, {dt, KSH_F32, KSH_F32}, {c.eps}, &kk) || enc(m, kk, ins, outs, n);
-    };
     if (get(m, KSH_COPY_SCALE_INDEXED, {h, c.vocab, t}, {m->g.dt_embd}, {std::sqrt((float)c.hidden)}, &k) ||
-        enc(m, k, {m->g.token_embd, m->c_tok}, {m->c_x}, n))
+        enc(m, k, {m->g.token_embd, ids_buf}, {m->c_x}, n))
         return 1;
     if (c.ple_dim > 0) {
         // ple_from_idx_batch + ple_prepass_batch (gemma_prim.rs:1333-1358)
         ksh_kernel *kg = nullptr, *kn = nullptr, *kmix = nullptr;
         if (get(m, KSH_COPY_SCALE_INDEXED, {pt, c.vocab, t}, {m->g.dt_ple}, {std::sqrt((float)c.ple_dim)}, &kg) ||
-            enc(m, kg, {m->g.ple_embd, m->c_tok}, {m->c_ple_tok}, n) ||
+            enc(m, kg, {m->g.ple_embd, ids_buf}, {m->c_ple_tok}, n) ||
             mm(m->g.dt_ple_proj, pt, h, m->g.ple_model_proj, m->c_x, m->c_ple_tmp) ||
             get(m, KSH_RMSNORM_PER_HEAD, {(int64_t)t * c.n_layers, c.ple_dim, 0}, {}, {c.eps}, &kn) ||
             enc(m, kn, {m->c_ple_tmp, m->g.ple_proj_norm}, {m->c_ple_ctx}, n) ||
@@ -548,37 +613,44 @@ int forward_prefill_chunk4(ksh_gemma4 *m, const uint32_t *tokens, int t)
         const ksh_gemma4_layer &L = m->layers[l];
         const LayerPlan &P = m->plan[l];
         ksh_buf *rope_tab = P.swa ? m->rope_swa : m->rope_full;
-        ksh_buf *kc = m->kv_k[P.src], *vc = m->kv_v[P.src];
+        ksh_buf *kc = joint ? ksh_kvpool_layer_k(joint->pool, P.src) : m->kv_k[P.src], *vc = joint ? ksh_kvpool_layer_v(joint->pool, P.src) : m->kv_v[P.src];
+        const size_t o_meta = P.swa ? o_swa : o_full;
         ksh_kernel *k_head = nullptr, *k_sdpa = nullptr, *k_gelu = nullptr;
         const bool qkv_merged = merged && P.owns && L.dt_q == L.dt_k && L.dt_q == L.dt_v;
         const bool q_inside = inside && (qkv_merged || !P.owns);
         if (q_inside) {
-            if (qkv_merged ? mm_pro(L.dt_q, {P.qd, h, tp, P.kvd, P.kvd, 1}, {L.wq, m->c_x, L.wk, L.wv, L.attn_norm}, {m->c_q, m->c_k, m->c_v})
-                           : mm_pro(L.dt_q, {P.qd, h, tp, 0, 0, 1}, {L.wq, m->c_x, L.attn_norm}, {m->c_q}))
+            if (qkv_merged ? gemm(L.dt_q, {P.qd, h, tp, P.kvd, P.kvd, 1}, {L.wq, m->c_x, L.wk, L.wv, L.attn_norm}, {m->c_q, m->c_k, m->c_v})
+                           : gemm(L.dt_q, {P.qd, h, tp, 0, 0, 1}, {L.wq, m->c_x, L.attn_norm}, {m->c_q}))
                 return 1;
         } else {
             if (enc(m, k_norm, {m->c_x, L.attn_norm}, {m->c_x2}, n)) return 1;
             if (qkv_merged ? mm3(L.dt_q, P.qd, P.kvd, h, L.wq, L.wk, L.wv, m->c_x2, m->c_q, m->c_k, m->c_v) : mm(L.dt_q, P.qd, h, L.wq, m->c_x2, m->c_q)) return 1;
         }
         if (P.owns) {
-            if ((!qkv_merged && (mm(L.dt_k, P.kvd, h, L.wk, m->c_x2, m->c_k) || mm(L.dt_v, P.kvd, h, L.wv, m->c_x2, m->c_v))) ||
-                get(m, KSH_RMSNORM_PER_HEAD_QKV_Q40, {c.n_q, c.n_kv, P.hd, c.max_seq, t}, {}, {c.eps}, &k_head) ||
-                enc(m, k_head, {m->c_q, L.q_norm, rope_tab, m->c_k, L.k_norm, m->c_v, m->meta_full}, {m->c_q, kc, vc}, n))
+            if (!qkv_merged && (mm(L.dt_k, P.kvd, h, L.wk, m->c_x2, m->c_k) || mm(L.dt_v, P.kvd, h, L.wv, m->c_x2, m->c_v))) return 1;
+            if (joint ? get(m, KSH_RMSNORM_PER_HEAD_QKV_Q40, {c.n_q, c.n_kv, P.hd, c.max_seq, t, joint->max_batch, slot_stride}, {}, {c.eps}, &k_head) ||
+                            enc_off(m, k_head, {m->c_q, L.q_norm, rope_tab, m->c_k, L.k_norm, m->c_v, m->c_tab, m->c_tab}, {0, 0, 0, 0, 0, 0, o_meta, o_slots},
+                                    {m->c_q, kc, vc}, n)
+                      : get(m, KSH_RMSNORM_PER_HEAD_QKV_Q40, {c.n_q, c.n_kv, P.hd, c.max_seq, t}, {}, {c.eps}, &k_head) ||
+                            enc(m, k_head, {m->c_q, L.q_norm, rope_tab, m->c_k, L.k_norm, m->c_v, m->meta_full}, {m->c_q, kc, vc}, n))
                 return 1;
         } else {
-            if (get(m, KSH_RMSNORM_PER_HEAD, {(int64_t)t * c.n_q, P.hd, 2, c.max_seq, c.n_q}, {}, {c.eps}, &k_head) ||
-                enc(m, k_head, {m->c_q, L.q_norm, rope_tab, m->meta_full}, {m->c_q}, n))
+            if (get(m, KSH_RMSNORM_PER_HEAD, {(int64_t)t * c.n_q, P.hd, 2, c.max_seq, c.n_q, joint ? 1 : 0}, {}, {c.eps}, &k_head) ||
+                (joint ? enc_off(m, k_head, {m->c_q, L.q_norm, rope_tab, m->c_tab}, {0, 0, 0, o_meta}, {m->c_q}, n)
+                       : enc(m, k_head, {m->c_q, L.q_norm, rope_tab, m->meta_full}, {m->c_q}, n)))
                 return 1;
         }
         // (heads of 256 or 512 in chunks of more than 16 tokens take the attention's matrix-core form: one partition per token)
-        if (get(m, KSH_SDPA_BATCH, {c.n_q, c.n_kv, P.hd, c.max_seq, t, t > 16 && (P.hd == 256 || P.hd == 512) && c.n_q / c.n_kv <= 8 ? 1 : kChunkPartitions4}, {KSH_Q40, KSH_F32}, {c.attn_scale}, &k_sdpa) ||
-            enc(m, k_sdpa, {m->c_q, kc, vc, P.swa ? m->c_meta_swa : m->c_meta_full}, {m->c_tmp, m->c_o}, n))
+        if (joint ? get(m, KSH_SDPA_BATCH, {c.n_q, c.n_kv, P.hd, c.max_seq, t, 1, joint->max_batch, slot_stride}, {KSH_Q40, KSH_F32}, {c.attn_scale}, &k_sdpa) ||
+                        enc_off(m, k_sdpa, {m->c_q, kc, vc, m->c_tab, m->c_tab}, {0, 0, 0, o_meta, o_slots}, {m->c_tmp, m->c_o}, n)
+                  : get(m, KSH_SDPA_BATCH, {c.n_q, c.n_kv, P.hd, c.max_seq, t, t > 16 && (P.hd == 256 || P.hd == 512) && c.n_q / c.n_kv <= 8 ? 1 : kChunkPartitions4}, {KSH_Q40, KSH_F32}, {c.attn_scale}, &k_sdpa) ||
+                        enc(m, k_sdpa, {m->c_q, kc, vc, P.swa ? m->c_meta_swa : m->c_meta_full}, {m->c_tmp, m->c_o}, n))
             return 1;
         // With the producers inside, the o and the gate | up projection leave their K slices' partial sums unfolded
         // for the preparation that reads them (dims[6], dims[7]); the down projection folds (a plain norm reads it).
         ksh_kernel *u_o = nullptr, *u_gu = nullptr;
         bool travel = false;
-        if (inside && L.dt_gate == L.dt_up) {
+        if (inside && L.dt_gate == L.dt_up && !joint) {
             const size_t T = kChunk4;
             if (get(m, KSH_MATVEC_BATCH, {h, P.qd, tp, 0, 0, 0, 1}, {L.dt_o, KSH_F32, KSH_F32}, {c.eps}, &u_o) ||
                 get(m, KSH_MATVEC_BATCH, {L.ffn, h, tp, L.ffn, 0, 2, 1, (int64_t)u_o->info.grid[2]}, {L.dt_gate, KSH_F32, KSH_F32}, {c.eps}, &u_gu))
@@ -588,16 +660,16 @@ int forward_prefill_chunk4(ksh_gemma4 *m, const uint32_t *tokens, int t)
         if (travel) {
             if (enc(m, u_o, {L.wo, m->c_o}, {m->c_po}, n) ||
                 enc(m, u_gu, {L.wgate, m->c_po, L.wup, L.post_attn_norm, m->c_x, L.ffn_norm}, {m->c_pg, m->c_x}, n) ||
-                mm_pro(L.dt_down, {h, L.ffn, tp, 0, 0, 3, 0, (int64_t)u_gu->info.grid[2]}, {L.wdown, m->c_pg}, {m->c_y}))
+                gemm(L.dt_down, {h, L.ffn, tp, 0, 0, 3, 0, (int64_t)u_gu->info.grid[2]}, {L.wdown, m->c_pg}, {m->c_y}))
                 return 1;
         } else if (
             mm(L.dt_o, h, P.qd, L.wo, m->c_o, m->c_y) ||
             (inside && L.dt_gate == L.dt_up
-                 ? mm_pro(L.dt_gate, {L.ffn, h, tp, L.ffn, 0, 2}, {L.wgate, m->c_y, L.wup, L.post_attn_norm, m->c_x, L.ffn_norm}, {m->c_g, m->c_u, m->c_x})
+                 ? gemm(L.dt_gate, {L.ffn, h, tp, L.ffn, 0, 2}, {L.wgate, m->c_y, L.wup, L.post_attn_norm, m->c_x, L.ffn_norm}, {m->c_g, m->c_u, m->c_x})
                  : (enc(m, k_add_then, {m->c_y, L.post_attn_norm, m->c_x, L.ffn_norm}, {m->c_x, m->c_x2}, n) ||
                     (merged && L.dt_gate == L.dt_up ? mm2(L.dt_gate, L.ffn, h, L.wgate, L.wup, m->c_x2, m->c_g, m->c_u)
                                                     : (mm(L.dt_gate, L.ffn, h, L.wgate, m->c_x2, m->c_g) || mm(L.dt_up, L.ffn, h, L.wup, m->c_x2, m->c_u))))) ||
-            (inside ? mm_pro(L.dt_down, {h, L.ffn, tp, 0, 0, 3}, {L.wdown, m->c_g, m->c_u}, {m->c_y})
+            (inside ? gemm(L.dt_down, {h, L.ffn, tp, 0, 0, 3}, {L.wdown, m->c_g, m->c_u}, {m->c_y})
                     : (get(m, KSH_GELU_MUL, {(int64_t)t * L.ffn}, {}, {}, &k_gelu) || enc(m, k_gelu, {m->c_g, m->c_u}, {m->c_ff}, n) ||
                        mm(L.dt_down, h, L.ffn, L.wdown, m->c_ff, m->c_y))))
             return 1;
@@ -614,6 +686,7 @@ int forward_prefill_chunk4(ksh_gemma4 *m, const uint32_t *tokens, int t)
                 return 1;
         }
     }
+    if (joint) return 0;
     m->pos += t;
     const int at = std::min(m->pos, c.max_seq - 1);
     hipLaunchKernelGGL(seek4_kernel, dim3(1), dim3(64), 0, st, (float *)ksh_buffer_device_ptr(m->meta_full),
@@ -1069,6 +1142,41 @@ int pool_fits(const ksh_gemma4 *m, const ksh_kvpool *pool, int *max_batch, int *
                          c.max_seq, c.n_kv, std::max(c.hd_swa, c.hd_full));
     return 0;
 }
+
+// ksh::g_prefill_slots.  Where the attention of a long pass is not built for a layer's heads, and for a pool that does
+// not fit the model, the slots take passes of their own (which then say what is wrong).
+int prefill_slots4(ksh_gemma4 *m, ksh_kvpool *pool, const int32_t *slots, const uint32_t *const *tokens, const int *n, int count, uint8_t *taken)
+{
+    const ksh_gemma4_cfg &c = m->c;
+    JointPass joint;
+    joint.pool = pool;
+    if (pool_fits(m, pool, &joint.max_batch, &joint.pool_hd) || joint.max_batch > 4096) return 0;
+    for (const LayerPlan &P : m->plan)
+        if ((P.hd != 256 && P.hd != 512) || c.n_q / c.n_kv > 8) return 0;
+    int total = 0;
+    for (int s = 0; s < count; s++) {
+        const int pos = ksh_kvpool_seq_len(pool, slots[s]);
+        bool fits = n[s] > 0 && pos >= 0 && pos + n[s] <= c.max_seq && total + n[s] <= kChunk4;
+        for (int i = 0; i < n[s] && fits; i++) fits = tokens[s][i] < (uint32_t)c.vocab;
+        // (passes of up to 64 tokens take GEMMs of another form)
+        for (int i = 0, t = 0; i < n[s] && fits; i += t) { t = prefill_pass_tokens(n[s] - i); fits = t > kSmallPass; }
+        if (!fits) continue;
+        taken[s] = 1;
+        total += n[s];
+        joint.parts.push_back({slots[s], tokens[s], n[s]});
+        for (int i = 0, t = 0; i < n[s]; i += t) {
+            t = prefill_pass_tokens(n[s] - i);
+            const int len = (t + 31) / 32 * 32;
+            if (std::find(joint.alone.begin(), joint.alone.end(), len) == joint.alone.end()) joint.alone.push_back(len);
+        }
+    }
+    if (joint.parts.size() < 2) {
+        std::fill(taken, taken + count, (uint8_t)0);
+        return 0;
+    }
+    return forward_prefill_chunk4(m, nullptr, total, &joint) || ksh_synchronize(m->ctx);
+}
+[[maybe_unused]] const bool registered = (ksh::g_prefill_slots = prefill_slots4, true);
 
 int encode_round4(ksh_gemma4 *m, ksh_kvpool *pool, int t, int max_batch, int pool_hd);
 

@@ -34,6 +34,15 @@ inline int prefill_pass_tokens(int left)
     return left >= kPrefillPass ? kPrefillPass : left >= kPrefillPass / 2 ? kPrefillPass / 2 : left;
 }
 
+// The prompt tokens of several pool slots in one pass through the layers: n[i] tokens behind slot slots[i]'s sequence
+// length, at most kPrefillPass in all, with the bits of passes of their own.  taken[i] tells which slots went along (the
+// others, and every slot where fewer than two can, are left to the caller); nonzero with the error set when the pass of
+// those failed.  The scheduler finds the models' function here (null: no model code is linked in, every slot takes its
+// own pass).
+using PrefillSlotsFn = int (*)(ksh_gemma4 *m, ksh_kvpool *pool, const int32_t *slots, const uint32_t *const *tokens, const int *n, int count,
+                               uint8_t *taken);
+extern PrefillSlotsFn g_prefill_slots;
+
 constexpr int kMaxIn = 8;
 constexpr int kMaxOut = 4;
 
@@ -171,6 +180,7 @@ int bind_matvec_q4k_family(ksh_kernel &k);
 int bind_matvec_qkv(ksh_kernel &k);
 int bind_matvec_gate_up_gelu(ksh_kernel &k);
 int bind_matvec_batch(ksh_kernel &k);
+int matvec_batch_slices(const ksh_kernel_desc &d, int batch);   // K slices of the tile over `batch` tokens
 int bind_round_prep(ksh_kernel &k);
 int bind_matvec_round(ksh_kernel &k);
 int bind_dequant(ksh_kernel &k);

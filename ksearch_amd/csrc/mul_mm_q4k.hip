@@ -333,7 +333,39 @@ struct MmParams {
     // f32 activations (the kernel's LO form): the lo parts' fragments and 1 / s per token row (see mm_prep_rows_kernel)
     const _Float16 *Xf_lo;
     const float *inv_s;
+    // the kernel's CUT form: per row, the tokens of the launch whose K slices its sums are to be cut into
+    const float *cut_as;
 };
+
+// Tokens per workgroup of the tile.  64 (Q4_K): up to 64 tokens (the other half of a 128-token tile would be empty
+// rows), and wherever the 128-token tiles and their K slices are fewer than the compute units (bf16 activations) or
+// than twice the compute units (f32 activations, whose tile runs two products per converted weight) -- two
+// workgroups share a compute unit then, and twice as many of them fill the chip.  Beyond that the 128-token tile
+// (bf16, cfg2: 33.7 us against 40.3 with 64-token tiles; f32, prompts of 256 / 1024 / 4000 tokens through cfg4's
+// model: 5.05 / 14.1 / 67.7 ms with this rule, 5.07 / 14.25 / 68.0 with 64-token tiles throughout, 5.3 / 14.9 / 72.7
+// with 128-token tiles from 65 tokens on).
+__host__ __device__ constexpr int mm_tile_tokens(bool q6, bool f32x, int row_tiles, int batch, int ks)
+{
+    if (q6) return 128;
+    return batch <= 64 || (int64_t)((batch + BM - 1) / BM) * row_tiles * ks < (f32x ? 512 : 256) ? 64 : 128;
+}
+
+// Few tiles (a prompt of a few hundred tokens, or a narrow matrix): the nsb superblocks of a row are split into this many
+// K slices, until the grid is about one workgroup per compute unit; every slice has its own sum and the sums are added
+// in a fixed order.  (A slice of one superblock is all prologue; the workgroups are counted with the token tile they will
+// have, and f32 rows of more than half a prompt pass as that many: how a row's sum is cut does not depend on which pass
+// of its prompt the row is in.)
+__host__ __device__ constexpr int mm_k_slices(bool q6, bool f32x, int row_tiles, int nsb, int batch)
+{
+    const int counted = f32x && batch > kPrefillPass / 2 ? kPrefillPass / 2 : batch;
+    int ks = 1;
+    while (nsb % (ks * 2) == 0 && nsb / (ks * 2) >= 2) {
+        const int tm = mm_tile_tokens(q6, f32x, row_tiles, counted, ks * 2);
+        if ((int64_t)((counted + tm - 1) / tm) * row_tiles * ks * 2 > 256) break;
+        ks *= 2;
+    }
+    return ks;
+}
 
 __device__ __forceinline__ uint32_t pair_f16(uint32_t masked, uint32_t sc)
 {
@@ -378,7 +410,11 @@ constexpr size_t kLdsBytes64 = 2 * (size_t)(kLdsMain + (64 + BN) * PITCH2) * 2 +
 // LO = true: f32 activations as two f16 parts at the row's own scale.  Every converted weight meets the hi and the lo
 // fragment of a token tile in the same accumulator (twice the matrix instructions per conversion, and the
 // conversions are what a step waits for), and the finished sums are multiplied by 1 / s of their token.
-template <bool Q6, int TM, bool LO>
+// CUT = true (f32 activations): the rows belong to prompts that would each have had a launch of their own, whose K slices
+// depend on its length.  The workgroup takes all of K, and where a row's slice ends its sum is added to Y and starts
+// again from zero: the bits of those launches from one that fills the chip (a read and a write of the tile's results
+// per slice end, from L2).
+template <bool Q6, int TM, bool LO, bool CUT = false>
 __global__ __launch_bounds__(kThreadsMM, TM == 64 ? 2 : 1) void q_mul_mm_kernel(MmParams p)
 {
     constexpr int MT = TM / 64, kLdsMinT = (TM + BN) * PITCH2;
@@ -391,6 +427,7 @@ __global__ __launch_bounds__(kThreadsMM, TM == 64 ? 2 : 1) void q_mul_mm_kernel(
     // which matrix this row tile belongs to (the copy of the arguments is this workgroup's own)
     int by = blockIdx.y, ycol = 0;
     const int rows_all = p.rows + p.rows1 + p.rows2;
+    const int rows_of[3] = {p.rows, p.rows1, p.rows2};
     if (p.rows1) {
         const int ty0 = (p.rows + BN - 1) / BN, ty1 = (p.rows1 + BN - 1) / BN;
         if (by >= ty0 + ty1) { by -= ty0 + ty1; ycol = p.rows + p.rows1; p.W = p.W2; p.Y = p.Y2; p.rows = p.rows2; }
@@ -631,6 +668,12 @@ __global__ __launch_bounds__(kThreadsMM, TM == 64 ? 2 : 1) void q_mul_mm_kernel(
                 if (LO) r.al[mt][ks] = afrag_lo(mt, step, ks);
             }
     };
+    // CUT: lane t % 32 keeps the superblocks per slice of the tile's row t and what is left of the current one
+    int cut_len = nsb, cut_left = nsb;
+    if (CUT) {
+        const int row_tiles = (rows_of[0] + BN - 1) / BN + (rows_of[1] + BN - 1) / BN + (rows_of[2] + BN - 1) / BN;
+        cut_len = cut_left = nsb / mm_k_slices(Q6, true, row_tiles, nsb, (int)p.cut_as[min(t0 + wm * 32 + lm, p.batch - 1)]);
+    }
     ARegs a0, a1;
     fetch_a(0, a0);
     if (!LO) fetch_a(min(1, nsteps - 1), a1);
@@ -717,6 +760,49 @@ __global__ __launch_bounds__(kThreadsMM, TM == 64 ? 2 : 1) void q_mul_mm_kernel(
                     for (int i = 0; i < 16; i++)
                         F[mt][nt][i] = fmaf(dn, Cp[mt][nt][i], F[mt][nt][i]);
             }
+            if (CUT) {
+                static_assert(MW == 1, "one token tile per wave");
+                cut_left -= 1;
+                // (rows past the batch neither end nor start: their sums are never stored)
+                const bool live = t0 + wm * 32 + lm < p.batch;
+                uint32_t ends = (uint32_t)__ballot(live && cut_left == 0), first = (uint32_t)__ballot(sb + 1 == cut_len);
+                if (cut_left == 0) cut_left = cut_len;
+                if (ends) {
+                    // (opaque copies: what follows from them is worked out here, not kept in registers through the loop)
+                    const int h4 = 4 * (lane >> 5);
+                    int row = t0 + wm * 32 + h4;
+                    asm volatile("" : "+v"(row));
+                    ends >>= h4;
+                    first >>= h4;
+#pragma unroll
+                    for (int nt = 0; nt < NW_; nt++) {
+                        int r = r0 + wn * NSPAN + nt * 32 + lm;
+                        asm volatile("" : "+v"(r), "+v"(row));
+                        if (r < p.rows) {
+                            float *y = p.Y + (size_t)row * ystride + r;
+#pragma unroll
+                            for (int i0 = 0; i0 < 16; i0 += 4) {
+                                float sum[4], inv[4];
+#pragma unroll
+                                for (int i = 0; i < 4; i++) {
+                                    const int tr = 2 * i0 + i;
+                                    sum[i] = 0.f;
+                                    inv[i] = p.inv_s[min(row + tr, p.batch - 1)];
+                                    if ((ends & ~first) & (1u << tr)) sum[i] = y[(size_t)tr * ystride];
+                                }
+#pragma unroll
+                                for (int i = 0; i < 4; i++) {
+                                    const int tr = 2 * i0 + i;
+                                    if (ends & (1u << tr)) y[(size_t)tr * ystride] = sum[i] + F[0][nt][i0 + i] * inv[i];
+                                }
+                            }
+                        }
+#pragma unroll
+                        for (int i = 0; i < 16; i++)
+                            if (ends & (1u << (8 * (i / 4) + (i & 3)))) F[0][nt][i] = 0.f;
+                    }
+                }
+            }
         }
         __syncthreads();
     };
@@ -727,6 +813,7 @@ __global__ __launch_bounds__(kThreadsMM, TM == 64 ? 2 : 1) void q_mul_mm_kernel(
         mul_step(sb, std::integral_constant<int, 3>{}, LO ? a0 : a1);
     }
 
+    if (CUT) return;   // (the last slices' ends have stored everything)
     // accumulator layout of the 32x32 tile: column = lane % 32, row = 8*(i/4) + 4*(lane/32) + i%4
 #pragma unroll
     for (int mt = 0; mt < MW; mt++)
@@ -1419,20 +1506,7 @@ int launch_matvec_round(const ksh_kernel &k, const LaunchArgs &a, hipStream_t st
 
 constexpr int kSkinnyMaxBatch = 64;
 
-// Tokens per workgroup of the tile.  64 (Q4_K): up to 64 tokens (the other half of a 128-token tile would be empty
-// rows), and wherever the 128-token tiles and their K slices are fewer than the compute units (bf16 activations) or
-// than twice the compute units (f32 activations, whose tile runs two products per converted weight) -- two
-// workgroups share a compute unit then, and twice as many of them fill the chip.  Beyond that the 128-token tile
-// (bf16, cfg2: 33.7 us against 40.3 with 64-token tiles; f32, prompts of 256 / 1024 / 4000 tokens through cfg4's
-// model: 5.05 / 14.1 / 67.7 ms with this rule, 5.07 / 14.25 / 68.0 with 64-token tiles throughout, 5.3 / 14.9 / 72.7
-// with 128-token tiles from 65 tokens on).
-int mm_tile_tokens(const ksh_kernel_desc &d, int64_t batch, int64_t ks)
-{
-    if (d.dtypes[0] == KSH_Q6K) return 128;
-    const int64_t row_tiles = (d.dims[0] + BN - 1) / BN + (d.dims[3] + BN - 1) / BN + (d.dims[4] + BN - 1) / BN;
-    const int64_t fill = d.dtypes[1] == KSH_F32 ? 512 : 256;
-    return batch <= 64 || ((batch + BM - 1) / BM) * row_tiles * ks < fill ? 64 : 128;
-}
+int mm_row_tiles(const ksh_kernel_desc &d) { return (int)((d.dims[0] + BN - 1) / BN + (d.dims[3] + BN - 1) / BN + (d.dims[4] + BN - 1) / BN); }
 
 int launch_mul_mm(const ksh_kernel &k, const LaunchArgs &a, hipStream_t st)
 {
@@ -1452,7 +1526,7 @@ int launch_mul_mm(const ksh_kernel &k, const LaunchArgs &a, hipStream_t st)
     if (prologue) {
         // the rows' producer runs inside the preparation: in = W, X, [W1, W2,] then the prologue's operands
         const int xs = (int)k.desc.dims[7];
-        const int n_out0 = k.desc.dims[6] ? 1 : n_mat0;                    // (unfolded partial sums are one buffer)
+        const int n_out0 = k.desc.dims[6] == 1 ? 1 : n_mat0;                    // (unfolded partial sums are one buffer)
         const float *X = (const float *)a.in[1], *q0 = (const float *)a.in[1 + n_mat0];
         const float eps = k.desc.params[0];
         if (prologue == 1)
@@ -1473,7 +1547,7 @@ int launch_mul_mm(const ksh_kernel &k, const LaunchArgs &a, hipStream_t st)
     const int rows1 = (int)k.desc.dims[3], rows2 = (int)k.desc.dims[4];
     p.rows1 = rows1; p.rows2 = rows2;
     p.W1 = rows1 ? (const uint8_t *)a.in[2] : p.W; p.W2 = rows2 ? (const uint8_t *)a.in[3] : p.W;
-    const bool unfolded_out = k.desc.dims[6] != 0;
+    const bool unfolded_out = k.desc.dims[6] == 1;
     p.Y1 = rows1 && !unfolded_out ? (float *)a.out[1] : p.Y; p.Y2 = rows2 && !unfolded_out ? (float *)a.out[2] : p.Y;
     if (k.variant == 1) {
         // the small-batch form: one launch, the low parts riding along
@@ -1488,15 +1562,18 @@ int launch_mul_mm(const ksh_kernel &k, const LaunchArgs &a, hipStream_t st)
         const hipError_t e2 = hipGetLastError();
         return e2 == hipSuccess ? 0 : hip_fail(e2, "mul_mm (small batch) launch");
     }
-    const int tm = mm_tile_tokens(k.desc, batch, k.variant >= 2 ? k.variant >> 1 : 1);
+    const bool cut = k.desc.dims[6] == 2;
+    const int tm = mm_tile_tokens(k.desc.dtypes[0] == KSH_Q6K, f32x, mm_row_tiles(k.desc), batch, k.variant >= 2 ? k.variant >> 1 : 1);
     const dim3 grid((batch + tm - 1) / tm, (rows + BN - 1) / BN + (rows1 + BN - 1) / BN + (rows2 + BN - 1) / BN);
     p.Xf = Xf; p.SxA = SxA; p.Xf_lo = Xf_lo; p.inv_s = inv_s;
     p.ksplit = 0; p.Y_parts = nullptr;
+    p.cut_as = cut ? (const float *)a.in[k.info.n_inputs - 1] : nullptr;
     const bool q6 = k.desc.dtypes[0] == KSH_Q6K;
     auto launch_tile = [&](dim3 g) {
 #define KSH_TILE(Q6, TM, LDS) \
     do { \
-        if (f32x) hipLaunchKernelGGL((q_mul_mm_kernel<Q6, TM, true>), g, dim3(kThreadsMM), LDS, st, p); \
+        if (cut) hipLaunchKernelGGL((q_mul_mm_kernel<Q6, TM, true, true>), g, dim3(kThreadsMM), LDS, st, p); \
+        else if (f32x) hipLaunchKernelGGL((q_mul_mm_kernel<Q6, TM, true>), g, dim3(kThreadsMM), LDS, st, p); \
         else hipLaunchKernelGGL((q_mul_mm_kernel<Q6, TM, false>), g, dim3(kThreadsMM), LDS, st, p); \
     } while (0)
         if (q6) KSH_TILE(true, 128, kLdsBytes);
@@ -1508,7 +1585,7 @@ int launch_mul_mm(const ksh_kernel &k, const LaunchArgs &a, hipStream_t st)
         // few tiles: K slices as blockIdx.z of one launch, then the fold
         const int ks = k.variant >> 1;
         p.ksplit = ks;
-        const bool unfolded = k.desc.dims[6] != 0;                    // the partial sums are the result: the reader adds them
+        const bool unfolded = k.desc.dims[6] == 1;                    // the partial sums are the result: the reader adds them
         p.Y_parts = unfolded ? (float *)a.out[0] : (float *)((f32x ? SxA_lo : SxA) + sx_halves);     // (else behind the prepared activations)
         launch_tile(dim3(grid.x, grid.y, ks));
         hipError_t e3 = hipGetLastError();
@@ -1526,6 +1603,11 @@ int launch_mul_mm(const ksh_kernel &k, const LaunchArgs &a, hipStream_t st)
 }
 
 }  // namespace
+
+int matvec_batch_slices(const ksh_kernel_desc &d, int batch)
+{
+    return mm_k_slices(d.dtypes[0] == KSH_Q6K, d.dtypes[1] == KSH_F32, mm_row_tiles(d), (int)(d.dims[1] / 256), batch);
+}
 
 int bind_matvec_batch(ksh_kernel &k)
 {
@@ -1559,8 +1641,13 @@ int bind_matvec_batch(ksh_kernel &k)
     // matrices' columns side by side; slices = grid[2] of the bound kernel), for a reader that adds them itself --
     // dims[7] = the slices (grid[2]) of the GEMM whose unfolded result this one's X is (prologues 1 to 3; prologue 3
     // then reads gate | up from that one buffer and takes no `up` operand)
-    const int64_t unfolded = k.desc.dims[6], x_slices = k.desc.dims[7];
-    if (unfolded < 0 || unfolded > 1) return set_error("matvec_batch: dims[6]=%lld (0, or 1 for unfolded partial sums)", (long long)unfolded);
+    // dims[6] = 2: the rows belong to several prompts, each to be summed as in a launch of its own: one more input,
+    // f32[batch], the tokens of that launch for every row (more than 64).  For f32 activations.
+    const bool unfolded = k.desc.dims[6] == 1, cut = k.desc.dims[6] == 2;
+    const int64_t x_slices = k.desc.dims[7];
+    if (k.desc.dims[6] < 0 || k.desc.dims[6] > 2)
+        return set_error("matvec_batch: dims[6]=%lld (0, 1 for unfolded partial sums, 2 for rows summed as in launches of their own)", (long long)k.desc.dims[6]);
+    if (cut && !f32x) return set_error("matvec_batch: rows summed as in launches of their own (dims[6]=2) take F32 activations");
     if (x_slices && (!prologue || x_slices < 1 || x_slices > 64))
         return set_error("matvec_batch: X as unfolded partial sums (dims[7]=%lld) takes a prologue and 1 to 64 slices", (long long)k.desc.dims[7]);
     if (prologue) {
@@ -1575,13 +1662,17 @@ int bind_matvec_batch(ksh_kernel &k)
         k.info.n_inputs = ni;
         if (x_slices) k.in_bytes[1] = (size_t)x_slices * mat * (prologue == 3 ? 2 : 1);
     }
+    if (cut) {
+        const int ni = k.info.n_inputs++;
+        k.in_bytes[ni] = (size_t)batch * 4; k.in_align[ni] = 4;
+    }
     // f16 copy of X plus the min-term operand (32 halves per token and superblock)
     k.scratch_bytes = ((size_t)((batch + 31) / 32 * 32) * cols * 2 + (size_t)batch * (cols / 256) * 64) * (f32x ? 2 : 1);
     // schedule: nr0 = weight rows per workgroup.  32 = the small-batch form (Q4_K, up to 64 tokens: the default
     // there), 128 = the 128 x 128 tile.
     const uint32_t want = k.desc.sched.nr0;
     if (want && want != 32 && want != BN) return set_error("matvec_batch: unsupported schedule nr0=%u (32 or %d)", want, BN);
-    const bool can_skinny = !q6 && batch <= kSkinnyMaxBatch && n_mat == 1 && !unfolded;
+    const bool can_skinny = !q6 && batch <= kSkinnyMaxBatch && n_mat == 1 && !unfolded && !cut;
     if (want == 32 && !can_skinny) return set_error("matvec_batch: the small-batch form takes Q4_K weights and up to %d tokens", kSkinnyMaxBatch);
     // (long rows of a short matrix leave the small-batch form 64 workgroups with four superblocks per wave: from 33
     // tokens on the tile over K slices is faster there -- 2048 x 8192 at 63 tokens: 27.5 us against 41.0)
@@ -1595,23 +1686,15 @@ int bind_matvec_batch(ksh_kernel &k)
         k.launch = launch_mul_mm;
         return 0;
     }
-    // Few tiles (a prompt of a few hundred tokens, or a narrow matrix): the superblocks of a row are split into K
-    // slices and, for f32 activations, the hi and the lo part become workgroups of the same launch, until the grid is
-    // about one workgroup per compute unit; every slice stores its partial sums and a second launch adds them in a
-    // fixed order.  sched.k_split names the slice count (a divisor of cols / 256; 1 = none).
-    const int64_t row_tiles = (rows + BN - 1) / BN + (rows1 + BN - 1) / BN + (rows2 + BN - 1) / BN;
-    const int64_t nsb = cols / 256;
+    // K slices (mm_k_slices): workgroups of one launch, every slice storing its partial sums, and a second launch that adds
+    // them.  sched.k_split names the slice count (a divisor of cols / 256; 1 = none).
+    const int64_t row_tiles = mm_row_tiles(k.desc), nsb = cols / 256;
     int64_t ks = 1;
-    if (k.desc.sched.k_split) {
+    if (k.desc.sched.k_split && !cut) {
         ks = k.desc.sched.k_split;
         if (nsb % ks) return set_error("matvec_batch: k_split=%lld does not divide the %lld superblocks of a row", (long long)ks, (long long)nsb);
-    } else {
-        // (a slice of one superblock is all prologue; the workgroups are counted with the token tile they will have, and
-        // f32 rows of more than half a prompt pass as that many: how a row's sum is cut does not depend on which pass of its
-        // prompt the row is in)
-        const int64_t counted = f32x ? std::min<int64_t>(batch, kPrefillPass / 2) : batch;
-        auto workgroups = [&](int64_t s) { const int64_t tm_s = mm_tile_tokens(k.desc, counted, s); return ((counted + tm_s - 1) / tm_s) * row_tiles * s; };
-        while (nsb % (ks * 2) == 0 && nsb / (ks * 2) >= 2 && workgroups(ks * 2) <= 256) ks *= 2;
+    } else if (!cut) {
+        ks = mm_k_slices(q6, f32x, (int)row_tiles, (int)nsb, (int)batch);
     }
     const bool z_form = unfolded || ks > 1;
     k.variant = z_form ? (int)(ks << 1) : 0;
@@ -1622,12 +1705,13 @@ int bind_matvec_batch(ksh_kernel &k)
         k.out_bytes[0] = (size_t)ks * batch * rows_all * 4; k.out_align[0] = 16;
         k.info.n_outputs = 1 + keep;
     }
-    const int tm = mm_tile_tokens(k.desc, batch, ks);
+    const int tm = mm_tile_tokens(q6, f32x, (int)row_tiles, (int)batch, (int)ks);
     set_launch(k, (uint32_t)((batch + tm - 1) / tm), (uint32_t)row_tiles, z_form ? (uint32_t)ks : 1, kThreadsMM,
                (uint32_t)(tm == 64 ? kLdsBytes64 : kLdsBytes));
     k.info.sched.tg = kThreadsMM; k.info.sched.nsg = kThreadsMM / 64; k.info.sched.nr0 = BN; k.info.sched.k_split = (uint32_t)ks; k.info.sched.lds_tile = KS;
     set_name(k, "mul_mm_%s_%dx%dx%d%s%s%s%s", q6 ? "q6k" : "q4k", BM, BN, KS, f32x ? "_f32x" : "", z_form ? "_kz" : "", n_mat == 3 ? "_x3" : n_mat == 2 ? "_x2" : "",
              prologue == 1 ? "_rms" : prologue == 2 ? "_addrms" : prologue == 3 ? "_gelu" : "");
+    if (cut) { char nm[64]; snprintf(nm, sizeof(nm), "%s", k.info.name); set_name(k, "%s_cut", nm); }
     if (unfolded) { char nm[64]; snprintf(nm, sizeof(nm), "%s", k.info.name); set_name(k, "%s_unfolded", nm); }
     k.launch = launch_mul_mm;
     return 0;

@@ -477,6 +477,19 @@ int bind_sdpa(ksh_kernel &k)
         k.in_bytes[0] = (size_t)n_tok * n_q * hd * 4;
         k.in_bytes[1] = k.in_bytes[2] = kvb;
         k.in_bytes[3] = 12;
+        // dims[6], dims[7]: tokens of several prompts, each with its own record and its slot of the pools
+        const int64_t pool_slots = d[6], slot_stride = d[7];
+        if (pool_slots) {
+            if (pool_slots < 0 || pool_slots > 65535 || slot_stride < 0 || (slot_stride && ((size_t)slot_stride < kvb || slot_stride % 2)))
+                return set_error("sdpa_batch: pool slots=%lld, slot stride %lld", (long long)pool_slots, (long long)slot_stride);
+            if (!lanes || (hd != 256 && hd != 512) || n_tok <= 16 || k.desc.sched.vec == 1 || k.desc.sched.vec == 3)
+                return set_error("sdpa_batch: tokens that name their pool slot take the matrix-core form (more than 16 tokens, heads of 256 or 512, up to 8 q heads per kv head)");
+            k.info.n_inputs = 5;
+            k.in_bytes[1] = k.in_bytes[2] = (size_t)(pool_slots - 1) * (slot_stride ? (size_t)slot_stride : kvb) + kvb;
+            k.in_bytes[3] = (size_t)n_tok * 16;
+            k.in_bytes[4] = (size_t)n_tok * 4;
+            k.in_align[4] = 4;
+        }
         k.out_bytes[0] = (size_t)n_tok * n_q * nwg * (hd + 2) * 4;
         k.out_bytes[1] = (size_t)n_tok * n_q * hd * 4;
         k.out_align[1] = 4;

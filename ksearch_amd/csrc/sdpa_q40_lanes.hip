@@ -1707,6 +1707,11 @@ int launch_bound(const ksh_kernel &k, const LaunchArgs &a, hipStream_t st)
         p.kv_shared = 1;
         if (own_parts) {
             p.meta = (const float *)a.in[3];
+            if (k.desc.dims[6]) {   // tokens of several prompts
+                p.kv_shared = 0;
+                p.slot_ids = (const float *)a.in[4];
+                p.slot_stride = (size_t)k.desc.dims[7];
+            }
             p.balance = 0;
             p.mode = kModePart;
             if (hd == 512)   // two workgroups per kv head, each with half of the V dimensions
@@ -1789,7 +1794,7 @@ int bind_sdpa_lanes(ksh_kernel &k, int nwg, int n_slots)
     // cost (1024 tokens from an empty cache: 78 us against 422; heads of 512: 226 against 778): the default there;
     // vec = 3 asks for the register form, vec = 2 with up to 64 tokens for the form that deals the partitions by length.
     const bool long_batch = k.desc.kind == KSH_SDPA_BATCH && (hd == 256 || hd == 512) && n_q / n_kv <= 8 && n_slots > 16;
-    if (long_batch && ((k.desc.sched.vec == 2 && !batch_fits) || k.desc.sched.vec == 0)) {
+    if (long_batch && ((k.desc.sched.vec == 2 && (!batch_fits || k.desc.dims[6])) || k.desc.sched.vec == 0)) {
         if (k.desc.sched.lds_tile && k.desc.sched.lds_tile != 32) return set_error("sdpa_batch: the matrix-core form of a long chunk takes tiles of 32 rows (lds_tile=%u)", k.desc.sched.lds_tile);
         k.scratch_bytes = (((size_t)n_slots * n_kv * 4 + 15) & ~(size_t)15) + (size_t)n_slots * 16;
         // (heads of 512: two workgroups per kv head, each with all of the scores and half of the V dimensions)

@@ -40,6 +40,10 @@ struct Active {
 
 }  // namespace
 
+namespace ksh {
+PrefillSlotsFn g_prefill_slots = nullptr;
+}
+
 struct ksh_serve {
     ksh_gemma4 *model = nullptr;
     ksh_kvpool *pool = nullptr;
@@ -192,7 +196,48 @@ void decode_round(ksh_serve *s)
     }
 }
 
-// scheduler.rs:243-303
+// one request's share of a prefill round
+struct Share {
+    Active *a;
+    int n;
+};
+
+// The shares' tokens: those that the model takes so as one pass over the weights, the others slot by slot as the
+// reference runs them.
+void prefill_shares(ksh_serve *s, const Share *shares, size_t count)
+{
+    std::vector<uint8_t> taken(count, 0);
+    bool failed = false;
+    if (count > 1 && g_prefill_slots && !(s->cfg.use_graph & 2)) {
+        std::vector<int32_t> slots(count);
+        std::vector<const uint32_t *> tokens(count);
+        std::vector<int> n(count);
+        for (size_t i = 0; i < count; i++) {
+            slots[i] = shares[i].a->slot;
+            tokens[i] = shares[i].a->prompt.data() + shares[i].a->cursor;
+            n[i] = shares[i].n;
+        }
+        failed = g_prefill_slots(s->model, s->pool, slots.data(), tokens.data(), n.data(), (int)count, taken.data()) != 0;
+    }
+    const std::string why = failed ? ksh_last_error() : "";
+    for (size_t i = 0; i < count; i++) {
+        Active &a = *shares[i].a;
+        const int take = shares[i].n;
+        if ((taken[i] && failed) ||
+            (!taken[i] && (ksh_gemma4_bind_slot(s->model, s->pool, a.slot) ||
+                       ksh_gemma4_prefill_chunk(s->model, a.prompt.data() + a.cursor, take, s->cfg.use_graph))) ||
+            ksh_kvpool_bump_len_by(s->pool, a.slot, take, nullptr)) {
+            push_error(s, a.id, taken[i] && failed ? why : ksh_last_error());
+            finish(s, a, KSH_FINISH_ERROR);
+            continue;
+        }
+        a.cursor += (size_t)take;
+        if (a.cursor >= a.prompt.size() - 1) enter_decode(a);
+    }
+}
+
+// scheduler.rs:243-303.  The shares of the round's budget are dealt as there and go through the layers together, as many
+// to a pass as it takes tokens.
 void prefill_round(ksh_serve *s)
 {
     const size_t n = s->active.size();
@@ -200,6 +245,7 @@ void prefill_round(ksh_serve *s)
     const bool decoding = std::any_of(s->active.begin(), s->active.end(), [](const Active &a) { return !a.finished && !a.prefill; });
     size_t budget = (size_t)std::max(s->cfg.prefill_tokens_per_tick, s->cfg.prefill_chunk);
     size_t idx = s->prefill_cursor % n;
+    std::vector<Share> shares;
     for (size_t i = 0; i < n && budget; i++) {
         Active &a = s->active[idx];
         idx = (idx + 1) % n;
@@ -210,18 +256,15 @@ void prefill_round(ksh_serve *s)
         // small chunks while something decodes; otherwise the whole budget
         const size_t cap = decoding ? (size_t)s->cfg.prefill_chunk : budget;
         const size_t take = std::min({budget, cap, prefill_end - a.cursor});
-        if (ksh_gemma4_bind_slot(s->model, s->pool, a.slot) ||
-            ksh_gemma4_prefill_chunk(s->model, a.prompt.data() + a.cursor, (int)take, s->cfg.use_graph) ||
-            ksh_kvpool_bump_len_by(s->pool, a.slot, (int)take, nullptr)) {
-            push_error(s, a.id, ksh_last_error());
-            finish(s, a, KSH_FINISH_ERROR);
-            continue;
-        }
+        shares.push_back(Share{&a, (int)take});
         budget -= take;
-        a.cursor += take;
-        if (a.cursor >= prefill_end) enter_decode(a);
     }
     s->prefill_cursor = idx;
+    for (size_t i0 = 0, i1; i0 < shares.size(); i0 = i1) {
+        int total = 0;
+        for (i1 = i0; i1 < shares.size() && (i1 == i0 || total + shares[i1].n <= kPrefillPass); i1++) total += shares[i1].n;
+        prefill_shares(s, shares.data() + i0, i1 - i0);
+    }
 }
 
 // scheduler.rs:294-303 (reap_finished)

@@ -281,3 +281,38 @@ def test_draws_from_the_narrowed_logits_are_the_host_samplers(ctx, model, temper
     rows = m.round_logits(4)
     assert got == [hip.sample_softcap_min_p(rows[i], cfg["softcap"], temps[i], min_p, seeds[i]) for i in range(4)]
     pool.close()
+
+
+@pytest.mark.parametrize("lens", [(90, 1, 130, 66, 2, 65), (225, 225), (9, 129)])
+def test_prompts_prefilled_in_one_pass_fill_the_caches_of_passes_alone(ctx, lens):
+    """The prefilling requests of a tick with more than 64 tokens share one pass over the weights (heads of 256 and 512; 65
+    prompt tokens are 64 and the first decode input: a pass alone).  Every slot's K / V rows are the bytes of the prompt
+    alone -- slots, positions, windows and the K slices of every GEMM are each prompt's own -- and nothing is written
+    behind them."""
+    cfg = dict(synth.GEMMA4_TINY, hd_swa=256, hd_full=512, max_seq=256, sliding_window=40)
+    w = synth.gemma4_weights(cfg, 611, oracle.quantize_q4k, oracle.quantize_q6k, ffn=FFN, swa_pattern=PATTERN, std=0.05,
+                             q6k_tensors=((1, "wdown"), (2, "wv")))
+    m = hip.Gemma4(ctx, cfg, w)
+    prompts = prompts_of(cfg, lens, 705)
+    pool = make_pool(ctx, cfg, len(lens))
+    sv = hip.Serve(m, pool, slots=len(lens), eos=NO_EOS)
+    for p in prompts:
+        sv.submit(p, 2)
+    assert sv.tick() == []
+    assert [pool.seq_len(i) for i in range(len(lens))] == [n - 1 for n in lens]
+    owners = cfg["n_layers"] - cfg["shared_kv_layers"]
+    for slot, p in enumerate(prompts):
+        m.bind_slot(None, 0)
+        m.reset()
+        m.prefill_chunk(p[:-1])
+        for layer in range(owners):
+            row = cfg["n_kv"] * (cfg["hd_swa"] if PATTERN[layer] else cfg["hd_full"]) // 32 * 18
+            for which, buf in ((0, pool.k_buf(slot, layer)), (1, pool.v_buf(slot, layer))):
+                if len(p) > 1:
+                    own = hip.Buffer(ctx, hip.lib().ksh_gemma4_kv(m.h, layer, which), owned=False)
+                    assert np.array_equal(ctx.read_bytes(buf, row * (len(p) - 1)), ctx.read_bytes(own, row * (len(p) - 1))), (slot, layer, which)
+                assert not np.any(ctx.read_bytes(buf, row, row * (len(p) - 1)))
+    sv.close()
+    m.bind_slot(None, 0)
+    pool.close()
+    m.close()
