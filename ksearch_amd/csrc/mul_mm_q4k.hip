@@ -763,7 +763,8 @@ __global__ __launch_bounds__(kThreadsMM, TM == 64 ? 2 : 1) void q_mul_mm_kernel(
             if (CUT) {
                 static_assert(MW == 1, "one token tile per wave");
                 cut_left -= 1;
-                // (rows past the batch neither end nor start: their sums are never stored)
+                // (rows past the batch never end.  1 / s is a power of two: it can wait for the last slice)
+                const bool last = sb + 1 == nsb;
                 const bool live = t0 + wm * 32 + lm < p.batch;
                 uint32_t ends = (uint32_t)__ballot(live && cut_left == 0), first = (uint32_t)__ballot(sb + 1 == cut_len);
                 if (cut_left == 0) cut_left = cut_len;
@@ -781,19 +782,20 @@ __global__ __launch_bounds__(kThreadsMM, TM == 64 ? 2 : 1) void q_mul_mm_kernel(
                         if (r < p.rows) {
                             float *y = p.Y + (size_t)row * ystride + r;
 #pragma unroll
-                            for (int i0 = 0; i0 < 16; i0 += 4) {
-                                float sum[4], inv[4];
+                            for (int i0 = 0; i0 < 16; i0 += 8) {
+                                float sum[8];
 #pragma unroll
-                                for (int i = 0; i < 4; i++) {
-                                    const int tr = 2 * i0 + i;
+                                for (int i = 0; i < 8; i++) {
+                                    const int tr = 2 * i0 + 8 * (i / 4) + (i & 3);
                                     sum[i] = 0.f;
-                                    inv[i] = p.inv_s[min(row + tr, p.batch - 1)];
                                     if ((ends & ~first) & (1u << tr)) sum[i] = y[(size_t)tr * ystride];
                                 }
 #pragma unroll
-                                for (int i = 0; i < 4; i++) {
-                                    const int tr = 2 * i0 + i;
-                                    if (ends & (1u << tr)) y[(size_t)tr * ystride] = sum[i] + F[0][nt][i0 + i] * inv[i];
+                                for (int i = 0; i < 8; i++) {
+                                    const int tr = 2 * i0 + 8 * (i / 4) + (i & 3);
+                                    sum[i] += F[0][nt][i0 + i];
+                                    if (last) sum[i] *= p.inv_s[min(row + tr, p.batch - 1)];
+                                    if (ends & (1u << tr)) y[(size_t)tr * ystride] = sum[i];
                                 }
                             }
                         }
