@@ -169,6 +169,15 @@ __global__ __launch_bounds__(256) void mm_prep_x_f32_kernel(const float *__restr
 // subnormal f16 for elements below 2^-13 of the row's largest; what that costs is below 2^-35 of the largest.  The
 // sums of a sub-block are those of hi + lo, split in two halves as for bf16 rows; 1 / s goes to inv_s[row] for the
 // tile's last step.
+// Which row workgroup b prepares.  Eight neighbouring rows share every 128-byte line of the fragments, 16 bytes each, and
+// workgroups go to the eight dies in turn: taken as they come, a line was written in eight pieces from eight L2s.  Eight
+// rows in turn on one die meet in its L2 (2048 rows: 12288 columns 133 -> 102 us, 1536 columns 13.7 -> 11.2; 82 with the row kept instead of produced twice).
+__device__ __forceinline__ int prep_row(int b, int rows)
+{
+    const int turn = b >> 3;
+    return b < rows / 64 * 64 ? ((turn >> 3) * 8 + (b & 7)) * 8 + (turn & 7) : b;
+}
+
 template <int MODE>
 __global__ __launch_bounds__(1024) void mm_prep_rows_kernel(const float *__restrict__ X, const float *__restrict__ P0, const float *P1,
                                                              const float *__restrict__ P2, float *x_out, _Float16 *__restrict__ Xf_hi,
@@ -180,7 +189,7 @@ __global__ __launch_bounds__(1024) void mm_prep_rows_kernel(const float *__restr
     // cols (MODE 3: 2 * cols, gate | up side by side, and `up` is read from there); the slices are added here in the
     // fold's order
     __shared__ float red[3][16];
-    const int t = blockIdx.x, lane = threadIdx.x & 63, wave = threadIdx.x >> 6, nw = blockDim.x >> 6;
+    const int t = prep_row(blockIdx.x, gridDim.x), lane = threadIdx.x & 63, wave = threadIdx.x >> 6, nw = blockDim.x >> 6;
     auto ld8 = [](const float *p, float (&v)[8]) __attribute__((always_inline)) {
         const f32x4_t a = reinterpret_cast<const f32x4_t *>(p)[0], b = reinterpret_cast<const f32x4_t *>(p)[1];
         v[0] = a.x; v[1] = a.y; v[2] = a.z; v[3] = a.w; v[4] = b.x; v[5] = b.y; v[6] = b.z; v[7] = b.w;
@@ -245,16 +254,31 @@ __global__ __launch_bounds__(1024) void mm_prep_rows_kernel(const float *__restr
         }
     };
     const int octets = cols / 8;
-    const bool one_trip = octets <= (int)blockDim.x;
-    float kept[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+    // (rows of up to KEEP octets a thread are produced once and kept; the norms' sums want one)
+    constexpr int KEEP = MODE == 1 || MODE == 2 ? 1 : 2;
+    const bool keep = octets <= KEEP * (int)blockDim.x;
+    float kept[KEEP][8];
     float s = 1.0f;
     if (inv_s) {
-        // the row's largest magnitude (rows of one trip keep their elements; longer ones are produced again below)
+        // the row's largest magnitude (rows too long to keep are produced again below)
         float m = 0.f;
-        for (int j = threadIdx.x; j < octets; j += blockDim.x) {
-            produce(j, kept);
+        if (keep) {
 #pragma unroll
-            for (int i = 0; i < 8; i++) m = fmaxf(m, fabsf(kept[i]));
+            for (int u = 0; u < KEEP; u++) {
+                const int j = threadIdx.x + u * blockDim.x;
+                if (j < octets) {
+                    produce(j, kept[u]);
+#pragma unroll
+                    for (int i = 0; i < 8; i++) m = fmaxf(m, fabsf(kept[u][i]));
+                }
+            }
+        } else {
+            for (int j = threadIdx.x; j < octets; j += blockDim.x) {
+                float f[8];
+                produce(j, f);
+#pragma unroll
+                for (int i = 0; i < 8; i++) m = fmaxf(m, fabsf(f[i]));
+            }
         }
         m = wave_max(m);
         if (lane == 0) red[2][wave] = m;
@@ -265,14 +289,7 @@ __global__ __launch_bounds__(1024) void mm_prep_rows_kernel(const float *__restr
         s = as_f32((263u - e) << 23);
         if (threadIdx.x == 0) inv_s[t] = as_f32((e - 9u) << 23);
     }
-    for (int j = threadIdx.x; j < octets; j += blockDim.x) {
-        float f[8];
-        if (inv_s && one_trip) {
-#pragma unroll
-            for (int i = 0; i < 8; i++) f[i] = kept[i];
-        } else {
-            produce(j, f);
-        }
+    auto write = [&](int j, const float (&f)[8]) __attribute__((always_inline)) {
         h8 oh, ol;
         float fh[8], fl[8];
         const float lo_up = inv_s ? 1.0f : 2048.0f;
@@ -311,6 +328,17 @@ __global__ __launch_bounds__(1024) void mm_prep_rows_kernel(const float *__restr
                 dst[part][16 + jj] = lo;
                 dst[part][24 + jj] = (_Float16)0.f;
             }
+        }
+    };
+    if (inv_s && keep) {
+#pragma unroll
+        for (int u = 0; u < KEEP; u++)
+            if ((int)(threadIdx.x + u * blockDim.x) < octets) write(threadIdx.x + u * blockDim.x, kept[u]);
+    } else {
+        for (int j = threadIdx.x; j < octets; j += blockDim.x) {
+            float f[8];
+            produce(j, f);
+            write(j, f);
         }
     }
 }
@@ -1524,7 +1552,10 @@ int launch_mul_mm(const ksh_kernel &k, const LaunchArgs &a, hipStream_t st)
     // the sums of the lo parts (which the tile does not use)
     const bool tile = k.variant != 1;
     float *inv_s = f32x && tile ? reinterpret_cast<float *>(SxA_lo) : nullptr;
-    const dim3 pg((unsigned)batch), pb((unsigned)std::min((cols / 8 + 63) / 64 * 64, 1024));     // whole waves: the row-wide reductions read every lane
+    // whole waves: the row-wide reductions read every lane.  An octet of the row a thread, from 1024 octets on two (12288
+    // columns: 768 threads) where the tile keeps them
+    const int octets = cols / 8, pb1 = (octets + 63) / 64 * 64;
+    const dim3 pg((unsigned)batch), pb((unsigned)std::min(pb1 > 1024 && inv_s ? (octets / 2 + 63) / 64 * 64 : pb1, 1024));
     if (prologue) {
         // the rows' producer runs inside the preparation: in = W, X, [W1, W2,] then the prologue's operands
         const int xs = (int)k.desc.dims[7];
