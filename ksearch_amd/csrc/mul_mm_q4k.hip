@@ -29,6 +29,7 @@
 // stores are contiguous along Y's row index.  K advances 64 columns (one
 // 64-element group: 32 quant bytes per row) per step through a double-buffered
 // LDS stage, with the next step's global loads in flight under the MFMAs.
+#include <algorithm>
 #include <type_traits>
 
 #include "ksh_device.hpp"
@@ -343,6 +344,19 @@ __global__ __launch_bounds__(1024) void mm_prep_rows_kernel(const float *__restr
     }
 }
 
+// eight bf16 of a row as f16, in the order of the weights beside them (kperm)
+__device__ __forceinline__ h8 from_bf16(h8 raw)
+{
+    const u32x4_t w = __builtin_bit_cast(u32x4_t, raw);
+    h8 o;
+#pragma unroll
+    for (int i = 0; i < 4; i++) {
+        o[kperm(2 * i)] = (_Float16)as_f32(w[i] << 16);
+        o[kperm(2 * i + 1)] = (_Float16)as_f32(w[i] & 0xFFFF0000u);
+    }
+    return o;
+}
+
 struct MmParams {
     const uint8_t *W;
     const _Float16 *Xf, *SxA;   // fragment-ordered f16 activations (mm_prep_x_kernel), sums of x
@@ -365,34 +379,76 @@ struct MmParams {
     const float *cut_as;
 };
 
-// Tokens per workgroup of the tile.  64 (Q4_K): up to 64 tokens (the other half of a 128-token tile would be empty
-// rows), and wherever the 128-token tiles and their K slices are fewer than the compute units (bf16 activations) or
-// than twice the compute units (f32 activations, whose tile runs two products per converted weight) -- two
-// workgroups share a compute unit then, and twice as many of them fill the chip.  Beyond that the 128-token tile
-// (bf16, cfg2: 33.7 us against 40.3 with 64-token tiles; f32, prompts of 256 / 1024 / 4000 tokens through cfg4's
-// model: 5.05 / 14.1 / 67.7 ms with this rule, 5.07 / 14.25 / 68.0 with 64-token tiles throughout, 5.3 / 14.9 / 72.7
-// with 128-token tiles from 65 tokens on).
-__host__ __device__ constexpr int mm_tile_tokens(bool q6, bool f32x, int row_tiles, int batch, int ks)
+// F32 activations: tokens per workgroup of the tile.  64 (Q4_K): up to 64 tokens (the other half of a 128-token tile would
+// be empty rows), and wherever the 128-token tiles and their K slices are fewer than twice the compute units (the tile
+// runs two products per converted weight) -- two workgroups share a compute unit then, and twice as many of them fill the
+// chip.  Beyond that the 128-token tile (prompts of 256 / 1024 / 4000 tokens through cfg4's model: 5.05 / 14.1 / 67.7 ms
+// with this rule, 5.07 / 14.25 / 68.0 with 64-token tiles throughout, 5.3 / 14.9 / 72.7 with 128-token tiles from 65
+// tokens on).
+__host__ __device__ constexpr int mm_tile_tokens(bool q6, int row_tiles, int batch, int ks)
 {
     if (q6) return 128;
-    return batch <= 64 || (int64_t)((batch + BM - 1) / BM) * row_tiles * ks < (f32x ? 512 : 256) ? 64 : 128;
+    return batch <= 64 || (int64_t)((batch + BM - 1) / BM) * row_tiles * ks < 512 ? 64 : 128;
 }
 
-// Few tiles (a prompt of a few hundred tokens, or a narrow matrix): the nsb superblocks of a row are split into this many
-// K slices, until the grid is about one workgroup per compute unit; every slice has its own sum and the sums are added
-// in a fixed order.  (A slice of one superblock is all prologue; the workgroups are counted with the token tile they will
-// have, and f32 rows of more than half a prompt pass as that many: how a row's sum is cut does not depend on which pass
-// of its prompt the row is in.)
-__host__ __device__ constexpr int mm_k_slices(bool q6, bool f32x, int row_tiles, int nsb, int batch)
+// F32 activations, few tiles (a prompt of a few hundred tokens, or a narrow matrix): the nsb superblocks of a row are split
+// into this many K slices, until the grid is about one workgroup per compute unit; every slice has its own sum and the
+// sums are added in a fixed order.  (A slice of one superblock is all prologue; the workgroups are counted with the token
+// tile they will have, and rows of more than half a prompt pass as that many: how a row's sum is cut does not depend on
+// which pass of its prompt the row is in.)
+__host__ __device__ constexpr int mm_k_slices(bool q6, int row_tiles, int nsb, int batch)
 {
-    const int counted = f32x && batch > kPrefillPass / 2 ? kPrefillPass / 2 : batch;
+    const int counted = batch > kPrefillPass / 2 ? kPrefillPass / 2 : batch;
     int ks = 1;
     while (nsb % (ks * 2) == 0 && nsb / (ks * 2) >= 2) {
-        const int tm = mm_tile_tokens(q6, f32x, row_tiles, counted, ks * 2);
+        const int tm = mm_tile_tokens(q6, row_tiles, counted, ks * 2);
         if ((int64_t)((counted + tm - 1) / tm) * row_tiles * ks * 2 > 256) break;
         ks *= 2;
     }
     return ks;
+}
+
+// Bf16 activations: token tile and K slices (of any number of superblocks) of the tile by what the launches are made of, in
+// us, fitted to 300 .. 12288 rows of 1024 .. 8192 columns, 2 .. 2048 tokens, every slice count:
+//   a round of 128-token tiles (one workgroup a compute unit)        5 + 2.4 per superblock of the slice
+//   64-token tiles, one / two workgroups a compute unit              4.2 + 2.0 / 6 + 2.9
+//   the fold                                                         2.5 + the partial sums, written and read, at 4 TB/s
+// The tile of the smallest sum is within 5 % of the best of all (tile, slices) at those shapes.  Against slices by powers
+// of two until the chip is full: 333 tokens, 1536 x 6144 four -> six slices, 29.8 -> 25.4 us (Q6_K); 300 x 7936 (31
+// superblocks) one -> eight, 95 -> 27 at 512 tokens; 12288 x 4096 at 100 tokens one of 64 -> two of 128, 35.3 -> 29.2.
+struct MmPlan {
+    int tm, ks;
+    float us;
+};
+MmPlan mm_plan_bf16(bool q6, int row_tiles, int nsb, int64_t batch, int64_t rows_all, int ks_given)
+{
+    MmPlan best{128, 1, 1e30f};
+    const int ks_max = std::min(nsb, 64);
+    for (int tm = q6 ? 128 : 64; tm <= 128; tm += 64)
+        for (int ks = ks_given ? ks_given : 1; ks <= (ks_given ? ks_given : ks_max); ks++) {
+            const int64_t w = (batch + tm - 1) / tm * row_tiles * ks;
+            const float sb = (float)((nsb + ks - 1) / ks);
+            float us = tm == 128 ? (float)((w + 255) / 256) * (5.f + 2.4f * sb) : w <= 256 ? 4.2f + 2.0f * sb : (float)((w + 511) / 512) * (6.f + 2.9f * sb);
+            if (ks > 1) us += 2.5f + (float)ks * (float)(batch * rows_all) * 2e-6f;
+            if (us < best.us) best = MmPlan{tm, ks, us};
+        }
+    return best;
+}
+
+// The small-batch form beside it (bf16): a workgroup of eight waves per 32 rows, superblocks dealt to the waves; the numbers
+// carry what the tile's preparation and launch take more (2.4).
+float mm_skinny_us(int64_t rows, int nsb, int64_t batch)
+{
+    const float fill = (float)((rows + 31) / 32) / 256.f;
+    return 1.8f + (batch <= 32 ? 3.4f : 5.5f) * std::max(1.f, (float)nsb / 8.f) * std::max(1.f, 2.f * fill - 1.f);
+}
+
+// Bf16 rows of Q6_K products as they are (the kernel's ROWS form): the conversion between the matrix instructions costs 0.42
+// us per superblock and round, the preparation a launch (2.5 us) and its pass over X (12288 x 4096: 2048 tokens 337 us
+// against 308, 50 tokens 32.4 against 33.2; 2048 x 8192, 2048 tokens 107.9 against 116.6).
+bool mm_rows_direct(int64_t workgroups, int sb_per_slice, int64_t batch, int64_t cols)
+{
+    return 0.42f * (float)((workgroups + 255) / 256 * sb_per_slice) < 2.5f + (float)(batch * cols) * 1.1e-6f;
 }
 
 __device__ __forceinline__ uint32_t pair_f16(uint32_t masked, uint32_t sc)
@@ -442,7 +498,10 @@ constexpr size_t kLdsBytes64 = 2 * (size_t)(kLdsMain + (64 + BN) * PITCH2) * 2 +
 // depend on its length.  The workgroup takes all of K, and where a row's slice ends its sum is added to Y and starts
 // again from zero: the bits of those launches from one that fills the chip (a read and a write of the tile's results
 // per slice end, from L2).
-template <bool Q6, int TM, bool LO, bool CUT = false>
+// ROWS = true (bf16 activations, Q6_K weights: no sums of x are wanted): the A operands come from the rows of X as they are
+// and the multiplying waves convert them, eight values of a row a lane, between their matrix instructions -- no
+// preparation launch (mm_rows_direct; 333 tokens, 1536 x 6144 in six slices: 28.9 -> 25.4 us).
+template <bool Q6, int TM, bool LO, bool CUT = false, bool ROWS = false>
 __global__ __launch_bounds__(kThreadsMM, TM == 64 ? 2 : 1) void q_mul_mm_kernel(MmParams p)
 {
     constexpr int MT = TM / 64, kLdsMinT = (TM + BN) * PITCH2;
@@ -467,8 +526,8 @@ __global__ __launch_bounds__(kThreadsMM, TM == 64 ? 2 : 1) void q_mul_mm_kernel(
     size_t ystride = (size_t)p.rows;
     if (p.ksplit) {
         const int slice = blockIdx.z;
-        nsb = nsb_row / p.ksplit;
-        sb0 = slice * nsb;
+        sb0 = nsb_row * slice / p.ksplit;
+        nsb = nsb_row * (slice + 1) / p.ksplit - sb0;
         p.Y = p.Y_parts + (size_t)blockIdx.z * p.batch * rows_all + ycol;   // partial sums: all matrices' columns side by side
         ystride = (size_t)rows_all;
     }
@@ -675,11 +734,13 @@ __global__ __launch_bounds__(kThreadsMM, TM == 64 ? 2 : 1) void q_mul_mm_kernel(
     // set of hi and lo fragments, refilled for the next step -- a step is long against the way to the cache).
     const int ntt = (p.batch + 31) / 32;
     const h8 *xa[MW];
+    const uint16_t *xrow = reinterpret_cast<const uint16_t *>(p.Xf) + (size_t)min(t0 + wm * 32 + lm, p.batch - 1) * p.cols + (size_t)sb0 * 256 + lk;   // ROWS
 #pragma unroll
     for (int mt = 0; mt < MW; mt++)
         xa[mt] = reinterpret_cast<const h8 *>(p.Xf) + ((size_t)min((t0 + (wm * MW + mt) * 32) / 32, ntt - 1) * (p.cols / 16) + (size_t)sb0 * 16) * 64 + lane;
     const ptrdiff_t lo_delta = LO ? reinterpret_cast<const h8 *>(p.Xf_lo) - reinterpret_cast<const h8 *>(p.Xf) : 0;
     auto afrag = [&](int mt, int step, int ks) __attribute__((always_inline)) {
+        if (ROWS) return *reinterpret_cast<const h8 *>(xrow + step * KS + 16 * ks);      // (bf16 as yet)
         return xa[mt][(ptrdiff_t)(step * (KS / 16) + ks) * 64];
     };
     auto afrag_lo = [&](int mt, int step, int ks) __attribute__((always_inline)) {
@@ -700,7 +761,7 @@ __global__ __launch_bounds__(kThreadsMM, TM == 64 ? 2 : 1) void q_mul_mm_kernel(
     int cut_len = nsb, cut_left = nsb;
     if (CUT) {
         const int row_tiles = (rows_of[0] + BN - 1) / BN + (rows_of[1] + BN - 1) / BN + (rows_of[2] + BN - 1) / BN;
-        cut_len = cut_left = nsb / mm_k_slices(Q6, true, row_tiles, nsb, (int)p.cut_as[min(t0 + wm * 32 + lm, p.batch - 1)]);
+        cut_len = cut_left = nsb / mm_k_slices(Q6, row_tiles, nsb, (int)p.cut_as[min(t0 + wm * 32 + lm, p.batch - 1)]);
     }
     ARegs a0, a1;
     fetch_a(0, a0);
@@ -744,7 +805,7 @@ __global__ __launch_bounds__(kThreadsMM, TM == 64 ? 2 : 1) void q_mul_mm_kernel(
 #pragma unroll
                 for (int nt = 0; nt < NW_; nt++)
                     // a superblock's first product starts from the constant zero: no pass over the accumulators to clear them
-                    Cp[mt][nt] = __builtin_amdgcn_mfma_f32_32x32x16_f16(A.a[mt][ks], b[nt], (g == 0 && ks == 0) ? kZero16 : Cp[mt][nt], 0, 0, 0);
+                    Cp[mt][nt] = __builtin_amdgcn_mfma_f32_32x32x16_f16(ROWS ? from_bf16(A.a[mt][ks]) : A.a[mt][ks], b[nt], (g == 0 && ks == 0) ? kZero16 : Cp[mt][nt], 0, 0, 0);
             if (LO) {
 #pragma unroll
                 for (int mt = 0; mt < MW; mt++)
@@ -1342,8 +1403,16 @@ __global__ __launch_bounds__(256) void mm_parts_fold_kernel(const float *__restr
     const int rows_all = rows0 + rows1 + rows2, n = batch * rows_all;
     const int i = blockIdx.x * 256 + threadIdx.x;
     if (i >= n) return;
+    // (eight slices in flight: one at a time, 29 slices of 8 x 517 took 8 us)
     float s = part[i];
-    for (int k = 1; k < slices; k++) s += part[(size_t)k * n + i];
+    for (int k0 = 1; k0 < slices; k0 += 8) {
+        float v[8];
+#pragma unroll
+        for (int u = 0; u < 8; u++) v[u] = part[(size_t)min(k0 + u, slices - 1) * n + i];
+#pragma unroll
+        for (int u = 0; u < 8; u++)
+            if (k0 + u < slices) s += v[u];
+    }
     if (!rows1) { y0[i] = s; return; }
     const int t = i / rows_all, c = i - t * rows_all;
     if (c < rows0) y0[(size_t)t * rows0 + c] = s;
@@ -1535,6 +1604,9 @@ int launch_matvec_round(const ksh_kernel &k, const LaunchArgs &a, hipStream_t st
 }
 
 constexpr int kSkinnyMaxBatch = 64;
+// k.variant: 1 the small-batch form; else 2 * the K slices where their sums are folded (0: one slice), and this bit where
+// the tile reads bf16 rows as they are
+constexpr int kRowsDirect = 1 << 24;
 
 int mm_row_tiles(const ksh_kernel_desc &d) { return (int)((d.dims[0] + BN - 1) / BN + (d.dims[3] + BN - 1) / BN + (d.dims[4] + BN - 1) / BN); }
 
@@ -1556,6 +1628,8 @@ int launch_mul_mm(const ksh_kernel &k, const LaunchArgs &a, hipStream_t st)
     // columns: 768 threads) where the tile keeps them
     const int octets = cols / 8, pb1 = (octets + 63) / 64 * 64;
     const dim3 pg((unsigned)batch), pb((unsigned)std::min(pb1 > 1024 && inv_s ? (octets / 2 + 63) / 64 * 64 : pb1, 1024));
+    const bool rows_direct = (k.variant & kRowsDirect) != 0;
+    const int slices = (k.variant & ~kRowsDirect) >> 1;                  // 0: no fold
     if (prologue) {
         // the rows' producer runs inside the preparation: in = W, X, [W1, W2,] then the prologue's operands
         const int xs = (int)k.desc.dims[7];
@@ -1572,7 +1646,7 @@ int launch_mul_mm(const ksh_kernel &k, const LaunchArgs &a, hipStream_t st)
     } else if (f32x && tile)
         hipLaunchKernelGGL(mm_prep_rows_kernel<0>, pg, pb, 0, st, (const float *)a.in[1], nullptr, nullptr, nullptr, nullptr, Xf, Xf_lo, SxA, SxA_lo, cols, 0.f, 0, inv_s);
     else if (f32x) hipLaunchKernelGGL(mm_prep_x_f32_kernel, dim3((n + 255) / 256), dim3(256), 0, st, (const float *)a.in[1], Xf, Xf_lo, SxA, SxA_lo, batch, cols);
-    else hipLaunchKernelGGL(mm_prep_x_kernel, dim3(((batch + 31) / 32 * (cols / 32) + 3) / 4), dim3(256), 0, st, (const uint16_t *)a.in[1], Xf, SxA, batch, cols);
+    else if (!rows_direct) hipLaunchKernelGGL(mm_prep_x_kernel, dim3(((batch + 31) / 32 * (cols / 32) + 3) / 4), dim3(256), 0, st, (const uint16_t *)a.in[1], Xf, SxA, batch, cols);
     MmParams p;
     p.W = (const uint8_t *)a.in[0];
     p.Y = (float *)a.out[0];
@@ -1596,9 +1670,10 @@ int launch_mul_mm(const ksh_kernel &k, const LaunchArgs &a, hipStream_t st)
         return e2 == hipSuccess ? 0 : hip_fail(e2, "mul_mm (small batch) launch");
     }
     const bool cut = k.desc.dims[6] == 2;
-    const int tm = mm_tile_tokens(k.desc.dtypes[0] == KSH_Q6K, f32x, mm_row_tiles(k.desc), batch, k.variant >= 2 ? k.variant >> 1 : 1);
+    const int tm = k.info.lds_bytes == kLdsBytes64 ? 64 : 128;
     const dim3 grid((batch + tm - 1) / tm, (rows + BN - 1) / BN + (rows1 + BN - 1) / BN + (rows2 + BN - 1) / BN);
-    p.Xf = Xf; p.SxA = SxA; p.Xf_lo = Xf_lo; p.inv_s = inv_s;
+    p.Xf = rows_direct ? (const _Float16 *)a.in[1] : Xf;
+    p.SxA = SxA; p.Xf_lo = Xf_lo; p.inv_s = inv_s;
     p.ksplit = 0; p.Y_parts = nullptr;
     p.cut_as = cut ? (const float *)a.in[k.info.n_inputs - 1] : nullptr;
     const bool q6 = k.desc.dtypes[0] == KSH_Q6K;
@@ -1607,6 +1682,7 @@ int launch_mul_mm(const ksh_kernel &k, const LaunchArgs &a, hipStream_t st)
     do { \
         if (cut) hipLaunchKernelGGL((q_mul_mm_kernel<Q6, TM, true, true>), g, dim3(kThreadsMM), LDS, st, p); \
         else if (f32x) hipLaunchKernelGGL((q_mul_mm_kernel<Q6, TM, true>), g, dim3(kThreadsMM), LDS, st, p); \
+        else if (Q6 && rows_direct) hipLaunchKernelGGL((q_mul_mm_kernel<Q6, TM, false, false, Q6>), g, dim3(kThreadsMM), LDS, st, p); \
         else hipLaunchKernelGGL((q_mul_mm_kernel<Q6, TM, false>), g, dim3(kThreadsMM), LDS, st, p); \
     } while (0)
         if (q6) KSH_TILE(true, 128, kLdsBytes);
@@ -1614,9 +1690,9 @@ int launch_mul_mm(const ksh_kernel &k, const LaunchArgs &a, hipStream_t st)
         else KSH_TILE(false, 128, kLdsBytes);
 #undef KSH_TILE
     };
-    if (k.variant >= 2) {
+    if (slices) {
         // few tiles: K slices as blockIdx.z of one launch, then the fold
-        const int ks = k.variant >> 1;
+        const int ks = slices;
         p.ksplit = ks;
         const bool unfolded = k.desc.dims[6] == 1;                    // the partial sums are the result: the reader adds them
         p.Y_parts = unfolded ? (float *)a.out[0] : (float *)((f32x ? SxA_lo : SxA) + sx_halves);     // (else behind the prepared activations)
@@ -1637,9 +1713,10 @@ int launch_mul_mm(const ksh_kernel &k, const LaunchArgs &a, hipStream_t st)
 
 }  // namespace
 
+// (f32 activations)
 int matvec_batch_slices(const ksh_kernel_desc &d, int batch)
 {
-    return mm_k_slices(d.dtypes[0] == KSH_Q6K, d.dtypes[1] == KSH_F32, mm_row_tiles(d), (int)(d.dims[1] / 256), batch);
+    return mm_k_slices(d.dtypes[0] == KSH_Q6K, mm_row_tiles(d), (int)(d.dims[1] / 256), batch);
 }
 
 int bind_matvec_batch(ksh_kernel &k)
@@ -1707,9 +1784,11 @@ int bind_matvec_batch(ksh_kernel &k)
     if (want && want != 32 && want != BN) return set_error("matvec_batch: unsupported schedule nr0=%u (32 or %d)", want, BN);
     const bool can_skinny = !q6 && batch <= kSkinnyMaxBatch && n_mat == 1 && !unfolded && !cut;
     if (want == 32 && !can_skinny) return set_error("matvec_batch: the small-batch form takes Q4_K weights and up to %d tokens", kSkinnyMaxBatch);
-    // (long rows of a short matrix leave the small-batch form 64 workgroups with four superblocks per wave: from 33
-    // tokens on the tile over K slices is faster there -- 2048 x 8192 at 63 tokens: 27.5 us against 41.0)
-    const bool long_rows = batch > 32 && rows <= 2048 && cols >= 8192;
+    // (long rows of a short matrix leave the small-batch form 64 workgroups with four superblocks per wave: f32, from 33
+    // tokens on, the tile over K slices is faster there -- 2048 x 8192 at 63 tokens: 27.5 us against 41.0; bf16 rows take
+    // whichever form is estimated shorter -- 1536 x 6144 at 50 tokens: 16.1 against 21.1)
+    const bool long_rows = f32x ? batch > 32 && rows <= 2048 && cols >= 8192
+                                : mm_plan_bf16(q6, mm_row_tiles(k.desc), (int)(cols / 256), batch, rows_all, (int)k.desc.sched.k_split).us < mm_skinny_us(rows, (int)(cols / 256), batch);
     k.variant = (want == 32 || (want == 0 && can_skinny && !long_rows)) ? 1 : 0;
     k.info.sched = k.desc.sched;
     if (k.variant == 1) {
@@ -1719,18 +1798,23 @@ int bind_matvec_batch(ksh_kernel &k)
         k.launch = launch_mul_mm;
         return 0;
     }
-    // K slices (mm_k_slices): workgroups of one launch, every slice storing its partial sums, and a second launch that adds
-    // them.  sched.k_split names the slice count (a divisor of cols / 256; 1 = none).
+    // K slices: workgroups of one launch, every slice storing its partial sums, and a second launch that adds them
+    // (mm_k_slices, mm_plan_bf16).  sched.k_split names the slice count (a divisor of cols / 256; 1 = none).
     const int64_t row_tiles = mm_row_tiles(k.desc), nsb = cols / 256;
-    int64_t ks = 1;
-    if (k.desc.sched.k_split && !cut) {
-        ks = k.desc.sched.k_split;
-        if (nsb % ks) return set_error("matvec_batch: k_split=%lld does not divide the %lld superblocks of a row", (long long)ks, (long long)nsb);
-    } else if (!cut) {
-        ks = mm_k_slices(q6, f32x, (int)row_tiles, (int)nsb, (int)batch);
+    int64_t ks = cut ? 1 : k.desc.sched.k_split;
+    if (!cut && ks && nsb % ks) return set_error("matvec_batch: k_split=%lld does not divide the %lld superblocks of a row", (long long)ks, (long long)nsb);
+    int tm = 0;
+    if (f32x) {
+        if (!ks) ks = mm_k_slices(q6, (int)row_tiles, (int)nsb, (int)batch);
+        tm = mm_tile_tokens(q6, (int)row_tiles, (int)batch, (int)ks);
+    } else {
+        const MmPlan plan = mm_plan_bf16(q6, (int)row_tiles, (int)nsb, batch, rows_all, (int)ks);
+        ks = plan.ks;
+        tm = plan.tm;
     }
     const bool z_form = unfolded || ks > 1;
     k.variant = z_form ? (int)(ks << 1) : 0;
+    if (!f32x && q6 && mm_rows_direct((batch + tm - 1) / tm * row_tiles * ks, (int)((nsb + ks - 1) / ks), batch, cols)) k.variant |= kRowsDirect;
     if (z_form && !unfolded) k.scratch_bytes += (size_t)ks * batch * rows_all * 4;
     if (unfolded) {
         const int keep = prologue == 2 ? 1 : 0;                       // (the add-then-norm prologue's x_new stays an output)
@@ -1738,7 +1822,6 @@ int bind_matvec_batch(ksh_kernel &k)
         k.out_bytes[0] = (size_t)ks * batch * rows_all * 4; k.out_align[0] = 16;
         k.info.n_outputs = 1 + keep;
     }
-    const int tm = mm_tile_tokens(q6, f32x, (int)row_tiles, (int)batch, (int)ks);
     set_launch(k, (uint32_t)((batch + tm - 1) / tm), (uint32_t)row_tiles, z_form ? (uint32_t)ks : 1, kThreadsMM,
                (uint32_t)(tm == 64 ? kLdsBytes64 : kLdsBytes));
     k.info.sched.tg = kThreadsMM; k.info.sched.nsg = kThreadsMM / 64; k.info.sched.nr0 = BN; k.info.sched.k_split = (uint32_t)ks; k.info.sched.lds_tile = KS;

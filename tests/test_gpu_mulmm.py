@@ -325,6 +325,25 @@ def test_mul_mm_f32_both_parts_in_one_workgroup(ctx, unfolded, k_split):
     assert not got[7].any()
 
 
+@pytest.mark.parametrize("wdt,batch,rows,cols", [(DType.Q6K, 77, 300, 7936), (DType.Q4K, 77, 300, 7936), (DType.Q4K, 64, 129, 7936),
+                                                 (DType.Q6K, 1, 129, 2816), (DType.Q6K, 257, 10881, 1536), (DType.Q4K, 321, 7041, 768)])
+def test_mul_mm_bf16_default_tile_and_slices(ctx, wdt, batch, rows, cols):
+    """The launch bf16 rows get by themselves: slices of unequal length (31 and 11 superblocks), Q6_K products reading the
+    rows of X as they are and behind a preparation (two rounds of tiles), tiles of 64 tokens two to a compute unit;
+    ragged in both directions."""
+    nb = rows * cols // 256
+    w = synth.q4k_blocks(nb, 660) if wdt == DType.Q4K else synth.q6k_blocks(nb, 660)
+    xf, xb = synth.bf16_round(synth.normal_f32(batch * cols, 661))
+    k = ctx.compile(hip.make_desc(hip.Kind.MATVEC_BATCH, (rows, cols, batch), (wdt, DType.BF16, DType.F32)))
+    by = ctx.buffer_empty_f32(batch * rows)
+    ctx.encode_multi(k, [ctx.buffer_bytes(w), ctx.buffer_bytes(xb)], [by])
+    ctx.synchronize()
+    got = ctx.read_f32(by, batch * rows).reshape(batch, rows)
+    odt = oracle.Q4K if wdt == DType.Q4K else oracle.Q6K
+    for t in sorted({0, batch // 2, batch - 1}):
+        assert_close(got[t], oracle.matvec_f64(odt, w, rows, cols, xf.reshape(batch, cols)[t]), 1e-4, f"{k.name} t={t}")
+
+
 def test_mul_mm_k_slices_must_divide_the_row(ctx):
     with pytest.raises(hip.KshError, match="does not divide"):
         ctx.compile(hip.make_desc(hip.Kind.MATVEC_BATCH, (256, 2048, 100), (DType.Q4K, DType.BF16, DType.F32), (), dict(k_split=3)))
