@@ -1264,73 +1264,80 @@ __global__ __launch_bounds__(512) void q4k_mm_round_kernel(RoundParams p)
     const int sbc = min(sb, nsb - 1);
     const size_t woff = (size_t)min(r0 + n, rows - 1) * nsb * 144 + (size_t)sbc * 144;
 
-    // ---- every load of the wave, up front
-    u32x4_t hdr[NM];
-    u32x2_t q[NM][4][2];
+    // (the other waves ask for nothing: a quarter of the requests were for a row's last superblock again, and the vector-memory
+    // path is what the launch is busy with -- gate | up of 12288 x 1536 for 16 rows 18.8 -> 16.8 us)
+    if (active) {
+        // ---- every load of the wave, up front
+        u32x4_t hdr[NM];
+        u32x2_t q[NM][4][2];
 #pragma unroll
-    for (int m = 0; m < NM; m++) {
-        const uint8_t *blk = (m ? p.W1 : W) + woff;
-        hdr[m] = *reinterpret_cast<const u32x4_t *>(blk);
+        for (int m = 0; m < NM; m++) {
+            const uint8_t *blk = (m ? p.W1 : W) + woff;
+            hdr[m] = *reinterpret_cast<const u32x4_t *>(blk);
 #pragma unroll
-        for (int g = 0; g < 4; g++) {
-            q[m][g][0] = *reinterpret_cast<const u32x2_t *>(blk + 16 + 32 * g + 8 * h);
-            q[m][g][1] = *reinterpret_cast<const u32x2_t *>(blk + 16 + 32 * g + 16 + 8 * h);
-        }
-    }
-    const h8 *xa = reinterpret_cast<const h8 *>(p.Xp) + (size_t)sbc * 16 * 64 + lane;
-    h8 a[16];
-#pragma unroll
-    for (int j = 0; j < 16; j++) a[j] = xa[(size_t)j * 64];
-    // sums of x: rows 0..15 the tokens' hi parts, rows 16..31 their lo parts
-    const _Float16 *sx = p.Xp + round_xf_halves(p.cols) + (n >= 16 ? round_sx_halves(p.cols) : 0) + ((size_t)(n & 15) * nsb + sbc) * 32 + 8 * h;
-    const h8 a2[2] = {*reinterpret_cast<const h8 *>(sx), *reinterpret_cast<const h8 *>(sx + 16)};
-
-    const f16v kZero16 = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-    for (int m = 0; m < NM; m++) {
-        f16v C = kZero16;
-#pragma unroll
-        for (int g = 0; g < 4; g++) {
-            const uint4 s = q4k_group_scales(hdr[m].y, hdr[m].z, hdr[m].w, g);   // sc_lo, mn_lo, sc_hi, mn_hi
-#pragma unroll
-            for (int j = 0; j < 4; j++) {
-                // slice j: bytes (j & 1 ? 16 + 8h : 8h) .. +7, low nibbles for j < 2, high nibbles after
-                const u32x2_t qq = q[m][g][j & 1];
-                const uint32_t sc = j < 2 ? s.x : s.z;
-                uint32_t o[4];
-#pragma unroll
-                for (int i = 0; i < 2; i++) {
-                    const uint32_t d = j < 2 ? qq[i] : qq[i] >> 4;
-                    o[2 * i] = pair_f16(d & 0x000F000Fu, sc);
-                    o[2 * i + 1] = pair_f16((d >> 8) & 0x000F000Fu, sc);
-                }
-                const u32x4_t ov = {o[0], o[1], o[2], o[3]};
-                C = __builtin_amdgcn_mfma_f32_32x32x16_f16(a[4 * g + j], __builtin_bit_cast(h8, ov), C, 0, 0, 0);
+            for (int g = 0; g < 4; g++) {
+                q[m][g][0] = *reinterpret_cast<const u32x2_t *>(blk + 16 + 32 * g + 8 * h);
+                q[m][g][1] = *reinterpret_cast<const u32x2_t *>(blk + 16 + 32 * g + 16 + 8 * h);
             }
         }
-        // bias + mins of the superblock: the row's eight coefficients -(dmin*m_j + 1024*d) as f16 hi | lo, against the
-        // sums of x (hi[8] hi[8] lo[8] 0[8] per row and superblock): hi*hi + hi*lo + lo*hi
-        const float d = half_bits_to_f32(hdr[m].x & 0xFFFFu), dmin = half_bits_to_f32(hdr[m].x >> 16);
-        _Float16 chi[8], clo[8];
+        const h8 *xa = reinterpret_cast<const h8 *>(p.Xp) + (size_t)sbc * 16 * 64 + lane;
+        h8 a[16];
 #pragma unroll
-        for (int g = 0; g < 4; g++) {
-            const uint4 s = q4k_group_scales(hdr[m].y, hdr[m].z, hdr[m].w, g);
-            const float c0 = pinned(-(dmin * (float)s.y + 1024.f * d)), c1 = pinned(-(dmin * (float)s.w + 1024.f * d));
-            chi[2 * g] = (_Float16)c0; chi[2 * g + 1] = (_Float16)c1;
-            clo[2 * g] = (_Float16)(c0 - (float)chi[2 * g]); clo[2 * g + 1] = (_Float16)(c1 - (float)chi[2 * g + 1]);
+        for (int j = 0; j < 16; j++) a[j] = xa[(size_t)j * 64];
+        // sums of x: rows 0..15 the tokens' hi parts, rows 16..31 their lo parts
+        const _Float16 *sx = p.Xp + round_xf_halves(p.cols) + (n >= 16 ? round_sx_halves(p.cols) : 0) + ((size_t)(n & 15) * nsb + sbc) * 32 + 8 * h;
+        const h8 a2[2] = {*reinterpret_cast<const h8 *>(sx), *reinterpret_cast<const h8 *>(sx + 16)};
+
+        const f16v kZero16 = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int m = 0; m < NM; m++) {
+            f16v C = kZero16;
+#pragma unroll
+            for (int g = 0; g < 4; g++) {
+                const uint4 s = q4k_group_scales(hdr[m].y, hdr[m].z, hdr[m].w, g);   // sc_lo, mn_lo, sc_hi, mn_hi
+#pragma unroll
+                for (int j = 0; j < 4; j++) {
+                    // slice j: bytes (j & 1 ? 16 + 8h : 8h) .. +7, low nibbles for j < 2, high nibbles after
+                    const u32x2_t qq = q[m][g][j & 1];
+                    const uint32_t sc = j < 2 ? s.x : s.z;
+                    uint32_t o[4];
+#pragma unroll
+                    for (int i = 0; i < 2; i++) {
+                        const uint32_t d = j < 2 ? qq[i] : qq[i] >> 4;
+                        o[2 * i] = pair_f16(d & 0x000F000Fu, sc);
+                        o[2 * i + 1] = pair_f16((d >> 8) & 0x000F000Fu, sc);
+                    }
+                    const u32x4_t ov = {o[0], o[1], o[2], o[3]};
+                    C = __builtin_amdgcn_mfma_f32_32x32x16_f16(a[4 * g + j], __builtin_bit_cast(h8, ov), C, 0, 0, 0);
+                }
+            }
+            // bias + mins of the superblock: the row's eight coefficients -(dmin*m_j + 1024*d) as f16 hi | lo, against the
+            // sums of x (hi[8] hi[8] lo[8] 0[8] per row and superblock): hi*hi + hi*lo + lo*hi
+            const float d = half_bits_to_f32(hdr[m].x & 0xFFFFu), dmin = half_bits_to_f32(hdr[m].x >> 16);
+            _Float16 chi[8], clo[8];
+#pragma unroll
+            for (int g = 0; g < 4; g++) {
+                const uint4 s = q4k_group_scales(hdr[m].y, hdr[m].z, hdr[m].w, g);
+                const float c0 = pinned(-(dmin * (float)s.y + 1024.f * d)), c1 = pinned(-(dmin * (float)s.w + 1024.f * d));
+                chi[2 * g] = (_Float16)c0; chi[2 * g + 1] = (_Float16)c1;
+                clo[2 * g] = (_Float16)(c0 - (float)chi[2 * g]); clo[2 * g + 1] = (_Float16)(c1 - (float)chi[2 * g + 1]);
+            }
+            h8 b2[2];
+#pragma unroll
+            for (int i = 0; i < 8; i++) {
+                b2[0][i] = h ? clo[i] : chi[i];                 // columns 0..7: hi, 8..15: lo
+                b2[1][i] = h ? (_Float16)0.f : chi[i];          // columns 16..23: hi, 24..31: zero
+            }
+            f16v F = __builtin_amdgcn_mfma_f32_32x32x16_f16(a2[0], b2[0], kZero16, 0, 0, 0);
+            F = __builtin_amdgcn_mfma_f32_32x32x16_f16(a2[1], b2[1], F, 0, 0, 0);
+            // accumulator i of lane (n, h) is row 8*(i/4) + 4*h + i%4 of the tile: i < 8 a token's hi part, i + 8 its lo part
+#pragma unroll
+            for (int i = 0; i < 8; i++)
+                red[((wave * NM + m) * 8 + i) * 64 + lane] = fmaf(1.0f / 2048.0f, fmaf(d, C[i + 8], F[i + 8]), fmaf(d, C[i], F[i]));
         }
-        h8 b2[2];
+    } else {
 #pragma unroll
-        for (int i = 0; i < 8; i++) {
-            b2[0][i] = h ? clo[i] : chi[i];                 // columns 0..7: hi, 8..15: lo
-            b2[1][i] = h ? (_Float16)0.f : chi[i];          // columns 16..23: hi, 24..31: zero
-        }
-        f16v F = __builtin_amdgcn_mfma_f32_32x32x16_f16(a2[0], b2[0], kZero16, 0, 0, 0);
-        F = __builtin_amdgcn_mfma_f32_32x32x16_f16(a2[1], b2[1], F, 0, 0, 0);
-        // accumulator i of lane (n, h) is row 8*(i/4) + 4*h + i%4 of the tile: i < 8 a token's hi part, i + 8 its lo part
-#pragma unroll
-        for (int i = 0; i < 8; i++)
-            red[((wave * NM + m) * 8 + i) * 64 + lane] = active ? fmaf(1.0f / 2048.0f, fmaf(d, C[i + 8], F[i + 8]), fmaf(d, C[i], F[i])) : 0.f;
+        for (int i = 0; i < 8 * NM; i++) red[(wave * NM * 8 + i) * 64 + lane] = 0.f;
     }
     __syncthreads();
     // one output per thread: the eight waves' shares in a fixed order
