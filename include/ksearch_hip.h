@@ -83,6 +83,8 @@ enum ksh_kind {
      *   itself; out[1] = x_new with prologue 2.
      * dims[6] = 2 (F32 activations): the rows are several prompts', each summed as in a launch of its own -- one more
      *   input, the last, f32[batch]: the tokens of that launch (more than 64), whose K slices the row's sums are cut into.
+     * dims[6] = 3 (F32 activations, rows1 = rows, Q4_K, rows in one K slice): W and W1 are a gate and an up matrix and
+     *   out[0] = f32[batch, rows] of gelu(W x) * (W1 x); out[1] = x_new with prologue 2.
      * dims[7] = the slices (info.grid[2]) of the GEMM whose unfolded result this one's X is (with a prologue;
      *   prologue 3 then reads gate | up from that one buffer and takes no `up` operand).  The sums are added in the
      *   fold's order, so a chain of GEMMs gives the same numbers with and without its folds.

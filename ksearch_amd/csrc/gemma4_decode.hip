@@ -648,19 +648,30 @@ int forward_prefill_chunk4(ksh_gemma4 *m, const uint32_t *tokens, int t, const J
             return 1;
         // With the producers inside, the o and the gate | up projection leave their K slices' partial sums unfolded
         // for the preparation that reads them (dims[6], dims[7]); the down projection folds (a plain norm reads it).
+        // Where gate | up has its rows in one K slice it leaves gelu(gate) * up itself.
         ksh_kernel *u_o = nullptr, *u_gu = nullptr;
-        bool travel = false;
+        bool travel = false, pair = inside;
+        if (joint)
+            for (int len : joint->alone) pair = pair && gate_up_pair(L.dt_gate, L.dt_up, L.ffn, h, len);
+        else
+            pair = pair && gate_up_pair(L.dt_gate, L.dt_up, L.ffn, h, tp);
         if (inside && L.dt_gate == L.dt_up && !joint) {
             const size_t T = kChunk4;
             if (get(m, KSH_MATVEC_BATCH, {h, P.qd, tp, 0, 0, 0, 1}, {L.dt_o, KSH_F32, KSH_F32}, {c.eps}, &u_o) ||
-                get(m, KSH_MATVEC_BATCH, {L.ffn, h, tp, L.ffn, 0, 2, 1, (int64_t)u_o->info.grid[2]}, {L.dt_gate, KSH_F32, KSH_F32}, {c.eps}, &u_gu))
+                get(m, KSH_MATVEC_BATCH, {L.ffn, h, tp, L.ffn, 0, 2, pair ? 3 : 1, (int64_t)u_o->info.grid[2]}, {L.dt_gate, KSH_F32, KSH_F32}, {c.eps}, &u_gu))
                 return 1;
-            travel = u_o->out_bytes[0] <= kPartsRows4 * T * c.hidden * 4 && u_gu->out_bytes[0] <= ksh_buffer_size(m->c_pg);
+            travel = u_o->out_bytes[0] <= kPartsRows4 * T * c.hidden * 4 && u_gu->out_bytes[0] <= ksh_buffer_size(pair ? m->c_ff : m->c_pg);
         }
         if (travel) {
             if (enc(m, u_o, {L.wo, m->c_o}, {m->c_po}, n) ||
-                enc(m, u_gu, {L.wgate, m->c_po, L.wup, L.post_attn_norm, m->c_x, L.ffn_norm}, {m->c_pg, m->c_x}, n) ||
-                gemm(L.dt_down, {h, L.ffn, tp, 0, 0, 3, 0, (int64_t)u_gu->info.grid[2]}, {L.wdown, m->c_pg}, {m->c_y}))
+                enc(m, u_gu, {L.wgate, m->c_po, L.wup, L.post_attn_norm, m->c_x, L.ffn_norm}, {pair ? m->c_ff : m->c_pg, m->c_x}, n) ||
+                (pair ? mm(L.dt_down, h, L.ffn, L.wdown, m->c_ff, m->c_y)
+                      : gemm(L.dt_down, {h, L.ffn, tp, 0, 0, 3, 0, (int64_t)u_gu->info.grid[2]}, {L.wdown, m->c_pg}, {m->c_y})))
+                return 1;
+        } else if (pair) {
+            if (mm(L.dt_o, h, P.qd, L.wo, m->c_o, m->c_y) ||
+                gemm(L.dt_gate, {L.ffn, h, tp, L.ffn, 0, 2, 3}, {L.wgate, m->c_y, L.wup, L.post_attn_norm, m->c_x, L.ffn_norm}, {m->c_ff, m->c_x}) ||
+                mm(L.dt_down, h, L.ffn, L.wdown, m->c_ff, m->c_y))
                 return 1;
         } else if (
             mm(L.dt_o, h, P.qd, L.wo, m->c_o, m->c_y) ||

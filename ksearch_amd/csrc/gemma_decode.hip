@@ -406,14 +406,16 @@ int forward_prefill_chunk(ksh_gemma *m, const uint32_t *tokens, int t)
     // ... and the o, gate | up and down projections leave their K slices' partial sums unfolded for the preparation
     // that reads them (dims[6], dims[7]): no fold launches but q | k | v's, whose reader is not a GEMM
     ksh_kernel *u_o = nullptr, *u_gu = nullptr, *u_down = nullptr, *u_down_last = nullptr, *u_qkv = nullptr;
+    // (with its rows in one K slice gate | up leaves gelu(gate) * up itself)
     bool travel = false;
+    const bool pair = gate_up_pair(KSH_Q4K, KSH_Q4K, c.ffn, c.hidden, tp);
     if (fused && c.n_layers > 1) {
         const size_t T = kChunk;
         auto parts_of = [](ksh_kernel *kk) { return (int64_t)kk->info.grid[2]; };      // the planes of its unfolded result
         if (get(m, KSH_MATVEC_BATCH, {c.hidden, qd, tp, 0, 0, 0, 1}, {KSH_Q4K, KSH_F32, KSH_F32}, {c.eps}, &u_o) ||
-            get(m, KSH_MATVEC_BATCH, {c.ffn, c.hidden, tp, c.ffn, 0, 2, 1, parts_of(u_o)}, {KSH_Q4K, KSH_F32, KSH_F32}, {c.eps}, &u_gu) ||
-            get(m, KSH_MATVEC_BATCH, {c.hidden, c.ffn, tp, 0, 0, 3, 1, parts_of(u_gu)}, {KSH_Q4K, KSH_F32, KSH_F32}, {c.eps}, &u_down) ||
-            get(m, KSH_MATVEC_BATCH, {c.hidden, c.ffn, tp, 0, 0, 3, 0, parts_of(u_gu)}, {KSH_Q4K, KSH_F32, KSH_F32}, {c.eps}, &u_down_last) ||
+            get(m, KSH_MATVEC_BATCH, {c.ffn, c.hidden, tp, c.ffn, 0, 2, pair ? 3 : 1, parts_of(u_o)}, {KSH_Q4K, KSH_F32, KSH_F32}, {c.eps}, &u_gu) ||
+            get(m, KSH_MATVEC_BATCH, {c.hidden, c.ffn, tp, 0, 0, pair ? 0 : 3, 1, pair ? 0 : parts_of(u_gu)}, {KSH_Q4K, KSH_F32, KSH_F32}, {c.eps}, &u_down) ||
+            get(m, KSH_MATVEC_BATCH, {c.hidden, c.ffn, tp, 0, 0, pair ? 0 : 3, 0, pair ? 0 : parts_of(u_gu)}, {KSH_Q4K, KSH_F32, KSH_F32}, {c.eps}, &u_down_last) ||
             get(m, KSH_MATVEC_BATCH, {qd, c.hidden, tp, kvd, kvd, 2, 0, parts_of(u_down)}, {KSH_Q4K, KSH_F32, KSH_F32}, {c.eps}, &u_qkv))
             return 1;
         travel = u_o->out_bytes[0] <= kPartsRows * T * c.hidden * 4 && u_gu->out_bytes[0] <= 2 * T * 2 * c.ffn * 4 &&
@@ -421,6 +423,7 @@ int forward_prefill_chunk(ksh_gemma *m, const uint32_t *tokens, int t)
     }
     // ... and a layer's closing norm + add with the next layer's attention norm are one add-then-norm, in that
     // layer's q | k | v preparation (the residual rows it stores are the closed layer's)
+    ksh_buf *gu = pair ? m->c_ff : m->c_pg;
     ksh_kernel *k_mm_qkv_close = nullptr;
     if (fused && c.n_layers > 1 && get(m, KSH_MATVEC_BATCH, {qd, c.hidden, tp, kvd, kvd, 2}, {KSH_Q4K, KSH_F32, KSH_F32}, {c.eps}, &k_mm_qkv_close)) return 1;
     const float embed_scale = std::sqrt((float)c.hidden);
@@ -453,9 +456,9 @@ int forward_prefill_chunk(ksh_gemma *m, const uint32_t *tokens, int t)
                 enc(m, k_head, {m->c_q, L.q_norm, m->rope, m->c_k, L.k_norm, m->c_v, m->meta}, {m->c_q, m->kv_k[l], m->kv_v[l]}, n) ||
                 enc(m, k_sdpa, {m->c_q, m->kv_k[l], m->kv_v[l], m->c_meta}, {m->c_tmp, m->c_o}, n) ||
                 enc(m, u_o, {L.wo, m->c_o}, {m->c_po}, n) ||
-                enc(m, u_gu, {L.wgate, m->c_po, L.wup, L.post_attn_norm, m->c_x, L.ffn_norm}, {m->c_pg, m->c_x}, n) ||
-                (last ? (enc(m, u_down_last, {L.wdown, m->c_pg}, {m->c_y}, n) || enc(m, k_add, {m->c_y, L.post_ffw_norm, m->c_x}, {m->c_x}, n))
-                      : enc(m, u_down, {L.wdown, m->c_pg}, {m->c_pd}, n)))
+                enc(m, u_gu, {L.wgate, m->c_po, L.wup, L.post_attn_norm, m->c_x, L.ffn_norm}, {gu, m->c_x}, n) ||
+                (last ? (enc(m, u_down_last, {L.wdown, gu}, {m->c_y}, n) || enc(m, k_add, {m->c_y, L.post_ffw_norm, m->c_x}, {m->c_x}, n))
+                      : enc(m, u_down, {L.wdown, gu}, {m->c_pd}, n)))
                 return 1;
             continue;
         }

@@ -180,7 +180,9 @@ int bind_matvec_q4k_family(ksh_kernel &k);
 int bind_matvec_qkv(ksh_kernel &k);
 int bind_matvec_gate_up_gelu(ksh_kernel &k);
 int bind_matvec_batch(ksh_kernel &k);
-int matvec_batch_slices(const ksh_kernel_desc &d, int batch);   // K slices of the tile over `batch` tokens
+int matvec_batch_slices(const ksh_kernel_desc &d, int batch);   // K slices of the tile over `batch` tokens (F32 activations)
+// whether a gate and an up matrix of ffn x hidden take the GEMM that leaves gelu(gate) * up (KSH_MATVEC_BATCH, dims[6] = 3)
+bool gate_up_pair(int dt_gate, int dt_up, int64_t ffn, int64_t hidden, int64_t batch);
 int bind_round_prep(ksh_kernel &k);
 int bind_matvec_round(ksh_kernel &k);
 int bind_dequant(ksh_kernel &k);

@@ -501,7 +501,10 @@ constexpr size_t kLdsBytes64 = 2 * (size_t)(kLdsMain + (64 + BN) * PITCH2) * 2 +
 // ROWS = true (bf16 activations, Q6_K weights: no sums of x are wanted): the A operands come from the rows of X as they are
 // and the multiplying waves convert them, eight values of a row a lane, between their matrix instructions -- no
 // preparation launch (mm_rows_direct; 333 tokens, 1536 x 6144 in six slices: 28.9 -> 25.4 us).
-template <bool Q6, int TM, bool LO, bool CUT = false, bool ROWS = false>
+// PAIR = true (f32 activations, a gate and an up matrix of one size): a tile is 64 rows of each, in turns of 32, so that a wave
+// has a gate row's sums beside its up row's and stores gelu(gate) * up -- half the results, and the down projection's
+// preparation reads them as they are instead of two matrices (2048 tokens, 12288 x 1536: 394 + 82 us -> 380 + 54).
+template <bool Q6, int TM, bool LO, bool CUT = false, bool ROWS = false, bool PAIR = false>
 __global__ __launch_bounds__(kThreadsMM, TM == 64 ? 2 : 1) void q_mul_mm_kernel(MmParams p)
 {
     constexpr int MT = TM / 64, kLdsMinT = (TM + BN) * PITCH2;
@@ -515,12 +518,12 @@ __global__ __launch_bounds__(kThreadsMM, TM == 64 ? 2 : 1) void q_mul_mm_kernel(
     int by = blockIdx.y, ycol = 0;
     const int rows_all = p.rows + p.rows1 + p.rows2;
     const int rows_of[3] = {p.rows, p.rows1, p.rows2};
-    if (p.rows1) {
+    if (!PAIR && p.rows1) {
         const int ty0 = (p.rows + BN - 1) / BN, ty1 = (p.rows1 + BN - 1) / BN;
         if (by >= ty0 + ty1) { by -= ty0 + ty1; ycol = p.rows + p.rows1; p.W = p.W2; p.Y = p.Y2; p.rows = p.rows2; }
         else if (by >= ty0) { by -= ty0; ycol = p.rows; p.W = p.W1; p.Y = p.Y1; p.rows = p.rows1; }
     }
-    const int t0 = blockIdx.x * TM, r0 = by * BN;
+    const int t0 = blockIdx.x * TM, r0 = PAIR ? by * (BN / 2) : by * BN;
     const int nsb_row = p.cols / 256;                            // superblocks per weight row
     int nsb = nsb_row, sb0 = 0;                                  // this workgroup's share of them
     size_t ystride = (size_t)p.rows;
@@ -620,7 +623,8 @@ __global__ __launch_bounds__(kThreadsMM, TM == 64 ? 2 : 1) void q_mul_mm_kernel(
         // ------------------------------------------------------------------ loaders
         const int lt = tid - 256, lrow = lt >> 1, lh = lt & 1;   // two threads per tile row
         const size_t row_bytes = (size_t)nsb_row * 144;
-        const uint8_t *wrow = p.W + (size_t)min(r0 + lrow, p.rows - 1) * row_bytes + (size_t)sb0 * 144;
+        const uint8_t *wrow = PAIR ? ((lrow & 32) ? p.W1 : p.W) + (size_t)min(r0 + (lrow >> 6) * 32 + (lrow & 31), p.rows - 1) * row_bytes
+                                   : p.W + (size_t)min(r0 + lrow, p.rows - 1) * row_bytes + (size_t)sb0 * 144;
         const size_t sx_off = ((size_t)min(t0 + lrow, p.batch - 1) * nsb_row + sb0) * 32;
         const _Float16 *sxrow = p.SxA + sx_off;
 
@@ -905,6 +909,20 @@ __global__ __launch_bounds__(kThreadsMM, TM == 64 ? 2 : 1) void q_mul_mm_kernel(
     }
 
     if (CUT) return;   // (the last slices' ends have stored everything)
+    if (PAIR) {
+#pragma unroll
+        for (int nt = 0; nt < NW_; nt += 2) {
+            const int r = r0 + (wn + nt / 2) * 32 + lm;
+#pragma unroll
+            for (int i = 0; i < 16; i++) {
+                const int t = t0 + wm * 32 + 8 * (i / 4) + 4 * (lane >> 5) + (i & 3);
+                const float inv = p.inv_s[min(t, p.batch - 1)];
+                const float y = gelu_mul_f32(pinned(F[0][nt][i] * inv), pinned(F[0][nt + 1][i] * inv));
+                if (t < p.batch && r < p.rows) p.Y[(size_t)t * p.rows + r] = y;
+            }
+        }
+        return;
+    }
     // accumulator layout of the 32x32 tile: column = lane % 32, row = 8*(i/4) + 4*(lane/32) + i%4
 #pragma unroll
     for (int mt = 0; mt < MW; mt++)
@@ -1640,7 +1658,7 @@ int launch_mul_mm(const ksh_kernel &k, const LaunchArgs &a, hipStream_t st)
     if (prologue) {
         // the rows' producer runs inside the preparation: in = W, X, [W1, W2,] then the prologue's operands
         const int xs = (int)k.desc.dims[7];
-        const int n_out0 = k.desc.dims[6] == 1 ? 1 : n_mat0;                    // (unfolded partial sums are one buffer)
+        const int n_out0 = k.desc.dims[6] & 1 ? 1 : n_mat0;                    // (unfolded partial sums are one buffer)
         const float *X = (const float *)a.in[1], *q0 = (const float *)a.in[1 + n_mat0];
         const float eps = k.desc.params[0];
         if (prologue == 1)
@@ -1661,8 +1679,8 @@ int launch_mul_mm(const ksh_kernel &k, const LaunchArgs &a, hipStream_t st)
     const int rows1 = (int)k.desc.dims[3], rows2 = (int)k.desc.dims[4];
     p.rows1 = rows1; p.rows2 = rows2;
     p.W1 = rows1 ? (const uint8_t *)a.in[2] : p.W; p.W2 = rows2 ? (const uint8_t *)a.in[3] : p.W;
-    const bool unfolded_out = k.desc.dims[6] == 1;
-    p.Y1 = rows1 && !unfolded_out ? (float *)a.out[1] : p.Y; p.Y2 = rows2 && !unfolded_out ? (float *)a.out[2] : p.Y;
+    const bool unfolded_out = k.desc.dims[6] == 1, pair = k.desc.dims[6] == 3;
+    p.Y1 = rows1 && !unfolded_out && !pair ? (float *)a.out[1] : p.Y; p.Y2 = rows2 && !unfolded_out ? (float *)a.out[2] : p.Y;
     if (k.variant == 1) {
         // the small-batch form: one launch, the low parts riding along
         p.Xf = Xf; p.SxA = SxA;
@@ -1678,7 +1696,7 @@ int launch_mul_mm(const ksh_kernel &k, const LaunchArgs &a, hipStream_t st)
     }
     const bool cut = k.desc.dims[6] == 2;
     const int tm = k.info.lds_bytes == kLdsBytes64 ? 64 : 128;
-    const dim3 grid((batch + tm - 1) / tm, (rows + BN - 1) / BN + (rows1 + BN - 1) / BN + (rows2 + BN - 1) / BN);
+    const dim3 grid((batch + tm - 1) / tm, pair ? (rows + BN / 2 - 1) / (BN / 2) : (rows + BN - 1) / BN + (rows1 + BN - 1) / BN + (rows2 + BN - 1) / BN);
     p.Xf = rows_direct ? (const _Float16 *)a.in[1] : Xf;
     p.SxA = SxA; p.Xf_lo = Xf_lo; p.inv_s = inv_s;
     p.ksplit = 0; p.Y_parts = nullptr;
@@ -1687,7 +1705,8 @@ int launch_mul_mm(const ksh_kernel &k, const LaunchArgs &a, hipStream_t st)
     auto launch_tile = [&](dim3 g) {
 #define KSH_TILE(Q6, TM, LDS) \
     do { \
-        if (cut) hipLaunchKernelGGL((q_mul_mm_kernel<Q6, TM, true, true>), g, dim3(kThreadsMM), LDS, st, p); \
+        if (!Q6 && pair) hipLaunchKernelGGL((q_mul_mm_kernel<Q6, TM, true, false, false, !Q6>), g, dim3(kThreadsMM), LDS, st, p); \
+        else if (cut) hipLaunchKernelGGL((q_mul_mm_kernel<Q6, TM, true, true>), g, dim3(kThreadsMM), LDS, st, p); \
         else if (f32x) hipLaunchKernelGGL((q_mul_mm_kernel<Q6, TM, true>), g, dim3(kThreadsMM), LDS, st, p); \
         else if (Q6 && rows_direct) hipLaunchKernelGGL((q_mul_mm_kernel<Q6, TM, false, false, Q6>), g, dim3(kThreadsMM), LDS, st, p); \
         else hipLaunchKernelGGL((q_mul_mm_kernel<Q6, TM, false>), g, dim3(kThreadsMM), LDS, st, p); \
@@ -1726,6 +1745,12 @@ int matvec_batch_slices(const ksh_kernel_desc &d, int batch)
     return mm_k_slices(d.dtypes[0] == KSH_Q6K, mm_row_tiles(d), (int)(d.dims[1] / 256), batch);
 }
 
+bool gate_up_pair(int dt_gate, int dt_up, int64_t ffn, int64_t hidden, int64_t batch)
+{
+    const int row_tiles = (int)(2 * ((ffn + BN - 1) / BN));
+    return dt_gate == KSH_Q4K && dt_up == KSH_Q4K && mm_k_slices(false, row_tiles, (int)(hidden / 256), (int)batch) == 1;
+}
+
 int bind_matvec_batch(ksh_kernel &k)
 {
     const int64_t rows = k.desc.dims[0], cols = k.desc.dims[1], batch = k.desc.dims[2];
@@ -1760,10 +1785,15 @@ int bind_matvec_batch(ksh_kernel &k)
     // then reads gate | up from that one buffer and takes no `up` operand)
     // dims[6] = 2: the rows belong to several prompts, each to be summed as in a launch of its own: one more input,
     // f32[batch], the tokens of that launch for every row (more than 64).  For f32 activations.
-    const bool unfolded = k.desc.dims[6] == 1, cut = k.desc.dims[6] == 2;
+    // dims[6] = 3: W and W1 are a gate and an up matrix of one size and the result is gelu(W x) * (W1 x), f32[batch][rows].
+    // For f32 activations, Q4_K, and rows that are not cut into K slices (matvec_batch_slices = 1).
+    const bool unfolded = k.desc.dims[6] == 1, cut = k.desc.dims[6] == 2, pair = k.desc.dims[6] == 3;
     const int64_t x_slices = k.desc.dims[7];
-    if (k.desc.dims[6] < 0 || k.desc.dims[6] > 2)
-        return set_error("matvec_batch: dims[6]=%lld (0, 1 for unfolded partial sums, 2 for rows summed as in launches of their own)", (long long)k.desc.dims[6]);
+    if (k.desc.dims[6] < 0 || k.desc.dims[6] > 3)
+        return set_error("matvec_batch: dims[6]=%lld (0, 1 for unfolded partial sums, 2 for rows summed as in launches of their own, 3 for gelu(gate) * up)", (long long)k.desc.dims[6]);
+    if (pair && (!f32x || q6 || rows1 != rows || rows2 || k.desc.sched.nr0 == 32 ||
+                 (k.desc.sched.k_split ? k.desc.sched.k_split != 1 : matvec_batch_slices(k.desc, (int)batch) != 1)))
+        return set_error("matvec_batch: gelu(gate) * up (dims[6]=3) takes F32 activations, two Q4_K matrices of one size and rows in one K slice");
     if (cut && !f32x) return set_error("matvec_batch: rows summed as in launches of their own (dims[6]=2) take F32 activations");
     if (x_slices && (!prologue || x_slices < 1 || x_slices > 64))
         return set_error("matvec_batch: X as unfolded partial sums (dims[7]=%lld) takes a prologue and 1 to 64 slices", (long long)k.desc.dims[7]);
@@ -1779,6 +1809,10 @@ int bind_matvec_batch(ksh_kernel &k)
         k.info.n_inputs = ni;
         if (x_slices) k.in_bytes[1] = (size_t)x_slices * mat * (prologue == 3 ? 2 : 1);
     }
+    if (pair) {
+        if (prologue == 2) { k.out_bytes[1] = k.out_bytes[n_mat]; k.out_align[1] = 16; }
+        k.info.n_outputs = prologue == 2 ? 2 : 1;
+    }
     if (cut) {
         const int ni = k.info.n_inputs++;
         k.in_bytes[ni] = (size_t)batch * 4; k.in_align[ni] = 4;
@@ -1789,7 +1823,7 @@ int bind_matvec_batch(ksh_kernel &k)
     // there), 128 = the 128 x 128 tile.
     const uint32_t want = k.desc.sched.nr0;
     if (want && want != 32 && want != BN) return set_error("matvec_batch: unsupported schedule nr0=%u (32 or %d)", want, BN);
-    const bool can_skinny = !q6 && batch <= kSkinnyMaxBatch && n_mat == 1 && !unfolded && !cut;
+    const bool can_skinny = !q6 && batch <= kSkinnyMaxBatch && n_mat == 1 && !unfolded && !cut && !pair;
     if (want == 32 && !can_skinny) return set_error("matvec_batch: the small-batch form takes Q4_K weights and up to %d tokens", kSkinnyMaxBatch);
     // (long rows of a short matrix leave the small-batch form 64 workgroups with four superblocks per wave: f32, from 33
     // tokens on, the tile over K slices is faster there -- 2048 x 8192 at 63 tokens: 27.5 us against 41.0; bf16 rows take
@@ -1829,11 +1863,12 @@ int bind_matvec_batch(ksh_kernel &k)
         k.out_bytes[0] = (size_t)ks * batch * rows_all * 4; k.out_align[0] = 16;
         k.info.n_outputs = 1 + keep;
     }
-    set_launch(k, (uint32_t)((batch + tm - 1) / tm), (uint32_t)row_tiles, z_form ? (uint32_t)ks : 1, kThreadsMM,
+    set_launch(k, (uint32_t)((batch + tm - 1) / tm), pair ? (uint32_t)((rows + BN / 2 - 1) / (BN / 2)) : (uint32_t)row_tiles, z_form ? (uint32_t)ks : 1, kThreadsMM,
                (uint32_t)(tm == 64 ? kLdsBytes64 : kLdsBytes));
     k.info.sched.tg = kThreadsMM; k.info.sched.nsg = kThreadsMM / 64; k.info.sched.nr0 = BN; k.info.sched.k_split = (uint32_t)ks; k.info.sched.lds_tile = KS;
     set_name(k, "mul_mm_%s_%dx%dx%d%s%s%s%s", q6 ? "q6k" : "q4k", BM, BN, KS, f32x ? "_f32x" : "", z_form ? "_kz" : "", n_mat == 3 ? "_x3" : n_mat == 2 ? "_x2" : "",
              prologue == 1 ? "_rms" : prologue == 2 ? "_addrms" : prologue == 3 ? "_gelu" : "");
+    if (pair) { char nm[64]; snprintf(nm, sizeof(nm), "%s", k.info.name); set_name(k, "%s_gate_up", nm); }
     if (cut) { char nm[64]; snprintf(nm, sizeof(nm), "%s", k.info.name); set_name(k, "%s_cut", nm); }
     if (unfolded) { char nm[64]; snprintf(nm, sizeof(nm), "%s", k.info.name); set_name(k, "%s_unfolded", nm); }
     k.launch = launch_mul_mm;

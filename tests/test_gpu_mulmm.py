@@ -325,6 +325,32 @@ def test_mul_mm_f32_both_parts_in_one_workgroup(ctx, unfolded, k_split):
     assert not got[7].any()
 
 
+@pytest.mark.parametrize("rows,batch,prologue", [(31, 33, 0), (97, 64, 2), (200, 130, 0), (4130, 1000, 2)])
+def test_mul_mm_f32_gate_up_pair(ctx, rows, batch, prologue):
+    """dims[6] = 3: gelu(W x) * (W1 x) from one launch is the two matrices' products and KSH_GELU_MUL (tiles of 64 and of
+    128 tokens, 64 rows of each matrix a tile; ragged in both directions)."""
+    cols = 512 if prologue else 768
+    ws = [ctx.buffer_bytes(synth.q4k_blocks(rows * cols // 256, 670 + i)) for i in range(2)]
+    x, res, wv = (ctx.buffer_f32(synth.normal_f32(n, 672 + i)) for i, n in enumerate((batch * cols, batch * cols, cols)))
+    pro = [wv, res, wv] if prologue else []
+    outs = []
+    for mode in (0, 3):
+        k = ctx.compile(hip.make_desc(hip.Kind.MATVEC_BATCH, (rows, cols, batch, rows, 0, prologue, mode), (DType.Q4K, DType.F32, DType.F32), (1e-6,),
+                                      dict(k_split=1)))
+        ys = [ctx.buffer_empty_f32(batch * rows) for _ in range(1 if mode else 2)]
+        xn = [ctx.buffer_empty_f32(batch * cols)] if prologue else []
+        ctx.encode_multi(k, [ws[0], x, ws[1]] + pro, ys + xn)
+        if not mode:
+            y = ctx.buffer_empty_f32(batch * rows)
+            ctx.encode_multi(ctx.compile(hip.make_desc(hip.Kind.GELU_MUL, (batch * rows,))), ys, [y])
+            ys = [y]
+        ctx.synchronize()
+        outs.append([ctx.read_f32(ys[0], batch * rows)] + [ctx.read_f32(b, batch * cols) for b in xn])
+    assert_close(outs[1][0], outs[0][0], 1e-5, "gelu(gate) * up")
+    if prologue:
+        assert np.array_equal(outs[0][1], outs[1][1])
+
+
 @pytest.mark.parametrize("wdt,batch,rows,cols", [(DType.Q6K, 77, 300, 7936), (DType.Q4K, 77, 300, 7936), (DType.Q4K, 64, 129, 7936),
                                                  (DType.Q6K, 1, 129, 2816), (DType.Q6K, 257, 10881, 1536), (DType.Q4K, 321, 7041, 768)])
 def test_mul_mm_bf16_default_tile_and_slices(ctx, wdt, batch, rows, cols):
