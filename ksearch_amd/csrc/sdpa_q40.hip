@@ -224,6 +224,34 @@ __global__ __launch_bounds__(kThreads) void sdpa_reduce_kernel(const float *tmp,
     if (tid + kThreads < hd) act_st<H>(out, o + tid + kThreads, O1 * inv_l);
 }
 
+// The same for one slot and up to 64 partitions: a lane has one partition's (m, l), the weights are made once per wave and
+// handed out by lane, and sixteen partitions' values are on their way before them (5.2 -> 2.8 us for 8 heads of 256 in 16
+// partitions: a launch of eight workgroups takes as long as its program).
+template <bool H>
+__global__ __launch_bounds__(kThreads) void sdpa_reduce_few_kernel(const float *tmp, float *out, int n_q, int hd, int nwg)
+{
+    constexpr int B = 16;
+    const int head = blockIdx.x, tid = threadIdx.x, lane = tid & 63, rs = hd + 2;
+    const float *base = tmp + (size_t)head * nwg * rs;
+    const float2 ml = ldg_f2(base + min(lane, nwg - 1) * rs, 0);
+    for (int d = tid; d - lane < hd; d += kThreads) {
+        const float *vb = base + 2 + min(d, hd - 1);
+        float v[B];
+#pragma unroll
+        for (int u = 0; u < B; u++) v[u] = vb[min(u, nwg - 1) * rs];
+        const float m = wave_max(ml.x), w = lane < nwg ? __expf(ml.x - m) : 0.f, l = wave_sum(w * ml.y);
+        float o = 0.f;
+        for (int p0 = 0; p0 < nwg; p0 += B) {
+            if (p0)
+#pragma unroll
+                for (int u = 0; u < B; u++) v[u] = vb[min(p0 + u, nwg - 1) * rs];
+#pragma unroll
+            for (int u = 0; u < B; u++) o = fmaf(as_f32((uint32_t)__builtin_amdgcn_readlane((int)as_u32(w), (p0 + u) & 63)), v[u], o);
+        }
+        if (d < hd) act_st<H>(out, (size_t)head * hd + d, o / l);
+    }
+}
+
 size_t part_lds_bytes(int groups, int hd)
 {
     return ((size_t)groups * hd + 2 * (size_t)kTile * (hd + 4) + (size_t)kMaxGroups * kTile + kMaxGroups) * sizeof(float);
@@ -280,7 +308,8 @@ template <bool H>
 int launch_mwg_reduce(const ksh_kernel &k, const LaunchArgs &a, hipStream_t st)
 {
     const int n_q = (int)k.desc.dims[0], hd = (int)k.desc.dims[1], nwg = (int)k.desc.dims[2];
-    hipLaunchKernelGGL(sdpa_reduce_kernel<H>, dim3(n_q, 1), dim3(kThreads), 0, st, (const float *)a.in[0],
+    auto *kernel = nwg <= 64 ? sdpa_reduce_few_kernel<H> : sdpa_reduce_kernel<H>;
+    hipLaunchKernelGGL(kernel, dim3(n_q, 1), dim3(kThreads), 0, st, (const float *)a.in[0],
                        (float *)a.out[0], n_q, hd, nwg);
     return done("sdpa_mwg_reduce launch");
 }

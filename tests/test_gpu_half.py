@@ -260,7 +260,7 @@ def test_rmsnorm_half_every_row_length(ctx, n, res, scale, rows):
         assert rel_err(y[s], want.astype(np.float16).astype(np.float32)).max() <= BAR
 
 
-@pytest.mark.parametrize("n_q,n_kv,hd,nwg,tlen", [(8, 1, 256, 16, 700), (8, 1, 512, 5, 301), (4, 2, 128, 9, 77), (2, 2, 256, 1, 30)])
+@pytest.mark.parametrize("n_q,n_kv,hd,nwg,tlen", [(8, 1, 256, 16, 700), (8, 1, 512, 5, 301), (4, 2, 128, 9, 77), (2, 2, 256, 1, 30), (2, 1, 64, 64, 500), (2, 1, 256, 65, 500)])
 def test_split_kv_partials_and_merge_half(ctx, n_q, n_kv, hd, nwg, tlen):
     """Half q into split-KV partials (one head per workgroup at heads of 256 and 512), half result of the merge; partition
     counts around the merge's eight at a time."""
