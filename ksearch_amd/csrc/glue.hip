@@ -379,14 +379,27 @@ __device__ __forceinline__ void argmax_fold(float &bv, uint32_t &bi, float v, ui
     if (v > bv || (v == bv && i < bi)) { bv = v; bi = i; }
 }
 
+template <int CTRL>
+__device__ __forceinline__ uint32_t min_dpp_u32(uint32_t v)
+{
+    return min(v, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, CTRL, 0xF, 0xF, true));
+}
+
+__device__ __forceinline__ uint32_t wave_min_u32(uint32_t v)
+{
+    v = min_dpp_u32<0x140>(min_dpp_u32<0x141>(min_dpp_u32<0x4E>(min_dpp_u32<0xB1>(v))));   // (each row of sixteen lanes, as wave_max)
+    const uint32_t a = (uint32_t)__builtin_amdgcn_readlane((int)v, 0), b = (uint32_t)__builtin_amdgcn_readlane((int)v, 16);
+    const uint32_t c = (uint32_t)__builtin_amdgcn_readlane((int)v, 32), d = (uint32_t)__builtin_amdgcn_readlane((int)v, 48);
+    return min(min(a, b), min(c, d));
+}
+
 __device__ __forceinline__ void argmax_block(float &bv, uint32_t &bi, float *sv, uint32_t *si)
 {
-#pragma unroll
-    for (int off = 32; off >= 1; off >>= 1) {
-        const float ov = __shfl_xor(bv, off, 64);
-        const uint32_t oi = (uint32_t)__shfl_xor((int)bi, off, 64);
-        argmax_fold(bv, bi, ov, oi);
-    }
+    // the wave's largest value, then the smallest index that has it (in the lanes' registers: as six exchanges of a pair
+    // through the LDS path this was half a microsecond)
+    const float m = wave_max(bv);
+    bi = wave_min_u32(bv == m ? bi : 0xFFFFFFFFu);
+    bv = m;
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     if (lane == 0) { sv[wave] = bv; si[wave] = bi; }
     __syncthreads();
@@ -405,9 +418,15 @@ __global__ __launch_bounds__(kArgThreads) void softcap_argmax_part_kernel(const 
     x += (size_t)blockIdx.y * n;
     pv += (size_t)blockIdx.y * gridDim.x;
     pi += (size_t)blockIdx.y * gridDim.x;
-    for (int i = blockIdx.x * kArgThreads + threadIdx.x; i < n; i += gridDim.x * kArgThreads) {
-        const float y = cap > 0.0f ? cap * tanhf(x[i] / cap) : x[i];
-        argmax_fold(bv, bi, y, (uint32_t)i);
+    // (four values in flight: one at a time, 256 workgroups over 262144 values waited for memory four times)
+    const int stride = gridDim.x * kArgThreads;
+    for (int i0 = blockIdx.x * kArgThreads + threadIdx.x; i0 < n; i0 += 4 * stride) {
+        float v[4];
+#pragma unroll
+        for (int u = 0; u < 4; u++) v[u] = x[min((size_t)i0 + (size_t)u * stride, (size_t)n - 1)];
+#pragma unroll
+        for (int u = 0; u < 4; u++)
+            if (u == 0 || (size_t)i0 + (size_t)u * stride < (size_t)n) argmax_fold(bv, bi, cap > 0.0f ? cap * tanhf(v[u] / cap) : v[u], (uint32_t)(i0 + u * stride));
     }
     argmax_block(bv, bi, sv, si);
     if (threadIdx.x == 0) { pv[blockIdx.x] = bv; pi[blockIdx.x] = bi; }
@@ -457,11 +476,18 @@ __global__ __launch_bounds__(kArgThreads) void decode_tail_kernel(DecodeTail t)
     }
     int64_t id = (int64_t)s_id;
     id = id >= t.n_rows ? t.n_rows - 1 : id;    // never read outside the table
-    for (int i = threadIdx.x; i < t.n; i += kArgThreads) {
-        float v;
-        if (t.dtype == KSH_Q6K) v = deq_q6k_at(t.embd + (size_t)id * (size_t)(t.n / 256) * 210 + (size_t)(i >> 8) * 210, i & 255);
-        else v = deq_q4k_at(t.embd + (size_t)id * (size_t)(t.n / 256) * 144 + (size_t)(i >> 8) * 144, i & 255);
-        t.x_out[i] = t.scale * v;
+    // (a thread's elements of four superblocks in flight)
+    const uint8_t *row = t.embd + (size_t)id * (size_t)(t.n / 256) * (t.dtype == KSH_Q6K ? 210 : 144);
+    for (int s0 = 0; s0 < t.n / 256; s0 += 4) {
+        float v[4];
+#pragma unroll
+        for (int u = 0; u < 4; u++) {
+            const int sb = min(s0 + u, t.n / 256 - 1);
+            v[u] = t.dtype == KSH_Q6K ? deq_q6k_at(row + sb * 210, threadIdx.x) : deq_q4k_at(row + sb * 144, threadIdx.x);
+        }
+#pragma unroll
+        for (int u = 0; u < 4; u++)
+            if (s0 + u < t.n / 256) t.x_out[(s0 + u) * 256 + threadIdx.x] = t.scale * v[u];
     }
 }
 
