@@ -996,9 +996,10 @@ __device__ __forceinline__ int mfma_k_elem(int s, int kq)
 template <int HD>
 constexpr int mfma_k_pitch() { return HD / 32 * 18 + (HD == 512 ? 16 : 0); }
 
-// HDV < HD (heads of 512 as two halves of 256): the workgroups of blockIdx.y = 2 * kvh + half both work out the scores
-// and the softmax over all HD dimensions (the same numbers twice) and each takes P.V for its HDV dimensions of V,
-// whose accumulators are what limits the head size a wave can hold.
+// HDV < HD (heads of 512, whose accumulators of P.V are more than a wave can hold): a tile has two waves.  Each takes the
+// scores of sixteen of its rows over all HD dimensions -- K rows and their scales are its own -- the two trade scores
+// through LDS (one barrier a step, two buffers), both keep the softmax, and each multiplies all 32 rows into its HDV
+// dimensions of V.  As two workgroups that both worked out all the scores, 952 tokens behind 2048 took 825 us; so 497.
 // BAL: the launch whose partitions are dealt to the slots by length (p.balance), known when the kernel is built: either
 // form's front then holds its own way to its rows only.
 // PVX (eight waves with tiles of 16 rows, heads of 256): the waves share P.V by V block instead of by rows.  Every wave
@@ -1007,22 +1008,25 @@ constexpr int mfma_k_pitch() { return HD / 32 * 18 + (HD == 512 ? 16 : 0); }
 // the workgroup, so the eight-way fold of whole states through LDS and the pass that merges them fall away (they took
 // a quarter of the launch) and every wave stores its own slice of the record.
 template <int HD, int TR, int HDV = HD, bool BAL = false, bool PVX = false>
-__global__ __launch_bounds__(kMfmaRound / TR * 64, TR == 32 ? 2 : 1) void sdpa_mfma_kernel(LaneParams p_in)
+__global__ __launch_bounds__(kMfmaRound / TR * (HD / HDV) * 64, TR == 32 ? 2 : 1) void sdpa_mfma_kernel(LaneParams p_in)
 {
     LaneParams p = p_in;
     p.balance = BAL;
     static_assert(TR == 16 || TR == 32, "tile rows");
     static_assert(!PVX || (TR == 16 && HDV == HD && HD / 32 == kMfmaRound / TR), "a V block per wave");
-    static_assert(HD % HDV == 0 && (HDV == HD || TR == 32), "V halves come with tiles of 32 rows");
+    static_assert(HDV == HD || (HD == 2 * HDV && TR == 32 && !BAL), "two V halves come with tiles of 32 rows");
     touch_lane_params(p_in);   // every kernel argument in one round trip
     KSH_STAMP_BEGIN
-    constexpr int NW = kMfmaRound / TR, NT = NW * 64, NB = HD / 32, ROWB = NB * 18, TILEB = TR * mfma_k_pitch<HD>();
+    constexpr bool SHARE = HDV != HD;
+    constexpr int NW = kMfmaRound / TR, WAVES = NW * (HD / HDV), NT = WAVES * 64, NB = HD / 32, ROWB = NB * 18;   // NW tiles at a time
+    constexpr int TRK = SHARE ? TR / 2 : TR, TILEB = TRK * mfma_k_pitch<HD>();   // rows whose scores a wave takes
     constexpr int KPITCH = mfma_k_pitch<HD>();                             // bytes from one K row of the tile to the next in LDS
     constexpr int NBV = HDV / 32, ROWBV = NBV * 18, TILEBV = TR * ROWBV;   // this workgroup's share of a V row
-    constexpr int STRIP = TILEB + TILEBV + TR * NB * 4 + TR * NBV * 4;     // K bytes, V bytes, K scales, V scales
-    constexpr int PIECES = TR * ROWB / 16, PIECESV = TR * ROWBV / 16;      // 128-bit pieces of a tile
+    constexpr int STRIP = TILEB + TILEBV + TRK * NB * 4 + TR * NBV * 4;    // K bytes, V bytes, K scales, V scales
+    constexpr int PIECES = TRK * ROWB / 16, PIECESV = TR * ROWBV / 16;      // 128-bit pieces of a tile
     extern __shared__ __attribute__((aligned(16))) uint8_t lds_raw[];
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int tile = wave % NW, vhalf = wave / NW;      // (vhalf: 0 but for the second waves of the tiles of 512-wide heads)
     const int col = lane & 15, q4 = lane >> 4, head = col & 7, is_lo = col >> 3;
     const uint32_t odd_mask = 0u - (uint32_t)(q4 & 1);     // all ones in the lane groups whose accumulator rows are heads 4..7
     uint32_t nib_mask = 0x03C003C0u, nib_one = 0x4C004C00u;  // a nibble's place in an f16 mantissa; 16.0 twice
@@ -1033,10 +1037,10 @@ __global__ __launch_bounds__(kMfmaRound / TR * 64, TR == 32 ? 2 : 1) void sdpa_m
     const uint32_t drop = is_lo ? 0xFFFFE000u : 0u;
     uint8_t *strip = lds_raw + (size_t)wave * STRIP;
     uint8_t *kraw = strip, *vraw = strip + TILEB;
-    float *ksc = reinterpret_cast<float *>(strip + TILEB + TILEBV), *vsc = ksc + TR * NB;
+    float *ksc = reinterpret_cast<float *>(strip + TILEB + TILEBV), *vsc = ksc + TRK * NB;
 
     int part = blockIdx.x, slot = blockIdx.z, nparts = p.nwg;
-    const int kvh = blockIdx.y / (HD / HDV), vhalf = blockIdx.y % (HD / HDV), groups = p.groups, head0 = kvh * groups;
+    const int kvh = blockIdx.y, groups = p.groups, head0 = kvh * groups;
     size_t rec_base = 0;
     int p0, p1, start;
     if (p.balance) {
@@ -1073,8 +1077,8 @@ __global__ __launch_bounds__(kMfmaRound / TR * 64, TR == 32 ? 2 : 1) void sdpa_m
     constexpr int NPC = (PIECES + 63) / 64, NPCV = (PIECESV + 63) / 64;
     u32x4_t kpre[NPC], vpre[NPCV];
     auto fetch_tile = [&](int it) __attribute__((always_inline)) {
-        const int row0 = p0 + (it * NW + wave) * TR;
-        const int nvalid = max(0, min(TR, p1 - row0));
+        const int row0 = p0 + (it * NW + tile) * TR + (SHARE ? TRK * vhalf : 0);      // K (and, in one piece, V)
+        const int nvalid = max(0, min(TRK, p1 - row0));
 #pragma unroll
         for (int u = 0; u < NPC; u++) {
             const int idx = lane + 64 * u, row = idx / (ROWB / 16), pc = idx % (ROWB / 16);
@@ -1086,13 +1090,14 @@ __global__ __launch_bounds__(kMfmaRound / TR * 64, TR == 32 ? 2 : 1) void sdpa_m
                 if (HDV == HD) vpre[u] = *reinterpret_cast<const u32x4_t *>(vbase + off);
             }
         }
-        if (HDV != HD) {
+        if (SHARE) {
+            const int vrow0 = p0 + (it * NW + tile) * TR, vvalid = max(0, min(TR, p1 - vrow0));
 #pragma unroll
             for (int u = 0; u < NPCV; u++) {
                 const int idx = lane + 64 * u, row = idx / (ROWBV / 16), pc = idx % (ROWBV / 16);
                 vpre[u] = u32x4_t{0u, 0u, 0u, 0u};
-                if (idx < PIECESV && row < nvalid)
-                    vpre[u] = *reinterpret_cast<const u32x4_t *>(vbase + (size_t)(start + row0 + row) * row_stride + (size_t)pc * 16);
+                if (idx < PIECESV && row < vvalid)
+                    vpre[u] = *reinterpret_cast<const u32x4_t *>(vbase + (size_t)(start + vrow0 + row) * row_stride + (size_t)pc * 16);
             }
         }
     };
@@ -1101,27 +1106,27 @@ __global__ __launch_bounds__(kMfmaRound / TR * 64, TR == 32 ? 2 : 1) void sdpa_m
     // w, w + NW, ... and the workgroup shares them through LDS (behind the strips).  q is asked for before the tile:
     // loads come back in the order they went out, q is the short way (it was just written) and its preparation
     // then runs while the tile is on its way.
-    static_assert(NB % NW == 0, "the q blocks divide among the waves");
-    constexpr int QPW = NB / NW;
+    static_assert(NB % WAVES == 0, "the q blocks divide among the waves");
+    constexpr int QPW = NB / WAVES;
     h8v qop[NB];
     float qs24[NB];
     {
-        // (heads of 512: the shared operands lie over the strips, which nothing has written yet, so that two workgroups fit a compute unit)
-        h8v *qshare = reinterpret_cast<h8v *>(lds_raw + (HDV == HD ? (size_t)NW * STRIP : 0));       // [NB][64] operands
-        float *qsum_share = HDV == HD ? reinterpret_cast<float *>(qshare + NB * 64) : reinterpret_cast<float *>(lds_raw + (size_t)NW * STRIP);   // [NB][64]
+        // (heads of 512: the shared operands lie over the strips, which nothing has written yet, and both fit a compute unit's LDS beside the traded scores)
+        h8v *qshare = reinterpret_cast<h8v *>(lds_raw + (HDV == HD ? (size_t)WAVES * STRIP : 0));       // [NB][64] operands
+        float *qsum_share = HDV == HD ? reinterpret_cast<float *>(qshare + NB * 64) : reinterpret_cast<float *>(lds_raw + (size_t)WAVES * STRIP);   // [NB][64]
         const float *qh = p.q + ((size_t)slot * p.n_q + head0 + min(head, groups - 1)) * HD;
         const bool have = head < groups;
         float4 qlo[QPW], qhi[QPW];
 #pragma unroll
         for (int u = 0; u < QPW; u++) {
-            const int b = wave + NW * u;
+            const int b = wave + WAVES * u;
             qlo[u] = *reinterpret_cast<const float4 *>(qh + 32 * b + 4 * q4);        // elements 4kq .. 4kq+3
             qhi[u] = *reinterpret_cast<const float4 *>(qh + 32 * b + 16 + 4 * q4);   // 16+4kq .. 16+4kq+3
         }
         if (HDV == HD) fetch_tile(0);      // (heads of 512 have no registers to hold a tile across the q preparation)
 #pragma unroll
         for (int u = 0; u < QPW; u++) {
-            const int b = wave + NW * u;
+            const int b = wave + WAVES * u;
             const float4 lo4 = qlo[u], hi4 = qhi[u];
             const float x[8] = {lo4.x, lo4.z, hi4.x, hi4.z, lo4.y, lo4.w, hi4.y, hi4.w};       // slot order (mfma_k_elem)
             h8v op;
@@ -1164,8 +1169,9 @@ __global__ __launch_bounds__(kMfmaRound / TR * 64, TR == 32 ? 2 : 1) void sdpa_m
     const int ntiles = (p1 - p0 + TR - 1) / TR;
     const int nsteps = (ntiles + NW - 1) / NW;               // the same for every wave: the barriers below are uniform
     for (int it = 0; it < nsteps; it++) {
-        const int row0 = p0 + (it * NW + wave) * TR;
+        const int row0 = p0 + (it * NW + tile) * TR;
         const int nvalid = max(0, min(TR, p1 - row0));         // wave-uniform
+        const int kvalid = SHARE ? max(0, min(TRK, nvalid - TRK * vhalf)) : nvalid;   // of the rows whose scores are this wave's
         // The strip belongs to this wave alone, and a wave's LDS operations complete in the order they were issued:
         // no workgroup barrier in this loop, only fences that keep the compiler from moving accesses across them.
         // (Later tiles are requested here, not a tile ahead: forty registers less make room for a second wave per
@@ -1190,10 +1196,10 @@ __global__ __launch_bounds__(kMfmaRound / TR * 64, TR == 32 ? 2 : 1) void sdpa_m
         __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
         // ---- block scales as f32 tables [row][block]; rows past the end get 0 (their codes are zeros too)
 #pragma unroll
-        for (int u = 0; u < TR * NB / 64; u++) {
-            const int idx = lane + 64 * u, b = idx / TR, row = idx % TR;      // tables are [block][row]
+        for (int u = 0; u < TRK * NB / 64; u++) {
+            const int idx = lane + 64 * u, b = idx / TRK, row = idx % TRK;    // tables are [block][row]
             const uint32_t kb = *reinterpret_cast<const uint16_t *>(kraw + row * KPITCH + 18 * b);
-            ksc[idx] = row < nvalid ? half_bits_to_f32(kb) : 0.f;
+            ksc[idx] = row < kvalid ? half_bits_to_f32(kb) : 0.f;
             if (HDV == HD) {
                 const uint32_t vb = *reinterpret_cast<const uint16_t *>(vraw + row * ROWBV + 18 * b);
                 vsc[idx] = row < nvalid ? half_bits_to_f32(vb) : 0.f;
@@ -1301,33 +1307,48 @@ __global__ __launch_bounds__(kMfmaRound / TR * 64, TR == 32 ? 2 : 1) void sdpa_m
             Tl[0] += tsum;
             if (it + 1 == nsteps) { KSH_STAMP_USE(O[1][3]); KSH_STAMP(5); }
             if (it + 1 < nsteps) __syncthreads();      // the strips and the exchange are written again
-        } else
-        if (nvalid > 0) {
+        } else {
             // ---- scores of the tile's two 16-row halves: lane (col, q4) ends up with rows 4*q4 + r of each
             constexpr int NS = TR / 4;                       // scores (rows) per lane
             float sv[NS];
+            if (nvalid > 0) {
 #pragma unroll
-            for (int t = 0; t < TR / 16; t++) {
-                float acc[4] = {0.f, 0.f, 0.f, 0.f};
+                for (int t = 0; t < TRK / 16; t++) {
+                    float acc[4] = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-                for (int b = 0; b < NB; b++) {
-                    const float4 dk4 = *reinterpret_cast<const float4 *>(ksc + b * TR + 16 * t + 4 * q4);   // rows 4*q4 .. +3
-                    const float dk[4] = {dk4.x, dk4.y, dk4.z, dk4.w};
-                    // A operand: row (16t + lane % 16), bytes 4*q4 .. 4*q4+3 of block b (2-byte aligned)
-                    const uint8_t *src = kraw + (16 * t + col) * KPITCH + 18 * b + 2 + 4 * q4;
-                    const uint32_t d = (uint32_t)*reinterpret_cast<const uint16_t *>(src) |
-                                       ((uint32_t)*reinterpret_cast<const uint16_t *>(src + 2) << 16);
-                    const f4v c = __builtin_amdgcn_mfma_f32_16x16x32_f16(nibbles_f16(d, nib_mask, nib_one), qop[b], f4v{0.f, 0.f, 0.f, 0.f}, 0, 0, 0);
-                    const float q24 = HDV == HD ? qs24[b] : reinterpret_cast<const float *>(lds_raw + (size_t)NW * STRIP)[b * 64 + lane];
+                    for (int b = 0; b < NB; b++) {
+                        const float4 dk4 = *reinterpret_cast<const float4 *>(ksc + b * TRK + 16 * t + 4 * q4);   // rows 4*q4 .. +3
+                        const float dk[4] = {dk4.x, dk4.y, dk4.z, dk4.w};
+                        // A operand: row (16t + lane % 16), bytes 4*q4 .. 4*q4+3 of block b (2-byte aligned)
+                        const uint8_t *src = kraw + (16 * t + col) * KPITCH + 18 * b + 2 + 4 * q4;
+                        const uint32_t d = (uint32_t)*reinterpret_cast<const uint16_t *>(src) |
+                                           ((uint32_t)*reinterpret_cast<const uint16_t *>(src + 2) << 16);
+                        const f4v c = __builtin_amdgcn_mfma_f32_16x16x32_f16(nibbles_f16(d, nib_mask, nib_one), qop[b], f4v{0.f, 0.f, 0.f, 0.f}, 0, 0, 0);
+                        const float q24 = HDV == HD ? qs24[b] : reinterpret_cast<const float *>(lds_raw + (size_t)WAVES * STRIP)[b * 64 + lane];
 #pragma unroll
-                    for (int r = 0; r < 4; r++) acc[r] = fmaf(dk[r], c[r] - q24, acc[r]);
-                }
+                        for (int r = 0; r < 4; r++) acc[r] = fmaf(dk[r], c[r] - q24, acc[r]);
+                    }
 #pragma unroll
-                for (int r = 0; r < 4; r++) {
-                    const float tot = acc[r] + dpp_f32<0x128>(acc[r]);        // hi + lo column (row_ror:8)
-                    sv[4 * t + r] = (16 * t + 4 * q4 + r) < nvalid ? tot : -1.0e30f;
+                    for (int r = 0; r < 4; r++) {
+                        const float tot = acc[r] + dpp_f32<0x128>(acc[r]);        // hi + lo column (row_ror:8)
+                        sv[4 * t + r] = (16 * t + 4 * q4 + r) < kvalid ? tot : -1.0e30f;
+                    }
                 }
             }
+            if constexpr (SHARE) {
+                // (two buffers: the other wave may still be reading the last step's)
+                float4 *xch = reinterpret_cast<float4 *>(lds_raw + (size_t)WAVES * STRIP + (size_t)NB * 64 * 4) + ((it & 1) * NW + tile) * 2 * 64 + lane;
+                if (nvalid > 0) xch[64 * vhalf] = make_float4(sv[0], sv[1], sv[2], sv[3]);
+                __syncthreads();
+                if (nvalid > 0) {
+#pragma unroll
+                    for (int h = 0; h < 2; h++) {
+                        const float4 s4 = xch[64 * h];
+                        sv[4 * h] = s4.x; sv[4 * h + 1] = s4.y; sv[4 * h + 2] = s4.z; sv[4 * h + 3] = s4.w;
+                    }
+                }
+            }
+            if (nvalid > 0) {
             // ---- online softmax over the tile (per column; the maximum across the wave's four lane groups)
             float mt = sv[0];
 #pragma unroll
@@ -1404,6 +1425,7 @@ __global__ __launch_bounds__(kMfmaRound / TR * 64, TR == 32 ? 2 : 1) void sdpa_m
                     O[2 * b + 1] = __builtin_amdgcn_mfma_f32_16x16x16f16(pa4, __builtin_bit_cast(h4v, hi2), O[2 * b + 1], 0, 0, 0);
                 }
             }
+            }
         }
     }
 
@@ -1446,8 +1468,8 @@ __global__ __launch_bounds__(kMfmaRound / TR * 64, TR == 32 ? 2 : 1) void sdpa_m
     }
     // ---- fold: every wave's state to LDS (hi rows first, lo rows added), then one record per head
     __syncthreads();
-    float *ow = reinterpret_cast<float *>(lds_raw);            // [NW][8][HDV]
-    float *mlw = ow + NW * 8 * HDV;                            // [NW][8][2]
+    float *ow = reinterpret_cast<float *>(lds_raw);            // [V half][NW][8][HDV]
+    float *mlw = ow + WAVES * 8 * HDV;                         // [NW][8][2]
     const float l_tot = xor32_sum(xor16_sum(l_run));
     // sum(P') of head h and block b: the four lane groups of column h hold its parts.  The accumulator layout wants
     // it by row (head 4 * (q4 & 1) + r): read from lane h as a scalar, picked bitwise like the rescale factors.
@@ -1477,12 +1499,12 @@ __global__ __launch_bounds__(kMfmaRound / TR * 64, TR == 32 ? 2 : 1) void sdpa_m
             }
         }
     }
-    if (lane < 8) { mlw[(wave * 8 + lane) * 2] = m_run; mlw[(wave * 8 + lane) * 2 + 1] = l_tot; }
+    if (lane < 8 && wave < NW) { mlw[(wave * 8 + lane) * 2] = m_run; mlw[(wave * 8 + lane) * 2 + 1] = l_tot; }
     __syncthreads();
-    static_assert(NT % HDV == 0 || HDV % NT == 0, "whole heads per pass, or whole passes per head");
+    static_assert(NT % HD == 0 || HD % NT == 0, "whole heads per pass, or whole passes per head");
 #pragma unroll
-    for (int o = tid; o < 8 * HDV; o += NT) {
-        const int h = o / HDV, d = o % HDV, hq = head0 + h;      // (h is the same for a whole wave)
+    for (int o = tid; o < 8 * HD; o += NT) {
+        const int h = o / HD, d = o % HD, hq = head0 + h;      // (h is the same for a whole wave)
         if (h >= groups) break;
         float M = -1.0e30f;
 #pragma unroll
@@ -1492,19 +1514,19 @@ __global__ __launch_bounds__(kMfmaRound / TR * 64, TR == 32 ? 2 : 1) void sdpa_m
         for (int w = 0; w < NW; w++) {
             const float wt = __expf(mlw[(w * 8 + h) * 2] - M);
             L = fmaf(wt, mlw[(w * 8 + h) * 2 + 1], L);
-            a = fmaf(wt, ow[((size_t)w * 8 + h) * HDV + d], a);
+            a = fmaf(wt, ow[((size_t)(d / HDV * NW + w) * 8 + h) * HDV + d % HDV], a);
         }
         if (p.balance) {
             const size_t r = rec_base * p.n_q + hq;
             float *ml = p.tmp + (size_t)gridDim.z * p.nwg * p.n_q * HD;
-            p.tmp[r * HD + vhalf * HDV + d] = a;
-            if (d == 0 && vhalf == 0) { ml[2 * r] = M; ml[2 * r + 1] = L; }
+            p.tmp[r * HD + d] = a;
+            if (d == 0) { ml[2 * r] = M; ml[2 * r + 1] = L; }
         } else if (p.nwg == 1 && p.out) {
-            p.out[((size_t)slot * p.n_q + hq) * HD + vhalf * HDV + d] = a / L;      // one partition: nothing left to merge
+            p.out[((size_t)slot * p.n_q + hq) * HD + d] = a / L;      // one partition: nothing left to merge
         } else {
             float *rec = p.tmp + (size_t)slot * p.n_q * p.nwg * (HD + 2) + (size_t)hq * p.nwg * (HD + 2) + (size_t)part * (HD + 2);
-            rec[2 + vhalf * HDV + d] = a;
-            if (d == 0 && vhalf == 0) { rec[0] = M; rec[1] = L; }
+            rec[2 + d] = a;
+            if (d == 0) { rec[0] = M; rec[1] = L; }
         }
     }
 }
@@ -1531,12 +1553,13 @@ __global__ __launch_bounds__(HD) void sdpa_records_merge_kernel(const float *__r
 template <int HD, int TR, int HDV = HD, bool PVX = false>
 constexpr size_t mfma_lds_bytes()
 {
-    constexpr size_t waves = kMfmaRound / TR;
-    constexpr size_t strip = (size_t)TR * mfma_k_pitch<HD>() + (size_t)TR * (HDV / 32 * 18) + (size_t)TR * (HD / 32) * 4 + (size_t)TR * (HDV / 32) * 4;
+    constexpr size_t waves = kMfmaRound / TR * (HD / HDV), krows = TR / (HD / HDV);
+    constexpr size_t strip = krows * mfma_k_pitch<HD>() + (size_t)TR * (HDV / 32 * 18) + krows * (HD / 32) * 4 + (size_t)TR * (HDV / 32) * 4;
     constexpr size_t qshare = (size_t)(HD / 32) * 64 * (16 + 4);                 // the shared q operands and sums
     constexpr size_t fold = waves * 8 * HDV * 4 + waves * 8 * 2 * 4;
     constexpr size_t qsum = (size_t)(HD / 32) * 64 * 4;
-    constexpr size_t front = HDV == HD ? strip * waves + qshare : strip * waves + qsum;   // (HDV < HD: the operands lie over the strips, the sums behind them)
+    constexpr size_t trade = 2 * waves * 64 * 16;                                         // the scores two waves trade, two buffers
+    constexpr size_t front = HDV == HD ? strip * waves + qshare : strip * waves + qsum + trade;   // (HDV < HD: the operands lie over the strips, the sums behind them)
     if (PVX) return front + (8 * kMfmaRound + 2 * waves * 8) * 4;                         // + the probabilities, maxima and sums the waves exchange; no fold
     return front > fold ? front : fold;
 }
@@ -1714,8 +1737,8 @@ int launch_bound(const ksh_kernel &k, const LaunchArgs &a, hipStream_t st)
             }
             p.balance = 0;
             p.mode = kModePart;
-            if (hd == 512)   // two workgroups per kv head, each with half of the V dimensions
-                hipLaunchKernelGGL((sdpa_mfma_kernel<512, 32, 256>), dim3(p.nwg, p.n_kv * 2, n_slots), dim3(kMfmaRound / 32 * 64), (mfma_lds_bytes<512, 32, 256>()), st, p);
+            if (hd == 512)   // two waves a tile, each with half of the V dimensions
+                hipLaunchKernelGGL((sdpa_mfma_kernel<512, 32, 256>), dim3(p.nwg, p.n_kv, n_slots), dim3(kMfmaRound / 32 * 2 * 64), (mfma_lds_bytes<512, 32, 256>()), st, p);
             else
                 hipLaunchKernelGGL((sdpa_mfma_kernel<256, 32>), dim3(p.nwg, p.n_kv, n_slots), dim3(kMfmaRound / 32 * 64), (mfma_lds_bytes<256, 32>()), st, p);
             const hipError_t e0 = hipGetLastError();
@@ -1797,13 +1820,14 @@ int bind_sdpa_lanes(ksh_kernel &k, int nwg, int n_slots)
     if (long_batch && ((k.desc.sched.vec == 2 && (!batch_fits || k.desc.dims[6])) || k.desc.sched.vec == 0)) {
         if (k.desc.sched.lds_tile && k.desc.sched.lds_tile != 32) return set_error("sdpa_batch: the matrix-core form of a long chunk takes tiles of 32 rows (lds_tile=%u)", k.desc.sched.lds_tile);
         k.scratch_bytes = (((size_t)n_slots * n_kv * 4 + 15) & ~(size_t)15) + (size_t)n_slots * 16;
-        // (heads of 512: two workgroups per kv head, each with all of the scores and half of the V dimensions)
-        set_launch(k, (uint32_t)nwg, (uint32_t)(hd == 512 ? 2 * n_kv : n_kv), (uint32_t)n_slots, kMfmaRound / 32 * 64,
+        // (heads of 512: two waves a tile)
+        const int waves = kMfmaRound / 32 * (hd == 512 ? 2 : 1);
+        set_launch(k, (uint32_t)nwg, (uint32_t)n_kv, (uint32_t)n_slots, waves * 64,
                    (uint32_t)(hd == 512 ? mfma_lds_bytes<512, 32, 256>() : mfma_lds_bytes<256, 32>()));
         k.info.sched = k.desc.sched;
         k.info.sched.vec = 2;
-        k.info.sched.tg = kMfmaRound / 32 * 64;
-        k.info.sched.nsg = kMfmaRound / 32;
+        k.info.sched.tg = waves * 64;
+        k.info.sched.nsg = waves;
         k.info.sched.k_split = (uint32_t)nwg;
         k.info.sched.lds_tile = 32;
         k.info.sched.unroll = 1;
