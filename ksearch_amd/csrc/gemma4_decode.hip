@@ -1141,6 +1141,16 @@ constexpr int kRoundMax = 16;         // the attention launch shares its partiti
 constexpr int kRoundPartitions = 16;
 constexpr int kRoundStride = 16;      // floats per field of the table: ids | slots | full-attention records | sliding-window records
 
+// A round's table as an argument of the launch that stores it: the stream keeps the order, no wait for the copy engine (nor
+// for the previous round's last reader).
+struct RoundTable {
+    float v[kRoundStride * 10];
+};
+__global__ void round_table_kernel(RoundTable t, float *out)
+{
+    for (int i = threadIdx.x; i < kRoundStride * 10; i += 64) out[i] = t.v[i];
+}
+
 int pool_fits(const ksh_gemma4 *m, const ksh_kvpool *pool, int *max_batch, int *pool_hd)
 {
     const ksh_gemma4_cfg &c = m->c;
@@ -1212,7 +1222,8 @@ int forward_decode_round4(ksh_gemma4 *m, ksh_kvpool *pool, const int32_t *slots,
                       alloc(m, (size_t)kRoundMax * 4, &m->r_next) || alloc(m, (size_t)(64 * widest + 2048 * (widest / 256)), &m->r_xp) ||
                       alloc(m, (size_t)(64 * widest + 2048 * (widest / 256)), &m->r_xp2)))
         return 1;
-    float tab[kRoundStride * 10] = {};
+    RoundTable table{};
+    float *tab = table.v;
     for (int i = 0; i < t; i++) {
         const int pos = ksh_kvpool_seq_len(pool, slots[i]);
         const int kv_len = pos + 1, start = kv_len > c.sliding_window ? kv_len - c.sliding_window : 0;
@@ -1222,8 +1233,9 @@ int forward_decode_round4(ksh_gemma4 *m, ksh_kvpool *pool, const int32_t *slots,
         full[0] = (float)kv_len; full[3] = (float)pos;
         swa[0] = (float)(kv_len - start); swa[1] = (float)start; swa[2] = (float)c.sliding_window; swa[3] = (float)pos;
     }
-    if (ksh_synchronize(m->ctx)) return 1;   // the table may still be read by the previous round
-    if (ksh_buffer_write(m->ctx, m->r_tab, 0, tab, sizeof(tab), 1)) return 1;
+    hipLaunchKernelGGL(round_table_kernel, dim3(1), dim3(64), 0, (hipStream_t)ksh_stream(m->ctx), table, (float *)ksh_buffer_device_ptr(m->r_tab));
+    const hipError_t e = hipGetLastError();
+    if (e != hipSuccess) return hip_fail(e, "round table launch");
     m->r_count = t;
     // The launches of a round depend on its width alone (tokens, slots and positions are in the table): one graph per
     // width, captured at its second round (the first binds the width's kernels, which allocates, and a capture must

@@ -816,6 +816,25 @@ int bind_softcap_argmax(ksh_kernel &k)
 
 }  // namespace ksh
 
+namespace {
+__global__ void copy_short_kernel(uint8_t *dst, const uint8_t *src, int n)
+{
+    if (((uintptr_t)src | (uintptr_t)n) & 3) {
+        for (int i = threadIdx.x; i < n; i += 256) dst[i] = src[i];
+    } else {
+        for (int i = threadIdx.x; i < n / 4; i += 256) ((uint32_t *)dst)[i] = ((const uint32_t *)src)[i];
+    }
+}
+}  // namespace
+
+extern "C" int ksh_copy_short_launch(void *dst, const void *src, size_t bytes, hipStream_t st)
+{
+    using namespace ksh;
+    hipLaunchKernelGGL(copy_short_kernel, dim3(1), dim3(256), 0, st, (uint8_t *)dst, (const uint8_t *)src, (int)bytes);
+    const hipError_t e = hipGetLastError();
+    return e == hipSuccess ? 0 : hip_fail(e, "short copy launch");
+}
+
 extern "C" int ksh_fill_zero_launch(void *ptr, size_t bytes, hipStream_t st)
 {
     using namespace ksh;
