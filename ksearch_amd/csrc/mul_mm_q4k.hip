@@ -379,17 +379,11 @@ struct MmParams {
     const float *cut_as;
 };
 
-// F32 activations: tokens per workgroup of the tile.  64 (Q4_K): up to 64 tokens (the other half of a 128-token tile would
-// be empty rows), and wherever the 128-token tiles and their K slices are fewer than twice the compute units (the tile
-// runs two products per converted weight) -- two workgroups share a compute unit then, and twice as many of them fill the
-// chip.  Beyond that the 128-token tile (prompts of 256 / 1024 / 4000 tokens through cfg4's model: 5.05 / 14.1 / 67.7 ms
-// with this rule, 5.07 / 14.25 / 68.0 with 64-token tiles throughout, 5.3 / 14.9 / 72.7 with 128-token tiles from 65
-// tokens on).
-__host__ __device__ constexpr int mm_tile_tokens(bool q6, int row_tiles, int batch, int ks)
-{
-    if (q6) return 128;
-    return batch <= 64 || (int64_t)((batch + BM - 1) / BM) * row_tiles * ks < 512 ? 64 : 128;
-}
+// F32 activations: tokens per workgroup of the tile.  64 for Q4_K: two workgroups share a compute unit, and with two products
+// per converted weight the second conversion costs less than one workgroup's barriers, first loads and stores cost the
+// matrix pipe when it is alone there (prompts of 700 / 3000 tokens through the two synthetic models 11.7 / 53.7 ms with
+// 128-token tiles for the launches that fill the chip with them, 11.3 / 50.6 so).
+__host__ __device__ constexpr int mm_tile_tokens(bool q6) { return q6 ? 128 : 64; }
 
 // F32 activations, few tiles (a prompt of a few hundred tokens, or a narrow matrix): the nsb superblocks of a row are split
 // into this many K slices, until the grid is about one workgroup per compute unit; every slice has its own sum and the
@@ -401,7 +395,7 @@ __host__ __device__ constexpr int mm_k_slices(bool q6, int row_tiles, int nsb, i
     const int counted = batch > kPrefillPass / 2 ? kPrefillPass / 2 : batch;
     int ks = 1;
     while (nsb % (ks * 2) == 0 && nsb / (ks * 2) >= 2) {
-        const int tm = mm_tile_tokens(q6, row_tiles, counted, ks * 2);
+        const int tm = mm_tile_tokens(q6);
         if ((int64_t)((counted + tm - 1) / tm) * row_tiles * ks * 2 > 256) break;
         ks *= 2;
     }
@@ -777,9 +771,7 @@ __global__ __launch_bounds__(kThreadsMM, TM == 64 ? 2 : 1) void q_mul_mm_kernel(
         const _Float16 *Bs = main_stage(step);
         // B operands a k slice ahead (bf16 / f16 activations on the 128-token tile): left to itself the compiler reads a
         // slice's two operands into the registers the previous slice's products have just released, so every slice
-        // begins with an LDS round trip in front of its four matrix instructions (cfg2: 32.5 -> 31.1 us per pair; with
-        // f32 activations a slice has eight products to hide it behind: prompts of 1024 / 4000 tokens 14.1 / 67.6 ->
-        // 14.0 / 67.1 ms).  The 64-token tile loses by it (a 256-token prompt 5.1 -> 5.3 ms) and keeps the plain order.
+        // begins with an LDS round trip in front of its four matrix instructions (cfg2: 32.5 -> 31.1 us per pair).  The 64-token tile loses by it (a 256-token prompt 5.1 -> 5.3 ms) and keeps the plain order.
         constexpr bool BPIPE = TM == 128;
         h8 bb[2][NW_];
         if (BPIPE) {
@@ -1703,17 +1695,18 @@ int launch_mul_mm(const ksh_kernel &k, const LaunchArgs &a, hipStream_t st)
     p.cut_as = cut ? (const float *)a.in[k.info.n_inputs - 1] : nullptr;
     const bool q6 = k.desc.dtypes[0] == KSH_Q6K;
     auto launch_tile = [&](dim3 g) {
-#define KSH_TILE(Q6, TM, LDS) \
-    do { \
-        if (!Q6 && pair) hipLaunchKernelGGL((q_mul_mm_kernel<Q6, TM, true, false, false, !Q6>), g, dim3(kThreadsMM), LDS, st, p); \
-        else if (cut) hipLaunchKernelGGL((q_mul_mm_kernel<Q6, TM, true, true>), g, dim3(kThreadsMM), LDS, st, p); \
-        else if (f32x) hipLaunchKernelGGL((q_mul_mm_kernel<Q6, TM, true>), g, dim3(kThreadsMM), LDS, st, p); \
-        else if (Q6 && rows_direct) hipLaunchKernelGGL((q_mul_mm_kernel<Q6, TM, false, false, Q6>), g, dim3(kThreadsMM), LDS, st, p); \
-        else hipLaunchKernelGGL((q_mul_mm_kernel<Q6, TM, false>), g, dim3(kThreadsMM), LDS, st, p); \
-    } while (0)
-        if (q6) KSH_TILE(true, 128, kLdsBytes);
-        else if (tm == 64) KSH_TILE(false, 64, kLdsBytes64);
-        else KSH_TILE(false, 128, kLdsBytes);
+#define KSH_TILE(LDS, ...) hipLaunchKernelGGL((q_mul_mm_kernel<__VA_ARGS__>), g, dim3(kThreadsMM), LDS, st, p)
+        if (q6) {
+            if (cut) KSH_TILE(kLdsBytes, true, 128, true, true);
+            else if (f32x) KSH_TILE(kLdsBytes, true, 128, true);
+            else if (rows_direct) KSH_TILE(kLdsBytes, true, 128, false, false, true);
+            else KSH_TILE(kLdsBytes, true, 128, false);
+        } else if (f32x) {
+            if (pair) KSH_TILE(kLdsBytes64, false, 64, true, false, false, true);
+            else if (cut) KSH_TILE(kLdsBytes64, false, 64, true, true);
+            else KSH_TILE(kLdsBytes64, false, 64, true);
+        } else if (tm == 64) KSH_TILE(kLdsBytes64, false, 64, false);
+        else KSH_TILE(kLdsBytes, false, 128, false);
 #undef KSH_TILE
     };
     if (slices) {
@@ -1847,7 +1840,7 @@ int bind_matvec_batch(ksh_kernel &k)
     int tm = 0;
     if (f32x) {
         if (!ks) ks = mm_k_slices(q6, (int)row_tiles, (int)nsb, (int)batch);
-        tm = mm_tile_tokens(q6, (int)row_tiles, (int)batch, (int)ks);
+        tm = mm_tile_tokens(q6);
     } else {
         const MmPlan plan = mm_plan_bf16(q6, (int)row_tiles, (int)nsb, batch, rows_all, (int)ks);
         ks = plan.ks;

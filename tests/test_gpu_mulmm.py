@@ -327,8 +327,8 @@ def test_mul_mm_f32_both_parts_in_one_workgroup(ctx, unfolded, k_split):
 
 @pytest.mark.parametrize("rows,batch,prologue", [(31, 33, 0), (97, 64, 2), (200, 130, 0), (4130, 1000, 2)])
 def test_mul_mm_f32_gate_up_pair(ctx, rows, batch, prologue):
-    """dims[6] = 3: gelu(W x) * (W1 x) from one launch is the two matrices' products and KSH_GELU_MUL (tiles of 64 and of
-    128 tokens, 64 rows of each matrix a tile; ragged in both directions)."""
+    """dims[6] = 3: gelu(W x) * (W1 x) from one launch is the two matrices' products and KSH_GELU_MUL (64 rows of each
+    matrix a tile; ragged in both directions)."""
     cols = 512 if prologue else 768
     ws = [ctx.buffer_bytes(synth.q4k_blocks(rows * cols // 256, 670 + i)) for i in range(2)]
     x, res, wv = (ctx.buffer_f32(synth.normal_f32(n, 672 + i)) for i, n in enumerate((batch * cols, batch * cols, cols)))
