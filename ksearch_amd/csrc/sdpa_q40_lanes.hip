@@ -335,7 +335,11 @@ __device__ __forceinline__ void norm_rope_regs(const float (&xv)[HD / 64], const
 // least one), with c = ceil(T / (P - n_slots)) rows, so that they sum to at most P; what is left over exits.
 // Every workgroup derives the same table from the slots' lengths.  Slot s's partitions are the consecutive
 // flat indices from the sum of its predecessors' counts, and its records sit in that order.
-// round > 1: the rows per partition are rounded up to a multiple of it (the matrix-core form works in tiles of rows).
+// round > 1: the matrix-core form, whose workgroups take `round` rows at a time in tiles of 16 or 32.  A partition is one
+// whole round while that is enough (a part of one costs as much, and more partitions only make the merge longer); beyond,
+// its rows are rounded up to whole tiles of 32 only: 39000 rows over 252 workgroups are 155 each, so 160, where two whole
+// rounds left half of the workgroups without any (4 slots, 16384-row caches: 14.2 -> 12.9 us; what fits one round each, and
+// what fills two or more, as before).
 //
 // A whole wave works the deal out at once, as one short chain of vector instructions (a launch of this kind is a chain
 // of dependent steps: the first form of this routine -- two loops over the slots with a lane read each, three integer
@@ -382,7 +386,8 @@ __device__ __forceinline__ Deal deal_wave(const float *meta, int stride, int n_s
         Tf = (a + b) + (c + d);
     }
     uint32_t c = max(1u, ceil_div_rcp((uint32_t)Tf, spare, rspare));
-    c = (c + (uint32_t)round - 1u) & ~((uint32_t)round - 1u);
+    const uint32_t grain = round > 32 && c > (uint32_t)round ? 32u : (uint32_t)round;
+    c = (c + grain - 1u) & ~(grain - 1u);
     const int n = live ? (int)max(1u, ceil_div_rcp(len, c, __builtin_amdgcn_rcpf((float)c))) : 0;
     // partitions up to and with each lane's slot
     int incl = n;
@@ -1283,6 +1288,7 @@ __global__ __launch_bounds__(kMfmaRound / TR * (HD / HDV) * 64, TR == 32 ? 2 : 1
             float tsum = 0.f;
 #pragma unroll
             for (int j = 0; j < NW; j++) {
+                if (p0 + (it * NW + j) * TR >= p1) break;      // (no rows: the end of the partition)
                 const uint8_t *vj = lds_raw + (size_t)j * STRIP + TILEB;
                 const float *vscj = reinterpret_cast<const float *>(lds_raw + (size_t)j * STRIP + TILEB + TILEBV) + TR * NB;
                 const float4 p4 = *reinterpret_cast<const float4 *>(Psh + head * kMfmaRound + TR * j + 4 * q4);

@@ -165,6 +165,30 @@ def test_sdpa_slots_partitions_dealt_by_length(ctx, eng, n_slots, nwg, lens, sch
             assert_close(got[s], want, TOL, f"rep {rep} slot {s} len {lens[s]}")
 
 
+@pytest.mark.parametrize("nwg,lens", [
+    (7, [768, 768]),       # 128 rows each: one whole round
+    (7, [769, 768]),       # 129: tiles of 32 rows from here on (160)
+    (7, [961, 960]),       # 161: the next tile; the last partitions are short of one
+    (7, [1, 1921]),        # 192 rows each, a last partition and a slot of one row
+    (5, [641, 640]),       # the form whose waves keep P.V of their own tiles
+    (2, [2048, 2015]),     # and many rounds to a partition there
+])
+@pytest.mark.parametrize("sched", FORMS)
+def test_sdpa_slots_deal_beyond_a_round(ctx, eng, nwg, lens, sched):
+    """Partitions longer than the matrix-core form's round are cut at whole tiles of rows: every slot is the oracle's."""
+    n_q, n_kv, hd, max_t = 8, 1, 256, 2048
+    n = len(lens)
+    _, k, v, q = synth.cfg3_q40_attention(n, n_q, n_kv, hd, max_t, lo=1, seed=480)
+    meta = np.zeros((n, 4), dtype=np.float32)
+    meta[:, 0] = lens
+    tmp = ctx.buffer_empty_f32(n * n_q * nwg * (hd + 2))
+    out = ctx.buffer_empty_f32(n * n_q * hd)
+    eng.sdpa_slots(ctx, n_q, n_kv, hd, max_t, n, ctx.buffer_f32(q), ctx.buffer_bytes(k), ctx.buffer_bytes(v), ctx.buffer_f32(meta), tmp, out, 0.0625, nwg, sched)
+    got = ctx.read_f32(out, n * n_q * hd).reshape(n, -1)
+    for s in range(n):
+        assert_close(got[s], oracle.sdpa(q[s], k[s], v[s], n_q, n_kv, hd, lens[s], 0, 0.0625, f64=True), TOL, f"slot {s} len {lens[s]}")
+
+
 def test_sdpa_errors(ctx):
     with pytest.raises(hip.KshError, match="multiple of 32"):
         ctx.compile(hip.make_desc(hip.Kind.SDPA_NAIVE, (8, 1, 100, 64), (DType.Q40, DType.F32), (1.0,)))
