@@ -48,15 +48,15 @@ __device__ uint32_t f32_to_f16_ref(float value)
 }
 
 // The codes clamp(nearest_int(iscale * (x - mn)), 0, 15) of a sub-block, as floats.  Where every product is known to stay
-// below 2^22 in magnitude, the magic addition rounds and subtracting the constant again leaves the rounded value itself:
-// two additions and a median instead of the integer detour (mask, subtract, clamp, convert).  `lo` and `hi` bound x.
+// below 2^22 in magnitude, the magic addition rounds to the nearest integer and ties to the even one, which is what one
+// rounding instruction does: it and a median instead of the integer detour (add, mask, subtract, clamp, convert).
+// (A code may come out as -0: in the sums and in scale * code + min it is the 0 it stands for.)  `lo` and `hi` bound x.
 __device__ __forceinline__ void grid_codes(const float (&x)[32], float iscale, float mn, float lo, float hi, float (&lf)[32])
 {
-    constexpr float magic = 12582912.0f;
     const float reach = fabsf(iscale) * fmaxf(fabsf(lo - mn), fabsf(hi - mn));
     if (reach < 4000000.0f) {
 #pragma unroll
-        for (int i = 0; i < 32; i++) lf[i] = __builtin_amdgcn_fmed3f((iscale * (x[i] - mn) + magic) - magic, 0.0f, 15.0f);
+        for (int i = 0; i < 32; i++) lf[i] = __builtin_amdgcn_fmed3f(__builtin_rintf(iscale * (x[i] - mn)), 0.0f, 15.0f);
     } else {
         // (also where the reach is not a number: the host routine's integers, whatever they are)
 #pragma unroll
