@@ -109,7 +109,7 @@ int launch_decode_tail(const ksh_kernel &k_argmax, const float *logits, DecodeTa
 
 // The sampled decode step (sample_device.hip, sample.cpp): the entries of a row of logits that can survive its min-p
 // filter are gathered on the device, the reference's arithmetic runs on those on the host.
-constexpr int kSampleMaxRows = 16, kSampleInline = 126;
+constexpr int kSampleMaxRows = 16, kSampleInline = 126, kSampleParts = 128;
 struct SampleRow {
     float temperature;   // 0: a greedy row
     float below;         // candidates lie at most this far below the best soft-capped logit
@@ -123,7 +123,8 @@ struct SampleHead {
 struct SampleScratch {
     void *lists = nullptr, *joined = nullptr;   // device
     SampleHead *heads = nullptr;                // pinned host memory
-    int rows = 0, n = 0;
+    int rows = 0, n = 0;                        // what `lists` holds (0: nothing)
+    int reserve(int want_rows, int want_n, hipStream_t st);
     ~SampleScratch();
 };
 int launch_sample_candidates(SampleScratch &s, const float *logits, int n, int rows, float cap, const float *best_ids, const SampleRow *params,

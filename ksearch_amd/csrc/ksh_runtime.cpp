@@ -28,6 +28,7 @@ int set_error(const char *fmt, ...)
 
 int hip_fail(hipError_t e, const char *what)
 {
+    (void)hipGetLastError();   // reported here: the next launch's check does not find it again
     return set_error("HIP error %d (%s) in %s", (int)e, hipGetErrorString(e), what);
 }
 

@@ -38,6 +38,32 @@ bool sample_row_params(float temperature, float min_p, SampleRow *out)
     return true;
 }
 
+// Room for `rows` rows of n logits: two lists of (id, logit) per row, then a count and a sum per part.  The sizes say what
+// is allocated: after a failure nothing is, and the next call asks again.
+int SampleScratch::reserve(int want_rows, int want_n, hipStream_t st)
+{
+    if (!heads) KSH_HIP(hipHostMalloc((void **)&heads, sizeof(SampleHead) * kSampleMaxRows, hipHostMallocDefault));
+    if (rows >= want_rows && n >= want_n) return 0;
+    const int r = want_rows > rows ? want_rows : rows, m = want_n > n ? want_n : n;
+    if (lists) {
+        KSH_HIP(hipStreamSynchronize(st));
+        void *old = lists;
+        lists = joined = nullptr;
+        rows = n = 0;
+        KSH_HIP(hipFree(old));
+    }
+    KSH_HIP(hipMalloc(&lists, (size_t)r * ((size_t)m * 2 * sizeof(SampleCand) + kSampleParts * 8)));
+    rows = r;
+    n = m;
+    return 0;
+}
+
+SampleScratch::~SampleScratch()
+{
+    if (lists) (void)hipFree(lists);
+    if (heads) (void)hipHostFree(heads);
+}
+
 // ksh_sample_softcap_min_p below on the entries that can survive its filter.  The rest of the vocabulary takes part in
 // the result through the denominator alone, which scales every probability and the draw alike.
 bool sample_from_candidates(SampleCand *cand, size_t count, float sum, size_t n, float cap, float temperature, float min_p, uint32_t seed,

@@ -17,7 +17,7 @@
 namespace ksh {
 namespace {
 
-constexpr int kParts = 128, kThreads = 256;
+constexpr int kParts = kSampleParts, kThreads = 256;
 
 struct Rows {
     SampleRow r[kSampleMaxRows];
@@ -97,30 +97,13 @@ __global__ __launch_bounds__(kParts) void sample_join_kernel(const float *best_i
 
 }  // namespace
 
-SampleScratch::~SampleScratch()
-{
-    if (lists) (void)hipFree(lists);
-    if (heads) (void)hipHostFree(heads);
-}
-
 // Candidates of `rows` rows of n logits on the stream; best_ids: the rows' argmax (f32, on the device).  The records
 // are in s.heads once the stream has been waited for.
 int launch_sample_candidates(SampleScratch &s, const float *logits, int n, int rows, float cap, const float *best_ids, const SampleRow *params,
                              hipStream_t st)
 {
     if (rows < 1 || rows > kSampleMaxRows || n < 1) return set_error("sample: %d rows of %d logits", rows, n);
-    if (s.rows < rows || s.n < n) {
-        // two lists of (id, logit) per row, then a count and a sum per part
-        if (s.lists) {
-            KSH_HIP(hipStreamSynchronize(st));
-            KSH_HIP(hipFree(s.lists));
-            s.lists = nullptr;
-        }
-        s.rows = rows > s.rows ? rows : s.rows;
-        s.n = n > s.n ? n : s.n;
-        KSH_HIP(hipMalloc(&s.lists, (size_t)s.rows * ((size_t)s.n * 16 + kParts * 8)));
-        if (!s.heads) KSH_HIP(hipHostMalloc((void **)&s.heads, sizeof(SampleHead) * kSampleMaxRows, hipHostMallocDefault));
-    }
+    if (s.reserve(rows, n, st)) return 1;
     uint2 *lists = (uint2 *)s.lists;
     s.joined = lists + (size_t)s.rows * n;
     uint32_t *counts = (uint32_t *)((char *)s.lists + (size_t)s.rows * s.n * 16);

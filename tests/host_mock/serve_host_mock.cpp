@@ -1,6 +1,7 @@
-// Host-only stand-ins that let the slot scheduler (ksearch_amd/csrc/serve.cpp) and the KV pool
-// (ksearch_amd/csrc/kv_pool.cpp) be linked and driven without a GPU: buffers are host memory and the "model" is a
-// counter with a fixed next-token rule that logs what the scheduler asks of it.  Test infrastructure only: it is
+// Host-only stand-ins that let the slot scheduler (ksearch_amd/csrc/serve.cpp), the KV pool (ksearch_amd/csrc/
+// kv_pool.cpp) and the sampler (ksearch_amd/csrc/sample.cpp) be linked and driven without a GPU: buffers and the runtime's
+// allocations are host memory (the n-th can be made to fail) and the "model" is a counter with a fixed next-token rule
+// that logs what the scheduler asks of it.  Test infrastructure only: it is
 // compiled into tests/host_mock/libserve_host.so, never into the library.
 #include <cstdarg>
 #include <cstdlib>
@@ -22,6 +23,7 @@ int set_error(const char *fmt, ...)
     g_err = b;
     return 1;
 }
+int hip_fail(hipError_t e, const char *what) { return set_error("HIP error %d in %s", (int)e, what); }
 ksh_buf *buffer_view(ksh_buf *parent, size_t off, size_t bytes)
 {
     if (!parent || off > parent->bytes || bytes > parent->bytes - off) {
@@ -36,6 +38,23 @@ ksh_buf *buffer_view(ksh_buf *parent, size_t off, size_t bytes)
     return v;
 }
 }  // namespace ksh
+
+// allocations of the HIP runtime: host memory, counted; the one after g_alloc_left more fails (negative: none does)
+static int g_alloc_left = -1, g_allocated = 0;
+static hipError_t host_alloc(void **p, size_t bytes)
+{
+    if (g_alloc_left == 0) { g_alloc_left = -1; return hipErrorOutOfMemory; }
+    if (g_alloc_left > 0) g_alloc_left--;
+    *p = malloc(bytes ? bytes : 1);
+    g_allocated++;
+    return hipSuccess;
+}
+static hipError_t host_free(void *p)
+{
+    if (p) g_allocated--;
+    free(p);
+    return hipSuccess;
+}
 
 struct MockCall {
     int32_t kind;   // 0 bind_slot, 1 prefill_chunk, 2 decode_token_sampled, 3 one row of decode_round
@@ -55,6 +74,24 @@ struct ksh_gemma4 {
 };
 
 extern "C" {
+
+hipError_t hipMalloc(void **p, size_t bytes) { return host_alloc(p, bytes); }
+hipError_t hipFree(void *p) { return host_free(p); }
+hipError_t hipHostMalloc(void **p, size_t bytes, unsigned) { return host_alloc(p, bytes); }
+hipError_t hipHostFree(void *p) { return host_free(p); }
+hipError_t hipStreamSynchronize(hipStream_t) { return hipSuccess; }
+
+void mock_fail_alloc(int after) { g_alloc_left = after; }
+int mock_allocated(void) { return g_allocated; }
+ksh::SampleScratch *mock_sample_create(void) { return new ksh::SampleScratch; }
+void mock_sample_destroy(ksh::SampleScratch *s) { delete s; }
+// reserve()'s code; the sizes the scratch says it holds and whether its two allocations are there
+int mock_sample_reserve(ksh::SampleScratch *s, int rows, int n, int out[4])
+{
+    const int rc = s->reserve(rows, n, nullptr);
+    out[0] = s->rows; out[1] = s->n; out[2] = s->lists != nullptr; out[3] = s->heads != nullptr;
+    return rc;
+}
 
 const char *ksh_last_error(void) { return ksh::g_err.c_str(); }
 

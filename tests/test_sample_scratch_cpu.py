@@ -1,0 +1,42 @@
+"""The sampled step's allocations (ksearch_amd/csrc/sample.cpp) where one fails: the scratch never says that it holds what
+it does not, so that the step after a failed one asks again instead of launching over null pointers.  Host-only build
+against mock allocations; no GPU work."""
+import ctypes as C
+
+import pytest
+
+from tests import host_mock
+
+
+@pytest.fixture()
+def scratch():
+    lib = C.CDLL(host_mock.build())
+    lib.mock_sample_create.restype = C.c_void_p
+    lib.mock_sample_destroy.argtypes = [C.c_void_p]
+    lib.mock_sample_reserve.argtypes = [C.c_void_p, C.c_int, C.c_int, C.POINTER(C.c_int)]
+    before, h = lib.mock_allocated(), lib.mock_sample_create()
+    out = (C.c_int * 4)()
+
+    def reserve(rows, n, fail_after=-1):
+        lib.mock_fail_alloc(fail_after)
+        rc = lib.mock_sample_reserve(h, rows, n, out)
+        lib.mock_fail_alloc(-1)
+        return rc, *out
+
+    yield reserve
+    lib.mock_sample_destroy(h)
+    assert lib.mock_allocated() == before
+
+
+@pytest.mark.parametrize("fail_after", [0, 1])
+def test_a_failed_allocation_is_asked_for_again(scratch, fail_after):
+    rc, rows, n, lists, heads = scratch(4, 1000, fail_after)
+    assert rc == 1 and (lists and heads or (rows, n) == (0, 0))
+    assert scratch(4, 1000) == (0, 4, 1000, 1, 1)
+
+
+def test_a_failed_growth_leaves_nothing_behind_that_the_sizes_claim(scratch):
+    assert scratch(2, 1000) == (0, 2, 1000, 1, 1)
+    assert scratch(16, 1000, 0) == (1, 0, 0, 0, 1)
+    assert scratch(1, 500) == (0, 1, 500, 1, 1)
+    assert scratch(2, 400) == (0, 2, 500, 1, 1) and scratch(1, 500) == (0, 2, 500, 1, 1)
