@@ -473,17 +473,14 @@ int chunk_buffers4(ksh_gemma4 *m)
     size_t max_ff = 0;
     for (const ksh_gemma4_layer &L : m->layers) max_ff = std::max(max_ff, (size_t)L.ffn);
     const size_t pt = (size_t)c.n_layers * c.ple_dim;
-    if (alloc(m, T * 4, &m->c_tok) || alloc(m, T * 11 * 4, &m->c_tab) || alloc(m, T * c.hidden * 4, &m->c_x) || alloc(m, T * c.hidden * 4, &m->c_x2) ||
-        alloc(m, T * c.hidden * 4, &m->c_y) || alloc(m, T * qd * 4, &m->c_q) || alloc(m, T * kvd * 4, &m->c_k) ||
-        alloc(m, T * kvd * 4, &m->c_v) || alloc(m, T * qd * 4, &m->c_o) || alloc(m, T * max_ff * 4, &m->c_g) ||
-        alloc(m, T * max_ff * 4, &m->c_u) || alloc(m, T * max_ff * 4, &m->c_ff) ||
-        alloc(m, T * c.n_q * kChunkPartitions4 * (max_hd + 2) * 4, &m->c_tmp) || alloc(m, 16, &m->c_meta_full) || alloc(m, 16, &m->c_meta_swa) ||
-        alloc(m, kPartsRows4 * T * c.hidden * 4, &m->c_po) || alloc(m, 2 * T * 2 * max_ff * 4, &m->c_pg))
-        return 1;
-    if (c.ple_dim > 0 && (alloc(m, T * pt * 4, &m->c_ple_tok) || alloc(m, T * pt * 4, &m->c_ple_tmp) || alloc(m, T * pt * 4, &m->c_ple_ctx) ||
-                          alloc(m, T * c.ple_dim * 4, &m->c_ple_u)))
-        return 1;
-    return 0;
+    return alloc_together(m->ctx, m->bufs.owned,
+                          {{T * 4, &m->c_tok}, {T * 11 * 4, &m->c_tab}, {T * c.hidden * 4, &m->c_x}, {T * c.hidden * 4, &m->c_x2},
+                           {T * c.hidden * 4, &m->c_y}, {T * qd * 4, &m->c_q}, {T * kvd * 4, &m->c_k}, {T * kvd * 4, &m->c_v}, {T * qd * 4, &m->c_o},
+                           {T * max_ff * 4, &m->c_g}, {T * max_ff * 4, &m->c_u}, {T * max_ff * 4, &m->c_ff},
+                           {T * c.n_q * kChunkPartitions4 * (max_hd + 2) * 4, &m->c_tmp}, {16, &m->c_meta_full}, {16, &m->c_meta_swa},
+                           {kPartsRows4 * T * c.hidden * 4, &m->c_po}, {2 * T * 2 * max_ff * 4, &m->c_pg},
+                           {T * pt * 4, &m->c_ple_tok}, {T * pt * 4, &m->c_ple_tmp},
+                           {T * pt * 4, &m->c_ple_ctx}, {T * c.ple_dim * 4, &m->c_ple_u}});
 }
 
 // A pass over the prompts of several pool slots: each one's tokens behind its slot's sequence length.
@@ -1218,9 +1215,10 @@ int forward_decode_round4(ksh_gemma4 *m, ksh_kvpool *pool, const int32_t *slots,
     int64_t widest = std::max<int64_t>(c.hidden, c.ple_dim);
     for (int l = 0; l < c.n_layers; l++) widest = std::max<int64_t>(widest, std::max<int64_t>(m->layers[l].ffn, m->plan[l].qd));
     widest = (widest + 255) / 256 * 256;
-    if (!m->r_tab && (alloc(m, (size_t)kRoundStride * 10 * 4, &m->r_tab) || alloc(m, (size_t)kRoundMax * c.vocab * 4, &m->r_logits) ||
-                      alloc(m, (size_t)kRoundMax * 4, &m->r_next) || alloc(m, (size_t)(64 * widest + 2048 * (widest / 256)), &m->r_xp) ||
-                      alloc(m, (size_t)(64 * widest + 2048 * (widest / 256)), &m->r_xp2)))
+    const size_t xp = (size_t)(64 * widest + 2048 * (widest / 256));
+    if (!m->r_tab && alloc_together(m->ctx, m->bufs.owned,
+                                    {{(size_t)kRoundStride * 10 * 4, &m->r_tab}, {(size_t)kRoundMax * c.vocab * 4, &m->r_logits},
+                                     {(size_t)kRoundMax * 4, &m->r_next}, {xp, &m->r_xp}, {xp, &m->r_xp2}}))
         return 1;
     RoundTable table{};
     float *tab = table.v;

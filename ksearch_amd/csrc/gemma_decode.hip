@@ -370,12 +370,12 @@ int chunk_buffers(ksh_gemma *m)
     const ksh_gemma_cfg &c = m->c;
     const size_t T = kChunk, qd = (size_t)c.n_q * c.hd, kvd = (size_t)c.n_kv * c.hd;
     m->c_nwg = kChunkPartitions;
-    return alloc(m, T * 4, &m->c_tok) || alloc(m, T * c.hidden * 4, &m->c_x) || alloc(m, T * c.hidden * 4, &m->c_x2) ||
-           alloc(m, T * c.hidden * 4, &m->c_y) || alloc(m, T * qd * 4, &m->c_q) || alloc(m, T * kvd * 4, &m->c_k) ||
-           alloc(m, T * kvd * 4, &m->c_v) || alloc(m, T * qd * 4, &m->c_o) || alloc(m, T * c.ffn * 4, &m->c_g) ||
-           alloc(m, T * c.ffn * 4, &m->c_u) || alloc(m, T * c.ffn * 4, &m->c_ff) ||
-           alloc(m, T * c.n_q * m->c_nwg * (c.hd + 2) * 4, &m->c_tmp) || alloc(m, 16, &m->c_meta) ||
-           alloc(m, kPartsRows * T * c.hidden * 4, &m->c_po) || alloc(m, 2 * T * 2 * c.ffn * 4, &m->c_pg) || alloc(m, kPartsRows * T * c.hidden * 4, &m->c_pd);
+    return alloc_together(m->ctx, m->bufs.owned,
+                          {{T * 4, &m->c_tok}, {T * c.hidden * 4, &m->c_x}, {T * c.hidden * 4, &m->c_x2}, {T * c.hidden * 4, &m->c_y},
+                           {T * qd * 4, &m->c_q}, {T * kvd * 4, &m->c_k}, {T * kvd * 4, &m->c_v}, {T * qd * 4, &m->c_o},
+                           {T * c.ffn * 4, &m->c_g}, {T * c.ffn * 4, &m->c_u}, {T * c.ffn * 4, &m->c_ff},
+                           {T * c.n_q * m->c_nwg * (c.hd + 2) * 4, &m->c_tmp}, {16, &m->c_meta}, {kPartsRows * T * c.hidden * 4, &m->c_po},
+                           {2 * T * 2 * c.ffn * 4, &m->c_pg}, {kPartsRows * T * c.hidden * 4, &m->c_pd}});
 }
 
 // forward_prefill_chunk (gemma_prim.rs:1317-1607) for 2 <= t <= kChunk tokens already validated: the layer as

@@ -9,7 +9,9 @@
 #include <cstdint>
 #include <cstdio>
 #include <cstring>
+#include <initializer_list>
 #include <string>
+#include <vector>
 
 #include "../../include/ksearch_hip.h"
 
@@ -164,6 +166,28 @@ inline size_t packed_bytes(int dtype, size_t n)
     size_t e, b;
     if (!block_spec(dtype, e, b) || n % e) return 0;
     return n / e * b;
+}
+
+// Buffers that are there together or not at all: where one cannot be allocated the others are given back and every
+// pointer stays null, so that a later call asks for all of them again.  `owned` releases them in the end.
+struct BufWant {
+    size_t bytes;
+    ksh_buf **out;
+};
+inline int alloc_together(ksh_ctx *ctx, std::vector<ksh_buf *> &owned, std::initializer_list<BufWant> wants)
+{
+    const size_t had = owned.size();
+    for (const BufWant &w : wants) {
+        ksh_buf *b = nullptr;
+        if (ksh_buffer_alloc(ctx, w.bytes ? w.bytes : 16, nullptr, &b)) {
+            for (; owned.size() > had; owned.pop_back()) ksh_buffer_release(owned.back());
+            for (const BufWant &u : wants) *u.out = nullptr;
+            return 1;
+        }
+        owned.push_back(b);
+        *w.out = b;
+    }
+    return 0;
 }
 
 inline bool sched_is_zero(const ksh_sched &s)

@@ -93,12 +93,24 @@ int mock_sample_reserve(ksh::SampleScratch *s, int rows, int n, int out[4])
     return rc;
 }
 
+// three buffers needed together, allocated where they are not there yet; how many of the pointers are set
+int mock_together(ksh_buf **three, int *set)
+{
+    static std::vector<ksh_buf *> owned;
+    const int rc = three[0] ? 0 : ksh::alloc_together(nullptr, owned, {{64, &three[0]}, {0, &three[1]}, {32, &three[2]}});
+    *set = 0;
+    for (int i = 0; i < 3; i++) *set += three[i] != nullptr;
+    return rc;
+}
+
 const char *ksh_last_error(void) { return ksh::g_err.c_str(); }
 
 int ksh_buffer_alloc(ksh_ctx *, size_t bytes, const void *init, ksh_buf **out)
 {
+    void *ptr = nullptr;
+    if (host_alloc(&ptr, bytes) != hipSuccess) return ksh::set_error("mock allocation failure");
     ksh_buf *b = new ksh_buf;
-    b->ptr = malloc(bytes ? bytes : 1);
+    b->ptr = ptr;
     b->bytes = bytes;
     if (init) memcpy(b->ptr, init, bytes);
     *out = b;
@@ -110,7 +122,7 @@ void ksh_buffer_release(ksh_buf *b)
         if (b->parent)
             ksh_buffer_release(b->parent);
         else
-            free(b->ptr);
+            (void)host_free(b->ptr);
         delete b;
     }
 }

@@ -1,6 +1,6 @@
-"""The sampled step's allocations (ksearch_amd/csrc/sample.cpp) where one fails: the scratch never says that it holds what
-it does not, so that the step after a failed one asks again instead of launching over null pointers.  Host-only build
-against mock allocations; no GPU work."""
+"""Allocations made on first use where one fails: the sampled step's scratch (ksearch_amd/csrc/sample.cpp) and the buffers
+of a prompt pass or a decode round (alloc_together) never look as if they held what they do not, so that the call after a
+failed one asks again instead of launching over null pointers.  Host-only build against mock allocations; no GPU work."""
 import ctypes as C
 
 import pytest
@@ -40,3 +40,12 @@ def test_a_failed_growth_leaves_nothing_behind_that_the_sizes_claim(scratch):
     assert scratch(16, 1000, 0) == (1, 0, 0, 0, 1)
     assert scratch(1, 500) == (0, 1, 500, 1, 1)
     assert scratch(2, 400) == (0, 2, 500, 1, 1) and scratch(1, 500) == (0, 2, 500, 1, 1)
+
+
+@pytest.mark.parametrize("fail_after", [0, 1, 2])
+def test_buffers_needed_together_are_there_together_or_not_at_all(fail_after):
+    lib = C.CDLL(host_mock.build())
+    three, n, before = (C.c_void_p * 3)(), C.c_int(), lib.mock_allocated()
+    lib.mock_fail_alloc(fail_after)
+    assert lib.mock_together(three, C.byref(n)) == 1 and n.value == 0 and lib.mock_allocated() == before
+    assert lib.mock_together(three, C.byref(n)) == 0 and n.value == 3 and lib.mock_allocated() == before + 3
