@@ -91,7 +91,8 @@ enum ksh_kind {
      * F32 activations travel as hi + lo f16 parts.  The tile scales every row by its own power of two first (any
      * finite f32 row fits); the small-batch form does not: there |x| must stay below 65504.
      * sched.nr0 = 32 | 128 picks the small-batch form (Q4_K, up to 64 tokens, one matrix) or the 128 x 128 tile;
-     * sched.k_split = the tile's K slices (a divisor of cols / 256; 1 = whole rows; 0 = enough to fill the chip). */
+     * sched.k_split = the tile's K slices (a divisor of cols / 256, or for bf16 rows the count of a reported schedule;
+     * 1 = whole rows; 0 = enough to fill the chip). */
     KSH_MATVEC_BATCH = 2,
     /* MatvecQkv: three GEMVs sharing x.  dims: q_rows, kv_rows, cols.
      * in: Wq, Wk, Wv, x   out: q, k, v */

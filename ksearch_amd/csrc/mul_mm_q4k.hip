@@ -1833,10 +1833,12 @@ int bind_matvec_batch(ksh_kernel &k)
         return 0;
     }
     // K slices: workgroups of one launch, every slice storing its partial sums, and a second launch that adds them
-    // (mm_k_slices, mm_plan_bf16).  sched.k_split names the slice count (a divisor of cols / 256; 1 = none).
+    // (mm_k_slices, mm_plan_bf16).  sched.k_split names the slice count (a divisor of cols / 256; 1 = none).  For bf16 rows
+    // the plan takes any count, and a schedule that a bound kernel has reported (it names the tile too) takes it again.
     const int64_t row_tiles = mm_row_tiles(k.desc), nsb = cols / 256;
     int64_t ks = cut ? 1 : k.desc.sched.k_split;
-    if (!cut && ks && nsb % ks) return set_error("matvec_batch: k_split=%lld does not divide the %lld superblocks of a row", (long long)ks, (long long)nsb);
+    const bool reported = !f32x && want == BN && k.desc.sched.tg == kThreadsMM && k.desc.sched.lds_tile == KS && ks <= std::min<int64_t>(nsb, 64);
+    if (!cut && ks && nsb % ks && !reported) return set_error("matvec_batch: k_split=%lld does not divide the %lld superblocks of a row", (long long)ks, (long long)nsb);
     int tm = 0;
     if (f32x) {
         if (!ks) ks = mm_k_slices(q6, (int)row_tiles, (int)nsb, (int)batch);

@@ -375,6 +375,42 @@ def test_mul_mm_k_slices_must_divide_the_row(ctx):
         ctx.compile(hip.make_desc(hip.Kind.MATVEC_BATCH, (256, 2048, 100), (DType.Q4K, DType.BF16, DType.F32), (), dict(k_split=3)))
 
 
+@pytest.mark.parametrize("wdt,batch,rows,cols", [(DType.Q6K, 512, 300, 7936), (DType.Q4K, 512, 300, 7936), (DType.Q6K, 300, 1000, 2816),
+                                                 (DType.Q4K, 40, 256, 2048)])
+def test_mul_mm_reported_schedule_binds_again(ctx, wdt, batch, rows, cols, tmp_path, monkeypatch):
+    """The schedule a bf16 launch reports (slice counts that divide 31 or 11 superblocks unevenly; the small-batch form) and
+    the one a search saves are taken again, as an argument and from the plan file: the same launch, the same bits."""
+    monkeypatch.setenv("KSEARCH_BEAM_CACHE", str(tmp_path / "beam"))
+    nb = rows * cols // 256
+    bw = ctx.buffer_bytes(synth.q4k_blocks(nb, 662) if wdt == DType.Q4K else synth.q6k_blocks(nb, 662))
+    bx, by = ctx.buffer_bytes(synth.bf16_round(synth.normal_f32(batch * cols, 663))[1]), ctx.buffer_empty_f32(batch * rows)
+
+    def desc(sched=None):
+        return hip.make_desc(hip.Kind.MATVEC_BATCH, (rows, cols, batch), (wdt, DType.BF16, DType.F32), (), sched)
+
+    def launch(k):
+        ctx.encode_multi(k, [bw, bx], [by])
+        ctx.synchronize()
+        return k.name, tuple(k.grid), ctx.read_f32(by, batch * rows).tobytes()
+
+    k = ctx.compile(desc())
+    ks, nsb = k.info.sched.k_split, cols // 256
+    assert nsb == 8 or nsb % ks, "the shape is here for a count that does not divide its superblocks"
+    want = launch(k)
+    assert launch(ctx.compile(desc(k.info.sched))) == want
+    best, _, _ = ctx.beam_search(desc(), [bw, bx], [by], iters=3, force=True)
+    ctx.compile(desc(best))
+    # a plan file with that schedule, found by a context that has not bound the shape yet
+    hip.plan_save(hip.plan_kind(desc()), (rows, cols, batch), ctx.device_name(), k.info.sched, 0.001)
+    other = hip.Context()
+    planned = other.compile(desc())
+    assert (planned.name, tuple(planned.grid)) == want[:2]
+    other.close()
+    if nsb != 8:   # a bare count is held to divisors, as it was
+        with pytest.raises(hip.KshError, match="does not divide"):
+            ctx.compile(desc(dict(k_split=ks)))
+
+
 def test_mul_mm_cfg2_full_size(ctx, eng):
     tokens, rows, cols = 512, 8192, 2048
     w, xf, xb = synth.cfg2_q4k_prefill()
