@@ -227,6 +227,7 @@ int get(ksh_gemma4 *m, int kind, std::initializer_list<int64_t> dims, std::initi
     for (int v : dtypes) d.dtypes[i++] = v;
     i = 0;
     for (float v : params) d.params[i++] = v;
+    if (prompt_kind(kind)) d.sched.tg = ~0ull;
     return ksh_kernel_get(m->ctx, &d, out);
 }
 
@@ -552,6 +553,7 @@ int forward_prefill_chunk4(ksh_gemma4 *m, const uint32_t *tokens, int t, const J
         for (int64_t v : dims) d.dims[nd++] = v;
         d.dtypes[0] = dt; d.dtypes[1] = d.dtypes[2] = KSH_F32;
         if (d.dims[5]) d.params[0] = c.eps;
+        d.sched.tg = ~0ull;   // (prompt_kind)
         ksh_buf *ib[kMaxIn], *ob[kMaxOut];
         size_t io[kMaxIn] = {};
         int ni = 0, no = 0;
@@ -563,6 +565,7 @@ int forward_prefill_chunk4(ksh_gemma4 *m, const uint32_t *tokens, int t, const J
             int lo = 1 << 30, hi = 0;
             for (int len : joint->alone) { const int ks = matvec_batch_slices(d, len); lo = std::min(lo, ks); hi = std::max(hi, ks); }
             if (hi == 1 || (lo == hi && matvec_batch_slices(d, (int)tp) > 1)) {
+                d.sched.tg = 0;
                 d.sched.k_split = (uint32_t)hi;
             } else {
                 d.dims[6] = 2;

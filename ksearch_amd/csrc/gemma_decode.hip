@@ -154,6 +154,7 @@ int get(ksh_gemma *m, int kind, std::initializer_list<int64_t> dims, std::initia
     for (int v : dtypes) d.dtypes[i++] = v;
     i = 0;
     for (float v : params) d.params[i++] = v;
+    if (prompt_kind(kind)) d.sched.tg = ~0ull;
     return ksh_kernel_get(m->ctx, &d, out);
 }
 

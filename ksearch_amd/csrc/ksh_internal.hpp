@@ -36,6 +36,11 @@ inline int prefill_pass_tokens(int left)
     return left >= kPrefillPass ? kPrefillPass : left >= kPrefillPass / 2 ? kPrefillPass / 2 : left;
 }
 
+// The kinds of a prompt pass whose schedule says how a row's sums are cut.  The decode loops bind them by the library's own
+// rules (schedule tg = all ones), whatever the plan cache holds: a prompt's caches depend neither on the passes its tokens
+// were dealt to nor on a plan that a search has left for one of their lengths.
+inline bool prompt_kind(int kind) { return kind == KSH_MATVEC_BATCH || kind == KSH_SDPA_BATCH; }
+
 // The prompt tokens of several pool slots in one pass through the layers: n[i] tokens behind slot slots[i]'s sequence
 // length, at most kPrefillPass in all, with the bits of passes of their own.  taken[i] tells which slots went along (the
 // others, and every slot where fewer than two can, are left to the caller); nonzero with the error set when the pass of

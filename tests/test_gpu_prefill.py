@@ -269,6 +269,31 @@ def test_prefill_passes_of_2048_are_those_of_1024(ctx, n_prompt):
     gpu.close()
 
 
+def test_prefill_passes_do_not_depend_on_saved_plans(tmp_path, monkeypatch):
+    """A plan for the GEMMs of 1024 rows (whole rows where the library's rule has K slices) does not reach the prompt's
+    passes: one of 2048 tokens and two of 1024 leave the same bytes."""
+    monkeypatch.setenv("KSEARCH_BEAM_CACHE", str(tmp_path / "beam"))
+    ctx = hip.Context()
+    cfg = dict(n_layers=2, hidden=512, ffn=2048, n_q=4, n_kv=1, hd=256, vocab=1024, max_seq=2100,
+               eps=1e-6, softcap=30.0, rope_theta=10000.0, attn_scale=1.0 / 16.0)
+    h, qd, hd, f = cfg["hidden"], 1024, cfg["hd"], cfg["ffn"]
+    for dims in ((qd, h, 1024, hd, hd, 1), (h, qd, 1024, 0, 0, 0, 1), (h, f, 1024), (h, f, 1024, 0, 0, 0, 1), (hd, h, 1024), (qd, h, 1024)):
+        hip.plan_save("mul_mm_q4k", dims, ctx.device_name(), hip.Sched(tg=512, nsg=8, nr0=128, k_split=1, lds_tile=64), 0.001)
+    gpu = hip.Gemma(ctx, cfg, synth.gemma_weights(cfg, 764, oracle.quantize_q4k, oracle.quantize_q6k, std=0.05))
+    toks = np.random.default_rng(765).integers(0, cfg["vocab"], 2048)
+    got = []
+    for step in (2048, 1024):
+        gpu.reset()
+        for i in range(0, 2048, step):
+            gpu.prefill_chunk(toks[i:i + step])
+        got.append([ctx.read_bytes(hip.Buffer(ctx, hip.lib().ksh_gemma_kv(gpu.h, l, which), owned=False), hd // 32 * 18 * 2048, 0)
+                    for l in range(cfg["n_layers"]) for which in (0, 1)])
+    for a, b in zip(*got):
+        assert np.array_equal(a, b)
+    gpu.close()
+    ctx.close()
+
+
 def test_prefill_in_two_calls_and_serial_prefill_agree(ctx, small_model):
     """A prompt fed as 40 + 1 + 23 tokens (a single token goes through the decode step) leaves the same cache as one
     call, and generate() gives the same continuation with batched and with token-by-token prefill unless a Q4_0 flip

@@ -316,3 +316,42 @@ def test_prompts_prefilled_in_one_pass_fill_the_caches_of_passes_alone(ctx, lens
     m.bind_slot(None, 0)
     pool.close()
     m.close()
+
+
+def test_joint_prompt_passes_do_not_depend_on_saved_plans(tmp_path, monkeypatch):
+    """A plan that a search left for one of the pass lengths (whole rows where the library's rule cuts them into K slices)
+    changes neither a pass alone nor a joint one: the two keep filling the caches with the same bytes."""
+    monkeypatch.setenv("KSEARCH_BEAM_CACHE", str(tmp_path / "beam"))
+    ctx = hip.Context()
+    cfg = dict(synth.GEMMA4_TINY, hd_swa=256, hd_full=512, max_seq=256, sliding_window=40)
+    h, whole = cfg["hidden"], hip.Sched(tg=512, nsg=8, nr0=128, k_split=1, lds_tile=64)
+    for tp in (224, 512):                                  # a prompt of 225 alone; two of them in steps of 128 rows
+        for hd in (256, 512):
+            qd = cfg["n_q"] * hd
+            for dims in ((h, qd, tp, 0, 0, 0, 1), (h, qd, tp), (qd, h, tp, hd, hd, 1), (qd, h, tp, 0, 0, 1), (qd, h, tp)):
+                hip.plan_save("mul_mm_q4k", dims, ctx.device_name(), whole, 0.001)
+        for f in (1024, 2048):
+            for dims in ((h, f, tp), (h, f, tp, 0, 0, 3)):
+                hip.plan_save("mul_mm_q4k", dims, ctx.device_name(), whole, 0.001)
+    w = synth.gemma4_weights(cfg, 611, oracle.quantize_q4k, oracle.quantize_q6k, ffn=FFN, swa_pattern=PATTERN, std=0.05)
+    m = hip.Gemma4(ctx, cfg, w)
+    prompts = prompts_of(cfg, (225, 225), 707)
+    pool = make_pool(ctx, cfg, 2)
+    sv = hip.Serve(m, pool, slots=2, eos=NO_EOS)
+    for p in prompts:
+        sv.submit(p, 2)
+    assert sv.tick() == []
+    for slot, p in enumerate(prompts):
+        m.bind_slot(None, 0)
+        m.reset()
+        m.prefill_chunk(p[:-1])
+        for layer in range(cfg["n_layers"] - cfg["shared_kv_layers"]):
+            n = cfg["n_kv"] * (cfg["hd_swa"] if PATTERN[layer] else cfg["hd_full"]) // 32 * 18 * (len(p) - 1)
+            own = [hip.Buffer(ctx, hip.lib().ksh_gemma4_kv(m.h, layer, which), owned=False) for which in (0, 1)]
+            for buf, mine in zip((pool.k_buf(slot, layer), pool.v_buf(slot, layer)), own):
+                assert np.array_equal(ctx.read_bytes(buf, n), ctx.read_bytes(mine, n)), (slot, layer)
+    sv.close()
+    m.bind_slot(None, 0)
+    pool.close()
+    m.close()
+    ctx.close()
