@@ -392,7 +392,7 @@ int ksh_plan_save(const char *kind, const int64_t *dims, int n_dims, const char 
 int ksh_plan_load(const char *kind, const int64_t *dims, int n_dims, const char *chip,
                   ksh_sched *sched, double *ms);
 /* plan kind string for a descriptor ("matvec_q4k", "matvec_q6k", "mul_mm_q4k",
- * "sdpa_q40", ...; crates/ksearch_codegen/src/lib.rs:200-205) */
+ * "mul_mm_q4k_bf16", "sdpa_q40", ...; crates/ksearch_codegen/src/lib.rs:200-205) */
 const char *ksh_plan_kind(const ksh_kernel_desc *desc);
 /* BEAM: candidate schedules for a descriptor (beam.rs:26-65 retargeted) */
 int ksh_beam_candidates(const ksh_kernel_desc *desc, ksh_sched *out, int cap);

@@ -132,6 +132,17 @@ def test_plan_cache_reads_reference_format(tmp_path, monkeypatch):
     assert hip.plan_load("matvec_q6k", [262144, 2048], "gfx950") is None
 
 
+def test_plans_of_bf16_and_f32_gemms_are_apart(tmp_path, monkeypatch):
+    """The two take slice counts by different rules: a plan of one is not found for the other."""
+    monkeypatch.setenv("KSEARCH_BEAM_CACHE", str(tmp_path))
+    for wdt in (hip.DType.Q4K, hip.DType.Q6K):
+        kinds = [hip.plan_kind(hip.make_desc(hip.Kind.MATVEC_BATCH, (300, 7936, 512), (wdt, xdt, hip.DType.F32))) for xdt in (hip.DType.F32, hip.DType.BF16)]
+        assert len(set(kinds)) == 2
+        hip.plan_save(kinds[1], (300, 7936, 512), "gfx950", hip.Sched(tg=512, nsg=8, nr0=128, k_split=8, lds_tile=64), 0.02)
+        assert hip.plan_load(kinds[1], (300, 7936, 512), "gfx950")[0].k_split == 8
+        assert hip.plan_load(kinds[0], (300, 7936, 512), "gfx950") is None
+
+
 def test_plan_kinds_and_candidates():
     d = hip.make_desc(hip.Kind.MATVEC, (4096, 4096), (hip.DType.Q4K, hip.DType.F32))
     assert hip.plan_kind(d) == "matvec_q4k"
