@@ -105,7 +105,7 @@ struct LayerPlan {
 }  // namespace
 
 struct ksh_gemma4 {
-    std::vector<float> host_logits;   // a whole row read back, where the device cannot narrow it down (no min-p filter)
+    std::vector<float> host_logits;   // a whole row read back, where the device cannot narrow it down (no min-p filter, or too many pass it)
     ksh::SampleScratch sample;
     ksh_ctx *ctx = nullptr;
     ksh_gemma4_cfg c{};
@@ -157,36 +157,36 @@ namespace {
 using namespace ksh;
 
 // The ids of `rows` rows of logits that the stream is about to hold: greedy ids where temperature (may be null) is below
-// 1e-6, else sample_softcap_min_p's draw, on the entries that can survive its filter (launch_sample_candidates).  Waits
-// for the stream.
+// 1e-6, else sample_softcap_min_p's draw: on the entries that can survive its filter (launch_sample_candidates) where
+// there is one and they are few enough, on the whole row otherwise.  Waits for the stream.
 int draw_ids(ksh_gemma4 *m, ksh_buf *logits, ksh_buf *best_ids, int rows, const float *temperature, const float *min_p, const uint32_t *seed,
              uint32_t *next_ids)
 {
     const int n = m->c.vocab;
     SampleRow params[kSampleMaxRows] = {};
-    bool any = false, narrowed[kSampleMaxRows] = {};
+    bool filtered = false, narrowed[kSampleMaxRows] = {};
     for (int i = 0; i < rows; i++) {
         if (!temperature || temperature[i] < 1e-6f) continue;
-        any = true;
         narrowed[i] = sample_row_params(temperature[i], min_p[i], &params[i]);
+        filtered = filtered || narrowed[i];
     }
-    if (!any) {
+    if (!filtered) {   // nothing for the device to narrow down
         float ids[kSampleMaxRows];
         if (ksh_buffer_read(m->ctx, best_ids, 0, ids, (size_t)rows * 4, 1)) return 1;
         for (int i = 0; i < rows; i++) next_ids[i] = (uint32_t)ids[i];
-        return 0;
+    } else {
+        const float *dev = (const float *)ksh_buffer_device_ptr(logits);
+        if (launch_sample_candidates(m->sample, dev, n, rows, m->c.softcap, (const float *)ksh_buffer_device_ptr(best_ids), params,
+                                     (hipStream_t)ksh_stream(m->ctx)) ||
+            ksh_synchronize(m->ctx))
+            return 1;
+        for (int i = 0; i < rows; i++) next_ids[i] = m->sample.heads[i].best_id;
     }
-    const float *dev = (const float *)ksh_buffer_device_ptr(logits);
-    if (launch_sample_candidates(m->sample, dev, n, rows, m->c.softcap, (const float *)ksh_buffer_device_ptr(best_ids), params,
-                                 (hipStream_t)ksh_stream(m->ctx)) ||
-        ksh_synchronize(m->ctx))
-        return 1;
     std::vector<SampleCand> longer;
     for (int i = 0; i < rows; i++) {
-        SampleHead &h = m->sample.heads[i];
-        next_ids[i] = h.best_id;
         if (!temperature || temperature[i] < 1e-6f) continue;
-        if (narrowed[i]) {
+        if (narrowed[i] && m->sample.heads[i].count <= sample_most(n)) {
+            SampleHead &h = m->sample.heads[i];
             SampleCand *cand = h.cand;
             if (h.count > (uint32_t)kSampleInline) {
                 longer.resize(h.count);

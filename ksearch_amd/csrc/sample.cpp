@@ -69,7 +69,7 @@ SampleScratch::~SampleScratch()
 bool sample_from_candidates(SampleCand *cand, size_t count, float sum, size_t n, float cap, float temperature, float min_p, uint32_t seed,
                             uint32_t *out)
 {
-    if (!count || !std::isfinite(sum)) return false;
+    if (!count || count > sample_most((int64_t)n) || !std::isfinite(sum)) return false;
     std::sort(cand, cand + count, [](const SampleCand &a, const SampleCand &b) { return a.id < b.id; });
     uint32_t best_i = 0;
     float best_v = -INFINITY;

@@ -7,7 +7,8 @@
 // softmax's denominator, and hands the host a few hundred bytes; the host does the reference's arithmetic on them.
 //   pass 1  one read of the logits: 128 workgroups per row, each with its own list and its own partial denominator
 //   pass 2  one workgroup per row joins the lists behind one another (sums in a fixed order) and writes the row's
-//           record straight into pinned host memory
+//           record straight into pinned host memory; of a row with more candidates than the host takes (sample_most)
+//           only the count
 // Bound: launch latency (a row is one megabyte at the real vocabulary).  Sixteen requests served with sampling, prompts
 // of about 150 tokens and ten tokens of answer each: 552 ms with the whole rows read back and walked on the host, 146 ms
 // with the candidates.
@@ -17,7 +18,7 @@
 namespace ksh {
 namespace {
 
-constexpr int kParts = kSampleParts, kThreads = 256;
+constexpr int kParts = kSampleParts, kThreads = 256, kJoinThreads = 512;
 
 struct Rows {
     SampleRow r[kSampleMaxRows];
@@ -59,34 +60,38 @@ __global__ __launch_bounds__(kThreads) void sample_scan_kernel(const float *__re
     }
 }
 
-__global__ __launch_bounds__(kParts) void sample_join_kernel(const float *best_ids, int n, const uint2 *lists, const uint32_t *counts,
-                                                             const float *sums, uint2 *joined, SampleHead *heads)
+__global__ __launch_bounds__(kJoinThreads) void sample_join_kernel(const float *best_ids, int n, uint32_t most, const uint2 *lists, const uint32_t *counts,
+                                                                   const float *sums, uint2 *joined, SampleHead *heads)
 {
     __shared__ uint32_t s_at[kParts];
     __shared__ float s_sum[kParts];
     const int row = blockIdx.x, t = threadIdx.x;
-    const uint32_t mine = counts[row * kParts + t];
-    s_at[t] = mine;
-    s_sum[t] = sums[row * kParts + t];
+    if (t < kParts) {
+        s_at[t] = counts[row * kParts + t];
+        s_sum[t] = sums[row * kParts + t];
+    }
     __syncthreads();
     for (int d = 1; d < kParts; d <<= 1) {   // inclusive prefix sum
-        const uint32_t v = t >= d ? s_at[t - d] : 0u;
+        const uint32_t v = t < kParts && t >= d ? s_at[t - d] : 0u;
         __syncthreads();
-        s_at[t] += v;
+        if (t < kParts) s_at[t] += v;
         __syncthreads();
     }
-    const uint32_t total = s_at[kParts - 1], at = s_at[t] - mine;
+    const uint32_t total = s_at[kParts - 1];
     for (int d = kParts / 2; d; d >>= 1) {
         if (t < d) s_sum[t] += s_sum[t + d];
         __syncthreads();
     }
     const int per = (n + kParts - 1) / kParts;
-    const uint2 *list = lists + (size_t)row * n + (size_t)t * per;
     SampleHead *h = heads + row;
-    for (uint32_t i = 0; i < mine; i++) {
-        const uint2 c = list[i];
-        if (at + i < (uint32_t)kSampleInline) { h->cand[at + i].id = c.x; h->cand[at + i].logit = __uint_as_float(c.y); }
-        if (total > (uint32_t)kSampleInline) joined[(size_t)row * n + at + i] = c;
+    // entry j of the joined list: in the first part whose prefix sum lies above it
+    for (uint32_t j = t; total <= most && j < total; j += kJoinThreads) {
+        int part = 0;
+        for (int d = kParts / 2; d; d >>= 1)
+            if (s_at[part + d - 1] <= j) part += d;
+        const uint2 c = lists[(size_t)row * n + (size_t)part * per + (j - (part ? s_at[part - 1] : 0u))];
+        if (j < (uint32_t)kSampleInline) { h->cand[j].id = c.x; h->cand[j].logit = __uint_as_float(c.y); }
+        if (total > (uint32_t)kSampleInline) joined[(size_t)row * n + j] = c;
     }
     if (t == 0) {
         h->count = total;
@@ -111,7 +116,7 @@ int launch_sample_candidates(SampleScratch &s, const float *logits, int n, int r
     Rows r{};
     for (int i = 0; i < rows; i++) r.r[i] = params[i];
     hipLaunchKernelGGL(sample_scan_kernel, dim3(kParts, rows), dim3(kThreads), 0, st, logits, n, cap, best_ids, r, lists, counts, sums);
-    hipLaunchKernelGGL(sample_join_kernel, dim3(rows), dim3(kParts), 0, st, best_ids, n, lists, counts, sums, (uint2 *)s.joined, s.heads);
+    hipLaunchKernelGGL(sample_join_kernel, dim3(rows), dim3(kJoinThreads), 0, st, best_ids, n, sample_most(n), lists, counts, sums, (uint2 *)s.joined, s.heads);
     const hipError_t e = hipGetLastError();
     return e == hipSuccess ? 0 : hip_fail(e, "sample launch");
 }

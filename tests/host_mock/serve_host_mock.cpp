@@ -3,6 +3,8 @@
 // allocations are host memory (the n-th can be made to fail) and the "model" is a counter with a fixed next-token rule
 // that logs what the scheduler asks of it.  Test infrastructure only: it is
 // compiled into tests/host_mock/libserve_host.so, never into the library.
+#include <algorithm>
+#include <cmath>
 #include <cstdarg>
 #include <cstdlib>
 #include <cstring>
@@ -91,6 +93,25 @@ int mock_sample_reserve(ksh::SampleScratch *s, int rows, int n, int out[4])
     const int rc = s->reserve(rows, n, nullptr);
     out[0] = s->rows; out[1] = s->n; out[2] = s->lists != nullptr; out[3] = s->heads != nullptr;
     return rc;
+}
+
+// the draw on the entries of a row that can survive its filter; -1: the row is to be walked whole
+int64_t mock_sample_candidates(const float *logits, size_t n, float cap, float temperature, float min_p, uint32_t seed, size_t *count)
+{
+    ksh::SampleRow row;
+    if (!ksh::sample_row_params(temperature, min_p, &row)) return -1;
+    std::vector<float> y(n);
+    for (size_t i = 0; i < n; i++) y[i] = cap > 0.0f ? cap * std::tanh(logits[i] / cap) : logits[i];
+    const float best = *std::max_element(y.begin(), y.end());
+    std::vector<ksh::SampleCand> cand;
+    float sum = 0.0f;
+    for (size_t i = n; i-- > 0;) {
+        sum += std::exp((y[i] - best) / temperature);
+        if (y[i] >= best - row.below) cand.push_back({(uint32_t)i, logits[i]});
+    }
+    *count = cand.size();
+    uint32_t id = 0;
+    return ksh::sample_from_candidates(cand.data(), cand.size(), sum, n, cap, temperature, min_p, seed, &id) ? (int64_t)id : -1;
 }
 
 // three buffers needed together, allocated where they are not there yet; how many of the pointers are set

@@ -283,6 +283,35 @@ def test_draws_from_the_narrowed_logits_are_the_host_samplers(ctx, model, temper
     pool.close()
 
 
+def test_draws_of_rows_with_more_candidates_than_a_list_takes(ctx):
+    """A vocabulary of 40960: lists of up to 5120 candidates are drawn from (dense ones among them), rows with more and rows
+    without a filter are walked whole; all of them, and a greedy row, in one round."""
+    cfg = dict(synth.GEMMA4_TINY, vocab=40960)
+    dq4, dq6 = hip.device_quantizers(ctx, hip.Eng())
+    w = synth.gemma4_weights(cfg, 612, dq4, lambda x: dq6([x]), ffn=FFN, swa_pattern=PATTERN, std=0.05)
+    m = hip.Gemma4(ctx, cfg, w)
+    (p,) = prompts_of(cfg, (6,), 708)
+    pool = make_pool(ctx, cfg, 6)
+    slots = [pool.alloc() for _ in range(6)]
+    temps, min_p, seeds = [50.0, 0.0, 0.9, 1.0, 0.05, 0.0], [0.9, 0.5, 0.0, 0.05, 0.5, 0.0], [21, 22, 23, 24, 25, 26]
+    m.decode_round(pool, slots, p)
+    y = cfg["softcap"] * np.tanh(m.round_logits(6) / np.float32(cfg["softcap"]))
+    far = np.sort(y[3])[::-1][3000] - y[3].max()      # a temperature at which some three thousand of row 3 pass
+    temps[3] = float(far / np.log(min_p[3]))
+    counts = [int((y[i] >= y[i].max() + t * np.log(q)).sum()) for i, (t, q) in enumerate(zip(temps, min_p)) if q]
+    assert counts[0] > 5120 and 2500 < counts[2] < 3500 and counts[3] < 127, counts
+    for _ in range(3):                                # (eager, captured, replayed)
+        got = m.decode_round(pool, slots, p, temps, min_p, seeds)
+        rows = m.round_logits(6)
+        assert got == [hip.sample_softcap_min_p(rows[i], cfg["softcap"], temps[i], min_p[i], seeds[i]) for i in range(6)]
+    # rows without a filter only, and greedy ones only
+    got = m.decode_round(pool, slots, p, [0.9, 0.0] * 3, [0.0] * 6, seeds)
+    assert got == [hip.sample_softcap_min_p(rows[i], cfg["softcap"], 0.9 if i % 2 == 0 else 0.0, 0.0, seeds[i]) for i in range(6)]
+    assert m.decode_round(pool, slots, p) == [int(np.argmax(y[i])) for i in range(6)]
+    pool.close()
+    m.close()
+
+
 @pytest.mark.parametrize("lens", [(90, 1, 130, 66, 2, 65), (225, 225), (9, 129)])
 def test_prompts_prefilled_in_one_pass_fill_the_caches_of_passes_alone(ctx, lens):
     """The prefilling requests of a tick with more than 64 tokens share one pass over the weights (heads of 256 and 512; 65

@@ -1,10 +1,14 @@
 """The host-side sampler of forward_token's non-greedy branch (crates/ksearch_gemma/src/sample.rs): the reference's
 own unit tests restated for the oracle and for the library's function, the two against each other, and the draw
 against the closed-form distribution.  No GPU work."""
+import ctypes as C
+
 import numpy as np
+import pytest
 
 import oracle
 from ksearch_amd import hip
+from tests import host_mock
 
 BOTH = (oracle.sample_softcap_min_p, hip.sample_softcap_min_p)
 
@@ -46,3 +50,23 @@ def test_draw_follows_the_filtered_softmax():
     p /= p.sum()
     draws = np.bincount([hip.sample_softcap_min_p(x, cap, temp, min_p, s) for s in range(1, 8001, 2)], minlength=5) / 4000.0
     assert draws[4] == 0.0 and np.abs(draws - p).max() < 0.03
+
+
+@pytest.mark.parametrize("n", [4096, 40000, 262144])
+def test_draw_from_candidates_and_where_it_ends(n):
+    """On the entries that can survive its min-p filter the draw is the one on the whole row; from n / 8 of them on (4096 in a
+    small vocabulary) the row is left to the whole walk, which is then the faster of the two."""
+    lib = C.CDLL(host_mock.build())
+    lib.mock_sample_candidates.restype = C.c_int64
+    lib.mock_sample_candidates.argtypes = [C.c_void_p, C.c_size_t, C.c_float, C.c_float, C.c_float, C.c_uint32, C.POINTER(C.c_size_t)]
+    most, count = max(4096, n // 8), C.c_size_t()
+    for near in (1, 100, min(most, n), most + 1, n):
+        if near > n:
+            continue
+        x = np.full(n, -9.0, np.float32)                # `near` entries within the filter, the others far below it
+        rng = np.random.default_rng(n + near)
+        x[rng.permutation(n)[:near]] = rng.uniform(4.0, 5.0, near).astype(np.float32)
+        for seed in (3, 1234):
+            got = lib.mock_sample_candidates(x.ctypes.data, n, 30.0, 1.0, 0.1, seed, C.byref(count))
+            assert count.value == near
+            assert got == (hip.sample_softcap_min_p(x, 30.0, 1.0, 0.1, seed) if near <= most else -1), near
