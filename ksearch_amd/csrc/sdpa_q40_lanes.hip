@@ -1802,6 +1802,41 @@ bool sdpa_lanes_supports(int64_t n_q, int64_t n_kv, int64_t hd)
     return n_kv > 0 && n_q % n_kv == 0 && n_q / n_kv <= 8 && (hd == 128 || hd == 256 || hd == 512);
 }
 
+// Split-KV partials without a merge (KSH_SDPA_MWG_PART), heads of 256 and 512, sched.unroll and sched.nsg left open.
+// `launch`: partitions times kv heads, `rows`: cache rows per partition (of the cache's length; a call may attend fewer).
+// One q head per workgroup unpacks K and V once per head, which is free while the chip has idle compute units -- up to
+// 512 workgroups -- and is the whole cost beyond.  Four heads share an instance's registers as well as one does (two or
+// three pay for four), so beyond that line as many share a workgroup, except where eight in one fill the chip by
+// themselves.  us, by (workgroups per kv head, waves), at 8 heads of 256 over one kv head:
+//   rows, partitions      8, 4     8, 8     2, 4     2, 8     1, 4     1, 8
+//     4096,  16           10.2      8.5     16.0     13.1     23.9     20.0
+//    16384,  32           17.5     13.5     27.3     21.3     41.0     33.9
+//    16384, 128           12.4     13.5     10.3      9.1     15.1     13.1
+//    16384, 256           12.7     16.4      9.2     12.1     10.7      9.7
+//    65536, 256           34.0     36.4     21.8     24.8     23.8     20.2
+//    65536, 1024          39.1     56.1     24.4     43.7     39.2     35.3
+// and at 8 heads of 512 (eight waves): 4096, 16: 13.1 with eight workgroups, 21.3 with two; 65536, 256: 63.4, 43.1.
+static int parts_head_split(int64_t launch, int64_t rows, int groups, int hd)
+{
+    if (groups <= 2 || launch * groups <= 512) return groups;
+    if (hd == 512) return groups % 4 ? groups : groups / 4;
+    if (groups > 4 && launch > 128 && launch <= 256 && rows >= 256) return 1;
+    int split = 1;
+    while (groups % split || groups / split > 4) split++;
+    return split;
+}
+
+// ... and the waves of its workgroups: four of one head, eight where several heads leave at most 256 workgroups (two of
+// eight waves and several heads do not share a compute unit).  With more than 256 workgroups of one head, long partitions
+// keep the units busy to the end only with eight (32 heads over 8 kv heads, 16 partitions of 65536 rows: 152.6 us with
+// four, 129.6 with eight; of 4096 rows 14.0 and 13.3; a call that attends 200 rows of them: 4.6 and 6.1).
+static int parts_waves(int64_t workgroups, int64_t rows, int heads, int hd)
+{
+    if (hd == 512) return 8;
+    if (heads == 1) return workgroups > 256 && workgroups <= 512 && rows >= 1024 ? 8 : 4;
+    return workgroups <= 256 && rows >= 64 ? 8 : 4;
+}
+
 // Fills in the launch for a shape sdpa_lanes_supports(); the caller has
 // validated the shape and set the buffer sizes of the SDPA kinds.
 int bind_sdpa_lanes(ksh_kernel &k, int nwg, int n_slots)
@@ -1877,7 +1912,7 @@ int bind_sdpa_lanes(ksh_kernel &k, int nwg, int n_slots)
     // heads of 512, merging, 16 partitions, eight waves: one head per workgroup 8.3 / 9.6 / 15.2 us at 320 / 1000 / 3000
     // rows against 8.9 / 10.9 / 17.3 with two)
     int hsplit = k.desc.sched.unroll ? (int)k.desc.sched.unroll
-                 : k.desc.kind == KSH_SDPA_MWG_PART && (hd == 256 || hd == 512) ? total_groups   // (a partition of a few dozen rows: one head per workgroup, 5.6 us against 9.7 for 8 heads of 256, 700 rows, 16 partitions)
+                 : k.desc.kind == KSH_SDPA_MWG_PART && (hd == 256 || hd == 512) ? parts_head_split((int64_t)nwg * n_kv, d[3] / nwg, total_groups, hd)
                  : k.desc.kind != KSH_ATTEND_DECODE || total_groups < 4 ? 1
                  : k.desc.dims[5] || hd == 512 ? total_groups : (total_groups % 2 == 0 ? total_groups / 2 : 1);
     // heads of 512: at most four per workgroup (the fold's LDS)
@@ -1888,7 +1923,7 @@ int bind_sdpa_lanes(ksh_kernel &k, int nwg, int n_slots)
     // the unmerged decode step with one head per workgroup: four waves (eight row groups to fold instead of sixteen; in
     // cfg4's loop 1207-1210 against 1194-1197 tok/s with eight, per launch 4.1 against 4.7 us at 64 rows, equal at 300 - 600)
     if (!k.desc.sched.nsg && k.desc.kind == KSH_ATTEND_DECODE && k.desc.dims[5] != 0 && wg_groups == 1 && hd == 256) nw = 4;
-    if (!k.desc.sched.nsg && k.desc.kind == KSH_SDPA_MWG_PART && wg_groups == 1) nw = hd == 256 ? 4 : 8;
+    if (!k.desc.sched.nsg && k.desc.kind == KSH_SDPA_MWG_PART && (hd == 256 || hd == 512)) nw = parts_waves((int64_t)nwg * n_kv * hsplit, d[3] / nwg, wg_groups, hd);
     // heads of 512, one per workgroup, merging: eight waves at every partition length (16 row groups of 32 lanes)
     if (!k.desc.sched.nsg && k.desc.kind == KSH_ATTEND_DECODE && k.desc.dims[5] == 0 && wg_groups == 1 && hd == 512) nw = 8;
     const size_t lds = lanes_lds(hd, wg_groups, nw, k.desc.kind == KSH_ATTEND_DECODE && lanes_few_heads(1, k.desc.dims[5] ? kModeSplitPart : kModeMerge, wg_groups, hd));

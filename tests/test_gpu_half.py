@@ -260,6 +260,37 @@ def test_rmsnorm_half_every_row_length(ctx, n, res, scale, rows):
         assert rel_err(y[s], want.astype(np.float16).astype(np.float32)).max() <= BAR
 
 
+@pytest.mark.parametrize("n_q,n_kv,hd,max_t,nwg,half", [
+    (8, 1, 256, 1024, 16, 1), (8, 1, 256, 4096, 65, 1), (8, 1, 256, 4224, 128, 1), (16, 2, 256, 4096, 160, 0), (8, 2, 256, 8192, 256, 0),
+    (6, 1, 256, 4096, 100, 1), (7, 1, 256, 3000, 90, 0), (5, 1, 512, 4096, 128, 0), (8, 1, 512, 4096, 100, 1), (8, 4, 512, 2048, 64, 0),
+    (8, 1, 256, 70000, 200, 0), (16, 4, 256, 32768, 32, 0)])
+def test_split_kv_partials_by_launch_size(ctx, n_q, n_kv, hd, max_t, nwg, half):
+    """Partials of launches below and beyond the line from which the q heads share workgroups: one, two, four and eight heads
+    to a workgroup, four and eight waves, head counts that do not divide; the partials of a schedule that names one head per
+    workgroup, and the merged result of the oracle."""
+    tlen, scale = max_t - 7, 1.0 / np.sqrt(hd)
+    kk, vv = synth.q40_blocks(max_t * n_kv * hd // 32, 790), synth.q40_blocks(max_t * n_kv * hd // 32, 791)
+    q, meta = halfed(synth.normal_f32(n_q * hd, 792)), np.array([tlen, 0, 0, 0], np.float32)
+    bk, bv, bm, o = ctx.buffer_bytes(kk), ctx.buffer_bytes(vv), ctx.buffer_f32(meta), ctx.buffer_empty_f32(n_q * hd)
+    bq = ctx.buffer_bytes(q.astype(np.float16).view(np.uint8)) if half else ctx.buffer_f32(q)
+    red = ctx.compile(hip.make_desc(Kind.SDPA_MWG_REDUCE, (n_q, hd, nwg)))
+    got = []
+    for sched in (None, dict(unroll=n_q // n_kv, nsg=4)):
+        tmp = ctx.buffer_empty_f32(n_q * nwg * (hd + 2))
+        k = ctx.compile(hip.make_desc(Kind.SDPA_MWG_PART, (n_q, n_kv, hd, max_t, nwg), (DType.Q40, DType.F16 if half else DType.F32), (scale,), sched))
+        if sched is None and n_q // n_kv in (4, 8) and nwg * n_q > 512:   # a launch that fills the chip: heads share K and V
+            assert n_q // n_kv // k.info.sched.unroll >= 4
+        ctx.encode_multi(k, [bq, bk, bv, bm], [tmp])
+        ctx.encode_multi(red, [tmp], [o])
+        ctx.synchronize()
+        got.append(ctx.read_f32(o, n_q * hd))
+    if max_t <= 8192:
+        want = oracle.sdpa(q, kk, vv, n_q, n_kv, hd, tlen, 0, scale)
+        assert rel_err(got[0], want).max() <= 2e-5
+    # f32 sums of up to 70000 rows in another order
+    assert rel_err(got[0], got[1]).max() <= 2e-5
+
+
 @pytest.mark.parametrize("n_q,n_kv,hd,nwg,tlen", [(8, 1, 256, 16, 700), (8, 1, 512, 5, 301), (4, 2, 128, 9, 77), (2, 2, 256, 1, 30), (2, 1, 64, 64, 500), (2, 1, 256, 65, 500)])
 def test_split_kv_partials_and_merge_half(ctx, n_q, n_kv, hd, nwg, tlen):
     """Half q into split-KV partials (one head per workgroup at heads of 256 and 512), half result of the merge; partition
