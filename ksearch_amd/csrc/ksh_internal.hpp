@@ -44,7 +44,7 @@ inline bool prompt_kind(int kind) { return kind == KSH_MATVEC_BATCH || kind == K
 // The prompt tokens of several pool slots in one pass through the layers: n[i] tokens behind slot slots[i]'s sequence
 // length, at most kPrefillPass in all, with the bits of passes of their own.  taken[i] tells which slots went along (the
 // others, and every slot where fewer than two can, are left to the caller); nonzero with the error set when the pass of
-// those failed.  The scheduler finds the models' function here (null: no model code is linked in, every slot takes its
+// those failed (rows behind the slots' lengths may then have been written).  The scheduler finds the models' function here (null: no model code is linked in, every slot takes its
 // own pass).
 using PrefillSlotsFn = int (*)(ksh_gemma4 *m, ksh_kvpool *pool, const int32_t *slots, const uint32_t *const *tokens, const int *n, int count,
                                uint8_t *taken);

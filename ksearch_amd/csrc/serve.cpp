@@ -202,12 +202,13 @@ struct Share {
     int n;
 };
 
-// The shares' tokens: those that the model takes so as one pass over the weights, the others slot by slot as the
-// reference runs them.
-void prefill_shares(ksh_serve *s, const Share *shares, size_t count)
+// The shares' tokens: those that the model takes so as one pass over the weights, the others -- and all of them where that
+// pass fails, which says nothing about any one request -- slot by slot as the reference runs them.  Returns the tokens of
+// the requests that failed.
+size_t prefill_shares(ksh_serve *s, const std::vector<Share> &shares)
 {
+    const size_t count = shares.size();
     std::vector<uint8_t> taken(count, 0);
-    bool failed = false;
     if (count > 1 && g_prefill_slots && !(s->cfg.use_graph & 2)) {
         std::vector<int32_t> slots(count);
         std::vector<const uint32_t *> tokens(count);
@@ -217,27 +218,29 @@ void prefill_shares(ksh_serve *s, const Share *shares, size_t count)
             tokens[i] = shares[i].a->prompt.data() + shares[i].a->cursor;
             n[i] = shares[i].n;
         }
-        failed = g_prefill_slots(s->model, s->pool, slots.data(), tokens.data(), n.data(), (int)count, taken.data()) != 0;
+        // (the slots' lengths have not moved: a pass alone writes the same rows again)
+        if (g_prefill_slots(s->model, s->pool, slots.data(), tokens.data(), n.data(), (int)count, taken.data())) std::fill(taken.begin(), taken.end(), (uint8_t)0);
     }
-    const std::string why = failed ? ksh_last_error() : "";
+    size_t lost = 0;
     for (size_t i = 0; i < count; i++) {
         Active &a = *shares[i].a;
         const int take = shares[i].n;
-        if ((taken[i] && failed) ||
-            (!taken[i] && (ksh_gemma4_bind_slot(s->model, s->pool, a.slot) ||
-                       ksh_gemma4_prefill_chunk(s->model, a.prompt.data() + a.cursor, take, s->cfg.use_graph))) ||
+        if ((!taken[i] && (ksh_gemma4_bind_slot(s->model, s->pool, a.slot) ||
+                           ksh_gemma4_prefill_chunk(s->model, a.prompt.data() + a.cursor, take, s->cfg.use_graph))) ||
             ksh_kvpool_bump_len_by(s->pool, a.slot, take, nullptr)) {
-            push_error(s, a.id, taken[i] && failed ? why : ksh_last_error());
+            push_error(s, a.id, ksh_last_error());
             finish(s, a, KSH_FINISH_ERROR);
+            lost += (size_t)take;
             continue;
         }
         a.cursor += (size_t)take;
         if (a.cursor >= a.prompt.size() - 1) enter_decode(a);
     }
+    return lost;
 }
 
 // scheduler.rs:243-303.  The shares of the round's budget are dealt as there and go through the layers together, as many
-// to a pass as it takes tokens.
+// to a pass as it takes tokens; what a failing request leaves of its share goes to those after it.
 void prefill_round(ksh_serve *s)
 {
     const size_t n = s->active.size();
@@ -245,26 +248,27 @@ void prefill_round(ksh_serve *s)
     const bool decoding = std::any_of(s->active.begin(), s->active.end(), [](const Active &a) { return !a.finished && !a.prefill; });
     size_t budget = (size_t)std::max(s->cfg.prefill_tokens_per_tick, s->cfg.prefill_chunk);
     size_t idx = s->prefill_cursor % n;
-    std::vector<Share> shares;
-    for (size_t i = 0; i < n && budget; i++) {
-        Active &a = s->active[idx];
-        idx = (idx + 1) % n;
-        if (a.finished || !a.prefill) continue;
-        // the last prompt token is the first decode input, not a prefill step
-        const size_t prefill_end = a.prompt.size() - 1;
-        if (a.cursor >= prefill_end) { enter_decode(a); continue; }
-        // small chunks while something decodes; otherwise the whole budget
-        const size_t cap = decoding ? (size_t)s->cfg.prefill_chunk : budget;
-        const size_t take = std::min({budget, cap, prefill_end - a.cursor});
-        shares.push_back(Share{&a, (int)take});
-        budget -= take;
+    size_t had = 0;      // what the request at idx has got: the budget ended within its share
+    for (size_t i = 0; i < n && budget;) {
+        std::vector<Share> shares;
+        for (size_t total = 0; i < n && budget; i++, idx = (idx + 1) % n, had = 0) {
+            Active &a = s->active[idx];
+            if (a.finished || !a.prefill) continue;
+            // the last prompt token is the first decode input, not a prefill step
+            const size_t prefill_end = a.prompt.size() - 1;
+            if (a.cursor >= prefill_end) { enter_decode(a); continue; }
+            // small chunks while something decodes; otherwise the whole budget
+            const size_t left = prefill_end - a.cursor, want = decoding ? std::min((size_t)s->cfg.prefill_chunk - had, left) : left;
+            const size_t take = std::min(budget, want);
+            if (total && total + take > (size_t)kPrefillPass) break;
+            shares.push_back(Share{&a, (int)take});
+            total += take;
+            budget -= take;
+            if (take < want) { had += take; break; }
+        }
+        budget += prefill_shares(s, shares);
     }
-    s->prefill_cursor = idx;
-    for (size_t i0 = 0, i1; i0 < shares.size(); i0 = i1) {
-        int total = 0;
-        for (i1 = i0; i1 < shares.size() && (i1 == i0 || total + shares[i1].n <= kPrefillPass); i1++) total += shares[i1].n;
-        prefill_shares(s, shares.data() + i0, i1 - i0);
-    }
+    s->prefill_cursor = had ? (idx + 1) % n : idx;
 }
 
 // scheduler.rs:294-303 (reap_finished)

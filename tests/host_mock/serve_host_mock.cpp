@@ -59,7 +59,7 @@ static hipError_t host_free(void *p)
 }
 
 struct MockCall {
-    int32_t kind;   // 0 bind_slot, 1 prefill_chunk, 2 decode_token_sampled, 3 one row of decode_round
+    int32_t kind;   // 0 bind_slot, 1 prefill_chunk, 2 decode_token_sampled, 3 one row of decode_round, 4 one slot of a joint prompt pass
     int32_t slot, pos, n;
     uint32_t token, seed;
     float temperature, min_p;
@@ -67,7 +67,7 @@ struct MockCall {
 
 struct ksh_gemma4 {
     int max_seq = 64, vocab = 1000;
-    int mode = 0;              // 0: next = (31 * token + 7 * pos + 1) % vocab; 1: always `constant`; 2: decode fails at position fail_pos
+    int mode = 0;              // 0: next = (31 * token + 7 * pos + 1) % vocab; 1: always `constant`; 2: decode fails at position fail_pos; 3: prompt passes of slot fail_pos fail
     uint32_t constant = 5;
     int fail_pos = -1;
     int pos = 0, slot = -1;
@@ -195,9 +195,30 @@ int ksh_gemma4_bind_slot(ksh_gemma4 *m, ksh_kvpool *pool, int slot)
 int ksh_gemma4_prefill_chunk(ksh_gemma4 *m, const uint32_t *tokens, int n, int)
 {
     if (m->pos + n > m->max_seq) return ksh::set_error("max_seq exceeded");
+    if (m->mode == 3 && m->slot == m->fail_pos) return ksh::set_error("mock prompt failure in slot %d", m->slot);
     m->calls.push_back(MockCall{1, m->slot, m->pos, n, n ? tokens[0] : 0, 0, 0.f, 0.f});
     m->pos += n;
     return 0;
+}
+
+// the joint prompt pass: takes every slot; fails after logging where g_joint_fails
+static bool g_joint_fails = false;
+static int mock_prefill_slots(ksh_gemma4 *m, ksh_kvpool *pool, const int32_t *slots, const uint32_t *const *tokens, const int *n, int count, uint8_t *taken)
+{
+    int total = 0;
+    for (int i = 0; i < count; i++) {
+        m->calls.push_back(MockCall{4, slots[i], ksh_kvpool_seq_len(pool, slots[i]), n[i], tokens[i][0], 0, 0.f, 0.f});
+        taken[i] = 1;
+        total += n[i];
+    }
+    if (total > ksh::kPrefillPass) abort();
+    return g_joint_fails ? ksh::set_error("mock joint pass failure") : 0;
+}
+// 0: no joint passes, 1: joint passes, 2: joint passes that fail
+void mock_joint(int mode)
+{
+    ksh::g_prefill_slots = mode ? mock_prefill_slots : nullptr;
+    g_joint_fails = mode == 2;
 }
 
 int ksh_gemma4_decode_token_sampled(ksh_gemma4 *m, uint32_t token, float temperature, float min_p, uint32_t seed, int, uint32_t *next)

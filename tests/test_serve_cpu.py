@@ -108,7 +108,7 @@ class Rig:
     def calls(self, clear=True):
         buf = (Call * 4096)()
         n = self.L.mock_model_calls(self.model, buf, 4096)
-        out = [(("bind", "prefill", "decode", "round")[c.kind], c.slot, c.pos, c.n) for c in buf[:n]]
+        out = [(("bind", "prefill", "decode", "round", "joint")[c.kind], c.slot, c.pos, c.n) for c in buf[:n]]
         full = list(buf[:n])
         if clear:
             self.L.mock_model_clear_calls(self.model)
@@ -343,3 +343,62 @@ def test_batched_decode_more_requests_than_a_round_holds_and_errors(L):
     assert len(toks[a]) == 1 and len(toks[b]) == 1           # position 2 decoded, position 3 failed
     assert rig.occupied() == 0
     rig.close()
+
+
+def done_reason(r, request):
+    return split(r.run())[1][request][0]
+
+
+@pytest.fixture()
+def joint(L):
+    yield L.mock_joint
+    L.mock_joint(0)
+
+
+def test_a_failing_joint_pass_leaves_the_requests_their_own_passes(L, joint):
+    """The prompts of a tick go through the layers together; where that pass fails each takes one of its own, and only a
+    request whose own pass fails ends."""
+    p = [list(range(10 * i + 1, 10 * i + 9)) for i in range(3)]
+    for mode, slot in ((1, -1), (2, -1), (2, 1)):
+        joint(mode)
+        r = Rig(L, slots=3, mode=3, fail_pos=slot)
+        ids = [r.submit(q, 3) for q in p]
+        events = r.tick()
+        own = [c for i in range(3) for c in (("bind", i, 0, 0), ("prefill", i, 0, 7)) if mode == 2 and (c[0] == "bind" or i != slot)]
+        assert r.calls()[0] == [("joint", i, 0, 7) for i in range(3)] + own
+        toks, done, errs = split(events + r.run())
+        assert list(errs) == ([ids[slot]] if slot >= 0 else [])
+        for i in range(3):
+            if i != slot:
+                assert toks[ids[i]] == expected(p[i], 3) and done[ids[i]] == ("length", 8, 3)
+        assert r.occupied() == 0
+        r.close()
+
+
+def test_a_failing_request_leaves_its_share_of_the_budget(L, joint):
+    """scheduler.rs:271-289: the budget shrinks by what was prefilled.  A request that fails leaves its share to those after
+    it, the one the budget had cut short first."""
+    p = [list(range(10 * i + 1, 10 * i + 9)) for i in range(3)]
+    for mode in (0, 2):
+        joint(mode)
+        r = Rig(L, slots=3, prefill_chunk=4, prefill_tokens_per_tick=10, mode=3, fail_pos=0)
+        ids = [r.submit(q, 3) for q in p]
+        toks, done, errs = split(r.tick())
+        assert list(errs) == [ids[0]] and "slot 0" in errs[ids[0]]
+        calls = [c for c in r.calls()[0] if c[0] == "prefill"]
+        assert calls == [("prefill", 1, 0, 3), ("prefill", 1, 3, 4), ("prefill", 2, 0, 3)]     # 7 + 3 = the budget
+        toks, done, errs = split(r.run())
+        assert not errs and toks[ids[1]] == expected(p[1], 3) and toks[ids[2]] == expected(p[2], 3)
+        r.close()
+    # small chunks while something decodes: the share that is cut stays within its chunk
+    joint(0)
+    r = Rig(L, slots=4, prefill_chunk=4, prefill_tokens_per_tick=6, mode=3, fail_pos=1)
+    first = r.submit([5, 6], 20)
+    r.tick()
+    for q in p:
+        r.submit(q, 3)
+    r.calls()
+    r.tick()
+    assert [c for c in r.calls()[0] if c[0] == "prefill"] == [("prefill", 2, 0, 2), ("prefill", 2, 2, 2), ("prefill", 3, 0, 2)]
+    assert done_reason(r, first) == "length"
+    r.close()
