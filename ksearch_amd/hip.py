@@ -14,6 +14,7 @@ import enum
 import importlib.machinery
 import importlib.util
 import os
+import sys
 
 import numpy as np
 
@@ -254,25 +255,45 @@ SYMBOLS = {
 }
 
 _lib = None
-_encode = None      # pyext/encode.c's encode(ctx, kernel, inputs, in_offs, outputs, out_offs) -> ksh_encode's code
+_encode = None      # encode(ctx, kernel, inputs, in_offs, outputs, out_offs) -> ksh_encode's code (pyext/encode.c, or ctypes)
+
+
+def _encode_ctypes(fn):
+    """pyext/encode.c's call without the extension."""
+    def encode(ctx, kernel, inputs, in_offs, outputs, out_offs):
+        inputs, outputs = list(inputs), list(outputs)
+        return fn(ctx, kernel, _bufs(inputs), _offs(in_offs, len(inputs)), len(inputs),
+                  _bufs(outputs), _offs(out_offs, len(outputs)), len(outputs))
+    return encode
+
+
+def _load_encode(fn):
+    """The extension, where this interpreter can load it (CPython from 3.10 on), else the call through ctypes; the same
+    library function either way."""
+    if os.path.exists(ENCODE_PATH) and sys.version_info >= (3, 10):
+        try:
+            loader = importlib.machinery.ExtensionFileLoader("ksearch_amd._encode", ENCODE_PATH)
+            ext = importlib.util.module_from_spec(importlib.util.spec_from_loader(loader.name, loader))
+            loader.exec_module(ext)
+        except ImportError:
+            pass
+        else:
+            ext.setup(C.cast(fn, C.c_void_p).value)
+            return ext.encode
+    return _encode_ctypes(fn)
 
 
 def lib() -> C.CDLL:
     """Loads the prebuilt library; never builds and never falls back."""
     global _lib, _encode
     if _lib is None:
-        for path in (LIB_PATH, ENCODE_PATH):
-            if not os.path.exists(path):
-                raise KshError(f"{path} is missing: build it with `python -c 'import __graft_entry__ as g; g.build()'`")
+        if not os.path.exists(LIB_PATH):
+            raise KshError(f"{LIB_PATH} is missing: build it with `python -c 'import __graft_entry__ as g; g.build()'`")
         L = C.CDLL(LIB_PATH)
         for name, (res, args) in SYMBOLS.items():
             fn = getattr(L, name)
             fn.restype, fn.argtypes = res, args
-        loader = importlib.machinery.ExtensionFileLoader("ksearch_amd._encode", ENCODE_PATH)
-        ext = importlib.util.module_from_spec(importlib.util.spec_from_loader(loader.name, loader))
-        loader.exec_module(ext)
-        ext.setup(C.cast(L.ksh_encode, C.c_void_p).value)
-        _lib, _encode = L, ext.encode
+        _lib, _encode = L, _load_encode(L.ksh_encode)
     return _lib
 
 

@@ -6,9 +6,13 @@
  *
  *   setup(address of ksh_encode)
  *   encode(ctx, kernel, inputs, in_offs, outputs, out_offs) -> the library's return code
- * ctx and kernel are integers; inputs / outputs are lists or tuples of objects with a handle in attribute `h` (None: a
- * null binding, which the library refuses); offsets are None or sequences of byte offsets. */
+ * ctx and kernel are integers; inputs / outputs are iterables of objects with a handle in attribute `h` (None: a null
+ * binding, which the library refuses); offsets are None or iterables of byte offsets, taken as int() takes them.  The
+ * ctypes form of the same call (hip.py, _encode_ctypes) accepts and refuses what this one does.
+ *
+ * Built against the limited API: one binary for every CPython from 3.10 on. */
 #define PY_SSIZE_T_CLEAN
+#define Py_LIMITED_API 0x030a0000
 #include <Python.h>
 #include <stdint.h>
 
@@ -25,34 +29,38 @@ static int as_ptr(PyObject *o, void **out)
     return PyErr_Occurred() ? -1 : 0;
 }
 
-/* handles of a sequence of buffers, and their offsets (zero where there are none) */
+/* item i (borrowed) of what PySequence_Fast returned */
+static PyObject *item(PyObject *seq, int is_list, Py_ssize_t i) { return is_list ? PyList_GetItem(seq, i) : PyTuple_GetItem(seq, i); }
+
+/* handles of a sequence of buffers, and their offsets (zero where there are none); of more than any kernel has only the
+ * number, which the library refuses before it looks at them */
 static int bindings(PyObject *bufs, PyObject *offs, void **ptr, uint64_t *off)
 {
-    PyObject *b = PySequence_Fast(bufs, "bindings are a list or a tuple of buffers"), *o = NULL;
+    PyObject *b = PySequence_Fast(bufs, "bindings are an iterable of buffers"), *o = NULL;
     if (!b) return -1;
-    Py_ssize_t n = PySequence_Fast_GET_SIZE(b);
-    int rc = -1;
-    if (n > kMax) {
-        PyErr_Format(PyExc_ValueError, "%zd bindings (at most %d)", n, kMax);
-        goto done;
-    }
+    const int b_list = PyList_Check(b);
+    const Py_ssize_t n = PySequence_Size(b);
+    Py_ssize_t n_off = 0;
+    int rc = -1, o_list = 0;
     if (offs != Py_None) {
-        o = PySequence_Fast(offs, "offsets are a list or a tuple of numbers");
+        o = PySequence_Fast(offs, "offsets are an iterable of numbers");
         if (!o) goto done;
-        if (PySequence_Fast_GET_SIZE(o) > n) {
+        o_list = PyList_Check(o);
+        n_off = PySequence_Size(o);
+        if (n_off > (n ? n : 1)) {
             PyErr_SetString(PyExc_IndexError, "more offsets than bindings");
             goto done;
         }
     }
-    for (Py_ssize_t i = 0; i < n; i++) {
-        PyObject *h = PyObject_GetAttr(PySequence_Fast_GET_ITEM(b, i), g_h);
+    for (Py_ssize_t i = 0; i < n && i < kMax; i++) {
+        PyObject *e = item(b, b_list, i), *h = e ? PyObject_GetAttr(e, g_h) : NULL;
         if (!h) goto done;
         const int bad = as_ptr(h, &ptr[i]);
         Py_DECREF(h);
         if (bad) goto done;
         off[i] = 0;
-        if (o && i < PySequence_Fast_GET_SIZE(o)) {
-            PyObject *v = PyNumber_Index(PySequence_Fast_GET_ITEM(o, i));
+        if (i < n_off) {
+            PyObject *e_off = item(o, o_list, i), *v = e_off ? PyNumber_Long(e_off) : NULL;
             if (!v) goto done;
             off[i] = PyLong_AsUnsignedLongLongMask(v);
             Py_DECREF(v);
