@@ -579,7 +579,11 @@ class Eng:
 
     def _k(self, ctx: Context, kind, dims=(), dtypes=(), params=(), sched=None) -> Kernel:
         key = (kind, dims, dtypes, params, tuple(sorted(sched.items())) if isinstance(sched, dict) else None)
-        k = self.cache.get(key)
+        try:
+            k = self.cache.get(key)
+        except TypeError:       # lists (the library's own calls pass tuples, which need no copy)
+            key = (kind, tuple(dims), tuple(dtypes), tuple(params), key[-1])
+            k = self.cache.get(key)
         if k is None:
             k = ctx.compile(make_desc(kind, dims, dtypes, params, sched))
             self.cache[key] = k

@@ -161,3 +161,23 @@ def test_plan_kinds_and_candidates():
     assert mm(512, 8192, 2048, hip.DType.BF16) == [(128, 1)]
     assert mm(256, 2048, 2048, hip.DType.F32) == [(128, 1), (128, 2), (128, 4)]
     assert mm(40, 2048, 1536, hip.DType.F32) == [(128, 1), (32, 8), (128, 2)]
+
+
+def test_kernel_lookup_takes_any_sequence():
+    """Eng._k with lists, arrays and tuples of the same numbers finds one handle."""
+    import numpy as np
+
+    class Ctx:
+        made = 0
+
+        def compile(self, desc):
+            self.made += 1
+            return (self.made, desc.dims[0], desc.dtypes[0], desc.params[0])
+
+    ctx, eng = Ctx(), hip.Eng()
+    k = eng._k(ctx, hip.Kind.MATVEC, (512, 1024), (hip.DType.Q4K, hip.DType.F32), (0.5,))
+    assert k == (1, 512, int(hip.DType.Q4K), 0.5)
+    for seq in (list, np.array, tuple):
+        assert eng._k(ctx, hip.Kind.MATVEC, seq((512, 1024)), seq((hip.DType.Q4K, hip.DType.F32)), seq((0.5,))) is k
+        assert eng._k(ctx, int(hip.Kind.MATVEC), seq((512, 1024)), (2, 0), [0.5]) is k
+    assert eng._k(ctx, hip.Kind.MATVEC, [512, 1024], (2, 0), (0.5,), dict(nsg=4)) != k
