@@ -135,13 +135,15 @@ struct ksh_gemma4 {
     int bound_slot = -1;
     // prompt chunks (allocated at the first chunk): [kChunk, .] activations of the batched layer pass
     ksh_buf *c_tok = nullptr, *c_x = nullptr, *c_x2 = nullptr, *c_y = nullptr, *c_q = nullptr, *c_k = nullptr, *c_v = nullptr, *c_o = nullptr,
-            *c_g = nullptr, *c_u = nullptr, *c_ff = nullptr, *c_tmp = nullptr, *c_meta_full = nullptr, *c_meta_swa = nullptr,
+            *c_ff = nullptr, *c_tmp = nullptr, *c_meta_full = nullptr, *c_meta_swa = nullptr,
             *c_po = nullptr, *c_pg = nullptr,   // unfolded partial sums of the o and the gate | up projection of a chunk
+            *c_g = nullptr, *c_u = nullptr,     // gate and up apart (c_pg, c_g, c_u: by the passes whose gate | up does not leave gelu(gate) * up)
             *c_ple_tok = nullptr, *c_ple_tmp = nullptr, *c_ple_ctx = nullptr, *c_ple_u = nullptr,
             *c_tab = nullptr;                   // a pass over several slots: ids, slots, attended ranges per token
     // decode rounds over several KV slots (allocated at the first round): the per-token table (ids, slots, attended
     // ranges of the two layer kinds), the logits of every token of the round, the greedy ids
-    ksh_buf *r_tab = nullptr, *r_logits = nullptr, *r_next = nullptr, *r_xp = nullptr, *r_xp2 = nullptr;   // (r_xp, r_xp2: a round's prepared GEMM operands)
+    ksh_buf *r_tab = nullptr, *r_logits = nullptr, *r_next = nullptr, *r_xp = nullptr, *r_xp2 = nullptr,   // (r_xp, r_xp2: a round's prepared GEMM operands)
+            *r_g = nullptr, *r_u = nullptr;     // gate and up apart, or a down projection's unfolded sums
     // a round of t sequences is one graph per t, tied to the pool whose buffers it was captured over
     ksh_graph *round_graphs[17] = {};
     bool round_bound[17] = {};     // a width's kernels are bound (a first round launched kernel by kernel)
@@ -464,6 +466,8 @@ int write_token(ksh_gemma4 *m, uint32_t token)
 constexpr int kChunk4 = kPrefillPass;
 constexpr int kChunkPartitions4 = 8;
 constexpr int kSmallPass = 64;      // tokens up to which a GEMM of one matrix takes the small-batch form
+constexpr int kRoundMax = 16;       // sequences of a decode round: the attention launch shares its partitions among up to 16 entries by length
+constexpr int kRoundPartitions = 16;
 constexpr int kPartsRows4 = 4;      // room for the unfolded partial sums of a hidden-wide projection: this many chunks of rows
 
 int chunk_buffers4(ksh_gemma4 *m)
@@ -474,12 +478,15 @@ int chunk_buffers4(ksh_gemma4 *m)
     size_t max_ff = 0;
     for (const ksh_gemma4_layer &L : m->layers) max_ff = std::max(max_ff, (size_t)L.ffn);
     const size_t pt = (size_t)c.n_layers * c.ple_dim;
+    // attention partials: a token a partition where the long passes' form takes one (and then a short pass's or a round's)
+    bool one = c.n_q / c.n_kv <= 8;
+    for (const LayerPlan &P : m->plan) one = one && (P.hd == 256 || P.hd == 512);
+    const size_t parts = one ? std::max(T, (size_t)kRoundMax * kRoundPartitions) : T * kChunkPartitions4;
     return alloc_together(m->ctx, m->bufs.owned,
                           {{T * 4, &m->c_tok}, {T * 11 * 4, &m->c_tab}, {T * c.hidden * 4, &m->c_x}, {T * c.hidden * 4, &m->c_x2},
                            {T * c.hidden * 4, &m->c_y}, {T * qd * 4, &m->c_q}, {T * kvd * 4, &m->c_k}, {T * kvd * 4, &m->c_v}, {T * qd * 4, &m->c_o},
-                           {T * max_ff * 4, &m->c_g}, {T * max_ff * 4, &m->c_u}, {T * max_ff * 4, &m->c_ff},
-                           {T * c.n_q * kChunkPartitions4 * (max_hd + 2) * 4, &m->c_tmp}, {16, &m->c_meta_full}, {16, &m->c_meta_swa},
-                           {kPartsRows4 * T * c.hidden * 4, &m->c_po}, {2 * T * 2 * max_ff * 4, &m->c_pg},
+                           {T * max_ff * 4, &m->c_ff}, {parts * c.n_q * (max_hd + 2) * 4, &m->c_tmp}, {16, &m->c_meta_full}, {16, &m->c_meta_swa},
+                           {kPartsRows4 * T * c.hidden * 4, &m->c_po},
                            {T * pt * 4, &m->c_ple_tok}, {T * pt * 4, &m->c_ple_tmp},
                            {T * pt * 4, &m->c_ple_ctx}, {T * c.ple_dim * 4, &m->c_ple_u}});
 }
@@ -660,8 +667,11 @@ int forward_prefill_chunk4(ksh_gemma4 *m, const uint32_t *tokens, int t, const J
             if (get(m, KSH_MATVEC_BATCH, {h, P.qd, tp, 0, 0, 0, 1}, {L.dt_o, KSH_F32, KSH_F32}, {c.eps}, &u_o) ||
                 get(m, KSH_MATVEC_BATCH, {L.ffn, h, tp, L.ffn, 0, 2, pair ? 3 : 1, (int64_t)u_o->info.grid[2]}, {L.dt_gate, KSH_F32, KSH_F32}, {c.eps}, &u_gu))
                 return 1;
-            travel = u_o->out_bytes[0] <= kPartsRows4 * T * c.hidden * 4 && u_gu->out_bytes[0] <= ksh_buffer_size(pair ? m->c_ff : m->c_pg);
+            travel = u_o->out_bytes[0] <= kPartsRows4 * T * c.hidden * 4 && u_gu->out_bytes[0] <= ksh_buffer_size(m->c_ff) * (pair ? 1 : 4);
         }
+        if (!pair && (travel ? grow_buffer(m->ctx, m->bufs.owned, u_gu->out_bytes[0], &m->c_pg)
+                             : (grow_buffer(m->ctx, m->bufs.owned, (size_t)tp * L.ffn * 4, &m->c_g) || grow_buffer(m->ctx, m->bufs.owned, (size_t)tp * L.ffn * 4, &m->c_u))))
+            return 1;
         if (travel) {
             if (enc(m, u_o, {L.wo, m->c_o}, {m->c_po}, n) ||
                 enc(m, u_gu, {L.wgate, m->c_po, L.wup, L.post_attn_norm, m->c_x, L.ffn_norm}, {pair ? m->c_ff : m->c_pg, m->c_x}, n) ||
@@ -1137,8 +1147,6 @@ int ksh_gemma4_prefill_chunk(ksh_gemma4 *m, const uint32_t *tokens, int n, int u
 // gemma_prim.rs:1317-1607, with one position, one attended range and one KV slot per row), so the weights are read
 // once per round.  Row i appends to and attends the caches of pool slot slots[i] at that slot's sequence length.
 namespace {
-constexpr int kRoundMax = 16;         // the attention launch shares its partitions among up to 16 entries by length
-constexpr int kRoundPartitions = 16;
 constexpr int kRoundStride = 16;      // floats per field of the table: ids | slots | full-attention records | sliding-window records
 
 // A round's table as an argument of the launch that stores it: the stream keeps the order, no wait for the copy engine (nor
@@ -1218,10 +1226,10 @@ int forward_decode_round4(ksh_gemma4 *m, ksh_kvpool *pool, const int32_t *slots,
     int64_t widest = std::max<int64_t>(c.hidden, c.ple_dim);
     for (int l = 0; l < c.n_layers; l++) widest = std::max<int64_t>(widest, std::max<int64_t>(m->layers[l].ffn, m->plan[l].qd));
     widest = (widest + 255) / 256 * 256;
-    const size_t xp = (size_t)(64 * widest + 2048 * (widest / 256));
+    const size_t xp = (size_t)(64 * widest + 2048 * (widest / 256)), gate = (size_t)std::max<int64_t>(32 * widest, kRoundMax * (widest / 2048 + 1) * c.hidden) * 4;
     if (!m->r_tab && alloc_together(m->ctx, m->bufs.owned,
                                     {{(size_t)kRoundStride * 10 * 4, &m->r_tab}, {(size_t)kRoundMax * c.vocab * 4, &m->r_logits},
-                                     {(size_t)kRoundMax * 4, &m->r_next}, {xp, &m->r_xp}, {xp, &m->r_xp2}}))
+                                     {(size_t)kRoundMax * 4, &m->r_next}, {xp, &m->r_xp}, {xp, &m->r_xp2}, {gate, &m->r_g}, {gate, &m->r_u}}))
         return 1;
     RoundTable table{};
     float *tab = table.v;
@@ -1405,7 +1413,7 @@ int encode_round4(ksh_gemma4 *m, ksh_kvpool *pool, int t, int max_batch, int poo
         }
         const bool gu_q4k = L.dt_gate == KSH_Q4K && L.dt_up == KSH_Q4K && h <= 8192;
         const bool ple_q4k = c.ple_dim > 0 && L.dt_inp_gate == KSH_Q4K && L.dt_proj == KSH_Q4K && c.ple_dim % 256 == 0 && h <= 2048;
-        // a down projection whose columns are split leaves its slices' partial sums (in c_g) to the closing norm where
+        // a down projection whose columns are split leaves its slices' partial sums (in r_g) to the closing norm where
         // that norm is the kind that adds them up
         const int down_slices = (int)((L.ffn / 256 + 7) / 8);
         const bool down_unfolded = L.dt_down == KSH_Q4K && ple_q4k && down_slices > 1;
@@ -1424,17 +1432,17 @@ int encode_round4(ksh_gemma4 *m, ksh_kvpool *pool, int t, int max_batch, int poo
             if (chain) {
                 ksh_kernel *k_dn = nullptr;
                 if (get(m, KSH_MATVEC_ROUND, {h, L.ffn, t, 0, 0, 0, down_unfolded ? 2 : 0}, {KSH_Q4K}, {}, &k_dn) ||
-                    enc(m, k_dn, {L.wdown, m->r_xp2}, {down_unfolded ? m->c_g : m->c_y}, n))
+                    enc(m, k_dn, {L.wdown, m->r_xp2}, {down_unfolded ? m->r_g : m->c_y}, n))
                     return 1;
                 down_done = true;
             }
-        } else if (mm(L.dt_gate, L.ffn, h, L.wgate, m->c_x2, m->c_g) || mm(L.dt_up, L.ffn, h, L.wup, m->c_x2, m->c_u) ||
-                   get(m, KSH_GELU_MUL, {(int64_t)t * L.ffn}, {}, {}, &k_gelu) || enc(m, k_gelu, {m->c_g, m->c_u}, {m->c_ff}, n)) {
+        } else if (mm(L.dt_gate, L.ffn, h, L.wgate, m->c_x2, m->r_g) || mm(L.dt_up, L.ffn, h, L.wup, m->c_x2, m->r_u) ||
+                   get(m, KSH_GELU_MUL, {(int64_t)t * L.ffn}, {}, {}, &k_gelu) || enc(m, k_gelu, {m->r_g, m->r_u}, {m->c_ff}, n)) {
             return 1;
         }
         if (!down_done && down_unfolded) {
             ksh_kernel *k_dn = nullptr;
-            if (prep(L.ffn, m->c_ff) || get(m, KSH_MATVEC_ROUND, {h, L.ffn, t, 0, 0, 0, 2}, {KSH_Q4K}, {}, &k_dn) || enc(m, k_dn, {L.wdown, m->r_xp}, {m->c_g}, n))
+            if (prep(L.ffn, m->c_ff) || get(m, KSH_MATVEC_ROUND, {h, L.ffn, t, 0, 0, 0, 2}, {KSH_Q4K}, {}, &k_dn) || enc(m, k_dn, {L.wdown, m->r_xp}, {m->r_g}, n))
                 return 1;
             down_done = true;
         }
@@ -1447,7 +1455,7 @@ int encode_round4(ksh_gemma4 *m, ksh_kvpool *pool, int t, int max_batch, int poo
             // gelu(W x) * context leaves as the projection's prepared operand
             ksh_kernel *k_pa = nullptr, *k_pg = nullptr, *k_pp = nullptr, *k_as = nullptr;
             if (get(m, KSH_ROUND_PREP, {h, t, 3, down_unfolded ? down_slices : 0}, {KSH_F32}, {c.eps}, &k_pa) ||
-                enc(m, k_pa, {down_unfolded ? m->c_g : m->c_y, L.post_ffw_norm, m->c_x}, {m->r_xp, m->c_x}, n) ||
+                enc(m, k_pa, {down_unfolded ? m->r_g : m->c_y, L.post_ffw_norm, m->c_x}, {m->r_xp, m->c_x}, n) ||
                 get(m, KSH_MATVEC_ROUND, {c.ple_dim, h, t, 0, 0, 0, 1, pt}, {KSH_Q4K}, {}, &k_pg) ||
                 enc_off(m, k_pg, {L.inp_gate, m->r_xp, m->c_ple_ctx}, {0, 0, (size_t)l * c.ple_dim * 4}, {m->r_xp2}, n) ||
                 get(m, KSH_MATVEC_ROUND, {h, c.ple_dim, t, 0, 0, 0}, {KSH_Q4K}, {}, &k_pp) || enc(m, k_pp, {L.proj, m->r_xp2}, {m->c_y}, n) ||

@@ -125,8 +125,9 @@ struct ksh_gemma {
     std::vector<float> rope0;   // row 0 of the rope table, for reset
     // prompt chunks (allocated at the first chunk): [kChunk, .] activations of the batched layer pass
     ksh_buf *c_tok = nullptr, *c_x = nullptr, *c_x2 = nullptr, *c_y = nullptr, *c_q = nullptr, *c_k = nullptr, *c_v = nullptr, *c_o = nullptr,
-            *c_g = nullptr, *c_u = nullptr, *c_ff = nullptr, *c_tmp = nullptr, *c_meta = nullptr,
-            *c_po = nullptr, *c_pg = nullptr, *c_pd = nullptr;   // unfolded partial sums of the o, gate | up and down projections
+            *c_ff = nullptr, *c_tmp = nullptr, *c_meta = nullptr,
+            *c_po = nullptr, *c_pg = nullptr, *c_pd = nullptr,   // unfolded partial sums of the o, gate | up and down projections
+            *c_g = nullptr, *c_u = nullptr;                      // gate and up apart (c_pg, c_g, c_u: by the passes that need them)
     int c_nwg = 0;
     ksh::SectionTimer prof;   // KSEARCH_PROFILE (read when the model is created): per-section times of every decode step
 };
@@ -371,12 +372,13 @@ int chunk_buffers(ksh_gemma *m)
     const ksh_gemma_cfg &c = m->c;
     const size_t T = kChunk, qd = (size_t)c.n_q * c.hd, kvd = (size_t)c.n_kv * c.hd;
     m->c_nwg = kChunkPartitions;
+    // attention partials: a token a partition where the long passes' form takes one (and then a short pass's)
+    const size_t parts = c.hd == 256 && c.n_q / c.n_kv <= 8 ? T : T * m->c_nwg;
     return alloc_together(m->ctx, m->bufs.owned,
                           {{T * 4, &m->c_tok}, {T * c.hidden * 4, &m->c_x}, {T * c.hidden * 4, &m->c_x2}, {T * c.hidden * 4, &m->c_y},
                            {T * qd * 4, &m->c_q}, {T * kvd * 4, &m->c_k}, {T * kvd * 4, &m->c_v}, {T * qd * 4, &m->c_o},
-                           {T * c.ffn * 4, &m->c_g}, {T * c.ffn * 4, &m->c_u}, {T * c.ffn * 4, &m->c_ff},
-                           {T * c.n_q * m->c_nwg * (c.hd + 2) * 4, &m->c_tmp}, {16, &m->c_meta}, {kPartsRows * T * c.hidden * 4, &m->c_po},
-                           {2 * T * 2 * c.ffn * 4, &m->c_pg}, {kPartsRows * T * c.hidden * 4, &m->c_pd}});
+                           {T * c.ffn * 4, &m->c_ff}, {parts * c.n_q * (c.hd + 2) * 4, &m->c_tmp}, {16, &m->c_meta},
+                           {kPartsRows * T * c.hidden * 4, &m->c_po}, {kPartsRows * T * c.hidden * 4, &m->c_pd}});
 }
 
 // forward_prefill_chunk (gemma_prim.rs:1317-1607) for 2 <= t <= kChunk tokens already validated: the layer as
@@ -424,7 +426,6 @@ int forward_prefill_chunk(ksh_gemma *m, const uint32_t *tokens, int t)
     }
     // ... and a layer's closing norm + add with the next layer's attention norm are one add-then-norm, in that
     // layer's q | k | v preparation (the residual rows it stores are the closed layer's)
-    ksh_buf *gu = pair ? m->c_ff : m->c_pg;
     ksh_kernel *k_mm_qkv_close = nullptr;
     if (fused && c.n_layers > 1 && get(m, KSH_MATVEC_BATCH, {qd, c.hidden, tp, kvd, kvd, 2}, {KSH_Q4K, KSH_F32, KSH_F32}, {c.eps}, &k_mm_qkv_close)) return 1;
     const float embed_scale = std::sqrt((float)c.hidden);
@@ -448,6 +449,11 @@ int forward_prefill_chunk(ksh_gemma *m, const uint32_t *tokens, int t)
     if (hipGetLastError() != hipSuccess) return set_error("chunk_begin launch failed");
     int n = 0;
     if (enc(m, k_embed, {m->embd, m->c_tok}, {m->c_x}, n)) return 1;
+    const size_t apart = (size_t)tp * c.ffn * 4;
+    if (travel ? !pair && grow_buffer(m->ctx, m->bufs.owned, u_gu->out_bytes[0], &m->c_pg)
+               : grow_buffer(m->ctx, m->bufs.owned, apart, &m->c_g) || grow_buffer(m->ctx, m->bufs.owned, apart, &m->c_u))
+        return 1;
+    ksh_buf *gu = pair ? m->c_ff : m->c_pg;
     for (int l = 0; l < c.n_layers; l++) {
         const ksh_gemma_layer &L = m->layers[l];
         if (travel) {

@@ -198,6 +198,22 @@ inline int alloc_together(ksh_ctx *ctx, std::vector<ksh_buf *> &owned, std::init
     return 0;
 }
 
+// A buffer of at least `bytes` that only some calls need: made, or made larger (in steps of 16 MiB), by the first that does.
+// Its contents do not survive; nothing that keeps its address (a captured graph) may use it.
+inline int grow_buffer(ksh_ctx *ctx, std::vector<ksh_buf *> &owned, size_t bytes, ksh_buf **b)
+{
+    if (*b && ksh_buffer_size(*b) >= bytes) return 0;
+    if (*b) {
+        if (ksh_synchronize(ctx)) return 1;
+        for (size_t i = 0; i < owned.size(); i++)
+            if (owned[i] == *b) { owned.erase(owned.begin() + (long)i); break; }
+        ksh_buffer_release(*b);
+        *b = nullptr;
+    }
+    const size_t step = (size_t)16 << 20;
+    return alloc_together(ctx, owned, {{(bytes + step - 1) / step * step, b}});
+}
+
 inline bool sched_is_zero(const ksh_sched &s)
 {
     return s.tg == 0 && s.vec == 0 && s.unroll == 0 && s.nsg == 0 && s.nr0 == 0 && s.k_split == 0 &&

@@ -114,6 +114,15 @@ int64_t mock_sample_candidates(const float *logits, size_t n, float cap, float t
     return ksh::sample_from_candidates(cand.data(), cand.size(), sum, n, cap, temperature, min_p, seed, &id) ? (int64_t)id : -1;
 }
 
+// a buffer grown to each of the sizes in turn; the bytes it then has
+uint64_t mock_grow(uint64_t bytes)
+{
+    static std::vector<ksh_buf *> owned;
+    static ksh_buf *b = nullptr;
+    const int rc = ksh::grow_buffer(nullptr, owned, bytes, &b);
+    return rc || !b || owned.size() != 1 || owned[0] != b ? 0 : b->bytes;
+}
+
 // three buffers needed together, allocated where they are not there yet; how many of the pointers are set
 int mock_together(ksh_buf **three, int *set)
 {
@@ -147,6 +156,7 @@ void ksh_buffer_release(ksh_buf *b)
         delete b;
     }
 }
+size_t ksh_buffer_size(const ksh_buf *b) { return b->bytes; }
 int ksh_synchronize(ksh_ctx *) { return 0; }
 int ksh_buffer_fill_zero(ksh_ctx *, ksh_buf *b)
 {

@@ -49,3 +49,14 @@ def test_buffers_needed_together_are_there_together_or_not_at_all(fail_after):
     lib.mock_fail_alloc(fail_after)
     assert lib.mock_together(three, C.byref(n)) == 1 and n.value == 0 and lib.mock_allocated() == before
     assert lib.mock_together(three, C.byref(n)) == 0 and n.value == 3 and lib.mock_allocated() == before + 3
+
+
+def test_a_buffer_grows_in_steps_and_survives_a_failure():
+    lib = C.CDLL(host_mock.build())
+    lib.mock_grow.restype, lib.mock_grow.argtypes = C.c_uint64, [C.c_uint64]
+    step, before = 16 << 20, lib.mock_allocated()
+    assert [lib.mock_grow(n) for n in (1, step, 5, step + 1, 2 * step)] == [step, step, step, 2 * step, 2 * step]
+    assert lib.mock_allocated() == before + 1
+    lib.mock_fail_alloc(0)
+    assert lib.mock_grow(5 * step) == 0 and lib.mock_allocated() == before
+    assert lib.mock_grow(7) == step and lib.mock_allocated() == before + 1
