@@ -68,7 +68,8 @@ struct LaneParams {
     int groups;   // q heads this workgroup handles: (n_q / n_kv) / hsplit
     int hsplit;   // workgroups that share a kv head's rows, each with its own q heads
     int balance;  // the launch's nwg * n_slots partitions are dealt to the slots by length (kModeMerge, several slots)
-    int rope_row; // fused: `rope` is the current position's row of the table, not the table; otherwise: q is a half buffer
+    int rope_row; // fused: `rope` is the current position's row of the table, not the table
+    int q_half;   // not fused: q is a half buffer
     int kv_shared; // every slot attends the same cache (a chunk of prompt tokens, one meta record and one q per token)
     int no_append; // fused: the step's K / V row is in the cache already (a layer that reuses another layer's cache): q is normed and
                    // roped as usual, nothing is appended, every attended row comes from the cache
@@ -84,7 +85,7 @@ __device__ __forceinline__ void touch_lane_params(const LaneParams &p)
     asm volatile("" ::"s"(p.q), "s"(p.k), "s"(p.v), "s"(p.meta), "s"(p.slot_ids), "s"(p.slot_stride), "s"(p.tmp), "s"(p.out), "s"(p.counters));
     asm volatile("" ::"s"(p.qw), "s"(p.kw), "s"(p.rope), "s"(p.k_raw), "s"(p.v_raw), "s"(p.k_w), "s"(p.v_w));
     asm volatile("" ::"s"(p.eps), "s"(p.scale), "s"(p.n_q), "s"(p.n_kv), "s"(p.max_t), "s"(p.nwg), "s"(p.meta_stride), "s"(p.mode), "s"(p.fused),
-                 "s"(p.groups), "s"(p.hsplit), "s"(p.balance), "s"(p.rope_row), "s"(p.kv_shared), "s"(p.no_append));
+                 "s"(p.groups), "s"(p.hsplit), "s"(p.balance), "s"(p.rope_row), "s"(p.q_half), "s"(p.kv_shared), "s"(p.no_append));
 }
 
 __device__ __forceinline__ uint32_t ld32_a2(const uint8_t *p)
@@ -724,8 +725,8 @@ __global__ __launch_bounds__(NW * 64) void sdpa_lanes_kernel(LaneParams p_in)
         for (int h = 0; h < GP; h++) {
             const float *qh = qg + (size_t)min(h, groups - 1) * HD + 32 * b + 4 * w;
             const size_t i4 = (((size_t)slot * p.n_q + head0 + min(h, groups - 1)) * HD + 32 * b + 4 * w) / 4;
-            const float4 a = p.rope_row ? act_ld4<true>(p.q, i4) : *reinterpret_cast<const float4 *>(qh);
-            const float4 d = p.rope_row ? act_ld4<true>(p.q, i4 + 4) : *reinterpret_cast<const float4 *>(qh + 16);
+            const float4 a = p.q_half ? act_ld4<true>(p.q, i4) : *reinterpret_cast<const float4 *>(qh);
+            const float4 d = p.q_half ? act_ld4<true>(p.q, i4 + 4) : *reinterpret_cast<const float4 *>(qh + 16);
             const float sc = h < groups ? p.scale : 0.f;
             qv[h][0] = a.x * sc; qv[h][1] = a.y * sc; qv[h][2] = a.z * sc; qv[h][3] = a.w * sc;
             qv[h][4] = d.x * sc; qv[h][5] = d.y * sc; qv[h][6] = d.z * sc; qv[h][7] = d.w * sc;
@@ -1700,7 +1701,7 @@ int launch_bound(const ksh_kernel &k, const LaunchArgs &a, hipStream_t st)
         p.tmp = (float *)a.out[0];
         p.scale = k.desc.params[0];
         p.mode = kModePart;
-        p.rope_row = H;
+        p.q_half = H;
         break;
     case KSH_SDPA_SLOTS:
         n_slots = (int)k.desc.dims[4];
