@@ -81,8 +81,10 @@ __global__ __launch_bounds__(kNormThreads) void rmsnorm_kernel(const float *x, c
     }
 }
 
-// The same on half rows of a multiple of 4: four elements a load (with two-byte loads a row of 2048 was sixteen requests a
-// thread and as many address and range checks: one row 6.5 us in a trace, 2.7 so).  The sums of squares are added four by four.
+// The same on half rows of a multiple of 4 up to 2048: four elements a load (with two-byte loads a row of 2048 was sixteen
+// requests a thread and as many address and range checks: one row 6.5 us in a trace, 2.7 so).  Longer rows keep the two-byte
+// loads: no instance of more than two loads a thread is built.  The sums of squares are added four by four, which is not the
+// order of the f32 kernel's.
 template <int PER4>
 __global__ __launch_bounds__(kNormThreads) void rmsnorm_half4_kernel(const float *x, const float *__restrict__ w, const float *res, float *y, int n, float eps,
                                                                      int has_res, int has_scale, float scale)

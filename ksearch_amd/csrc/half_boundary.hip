@@ -12,8 +12,10 @@
 // that one launch.  Otherwise one launch widens all half inputs into f32
 // staging that belongs to the handle, the f32 kernel runs on the staging, one launch narrows the results
 // (round to nearest even, what the reference's kernels do when they store a half).  Arithmetic is therefore the
-// f32 path's, bit for bit, on the widened inputs.  The decode loops inside the library keep f32 activations and do
-// not pay the two conversion launches.
+// f32 path's on the widened inputs, bit for bit, with one exception: RMSNorm over half rows of a multiple of four
+// elements up to 2048 adds the squares four by four, the f32 kernel by stride, so that its f32 results may differ in
+// the last bits and now and then round to the neighbouring half.  (Bindings of either form need two bytes of alignment.)
+// The decode loops inside the library keep f32 activations and do not pay the two conversion launches.
 #include "ksh_device.hpp"
 #include "ksh_internal.hpp"
 
