@@ -1959,8 +1959,10 @@ int bind_matvec_round(ksh_kernel &k)
     return 0;
 }
 
-// schedules of the prefill GEMM: the 128 x 128 tile with K depth 64 (LDS-staged, one K range per workgroup) and, for
-// Q4_K weights and up to 64 tokens, 32 weight rows per workgroup with the K range split over its 8 waves
+// schedules of the prefill GEMM beside the library's own, which a search times first: the 128 x 128 tile with K depth 64
+// (LDS-staged, one K range per workgroup) and, for Q4_K weights and up to 64 tokens, 32 weight rows per workgroup with the
+// K range split over its 8 waves.  (bf16 rows: the token tile follows from the slice count, and counts that do not divide a
+// row come from the library's own schedule only.)
 int mul_mm_candidates(const ksh_kernel_desc &d, ksh_sched *out, int cap)
 {
     int n = 0;

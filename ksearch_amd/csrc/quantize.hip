@@ -67,8 +67,9 @@ __device__ __forceinline__ void grid_codes(const float (&x)[32], float iscale, f
 // gguf_impl.rs:811-901 with nmax=15, rmin=-1, rdelta=0.1, nstep=20, squared error.  One thread runs one 32-element
 // sub-block with every array in registers (the loops over the elements are unrolled; the sums run in the host
 // routine's order, element after element, so every rounding is the host's).
-// Bound: the vector ALU -- 22 passes over the elements, 11 instructions an element for a candidate's codes and sums and 6
-// for its error (24 with integer codes packed and unpacked between the two: 200 us for 16.8M weights, 130 so).
+// Bound: the vector ALU -- 22 passes over the elements, 10 instructions an element for a candidate's codes and sums and 6
+// for its error (24 with integer codes packed and unpacked between the two: 200 us for 16.8M weights, 130 so; the last of
+// the 11 that the codes and sums once took, a second addition in the rounding, went without a measurable difference).
 // The codes of the chosen candidate are not kept: *code_iscale and *code_min name the grid that makes them again (*flat: all 0).
 __device__ __forceinline__ float make_qkx2_quants(const float (&x)[32], const float (&weights)[32], float *the_min, float *code_iscale, float *code_min, bool *flat)
 {

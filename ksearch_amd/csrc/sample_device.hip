@@ -11,7 +11,7 @@
 //           only the count
 // Bound: launch latency (a row is one megabyte at the real vocabulary).  Sixteen requests served with sampling, prompts
 // of about 150 tokens and ten tokens of answer each: 552 ms with the whole rows read back and walked on the host, 146 ms
-// with the candidates.
+// with the candidates (72 since their prompts share a pass).
 #include "ksh_device.hpp"
 #include "ksh_internal.hpp"
 
