@@ -1927,7 +1927,9 @@ int bind_sdpa_lanes(ksh_kernel &k, int nwg, int n_slots)
     if (!k.desc.sched.nsg && k.desc.kind == KSH_SDPA_MWG_PART && (hd == 256 || hd == 512)) nw = parts_waves((int64_t)nwg * n_kv * hsplit, d[3] / nwg, wg_groups, hd);
     // heads of 512, one per workgroup, merging: eight waves at every partition length (16 row groups of 32 lanes)
     if (!k.desc.sched.nsg && k.desc.kind == KSH_ATTEND_DECODE && k.desc.dims[5] == 0 && wg_groups == 1 && hd == 512) nw = 8;
-    const size_t lds = lanes_lds(hd, wg_groups, nw, k.desc.kind == KSH_ATTEND_DECODE && lanes_few_heads(1, k.desc.dims[5] ? kModeSplitPart : kModeMerge, wg_groups, hd));
+    const bool few_heads = k.desc.kind == KSH_ATTEND_DECODE ? lanes_few_heads(1, k.desc.dims[5] ? kModeSplitPart : kModeMerge, wg_groups, hd)
+                                                            : k.desc.kind == KSH_SDPA_MWG_PART && lanes_few_heads(0, kModePart, wg_groups, hd);
+    const size_t lds = lanes_lds(hd, wg_groups, nw, few_heads);
     const bool merges = k.desc.kind == KSH_SDPA_SLOTS || k.desc.kind == KSH_SDPA_BATCH || (k.desc.kind == KSH_ATTEND_DECODE && !k.desc.dims[5]);
     if (merges && !(k.desc.kind == KSH_SDPA_SLOTS && balanced_slots(n_slots, nwg)) &&   // (those merge in a launch of their own)
         (size_t)wg_groups * (nwg + 16) * 3 * 4 > (size_t)nw * (64 / (hd / 8)) * ((wg_groups <= 4 ? 4 : 8) * hd) * 4)

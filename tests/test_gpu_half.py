@@ -339,6 +339,8 @@ def test_split_kv_partials_by_launch_size(ctx, n_q, n_kv, hd, max_t, nwg, half):
         k = ctx.compile(hip.make_desc(Kind.SDPA_MWG_PART, (n_q, n_kv, hd, max_t, nwg), (DType.Q40, DType.F16 if half else DType.F32), (scale,), sched))
         if sched is None and n_q // n_kv in (4, 8) and nwg * n_q > 512:   # a launch that fills the chip: heads share K and V
             assert n_q // n_kv // k.info.sched.unroll >= 4
+        if sched and hd == 256:      # the instance of one head and four waves: q, eight row groups' values and pairs, tables
+            assert k.info.lds_bytes == (256 + 8 * (256 + 4) + 8 + 2) * 4 + 2 * 8 * 18 + 16
         ctx.encode_multi(k, [bq, bk, bv, bm], [tmp])
         ctx.encode_multi(red, [tmp], [o])
         ctx.synchronize()
