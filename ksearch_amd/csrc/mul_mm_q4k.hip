@@ -324,10 +324,13 @@ __global__ __launch_bounds__(1024) void mm_prep_rows_kernel(const float *__restr
                 const float sum = pinned(sums[part]);
                 const _Float16 hi = (_Float16)sum;
                 const _Float16 lo = (_Float16)(sum - (float)hi);
-                dst[part][jj] = hi;
-                dst[part][8 + jj] = hi;
-                dst[part][16 + jj] = lo;
-                dst[part][24 + jj] = (_Float16)0.f;
+                // (the tile's: fragments of 32 tokens too, hi | hi and lo | 0)
+                _Float16 *a2 = inv_s ? SxA_hi + (((size_t)(t >> 5) * (cols / 256) + sbk / 8) * 128 + (t & 31)) * 8 : dst[part];
+                const int h1 = inv_s ? 256 : 8, k1 = inv_s ? 512 : 16;
+                a2[jj] = hi;
+                a2[h1 + jj] = hi;
+                a2[k1 + jj] = lo;
+                a2[k1 + h1 + jj] = (_Float16)0.f;
             }
         }
     };
@@ -379,10 +382,8 @@ struct MmParams {
     const float *cut_as;
 };
 
-// F32 activations: tokens per workgroup of the tile.  64 for Q4_K: two workgroups share a compute unit, and with two products
-// per converted weight the second conversion costs less than one workgroup's barriers, first loads and stores cost the
-// matrix pipe when it is alone there (prompts of 700 / 3000 tokens through the two synthetic models 11.7 / 53.7 ms with
-// 128-token tiles for the launches that fill the chip with them, 11.3 / 50.6 so).
+// F32 activations: the tokens and weight rows (BN) of the tiles that the rule of the K slices counts.  How a row's sum is cut
+// decides its bits, so the rule stays when the tiles that do the work change (q4k_mm_rows_kernel's are others).
 __host__ __device__ constexpr int mm_tile_tokens(bool q6) { return q6 ? 128 : 64; }
 
 // F32 activations, few tiles (a prompt of a few hundred tokens, or a narrow matrix): the nsb superblocks of a row are split
@@ -495,12 +496,11 @@ constexpr size_t kLdsBytes64 = 2 * (size_t)(kLdsMain + (64 + BN) * PITCH2) * 2 +
 // ROWS = true (bf16 activations, Q6_K weights: no sums of x are wanted): the A operands come from the rows of X as they are
 // and the multiplying waves convert them, eight values of a row a lane, between their matrix instructions -- no
 // preparation launch (mm_rows_direct; 333 tokens, 1536 x 6144 in six slices: 28.9 -> 25.4 us).
-// PAIR = true (f32 activations, a gate and an up matrix of one size): a tile is 64 rows of each, in turns of 32, so that a wave
-// has a gate row's sums beside its up row's and stores gelu(gate) * up -- half the results, and the down projection's
-// preparation reads them as they are instead of two matrices (2048 tokens, 12288 x 1536: 394 + 82 us -> 380 + 54).
-template <bool Q6, int TM, bool LO, bool CUT = false, bool ROWS = false, bool PAIR = false>
+// (F32 rows of Q4_K take q4k_mm_rows_kernel.)
+template <bool Q6, int TM, bool LO, bool CUT = false, bool ROWS = false>
 __global__ __launch_bounds__(kThreadsMM, TM == 64 ? 2 : 1) void q_mul_mm_kernel(MmParams p)
 {
+    static_assert(Q6 || !LO, "");
     constexpr int MT = TM / 64, kLdsMinT = (TM + BN) * PITCH2;
     extern __shared__ __attribute__((aligned(16))) _Float16 lds[];
     auto main_stage = [&](int i) { return lds + (i & 1) * kLdsMain; };
@@ -512,12 +512,12 @@ __global__ __launch_bounds__(kThreadsMM, TM == 64 ? 2 : 1) void q_mul_mm_kernel(
     int by = blockIdx.y, ycol = 0;
     const int rows_all = p.rows + p.rows1 + p.rows2;
     const int rows_of[3] = {p.rows, p.rows1, p.rows2};
-    if (!PAIR && p.rows1) {
+    if (p.rows1) {
         const int ty0 = (p.rows + BN - 1) / BN, ty1 = (p.rows1 + BN - 1) / BN;
         if (by >= ty0 + ty1) { by -= ty0 + ty1; ycol = p.rows + p.rows1; p.W = p.W2; p.Y = p.Y2; p.rows = p.rows2; }
         else if (by >= ty0) { by -= ty0; ycol = p.rows; p.W = p.W1; p.Y = p.Y1; p.rows = p.rows1; }
     }
-    const int t0 = blockIdx.x * TM, r0 = PAIR ? by * (BN / 2) : by * BN;
+    const int t0 = blockIdx.x * TM, r0 = by * BN;
     const int nsb_row = p.cols / 256;                            // superblocks per weight row
     int nsb = nsb_row, sb0 = 0;                                  // this workgroup's share of them
     size_t ystride = (size_t)p.rows;
@@ -617,8 +617,7 @@ __global__ __launch_bounds__(kThreadsMM, TM == 64 ? 2 : 1) void q_mul_mm_kernel(
         // ------------------------------------------------------------------ loaders
         const int lt = tid - 256, lrow = lt >> 1, lh = lt & 1;   // two threads per tile row
         const size_t row_bytes = (size_t)nsb_row * 144;
-        const uint8_t *wrow = PAIR ? ((lrow & 32) ? p.W1 : p.W) + (size_t)min(r0 + (lrow >> 6) * 32 + (lrow & 31), p.rows - 1) * row_bytes
-                                   : p.W + (size_t)min(r0 + lrow, p.rows - 1) * row_bytes + (size_t)sb0 * 144;
+        const uint8_t *wrow = p.W + (size_t)min(r0 + lrow, p.rows - 1) * row_bytes + (size_t)sb0 * 144;
         const size_t sx_off = ((size_t)min(t0 + lrow, p.batch - 1) * nsb_row + sb0) * 32;
         const _Float16 *sxrow = p.SxA + sx_off;
 
@@ -901,20 +900,6 @@ __global__ __launch_bounds__(kThreadsMM, TM == 64 ? 2 : 1) void q_mul_mm_kernel(
     }
 
     if (CUT) return;   // (the last slices' ends have stored everything)
-    if (PAIR) {
-#pragma unroll
-        for (int nt = 0; nt < NW_; nt += 2) {
-            const int r = r0 + (wn + nt / 2) * 32 + lm;
-#pragma unroll
-            for (int i = 0; i < 16; i++) {
-                const int t = t0 + wm * 32 + 8 * (i / 4) + 4 * (lane >> 5) + (i & 3);
-                const float inv = p.inv_s[min(t, p.batch - 1)];
-                const float y = gelu_mul_f32(pinned(F[0][nt][i] * inv), pinned(F[0][nt + 1][i] * inv));
-                if (t < p.batch && r < p.rows) p.Y[(size_t)t * p.rows + r] = y;
-            }
-        }
-        return;
-    }
     // accumulator layout of the 32x32 tile: column = lane % 32, row = 8*(i/4) + 4*(lane/32) + i%4
 #pragma unroll
     for (int mt = 0; mt < MW; mt++)
@@ -928,6 +913,14 @@ __global__ __launch_bounds__(kThreadsMM, TM == 64 ? 2 : 1) void q_mul_mm_kernel(
             }
         }
 }
+
+}  // namespace
+}  // namespace ksh
+
+#include "q4k_mm_rows.hpp"
+
+namespace ksh {
+namespace {
 
 // ---- small batches (up to 64 tokens): a GEMV-shaped launch on the matrix cores ---------------------------------
 // A prompt remainder or a round of decoding slots is a few dozen tokens: the 128 x 128 tile then leaves most of the
@@ -1624,6 +1617,34 @@ constexpr int kSkinnyMaxBatch = 64;
 // k.variant: 1 the small-batch form; else 2 * the K slices where their sums are folded (0: one slice), and this bit where
 // the tile reads bf16 rows as they are
 constexpr int kRowsDirect = 1 << 24;
+// ... and this one where f32 rows of Q4_K take the tall shape of q4k_mm_rows_kernel
+constexpr int kTall = 1 << 25;
+using MmRowsTall = MmRows<2, 2, 1, 4>;      // 64 tokens x 256 rows
+using MmRowsShort = MmRows<1, 2, 1, 4>;     // 32 tokens x 256 rows
+
+// Workgroups of a launch of `tm` tokens and MmRowsTall::TN rows (gate | up: of half as many of each) a workgroup
+dim3 mm_rows_grid(const ksh_kernel_desc &d, int tm, bool pair, int64_t ks)
+{
+    constexpr int TN = MmRowsTall::TN;
+    static_assert(TN == MmRowsShort::TN, "");
+    const int64_t y = pair ? (d.dims[0] + TN / 2 - 1) / (TN / 2) : (d.dims[0] + TN - 1) / TN + (d.dims[3] + TN - 1) / TN + (d.dims[4] + TN - 1) / TN;
+    return dim3((unsigned)((d.dims[2] + tm - 1) / tm), (unsigned)y, (unsigned)ks);
+}
+
+// Tall or short: us a superblock takes the busiest compute unit, fitted to 256 .. 24576 rows of 256 .. 12288 columns and 63 ..
+// 2048 tokens.  A tall workgroup alone on its compute unit 3.1, two of them 6.5 (the chip is then at its power limit, and more
+// take turns); a short one alone 2.45, each further one 2.2.  Either side at its line: 1536 x 12288, 952 tokens (90 tall
+// workgroups or 180 short ones) 158 us or 145, 2048 tokens (192 or 384) 216 or 247; gate | up of 12288 x 1536, 140 tokens (288
+// or 480) 51 or 41.
+bool mm_rows_tall(const ksh_kernel_desc &d, bool pair, int64_t ks)
+{
+    auto turns = [&](int tm) {
+        const dim3 g = mm_rows_grid(d, tm, pair, ks);
+        return (float)(((int64_t)g.x * g.y * g.z + 255) / 256);
+    };
+    const float tall = turns(MmRowsTall::TM), small = turns(MmRowsShort::TM);
+    return (tall == 1.f ? 3.1f : 3.25f * tall) < (small == 1.f ? 2.45f : 2.2f * small);
+}
 
 int mm_row_tiles(const ksh_kernel_desc &d) { return (int)((d.dims[0] + BN - 1) / BN + (d.dims[3] + BN - 1) / BN + (d.dims[4] + BN - 1) / BN); }
 
@@ -1631,7 +1652,7 @@ int launch_mul_mm(const ksh_kernel &k, const LaunchArgs &a, hipStream_t st)
 {
     const int rows = (int)k.desc.dims[0], cols = (int)k.desc.dims[1], batch = (int)k.desc.dims[2];
     const bool f32x = k.desc.dtypes[1] == KSH_F32;
-    const size_t xf_halves = (size_t)((batch + 31) / 32 * 32) * cols, sx_halves = (size_t)batch * (cols / 256) * 32;
+    const size_t xf_halves = (size_t)((batch + 31) / 32 * 32) * cols, sx_halves = (size_t)(f32x ? (batch + 31) / 32 * 32 : batch) * (cols / 256) * 32;
     _Float16 *Xf = (_Float16 *)k.scratch;
     _Float16 *SxA = Xf + xf_halves;
     _Float16 *Xf_lo = SxA + sx_halves, *SxA_lo = Xf_lo + xf_halves;     // f32 activations only
@@ -1646,7 +1667,7 @@ int launch_mul_mm(const ksh_kernel &k, const LaunchArgs &a, hipStream_t st)
     const int octets = cols / 8, pb1 = (octets + 63) / 64 * 64;
     const dim3 pg((unsigned)batch), pb((unsigned)std::min(pb1 > 1024 && inv_s ? (octets / 2 + 63) / 64 * 64 : pb1, 1024));
     const bool rows_direct = (k.variant & kRowsDirect) != 0;
-    const int slices = (k.variant & ~kRowsDirect) >> 1;                  // 0: no fold
+    const int slices = (k.variant & ~(kRowsDirect | kTall)) >> 1;                  // 0: no fold
     if (prologue) {
         // the rows' producer runs inside the preparation: in = W, X, [W1, W2,] then the prologue's operands
         const int xs = (int)k.desc.dims[7];
@@ -1688,12 +1709,22 @@ int launch_mul_mm(const ksh_kernel &k, const LaunchArgs &a, hipStream_t st)
     }
     const bool cut = k.desc.dims[6] == 2;
     const int tm = k.info.lds_bytes == kLdsBytes64 ? 64 : 128;
-    const dim3 grid((batch + tm - 1) / tm, pair ? (rows + BN / 2 - 1) / (BN / 2) : (rows + BN - 1) / BN + (rows1 + BN - 1) / BN + (rows2 + BN - 1) / BN);
+    const dim3 grid((batch + tm - 1) / tm, (rows + BN - 1) / BN + (rows1 + BN - 1) / BN + (rows2 + BN - 1) / BN);   // (q_mul_mm_kernel's)
     p.Xf = rows_direct ? (const _Float16 *)a.in[1] : Xf;
     p.SxA = SxA; p.Xf_lo = Xf_lo; p.inv_s = inv_s;
     p.ksplit = 0; p.Y_parts = nullptr;
     p.cut_as = cut ? (const float *)a.in[k.info.n_inputs - 1] : nullptr;
     const bool q6 = k.desc.dtypes[0] == KSH_Q6K;
+    auto launch_rows = [&](dim3 g) {
+#define KSH_ROWS(S, ...) hipLaunchKernelGGL((q4k_mm_rows_kernel<S, __VA_ARGS__>), g, dim3(S::kThreads), S::kLds, st, p)
+        if (cut) KSH_ROWS(MmRowsShort, true, false);
+        else if (k.variant & kTall) {
+            if (pair) KSH_ROWS(MmRowsTall, false, true);
+            else KSH_ROWS(MmRowsTall, false, false);
+        } else if (pair) KSH_ROWS(MmRowsShort, false, true);
+        else KSH_ROWS(MmRowsShort, false, false);
+#undef KSH_ROWS
+    };
     auto launch_tile = [&](dim3 g) {
 #define KSH_TILE(LDS, ...) hipLaunchKernelGGL((q_mul_mm_kernel<__VA_ARGS__>), g, dim3(kThreadsMM), LDS, st, p)
         if (q6) {
@@ -1702,9 +1733,7 @@ int launch_mul_mm(const ksh_kernel &k, const LaunchArgs &a, hipStream_t st)
             else if (rows_direct) KSH_TILE(kLdsBytes, true, 128, false, false, true);
             else KSH_TILE(kLdsBytes, true, 128, false);
         } else if (f32x) {
-            if (pair) KSH_TILE(kLdsBytes64, false, 64, true, false, false, true);
-            else if (cut) KSH_TILE(kLdsBytes64, false, 64, true, true);
-            else KSH_TILE(kLdsBytes64, false, 64, true);
+            launch_rows(dim3(k.info.grid[0], k.info.grid[1], g.z));
         } else if (tm == 64) KSH_TILE(kLdsBytes64, false, 64, false);
         else KSH_TILE(kLdsBytes, false, 128, false);
 #undef KSH_TILE
@@ -1811,7 +1840,8 @@ int bind_matvec_batch(ksh_kernel &k)
         k.in_bytes[ni] = (size_t)batch * 4; k.in_align[ni] = 4;
     }
     // f16 copy of X plus the min-term operand (32 halves per token and superblock)
-    k.scratch_bytes = ((size_t)((batch + 31) / 32 * 32) * cols * 2 + (size_t)batch * (cols / 256) * 64) * (f32x ? 2 : 1);
+    const size_t batch32 = (size_t)((batch + 31) / 32 * 32);
+    k.scratch_bytes = (batch32 * cols * 2 + (f32x ? batch32 : (size_t)batch) * (cols / 256) * 64) * (f32x ? 2 : 1);
     // schedule: nr0 = weight rows per workgroup.  32 = the small-batch form (Q4_K, up to 64 tokens: the default
     // there), 128 = the 128 x 128 tile.
     const uint32_t want = k.desc.sched.nr0;
@@ -1858,11 +1888,21 @@ int bind_matvec_batch(ksh_kernel &k)
         k.out_bytes[0] = (size_t)ks * batch * rows_all * 4; k.out_align[0] = 16;
         k.info.n_outputs = 1 + keep;
     }
-    set_launch(k, (uint32_t)((batch + tm - 1) / tm), pair ? (uint32_t)((rows + BN / 2 - 1) / (BN / 2)) : (uint32_t)row_tiles, z_form ? (uint32_t)ks : 1, kThreadsMM,
-               (uint32_t)(tm == 64 ? kLdsBytes64 : kLdsBytes));
-    k.info.sched.tg = kThreadsMM; k.info.sched.nsg = kThreadsMM / 64; k.info.sched.nr0 = BN; k.info.sched.k_split = (uint32_t)ks; k.info.sched.lds_tile = KS;
-    set_name(k, "mul_mm_%s_%dx%dx%d%s%s%s%s", q6 ? "q6k" : "q4k", BM, BN, KS, f32x ? "_f32x" : "", z_form ? "_kz" : "", n_mat == 3 ? "_x3" : n_mat == 2 ? "_x2" : "",
-             prologue == 1 ? "_rms" : prologue == 2 ? "_addrms" : prologue == 3 ? "_gelu" : "");
+    if (f32x && !q6) {
+        const bool tall = !cut && mm_rows_tall(k.desc, pair, z_form ? ks : 1);
+        if (tall) k.variant |= kTall;
+        const int tmr = tall ? MmRowsTall::TM : MmRowsShort::TM;
+        const dim3 g = mm_rows_grid(k.desc, tmr, pair, z_form ? ks : 1);
+        set_launch(k, g.x, g.y, g.z, MmRowsTall::kThreads, (uint32_t)(tall ? MmRowsTall::kLds : MmRowsShort::kLds));
+        k.info.sched.tg = MmRowsTall::kThreads; k.info.sched.nsg = MmRowsTall::kThreads / 64; k.info.sched.nr0 = BN; k.info.sched.k_split = (uint32_t)ks; k.info.sched.lds_tile = 32;
+        set_name(k, "mul_mm_q4k_%dx%dx32_f32x%s%s%s", tmr, MmRowsTall::TN, z_form ? "_kz" : "", n_mat == 3 ? "_x3" : n_mat == 2 ? "_x2" : "",
+                 prologue == 1 ? "_rms" : prologue == 2 ? "_addrms" : prologue == 3 ? "_gelu" : "");
+    } else {
+        set_launch(k, (uint32_t)((batch + tm - 1) / tm), (uint32_t)row_tiles, z_form ? (uint32_t)ks : 1, kThreadsMM, (uint32_t)(tm == 64 ? kLdsBytes64 : kLdsBytes));
+        k.info.sched.tg = kThreadsMM; k.info.sched.nsg = kThreadsMM / 64; k.info.sched.nr0 = BN; k.info.sched.k_split = (uint32_t)ks; k.info.sched.lds_tile = KS;
+        set_name(k, "mul_mm_%s_%dx%dx%d%s%s%s%s", q6 ? "q6k" : "q4k", BM, BN, KS, f32x ? "_f32x" : "", z_form ? "_kz" : "", n_mat == 3 ? "_x3" : n_mat == 2 ? "_x2" : "",
+                 prologue == 1 ? "_rms" : prologue == 2 ? "_addrms" : prologue == 3 ? "_gelu" : "");
+    }
     if (pair) { char nm[64]; snprintf(nm, sizeof(nm), "%s", k.info.name); set_name(k, "%s_gate_up", nm); }
     if (cut) { char nm[64]; snprintf(nm, sizeof(nm), "%s", k.info.name); set_name(k, "%s_cut", nm); }
     if (unfolded) { char nm[64]; snprintf(nm, sizeof(nm), "%s", k.info.name); set_name(k, "%s_unfolded", nm); }

@@ -1,0 +1,427 @@
+// The prompt GEMM over Q4_K weights and f32 rows (two f16 parts at the row's own scale, mm_prep_rows_kernel): every wave
+// converts its own weights in registers and multiplies them with fragments that the workgroup shares in LDS.
+//
+// What bounds it: the matrix pipe and the chip's power.  With two workgroups on every compute unit the pipe is busy 60 % of the
+// cycles, at 1.7 - 1.8 GHz; a launch of nothing but its matrix instructions holds 1.6 GHz.  In its place was a tile of four waves
+// that loaded and converted, handing weights to four that multiplied through LDS, and of fragments from memory to registers:
+// at 32 x 64 a wave the fragments alone keep the path from L1 busy for as long as the matrix instructions take, and the roles
+// waited for each other at every step (pipe busy 44 %).  Here a wave has 64 tokens x 64 rows (or 32 x 64), a converted weight
+// meets four fragments, a fragment comes from memory once a workgroup, and nobody waits for a converted weight.  With its
+// preparation (64 x 64 a wave): 2048 tokens, gate | up of 12288 x 1536 380 -> 298 us, 1536 x 12288 252 -> 208, 4096 x 1536
+// 82 -> 60; 952 tokens, 1536 x 12288 (32 x 64) 152 -> 146; rows cut as in launches of their own, 1989 tokens, 1536 x 12288
+// 285 -> 245.
+//
+// The sums are those of that tile (q_mul_mm_kernel's, which other types still take), instruction by instruction, so results have
+// its bits: per 16 columns the hi and the lo part against the same weights into a superblock's own accumulator, then F = (bias
+// and mins, two short products) + F and F = d * C + F.
+//
+// CUT: the rows belong to prompts that would each have had a launch of their own, whose K slices depend on its length; the
+// workgroup takes all of K, and where a row's slice ends its sum goes to a second accumulator and starts again from zero (the
+// bits of those launches; through memory, as the tile has it, a slice end was a round trip of the results).
+// PAIR: a gate and an up matrix of one size: a wave has a gate tile beside its up tile and stores gelu(gate) * up.
+#pragma once
+#include "ksh_device.hpp"
+#include "ksh_internal.hpp"
+
+namespace ksh {
+namespace {
+
+// Shape of a launch's workgroups: WM x WN = 4 waves, each MT x NT tiles of 32 tokens x 32 weight rows.
+template <int MT_, int NT_, int WM_, int WN_>
+struct MmRows {
+    static constexpr int MT = MT_, NT = NT_, WM = WM_, WN = WN_;
+    static constexpr int TT = WM * MT, TM = 32 * TT, TN = 32 * WN * NT, kThreads = 64 * WM * WN;
+    static constexpr int kStage = TT * 4 * 1024;      // bytes of the fragments of 32 columns: [token tile][hi | lo][k slice][lane][16]
+    static constexpr int kSums = TT * 2 * 1024;       // bytes of a superblock's sums of x: [token tile][k slice][lane][16]
+    static constexpr int kTile = 5 * 1024;            // bytes of a superblock of 32 weight rows: [row][144], whole kilobytes
+    static constexpr int kInv = 256;                  // the tokens' 1 / s
+    static constexpr int kLds = 4 * kStage + kSums + WM * WN * NT * kTile + kInv;
+    static_assert(WM * WN == 4 && TT <= 2 && MT <= 2 && NT == 2, "a wave fetches TT fragments of a half step, from one part of one token tile");
+};
+
+// Memory operations that the compiler does not count: it would wait for all that is on its way into LDS in front of every read
+// of LDS.  Read values are used behind lds_wait and arrived only; what comes into LDS is waited for by the number of younger
+// operations, so every one of them is issued whatever the sizes (addresses are clamped instead).
+__device__ __forceinline__ void to_lds16(const uint8_t *base, uint32_t off, uint32_t dst)
+{
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(dst), "v"(off), "s"(base) : "memory");
+}
+__device__ __forceinline__ void to_lds4(const uint8_t *base, uint32_t off, uint32_t dst)
+{
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dword %1, %2" ::"s"(dst), "v"(off), "s"(base) : "memory");
+}
+template <int OFF, class V>
+__device__ __forceinline__ void lds_ask(V &v, uint32_t addr)
+{
+    asm volatile("ds_read_b128 %0, %1 offset:%2" : "=v"(v) : "v"(addr), "n"(OFF));
+}
+__device__ __forceinline__ void lds_wait() { asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory"); }
+template <class V>
+__device__ __forceinline__ void arrived(V &v)
+{
+    asm volatile("" : "+v"(v));
+}
+
+template <class S, bool CUT, bool PAIR>
+__global__ __launch_bounds__(S::kThreads, 2) void q4k_mm_rows_kernel(MmParams p)
+{
+    constexpr int MT = S::MT, NT = S::NT, TT = S::TT;
+    extern __shared__ __attribute__((aligned(16))) uint8_t lds_rows[];
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int wm = wave / S::WN, wn = wave % S::WN, lm = lane & 31, h = lane >> 5;
+
+    // which matrix this row tile belongs to (the copy of the arguments is this workgroup's own)
+    int by = blockIdx.y, ycol = 0;
+    const int rows_all = p.rows + p.rows1 + p.rows2;
+    const int rows_of[3] = {p.rows, p.rows1, p.rows2};
+    if (!PAIR && p.rows1) {
+        const int ty0 = (p.rows + S::TN - 1) / S::TN, ty1 = (p.rows1 + S::TN - 1) / S::TN;
+        if (by >= ty0 + ty1) { by -= ty0 + ty1; ycol = p.rows + p.rows1; p.W = p.W2; p.Y = p.Y2; p.rows = p.rows2; }
+        else if (by >= ty0) { by -= ty0; ycol = p.rows; p.W = p.W1; p.Y = p.Y1; p.rows = p.rows1; }
+    }
+    const int t0 = blockIdx.x * S::TM, r0 = by * (PAIR ? S::TN / 2 : S::TN);
+    const int nsb_row = p.cols / 256;
+    int nsb = nsb_row, sb0 = 0;
+    size_t ystride = (size_t)p.rows;
+    if (p.ksplit) {
+        const int slice = blockIdx.z;
+        sb0 = nsb_row * slice / p.ksplit;
+        nsb = nsb_row * (slice + 1) / p.ksplit - sb0;
+        p.Y = p.Y_parts + (size_t)slice * p.batch * rows_all + ycol;   // partial sums: all matrices' columns side by side
+        ystride = (size_t)rows_all;
+    }
+
+    // ---- everything the loop reads comes straight from memory into LDS: of the 4 TT kilobytes of a half step this wave asks for
+    // TT; the sums of a superblock; and its own weight rows, a row's 144 bytes in nine lanes.  (Asked for in the order the
+    // matrix instruction wants them, a row a lane, weights are 64 pieces of 16 bytes to an instruction: 2048 tokens, 12288 x
+    // 1536, gate | up 312 us instead of 294.)
+    const uint32_t l0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) uint8_t *)lds_rows;
+    constexpr uint32_t kAtSums = 4 * S::kStage, kAtW = kAtSums + S::kSums, kAtInv = kAtW + 4 * NT * S::kTile;
+    const int f0 = wave * TT, ntt = (p.batch + 31) / 32, fsum = wave % (2 * TT);
+    const uint8_t *xsrc = reinterpret_cast<const uint8_t *>((f0 >> 1) & 1 ? p.Xf_lo : p.Xf) +
+                          ((size_t)min(t0 / 32 + (f0 >> 2), ntt - 1) * nsb_row + sb0) * 16384 + (f0 & 1) * 1024;
+    const uint8_t *sxsrc = reinterpret_cast<const uint8_t *>(p.SxA) + (((size_t)min(t0 / 32 + (fsum >> 1), ntt - 1) * nsb_row + sb0) * 2 + (fsum & 1)) * 1024;
+    const uint32_t lane16 = 16u * (uint32_t)lane, lw = l0 + kAtW + (uint32_t)(wave * NT * S::kTile);
+    auto ask_rows = [&](int hs, int stage, int i) __attribute__((always_inline)) {
+        to_lds16(xsrc + (size_t)min(hs, 8 * nsb - 1) * 2048 + i * 1024, lane16, l0 + (uint32_t)(stage * S::kStage + (f0 + i) * 1024));
+    };
+    auto ask_sums = [&](int sb) __attribute__((always_inline)) { to_lds16(sxsrc + (size_t)min(sb, nsb - 1) * 2048, lane16, l0 + kAtSums + (uint32_t)(fsum * 1024)); };
+    const size_t row_bytes = (size_t)nsb_row * 144;
+    const uint8_t *wbase[2];
+    wbase[0] = p.W + (size_t)r0 * row_bytes + (size_t)sb0 * 144;
+    wbase[1] = PAIR ? p.W1 + (size_t)r0 * row_bytes : wbase[0];
+    uint32_t woff[NT][5];                             // piece 64 i + lane of a tile's rows (past the tile: its last row again)
+#pragma unroll
+    for (int nt = 0; nt < NT; nt++)
+#pragma unroll
+        for (int i = 0; i < 5; i++) {
+            const int c = 64 * i + lane, row = min(c / 9, 31), r = PAIR ? wn * 32 + row : (wn * NT + nt) * 32 + row;
+            woff[nt][i] = (uint32_t)min(r, p.rows - 1 - r0) * (uint32_t)row_bytes + 16u * (uint32_t)(c % 9);
+        }
+    auto ask_weights = [&](int sb, int j) __attribute__((always_inline)) {
+        to_lds16(wbase[j / 5] + (size_t)min(sb, nsb - 1) * 144, woff[j / 5][j % 5], lw + (uint32_t)(j / 5 * S::kTile + j % 5 * 1024));
+    };
+
+    f16v F[MT][NT], C[MT][NT];
+    const f16v kZero16 = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int mt = 0; mt < MT; mt++)
+#pragma unroll
+        for (int nt = 0; nt < NT; nt++) F[mt][nt] = C[mt][nt] = kZero16;
+    // lane (lm, h) has row lm of each of its tiles: the header and bytes 16 h .. 16 h + 15 of every group's 32
+    u32x4_t q[4][NT], hdr[NT];
+    uint32_t scA[NT], scB[NT], s_lo[NT], s_hi[NT];   // the eight scales of a superblock; the two of the group being converted
+    float dn[NT];
+#pragma unroll
+    for (int nt = 0; nt < NT; nt++) dn[nt] = 0.f;
+    h8 b[2][NT];                                      // converted weights of a k slice, and of the next
+    h8 a[2][2];                                       // a unit's fragments, and the next one's
+    u32x4_t b2[NT];
+    h8 s2[2];
+
+    auto scales = [&]() __attribute__((always_inline)) {   // of the superblock whose header has arrived
+#pragma unroll
+        for (int nt = 0; nt < NT; nt++) {
+            scA[nt] = hdr[nt].y & 0x3F3F3F3Fu;
+            scB[nt] = (hdr[nt].w & 0x0F0F0F0Fu) | ((hdr[nt].y & 0xC0C0C0C0u) >> 2);
+        }
+    };
+    auto open_group = [&](auto gtag, int nt) __attribute__((always_inline)) {
+        constexpr int g = decltype(gtag)::value;
+        const uint32_t s = (g < 2 ? scA : scB)[nt];
+        s_lo[nt] = (s >> (16 * (g & 1))) & 0xFFu;
+        s_hi[nt] = (s >> (16 * (g & 1) + 8)) & 0xFFu;
+        // bytes 8h .. 8h+7 and 16+8h .. 16+8h+7 of the group, which is what the matrix instruction wants of lane (lm, h)
+        const auto x = __builtin_amdgcn_permlane32_swap(q[g][nt].x, q[g][nt].z, false, false);
+        const auto y = __builtin_amdgcn_permlane32_swap(q[g][nt].y, q[g][nt].w, false, false);
+        q[g][nt] = u32x4_t{x[0], y[0], x[1], y[1]};
+    };
+    auto convert = [&](auto gtag, auto ktag, int nt) __attribute__((always_inline)) {
+        constexpr int g = decltype(gtag)::value, ks = decltype(ktag)::value;
+        const uint32_t w0 = q[g][nt][2 * (ks & 1)], w1 = q[g][nt][2 * (ks & 1) + 1], sc = ks < 2 ? s_lo[nt] : s_hi[nt];
+        constexpr int sh = ks < 2 ? 0 : 4;
+        const u32x4_t o = {pair_f16((w0 >> sh) & 0x000F000Fu, sc), pair_f16((w0 >> (8 + sh)) & 0x000F000Fu, sc), pair_f16((w1 >> sh) & 0x000F000Fu, sc),
+                           pair_f16((w1 >> (8 + sh)) & 0x000F000Fu, sc)};
+        b[ks & 1][nt] = __builtin_bit_cast(h8, o);
+    };
+    // the row's eight coefficients -(dmin*m_j + 1024*d) as f16: hi[8] in lanes h = 0, lo[8] in lanes h = 1; two of this lane's
+    // four at a time
+    auto min_operand = [&](int nt, int i) __attribute__((always_inline)) {
+        const float d = half_bits_to_f32(hdr[nt].x & 0xFFFFu), dmin = half_bits_to_f32(hdr[nt].x >> 16);
+        if (i == 0) dn[nt] = d;
+        const uint32_t mA = hdr[nt].z & 0x3F3F3F3Fu, mB = ((hdr[nt].w >> 4) & 0x0F0F0F0Fu) | ((hdr[nt].z & 0xC0C0C0C0u) >> 2);
+        const uint32_t m = h ? mB : mA;
+        const float c0 = pinned(-(dmin * (i ? ubyte_f32<2>(m) : ubyte_f32<0>(m)) + 1024.f * d)), c1 = pinned(-(dmin * (i ? ubyte_f32<3>(m) : ubyte_f32<1>(m)) + 1024.f * d));
+        const _Float16 h0 = (_Float16)c0, h1 = (_Float16)c1;
+        const _Float16 l0_ = (_Float16)(c0 - (float)h0), l1_ = (_Float16)(c1 - (float)h1);
+        const auto x = __builtin_amdgcn_permlane32_swap((uint32_t)__builtin_bit_cast(uint16_t, h0) | ((uint32_t)__builtin_bit_cast(uint16_t, h1) << 16),
+                                                        (uint32_t)__builtin_bit_cast(uint16_t, l0_) | ((uint32_t)__builtin_bit_cast(uint16_t, l1_) << 16), false, false);
+        b2[nt][i] = x[0];
+        b2[nt][2 + i] = x[1];
+    };
+    auto fold = [&](int mt, int nt) __attribute__((always_inline)) {
+#pragma unroll
+        for (int i = 0; i < 16; i++) F[mt][nt][i] = fmaf(dn[nt], C[mt][nt][i], F[mt][nt][i]);
+    };
+
+    // CUT: lane t % 32 keeps the superblocks per slice of the tile's row t and what is left of the current one; finished slices
+    // add up in T
+    static_assert(!CUT || MT == 1, "one token tile to a wave leaves registers for T");
+    f16v T[NT];
+    int cut_len = nsb, cut_left = nsb;
+    if (CUT) {
+        const int row_tiles = (rows_of[0] + BN - 1) / BN + (rows_of[1] + BN - 1) / BN + (rows_of[2] + BN - 1) / BN;
+        cut_len = cut_left = nsb / mm_k_slices(false, row_tiles, nsb, (int)p.cut_as[min(t0 + wm * 32 + lm, p.batch - 1)]);
+#pragma unroll
+        for (int nt = 0; nt < NT; nt++) T[nt] = kZero16;
+    }
+    auto cut_ends = [&]() __attribute__((always_inline)) {   // behind a superblock's fold
+        cut_left -= 1;
+        uint32_t ends = (uint32_t)__ballot(cut_left == 0);
+        if (cut_left == 0) cut_left = cut_len;
+        if (!ends) return;
+        ends >>= 4 * h;
+#pragma unroll
+        for (int nt = 0; nt < NT; nt++)
+#pragma unroll
+            for (int i = 0; i < 16; i++)
+                if (ends & (1u << (8 * (i / 4) + (i & 3)))) {
+                    T[nt][i] += F[0][nt][i];
+                    F[0][nt][i] = 0.f;
+                }
+    };
+
+    // A unit of the loop is four matrix instructions for one set of fragments: one part of a k slice for two token tiles (the
+    // parts in turn), or both parts of it for one.  U units to a half step.
+    constexpr int U = 2 * MT;
+    const uint32_t la = l0 + (uint32_t)(wm * MT) * 4096u + lane16;   // + stage, token tile, part, k slice
+    const uint32_t lsum = l0 + kAtSums + (uint32_t)(wm * MT) * 2048u + lane16;
+    const uint32_t lh = lw + 144u * (uint32_t)lm, lq = lh + 16u * (uint32_t)h;
+    auto read_rows = [&](auto htag, auto utag, h8 (&v)[2]) __attribute__((always_inline)) {   // of unit U of a half step
+        constexpr int hs = decltype(htag)::value & 3, u = decltype(utag)::value;
+        constexpr int off = hs * S::kStage + (MT == 2 ? (u >> 1) * 1024 + (u & 1) * 2048 : u * 1024);
+        lds_ask<off>(v[0], la);
+        lds_ask<off + (MT == 2 ? 4096 : 2048)>(v[1], la);
+    };
+    auto read_group = [&](auto gtag) __attribute__((always_inline)) {
+        constexpr int o = 16 + 32 * decltype(gtag)::value;
+        lds_ask<o>(q[decltype(gtag)::value][0], lq);
+        lds_ask<o + S::kTile>(q[decltype(gtag)::value][1], lq);
+    };
+    auto read_header = [&]() __attribute__((always_inline)) {
+        lds_ask<0>(hdr[0], lh);
+        lds_ask<S::kTile>(hdr[1], lh);
+    };
+    auto settle = [&](auto &v) __attribute__((always_inline)) {
+        arrived(v[0]);
+        arrived(v[1]);
+    };
+    constexpr std::integral_constant<int, 0> n0{};
+    constexpr std::integral_constant<int, 1> n1{};
+    constexpr std::integral_constant<int, 2> n2{};
+    constexpr std::integral_constant<int, 3> n3{};
+
+    // ---- in front of the loop: the first superblock's weights, three half steps of fragments; the first slice converted
+    to_lds4(reinterpret_cast<const uint8_t *>(p.inv_s), 4u * (uint32_t)min(t0 + lane, p.batch - 1), l0 + kAtInv);   // (every wave the same)
+#pragma unroll
+    for (int j = 0; j < 5 * NT; j++) ask_weights(0, j);
+    ask_sums(0);
+#pragma unroll
+    for (int hs = 0; hs < 3; hs++)
+#pragma unroll
+        for (int i = 0; i < TT; i++) ask_rows(hs, hs, i);
+    asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" ::"n"(2 * TT) : "memory");
+    read_group(n0);
+    read_group(n1);
+    read_group(n2);
+    read_group(n3);
+    read_header();
+    read_rows(n0, n0, a[0]);
+    lds_wait();
+    settle(q[0]); settle(q[1]); settle(q[2]); settle(q[3]); settle(hdr); settle(a[0]);
+    scales();
+#pragma unroll
+    for (int nt = 0; nt < NT; nt++) {
+        open_group(n0, nt);
+        convert(n0, n0, nt);
+    }
+
+    // Unit `place` of half step `half` of a superblock.  Under its matrix instructions the next unit's fragments come from LDS
+    // and the next slice's weights are converted, spread evenly (the compiler's own order issues most matrix instructions back
+    // to back and leaves their pipe idle under the rest).
+    auto unit = [&](int sb, auto htag, auto utag) __attribute__((always_inline)) {
+        constexpr int half = decltype(htag)::value, place = decltype(utag)::value;
+        constexpr int g = half >> 1, ks = 2 * (half & 1) + place / MT, part = MT == 2 ? place & 1 : 0, set = place & 1;
+        constexpr int gn = ks == 3 ? (g + 1) & 3 : g, kn = (ks + 1) & 3;               // the next slice
+        constexpr bool last = place == U - 1;
+        // Memory operations of a half step: its first units ask for the fragments of three half steps on; the last two (the
+        // last, MT = 1) of half steps 0 .. 4 for two pieces of the next superblock's weights, of half step 5 for its sums.
+        constexpr auto extra = [](int hh) { return hh < 5 ? 2 : hh == 5 ? 1 : 0; };
+        __builtin_amdgcn_sched_barrier(0);
+        constexpr bool opens = half == 0 && place == 0;
+        if constexpr (opens && CUT) {
+            if (sb > 0) {
+#pragma unroll
+                for (int mt = 0; mt < MT; mt++)
+#pragma unroll
+                    for (int nt = 0; nt < NT; nt++) fold(mt, nt);
+                cut_ends();
+            }
+        }
+        constexpr int mins = MT == 2 ? (g == 1 && part == 0 && ks < 2 ? ks : -1) : (g == 1 && ks == 1 ? 0 : -1);
+        constexpr bool take0 = half == 7 && place == 0, take3 = half == 7 && last;
+        // (behind the first matrix instruction, whose 32 cycles cover part of it: a request to memory takes some 40 to issue)
+        auto ask = [&]() __attribute__((always_inline)) {
+            if constexpr (last) {
+                // every wave has this half step's fragments in registers; the next one's, which this wave has asked for two half
+                // steps ago, are in LDS (and at the end of half step 6 the weights, which are 1 + 2 TT operations back)
+                constexpr int pending = half == 6 ? 1 + 2 * TT : extra((half + 6) & 7) + TT + extra((half + 7) & 7) + TT + (MT == 2 && extra(half) > 0 ? 1 : 0);
+                asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" ::"n"(pending) : "memory");
+            }
+            read_rows(std::integral_constant<int, (last ? half + 1 : half) & 7>{}, std::integral_constant<int, last ? 0 : place + 1>{}, a[set ^ 1]);
+            // the short second product's: the sums of x of a token tile
+            if constexpr (mins >= 0) {
+                lds_ask<mins * 2048>(s2[0], lsum);
+                lds_ask<mins * 2048 + 1024>(s2[1], lsum);
+            }
+            // the next superblock's weights, into the registers whose group has been converted
+            if constexpr (take0) { read_group(n0); read_header(); }
+            if constexpr (take3) { read_group(n1); read_group(n2); read_group(n3); }
+            if constexpr (MT == 2) {
+                if constexpr (place < TT) ask_rows(8 * sb + half + 3, (half + 3) & 3, place);
+                if constexpr (place >= 2 && half < 5) ask_weights(sb + 1, 2 * half + place - 2);
+            } else if constexpr (place == 0) {
+#pragma unroll
+                for (int i = 0; i < TT; i++) ask_rows(8 * sb + half + 3, (half + 3) & 3, i);
+            } else if constexpr (half < 5) {
+                ask_weights(sb + 1, 2 * half);
+                ask_weights(sb + 1, 2 * half + 1);
+            }
+            if constexpr (place == U / 2 && half == 5) ask_sums(sb + 1);
+        };
+#pragma unroll
+        for (int i = 0; i < 2; i++)
+#pragma unroll
+            for (int nt = 0; nt < NT; nt++) {
+                const int mt = MT == 2 ? i : 0;
+                const bool first = opens && (MT == 2 || i == 0);   // (a superblock's first product starts from the constant zero)
+                if (first && !CUT) fold(mt, nt);
+                C[mt][nt] = __builtin_amdgcn_mfma_f32_32x32x16_f16(a[set][i], b[ks & 1][nt], first ? kZero16 : C[mt][nt], 0, 0, 0);
+                if (i == 0 && nt == 0) {
+                    __builtin_amdgcn_sched_barrier(0);
+                    ask();
+                    __builtin_amdgcn_sched_barrier(0);
+                }
+            }
+        std::integral_constant<int, gn> gnext{};
+        std::integral_constant<int, kn> knext{};
+        std::integral_constant<int, (g + 1) & 3> gopen{};
+        // (groups are opened a unit ahead of their first conversion, MT = 1: in front of it; the short product's operand in the
+        // quiet units of the first steps)
+        constexpr bool op0 = MT == 2 ? ks == 2 && part == 1 : ks == 3, op1 = MT == 2 ? ks == 3 && part == 0 : ks == 3, sc = op0 && g == 3;
+        constexpr int mu = (half * U + place) - (MT == 2 ? 1 : 0), mn = MT == 2 ? (mu >= 0 && mu < 4 ? mu : -1) : (mu < 3 ? mu : mu == 4 ? 3 : -1);
+        if constexpr (sc) scales();
+        if constexpr (MT == 1) {
+            if constexpr (op0) { open_group(gopen, 0); open_group(gopen, 1); }
+            convert(gnext, knext, 0);
+            convert(gnext, knext, 1);
+        } else {
+            convert(gnext, knext, part);
+            if constexpr (op0) open_group(gopen, 0);
+            if constexpr (op1) open_group(gopen, 1);
+        }
+        if constexpr (mn >= 0) min_operand(mn >> 1, mn & 1);
+        constexpr int valu = (MT == 2 ? 11 : 22) + (op0 ? 8 : 0) + (op1 ? 8 : 0) + (sc ? 10 : 0) + (mn >= 0 ? 22 : 0);
+        if constexpr (!opens) {
+#pragma unroll
+            for (int i = 0; i < 3; i++) {
+                __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+                __builtin_amdgcn_sched_group_barrier(0x002, (valu + 2) / 3, 0);
+            }
+        }
+        __builtin_amdgcn_sched_barrier(0);
+        lds_wait();
+        settle(a[set ^ 1]);
+        if constexpr (take0) { settle(q[0]); settle(hdr); }
+        if constexpr (take3) { settle(q[1]); settle(q[2]); settle(q[3]); }
+        if constexpr (mins >= 0) {
+            settle(s2);
+#pragma unroll
+            for (int nt = 0; nt < NT; nt++) F[mins][nt] = __builtin_amdgcn_mfma_f32_32x32x16_f16(s2[0], __builtin_bit_cast(h8, b2[nt]), F[mins][nt], 0, 0, 0);
+#pragma unroll
+            for (int nt = 0; nt < NT; nt++) {
+                const u32x4_t o = {h ? 0u : b2[nt].x, h ? 0u : b2[nt].y, h ? 0u : b2[nt].z, h ? 0u : b2[nt].w};
+                F[mins][nt] = __builtin_amdgcn_mfma_f32_32x32x16_f16(s2[1], __builtin_bit_cast(h8, o), F[mins][nt], 0, 0, 0);
+            }
+        }
+    };
+    for (int sb = 0; sb < nsb; sb++) {
+#define KSH_HALF(H)                                                 \
+    do {                                                            \
+        constexpr std::integral_constant<int, H> hh{};              \
+        unit(sb, hh, n0);                                           \
+        unit(sb, hh, n1);                                           \
+        if constexpr (U == 4) { unit(sb, hh, n2); unit(sb, hh, n3); } \
+    } while (0)
+        KSH_HALF(0); KSH_HALF(1); KSH_HALF(2); KSH_HALF(3); KSH_HALF(4); KSH_HALF(5); KSH_HALF(6); KSH_HALF(7);
+#undef KSH_HALF
+    }
+    // (what is still on its way into LDS arrives before the workgroup gives it back)
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+#pragma unroll
+    for (int mt = 0; mt < MT; mt++)
+#pragma unroll
+        for (int nt = 0; nt < NT; nt++) fold(mt, nt);
+    if (CUT) {
+        cut_ends();
+#pragma unroll
+        for (int nt = 0; nt < NT; nt++) F[0][nt] = T[nt];
+    }
+    // accumulator layout of the 32x32 tile: column = lane % 32, row = 8*(i/4) + 4*(lane/32) + i%4
+#pragma unroll
+    for (int mt = 0; mt < MT; mt++) {
+        const int tb = t0 + (wm * MT + mt) * 32 + 4 * h, left = p.batch - tb;
+        f32x4_t inv[4];
+#pragma unroll
+        for (int i4 = 0; i4 < 4; i4++) asm volatile("ds_read_b128 %0, %1" : "=v"(inv[i4]) : "v"(l0 + kAtInv + 4u * (uint32_t)(tb - t0 + 8 * i4)));
+        lds_wait();
+#pragma unroll
+        for (int i4 = 0; i4 < 4; i4++) arrived(inv[i4]);
+#pragma unroll
+        for (int nt = 0; nt < NT; nt += PAIR ? 2 : 1) {
+            const int r = r0 + (PAIR ? wn : wn * NT + nt) * 32 + lm;
+            if (r >= p.rows) continue;
+            float *y = p.Y + (size_t)tb * ystride + r;
+#pragma unroll
+            for (int i = 0; i < 16; i++) {
+                const int t = 8 * (i / 4) + (i & 3);
+                float v = F[mt][nt][i] * inv[i / 4][i & 3];
+                if (PAIR) v = gelu_mul_f32(pinned(v), pinned(F[mt][1][i] * inv[i / 4][i & 3]));
+                if (t < left) y[(size_t)t * ystride] = v;
+            }
+        }
+    }
+}
+
+}  // namespace
+}  // namespace ksh

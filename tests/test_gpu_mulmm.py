@@ -325,6 +325,50 @@ def test_mul_mm_f32_both_parts_in_one_workgroup(ctx, unfolded, k_split):
     assert not got[7].any()
 
 
+@pytest.mark.parametrize("rows,batch,cols,mode,shape", [
+    (1, 65, 256, 0, "32x256"), (257, 33, 768, 0, "32x256"), (255, 96, 7936, 0, "32x256"), (300, 129, 1024, 2, "32x256"),
+    (129, 65, 512, 3, "32x256"), (4097, 1000, 256, 0, "64x256"), (7937, 545, 512, 3, "64x256")])
+def test_mul_mm_f32_rows_at_the_edges_of_its_tiles(ctx, rows, batch, cols, mode, shape):
+    """Both shapes of the f32 rows' kernel where they can go wrong: one superblock and thirty-one, a row or a token past a
+    tile or short of it, two matrices side by side (gelu(gate) * up), rows summed as in launches of their own.  Against
+    float64 at the bar of the others (two f16 parts hold 22 bits of a row's largest, f32 sums: 2e-5); rows cut as in
+    launches of their own against those launches, bit for bit."""
+    ws = [ctx.buffer_bytes(synth.q4k_blocks(rows * cols // 256, 700 + i)) for i in range(2)]
+    xs = synth.normal_f32(batch * cols, 702).reshape(batch, cols)
+    x = ctx.buffer_f32(xs)
+
+    def launch(dims, ins, sched=None):
+        k = ctx.compile(hip.make_desc(hip.Kind.MATVEC_BATCH, dims, (DType.Q4K, DType.F32, DType.F32), (), sched))
+        y = ctx.buffer_empty_f32(dims[2] * rows)
+        ctx.encode_multi(k, ins, [y])
+        ctx.synchronize()
+        return k, ctx.read_f32(y, dims[2] * rows).reshape(dims[2], rows)
+
+    if mode == 2:
+        lens = [70, batch - 70] if batch - 70 <= 64 else [batch]     # (a prompt of up to 64 rows is summed as one of 65)
+        as_ = np.concatenate([np.full(n, max(n, 65), np.float32) for n in lens])
+        k, got = launch((rows, cols, batch, 0, 0, 0, 2), [ws[0], x, ctx.buffer_f32(as_)])
+        for n, at in zip(lens, np.cumsum([0] + lens[:-1])):
+            pad = np.zeros((max(n, 65), cols), np.float32)
+            pad[:n] = xs[at:at + n]
+            _, want = launch((rows, cols, len(pad)), [ws[0], ctx.buffer_f32(pad)], dict(nr0=128))
+            assert np.array_equal(got[at:at + n], want[:n]), (n, at)
+    else:
+        dims = (rows, cols, batch, rows, 0, 0, 3) if mode == 3 else (rows, cols, batch)
+        k, got = launch(dims, [ws[0], x, ws[1]] if mode == 3 else [ws[0], x], dict(k_split=1, nr0=128 if mode == 0 else 0))
+        for t in sorted({0, 31, 32, batch // 2, batch - 1}):
+            want = [oracle.matvec_f64(oracle.Q4K, synth.q4k_blocks(rows * cols // 256, 700 + i), rows, cols, xs[t]) for i in range(2)]
+            if mode == 3:
+                g = np.clip(want[0], -20.0, 20.0)     # (the kernels' gelu: tanh of a cubic, its argument held to +-20)
+                want = 0.5 * g * (1.0 + np.tanh(0.7978845608 * (g + 0.044715 * g ** 3))) * want[1]
+                # (either factor off by 2e-5 of its rms or value, the other up to four times its rms, gelu' <= 1.13, against a
+                # product of at least 0.6 of the two rms: 2 * 4 * 1.13 / 0.6 * 2e-5)
+                assert rel_err(got[t], want).max() <= 3e-4, t
+            else:
+                assert rel_err(got[t], want[0]).max() <= 2e-5, t
+    assert shape in k.name, k.name
+
+
 @pytest.mark.parametrize("rows,batch,prologue", [(31, 33, 0), (97, 64, 2), (200, 130, 0), (4130, 1000, 2)])
 def test_mul_mm_f32_gate_up_pair(ctx, rows, batch, prologue):
     """dims[6] = 3: gelu(W x) * (W1 x) from one launch is the two matrices' products and KSH_GELU_MUL (64 rows of each
