@@ -131,6 +131,17 @@ __device__ __forceinline__ void act_st(float *p, size_t i, float v)
     else ((KSH_GLOBAL _Float16 *)p)[i] = half_rn(v);
 }
 
+// 16 (or 4) bytes a lane straight from memory into LDS: lane l's at dst + 16 l (4 l).  The compiler does not count these (it
+// answers them with a wait for all in front of every read of LDS): whoever asks waits by the number of younger operations.
+__device__ __forceinline__ void to_lds16(const uint8_t *base, uint32_t off, uint32_t dst)
+{
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(dst), "v"(off), "s"(base) : "memory");
+}
+__device__ __forceinline__ void to_lds4(const uint8_t *base, uint32_t off, uint32_t dst)
+{
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dword %1, %2" ::"s"(dst), "v"(off), "s"(base) : "memory");
+}
+
 constexpr int kWave = 64;
 
 // A zero the compiler cannot see through, in a vector register.  Added to the index of a load whose address is the

@@ -42,14 +42,6 @@ struct MmRows {
 // Memory operations that the compiler does not count: it would wait for all that is on its way into LDS in front of every read
 // of LDS.  Read values are used behind lds_wait and arrived only; what comes into LDS is waited for by the number of younger
 // operations, so every one of them is issued whatever the sizes (addresses are clamped instead).
-__device__ __forceinline__ void to_lds16(const uint8_t *base, uint32_t off, uint32_t dst)
-{
-    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(dst), "v"(off), "s"(base) : "memory");
-}
-__device__ __forceinline__ void to_lds4(const uint8_t *base, uint32_t off, uint32_t dst)
-{
-    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dword %1, %2" ::"s"(dst), "v"(off), "s"(base) : "memory");
-}
 template <int OFF, class V>
 __device__ __forceinline__ void lds_ask(V &v, uint32_t addr)
 {

@@ -1538,6 +1538,14 @@ __global__ __launch_bounds__(kMfmaRound / TR * (HD / HDV) * 64, TR == 32 ? 2 : 1
     }
 }
 
+}  // namespace
+}  // namespace ksh
+
+#include "sdpa_prompt.hpp"
+
+namespace ksh {
+namespace {
+
 // Merge of split-KV partials kept as records (m, l, o[HD]) per (token, head, partition) -- the layout and the rule
 // of SdpaMwgReduce (crates/ksearch_codegen/src/lower.rs:5897-6087) -- for the launch that gives every token of a long
 // prompt chunk its own workgroups.  grid = (n_q, n_tok), HD threads.
@@ -1648,6 +1656,33 @@ LaneParams base_params(const ksh_kernel &k)
 // to derive the table itself.
 bool balanced_slots(int n_slots, int nwg) { return n_slots > 1 && n_slots <= 16 && nwg >= 2 && nwg <= 64; }
 
+// One partition per token, over rows that can be fetched 16 bytes at a time and reached by a 32-bit offset (sdpa_prompt_kernel;
+// the rest keeps sdpa_mfma_kernel)
+bool prompt_rows(int64_t n_kv, int64_t hd, int64_t max_t, int nwg)
+{
+    const int64_t row = n_kv * (hd / 32 * 18);
+    return nwg == 1 && max_t * row < ((int64_t)1 << 32) && row < (1 << 24);
+}
+bool prompt_rows_aligned(const LaneParams &p) { return (((uintptr_t)p.k | (uintptr_t)p.v | p.slot_stride) & 15) == 0; }
+
+// Two tokens to a workgroup, of one prompt and where half as many workgroups still fill the chip (two to a compute unit of
+// heads of 256, one of heads of 512): see the figures at sdpa_prompt_kernel; 1024 tokens of heads of 256 59 us with one token,
+// 61 with two, 699 40 and 46.
+bool prompt_pairs(int64_t n_kv, int64_t hd, int64_t n_tok, bool one_prompt)
+{
+    return one_prompt && n_tok * n_kv >= (hd == 512 ? 512 : 896);
+}
+
+template <int HD, int T>
+int launch_prompt(const LaneParams &p, int n_tok, hipStream_t st)
+{
+    using S = SdpaPrompt<HD, T>;
+    const unsigned z = T == 2 ? (unsigned)((n_tok + 63) / 64 * 64) : (unsigned)n_tok;
+    hipLaunchKernelGGL((sdpa_prompt_kernel<HD, T>), dim3(1, p.n_kv, z), dim3(S::WAVES * 64), S::kLds, st, p, n_tok);
+    const hipError_t e = hipGetLastError();
+    return e == hipSuccess ? 0 : hip_fail(e, "sdpa_batch (prompt) launch");
+}
+
 // variant: nwg | NW << 16 | hsplit << 24.  H: q is a half buffer (split-KV partials)
 template <bool H = false>
 int launch_bound(const ksh_kernel &k, const LaunchArgs &a, hipStream_t st)
@@ -1744,6 +1779,11 @@ int launch_bound(const ksh_kernel &k, const LaunchArgs &a, hipStream_t st)
             }
             p.balance = 0;
             p.mode = kModePart;
+            if (prompt_rows(p.n_kv, hd, p.max_t, p.nwg) && prompt_rows_aligned(p)) {
+                const bool two = prompt_pairs(p.n_kv, hd, n_slots, p.kv_shared != 0);
+                if (hd == 512) return two ? launch_prompt<512, 2>(p, n_slots, st) : launch_prompt<512, 1>(p, n_slots, st);
+                return two ? launch_prompt<256, 2>(p, n_slots, st) : launch_prompt<256, 1>(p, n_slots, st);
+            }
             if (hd == 512)   // two waves a tile, each with half of the V dimensions
                 hipLaunchKernelGGL((sdpa_mfma_kernel<512, 32, 256>), dim3(p.nwg, p.n_kv, n_slots), dim3(kMfmaRound / 32 * 2 * 64), (mfma_lds_bytes<512, 32, 256>()), st, p);
             else
@@ -1864,8 +1904,13 @@ int bind_sdpa_lanes(ksh_kernel &k, int nwg, int n_slots)
         k.scratch_bytes = (((size_t)n_slots * n_kv * 4 + 15) & ~(size_t)15) + (size_t)n_slots * 16;
         // (heads of 512: two waves a tile)
         const int waves = kMfmaRound / 32 * (hd == 512 ? 2 : 1);
-        set_launch(k, (uint32_t)nwg, (uint32_t)n_kv, (uint32_t)n_slots, waves * 64,
-                   (uint32_t)(hd == 512 ? mfma_lds_bytes<512, 32, 256>() : mfma_lds_bytes<256, 32>()));
+        if (prompt_rows(n_kv, hd, d[3], nwg)) {      // (what caches at 16-byte addresses take)
+            const bool two = prompt_pairs(n_kv, hd, n_slots, !k.desc.dims[6]);
+            const int lds = hd == 512 ? (two ? SdpaPrompt<512, 2>::kLds : SdpaPrompt<512, 1>::kLds) : (two ? SdpaPrompt<256, 2>::kLds : SdpaPrompt<256, 1>::kLds);
+            set_launch(k, 1, (uint32_t)n_kv, (uint32_t)(two ? (n_slots + 63) / 64 * 64 : n_slots), waves * 64, (uint32_t)lds);
+        } else
+            set_launch(k, (uint32_t)nwg, (uint32_t)n_kv, (uint32_t)n_slots, waves * 64,
+                       (uint32_t)(hd == 512 ? mfma_lds_bytes<512, 32, 256>() : mfma_lds_bytes<256, 32>()));
         k.info.sched = k.desc.sched;
         k.info.sched.vec = 2;
         k.info.sched.tg = waves * 64;

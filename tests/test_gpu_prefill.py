@@ -133,6 +133,38 @@ def test_sdpa_batch_equals_the_serial_oracle(ctx, hd, n_q, n_kv, sched, t, pos0,
     del row
 
 
+@pytest.mark.parametrize("hd,n_q,n_kv,t,pos0,window,slots", [
+    (256, 8, 1, 17, 0, 4096, 0), (256, 5, 1, 70, 29, 33, 0), (256, 16, 2, 129, 100, 64, 0), (512, 8, 1, 45, 31, 4096, 0), (512, 6, 2, 33, 0, 1, 0),
+    (256, 8, 1, 900, 0, 250, 0), (256, 6, 2, 451, 3, 4096, 0), (256, 7, 1, 961, 60, 31, 0), (512, 8, 1, 545, 5, 4096, 0), (512, 4, 2, 300, 90, 65, 0),
+    (256, 8, 1, 150, 0, 100, 3), (512, 8, 1, 200, 0, 4096, 3)])
+def test_prompt_attention_has_the_bits_of_the_form_of_several_partitions(ctx, hd, n_q, n_kv, t, pos0, window, slots):
+    """One and two tokens to a workgroup, at the edges of tiles, windows and chunks (a window of one row and of a tile and
+    one, a tile that ends for one of two tokens, a last token without a partner, tokens of several prompts): the same bits
+    as the kernel that takes caches at any address, which the same caches two bytes further on go to."""
+    max_t = 1100
+    scale, rows = 1.0 / np.sqrt(hd), max_t * n_kv * hd // 32
+    kv = [synth.q40_blocks(max(1, slots) * rows, 713 + i) for i in range(2)]
+    q = ctx.buffer_f32(synth.normal_f32(t * n_q * hd, 715))
+    k = ctx.compile(hip.make_desc(Kind.SDPA_BATCH, (n_q, n_kv, hd, max_t, t, 1, slots), (DType.Q40, DType.F32), (scale,)))
+    tmp = ctx.buffer_empty_f32(t * n_q * (hd + 2))
+    if slots:
+        n = np.arange(t) % (t // slots + 1) + 1                      # attended rows: prompts one after the other
+        l = np.minimum(n, window)
+        meta, ids = np.stack([l, n - l, l * 0, l * 0], 1).astype(np.float32), (np.arange(t) // (t // slots + 1)).astype(np.float32)
+        more = [ctx.buffer_f32(meta), ctx.buffer_f32(ids)]
+    else:
+        more = [ctx.buffer_f32(np.array([pos0 + 1, 0, window, 0], np.float32))]
+    got = []
+    for at in (0, 2):
+        bufs = [ctx.buffer_bytes(np.concatenate([np.zeros(at, np.uint8), np.frombuffer(bytes(x), np.uint8)])) for x in kv]
+        out = ctx.buffer_empty_f32(t * n_q * hd)
+        ctx.encode_offsets_multi(k, [q] + bufs + more, [0, at, at] + [0] * len(more), [tmp, out], None)
+        ctx.synchronize()
+        got.append(ctx.read_f32(out, t * n_q * hd).reshape(t, -1))
+    assert np.isfinite(got[1]).all() and np.abs(got[1]).max() > 0
+    assert np.array_equal(got[0], got[1]), np.flatnonzero((got[0] != got[1]).any(axis=1))[:8]
+
+
 @pytest.mark.parametrize("wdt,batch,sched", [(DType.Q4K, 45, None), (DType.Q6K, 45, None), (DType.Q4K, 5, None), (DType.Q4K, 32, None),
                                              (DType.Q4K, 64, None), (DType.Q4K, 45, dict(nr0=128)), (DType.Q4K, 100, None)])
 def test_mul_mm_f32_activations(ctx, wdt, batch, sched):
