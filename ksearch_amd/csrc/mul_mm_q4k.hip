@@ -1620,30 +1620,33 @@ constexpr int kRowsDirect = 1 << 24;
 // ... and this one where f32 rows of Q4_K take the tall shape of q4k_mm_rows_kernel
 constexpr int kTall = 1 << 25;
 using MmRowsTall = MmRows<2, 2, 1, 4>;      // 64 tokens x 256 rows
-using MmRowsShort = MmRows<1, 2, 1, 4>;     // 32 tokens x 256 rows
+using MmRowsShort = MmRows<1, 2, 1, 4>;     // 32 tokens x 256 rows: gate | up, and CUT
+using MmRowsSmall = MmRows<1, 1, 1, 4>;     // 32 tokens x 128 rows: the others
 
-// Workgroups of a launch of `tm` tokens and MmRowsTall::TN rows (gate | up: of half as many of each) a workgroup
-dim3 mm_rows_grid(const ksh_kernel_desc &d, int tm, bool pair, int64_t ks)
+// Workgroups of a launch of `tm` tokens and `tn` rows (gate | up: half as many of each) a workgroup
+dim3 mm_rows_grid(const ksh_kernel_desc &d, int tm, int tn, bool pair, int64_t ks)
 {
-    constexpr int TN = MmRowsTall::TN;
-    static_assert(TN == MmRowsShort::TN, "");
-    const int64_t y = pair ? (d.dims[0] + TN / 2 - 1) / (TN / 2) : (d.dims[0] + TN - 1) / TN + (d.dims[3] + TN - 1) / TN + (d.dims[4] + TN - 1) / TN;
+    const int64_t y = pair ? (d.dims[0] + tn / 2 - 1) / (tn / 2) : (d.dims[0] + tn - 1) / tn + (d.dims[3] + tn - 1) / tn + (d.dims[4] + tn - 1) / tn;
     return dim3((unsigned)((d.dims[2] + tm - 1) / tm), (unsigned)y, (unsigned)ks);
 }
 
-// Tall or short: us a superblock takes the busiest compute unit, fitted to 256 .. 24576 rows of 256 .. 12288 columns and 63 ..
+// Tall or not: us a superblock takes the busiest compute unit, fitted to 256 .. 24576 rows of 256 .. 12288 columns and 63 ..
 // 2048 tokens.  A tall workgroup alone on its compute unit 3.1, two of them 6.5 (the chip is then at its power limit, and more
-// take turns); a short one alone 2.45, each further one 2.2.  Either side at its line: 1536 x 12288, 952 tokens (90 tall
-// workgroups or 180 short ones) 158 us or 145, 2048 tokens (192 or 384) 216 or 247; gate | up of 12288 x 1536, 140 tokens (288
-// or 480) 51 or 41.
+// take turns); a short one alone 2.45, each further one 2.2; a small one alone 1.75, two or more 1.18 each.  Either side of its
+// line: 1536 x 12288, 952 tokens (90 tall workgroups or 360 small ones) 158 us or 134, 2048 tokens (192 or 768) 201 or 221;
+// 4096 x 1536, 2048 tokens (512 or 2048) 61 or 74; gate | up of 12288 x 1536, 140 tokens (288 tall or 480 short) 51 or 41.
+// (A wave of two row tiles alone on its SIMD leaves the matrix pipe idle for half of the time.  Small for short: 2048 x 8192,
+// 700 tokens 93 -> 87 us, 2048 x 2048, 63 tokens in four slices 12.8 -> 10.2, 1536 x 12288, 140 tokens 41.8 -> 35.7.  CUT stays
+// short: 1989 tokens, 1536 x 12288 240 or 243 us, 1536 x 6144 129 or 131, 1536 x 2048 52 or 49.)
 bool mm_rows_tall(const ksh_kernel_desc &d, bool pair, int64_t ks)
 {
-    auto turns = [&](int tm) {
-        const dim3 g = mm_rows_grid(d, tm, pair, ks);
+    auto turns = [&](int tm, int tn) {
+        const dim3 g = mm_rows_grid(d, tm, tn, pair, ks);
         return (float)(((int64_t)g.x * g.y * g.z + 255) / 256);
     };
-    const float tall = turns(MmRowsTall::TM), small = turns(MmRowsShort::TM);
-    return (tall == 1.f ? 3.1f : 3.25f * tall) < (small == 1.f ? 2.45f : 2.2f * small);
+    const float tall = turns(MmRowsTall::TM, MmRowsTall::TN);
+    const float other = pair ? turns(MmRowsShort::TM, MmRowsShort::TN) : turns(MmRowsSmall::TM, MmRowsSmall::TN);
+    return (tall == 1.f ? 3.1f : 3.25f * tall) < (pair ? (other == 1.f ? 2.45f : 2.2f * other) : (other == 1.f ? 1.75f : 1.18f * other));
 }
 
 int mm_row_tiles(const ksh_kernel_desc &d) { return (int)((d.dims[0] + BN - 1) / BN + (d.dims[3] + BN - 1) / BN + (d.dims[4] + BN - 1) / BN); }
@@ -1722,7 +1725,7 @@ int launch_mul_mm(const ksh_kernel &k, const LaunchArgs &a, hipStream_t st)
             if (pair) KSH_ROWS(MmRowsTall, false, true);
             else KSH_ROWS(MmRowsTall, false, false);
         } else if (pair) KSH_ROWS(MmRowsShort, false, true);
-        else KSH_ROWS(MmRowsShort, false, false);
+        else KSH_ROWS(MmRowsSmall, false, false);
 #undef KSH_ROWS
     };
     auto launch_tile = [&](dim3 g) {
@@ -1891,11 +1894,12 @@ int bind_matvec_batch(ksh_kernel &k)
     if (f32x && !q6) {
         const bool tall = !cut && mm_rows_tall(k.desc, pair, z_form ? ks : 1);
         if (tall) k.variant |= kTall;
-        const int tmr = tall ? MmRowsTall::TM : MmRowsShort::TM;
-        const dim3 g = mm_rows_grid(k.desc, tmr, pair, z_form ? ks : 1);
-        set_launch(k, g.x, g.y, g.z, MmRowsTall::kThreads, (uint32_t)(tall ? MmRowsTall::kLds : MmRowsShort::kLds));
+        const bool small = !tall && !pair && !cut;
+        const int tmr = tall ? MmRowsTall::TM : MmRowsShort::TM, tnr = small ? MmRowsSmall::TN : MmRowsTall::TN;
+        const dim3 g = mm_rows_grid(k.desc, tmr, tnr, pair, z_form ? ks : 1);
+        set_launch(k, g.x, g.y, g.z, MmRowsTall::kThreads, (uint32_t)(tall ? MmRowsTall::kLds : small ? MmRowsSmall::kLds : MmRowsShort::kLds));
         k.info.sched.tg = MmRowsTall::kThreads; k.info.sched.nsg = MmRowsTall::kThreads / 64; k.info.sched.nr0 = BN; k.info.sched.k_split = (uint32_t)ks; k.info.sched.lds_tile = 32;
-        set_name(k, "mul_mm_q4k_%dx%dx32_f32x%s%s%s", tmr, MmRowsTall::TN, z_form ? "_kz" : "", n_mat == 3 ? "_x3" : n_mat == 2 ? "_x2" : "",
+        set_name(k, "mul_mm_q4k_%dx%dx32_f32x%s%s%s", tmr, tnr, z_form ? "_kz" : "", n_mat == 3 ? "_x3" : n_mat == 2 ? "_x2" : "",
                  prologue == 1 ? "_rms" : prologue == 2 ? "_addrms" : prologue == 3 ? "_gelu" : "");
     } else {
         set_launch(k, (uint32_t)((batch + tm - 1) / tm), (uint32_t)row_tiles, z_form ? (uint32_t)ks : 1, kThreadsMM, (uint32_t)(tm == 64 ? kLdsBytes64 : kLdsBytes));

@@ -5,11 +5,11 @@
 // cycles, at 1.7 - 1.8 GHz; a launch of nothing but its matrix instructions holds 1.6 GHz.  In its place was a tile of four waves
 // that loaded and converted, handing weights to four that multiplied through LDS, and of fragments from memory to registers:
 // at 32 x 64 a wave the fragments alone keep the path from L1 busy for as long as the matrix instructions take, and the roles
-// waited for each other at every step (pipe busy 44 %).  Here a wave has 64 tokens x 64 rows (or 32 x 64), a converted weight
-// meets four fragments, a fragment comes from memory once a workgroup, and nobody waits for a converted weight.  With its
-// preparation (64 x 64 a wave): 2048 tokens, gate | up of 12288 x 1536 380 -> 298 us, 1536 x 12288 252 -> 208, 4096 x 1536
-// 82 -> 60; 952 tokens, 1536 x 12288 (32 x 64) 152 -> 146; rows cut as in launches of their own, 1989 tokens, 1536 x 12288
-// 285 -> 245.
+// waited for each other at every step (pipe busy 44 %).  Here a wave has 64 tokens x 64 rows (or 32 x 64, or 32 x 32), a
+// converted weight meets four fragments (or two), a fragment comes from memory once a workgroup, and nobody waits for a
+// converted weight.  With its preparation (64 x 64 a wave): 2048 tokens, gate | up of 12288 x 1536 380 -> 298 us, 1536 x 12288
+// 252 -> 208, 4096 x 1536 82 -> 60; (32 x 32) 952 tokens, 1536 x 12288 152 -> 134, 700 tokens, 2048 x 8192 99 -> 87; rows cut
+// as in launches of their own, 1989 tokens, 1536 x 12288 285 -> 245.
 //
 // The sums are those of that tile (q_mul_mm_kernel's, which other types still take), instruction by instruction, so results have
 // its bits: per 16 columns the hi and the lo part against the same weights into a superblock's own accumulator, then F = (bias
@@ -26,17 +26,20 @@
 namespace ksh {
 namespace {
 
-// Shape of a launch's workgroups: WM x WN = 4 waves, each MT x NT tiles of 32 tokens x 32 weight rows.
-template <int MT_, int NT_, int WM_, int WN_>
+// Shape of a launch's workgroups: WM x WN = 4 waves, each MT x NT tiles of 32 tokens x 32 weight rows; LO: rows of f32, in two
+// parts (else bf16, one part).
+template <int MT_, int NT_, int WM_, int WN_, bool LO_ = true>
 struct MmRows {
-    static constexpr int MT = MT_, NT = NT_, WM = WM_, WN = WN_;
+    static constexpr int MT = MT_, NT = NT_, WM = WM_, WN = WN_, PARTS = LO_ ? 2 : 1;
+    static constexpr bool LO = LO_;
     static constexpr int TT = WM * MT, TM = 32 * TT, TN = 32 * WN * NT, kThreads = 64 * WM * WN;
-    static constexpr int kStage = TT * 4 * 1024;      // bytes of the fragments of 32 columns: [token tile][hi | lo][k slice][lane][16]
+    static constexpr int TF = TT * PARTS / 2;         // fragments of a half step that a wave fetches
+    static constexpr int kStage = TT * 2 * PARTS * 1024;   // bytes of the fragments of 32 columns: [token tile][hi | lo][k slice][lane][16]
     static constexpr int kSums = TT * 2 * 1024;       // bytes of a superblock's sums of x: [token tile][k slice][lane][16]
     static constexpr int kTile = 5 * 1024;            // bytes of a superblock of 32 weight rows: [row][144], whole kilobytes
     static constexpr int kInv = 256;                  // the tokens' 1 / s
     static constexpr int kLds = 4 * kStage + kSums + WM * WN * NT * kTile + kInv;
-    static_assert(WM * WN == 4 && TT <= 2 && MT <= 2 && NT == 2, "a wave fetches TT fragments of a half step, from one part of one token tile");
+    static_assert(WM * WN == 4 && TT <= 2 && MT * PARTS >= 2 && NT <= 2, "a wave fetches TF fragments of a half step, from one part of one token tile");
 };
 
 // Memory operations that the compiler does not count: it would wait for all that is on its way into LDS in front of every read
@@ -57,7 +60,7 @@ __device__ __forceinline__ void arrived(V &v)
 template <class S, bool CUT, bool PAIR>
 __global__ __launch_bounds__(S::kThreads, 2) void q4k_mm_rows_kernel(MmParams p)
 {
-    constexpr int MT = S::MT, NT = S::NT, TT = S::TT;
+    constexpr int MT = S::MT, NT = S::NT, TT = S::TT, TF = S::TF, PARTS = S::PARTS;
     extern __shared__ __attribute__((aligned(16))) uint8_t lds_rows[];
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int wm = wave / S::WN, wn = wave % S::WN, lm = lane & 31, h = lane >> 5;
@@ -83,15 +86,15 @@ __global__ __launch_bounds__(S::kThreads, 2) void q4k_mm_rows_kernel(MmParams p)
         ystride = (size_t)rows_all;
     }
 
-    // ---- everything the loop reads comes straight from memory into LDS: of the 4 TT kilobytes of a half step this wave asks for
-    // TT; the sums of a superblock; and its own weight rows, a row's 144 bytes in nine lanes.  (Asked for in the order the
+    // ---- everything the loop reads comes straight from memory into LDS: of the 4 TF kilobytes of a half step this wave asks for
+    // TF; the sums of a superblock; and its own weight rows, a row's 144 bytes in nine lanes.  (Asked for in the order the
     // matrix instruction wants them, a row a lane, weights are 64 pieces of 16 bytes to an instruction: 2048 tokens, 12288 x
     // 1536, gate | up 312 us instead of 294.)
     const uint32_t l0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) uint8_t *)lds_rows;
     constexpr uint32_t kAtSums = 4 * S::kStage, kAtW = kAtSums + S::kSums, kAtInv = kAtW + 4 * NT * S::kTile;
-    const int f0 = wave * TT, ntt = (p.batch + 31) / 32, fsum = wave % (2 * TT);
-    const uint8_t *xsrc = reinterpret_cast<const uint8_t *>((f0 >> 1) & 1 ? p.Xf_lo : p.Xf) +
-                          ((size_t)min(t0 / 32 + (f0 >> 2), ntt - 1) * nsb_row + sb0) * 16384 + (f0 & 1) * 1024;
+    const int f0 = wave * TF, ntt = (p.batch + 31) / 32, fsum = wave % (2 * TT);
+    const uint8_t *xsrc = reinterpret_cast<const uint8_t *>(S::LO && ((f0 >> 1) & 1) ? p.Xf_lo : p.Xf) +
+                          ((size_t)min(t0 / 32 + f0 / (2 * PARTS), ntt - 1) * nsb_row + sb0) * 16384 + (f0 & 1) * 1024;
     const uint8_t *sxsrc = reinterpret_cast<const uint8_t *>(p.SxA) + (((size_t)min(t0 / 32 + (fsum >> 1), ntt - 1) * nsb_row + sb0) * 2 + (fsum & 1)) * 1024;
     const uint32_t lane16 = 16u * (uint32_t)lane, lw = l0 + kAtW + (uint32_t)(wave * NT * S::kTile);
     auto ask_rows = [&](int hs, int stage, int i) __attribute__((always_inline)) {
@@ -203,30 +206,30 @@ __global__ __launch_bounds__(S::kThreads, 2) void q4k_mm_rows_kernel(MmParams p)
                 }
     };
 
-    // A unit of the loop is four matrix instructions for one set of fragments: one part of a k slice for two token tiles (the
-    // parts in turn), or both parts of it for one.  U units to a half step.
-    constexpr int U = 2 * MT;
-    const uint32_t la = l0 + (uint32_t)(wm * MT) * 4096u + lane16;   // + stage, token tile, part, k slice
+    // A unit of the loop is 2 NT matrix instructions for two fragments: one part of a k slice for two token tiles (the parts, if
+    // there are two, in turn), or both parts of it for one.  U units to a half step.
+    constexpr int U = MT * PARTS;
+    constexpr uint32_t kTokens = PARTS * 2048;                         // bytes of a token tile's fragments
+    const uint32_t la = l0 + (uint32_t)(wm * MT) * kTokens + lane16;   // + stage, token tile, part, k slice
     const uint32_t lsum = l0 + kAtSums + (uint32_t)(wm * MT) * 2048u + lane16;
     const uint32_t lh = lw + 144u * (uint32_t)lm, lq = lh + 16u * (uint32_t)h;
     auto read_rows = [&](auto htag, auto utag, h8 (&v)[2]) __attribute__((always_inline)) {   // of unit U of a half step
         constexpr int hs = decltype(htag)::value & 3, u = decltype(utag)::value;
-        constexpr int off = hs * S::kStage + (MT == 2 ? (u >> 1) * 1024 + (u & 1) * 2048 : u * 1024);
+        constexpr int off = hs * S::kStage + (U == 4 ? (u >> 1) * 1024 + (u & 1) * 2048 : u * 1024);
         lds_ask<off>(v[0], la);
-        lds_ask<off + (MT == 2 ? 4096 : 2048)>(v[1], la);
+        lds_ask<off + (MT == 2 ? kTokens : 2048)>(v[1], la);
     };
     auto read_group = [&](auto gtag) __attribute__((always_inline)) {
         constexpr int o = 16 + 32 * decltype(gtag)::value;
         lds_ask<o>(q[decltype(gtag)::value][0], lq);
-        lds_ask<o + S::kTile>(q[decltype(gtag)::value][1], lq);
+        if constexpr (NT == 2) lds_ask<o + S::kTile>(q[decltype(gtag)::value][1], lq);
     };
     auto read_header = [&]() __attribute__((always_inline)) {
         lds_ask<0>(hdr[0], lh);
-        lds_ask<S::kTile>(hdr[1], lh);
+        if constexpr (NT == 2) lds_ask<S::kTile>(hdr[1], lh);
     };
     auto settle = [&](auto &v) __attribute__((always_inline)) {
-        arrived(v[0]);
-        arrived(v[1]);
+        for (auto &e : v) arrived(e);
     };
     constexpr std::integral_constant<int, 0> n0{};
     constexpr std::integral_constant<int, 1> n1{};
@@ -234,15 +237,15 @@ __global__ __launch_bounds__(S::kThreads, 2) void q4k_mm_rows_kernel(MmParams p)
     constexpr std::integral_constant<int, 3> n3{};
 
     // ---- in front of the loop: the first superblock's weights, three half steps of fragments; the first slice converted
-    to_lds4(reinterpret_cast<const uint8_t *>(p.inv_s), 4u * (uint32_t)min(t0 + lane, p.batch - 1), l0 + kAtInv);   // (every wave the same)
+    if (S::LO) to_lds4(reinterpret_cast<const uint8_t *>(p.inv_s), 4u * (uint32_t)min(t0 + lane, p.batch - 1), l0 + kAtInv);   // (every wave the same)
 #pragma unroll
     for (int j = 0; j < 5 * NT; j++) ask_weights(0, j);
     ask_sums(0);
 #pragma unroll
     for (int hs = 0; hs < 3; hs++)
 #pragma unroll
-        for (int i = 0; i < TT; i++) ask_rows(hs, hs, i);
-    asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" ::"n"(2 * TT) : "memory");
+        for (int i = 0; i < TF; i++) ask_rows(hs, hs, i);
+    asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" ::"n"(2 * TF) : "memory");
     read_group(n0);
     read_group(n1);
     read_group(n2);
@@ -263,12 +266,12 @@ __global__ __launch_bounds__(S::kThreads, 2) void q4k_mm_rows_kernel(MmParams p)
     // to back and leaves their pipe idle under the rest).
     auto unit = [&](int sb, auto htag, auto utag) __attribute__((always_inline)) {
         constexpr int half = decltype(htag)::value, place = decltype(utag)::value;
-        constexpr int g = half >> 1, ks = 2 * (half & 1) + place / MT, part = MT == 2 ? place & 1 : 0, set = place & 1;
+        constexpr int g = half >> 1, ks = 2 * (half & 1) + place / (U / 2), part = U == 4 ? place & 1 : 0, set = place & 1;
         constexpr int gn = ks == 3 ? (g + 1) & 3 : g, kn = (ks + 1) & 3;               // the next slice
         constexpr bool last = place == U - 1;
         // Memory operations of a half step: its first units ask for the fragments of three half steps on; the last two (the
-        // last, MT = 1) of half steps 0 .. 4 for two pieces of the next superblock's weights, of half step 5 for its sums.
-        constexpr auto extra = [](int hh) { return hh < 5 ? 2 : hh == 5 ? 1 : 0; };
+        // last, U = 2) of half steps 0 .. 4 for a piece of the next superblock's weights a tile, of half step 5 for its sums.
+        constexpr auto extra = [](int hh) { return hh < 5 ? NT : hh == 5 ? 1 : 0; };
         __builtin_amdgcn_sched_barrier(0);
         constexpr bool opens = half == 0 && place == 0;
         if constexpr (opens && CUT) {
@@ -280,14 +283,14 @@ __global__ __launch_bounds__(S::kThreads, 2) void q4k_mm_rows_kernel(MmParams p)
                 cut_ends();
             }
         }
-        constexpr int mins = MT == 2 ? (g == 1 && part == 0 && ks < 2 ? ks : -1) : (g == 1 && ks == 1 ? 0 : -1);
+        constexpr int mins = U == 4 ? (g == 1 && part == 0 && ks < 2 ? ks : -1) : (g == 1 && ks >= 1 && ks <= MT ? ks - 1 : -1);
         constexpr bool take0 = half == 7 && place == 0, take3 = half == 7 && last;
         // (behind the first matrix instruction, whose 32 cycles cover part of it: a request to memory takes some 40 to issue)
         auto ask = [&]() __attribute__((always_inline)) {
             if constexpr (last) {
                 // every wave has this half step's fragments in registers; the next one's, which this wave has asked for two half
-                // steps ago, are in LDS (and at the end of half step 6 the weights, which are 1 + 2 TT operations back)
-                constexpr int pending = half == 6 ? 1 + 2 * TT : extra((half + 6) & 7) + TT + extra((half + 7) & 7) + TT + (MT == 2 && extra(half) > 0 ? 1 : 0);
+                // steps ago, are in LDS (and at the end of half step 6 the weights, which are 1 + 2 TF operations back)
+                constexpr int pending = half == 6 ? 1 + 2 * TF : extra((half + 6) & 7) + TF + extra((half + 7) & 7) + TF + (U == 4 && (half == 5 || (half < 5 && NT == 2)) ? 1 : 0);
                 asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" ::"n"(pending) : "memory");
             }
             read_rows(std::integral_constant<int, (last ? half + 1 : half) & 7>{}, std::integral_constant<int, last ? 0 : place + 1>{}, a[set ^ 1]);
@@ -299,15 +302,15 @@ __global__ __launch_bounds__(S::kThreads, 2) void q4k_mm_rows_kernel(MmParams p)
             // the next superblock's weights, into the registers whose group has been converted
             if constexpr (take0) { read_group(n0); read_header(); }
             if constexpr (take3) { read_group(n1); read_group(n2); read_group(n3); }
-            if constexpr (MT == 2) {
-                if constexpr (place < TT) ask_rows(8 * sb + half + 3, (half + 3) & 3, place);
-                if constexpr (place >= 2 && half < 5) ask_weights(sb + 1, 2 * half + place - 2);
+            if constexpr (U == 4) {
+                if constexpr (place < TF) ask_rows(8 * sb + half + 3, (half + 3) & 3, place);
+                if constexpr (place >= 4 - NT && half < 5) ask_weights(sb + 1, NT * half + place - (4 - NT));
             } else if constexpr (place == 0) {
 #pragma unroll
-                for (int i = 0; i < TT; i++) ask_rows(8 * sb + half + 3, (half + 3) & 3, i);
+                for (int i = 0; i < TF; i++) ask_rows(8 * sb + half + 3, (half + 3) & 3, i);
             } else if constexpr (half < 5) {
-                ask_weights(sb + 1, 2 * half);
-                ask_weights(sb + 1, 2 * half + 1);
+#pragma unroll
+                for (int i = 0; i < NT; i++) ask_weights(sb + 1, NT * half + i);
             }
             if constexpr (place == U / 2 && half == 5) ask_sums(sb + 1);
         };
@@ -328,27 +331,30 @@ __global__ __launch_bounds__(S::kThreads, 2) void q4k_mm_rows_kernel(MmParams p)
         std::integral_constant<int, gn> gnext{};
         std::integral_constant<int, kn> knext{};
         std::integral_constant<int, (g + 1) & 3> gopen{};
-        // (groups are opened a unit ahead of their first conversion, MT = 1: in front of it; the short product's operand in the
+        // (groups are opened a unit ahead of their first conversion, U = 2: in front of it; the short product's operand in the
         // quiet units of the first steps)
-        constexpr bool op0 = MT == 2 ? ks == 2 && part == 1 : ks == 3, op1 = MT == 2 ? ks == 3 && part == 0 : ks == 3, sc = op0 && g == 3;
-        constexpr int mu = (half * U + place) - (MT == 2 ? 1 : 0), mn = MT == 2 ? (mu >= 0 && mu < 4 ? mu : -1) : (mu < 3 ? mu : mu == 4 ? 3 : -1);
+        constexpr bool op0 = U == 4 ? ks == 2 && part == 1 : ks == 3, op1 = NT == 2 && (U == 4 ? ks == 3 && part == 0 : ks == 3), sc = op0 && g == 3;
+        constexpr int mu = (half * U + place) - (U == 4 ? 1 : 0), mn = NT == 1 ? (mu < 2 ? mu : -1) : U == 4 ? (mu < 4 ? mu : -1) : (mu < 3 ? mu : mu == 4 ? 3 : -1);
+        constexpr int converted = U == 2 ? NT : part < NT ? 1 : 0;
         if constexpr (sc) scales();
-        if constexpr (MT == 1) {
-            if constexpr (op0) { open_group(gopen, 0); open_group(gopen, 1); }
-            convert(gnext, knext, 0);
-            convert(gnext, knext, 1);
+        if constexpr (U == 2) {
+#pragma unroll
+            for (int nt = 0; nt < NT; nt++) {
+                if constexpr (op0) open_group(gopen, nt);
+                convert(gnext, knext, nt);
+            }
         } else {
-            convert(gnext, knext, part);
+            if constexpr (converted) convert(gnext, knext, part);
             if constexpr (op0) open_group(gopen, 0);
             if constexpr (op1) open_group(gopen, 1);
         }
         if constexpr (mn >= 0) min_operand(mn >> 1, mn & 1);
-        constexpr int valu = (MT == 2 ? 11 : 22) + (op0 ? 8 : 0) + (op1 ? 8 : 0) + (sc ? 10 : 0) + (mn >= 0 ? 22 : 0);
+        constexpr int valu = 11 * converted + (op0 ? 8 : 0) + (op1 ? 8 : 0) + (sc ? 5 * NT : 0) + (mn >= 0 ? 22 : 0), gaps = 2 * NT - 1;
         if constexpr (!opens) {
 #pragma unroll
-            for (int i = 0; i < 3; i++) {
+            for (int i = 0; i < gaps; i++) {
                 __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
-                __builtin_amdgcn_sched_group_barrier(0x002, (valu + 2) / 3, 0);
+                __builtin_amdgcn_sched_group_barrier(0x002, (valu + gaps - 1) / gaps, 0);
             }
         }
         __builtin_amdgcn_sched_barrier(0);
@@ -394,11 +400,13 @@ __global__ __launch_bounds__(S::kThreads, 2) void q4k_mm_rows_kernel(MmParams p)
     for (int mt = 0; mt < MT; mt++) {
         const int tb = t0 + (wm * MT + mt) * 32 + 4 * h, left = p.batch - tb;
         f32x4_t inv[4];
+        if (S::LO) {
 #pragma unroll
-        for (int i4 = 0; i4 < 4; i4++) asm volatile("ds_read_b128 %0, %1" : "=v"(inv[i4]) : "v"(l0 + kAtInv + 4u * (uint32_t)(tb - t0 + 8 * i4)));
-        lds_wait();
+            for (int i4 = 0; i4 < 4; i4++) asm volatile("ds_read_b128 %0, %1" : "=v"(inv[i4]) : "v"(l0 + kAtInv + 4u * (uint32_t)(tb - t0 + 8 * i4)));
+            lds_wait();
 #pragma unroll
-        for (int i4 = 0; i4 < 4; i4++) arrived(inv[i4]);
+            for (int i4 = 0; i4 < 4; i4++) arrived(inv[i4]);
+        }
 #pragma unroll
         for (int nt = 0; nt < NT; nt += PAIR ? 2 : 1) {
             const int r = r0 + (PAIR ? wn : wn * NT + nt) * 32 + lm;
@@ -407,8 +415,8 @@ __global__ __launch_bounds__(S::kThreads, 2) void q4k_mm_rows_kernel(MmParams p)
 #pragma unroll
             for (int i = 0; i < 16; i++) {
                 const int t = 8 * (i / 4) + (i & 3);
-                float v = F[mt][nt][i] * inv[i / 4][i & 3];
-                if (PAIR) v = gelu_mul_f32(pinned(v), pinned(F[mt][1][i] * inv[i / 4][i & 3]));
+                float v = S::LO ? F[mt][nt][i] * inv[i / 4][i & 3] : F[mt][nt][i];
+                if constexpr (PAIR) v = gelu_mul_f32(pinned(v), pinned(F[mt][1][i] * inv[i / 4][i & 3]));
                 if (t < left) y[(size_t)t * ystride] = v;
             }
         }

@@ -326,8 +326,8 @@ def test_mul_mm_f32_both_parts_in_one_workgroup(ctx, unfolded, k_split):
 
 
 @pytest.mark.parametrize("rows,batch,cols,mode,shape", [
-    (1, 65, 256, 0, "32x256"), (257, 33, 768, 0, "32x256"), (255, 96, 7936, 0, "32x256"), (300, 129, 1024, 2, "32x256"),
-    (129, 65, 512, 3, "32x256"), (4097, 1000, 256, 0, "64x256"), (7937, 545, 512, 3, "64x256")])
+    (1, 65, 256, 0, "32x128"), (257, 33, 768, 0, "32x128"), (255, 96, 7936, 0, "32x128"), (300, 129, 1024, 2, "32x256"),
+    (129, 65, 512, 3, "32x256"), (4095, 1000, 256, 0, "64x256"), (7937, 545, 512, 3, "64x256")])
 def test_mul_mm_f32_rows_at_the_edges_of_its_tiles(ctx, rows, batch, cols, mode, shape):
     """Both shapes of the f32 rows' kernel where they can go wrong: one superblock and thirty-one, a row or a token past a
     tile or short of it, two matrices side by side (gelu(gate) * up), rows summed as in launches of their own.  Against
