@@ -22,13 +22,9 @@
 // X is bf16, which converts to f16 without loss for |x| >= 2^-17 (smaller
 // values lose at most 2^-25 absolutely).
 //
-// Tiling: a workgroup owns 128 tokens x 128 weight rows; each of its four
-// multiplying waves owns 32 tokens x 128 rows as 1 x 4 v_mfma_f32_32x32x16_f16
-// tiles (four more waves load and convert).  M = tokens, N = weight
+// Tiling: q4k_mm_rows.hpp (prompts), q4k_mm_skinny_kernel (up to 64 tokens); M = tokens, N = weight
 // rows, so a lane's accumulator column is one weight row (one d per lane) and
-// stores are contiguous along Y's row index.  K advances 64 columns (one
-// 64-element group: 32 quant bytes per row) per step through a double-buffered
-// LDS stage, with the next step's global loads in flight under the MFMAs.
+// stores are contiguous along Y's row index.  Q6_K weights: q6k_mul_mm_kernel.
 #include <algorithm>
 #include <type_traits>
 
@@ -46,7 +42,6 @@ typedef uint32_t u32x2_t __attribute__((ext_vector_type(2)));
 
 constexpr int BM = 128, BN = 128, KS = 64;
 constexpr int PITCH = KS + 8;      // halves per LDS row of the main tiles (144 B: conflict-free 16 B reads)
-constexpr int PITCH2 = 32 + 8;     // halves per LDS row of the min-term tiles
 
 // X bf16 -> f16 (permuted) in the order the matrix instruction wants its A operand, plus the min-term
 // operand per (token, superblock): 32 halves = Sx_hi[8] | Sx_hi[8] | Sx_lo[8] | 0[8].
@@ -59,6 +54,7 @@ constexpr int PITCH2 = 32 + 8;     // halves per LDS row of the min-term tiles
 // Xf came from eight workgroups: 5.7 us for 2 MB).  The four waves of a workgroup take neighbouring sub-blocks, so
 // that together they read whole lines of X.  The sub-block's sum is (run 0 + run 1) + (run 2 + run 3), the two
 // halves of the wave trading their runs' sums.
+template <bool IN_ORDER>
 __global__ __launch_bounds__(256) void mm_prep_x_kernel(const uint16_t *__restrict__ X, _Float16 *__restrict__ Xf,
                                                         _Float16 *__restrict__ SxA, int batch, int cols)
 {
@@ -96,12 +92,13 @@ __global__ __launch_bounds__(256) void mm_prep_x_kernel(const uint16_t *__restri
         sum = pinned(sum);
         const _Float16 hi = (_Float16)sum;
         const _Float16 lo = (_Float16)(sum - (float)hi);
-        _Float16 *a2 = SxA + ((size_t)t * (cols / 256) + s / 8) * 32;
         const int jj = s % 8;
+        constexpr int step = IN_ORDER ? 256 : 8;
+        _Float16 *a2 = IN_ORDER ? SxA + ((size_t)tb * (cols / 256) + s / 8) * 1024 + lane * 8 : SxA + ((size_t)t * (cols / 256) + s / 8) * 32;
         a2[jj] = hi;
-        a2[8 + jj] = hi;
-        a2[16 + jj] = lo;
-        a2[24 + jj] = (_Float16)0.f;
+        a2[step + jj] = hi;
+        a2[2 * step + jj] = lo;
+        a2[3 * step + jj] = (_Float16)0.f;
     }
 }
 
@@ -403,14 +400,16 @@ __host__ __device__ constexpr int mm_k_slices(bool q6, int row_tiles, int nsb, i
     return ks;
 }
 
-// Bf16 activations: token tile and K slices (of any number of superblocks) of the tile by what the launches are made of, in
-// us, fitted to 300 .. 12288 rows of 1024 .. 8192 columns, 2 .. 2048 tokens, every slice count:
-//   a round of 128-token tiles (one workgroup a compute unit)        5 + 2.4 per superblock of the slice
-//   64-token tiles, one / two workgroups a compute unit              4.2 + 2.0 / 6 + 2.9
-//   the fold                                                         2.5 + the partial sums, written and read, at 4 TB/s
-// The tile of the smallest sum is within 5 % of the best of all (tile, slices) at those shapes.  Against slices by powers
-// of two until the chip is full: 333 tokens, 1536 x 6144 four -> six slices, 29.8 -> 25.4 us (Q6_K); 300 x 7936 (31
-// superblocks) one -> eight, 95 -> 27 at 512 tokens; 12288 x 4096 at 100 tokens one of 64 -> two of 128, 35.3 -> 29.2.
+// Bf16 activations: token tile and K slices (of any number of superblocks) by what the launches are made of, in us, fitted to
+// 256 .. 12288 rows of 512 .. 8192 columns, 2 .. 2048 tokens, every slice count:
+//   Q6_K, a round of 128-token tiles (one workgroup a compute unit)  5 + 2.4 per superblock of the slice; the fold 2.5 + the
+//                    partial sums, written and read, at 4 TB/s
+//   Q4_K             with its preparation, 64 tokens a workgroup (128): 5.2 (6.4) + 0.6 per round of workgroups over the compute
+//                    units + what rows and results cost; a superblock 1.45 in one round, 1.7 in two, 0.73 a round in more (1.87,
+//                    1.31 a round), and up to 36 % (16 %) more as the chip fills; the fold 4.2 (4.6) + 1.4 per million partial sums
+// Its choice is on average within 1 % of the best (tile, slices) at those shapes, within 8 % at all.  Q6_K, 333 tokens, 1536 x
+// 6144: four -> six slices 29.8 -> 25.4 us.  Q4_K: 2048 tokens of 12288 x 4096 262 us with 64 tokens a workgroup, 227 with 128; 300
+// tokens of 12288 x 1536 24.4 or 30.8; 65 tokens of 12288 x 8192 47 us in two slices of 64 tokens, 40 in eight of 128.
 struct MmPlan {
     int tm, ks;
     float us;
@@ -419,23 +418,27 @@ MmPlan mm_plan_bf16(bool q6, int row_tiles, int nsb, int64_t batch, int64_t rows
 {
     MmPlan best{128, 1, 1e30f};
     const int ks_max = std::min(nsb, 64);
+    const float m = (float)(batch * rows_all) * 1e-6f;
     for (int tm = q6 ? 128 : 64; tm <= 128; tm += 64)
         for (int ks = ks_given ? ks_given : 1; ks <= (ks_given ? ks_given : ks_max); ks++) {
-            const int64_t w = (batch + tm - 1) / tm * row_tiles * ks;
-            const float sb = (float)((nsb + ks - 1) / ks);
-            float us = tm == 128 ? (float)((w + 255) / 256) * (5.f + 2.4f * sb) : w <= 256 ? 4.2f + 2.0f * sb : (float)((w + 511) / 512) * (6.f + 2.9f * sb);
-            if (ks > 1) us += 2.5f + (float)ks * (float)(batch * rows_all) * 2e-6f;
+            const int64_t wgs = (batch + tm - 1) / tm * row_tiles * ks;
+            const float sb = (float)((nsb + ks - 1) / ks), w = (float)wgs / 256.f, rounds = (float)((wgs + 255) / 256);
+            float us;
+            if (q6) us = rounds * (5.f + 2.4f * sb) + (ks > 1 ? 2.5f + 2.f * (float)ks * m : 0.f);
+            else if (tm == 64) us = 5.2f + 1.4f * m + (rounds <= 1.f ? 1.45f : rounds <= 2.f ? 1.7f : 0.73f * rounds) * (1.f + 0.18f * std::min(w, 2.f)) * sb + (ks > 1 ? 4.2f + 1.4f * (float)ks * m : 0.f);
+            else us = 6.4f + 2.f * m + (rounds <= 1.f ? 1.87f : 1.31f * rounds) * (1.f + 0.08f * std::min(w, 2.f)) * sb + (ks > 1 ? 4.6f + 1.4f * (float)ks * m : 0.f);
+            if (!q6) us += 0.6f * rounds + (float)(batch * nsb) * 256e-6f;
             if (us < best.us) best = MmPlan{tm, ks, us};
         }
     return best;
 }
 
-// The small-batch form beside it (bf16): a workgroup of eight waves per 32 rows, superblocks dealt to the waves; the numbers
-// carry what the tile's preparation and launch take more (2.4).
+// The small-batch form beside it (Q4_K, bf16), with its preparation: a workgroup of eight waves per 32 rows, superblocks dealt to
+// the waves (300 .. 12288 rows of 512 .. 6144 columns).
 float mm_skinny_us(int64_t rows, int nsb, int64_t batch)
 {
-    const float fill = (float)((rows + 31) / 32) / 256.f;
-    return 1.8f + (batch <= 32 ? 3.4f : 5.5f) * std::max(1.f, (float)nsb / 8.f) * std::max(1.f, 2.f * fill - 1.f);
+    const float turns = std::max(1.f, (float)((rows + 31) / 32) / 128.f - 1.f), each = (float)nsb / 8.f;
+    return batch <= 32 ? 5.5f + 3.1f * each * turns : 6.4f + 5.f * std::max(each, 0.45f) * turns;
 }
 
 // Bf16 rows of Q6_K products as they are (the kernel's ROWS form): the conversion between the matrix instructions costs 0.42
@@ -451,41 +454,24 @@ __device__ __forceinline__ uint32_t pair_f16(uint32_t masked, uint32_t sc)
     return __umul24(masked, sc) + 0x64006400u;     // half 1024.0 twice
 }
 
-// what a loader thread (two per tile row) holds per superblock: of each of the four 64-column groups the 16 quant
-// bytes it converts (all requested when the superblock opens, so that a weight row's cache lines are fetched once,
-// not once per step), the header and half of the token's sums of x
-// (native vector types: with HIP's uint4 class the copies become memcpys that keep these sets in scratch memory)
-struct SbRegs {
-    u32x4_t q[4];      // of each of the four 64-column groups, the 16 quant bytes this thread converts
-    u32x4_t hdr, sx0, sx1;
-};
-
 constexpr int kThreadsMM = 512;
 constexpr int kLdsMain = BN * PITCH;             // halves per main stage (the dequantized weight tile)
-constexpr int kLdsMin = (BM + BN) * PITCH2;      // halves per min-term stage
-constexpr size_t kLdsBytes = 2 * (size_t)(kLdsMain + kLdsMin) * 2 + 2 * BN * 4;
-constexpr size_t kLdsBytes64 = 2 * (size_t)(kLdsMain + (64 + BN) * PITCH2) * 2 + 2 * BN * 4;   // the 64-token tile
+constexpr size_t kLdsBytes = 2 * (size_t)kLdsMain * 2 + 2 * BN * 4;
 
-// Eight waves in two roles, one of each per SIMD.  Waves 0..3 only multiply:
-// each owns 32 tokens x 128 columns of the 128-token tile (1 x 4 MFMA tiles; of
-// the 64-token tile 32 x 64) and works on LDS stage s&1.  Waves 4..7 only
+// The GEMM over Q6_K weights (K3b of the reference's plan: Q6_K tensors in prefill): 128 tokens x 128 weight rows a workgroup,
+// eight waves in two roles, one of each per SIMD.  Waves 0..3 only multiply:
+// each owns 32 tokens x 128 columns (1 x 4 MFMA tiles) and works on LDS stage s&1.  Waves 4..7 only
 // load and convert: during the same step they request the activations of step
 // s+4 (and, when a superblock opens, the next superblock's weights) and write
 // step s+1 into stage (s+1)&1.  One barrier per K step joins them, so the
 // conversions and the LDS writes of one role run in the shadow of the other
-// role's matrix instructions.  The min-term operands of a superblock are
-// written together with its first step into their own double buffer and
-// consumed after its fourth.
+// role's matrix instructions.
 //
-// Q6 = true: the same tile and roles over Q6_K weights (K3b of the reference's plan: Q6_K tensors in prefill).
 // w = d * sc_j * q with q = code - 32 in [-32, 31] and sc_j an int8 per 16 columns; the loaders build the f16
 // pair (1024 + code) by an OR into the mantissa, subtract 1056 and multiply by sc_j, both as packed f16.
 // sc_j * q is exact in f16 up to 2048; beyond that (needs |sc_j| > 64) it rounds to the nearest even integer, a
 // relative 2^-11 at most and on those weights only (the reference's tile rounds every weight to half, the same
-// bound).  There is no min term, so the short second product is skipped; d is applied per superblock as for Q4_K.
-// TM = tokens per workgroup.  128: each multiplying wave owns 32 x 128.  64: each owns 32 x 64 with half the
-// accumulators, the kernel fits 128 registers and 70 KB of LDS, and two workgroups share a compute unit, so that one's
-// barriers and first loads fall into the other's products (the weights are converted once per 64 tokens then).
+// bound).  There is no min term; d is applied per superblock as for Q4_K.
 // LO = true: f32 activations as two f16 parts at the row's own scale.  Every converted weight meets the hi and the lo
 // fragment of a token tile in the same accumulator (twice the matrix instructions per conversion, and the
 // conversions are what a step waits for), and the finished sums are multiplied by 1 / s of their token.
@@ -493,19 +479,15 @@ constexpr size_t kLdsBytes64 = 2 * (size_t)(kLdsMain + (64 + BN) * PITCH2) * 2 +
 // depend on its length.  The workgroup takes all of K, and where a row's slice ends its sum is added to Y and starts
 // again from zero: the bits of those launches from one that fills the chip (a read and a write of the tile's results
 // per slice end, from L2).
-// ROWS = true (bf16 activations, Q6_K weights: no sums of x are wanted): the A operands come from the rows of X as they are
+// ROWS = true (bf16 activations; no sums of x are wanted): the A operands come from the rows of X as they are
 // and the multiplying waves convert them, eight values of a row a lane, between their matrix instructions -- no
 // preparation launch (mm_rows_direct; 333 tokens, 1536 x 6144 in six slices: 28.9 -> 25.4 us).
-// (F32 rows of Q4_K take q4k_mm_rows_kernel.)
-template <bool Q6, int TM, bool LO, bool CUT = false, bool ROWS = false>
-__global__ __launch_bounds__(kThreadsMM, TM == 64 ? 2 : 1) void q_mul_mm_kernel(MmParams p)
+template <bool LO, bool CUT = false, bool ROWS = false>
+__global__ __launch_bounds__(kThreadsMM, 1) void q6k_mul_mm_kernel(MmParams p)
 {
-    static_assert(Q6 || !LO, "");
-    constexpr int MT = TM / 64, kLdsMinT = (TM + BN) * PITCH2;
     extern __shared__ __attribute__((aligned(16))) _Float16 lds[];
     auto main_stage = [&](int i) { return lds + (i & 1) * kLdsMain; };
-    auto min_stage = [&](int i) { return lds + 2 * kLdsMain + (i & 1) * kLdsMinT; };
-    auto dsc_stage = [&](int i) { return reinterpret_cast<float *>(lds + 2 * kLdsMain + 2 * kLdsMinT) + (i & 1) * BN; };
+    auto dsc_stage = [&](int i) { return reinterpret_cast<float *>(lds + 2 * kLdsMain) + (i & 1) * BN; };
 
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     // which matrix this row tile belongs to (the copy of the arguments is this workgroup's own)
@@ -517,7 +499,7 @@ __global__ __launch_bounds__(kThreadsMM, TM == 64 ? 2 : 1) void q_mul_mm_kernel(
         if (by >= ty0 + ty1) { by -= ty0 + ty1; ycol = p.rows + p.rows1; p.W = p.W2; p.Y = p.Y2; p.rows = p.rows2; }
         else if (by >= ty0) { by -= ty0; ycol = p.rows; p.W = p.W1; p.Y = p.Y1; p.rows = p.rows1; }
     }
-    const int t0 = blockIdx.x * TM, r0 = by * BN;
+    const int t0 = blockIdx.x * BM, r0 = by * BN;
     const int nsb_row = p.cols / 256;                            // superblocks per weight row
     int nsb = nsb_row, sb0 = 0;                                  // this workgroup's share of them
     size_t ystride = (size_t)p.rows;
@@ -530,8 +512,8 @@ __global__ __launch_bounds__(kThreadsMM, TM == 64 ? 2 : 1) void q_mul_mm_kernel(
     }
     const int nsteps = nsb * 4;
 
-    if (Q6 && wave >= 4) {
-        // ------------------------------------------------------------------ loaders, Q6_K
+    if (wave >= 4) {
+        // ------------------------------------------------------------------ loaders
         // thread lh of a row's pair converts columns 32*lh .. 32*lh+31 of every 64-column step: step (h, part)
         // of a superblock = ql bytes 64h + 32lh .. +31 (nibble `part`), qh bytes 32h .. +31 (bit pair
         // 4*part + 2*lh), scales 8h + 4*part + 2*lh and the next one.  Blocks are 2-byte aligned.
@@ -613,152 +595,45 @@ __global__ __launch_bounds__(kThreadsMM, TM == 64 ? 2 : 1) void q_mul_mm_kernel(
         return;
     }
 
-    if (!Q6 && wave >= 4) {
-        // ------------------------------------------------------------------ loaders
-        const int lt = tid - 256, lrow = lt >> 1, lh = lt & 1;   // two threads per tile row
-        const size_t row_bytes = (size_t)nsb_row * 144;
-        const uint8_t *wrow = p.W + (size_t)min(r0 + lrow, p.rows - 1) * row_bytes + (size_t)sb0 * 144;
-        const size_t sx_off = ((size_t)min(t0 + lrow, p.batch - 1) * nsb_row + sb0) * 32;
-        const _Float16 *sxrow = p.SxA + sx_off;
-
-        auto fetch_sb = [&](int sb, SbRegs &r) __attribute__((always_inline)) {
-            const u32x4_t *w = reinterpret_cast<const u32x4_t *>(wrow + (size_t)sb * 144);
-            r.hdr = w[0];
-#pragma unroll
-            for (int i = 0; i < 4; i++) r.q[i] = w[1 + 2 * i + lh];     // the 16 bytes of group i that this thread converts
-            const u32x4_t *sx = reinterpret_cast<const u32x4_t *>(sxrow + sb * 32 + 16 * lh);
-            r.sx0 = sx[0];
-            r.sx1 = sx[1];
-        };
-        // G = the step's group: this thread converts bytes 16*lh .. 16*lh+15 of its 32 quant bytes
-        auto stage = [&](int step, auto gtag, const SbRegs &w) __attribute__((always_inline)) {
-            constexpr int G = decltype(gtag)::value;
-            const int sb = step >> 2;
-            _Float16 *Bs = main_stage(step);
-            {
-                const u32x4_t c = w.q[G];
-                const uint32_t q[4] = {c[0], c[1], c[2], c[3]};
-                const uint4 s = q4k_group_scales(w.hdr.y, w.hdr.z, w.hdr.w, G);   // sc_lo, mn_lo, sc_hi, mn_hi
-                uint32_t lo[8], hi[8];
-#pragma unroll
-                for (int i = 0; i < 4; i++) {
-                    const uint32_t t4 = q[i] >> 4;
-                    lo[2 * i] = pair_f16(q[i] & 0x000F000Fu, s.x);
-                    lo[2 * i + 1] = pair_f16((q[i] >> 8) & 0x000F000Fu, s.x);
-                    hi[2 * i] = pair_f16(t4 & 0x000F000Fu, s.z);
-                    hi[2 * i + 1] = pair_f16((t4 >> 8) & 0x000F000Fu, s.z);
-                }
-                uint4 *dlo = reinterpret_cast<uint4 *>(&Bs[lrow * PITCH + 16 * lh]);
-                uint4 *dhi = reinterpret_cast<uint4 *>(&Bs[lrow * PITCH + 32 + 16 * lh]);
-                dlo[0] = make_uint4(lo[0], lo[1], lo[2], lo[3]);
-                dlo[1] = make_uint4(lo[4], lo[5], lo[6], lo[7]);
-                dhi[0] = make_uint4(hi[0], hi[1], hi[2], hi[3]);
-                dhi[1] = make_uint4(hi[4], hi[5], hi[6], hi[7]);
-            }
-            if (G == 0) {
-                // bias + mins of this superblock, for the short second product after its fourth step
-                _Float16 *A2s = min_stage(sb), *B2s = A2s + TM * PITCH2;
-                const float d = half_bits_to_f32(w.hdr.x & 0xFFFFu), dmin = half_bits_to_f32(w.hdr.x >> 16);
-                // this thread covers sub-blocks 4*lh .. 4*lh+3 of its row: groups 2*lh, 2*lh+1
-                uint32_t hi2[2], lo2[2];
-#pragma unroll
-                for (int gg = 0; gg < 2; gg++) {
-                    const uint4 s = q4k_group_scales(w.hdr.y, w.hdr.z, w.hdr.w, 2 * lh + gg);
-                    const float c0 = pinned(-(dmin * (float)s.y + 1024.f * d)), c1 = pinned(-(dmin * (float)s.w + 1024.f * d));
-                    const _Float16 h0 = (_Float16)c0, h1 = (_Float16)c1;
-                    const _Float16 l0 = (_Float16)(c0 - (float)h0), l1 = (_Float16)(c1 - (float)h1);
-                    hi2[gg] = (uint32_t)__builtin_bit_cast(uint16_t, h0) | ((uint32_t)__builtin_bit_cast(uint16_t, h1) << 16);
-                    lo2[gg] = (uint32_t)__builtin_bit_cast(uint16_t, l0) | ((uint32_t)__builtin_bit_cast(uint16_t, l1) << 16);
-                }
-                // row layout (32 halves): hi[8] | lo[8] | hi[8] | 0[8]; this thread owns halves 4*lh .. +3 of each octet
-                uint2 *b2 = reinterpret_cast<uint2 *>(&B2s[lrow * PITCH2 + 4 * lh]);
-                b2[0] = make_uint2(hi2[0], hi2[1]);
-                b2[2] = make_uint2(lo2[0], lo2[1]);
-                b2[4] = make_uint2(hi2[0], hi2[1]);
-                b2[6] = make_uint2(0u, 0u);
-                if (lh == 0) dsc_stage(sb)[lrow] = d;
-                if (lrow < TM) {
-                    u32x4_t *dst = reinterpret_cast<u32x4_t *>(&A2s[lrow * PITCH2 + 16 * lh]);
-                    dst[0] = w.sx0;
-                    dst[1] = w.sx1;
-                }
-            }
-        };
-
-        // the next superblock's weights are requested when a superblock opens: four steps to arrive
-        SbRegs wcur, wnext;
-        fetch_sb(0, wcur);
-        stage(0, std::integral_constant<int, 0>{}, wcur);
-        __syncthreads();
-        auto step_body = [&](int sb, auto gtag) __attribute__((always_inline)) {
-            constexpr int g = decltype(gtag)::value;
-            const int step = 4 * sb + g;
-            if (g == 0) fetch_sb(min(sb + 1, nsb - 1), wnext);
-            if (step + 1 < nsteps) {
-                if (g == 3) wcur = wnext;
-                stage(step + 1, std::integral_constant<int, (g + 1) & 3>{}, wcur);
-            }
-            __syncthreads();
-        };
-        for (int sb = 0; sb < nsb; sb++) {
-            step_body(sb, std::integral_constant<int, 0>{});
-            step_body(sb, std::integral_constant<int, 1>{});
-            step_body(sb, std::integral_constant<int, 2>{});
-            step_body(sb, std::integral_constant<int, 3>{});
-        }
-        return;
-    }
-
     // ---------------------------------------------------------------------- multipliers
-    // WIDE (the 128-token tiles): a multiplying wave owns 32 tokens x all 128 columns instead of 64 x 64 -- one A fragment
-    // per k slice serves four products, so the activations cross the vector-memory path once per workgroup instead of
-    // twice (that path was busy for two thirds of the kernel), and all four waves read every B operand from LDS (twice
-    // the LDS reads, which the operands requested a slice ahead hide): cfg2 31.5 -> 30.5 us per pair.
-    constexpr bool WIDE = TM == 128;
-    constexpr int MW = WIDE ? 1 : MT, NW_ = WIDE ? 4 : 2, NSPAN = WIDE ? 0 : 64;
-    const int wm = WIDE ? wave : wave >> 1, wn = WIDE ? 0 : wave & 1;
-    f16v F[MW][NW_], Cp[MW][NW_];
+    // A multiplying wave owns 32 tokens x all 128 columns instead of 64 x 64 -- one A fragment per k slice serves four
+    // products, so the activations cross the vector-memory path once per workgroup instead of twice, and all four waves read
+    // every B operand from LDS (twice the LDS reads, which the operands requested a slice ahead hide).
+    constexpr int NW_ = 4;
+    const int wm = wave;
+    f16v F[NW_], Cp[NW_];
 #pragma unroll
-    for (int a = 0; a < MW; a++)
+    for (int b = 0; b < NW_; b++)
 #pragma unroll
-        for (int b = 0; b < NW_; b++)
-#pragma unroll
-            for (int i = 0; i < 16; i++) { F[a][b][i] = 0.f; Cp[a][b][i] = 0.f; }
+        for (int i = 0; i < 16; i++) { F[b][i] = 0.f; Cp[b][i] = 0.f; }
     const int lm = lane & 31, lk = (lane >> 5) * 8;
     const f16v kZero16 = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
     // A operands straight from memory: fragment (token tile, k / 16) is 64 lanes x 16 bytes, 1 KB apart along k.
     // Two register sets, each refilled for two steps ahead as soon as its own step's instructions are issued (LO: one
     // set of hi and lo fragments, refilled for the next step -- a step is long against the way to the cache).
     const int ntt = (p.batch + 31) / 32;
-    const h8 *xa[MW];
     const uint16_t *xrow = reinterpret_cast<const uint16_t *>(p.Xf) + (size_t)min(t0 + wm * 32 + lm, p.batch - 1) * p.cols + (size_t)sb0 * 256 + lk;   // ROWS
-#pragma unroll
-    for (int mt = 0; mt < MW; mt++)
-        xa[mt] = reinterpret_cast<const h8 *>(p.Xf) + ((size_t)min((t0 + (wm * MW + mt) * 32) / 32, ntt - 1) * (p.cols / 16) + (size_t)sb0 * 16) * 64 + lane;
+    const h8 *xa = reinterpret_cast<const h8 *>(p.Xf) + ((size_t)min(t0 / 32 + wm, ntt - 1) * (p.cols / 16) + (size_t)sb0 * 16) * 64 + lane;
     const ptrdiff_t lo_delta = LO ? reinterpret_cast<const h8 *>(p.Xf_lo) - reinterpret_cast<const h8 *>(p.Xf) : 0;
-    auto afrag = [&](int mt, int step, int ks) __attribute__((always_inline)) {
+    auto afrag = [&](int step, int ks) __attribute__((always_inline)) {
         if (ROWS) return *reinterpret_cast<const h8 *>(xrow + step * KS + 16 * ks);      // (bf16 as yet)
-        return xa[mt][(ptrdiff_t)(step * (KS / 16) + ks) * 64];
+        return xa[(ptrdiff_t)(step * (KS / 16) + ks) * 64];
     };
-    auto afrag_lo = [&](int mt, int step, int ks) __attribute__((always_inline)) {
-        return xa[mt][(ptrdiff_t)(step * (KS / 16) + ks) * 64 + lo_delta];
-    };
+    auto afrag_lo = [&](int step, int ks) __attribute__((always_inline)) { return xa[(ptrdiff_t)(step * (KS / 16) + ks) * 64 + lo_delta]; };
     constexpr int AHEAD = LO ? 1 : 2;
-    struct ARegs { h8 a[MW][KS / 16], al[LO ? MW : 1][KS / 16]; };
+    struct ARegs { h8 a[KS / 16], al[LO ? KS / 16 : 1]; };
     auto fetch_a = [&](int step, ARegs &r) __attribute__((always_inline)) {
 #pragma unroll
-        for (int mt = 0; mt < MW; mt++)
-#pragma unroll
-            for (int ks = 0; ks < KS / 16; ks++) {
-                r.a[mt][ks] = afrag(mt, step, ks);
-                if (LO) r.al[mt][ks] = afrag_lo(mt, step, ks);
-            }
+        for (int ks = 0; ks < KS / 16; ks++) {
+            r.a[ks] = afrag(step, ks);
+            if (LO) r.al[ks] = afrag_lo(step, ks);
+        }
     };
     // CUT: lane t % 32 keeps the superblocks per slice of the tile's row t and what is left of the current one
     int cut_len = nsb, cut_left = nsb;
     if (CUT) {
         const int row_tiles = (rows_of[0] + BN - 1) / BN + (rows_of[1] + BN - 1) / BN + (rows_of[2] + BN - 1) / BN;
-        cut_len = cut_left = nsb / mm_k_slices(Q6, row_tiles, nsb, (int)p.cut_as[min(t0 + wm * 32 + lm, p.batch - 1)]);
+        cut_len = cut_left = nsb / mm_k_slices(true, row_tiles, nsb, (int)p.cut_as[min(t0 + wm * 32 + lm, p.batch - 1)]);
     }
     ARegs a0, a1;
     fetch_a(0, a0);
@@ -768,84 +643,43 @@ __global__ __launch_bounds__(kThreadsMM, TM == 64 ? 2 : 1) void q_mul_mm_kernel(
         constexpr int g = decltype(gtag)::value;
         const int step = 4 * sb + g;
         const _Float16 *Bs = main_stage(step);
-        // B operands a k slice ahead (bf16 / f16 activations on the 128-token tile): left to itself the compiler reads a
-        // slice's two operands into the registers the previous slice's products have just released, so every slice
-        // begins with an LDS round trip in front of its four matrix instructions (cfg2: 32.5 -> 31.1 us per pair).  The 64-token tile loses by it (a 256-token prompt 5.1 -> 5.3 ms) and keeps the plain order.
-        constexpr bool BPIPE = TM == 128;
-        h8 bb[2][NW_];
-        if (BPIPE) {
+        // B operands a k slice ahead: left to itself the compiler reads a slice's operands into the registers the previous
+        // slice's products have just released, so every slice begins with an LDS round trip in front of its four matrix
+        // instructions.
+        h8 b[2][NW_];
 #pragma unroll
-            for (int nt = 0; nt < NW_; nt++)
-                bb[0][nt] = *reinterpret_cast<const h8 *>(&Bs[(wn * NSPAN + nt * 32 + lm) * PITCH + lk]);
-        }
+        for (int nt = 0; nt < NW_; nt++) b[0][nt] = *reinterpret_cast<const h8 *>(&Bs[(nt * 32 + lm) * PITCH + lk]);
 #pragma unroll
         for (int ks = 0; ks < KS / 16; ks++) {
-            h8 b[NW_];
-            if (BPIPE) {
-                if (ks + 1 < KS / 16) {
-#pragma unroll
-                    for (int nt = 0; nt < NW_; nt++)
-                        bb[(ks + 1) & 1][nt] = *reinterpret_cast<const h8 *>(&Bs[(wn * NSPAN + nt * 32 + lm) * PITCH + 16 * (ks + 1) + lk]);
-                }
-                __builtin_amdgcn_sched_barrier(0);   // (the requests stay in front of this slice's products)
-#pragma unroll
-                for (int nt = 0; nt < NW_; nt++) b[nt] = bb[ks & 1][nt];
-            } else {
+            if (ks + 1 < KS / 16) {
 #pragma unroll
                 for (int nt = 0; nt < NW_; nt++)
-                    b[nt] = *reinterpret_cast<const h8 *>(&Bs[(wn * NSPAN + nt * 32 + lm) * PITCH + 16 * ks + lk]);
+                    b[(ks + 1) & 1][nt] = *reinterpret_cast<const h8 *>(&Bs[(nt * 32 + lm) * PITCH + 16 * (ks + 1) + lk]);
             }
+            __builtin_amdgcn_sched_barrier(0);   // (the requests stay in front of this slice's products)
 #pragma unroll
-            for (int mt = 0; mt < MW; mt++)
-#pragma unroll
-                for (int nt = 0; nt < NW_; nt++)
-                    // a superblock's first product starts from the constant zero: no pass over the accumulators to clear them
-                    Cp[mt][nt] = __builtin_amdgcn_mfma_f32_32x32x16_f16(ROWS ? from_bf16(A.a[mt][ks]) : A.a[mt][ks], b[nt], (g == 0 && ks == 0) ? kZero16 : Cp[mt][nt], 0, 0, 0);
+            for (int nt = 0; nt < NW_; nt++)
+                // a superblock's first product starts from the constant zero: no pass over the accumulators to clear them
+                Cp[nt] = __builtin_amdgcn_mfma_f32_32x32x16_f16(ROWS ? from_bf16(A.a[ks]) : A.a[ks], b[ks & 1][nt], (g == 0 && ks == 0) ? kZero16 : Cp[nt], 0, 0, 0);
             if (LO) {
 #pragma unroll
-                for (int mt = 0; mt < MW; mt++)
-#pragma unroll
-                    for (int nt = 0; nt < NW_; nt++)
-                        Cp[mt][nt] = __builtin_amdgcn_mfma_f32_32x32x16_f16(A.al[mt][ks], b[nt], Cp[mt][nt], 0, 0, 0);
+                for (int nt = 0; nt < NW_; nt++) Cp[nt] = __builtin_amdgcn_mfma_f32_32x32x16_f16(A.al[ks], b[ks & 1][nt], Cp[nt], 0, 0, 0);
             }
             // this k slice's fragments are spent: ask for the ones of AHEAD steps on right away
-#pragma unroll
-            for (int mt = 0; mt < MW; mt++) {
-                A.a[mt][ks] = afrag(mt, min(step + AHEAD, nsteps - 1), ks);
-                if (LO) A.al[mt][ks] = afrag_lo(mt, min(step + AHEAD, nsteps - 1), ks);
-            }
-            if (BPIPE) __builtin_amdgcn_sched_barrier(0);
+            A.a[ks] = afrag(min(step + AHEAD, nsteps - 1), ks);
+            if (LO) A.al[ks] = afrag_lo(min(step + AHEAD, nsteps - 1), ks);
+            __builtin_amdgcn_sched_barrier(0);
         }
         if (g == 3) {
-            // ---- end of the superblock: bias + mins through the short second product, then the row scale
-            const _Float16 *A2s = min_stage(sb), *B2s = A2s + TM * PITCH2;
+            // ---- end of the superblock: the row scale
             const float *dsc = dsc_stage(sb);
 #pragma unroll
-            for (int ks = 0; ks < (Q6 ? 0 : 2); ks++) {
-                h8 a[MW], b[NW_];
-#pragma unroll
-                for (int mt = 0; mt < MW; mt++)
-                    a[mt] = *reinterpret_cast<const h8 *>(&A2s[((wm * MW + mt) * 32 + lm) * PITCH2 + 16 * ks + lk]);
-#pragma unroll
-                for (int nt = 0; nt < NW_; nt++)
-                    b[nt] = *reinterpret_cast<const h8 *>(&B2s[(wn * NSPAN + nt * 32 + lm) * PITCH2 + 16 * ks + lk]);
-#pragma unroll
-                for (int mt = 0; mt < MW; mt++)
-#pragma unroll
-                    for (int nt = 0; nt < NW_; nt++)
-                        F[mt][nt] = __builtin_amdgcn_mfma_f32_32x32x16_f16(a[mt], b[nt], F[mt][nt], 0, 0, 0);
-            }
-#pragma unroll
             for (int nt = 0; nt < NW_; nt++) {
-                const float dn = dsc[wn * NSPAN + nt * 32 + lm];
+                const float dn = dsc[nt * 32 + lm];
 #pragma unroll
-                for (int mt = 0; mt < MW; mt++)
-#pragma unroll
-                    for (int i = 0; i < 16; i++)
-                        F[mt][nt][i] = fmaf(dn, Cp[mt][nt][i], F[mt][nt][i]);
+                for (int i = 0; i < 16; i++) F[nt][i] = fmaf(dn, Cp[nt][i], F[nt][i]);
             }
             if (CUT) {
-                static_assert(MW == 1, "one token tile per wave");
                 cut_left -= 1;
                 // (rows past the batch never end.  1 / s is a power of two: it can wait for the last slice)
                 const bool last = sb + 1 == nsb;
@@ -861,7 +695,7 @@ __global__ __launch_bounds__(kThreadsMM, TM == 64 ? 2 : 1) void q_mul_mm_kernel(
                     first >>= h4;
 #pragma unroll
                     for (int nt = 0; nt < NW_; nt++) {
-                        int r = r0 + wn * NSPAN + nt * 32 + lm;
+                        int r = r0 + nt * 32 + lm;
                         asm volatile("" : "+v"(r), "+v"(row));
                         if (r < p.rows) {
                             float *y = p.Y + (size_t)row * ystride + r;
@@ -877,7 +711,7 @@ __global__ __launch_bounds__(kThreadsMM, TM == 64 ? 2 : 1) void q_mul_mm_kernel(
 #pragma unroll
                                 for (int i = 0; i < 8; i++) {
                                     const int tr = 2 * i0 + 8 * (i / 4) + (i & 3);
-                                    sum[i] += F[0][nt][i0 + i];
+                                    sum[i] += F[nt][i0 + i];
                                     if (last) sum[i] *= p.inv_s[min(row + tr, p.batch - 1)];
                                     if (ends & (1u << tr)) y[(size_t)tr * ystride] = sum[i];
                                 }
@@ -885,7 +719,7 @@ __global__ __launch_bounds__(kThreadsMM, TM == 64 ? 2 : 1) void q_mul_mm_kernel(
                         }
 #pragma unroll
                         for (int i = 0; i < 16; i++)
-                            if (ends & (1u << (8 * (i / 4) + (i & 3)))) F[0][nt][i] = 0.f;
+                            if (ends & (1u << (8 * (i / 4) + (i & 3)))) F[nt][i] = 0.f;
                     }
                 }
             }
@@ -902,16 +736,14 @@ __global__ __launch_bounds__(kThreadsMM, TM == 64 ? 2 : 1) void q_mul_mm_kernel(
     if (CUT) return;   // (the last slices' ends have stored everything)
     // accumulator layout of the 32x32 tile: column = lane % 32, row = 8*(i/4) + 4*(lane/32) + i%4
 #pragma unroll
-    for (int mt = 0; mt < MW; mt++)
+    for (int nt = 0; nt < NW_; nt++) {
+        const int r = r0 + nt * 32 + lm;
 #pragma unroll
-        for (int nt = 0; nt < NW_; nt++) {
-            const int r = r0 + wn * NSPAN + nt * 32 + lm;
-#pragma unroll
-            for (int i = 0; i < 16; i++) {
-                const int t = t0 + (wm * MW + mt) * 32 + 8 * (i / 4) + 4 * (lane >> 5) + (i & 3);
-                if (t < p.batch && r < p.rows) p.Y[(size_t)t * ystride + r] = LO ? F[mt][nt][i] * p.inv_s[t] : F[mt][nt][i];
-            }
+        for (int i = 0; i < 16; i++) {
+            const int t = t0 + wm * 32 + 8 * (i / 4) + 4 * (lane >> 5) + (i & 3);
+            if (t < p.batch && r < p.rows) p.Y[(size_t)t * ystride + r] = LO ? F[nt][i] * p.inv_s[t] : F[nt][i];
         }
+    }
 }
 
 }  // namespace
@@ -1617,11 +1449,15 @@ constexpr int kSkinnyMaxBatch = 64;
 // k.variant: 1 the small-batch form; else 2 * the K slices where their sums are folded (0: one slice), and this bit where
 // the tile reads bf16 rows as they are
 constexpr int kRowsDirect = 1 << 24;
-// ... and this one where f32 rows of Q4_K take the tall shape of q4k_mm_rows_kernel
+// ... and this one where the rows of Q4_K take the tall shape of q4k_mm_rows_kernel
 constexpr int kTall = 1 << 25;
 using MmRowsTall = MmRows<2, 2, 1, 4>;      // 64 tokens x 256 rows
 using MmRowsShort = MmRows<1, 2, 1, 4>;     // 32 tokens x 256 rows: gate | up, and CUT
 using MmRowsSmall = MmRows<1, 1, 1, 4>;     // 32 tokens x 128 rows: the others
+// bf16 rows (mm_plan_bf16)
+using MmRowsBfTall = MmRows<4, 1, 1, 4, false>;   // 128 tokens x 128 rows
+using MmRowsBf = MmRows<2, 1, 1, 4, false>;       // 64 x 128
+static_assert(MmRowsBfTall::TN == BN && MmRowsBf::TN == BN, "mm_plan_bf16 counts rows of tiles so");
 
 // Workgroups of a launch of `tm` tokens and `tn` rows (gate | up: half as many of each) a workgroup
 dim3 mm_rows_grid(const ksh_kernel_desc &d, int tm, int tn, bool pair, int64_t ks)
@@ -1655,7 +1491,7 @@ int launch_mul_mm(const ksh_kernel &k, const LaunchArgs &a, hipStream_t st)
 {
     const int rows = (int)k.desc.dims[0], cols = (int)k.desc.dims[1], batch = (int)k.desc.dims[2];
     const bool f32x = k.desc.dtypes[1] == KSH_F32;
-    const size_t xf_halves = (size_t)((batch + 31) / 32 * 32) * cols, sx_halves = (size_t)(f32x ? (batch + 31) / 32 * 32 : batch) * (cols / 256) * 32;
+    const size_t xf_halves = (size_t)((batch + 31) / 32 * 32) * cols, sx_halves = (size_t)((batch + 31) / 32 * 32) * (cols / 256) * 32;
     _Float16 *Xf = (_Float16 *)k.scratch;
     _Float16 *SxA = Xf + xf_halves;
     _Float16 *Xf_lo = SxA + sx_halves, *SxA_lo = Xf_lo + xf_halves;     // f32 activations only
@@ -1687,7 +1523,11 @@ int launch_mul_mm(const ksh_kernel &k, const LaunchArgs &a, hipStream_t st)
     } else if (f32x && tile)
         hipLaunchKernelGGL(mm_prep_rows_kernel<0>, pg, pb, 0, st, (const float *)a.in[1], nullptr, nullptr, nullptr, nullptr, Xf, Xf_lo, SxA, SxA_lo, cols, 0.f, 0, inv_s);
     else if (f32x) hipLaunchKernelGGL(mm_prep_x_f32_kernel, dim3((n + 255) / 256), dim3(256), 0, st, (const float *)a.in[1], Xf, Xf_lo, SxA, SxA_lo, batch, cols);
-    else if (!rows_direct) hipLaunchKernelGGL(mm_prep_x_kernel, dim3(((batch + 31) / 32 * (cols / 32) + 3) / 4), dim3(256), 0, st, (const uint16_t *)a.in[1], Xf, SxA, batch, cols);
+    else if (!rows_direct) {
+        const dim3 xg(((batch + 31) / 32 * (cols / 32) + 3) / 4);
+        if (tile) hipLaunchKernelGGL(mm_prep_x_kernel<true>, xg, dim3(256), 0, st, (const uint16_t *)a.in[1], Xf, SxA, batch, cols);
+        else hipLaunchKernelGGL(mm_prep_x_kernel<false>, xg, dim3(256), 0, st, (const uint16_t *)a.in[1], Xf, SxA, batch, cols);
+    }
     MmParams p;
     p.W = (const uint8_t *)a.in[0];
     p.Y = (float *)a.out[0];
@@ -1711,16 +1551,18 @@ int launch_mul_mm(const ksh_kernel &k, const LaunchArgs &a, hipStream_t st)
         return e2 == hipSuccess ? 0 : hip_fail(e2, "mul_mm (small batch) launch");
     }
     const bool cut = k.desc.dims[6] == 2;
-    const int tm = k.info.lds_bytes == kLdsBytes64 ? 64 : 128;
-    const dim3 grid((batch + tm - 1) / tm, (rows + BN - 1) / BN + (rows1 + BN - 1) / BN + (rows2 + BN - 1) / BN);   // (q_mul_mm_kernel's)
+    const dim3 grid(k.info.grid[0], k.info.grid[1], k.info.grid[2]);
     p.Xf = rows_direct ? (const _Float16 *)a.in[1] : Xf;
     p.SxA = SxA; p.Xf_lo = Xf_lo; p.inv_s = inv_s;
     p.ksplit = 0; p.Y_parts = nullptr;
     p.cut_as = cut ? (const float *)a.in[k.info.n_inputs - 1] : nullptr;
     const bool q6 = k.desc.dtypes[0] == KSH_Q6K;
-    auto launch_rows = [&](dim3 g) {
-#define KSH_ROWS(S, ...) hipLaunchKernelGGL((q4k_mm_rows_kernel<S, __VA_ARGS__>), g, dim3(S::kThreads), S::kLds, st, p)
-        if (cut) KSH_ROWS(MmRowsShort, true, false);
+    auto launch_rows = [&]() {
+#define KSH_ROWS(S, ...) hipLaunchKernelGGL((q4k_mm_rows_kernel<S, __VA_ARGS__>), grid, dim3(S::kThreads), S::kLds, st, p)
+        if (!f32x) {
+            if (k.variant & kTall) KSH_ROWS(MmRowsBfTall, false, false);
+            else KSH_ROWS(MmRowsBf, false, false);
+        } else if (cut) KSH_ROWS(MmRowsShort, true, false);
         else if (k.variant & kTall) {
             if (pair) KSH_ROWS(MmRowsTall, false, true);
             else KSH_ROWS(MmRowsTall, false, false);
@@ -1728,17 +1570,13 @@ int launch_mul_mm(const ksh_kernel &k, const LaunchArgs &a, hipStream_t st)
         else KSH_ROWS(MmRowsSmall, false, false);
 #undef KSH_ROWS
     };
-    auto launch_tile = [&](dim3 g) {
-#define KSH_TILE(LDS, ...) hipLaunchKernelGGL((q_mul_mm_kernel<__VA_ARGS__>), g, dim3(kThreadsMM), LDS, st, p)
-        if (q6) {
-            if (cut) KSH_TILE(kLdsBytes, true, 128, true, true);
-            else if (f32x) KSH_TILE(kLdsBytes, true, 128, true);
-            else if (rows_direct) KSH_TILE(kLdsBytes, true, 128, false, false, true);
-            else KSH_TILE(kLdsBytes, true, 128, false);
-        } else if (f32x) {
-            launch_rows(dim3(k.info.grid[0], k.info.grid[1], g.z));
-        } else if (tm == 64) KSH_TILE(kLdsBytes64, false, 64, false);
-        else KSH_TILE(kLdsBytes, false, 128, false);
+    auto launch_tile = [&]() {
+#define KSH_TILE(...) hipLaunchKernelGGL((q6k_mul_mm_kernel<__VA_ARGS__>), grid, dim3(kThreadsMM), kLdsBytes, st, p)
+        if (!q6) launch_rows();
+        else if (cut) KSH_TILE(true, true);
+        else if (f32x) KSH_TILE(true);
+        else if (rows_direct) KSH_TILE(false, false, true);
+        else KSH_TILE(false);
 #undef KSH_TILE
     };
     if (slices) {
@@ -1747,7 +1585,7 @@ int launch_mul_mm(const ksh_kernel &k, const LaunchArgs &a, hipStream_t st)
         p.ksplit = ks;
         const bool unfolded = k.desc.dims[6] == 1;                    // the partial sums are the result: the reader adds them
         p.Y_parts = unfolded ? (float *)a.out[0] : (float *)((f32x ? SxA_lo : SxA) + sx_halves);     // (else behind the prepared activations)
-        launch_tile(dim3(grid.x, grid.y, ks));
+        launch_tile();
         hipError_t e3 = hipGetLastError();
         if (e3 != hipSuccess) return hip_fail(e3, "mul_mm (K slices) launch");
         if (unfolded) return 0;
@@ -1757,7 +1595,7 @@ int launch_mul_mm(const ksh_kernel &k, const LaunchArgs &a, hipStream_t st)
         e3 = hipGetLastError();
         return e3 == hipSuccess ? 0 : hip_fail(e3, "mul_mm fold launch");
     }
-    launch_tile(grid);
+    launch_tile();
     const hipError_t e = hipGetLastError();
     return e == hipSuccess ? 0 : hip_fail(e, "mul_mm launch");
 }
@@ -1844,7 +1682,7 @@ int bind_matvec_batch(ksh_kernel &k)
     }
     // f16 copy of X plus the min-term operand (32 halves per token and superblock)
     const size_t batch32 = (size_t)((batch + 31) / 32 * 32);
-    k.scratch_bytes = (batch32 * cols * 2 + (f32x ? batch32 : (size_t)batch) * (cols / 256) * 64) * (f32x ? 2 : 1);
+    k.scratch_bytes = (batch32 * cols * 2 + batch32 * (cols / 256) * 64) * (f32x ? 2 : 1);
     // schedule: nr0 = weight rows per workgroup.  32 = the small-batch form (Q4_K, up to 64 tokens: the default
     // there), 128 = the 128 x 128 tile.
     const uint32_t want = k.desc.sched.nr0;
@@ -1870,7 +1708,8 @@ int bind_matvec_batch(ksh_kernel &k)
     // the plan takes any count, and a schedule that a bound kernel has reported (it names the tile too) takes it again.
     const int64_t row_tiles = mm_row_tiles(k.desc), nsb = cols / 256;
     int64_t ks = cut ? 1 : k.desc.sched.k_split;
-    const bool reported = !f32x && want == BN && k.desc.sched.tg == kThreadsMM && k.desc.sched.lds_tile == KS && ks <= std::min<int64_t>(nsb, 64);
+    const bool reported = !f32x && want == BN && ((k.desc.sched.tg == kThreadsMM && k.desc.sched.lds_tile == KS) || (!q6 && k.desc.sched.tg == MmRowsBf::kThreads && k.desc.sched.lds_tile == 32)) &&
+                          ks <= std::min<int64_t>(nsb, 64);
     if (!cut && ks && nsb % ks && !reported) return set_error("matvec_batch: k_split=%lld does not divide the %lld superblocks of a row", (long long)ks, (long long)nsb);
     int tm = 0;
     if (f32x) {
@@ -1901,10 +1740,15 @@ int bind_matvec_batch(ksh_kernel &k)
         k.info.sched.tg = MmRowsTall::kThreads; k.info.sched.nsg = MmRowsTall::kThreads / 64; k.info.sched.nr0 = BN; k.info.sched.k_split = (uint32_t)ks; k.info.sched.lds_tile = 32;
         set_name(k, "mul_mm_q4k_%dx%dx32_f32x%s%s%s", tmr, tnr, z_form ? "_kz" : "", n_mat == 3 ? "_x3" : n_mat == 2 ? "_x2" : "",
                  prologue == 1 ? "_rms" : prologue == 2 ? "_addrms" : prologue == 3 ? "_gelu" : "");
+    } else if (!q6) {
+        if (tm == MmRowsBfTall::TM) k.variant |= kTall;
+        set_launch(k, (uint32_t)((batch + tm - 1) / tm), (uint32_t)row_tiles, z_form ? (uint32_t)ks : 1, MmRowsBf::kThreads, (uint32_t)(tm == MmRowsBfTall::TM ? MmRowsBfTall::kLds : MmRowsBf::kLds));
+        k.info.sched.tg = MmRowsBf::kThreads; k.info.sched.nsg = MmRowsBf::kThreads / 64; k.info.sched.nr0 = BN; k.info.sched.k_split = (uint32_t)ks; k.info.sched.lds_tile = 32;
+        set_name(k, "mul_mm_q4k_%dx%dx32%s%s", tm, BN, z_form ? "_kz" : "", n_mat == 3 ? "_x3" : n_mat == 2 ? "_x2" : "");
     } else {
-        set_launch(k, (uint32_t)((batch + tm - 1) / tm), (uint32_t)row_tiles, z_form ? (uint32_t)ks : 1, kThreadsMM, (uint32_t)(tm == 64 ? kLdsBytes64 : kLdsBytes));
+        set_launch(k, (uint32_t)((batch + tm - 1) / tm), (uint32_t)row_tiles, z_form ? (uint32_t)ks : 1, kThreadsMM, (uint32_t)kLdsBytes);
         k.info.sched.tg = kThreadsMM; k.info.sched.nsg = kThreadsMM / 64; k.info.sched.nr0 = BN; k.info.sched.k_split = (uint32_t)ks; k.info.sched.lds_tile = KS;
-        set_name(k, "mul_mm_%s_%dx%dx%d%s%s%s%s", q6 ? "q6k" : "q4k", BM, BN, KS, f32x ? "_f32x" : "", z_form ? "_kz" : "", n_mat == 3 ? "_x3" : n_mat == 2 ? "_x2" : "",
+        set_name(k, "mul_mm_q6k_%dx%dx%d%s%s%s%s", BM, BN, KS, f32x ? "_f32x" : "", z_form ? "_kz" : "", n_mat == 3 ? "_x3" : n_mat == 2 ? "_x2" : "",
                  prologue == 1 ? "_rms" : prologue == 2 ? "_addrms" : prologue == 3 ? "_gelu" : "");
     }
     if (pair) { char nm[64]; snprintf(nm, sizeof(nm), "%s", k.info.name); set_name(k, "%s_gate_up", nm); }

@@ -1,4 +1,5 @@
-// The prompt GEMM over Q4_K weights and f32 rows (two f16 parts at the row's own scale, mm_prep_rows_kernel): every wave
+// The prompt GEMM over Q4_K weights and f32 rows (two f16 parts at the row's own scale, mm_prep_rows_kernel) or bf16 rows (one
+// part, mm_prep_x_kernel): every wave
 // converts its own weights in registers and multiplies them with fragments that the workgroup shares in LDS.
 //
 // What bounds it: the matrix pipe and the chip's power.  With two workgroups on every compute unit the pipe is busy 60 % of the
@@ -11,8 +12,13 @@
 // 252 -> 208, 4096 x 1536 82 -> 60; (32 x 32) 952 tokens, 1536 x 12288 152 -> 134, 700 tokens, 2048 x 8192 99 -> 87; rows cut
 // as in launches of their own, 1989 tokens, 1536 x 12288 285 -> 245.
 //
-// The sums are those of that tile (q_mul_mm_kernel's, which other types still take), instruction by instruction, so results have
-// its bits: per 16 columns the hi and the lo part against the same weights into a superblock's own accumulator, then F = (bias
+// With bf16 rows there are half as many matrix instructions to a converted weight, and a wave has 64 tokens x 32 rows, or 128 x
+// 32 where the chip is full: 2048 tokens, 12288 x 4096 257 -> 221 us, 300 tokens, 12288 x 1536 29.7 -> 24.1, 65 tokens, 12288 x
+// 8192 46 -> 40; 512 tokens, 8192 x 2048 30.5 -> 30.2, where the vector instructions (318 a superblock and wave) and the matrix
+// instructions fill a SIMD's time one after the other (20 and 18 thousand of 39 thousand cycles; neither fragments read two
+// units ahead nor eight half steps on their way change it).
+//
+// A product's order is fixed, so its bits do not depend on the shape that does it: per 16 columns the hi and the lo part against the same weights into a superblock's own accumulator, then F = (bias
 // and mins, two short products) + F and F = d * C + F.
 //
 // CUT: the rows belong to prompts that would each have had a launch of their own, whose K slices depend on its length; the
@@ -34,12 +40,13 @@ struct MmRows {
     static constexpr bool LO = LO_;
     static constexpr int TT = WM * MT, TM = 32 * TT, TN = 32 * WN * NT, kThreads = 64 * WM * WN;
     static constexpr int TF = TT * PARTS / 2;         // fragments of a half step that a wave fetches
+    static constexpr int SUMS = TT == 4 ? 2 : 1;      // ... and fragments of a superblock's sums
     static constexpr int kStage = TT * 2 * PARTS * 1024;   // bytes of the fragments of 32 columns: [token tile][hi | lo][k slice][lane][16]
     static constexpr int kSums = TT * 2 * 1024;       // bytes of a superblock's sums of x: [token tile][k slice][lane][16]
     static constexpr int kTile = 5 * 1024;            // bytes of a superblock of 32 weight rows: [row][144], whole kilobytes
     static constexpr int kInv = 256;                  // the tokens' 1 / s
     static constexpr int kLds = 4 * kStage + kSums + WM * WN * NT * kTile + kInv;
-    static_assert(WM * WN == 4 && TT <= 2 && MT * PARTS >= 2 && NT <= 2, "a wave fetches TF fragments of a half step, from one part of one token tile");
+    static_assert(WM * WN == 4 && TT * PARTS <= 4 && MT * PARTS >= 2 && NT <= 2, "a wave fetches TF fragments of a half step, from one part of one token tile");
 };
 
 // Memory operations that the compiler does not count: it would wait for all that is on its way into LDS in front of every read
@@ -92,7 +99,7 @@ __global__ __launch_bounds__(S::kThreads, 2) void q4k_mm_rows_kernel(MmParams p)
     // 1536, gate | up 312 us instead of 294.)
     const uint32_t l0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) uint8_t *)lds_rows;
     constexpr uint32_t kAtSums = 4 * S::kStage, kAtW = kAtSums + S::kSums, kAtInv = kAtW + 4 * NT * S::kTile;
-    const int f0 = wave * TF, ntt = (p.batch + 31) / 32, fsum = wave % (2 * TT);
+    const int f0 = wave * TF, ntt = (p.batch + 31) / 32, fsum = wave * S::SUMS % (2 * TT);
     const uint8_t *xsrc = reinterpret_cast<const uint8_t *>(S::LO && ((f0 >> 1) & 1) ? p.Xf_lo : p.Xf) +
                           ((size_t)min(t0 / 32 + f0 / (2 * PARTS), ntt - 1) * nsb_row + sb0) * 16384 + (f0 & 1) * 1024;
     const uint8_t *sxsrc = reinterpret_cast<const uint8_t *>(p.SxA) + (((size_t)min(t0 / 32 + (fsum >> 1), ntt - 1) * nsb_row + sb0) * 2 + (fsum & 1)) * 1024;
@@ -100,7 +107,7 @@ __global__ __launch_bounds__(S::kThreads, 2) void q4k_mm_rows_kernel(MmParams p)
     auto ask_rows = [&](int hs, int stage, int i) __attribute__((always_inline)) {
         to_lds16(xsrc + (size_t)min(hs, 8 * nsb - 1) * 2048 + i * 1024, lane16, l0 + (uint32_t)(stage * S::kStage + (f0 + i) * 1024));
     };
-    auto ask_sums = [&](int sb) __attribute__((always_inline)) { to_lds16(sxsrc + (size_t)min(sb, nsb - 1) * 2048, lane16, l0 + kAtSums + (uint32_t)(fsum * 1024)); };
+    auto ask_sums = [&](int sb, int i) __attribute__((always_inline)) { to_lds16(sxsrc + (size_t)min(sb, nsb - 1) * 2048 + i * 1024, lane16, l0 + kAtSums + (uint32_t)((fsum + i) * 1024)); };
     const size_t row_bytes = (size_t)nsb_row * 144;
     const uint8_t *wbase[2];
     wbase[0] = p.W + (size_t)r0 * row_bytes + (size_t)sb0 * 144;
@@ -215,9 +222,9 @@ __global__ __launch_bounds__(S::kThreads, 2) void q4k_mm_rows_kernel(MmParams p)
     const uint32_t lh = lw + 144u * (uint32_t)lm, lq = lh + 16u * (uint32_t)h;
     auto read_rows = [&](auto htag, auto utag, h8 (&v)[2]) __attribute__((always_inline)) {   // of unit U of a half step
         constexpr int hs = decltype(htag)::value & 3, u = decltype(utag)::value;
-        constexpr int off = hs * S::kStage + (U == 4 ? (u >> 1) * 1024 + (u & 1) * 2048 : u * 1024);
+        constexpr int off = hs * S::kStage + (U == 4 ? (u >> 1) * 1024 + (u & 1) * (PARTS == 2 ? 2048 : 2 * kTokens) : u * 1024);
         lds_ask<off>(v[0], la);
-        lds_ask<off + (MT == 2 ? kTokens : 2048)>(v[1], la);
+        lds_ask<off + (MT == 1 ? 2048 : kTokens)>(v[1], la);
     };
     auto read_group = [&](auto gtag) __attribute__((always_inline)) {
         constexpr int o = 16 + 32 * decltype(gtag)::value;
@@ -240,7 +247,8 @@ __global__ __launch_bounds__(S::kThreads, 2) void q4k_mm_rows_kernel(MmParams p)
     if (S::LO) to_lds4(reinterpret_cast<const uint8_t *>(p.inv_s), 4u * (uint32_t)min(t0 + lane, p.batch - 1), l0 + kAtInv);   // (every wave the same)
 #pragma unroll
     for (int j = 0; j < 5 * NT; j++) ask_weights(0, j);
-    ask_sums(0);
+#pragma unroll
+    for (int i = 0; i < S::SUMS; i++) ask_sums(0, i);
 #pragma unroll
     for (int hs = 0; hs < 3; hs++)
 #pragma unroll
@@ -271,7 +279,7 @@ __global__ __launch_bounds__(S::kThreads, 2) void q4k_mm_rows_kernel(MmParams p)
         constexpr bool last = place == U - 1;
         // Memory operations of a half step: its first units ask for the fragments of three half steps on; the last two (the
         // last, U = 2) of half steps 0 .. 4 for a piece of the next superblock's weights a tile, of half step 5 for its sums.
-        constexpr auto extra = [](int hh) { return hh < 5 ? NT : hh == 5 ? 1 : 0; };
+        constexpr auto extra = [](int hh) { return hh < 5 ? NT : hh == 5 ? S::SUMS : 0; };
         __builtin_amdgcn_sched_barrier(0);
         constexpr bool opens = half == 0 && place == 0;
         if constexpr (opens && CUT) {
@@ -283,14 +291,14 @@ __global__ __launch_bounds__(S::kThreads, 2) void q4k_mm_rows_kernel(MmParams p)
                 cut_ends();
             }
         }
-        constexpr int mins = U == 4 ? (g == 1 && part == 0 && ks < 2 ? ks : -1) : (g == 1 && ks >= 1 && ks <= MT ? ks - 1 : -1);
+        constexpr int mins = MT == 4 ? (half == 2 ? place : -1) : U == 4 ? (g == 1 && part == 0 && ks < 2 ? ks : -1) : (g == 1 && ks >= 1 && ks <= MT ? ks - 1 : -1);
         constexpr bool take0 = half == 7 && place == 0, take3 = half == 7 && last;
         // (behind the first matrix instruction, whose 32 cycles cover part of it: a request to memory takes some 40 to issue)
         auto ask = [&]() __attribute__((always_inline)) {
             if constexpr (last) {
                 // every wave has this half step's fragments in registers; the next one's, which this wave has asked for two half
-                // steps ago, are in LDS (and at the end of half step 6 the weights, which are 1 + 2 TF operations back)
-                constexpr int pending = half == 6 ? 1 + 2 * TF : extra((half + 6) & 7) + TF + extra((half + 7) & 7) + TF + (U == 4 && (half == 5 || (half < 5 && NT == 2)) ? 1 : 0);
+                // steps ago, are in LDS (and at the end of half step 6 the weights, which are SUMS + 2 TF operations back)
+                constexpr int pending = half == 6 ? S::SUMS + 2 * TF : extra((half + 6) & 7) + TF + extra((half + 7) & 7) + TF + (U == 4 && (half == 5 || (half < 5 && NT == 2)) ? 1 : 0);
                 asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" ::"n"(pending) : "memory");
             }
             read_rows(std::integral_constant<int, (last ? half + 1 : half) & 7>{}, std::integral_constant<int, last ? 0 : place + 1>{}, a[set ^ 1]);
@@ -312,14 +320,14 @@ __global__ __launch_bounds__(S::kThreads, 2) void q4k_mm_rows_kernel(MmParams p)
 #pragma unroll
                 for (int i = 0; i < NT; i++) ask_weights(sb + 1, NT * half + i);
             }
-            if constexpr (place == U / 2 && half == 5) ask_sums(sb + 1);
+            if constexpr (place >= U / 2 && place < U / 2 + S::SUMS && half == 5) ask_sums(sb + 1, place - U / 2);
         };
 #pragma unroll
         for (int i = 0; i < 2; i++)
 #pragma unroll
             for (int nt = 0; nt < NT; nt++) {
-                const int mt = MT == 2 ? i : 0;
-                const bool first = opens && (MT == 2 || i == 0);   // (a superblock's first product starts from the constant zero)
+                const int mt = MT == 4 ? 2 * part + i : MT == 2 ? i : 0;
+                const bool first = MT == 4 ? half == 0 && ks == 0 : opens && (MT == 2 || i == 0);   // (a superblock's first product starts from the constant zero)
                 if (first && !CUT) fold(mt, nt);
                 C[mt][nt] = __builtin_amdgcn_mfma_f32_32x32x16_f16(a[set][i], b[ks & 1][nt], first ? kZero16 : C[mt][nt], 0, 0, 0);
                 if (i == 0 && nt == 0) {

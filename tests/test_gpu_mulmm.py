@@ -369,6 +369,27 @@ def test_mul_mm_f32_rows_at_the_edges_of_its_tiles(ctx, rows, batch, cols, mode,
     assert shape in k.name, k.name
 
 
+@pytest.mark.parametrize("rows,batch,cols,ks,shape", [
+    (1, 2, 256, 1, "64x128"), (129, 65, 768, 1, "64x128"), (257, 63, 7936, 7, "64x128"), (127, 193, 2816, 11, "64x128"),
+    (8193, 1025, 4096, 1, "128x128"), (4095, 1023, 1280, 5, "128x128")])
+def test_mul_mm_bf16_rows_at_the_edges_of_its_tiles(ctx, rows, batch, cols, ks, shape):
+    """Both shapes of the bf16 rows' kernel where they can go wrong: one superblock, a row or a token past a tile or short of
+    it, slices of unequal length and of one superblock.  Against float64: bf16 values of normal size and codes times scales
+    are exact in f16, the sums of x hold 22 bits, sums are f32 (2e-5, as for f32 rows)."""
+    w = synth.q4k_blocks(rows * cols // 256, 730)
+    xf, xb = synth.bf16_round(synth.normal_f32(batch * cols, 731))
+    xs = xf.reshape(batch, cols)
+    k = ctx.compile(hip.make_desc(hip.Kind.MATVEC_BATCH, (rows, cols, batch), (DType.Q4K, DType.BF16, DType.F32), (),
+                                  dict(nr0=128, tg=256, lds_tile=32, k_split=ks)))
+    assert f"_{shape}x32" in k.name and k.info.sched.k_split == ks
+    y = ctx.buffer_empty_f32(batch * rows)
+    ctx.encode_multi(k, [ctx.buffer_bytes(w), ctx.buffer_bytes(xb)], [y])
+    ctx.synchronize()
+    got = ctx.read_f32(y, batch * rows).reshape(batch, rows)
+    for t in sorted({0, 1, 31, 32, 62, 63, 64, 127, 128, batch - 2, batch - 1} & set(range(batch))):
+        assert float(rel_err(got[t], oracle.matvec_f64(oracle.Q4K, w, rows, cols, xs[t])).max()) <= 2e-5, t
+
+
 @pytest.mark.parametrize("rows,batch,prologue", [(31, 33, 0), (97, 64, 2), (200, 130, 0), (4130, 1000, 2)])
 def test_mul_mm_f32_gate_up_pair(ctx, rows, batch, prologue):
     """dims[6] = 3: gelu(W x) * (W1 x) from one launch is the two matrices' products and KSH_GELU_MUL (64 rows of each
