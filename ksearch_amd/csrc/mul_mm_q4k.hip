@@ -377,6 +377,9 @@ struct MmParams {
     const float *inv_s;
     // the kernel's CUT form: per row, the tokens of the launch whose K slices its sums are to be cut into
     const float *cut_as;
+    // q4k_mm_rows_kernel's numbering of the workgroups: how many there are, in x and in y, ceil(2^32 / gx) and ceil(2^32 / gy)
+    // (exact quotients where wgs * gx and wgs * gy stay below 2^32; wgs = 0: as the launch numbers them)
+    uint32_t wgs, gx, gy, per_gx, per_gy;
 };
 
 // F32 activations: the tokens and weight rows (BN) of the tiles that the rule of the K slices counts.  How a row's sum is cut
@@ -1557,6 +1560,10 @@ int launch_mul_mm(const ksh_kernel &k, const LaunchArgs &a, hipStream_t st)
     p.ksplit = 0; p.Y_parts = nullptr;
     p.cut_as = cut ? (const float *)a.in[k.info.n_inputs - 1] : nullptr;
     const bool q6 = k.desc.dtypes[0] == KSH_Q6K;
+    const uint64_t wgs = (uint64_t)grid.x * grid.y * grid.z;
+    p.wgs = wgs * std::max(grid.x, grid.y) < (1ull << 32) && grid.x > 1 && grid.y > 1 ? (uint32_t)wgs : 0;
+    p.gx = grid.x; p.gy = grid.y;
+    p.per_gx = (uint32_t)(((1ull << 32) + grid.x - 1) / grid.x); p.per_gy = (uint32_t)(((1ull << 32) + grid.y - 1) / grid.y);
     auto launch_rows = [&]() {
 #define KSH_ROWS(S, ...) hipLaunchKernelGGL((q4k_mm_rows_kernel<S, __VA_ARGS__>), grid, dim3(S::kThreads), S::kLds, st, p)
         if (!f32x) {

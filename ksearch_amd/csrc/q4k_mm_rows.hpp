@@ -40,6 +40,7 @@ struct MmRows {
     static constexpr bool LO = LO_;
     static constexpr int TT = WM * MT, TM = 32 * TT, TN = 32 * WN * NT, kThreads = 64 * WM * WN;
     static constexpr int TF = TT * PARTS / 2;         // fragments of a half step that a wave fetches
+    static constexpr bool kNeighbours = NT == 1 && MT <= 2;   // an L2's workgroups are neighbours
     static constexpr int SUMS = TT == 4 ? 2 : 1;      // ... and fragments of a superblock's sums
     static constexpr int kStage = TT * 2 * PARTS * 1024;   // bytes of the fragments of 32 columns: [token tile][hi | lo][k slice][lane][16]
     static constexpr int kSums = TT * 2 * 1024;       // bytes of a superblock's sums of x: [token tile][k slice][lane][16]
@@ -72,21 +73,38 @@ __global__ __launch_bounds__(S::kThreads, 2) void q4k_mm_rows_kernel(MmParams p)
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int wm = wave / S::WN, wn = wave % S::WN, lm = lane & 31, h = lane >> 5;
 
+    // Shapes for launches that do not fill the chip: consecutive workgroups go round the eight L2s, so as they are numbered each
+    // L2 would fetch most of X and of W.  Here an L2's workgroups are neighbours, all weight rows of a few token tiles (and of a
+    // K slice): 952 tokens, 1536 x 2048 30.6 -> 28.9 us, 700 tokens, 2048 x 2048 29.6 -> 27.9, 2048 tokens, 2560 x 1536 52.2 -> 49.6;
+    // bf16, 700 tokens, 2048 x 8192 53 -> 47, though 333 tokens, 1536 x 6144 24.1 -> 25.5.  Where the chip is full the walk along the
+    // tokens is the better one (2048 tokens, gate | up 12288 x 1536 312 or 318, bf16, 12288 x 4096 221 or 228).
+    // (The quotients come from the host's reciprocals: divided here, they are 0.5 us in front of the first request.)
+    uint32_t bx = blockIdx.x, by = blockIdx.y, bz = blockIdx.z;
+    if constexpr (S::kNeighbours) {
+        if (p.wgs) {
+            const uint32_t n = bx + p.gx * (by + p.gy * bz), l2 = n & 7;
+            const uint32_t at = l2 * (p.wgs >> 3) + min(l2, p.wgs & 7) + (n >> 3), column = __umulhi(at, p.per_gy);
+            bz = __umulhi(column, p.per_gx);
+            by = at - column * p.gy;
+            bx = column - bz * p.gx;
+        }
+    }
+
     // which matrix this row tile belongs to (the copy of the arguments is this workgroup's own)
-    int by = blockIdx.y, ycol = 0;
+    int ycol = 0;
     const int rows_all = p.rows + p.rows1 + p.rows2;
     const int rows_of[3] = {p.rows, p.rows1, p.rows2};
     if (!PAIR && p.rows1) {
         const int ty0 = (p.rows + S::TN - 1) / S::TN, ty1 = (p.rows1 + S::TN - 1) / S::TN;
-        if (by >= ty0 + ty1) { by -= ty0 + ty1; ycol = p.rows + p.rows1; p.W = p.W2; p.Y = p.Y2; p.rows = p.rows2; }
-        else if (by >= ty0) { by -= ty0; ycol = p.rows; p.W = p.W1; p.Y = p.Y1; p.rows = p.rows1; }
+        if ((int)by >= ty0 + ty1) { by -= ty0 + ty1; ycol = p.rows + p.rows1; p.W = p.W2; p.Y = p.Y2; p.rows = p.rows2; }
+        else if ((int)by >= ty0) { by -= ty0; ycol = p.rows; p.W = p.W1; p.Y = p.Y1; p.rows = p.rows1; }
     }
-    const int t0 = blockIdx.x * S::TM, r0 = by * (PAIR ? S::TN / 2 : S::TN);
+    const int t0 = (int)bx * S::TM, r0 = (int)by * (PAIR ? S::TN / 2 : S::TN);
     const int nsb_row = p.cols / 256;
     int nsb = nsb_row, sb0 = 0;
     size_t ystride = (size_t)p.rows;
     if (p.ksplit) {
-        const int slice = blockIdx.z;
+        const int slice = (int)bz;
         sb0 = nsb_row * slice / p.ksplit;
         nsb = nsb_row * (slice + 1) / p.ksplit - sb0;
         p.Y = p.Y_parts + (size_t)slice * p.batch * rows_all + ycol;   // partial sums: all matrices' columns side by side
