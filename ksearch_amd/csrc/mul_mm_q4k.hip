@@ -405,33 +405,36 @@ __host__ __device__ constexpr int mm_k_slices(bool q6, int row_tiles, int nsb, i
 
 // Bf16 activations: token tile and K slices (of any number of superblocks) by what the launches are made of, in us, fitted to
 // 256 .. 12288 rows of 512 .. 8192 columns, 2 .. 2048 tokens, every slice count:
-//   Q6_K, a round of 128-token tiles (one workgroup a compute unit)  5 + 2.4 per superblock of the slice; the fold 2.5 + the
-//                    partial sums, written and read, at 4 TB/s
-//   Q4_K             with its preparation, 64 tokens a workgroup (128): 5.2 (6.4) + 0.6 per round of workgroups over the compute
-//                    units + what rows and results cost; a superblock 1.45 in one round, 1.7 in two, 0.73 a round in more (1.87,
-//                    1.31 a round), and up to 36 % (16 %) more as the chip fills; the fold 4.2 (4.6) + 1.4 per million partial sums
-// Its choice is on average within 1 % of the best (tile, slices) at those shapes, within 8 % at all.  Q6_K, 333 tokens, 1536 x
-// 6144: four -> six slices 29.8 -> 25.4 us.  Q4_K: 2048 tokens of 12288 x 4096 262 us with 64 tokens a workgroup, 227 with 128; 300
-// tokens of 12288 x 1536 24.4 or 30.8; 65 tokens of 12288 x 8192 47 us in two slices of 64 tokens, 40 in eight of 128.
+//   preparation (Q4_K), launches, what rows and results cost; per round of workgroups over the compute units; per superblock of
+//   the slice in one round, in two, in more (each), more as the chip fills; the fold
+// The choice is on average within 1 % of the best (tile, slices) at those shapes, within 10 % at all.  Q4_K: 2048 tokens of 12288 x
+// 4096 262 us with 64 tokens a workgroup, 227 with 128; 300 tokens of 12288 x 1536 24.4 or 30.8; 65 tokens of 12288 x 8192 47 us in
+// two slices of 64 tokens, 40 in eight of 128.  Q6_K (32 or 64 tokens: q6k_mm_rows_kernel; 128: q6k_mul_mm_kernel): 8 tokens of 1536 x 6144
+// 10.7 / 11.9 / 13.2 us, 50 of 4096 x 6144 19.6 / 18.0 / 20.9, 333 of 1536 x 6144 38 / 29 / 26.
 struct MmPlan {
     int tm, ks;
     float us;
 };
 MmPlan mm_plan_bf16(bool q6, int row_tiles, int nsb, int64_t batch, int64_t rows_all, int ks_given)
 {
+    struct Cost {
+        int tm;
+        float launch, round, one, two, more, fill, out, fold, part;
+    };
+    constexpr Cost kQ4[] = {{64, 5.2f, 0.6f, 1.45f, 1.7f, 0.73f, 0.18f, 1.4f, 4.2f, 1.4f}, {128, 6.4f, 0.6f, 1.87f, 2.62f, 1.31f, 0.08f, 2.f, 4.6f, 1.4f}};
+    constexpr Cost kQ6[] = {{32, 2.65f, 0.75f, 2.2f, 3.3f, 1.36f, 0.084f, 1.44f, 2.35f, 0.9f}, {64, 2.8f, 1.1f, 2.5f, 3.65f, 1.6f, 0.124f, 1.23f, 2.4f, 1.16f},
+                            {128, 2.3f, 2.57f, 2.7f, 5.4f, 2.7f, 0.058f, 2.25f, 2.8f, 1.3f}};
     MmPlan best{128, 1, 1e30f};
     const int ks_max = std::min(nsb, 64);
     const float m = (float)(batch * rows_all) * 1e-6f;
-    for (int tm = q6 ? 128 : 64; tm <= 128; tm += 64)
+    for (const Cost *c = q6 ? kQ6 : kQ4, *end = c + (q6 ? 3 : 2); c < end; c++)
         for (int ks = ks_given ? ks_given : 1; ks <= (ks_given ? ks_given : ks_max); ks++) {
-            const int64_t wgs = (batch + tm - 1) / tm * row_tiles * ks;
-            const float sb = (float)((nsb + ks - 1) / ks), w = (float)wgs / 256.f, rounds = (float)((wgs + 255) / 256);
-            float us;
-            if (q6) us = rounds * (5.f + 2.4f * sb) + (ks > 1 ? 2.5f + 2.f * (float)ks * m : 0.f);
-            else if (tm == 64) us = 5.2f + 1.4f * m + (rounds <= 1.f ? 1.45f : rounds <= 2.f ? 1.7f : 0.73f * rounds) * (1.f + 0.18f * std::min(w, 2.f)) * sb + (ks > 1 ? 4.2f + 1.4f * (float)ks * m : 0.f);
-            else us = 6.4f + 2.f * m + (rounds <= 1.f ? 1.87f : 1.31f * rounds) * (1.f + 0.08f * std::min(w, 2.f)) * sb + (ks > 1 ? 4.6f + 1.4f * (float)ks * m : 0.f);
-            if (!q6) us += 0.6f * rounds + (float)(batch * nsb) * 256e-6f;
-            if (us < best.us) best = MmPlan{tm, ks, us};
+            const int64_t wgs = (batch + c->tm - 1) / c->tm * row_tiles * ks;
+            const float sb = (float)((nsb + ks - 1) / ks), w = std::min((float)wgs / 256.f, 2.f), rounds = (float)((wgs + 255) / 256);
+            const float each = rounds <= 1.f ? c->one : rounds <= 2.f ? c->two : c->more * rounds;
+            const float us = c->launch + c->round * rounds + each * (1.f + c->fill * w) * sb + c->out * m + (q6 ? 0.f : (float)(batch * nsb) * 256e-6f) +
+                             (ks > 1 ? c->fold + c->part * (float)ks * m : 0.f);
+            if (us < best.us) best = MmPlan{c->tm, ks, us};
         }
     return best;
 }
@@ -753,6 +756,7 @@ __global__ __launch_bounds__(kThreadsMM, 1) void q6k_mul_mm_kernel(MmParams p)
 }  // namespace ksh
 
 #include "q4k_mm_rows.hpp"
+#include "q6k_mm_rows.hpp"
 
 namespace ksh {
 namespace {
@@ -1452,8 +1456,9 @@ constexpr int kSkinnyMaxBatch = 64;
 // k.variant: 1 the small-batch form; else 2 * the K slices where their sums are folded (0: one slice), and this bit where
 // the tile reads bf16 rows as they are
 constexpr int kRowsDirect = 1 << 24;
-// ... and this one where the rows of Q4_K take the tall shape of q4k_mm_rows_kernel
+// ... and this one where the rows of Q4_K take the tall shape of q4k_mm_rows_kernel (of Q6_K, of q6k_mm_rows_kernel)
 constexpr int kTall = 1 << 25;
+constexpr int kRows6 = 1 << 26;             // bf16 rows of Q6_K: q6k_mm_rows_kernel
 using MmRowsTall = MmRows<2, 2, 1, 4>;      // 64 tokens x 256 rows
 using MmRowsShort = MmRows<1, 2, 1, 4>;     // 32 tokens x 256 rows: gate | up, and CUT
 using MmRowsSmall = MmRows<1, 1, 1, 4>;     // 32 tokens x 128 rows: the others
@@ -1508,8 +1513,8 @@ int launch_mul_mm(const ksh_kernel &k, const LaunchArgs &a, hipStream_t st)
     // columns: 768 threads) where the tile keeps them
     const int octets = cols / 8, pb1 = (octets + 63) / 64 * 64;
     const dim3 pg((unsigned)batch), pb((unsigned)std::min(pb1 > 1024 && inv_s ? (octets / 2 + 63) / 64 * 64 : pb1, 1024));
-    const bool rows_direct = (k.variant & kRowsDirect) != 0;
-    const int slices = (k.variant & ~(kRowsDirect | kTall)) >> 1;                  // 0: no fold
+    const bool rows_direct = (k.variant & (kRowsDirect | kRows6)) != 0;
+    const int slices = (k.variant & ~(kRowsDirect | kTall | kRows6)) >> 1;                  // 0: no fold
     if (prologue) {
         // the rows' producer runs inside the preparation: in = W, X, [W1, W2,] then the prologue's operands
         const int xs = (int)k.desc.dims[7];
@@ -1582,6 +1587,10 @@ int launch_mul_mm(const ksh_kernel &k, const LaunchArgs &a, hipStream_t st)
         if (!q6) launch_rows();
         else if (cut) KSH_TILE(true, true);
         else if (f32x) KSH_TILE(true);
+        else if (k.variant & kRows6) {
+            if (k.variant & kTall) hipLaunchKernelGGL(q6k_mm_rows_kernel<2>, grid, dim3(Mm6Rows<2>::kThreads), Mm6Rows<2>::kLds, st, p);
+            else hipLaunchKernelGGL(q6k_mm_rows_kernel<1>, grid, dim3(Mm6Rows<1>::kThreads), Mm6Rows<1>::kLds, st, p);
+        }
         else if (rows_direct) KSH_TILE(false, false, true);
         else KSH_TILE(false);
 #undef KSH_TILE
@@ -1715,7 +1724,7 @@ int bind_matvec_batch(ksh_kernel &k)
     // the plan takes any count, and a schedule that a bound kernel has reported (it names the tile too) takes it again.
     const int64_t row_tiles = mm_row_tiles(k.desc), nsb = cols / 256;
     int64_t ks = cut ? 1 : k.desc.sched.k_split;
-    const bool reported = !f32x && want == BN && ((k.desc.sched.tg == kThreadsMM && k.desc.sched.lds_tile == KS) || (!q6 && k.desc.sched.tg == MmRowsBf::kThreads && k.desc.sched.lds_tile == 32)) &&
+    const bool reported = !f32x && want == BN && ((k.desc.sched.tg == kThreadsMM && k.desc.sched.lds_tile == KS) || (k.desc.sched.tg == MmRowsBf::kThreads && k.desc.sched.lds_tile == (q6 ? KS : 32))) &&
                           ks <= std::min<int64_t>(nsb, 64);
     if (!cut && ks && nsb % ks && !reported) return set_error("matvec_batch: k_split=%lld does not divide the %lld superblocks of a row", (long long)ks, (long long)nsb);
     int tm = 0;
@@ -1729,7 +1738,8 @@ int bind_matvec_batch(ksh_kernel &k)
     }
     const bool z_form = unfolded || ks > 1;
     k.variant = z_form ? (int)(ks << 1) : 0;
-    if (!f32x && q6 && mm_rows_direct((batch + tm - 1) / tm * row_tiles * ks, (int)((nsb + ks - 1) / ks), batch, cols)) k.variant |= kRowsDirect;
+    if (!f32x && q6 && tm < BM) k.variant |= kRows6 | (tm == Mm6Rows<2>::TM ? kTall : 0);
+    else if (!f32x && q6 && mm_rows_direct((batch + tm - 1) / tm * row_tiles * ks, (int)((nsb + ks - 1) / ks), batch, cols)) k.variant |= kRowsDirect;
     if (z_form && !unfolded) k.scratch_bytes += (size_t)ks * batch * rows_all * 4;
     if (unfolded) {
         const int keep = prologue == 2 ? 1 : 0;                       // (the add-then-norm prologue's x_new stays an output)
@@ -1752,6 +1762,11 @@ int bind_matvec_batch(ksh_kernel &k)
         set_launch(k, (uint32_t)((batch + tm - 1) / tm), (uint32_t)row_tiles, z_form ? (uint32_t)ks : 1, MmRowsBf::kThreads, (uint32_t)(tm == MmRowsBfTall::TM ? MmRowsBfTall::kLds : MmRowsBf::kLds));
         k.info.sched.tg = MmRowsBf::kThreads; k.info.sched.nsg = MmRowsBf::kThreads / 64; k.info.sched.nr0 = BN; k.info.sched.k_split = (uint32_t)ks; k.info.sched.lds_tile = 32;
         set_name(k, "mul_mm_q4k_%dx%dx32%s%s", tm, BN, z_form ? "_kz" : "", n_mat == 3 ? "_x3" : n_mat == 2 ? "_x2" : "");
+    } else if (k.variant & kRows6) {
+        const int lds = tm == Mm6Rows<2>::TM ? Mm6Rows<2>::kLds : Mm6Rows<1>::kLds;
+        set_launch(k, (uint32_t)((batch + tm - 1) / tm), (uint32_t)row_tiles, z_form ? (uint32_t)ks : 1, Mm6Rows<2>::kThreads, (uint32_t)lds);
+        k.info.sched.tg = Mm6Rows<2>::kThreads; k.info.sched.nsg = Mm6Rows<2>::kThreads / 64; k.info.sched.nr0 = BN; k.info.sched.k_split = (uint32_t)ks; k.info.sched.lds_tile = KS;
+        set_name(k, "mul_mm_q6k_%dx%dx%d%s%s", tm, BN, KS, z_form ? "_kz" : "", n_mat == 3 ? "_x3" : n_mat == 2 ? "_x2" : "");
     } else {
         set_launch(k, (uint32_t)((batch + tm - 1) / tm), (uint32_t)row_tiles, z_form ? (uint32_t)ks : 1, kThreadsMM, (uint32_t)kLdsBytes);
         k.info.sched.tg = kThreadsMM; k.info.sched.nsg = kThreadsMM / 64; k.info.sched.nr0 = BN; k.info.sched.k_split = (uint32_t)ks; k.info.sched.lds_tile = KS;

@@ -390,6 +390,28 @@ def test_mul_mm_bf16_rows_at_the_edges_of_its_tiles(ctx, rows, batch, cols, ks, 
         assert float(rel_err(got[t], oracle.matvec_f64(oracle.Q4K, w, rows, cols, xs[t])).max()) <= 2e-5, t
 
 
+@pytest.mark.parametrize("rows,batch,cols,ks,at,shape", [
+    (1, 1, 256, 1, 0, "32x128"), (33, 31, 768, 3, 2, "32x128"), (129, 33, 2816, 7, 14, "32x128"), (127, 32, 256, 1, 6, "32x128"),
+    (4095, 65, 2816, 1, 10, "32x128"), (4097, 63, 6144, 8, 8, "64x128"), (4130, 64, 7936, 5, 4, "64x128"), (4223, 193, 768, 1, 12, "32x128")])
+def test_mul_mm_q6k_few_bf16_rows(ctx, rows, batch, cols, ks, at, shape):
+    """The Q6_K kernel of 32 or 64 tokens a workgroup where it can go wrong: a row or a token past a tile or short of it, slices
+    of unequal length and of one superblock, blocks from any even address on (rows of 210 bytes begin at every one of eight).
+    Against float64: these scales times codes stay below 2^11 and bf16 values are normal, both exact in f16; f32 sums (2e-5)."""
+    w = synth.q6k_blocks(rows * cols // 256, 740)
+    bw = ctx.buffer_bytes(bytes(at) + bytes(w))
+    xf, xb = synth.bf16_round(synth.normal_f32(batch * cols, 741))
+    k = ctx.compile(hip.make_desc(hip.Kind.MATVEC_BATCH, (rows, cols, batch), (DType.Q6K, DType.BF16, DType.F32), (),
+                                  dict(nr0=128, tg=256, lds_tile=64, k_split=ks)))
+    assert f"_{shape}x64" in k.name and k.info.sched.k_split == ks, k.name
+    y = ctx.buffer_empty_f32(batch * rows)
+    ctx.encode_offsets_multi(k, [bw, ctx.buffer_bytes(xb)], [at, 0], [y], None)
+    ctx.synchronize()
+    got = ctx.read_f32(y, batch * rows).reshape(batch, rows)
+    for t in sorted({0, 1, 30, 31, 32, 62, 63, 64, batch - 1} & set(range(batch))):
+        want = oracle.matvec_f64(oracle.Q6K, w, rows, cols, xf.reshape(batch, cols)[t])
+        assert rel_err(got[t], want).max() <= 2e-5, t
+
+
 @pytest.mark.parametrize("rows,batch,prologue", [(31, 33, 0), (97, 64, 2), (200, 130, 0), (4130, 1000, 2)])
 def test_mul_mm_f32_gate_up_pair(ctx, rows, batch, prologue):
     """dims[6] = 3: gelu(W x) * (W1 x) from one launch is the two matrices' products and KSH_GELU_MUL (64 rows of each
