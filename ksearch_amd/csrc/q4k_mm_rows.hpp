@@ -14,12 +14,12 @@
 //
 // With bf16 rows there are half as many matrix instructions to a converted weight, and a wave has 64 tokens x 32 rows, or 128 x
 // 32 where the chip is full: 2048 tokens, 12288 x 4096 257 -> 221 us, 300 tokens, 12288 x 1536 29.7 -> 24.1, 65 tokens, 12288 x
-// 8192 46 -> 40; 512 tokens, 8192 x 2048 30.5 -> 30.2, where the vector instructions (318 a superblock and wave) and the matrix
+// 8192 46 -> 40; 512 tokens, 8192 x 2048 30.8 -> 29.5, where the vector instructions (318 a superblock and wave) and the matrix
 // instructions fill a SIMD's time one after the other (20 and 18 thousand of 39 thousand cycles; neither fragments read two
 // units ahead nor eight half steps on their way change it).
 //
-// A product's order is fixed, so its bits do not depend on the shape that does it: per 16 columns the hi and the lo part against the same weights into a superblock's own accumulator, then F = (bias
-// and mins, two short products) + F and F = d * C + F.
+// A product's order is fixed, so its bits do not depend on the shape that does it: per 16 columns the hi and the lo part against
+// the same weights into a superblock's own accumulator, then F = (bias and mins, two short products) + F and F = d * C + F.
 //
 // CUT: the rows belong to prompts that would each have had a launch of their own, whose K slices depend on its length; the
 // workgroup takes all of K, and where a row's slice ends its sum goes to a second accumulator and starts again from zero (the
@@ -40,7 +40,7 @@ struct MmRows {
     static constexpr bool LO = LO_;
     static constexpr int TT = WM * MT, TM = 32 * TT, TN = 32 * WN * NT, kThreads = 64 * WM * WN;
     static constexpr int TF = TT * PARTS / 2;         // fragments of a half step that a wave fetches
-    static constexpr bool kNeighbours = NT == 1 && MT <= 2;   // an L2's workgroups are neighbours
+    static constexpr bool kNeighbours = NT == 1 && LO;   // an L2's workgroups are neighbours
     static constexpr int SUMS = TT == 4 ? 2 : 1;      // ... and fragments of a superblock's sums
     static constexpr int kStage = TT * 2 * PARTS * 1024;   // bytes of the fragments of 32 columns: [token tile][hi | lo][k slice][lane][16]
     static constexpr int kSums = TT * 2 * 1024;       // bytes of a superblock's sums of x: [token tile][k slice][lane][16]
@@ -75,9 +75,9 @@ __global__ __launch_bounds__(S::kThreads, 2) void q4k_mm_rows_kernel(MmParams p)
 
     // Shapes for launches that do not fill the chip: consecutive workgroups go round the eight L2s, so as they are numbered each
     // L2 would fetch most of X and of W.  Here an L2's workgroups are neighbours, all weight rows of a few token tiles (and of a
-    // K slice): 952 tokens, 1536 x 2048 30.6 -> 28.9 us, 700 tokens, 2048 x 2048 29.6 -> 27.9, 2048 tokens, 2560 x 1536 52.2 -> 49.6;
-    // bf16, 700 tokens, 2048 x 8192 53 -> 47, though 333 tokens, 1536 x 6144 24.1 -> 25.5.  Where the chip is full the walk along the
-    // tokens is the better one (2048 tokens, gate | up 12288 x 1536 312 or 318, bf16, 12288 x 4096 221 or 228).
+    // K slice): 952 tokens, 1536 x 2048 30.6 -> 28.9 us, 700 tokens, 2048 x 2048 29.6 -> 27.9, 2048 tokens, 2560 x 1536 52.2 -> 49.6.
+    // Where the chip is full the walk along the tokens is the better one (2048 tokens, gate | up 12288 x 1536 312 or 318), and with
+    // bf16 rows, half the bytes, it is so mostly (1024 tokens, 4096 x 4096 50.1 or 51.8; 700, 2048 x 8192 53 or 47).
     // (The quotients come from the host's reciprocals: divided here, they are 0.5 us in front of the first request.)
     uint32_t bx = blockIdx.x, by = blockIdx.y, bz = blockIdx.z;
     if constexpr (S::kNeighbours) {
@@ -422,6 +422,9 @@ __global__ __launch_bounds__(S::kThreads, 2) void q4k_mm_rows_kernel(MmParams p)
         for (int nt = 0; nt < NT; nt++) F[0][nt] = T[nt];
     }
     // accumulator layout of the 32x32 tile: column = lane % 32, row = 8*(i/4) + 4*(lane/32) + i%4
+    // (bf16 rows: stored past the L2s, since what those hold of it at the kernel's end is written out before the next kernel
+    // starts; 512 tokens, 8192 x 2048 30.8 -> 29.5 us, 300 tokens, 12288 x 1536 24.1 -> 22.9.  In a prompt's chain of launches it is even,
+    // 700 tokens 10.09 ms.)
 #pragma unroll
     for (int mt = 0; mt < MT; mt++) {
         const int tb = t0 + (wm * MT + mt) * 32 + 4 * h, left = p.batch - tb;
@@ -443,7 +446,10 @@ __global__ __launch_bounds__(S::kThreads, 2) void q4k_mm_rows_kernel(MmParams p)
                 const int t = 8 * (i / 4) + (i & 3);
                 float v = S::LO ? F[mt][nt][i] * inv[i / 4][i & 3] : F[mt][nt][i];
                 if constexpr (PAIR) v = gelu_mul_f32(pinned(v), pinned(F[mt][1][i] * inv[i / 4][i & 3]));
-                if (t < left) y[(size_t)t * ystride] = v;
+                if (t < left) {
+                    if (S::LO) y[(size_t)t * ystride] = v;
+                    else __builtin_nontemporal_store(v, &y[(size_t)t * ystride]);
+                }
             }
         }
     }
