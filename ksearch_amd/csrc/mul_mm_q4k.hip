@@ -747,7 +747,10 @@ __global__ __launch_bounds__(kThreadsMM, 1) void q6k_mul_mm_kernel(MmParams p)
 #pragma unroll
         for (int i = 0; i < 16; i++) {
             const int t = t0 + wm * 32 + 8 * (i / 4) + 4 * (lane >> 5) + (i & 3);
-            if (t < p.batch && r < p.rows) p.Y[(size_t)t * ystride + r] = LO ? F[nt][i] * p.inv_s[t] : F[nt][i];
+            if (t < p.batch && r < p.rows) {
+                if (LO) p.Y[(size_t)t * ystride + r] = F[nt][i] * p.inv_s[t];
+                else __builtin_nontemporal_store(F[nt][i], &p.Y[(size_t)t * ystride + r]);
+            }
         }
     }
 }

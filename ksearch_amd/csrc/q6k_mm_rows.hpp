@@ -201,7 +201,7 @@ __global__ __launch_bounds__(256, 2) void q6k_mm_rows_kernel(MmParams p)
 #pragma unroll
         for (int i = 0; i < 16; i++) {
             const int t = 8 * (i / 4) + (i & 3);
-            if (t < left) y[(size_t)t * ystride] = F[mt][i];
+            if (t < left) __builtin_nontemporal_store((float)F[mt][i], &y[(size_t)t * ystride]);
         }
     }
 }
