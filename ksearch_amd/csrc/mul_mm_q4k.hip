@@ -462,7 +462,75 @@ __device__ __forceinline__ uint32_t pair_f16(uint32_t masked, uint32_t sc)
 
 constexpr int kThreadsMM = 512;
 constexpr int kLdsMain = BN * PITCH;             // halves per main stage (the dequantized weight tile)
-constexpr size_t kLdsBytes = 2 * (size_t)kLdsMain * 2 + 2 * BN * 4;
+
+// A wave's way to 32 rows of a Q6_K superblock: 16-byte pieces at 16-byte addresses, 14 of them around a row's 210 bytes (which
+// begin at any even one), lane after lane along the rows, and by way of LDS to the lanes that want them.  A row a lane, at those
+// odd addresses, takes L1 186 cycles a load of 16 bytes (of 8 bytes 72), and L1 was busy for as long as the kernels ran.
+// (A piece holds a byte of the matrix at least: what else it reads lies in the same 16 bytes.)
+struct Q6Way {
+    static constexpr int kPitch = 240, kBytes = 32 * kPitch;
+    struct Pieces { u32x4_t v[7]; };
+    const uint8_t *tile;
+    uint8_t *lds;
+    uint32_t row_bytes, off[7];
+    int last, slot[7], at[7], nsb;
+
+    __device__ __forceinline__ Q6Way(const uint8_t *W, int r0, int rows, int nsb_row, int sb0, int nsb_, uint8_t *lds_, int lane)
+        : tile(W + ((size_t)min(r0, rows - 1) * nsb_row + sb0) * 210), lds(lds_), row_bytes((uint32_t)nsb_row * 210u), last(min(32, max(1, rows - r0)) - 1), nsb(nsb_)
+    {
+#pragma unroll
+        for (int i = 0; i < 7; i++) {
+            const int c = 64 * i + lane, row = c / 14;
+            off[i] = (uint32_t)min(row, last) * row_bytes;
+            slot[i] = 16 * (c % 14);
+            at[i] = row * kPitch + slot[i];
+        }
+    }
+    __device__ __forceinline__ void fetch(int sb, Pieces &w) const
+    {
+        const uint8_t *b = tile + (size_t)min(sb, nsb - 1) * 210;
+        const uint32_t low = (uint32_t)(uintptr_t)b & 15u;
+        b -= low;
+#pragma unroll
+        for (int i = 0; i < 7; i++) w.v[i] = *reinterpret_cast<const u32x4_t *>(b + (((off[i] + low) & ~15u) + (uint32_t)slot[i]));
+    }
+    // (a wave's LDS operations complete in order: the fences keep the compiler from moving them)
+    __device__ __forceinline__ void put(const Pieces &w) const
+    {
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+#pragma unroll
+        for (int i = 0; i < 7; i++) *reinterpret_cast<u32x4_t *>(lds + at[i]) = w.v[i];
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    }
+    // the words that row r's block begins in, and the bits of the first that come before it
+    __device__ __forceinline__ const uint32_t *row(int sb, int r, uint32_t &bits) const
+    {
+        const uint32_t a = (uint32_t)(uintptr_t)(tile + (size_t)min(sb, nsb - 1) * 210 + (uint32_t)min(r, last) * row_bytes) & 15u;
+        bits = (a & 2u) * 8u;
+        return reinterpret_cast<const uint32_t *>(lds + r * kPitch + (a & 12u));
+    }
+};
+// A code as it stands, the bits of a half, is code * 2^-24; with a scale 2^8 up, fma(code, scale, -32 * scale) is q * sc * 2^-16 in
+// one instruction, rounded as the product q * sc of halves is, and d takes the 2^16 back (f16 of any size counts in full here, the
+// subnormal ones too).
+constexpr float kQ6Unit = 65536.f;
+constexpr _Float16 kQ6Offset = (_Float16)(-32.f / 16777216.f);
+__device__ __forceinline__ h2 q6_scale(int8_t sc)
+{
+    const _Float16 s = (_Float16)(float)((int)sc * 256);
+    return h2{s, s};
+}
+// N words of a block from word `at` on
+template <int N>
+__device__ __forceinline__ void q6_words(const uint32_t *row, uint32_t bits, int at, uint32_t *v)
+{
+    uint32_t raw[N + 1];
+#pragma unroll
+    for (int i = 0; i <= N; i++) raw[i] = row[at + i];
+#pragma unroll
+    for (int i = 0; i < N; i++) v[i] = __builtin_amdgcn_alignbit(raw[i + 1], raw[i], bits);
+}
+constexpr size_t kLdsBytes = 2 * (size_t)kLdsMain * 2 + 2 * BN * 4 + 4 * Q6Way::kBytes;
 
 // The GEMM over Q6_K weights (K3b of the reference's plan: Q6_K tensors in prefill): 128 tokens x 128 weight rows a workgroup,
 // eight waves in two roles, one of each per SIMD.  Waves 0..3 only multiply:
@@ -473,8 +541,12 @@ constexpr size_t kLdsBytes = 2 * (size_t)kLdsMain * 2 + 2 * BN * 4;
 // conversions and the LDS writes of one role run in the shadow of the other
 // role's matrix instructions.
 //
-// w = d * sc_j * q with q = code - 32 in [-32, 31] and sc_j an int8 per 16 columns; the loaders build the f16
-// pair (1024 + code) by an OR into the mantissa, subtract 1056 and multiply by sc_j, both as packed f16.
+// w = d * sc_j * q with q = code - 32 in [-32, 31] and sc_j an int8 per 16 columns; the loaders build sc_j * q two at a time,
+// as a packed fma of halves (q6_scale).
+// What bounds it: the vector instructions, which here add to the matrix instructions' time (one loading and one multiplying wave
+// on a SIMD; pipe busy a third of the cycles).  Hence words by alignbit and perm and one fma a pair, 9 instructions to four
+// weights where 11.5 were, and the weights by pieces (Q6Way): 2048 tokens, 12288 x 4096 309 -> 279 us, 512 tokens, 8192 x 2048
+// 35.4 -> 32.5, 333 tokens, 1536 x 6144 in six slices 25.3 -> 23.3.
 // sc_j * q is exact in f16 up to 2048; beyond that (needs |sc_j| > 64) it rounds to the nearest even integer, a
 // relative 2^-11 at most and on those weights only (the reference's tile rounds every weight to half, the same
 // bound).  There is no min term; d is applied per superblock as for Q4_K.
@@ -524,71 +596,66 @@ __global__ __launch_bounds__(kThreadsMM, 1) void q6k_mul_mm_kernel(MmParams p)
         // of a superblock = ql bytes 64h + 32lh .. +31 (nibble `part`), qh bytes 32h .. +31 (bit pair
         // 4*part + 2*lh), scales 8h + 4*part + 2*lh and the next one.  Blocks are 2-byte aligned.
         const int lt = tid - 256, lrow = lt >> 1, lh = lt & 1;
-        const size_t row_bytes = (size_t)nsb_row * 210;
-        const uint8_t *wrow = p.W + (size_t)min(r0 + lrow, p.rows - 1) * row_bytes + (size_t)sb0 * 210;
+        const Q6Way rows(p.W, r0 + 32 * (wave - 4), p.rows, nsb_row, sb0, nsb, reinterpret_cast<uint8_t *>(lds + 2 * kLdsMain) + 2 * BN * 4 + (wave - 4) * Q6Way::kBytes, lane);
         struct Sb6Regs {
-            u32x2_t ql[8];    // [4h + i]: ql bytes 64h + 32lh + 8i .. +7
-            u32x2_t qh[8];    // all 64 qh bytes
-            u32x2_t sc[2];    // the 16 int8 scales
+            uint32_t ql[16];  // [8h + i]: ql bytes 64h + 32lh + 4i .. +3
+            uint32_t qh[16];  // all 64 qh bytes
+            uint32_t sc[4];   // the 16 int8 scales
             uint32_t d;
         };
-        auto ld64 = [](const uint8_t *a) __attribute__((always_inline)) {
-            u32x2_t v;
-            __builtin_memcpy(&v, a, 8);
-            return v;
-        };
-        auto fetch_sb = [&](int sb, Sb6Regs &r) __attribute__((always_inline)) {
-            const uint8_t *blk = wrow + (size_t)sb * 210;
-#pragma unroll
-            for (int i = 0; i < 4; i++) {
-                r.ql[i] = ld64(blk + 32 * lh + 8 * i);
-                r.ql[4 + i] = ld64(blk + 64 + 32 * lh + 8 * i);
-            }
-#pragma unroll
-            for (int i = 0; i < 8; i++) r.qh[i] = ld64(blk + 128 + 8 * i);
-            r.sc[0] = ld64(blk + 192);
-            r.sc[1] = ld64(blk + 200);
-            uint16_t d;
-            __builtin_memcpy(&d, blk + 208, 2);
-            r.d = d;
+        auto take = [&](int sb, Sb6Regs &r) __attribute__((always_inline)) {
+            uint32_t bits;
+            const uint32_t *q = rows.row(sb, lane >> 1, bits);
+            q6_words<8>(q, bits, 8 * lh, r.ql);
+            q6_words<8>(q, bits, 16 + 8 * lh, r.ql + 8);
+            q6_words<16>(q, bits, 32, r.qh);
+            q6_words<4>(q, bits, 48, r.sc);
+            r.d = (q[52] >> bits) & 0xFFFFu;
         };
         auto stage = [&](int step, auto gtag, const Sb6Regs &w) __attribute__((always_inline)) {
             constexpr int G = decltype(gtag)::value, H = G >> 1, P = G & 1;
             _Float16 *Bs = main_stage(step);
-            const uint32_t s16 = (w.sc[H][P] >> (16 * lh)) & 0xFFFFu;
-            const _Float16 sa = (_Float16)(int)(int8_t)(s16 & 0xFFu), sb_ = (_Float16)(int)(int8_t)(s16 >> 8);
-            const h2 sc2[2] = {h2{sa, sa}, h2{sb_, sb_}};
-            const h2 bias = {(_Float16)1056.f, (_Float16)1056.f};
+            const uint32_t s16 = (w.sc[2 * H + P] >> (16 * lh)) & 0xFFFFu;
+            const h2 sc2[2] = {q6_scale((int8_t)(s16 & 0xFFu)), q6_scale((int8_t)(s16 >> 8))};
+            const h2 off2[2] = {sc2[0] * kQ6Offset, sc2[1] * kQ6Offset};
             const int hsh = 4 * P + 2 * lh;
             uint32_t o[16];
 #pragma unroll
             for (int j = 0; j < 8; j++) {   // 4 columns per dword; dwords 0..3 take the first scale, 4..7 the second
-                const uint32_t L = w.ql[4 * H + (j >> 1)][j & 1], Q = w.qh[4 * H + (j >> 1)][j & 1];
+                const uint32_t L = w.ql[8 * H + j], Q = w.qh[8 * H + j];
                 const uint32_t nib = (P ? (L >> 4) : L) & 0x0F0F0F0Fu;
-                const uint32_t c = nib | (((Q >> hsh) & 0x03030303u) << 4);   // four 6-bit codes
-                const uint32_t pa = (c & 0x00FF00FFu) | 0x64006400u;          // columns (0, 2) as 1024 + code
-                const uint32_t pb = ((c >> 8) & 0x00FF00FFu) | 0x64006400u;   // columns (1, 3)
-                const h2 va = (__builtin_bit_cast(h2, pa) - bias) * sc2[j >> 2];
-                const h2 vb = (__builtin_bit_cast(h2, pb) - bias) * sc2[j >> 2];
+                const uint32_t c = nib | (__builtin_amdgcn_alignbit(Q, Q, (uint32_t)(hsh - 4) & 31u) & 0x30303030u);   // four 6-bit codes (turned: only whole bytes' bits stay)
+                // columns (0, 2) and (1, 3), as halves
+                const h2 va = __builtin_elementwise_fma(__builtin_bit_cast(h2, __builtin_amdgcn_perm(0u, c, 0x0C020C00u)), sc2[j >> 2], off2[j >> 2]);
+                const h2 vb = __builtin_elementwise_fma(__builtin_bit_cast(h2, __builtin_amdgcn_perm(0u, c, 0x0C030C01u)), sc2[j >> 2], off2[j >> 2]);
                 o[2 * j] = __builtin_bit_cast(uint32_t, va);
                 o[2 * j + 1] = __builtin_bit_cast(uint32_t, vb);
             }
             uint4 *dst = reinterpret_cast<uint4 *>(&Bs[lrow * PITCH + 32 * lh]);
 #pragma unroll
             for (int i = 0; i < 4; i++) dst[i] = make_uint4(o[4 * i], o[4 * i + 1], o[4 * i + 2], o[4 * i + 3]);
-            if (G == 0 && lh == 0) dsc_stage(step >> 2)[lrow] = half_bits_to_f32(w.d);
+            if (G == 0 && lh == 0) dsc_stage(step >> 2)[lrow] = half_bits_to_f32(w.d) * kQ6Unit;
         };
-        Sb6Regs wcur, wnext;
-        fetch_sb(0, wcur);
-        stage(0, std::integral_constant<int, 0>{}, wcur);
+        Q6Way::Pieces next;
+        Sb6Regs w;
+        rows.fetch(0, next);
+        rows.put(next);
+        take(0, w);
+        stage(0, std::integral_constant<int, 0>{}, w);
         __syncthreads();
         auto step_body = [&](int sb, auto gtag) __attribute__((always_inline)) {
             constexpr int g = decltype(gtag)::value;
             const int step = 4 * sb + g;
-            if (g == 0) fetch_sb(min(sb + 1, nsb - 1), wnext);
+            if (g == 0) {
+                rows.fetch(sb + 1, next);
+                __builtin_amdgcn_sched_barrier(0);
+            }
             if (step + 1 < nsteps) {
-                if (g == 3) wcur = wnext;
-                stage(step + 1, std::integral_constant<int, (g + 1) & 3>{}, wcur);
+                if (g == 3) {
+                    rows.put(next);
+                    take(sb + 1, w);
+                }
+                stage(step + 1, std::integral_constant<int, (g + 1) & 3>{}, w);
             }
             __syncthreads();
         };

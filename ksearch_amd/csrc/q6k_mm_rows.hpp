@@ -22,8 +22,7 @@ struct Mm6Rows {
     static constexpr int MT = MT_, TM = 32 * MT, TN = 128, kThreads = 256;
     static constexpr int kHalf = 512 + 16, kFrag = 2 * kHalf;   // bytes of a fragment's half (eight writes of a row in eight places)
     static constexpr int kStage = MT * 4 * kFrag;           // 64 columns: [token tile][k slice][lane][16]
-    static constexpr int kPitch = 240, kTile = 32 * kPitch;   // bytes of a superblock's row, of a wave's rows
-    static constexpr int kLds = 2 * kStage + 4 * kTile;
+    static constexpr int kLds = 2 * kStage + 4 * Q6Way::kBytes;
 };
 
 template <int MT_>
@@ -72,58 +71,19 @@ __global__ __launch_bounds__(256, 2) void q6k_mm_rows_kernel(MmParams p)
         for (int i = 0; i < MT; i++) *reinterpret_cast<h8 *>(f + 4 * i * S::kFrag) = from_bf16(__builtin_bit_cast(h8, x.v[i]));
     };
 
-    // ---- weights: 16-byte pieces at 16-byte addresses, 14 of them around a row's 210 bytes (which begin at any even one), lane
-    // after lane along the rows; by way of LDS into the registers of the lanes that want them.  (A piece holds a byte of the
-    // matrix at least: what else it reads is of the same 16 bytes.)
-    const uint8_t *wtile = p.W + ((size_t)min(r0, p.rows - 1) * nsb_row + sb0) * 210;
-    const uint32_t row_bytes = (uint32_t)nsb_row * 210u;
-    const int rows_here = min(32, max(1, p.rows - r0));
-    uint32_t poff[7];
-    int pslot[7];
-#pragma unroll
-    for (int i = 0; i < 7; i++) {
-        const int c = 64 * i + lane, row = c / 14;
-        poff[i] = (uint32_t)min(row, rows_here - 1) * row_bytes;
-        pslot[i] = c % 14;
-    }
-    uint8_t *wlds = lds6 + 2 * S::kStage + wave * S::kTile;
-    const uint32_t my_off = (uint32_t)min(lm, rows_here - 1) * row_bytes;
-    struct Pieces { u32x4_t v[7]; };
-    auto fetch_w = [&](int sb, Pieces &w) __attribute__((always_inline)) {
-        const uint8_t *b = wtile + (size_t)min(sb, nsb - 1) * 210;
-        const uint32_t low = (uint32_t)(uintptr_t)b & 15u;
-        b -= low;
-#pragma unroll
-        for (int i = 0; i < 7; i++) w.v[i] = *reinterpret_cast<const u32x4_t *>(b + (((poff[i] + low) & ~15u) + 16u * (uint32_t)pslot[i]));
-    };
-    // (a wave's LDS operations complete in order: the fences keep the compiler from moving them)
-    auto put_w = [&](const Pieces &w) __attribute__((always_inline)) {
-        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-#pragma unroll
-        for (int i = 0; i < 7; i++) *reinterpret_cast<u32x4_t *>(wlds + (64 * i + lane) / 14 * S::kPitch + 16 * pslot[i]) = w.v[i];
-        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-    };
+    // ---- weights
+    const Q6Way rows(p.W, r0, p.rows, nsb_row, sb0, nsb, lds6 + 2 * S::kStage + wave * Q6Way::kBytes, lane);
     // lane (lm, h): bytes 8h .. 8h+7 of every 16 of its row's codes, the scales, d
-    struct WRegs { u32x2_t ql[8], qh[4]; u32x4_t sc; uint32_t d; };
+    struct WRegs { uint32_t ql[8][2], qh[4][2], sc[4], d; };
     auto take_w = [&](int sb, WRegs &w) __attribute__((always_inline)) {
-        const uint32_t at = (uint32_t)(uintptr_t)(wtile + (size_t)sb * 210 + my_off) & 15u;
-        const uint32_t *row = reinterpret_cast<const uint32_t *>(wlds + lm * S::kPitch + (at & 12u));
-        const uint32_t sh = (at & 2u) * 8u;
-        auto eight = [&](int byte, u32x2_t &v) __attribute__((always_inline)) {
-            const uint32_t *q = row + byte / 4 + 2 * h;
-            const uint32_t a = q[0], b = q[1], c = q[2];
-            v = u32x2_t{__builtin_amdgcn_alignbit(b, a, sh), __builtin_amdgcn_alignbit(c, b, sh)};
-        };
+        uint32_t bits;
+        const uint32_t *q = rows.row(sb, lm, bits);
 #pragma unroll
-        for (int i = 0; i < 8; i++) eight(16 * i, w.ql[i]);
+        for (int i = 0; i < 8; i++) q6_words<2>(q, bits, 4 * i + 2 * h, w.ql[i]);
 #pragma unroll
-        for (int i = 0; i < 4; i++) eight(128 + 16 * i, w.qh[i]);
-        uint32_t s[6];
-#pragma unroll
-        for (int i = 0; i < 5; i++) s[i] = row[48 + i];
-#pragma unroll
-        for (int i = 0; i < 4; i++) w.sc[i] = __builtin_amdgcn_alignbit(s[i + 1], s[i], sh);
-        w.d = (s[4] >> sh) & 0xFFFFu;
+        for (int i = 0; i < 4; i++) q6_words<2>(q, bits, 32 + 4 * i + 2 * h, w.qh[i]);
+        q6_words<4>(q, bits, 48, w.sc);
+        w.d = (q[52] >> bits) & 0xFFFFu;
     };
 
     f16v F[MT], C[MT];
@@ -133,22 +93,22 @@ __global__ __launch_bounds__(256, 2) void q6k_mm_rows_kernel(MmParams p)
     const uint8_t *fr = lds6 + h * S::kHalf + lm * 16;
 
     XRegs x[4];
-    Pieces wp;
+    Q6Way::Pieces wp;
     WRegs w;
     fetch_x(0, x[0]);
-    fetch_w(0, wp);
+    rows.fetch(0, wp);
     fetch_x(1, x[1]);
     fetch_x(2, x[2]);
     fetch_x(3, x[3]);
     put_x(0, x[0]);
-    put_w(wp);
+    rows.put(wp);
     take_w(0, w);
     __syncthreads();
     auto step_body = [&](int sb, auto gtag) __attribute__((always_inline)) {
         constexpr int g = decltype(gtag)::value, H = g >> 1, P = g & 1;
         const int step = 4 * sb + g;
         fetch_x(step + 4, x[g]);
-        if (g == 0) fetch_w(sb + 1, wp);
+        if (g == 0) rows.fetch(sb + 1, wp);
         __builtin_amdgcn_sched_barrier(0);
         const uint32_t sc4 = w.sc[g];
 #pragma unroll
@@ -156,8 +116,7 @@ __global__ __launch_bounds__(256, 2) void q6k_mm_rows_kernel(MmParams p)
             h8 a[MT];
 #pragma unroll
             for (int mt = 0; mt < MT; mt++) a[mt] = *reinterpret_cast<const h8 *>(fr + (g & 1) * S::kStage + (mt * 4 + ks) * S::kFrag);
-            const _Float16 s = (_Float16)(int)(int8_t)(sc4 >> (8 * ks));
-            const h2 s2 = {s, s}, bias = {(_Float16)1056.f, (_Float16)1056.f};
+            const h2 s2 = q6_scale((int8_t)(sc4 >> (8 * ks))), off2 = s2 * kQ6Offset;
             u32x4_t o;
 #pragma unroll
             for (int i = 0; i < 2; i++) {
@@ -165,9 +124,8 @@ __global__ __launch_bounds__(256, 2) void q6k_mm_rows_kernel(MmParams p)
                 const int sh = 4 * P + 2 * (ks >> 1);
                 const uint32_t hi = sh < 4 ? Q << (4 - sh) : Q >> (sh - 4);
                 const uint32_t c = (hi & 0x30303030u) | ((P ? L >> 4 : L) & 0x0F0F0F0Fu);
-                const uint32_t pa = __builtin_amdgcn_perm(0x64646464u, c, 0x04020400u), pb = __builtin_amdgcn_perm(0x64646464u, c, 0x04030401u);
-                o[2 * i] = __builtin_bit_cast(uint32_t, (__builtin_bit_cast(h2, pa) - bias) * s2);
-                o[2 * i + 1] = __builtin_bit_cast(uint32_t, (__builtin_bit_cast(h2, pb) - bias) * s2);
+                o[2 * i] = __builtin_bit_cast(uint32_t, __builtin_elementwise_fma(__builtin_bit_cast(h2, __builtin_amdgcn_perm(0u, c, 0x0C020C00u)), s2, off2));
+                o[2 * i + 1] = __builtin_bit_cast(uint32_t, __builtin_elementwise_fma(__builtin_bit_cast(h2, __builtin_amdgcn_perm(0u, c, 0x0C030C01u)), s2, off2));
             }
             const h8 b = __builtin_bit_cast(h8, o);
 #pragma unroll
@@ -176,13 +134,13 @@ __global__ __launch_bounds__(256, 2) void q6k_mm_rows_kernel(MmParams p)
             if (ks == 1) put_x((g + 1) & 1, x[(g + 1) & 3]);
         }
         if (g == 3) {
-            const float d = half_bits_to_f32(w.d);
+            const float d = half_bits_to_f32(w.d) * kQ6Unit;
 #pragma unroll
             for (int mt = 0; mt < MT; mt++)
 #pragma unroll
                 for (int i = 0; i < 16; i++) F[mt][i] = fmaf(d, C[mt][i], F[mt][i]);
-            put_w(wp);
-            take_w(min(sb + 1, nsb - 1), w);
+            rows.put(wp);
+            take_w(sb + 1, w);
         }
         __syncthreads();
     };
