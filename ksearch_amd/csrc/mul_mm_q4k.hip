@@ -1156,10 +1156,12 @@ struct RoundParams {
 };
 
 // NM = 2: the gate | up pair (W0, W1 of rows0 rows each; gelu(W0 x) * (W1 x) to Y0)
+constexpr int kRoundTile = 32 * 144 / 4;      // 32 rows of a superblock
 template <int NM>
-__global__ __launch_bounds__(512) void q4k_mm_round_kernel(RoundParams p)
+__global__ __launch_bounds__(512, 4) void q4k_mm_round_kernel(RoundParams p)
 {
-    extern __shared__ __attribute__((aligned(16))) float red[];   // [8][NM][8][64]
+    // a wave's weight rows per matrix, and over them its shares of the results, [8][64]: kRoundTile floats each
+    extern __shared__ __attribute__((aligned(16))) float red[];   // [8][NM][kRoundTile]
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int n = lane & 31, h = lane >> 5;
     // the workgroup's matrix: a choice between arguments already fetched, not an indexed read of them
@@ -1174,22 +1176,25 @@ __global__ __launch_bounds__(512) void q4k_mm_round_kernel(RoundParams p)
     const int sb = blockIdx.y * 8 + wave;
     const bool active = sb < nsb;                        // (wave-uniform: a row of 1536 columns leaves two waves idle)
     const int sbc = min(sb, nsb - 1);
-    const size_t woff = (size_t)min(r0 + n, rows - 1) * nsb * 144 + (size_t)sbc * 144;
 
     // (the other waves ask for nothing: a quarter of the requests were for a row's last superblock again, and the vector-memory
     // path is what the launch is busy with -- gate | up of 12288 x 1536 for 16 rows 18.8 -> 16.8 us)
     if (active) {
-        // ---- every load of the wave, up front
-        u32x4_t hdr[NM];
-        u32x2_t q[NM][4][2];
+        // ---- every load of the wave, up front: the weights as pieces of 16 bytes, lane after lane along the rows, straight into
+        // LDS.  (A row a lane, an instruction is 64 places of L1 instead of some 20, and L1's path was the busy unit; read back
+        // matrix by matrix they also leave registers for a second workgroup on the compute unit.  16 rows: gate | up of 12288 x
+        // 1536 17.1 -> 14.3 us, 1536 x 12288 11.9 -> 9.7, 1536 x 2048 5.6 -> 4.9; 6144 x 1536, one workgroup a unit, 9.7 -> 10.0.)
+        float *mine = red + wave * NM * kRoundTile;
+        const uint32_t l0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) float *)mine;
+        const int last = rows - 1 - r0;
+        const uint32_t row_bytes = (uint32_t)nsb * 144u;
 #pragma unroll
         for (int m = 0; m < NM; m++) {
-            const uint8_t *blk = (m ? p.W1 : W) + woff;
-            hdr[m] = *reinterpret_cast<const u32x4_t *>(blk);
+            const uint8_t *blk = (m ? p.W1 : W) + (size_t)r0 * row_bytes + (size_t)sbc * 144;
 #pragma unroll
-            for (int g = 0; g < 4; g++) {
-                q[m][g][0] = *reinterpret_cast<const u32x2_t *>(blk + 16 + 32 * g + 8 * h);
-                q[m][g][1] = *reinterpret_cast<const u32x2_t *>(blk + 16 + 32 * g + 16 + 8 * h);
+            for (int i = 0; i < 5; i++) {
+                const int c = 64 * i + lane, row = c / 9;
+                if (i < 4 || lane < 32) to_lds16(blk, (uint32_t)min(row, last) * row_bytes + 16u * (uint32_t)(c % 9), l0 + (uint32_t)(m * kRoundTile * 4 + i * 1024));
             }
         }
         const h8 *xa = reinterpret_cast<const h8 *>(p.Xp) + (size_t)sbc * 16 * 64 + lane;
@@ -1199,18 +1204,27 @@ __global__ __launch_bounds__(512) void q4k_mm_round_kernel(RoundParams p)
         // sums of x: rows 0..15 the tokens' hi parts, rows 16..31 their lo parts
         const _Float16 *sx = p.Xp + round_xf_halves(p.cols) + (n >= 16 ? round_sx_halves(p.cols) : 0) + ((size_t)(n & 15) * nsb + sbc) * 32 + 8 * h;
         const h8 a2[2] = {*reinterpret_cast<const h8 *>(sx), *reinterpret_cast<const h8 *>(sx + 16)};
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
 
         const f16v kZero16 = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
 #pragma unroll
         for (int m = 0; m < NM; m++) {
+            const uint8_t *blk = reinterpret_cast<const uint8_t *>(mine + m * kRoundTile) + 144 * n;
+            const u32x4_t hdr = *reinterpret_cast<const u32x4_t *>(blk);
+            u32x2_t q[4][2];
+#pragma unroll
+            for (int g = 0; g < 4; g++) {
+                q[g][0] = *reinterpret_cast<const u32x2_t *>(blk + 16 + 32 * g + 8 * h);
+                q[g][1] = *reinterpret_cast<const u32x2_t *>(blk + 16 + 32 * g + 16 + 8 * h);
+            }
             f16v C = kZero16;
 #pragma unroll
             for (int g = 0; g < 4; g++) {
-                const uint4 s = q4k_group_scales(hdr[m].y, hdr[m].z, hdr[m].w, g);   // sc_lo, mn_lo, sc_hi, mn_hi
+                const uint4 s = q4k_group_scales(hdr.y, hdr.z, hdr.w, g);   // sc_lo, mn_lo, sc_hi, mn_hi
 #pragma unroll
                 for (int j = 0; j < 4; j++) {
                     // slice j: bytes (j & 1 ? 16 + 8h : 8h) .. +7, low nibbles for j < 2, high nibbles after
-                    const u32x2_t qq = q[m][g][j & 1];
+                    const u32x2_t qq = q[g][j & 1];
                     const uint32_t sc = j < 2 ? s.x : s.z;
                     uint32_t o[4];
 #pragma unroll
@@ -1225,11 +1239,11 @@ __global__ __launch_bounds__(512) void q4k_mm_round_kernel(RoundParams p)
             }
             // bias + mins of the superblock: the row's eight coefficients -(dmin*m_j + 1024*d) as f16 hi | lo, against the
             // sums of x (hi[8] hi[8] lo[8] 0[8] per row and superblock): hi*hi + hi*lo + lo*hi
-            const float d = half_bits_to_f32(hdr[m].x & 0xFFFFu), dmin = half_bits_to_f32(hdr[m].x >> 16);
+            const float d = half_bits_to_f32(hdr.x & 0xFFFFu), dmin = half_bits_to_f32(hdr.x >> 16);
             _Float16 chi[8], clo[8];
 #pragma unroll
             for (int g = 0; g < 4; g++) {
-                const uint4 s = q4k_group_scales(hdr[m].y, hdr[m].z, hdr[m].w, g);
+                const uint4 s = q4k_group_scales(hdr.y, hdr.z, hdr.w, g);
                 const float c0 = pinned(-(dmin * (float)s.y + 1024.f * d)), c1 = pinned(-(dmin * (float)s.w + 1024.f * d));
                 chi[2 * g] = (_Float16)c0; chi[2 * g + 1] = (_Float16)c1;
                 clo[2 * g] = (_Float16)(c0 - (float)chi[2 * g]); clo[2 * g + 1] = (_Float16)(c1 - (float)chi[2 * g + 1]);
@@ -1245,11 +1259,11 @@ __global__ __launch_bounds__(512) void q4k_mm_round_kernel(RoundParams p)
             // accumulator i of lane (n, h) is row 8*(i/4) + 4*h + i%4 of the tile: i < 8 a token's hi part, i + 8 its lo part
 #pragma unroll
             for (int i = 0; i < 8; i++)
-                red[((wave * NM + m) * 8 + i) * 64 + lane] = fmaf(1.0f / 2048.0f, fmaf(d, C[i + 8], F[i + 8]), fmaf(d, C[i], F[i]));
+                mine[m * kRoundTile + i * 64 + lane] = fmaf(1.0f / 2048.0f, fmaf(d, C[i + 8], F[i + 8]), fmaf(d, C[i], F[i]));
         }
     } else {
 #pragma unroll
-        for (int i = 0; i < 8 * NM; i++) red[(wave * NM * 8 + i) * 64 + lane] = 0.f;
+        for (int i = 0; i < 8 * NM; i++) red[(wave * NM + i / 8) * kRoundTile + (i & 7) * 64 + lane] = 0.f;
     }
     __syncthreads();
     // one output per thread: the eight waves' shares in a fixed order
@@ -1259,13 +1273,13 @@ __global__ __launch_bounds__(512) void q4k_mm_round_kernel(RoundParams p)
     for (int m = 0; m < NM; m++) {
         v[m] = 0.f;
 #pragma unroll
-        for (int w = 0; w < 8; w++) v[m] += red[((w * NM + m) * 8 + i) * 64 + lane];
+        for (int w = 0; w < 8; w++) v[m] += red[(w * NM + m) * kRoundTile + i * 64 + lane];
     }
-    const bool mine = t < p.batch && r < rows;
+    const bool in = t < p.batch && r < rows;
     float y = NM == 2 ? gelu_mul_f32(v[0], v[NM - 1]) : v[0];
     if (NM == 1 && p.mul) y = gelu_mul_f32(y, p.mul[(size_t)min(t, p.batch - 1) * p.mul_stride + min(r, rows - 1)]);
     if (!p.emit) {
-        if (mine) {
+        if (in) {
             if (gridDim.y == 1) Y[(size_t)t * rows + r] = y;
             else p.part[((size_t)blockIdx.y * p.batch + t) * rows + r] = y;
         }
@@ -1274,8 +1288,8 @@ __global__ __launch_bounds__(512) void q4k_mm_round_kernel(RoundParams p)
     // The tile's 16 x 32 results are 32 columns of the next GEMM's input: two fragments' worth of every token row and
     // exactly one sub-block of sums, so the workgroup writes its share of the prepared operand itself (rows0 is a
     // multiple of 256 and the columns are not split: host-checked).  Rows past the batch are written as zeros.
-    float *T = red + 8 * NM * 8 * 64;             // [16][33]
-    T[t * 33 + n] = mine ? y : 0.f;
+    float *T = red + 8 * NM * kRoundTile;         // [16][33]
+    T[t * 33 + n] = in ? y : 0.f;
     __syncthreads();
     if (tid < 64) {
         const int tt = tid & 15, ks = (tid >> 4) & 1, kh = tid >> 5;
@@ -1930,7 +1944,7 @@ int bind_matvec_round(ksh_kernel &k)
     k.scratch_bytes = slices > 1 && !unfolded ? (size_t)slices * batch * rows0 * 4 : 0;
     if (unfolded) k.out_bytes[0] = (size_t)slices * batch * rows0 * 4;
     const int64_t tiles = pair ? (rows0 + 31) / 32 : (rows0 + 31) / 32 + (rows1 + 31) / 32 + (rows2 + 31) / 32;
-    set_launch(k, (uint32_t)tiles, (uint32_t)slices, 1, 512, (uint32_t)(8 * (pair ? 2 : 1) * 8 * 64 * 4 + (emit ? 16 * 33 * 4 : 0)));
+    set_launch(k, (uint32_t)tiles, (uint32_t)slices, 1, 512, (uint32_t)(8 * (pair ? 2 : 1) * kRoundTile * 4 + (emit ? 16 * 33 * 4 : 0)));
     k.info.sched = k.desc.sched;
     k.info.sched.tg = 512; k.info.sched.nsg = 8; k.info.sched.nr0 = 32; k.info.sched.k_split = (uint32_t)slices; k.info.sched.lds_tile = 16;
     set_name(k, "matvec_round_q4k_%s%s%s", pair ? "gate_up_gelu" : mul_stride ? "gelu_mul" : n_mat == 3 ? "x3" : n_mat == 2 ? "x2" : "x1",

@@ -71,6 +71,21 @@ def test_matvec_round_gate_up_gelu(ctx, rows, cols, batch):
     assert_close(got, oracle.gelu_mul(g.reshape(-1), u.reshape(-1)).reshape(batch, rows), 1e-3, f"gate|up {rows}x{cols} b{batch}")
 
 
+@pytest.mark.parametrize("rows,cols,batch", [(1, 256, 1), (33, 1792, 16), (63, 2048, 2), (2049, 512, 15)])
+def test_matvec_round_gate_up_ragged_tiles(ctx, rows, cols, batch):
+    """Tiles of both matrices that end inside their 32 rows (the rest of the tile's pieces are the last row's again), one
+    superblock, waves without one.  gelu(g) * u of float64 products: either factor off by 2e-5 of its rms or value, gelu' <= 1.13,
+    against a product of at least 0.6 of the two rms at up to four times them (2 * 4 * 1.13 / 0.6 * 2e-5)."""
+    ws = [synth.q4k_blocks(rows * cols // 256, seed=914 + i) for i in range(2)]
+    x = synth.normal_f32(batch * cols, 913).reshape(batch, cols) * 0.25
+    _, (got,) = round_mm(ctx, ws, (rows,), cols, x, batch, pair=True)
+    for t in (0, batch - 1):
+        g, u = (oracle.matvec_f64(oracle.Q4K, w, rows, cols, x[t]) for w in ws)
+        g_ = np.clip(g, -20.0, 20.0)
+        want = 0.5 * g_ * (1.0 + np.tanh(0.7978845608 * (g_ + 0.044715 * g_ ** 3))) * u
+        assert np.max(np.abs(got[t] - want) / np.maximum(np.abs(want), np.sqrt(np.mean(want ** 2)))) <= 3e-4
+
+
 @pytest.mark.parametrize("batch", [16, 3])
 def test_matvec_round_result_as_prepared_operand(ctx, batch):
     """dims[6] = 1: a launch's result leaves as the next GEMM's prepared operand (here gate | up -> down, and the
