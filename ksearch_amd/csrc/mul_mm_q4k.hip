@@ -444,7 +444,7 @@ MmPlan mm_plan_bf16(bool q6, int row_tiles, int nsb, int64_t batch, int64_t rows
 float mm_skinny_us(int64_t rows, int nsb, int64_t batch)
 {
     const float turns = std::max(1.f, (float)((rows + 31) / 32) / 128.f - 1.f), each = (float)nsb / 8.f;
-    return batch <= 32 ? 5.5f + 3.1f * each * turns : 6.4f + 5.f * std::max(each, 0.45f) * turns;
+    return batch <= 32 ? 5.4f + 2.f * each * turns : 6.2f + 4.3f * std::max(each, 0.45f) * turns;
 }
 
 // Bf16 rows of Q6_K products as they are (the kernel's ROWS form): the conversion between the matrix instructions costs 0.42
@@ -831,6 +831,19 @@ __global__ __launch_bounds__(kThreadsMM, 1) void q6k_mul_mm_kernel(MmParams p)
 namespace ksh {
 namespace {
 
+// A wave's request for its 32 rows of a Q4_K superblock, as pieces of 16 bytes, lane after lane along the rows, straight into LDS
+// at `dst` ([row][144]).  (A row a lane, an instruction is 64 places of L1 instead of some 20, and that path is what launches of a
+// few tokens are busy with.)  `blk`: row 0's superblock; `last`: the last row there is.
+constexpr int kRoundTile = 32 * 144 / 4;      // floats
+__device__ __forceinline__ void ask_q4k_tile(const uint8_t *blk, uint32_t row_bytes, int last, int lane, uint32_t dst)
+{
+#pragma unroll
+    for (int i = 0; i < 5; i++) {
+        const int c = 64 * i + lane, row = c / 9;
+        if (i < 4 || lane < 32) to_lds16(blk, (uint32_t)min(row, last) * row_bytes + 16u * (uint32_t)(c % 9), dst + (uint32_t)(i * 1024));
+    }
+}
+
 // ---- small batches (up to 64 tokens): a GEMV-shaped launch on the matrix cores ---------------------------------
 // A prompt remainder or a round of decoding slots is a few dozen tokens: the 128 x 128 tile then leaves most of the
 // chip idle (rows / 128 workgroups) and half of every tile empty.  Here a workgroup owns 32 weight rows and all
@@ -841,16 +854,27 @@ namespace {
 // two 8-byte loads.  Conversion (sc*n as exact f16, biased by 1024), the per-superblock scale and the bias / min
 // product are those of the big tile; the activations come as the same fragments, hi and lo part in the same pass
 // (each converted weight is used for both), so f32 activations cost one launch.
-template <int MT, bool HAS_LO>
+//
+// PIECES: the weights come as pieces of 16 bytes by way of LDS, which costs a second round trip and saves most of the time in L1.
+// Measured (us, rows a lane -> pieces; 1536 rows, or as said): up to 32 tokens 2048 columns 8.4 -> 6.9, 6144 15.2 -> 11.0, 12288
+// rows of 2048 11.8 -> 9.1; 33 .. 64 tokens 10.6 -> 9.9, 21 -> 19, 17 -> 15.  Where two waves do everything (512 columns) it is
+// the round trip that counts, 5.8 -> 6.3 and 8.0 -> 8.5: rows a lane up to 4 superblocks.  So also for two parts of 64 tokens,
+// which have no registers left for it.
+constexpr int skinny_wave(int mt, bool pieces) { return pieces && mt == 1 ? kRoundTile : mt * 16 * 64; }      // floats of LDS
+constexpr bool skinny_pieces(int mt, bool lo, int nsb) { return nsb > 4 && !(mt == 2 && lo); }
+template <int MT, bool HAS_LO, bool PIECES>
 __global__ __launch_bounds__(512) void q4k_mm_skinny_kernel(MmParams p, const _Float16 *__restrict__ Xf_lo, const _Float16 *__restrict__ SxA_lo,
                                                              float lo_scale)
 {
-    extern __shared__ __attribute__((aligned(16))) float red[];   // [8][MT][16][64]
+    extern __shared__ __attribute__((aligned(16))) float red[];   // [8][WAVE]: a wave's weight rows, then its [MT][16][64]
+    constexpr int WAVE = skinny_wave(MT, PIECES);
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int n = lane & 31, h = lane >> 5;
     const int r0 = blockIdx.x * 32, nsb = p.cols / 256;
     const size_t row_bytes = (size_t)nsb * 144;
     const uint8_t *wrow = p.W + (size_t)min(r0 + n, p.rows - 1) * row_bytes;
+    const float *mine = red + wave * WAVE;
+    const uint32_t l0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) float *)(red + wave * WAVE);
     const int ntt = (p.batch + 31) / 32;
     const h8 *xa[MT], *xl[MT];
     const _Float16 *sxa[MT], *sxl[MT];
@@ -869,7 +893,11 @@ __global__ __launch_bounds__(512) void q4k_mm_skinny_kernel(MmParams p, const _F
     for (int mt = 0; mt < MT; mt++) { F[mt] = kZero16; Fl[mt] = kZero16; }
 
     for (int sb = wave; sb < nsb; sb += 8) {
-        const uint8_t *blk = wrow + (size_t)sb * 144;
+        if constexpr (PIECES) {
+            ask_q4k_tile(p.W + (size_t)r0 * row_bytes + (size_t)sb * 144, (uint32_t)row_bytes, p.rows - 1 - r0, lane, l0);
+            asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+        }
+        const uint8_t *blk = PIECES ? reinterpret_cast<const uint8_t *>(mine) + 144 * n : wrow + (size_t)sb * 144;
         const u32x4_t hdr = *reinterpret_cast<const u32x4_t *>(blk);
         u32x2_t q[4][2];
 #pragma unroll
@@ -877,6 +905,7 @@ __global__ __launch_bounds__(512) void q4k_mm_skinny_kernel(MmParams p, const _F
             q[g][0] = *reinterpret_cast<const u32x2_t *>(blk + 16 + 32 * g + 8 * h);
             q[g][1] = *reinterpret_cast<const u32x2_t *>(blk + 16 + 32 * g + 16 + 8 * h);
         }
+        if constexpr (PIECES) asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");      // (the next superblock's rows come to the same place)
         f16v C[MT], Cl[MT];
 #pragma unroll
         for (int g = 0; g < 4; g++) {
@@ -953,12 +982,12 @@ __global__ __launch_bounds__(512) void q4k_mm_skinny_kernel(MmParams p, const _F
     for (int mt = 0; mt < MT; mt++)
 #pragma unroll
         for (int i = 0; i < 16; i++)
-            red[((wave * MT + mt) * 16 + i) * 64 + lane] = HAS_LO ? fmaf(lo_scale, Fl[mt][i], F[mt][i]) : F[mt][i];
+            red[wave * WAVE + (mt * 16 + i) * 64 + lane] = HAS_LO ? fmaf(lo_scale, Fl[mt][i], F[mt][i]) : F[mt][i];
     __syncthreads();
     for (int o = tid; o < MT * 16 * 64; o += 512) {
         float sum = 0.f;
 #pragma unroll
-        for (int w = 0; w < 8; w++) sum += red[w * MT * 16 * 64 + o];
+        for (int w = 0; w < 8; w++) sum += red[w * WAVE + o];
         const int mt = o / (16 * 64), i = (o / 64) & 15, l = o & 63;
         const int t = mt * 32 + 8 * (i / 4) + 4 * (l >> 5) + (i & 3), r = r0 + (l & 31);
         if (t < p.batch && r < p.rows) p.Y[(size_t)t * p.rows + r] = sum;
@@ -1156,7 +1185,6 @@ struct RoundParams {
 };
 
 // NM = 2: the gate | up pair (W0, W1 of rows0 rows each; gelu(W0 x) * (W1 x) to Y0)
-constexpr int kRoundTile = 32 * 144 / 4;      // 32 rows of a superblock
 template <int NM>
 __global__ __launch_bounds__(512, 4) void q4k_mm_round_kernel(RoundParams p)
 {
@@ -1190,12 +1218,7 @@ __global__ __launch_bounds__(512, 4) void q4k_mm_round_kernel(RoundParams p)
         const uint32_t row_bytes = (uint32_t)nsb * 144u;
 #pragma unroll
         for (int m = 0; m < NM; m++) {
-            const uint8_t *blk = (m ? p.W1 : W) + (size_t)r0 * row_bytes + (size_t)sbc * 144;
-#pragma unroll
-            for (int i = 0; i < 5; i++) {
-                const int c = 64 * i + lane, row = c / 9;
-                if (i < 4 || lane < 32) to_lds16(blk, (uint32_t)min(row, last) * row_bytes + 16u * (uint32_t)(c % 9), l0 + (uint32_t)(m * kRoundTile * 4 + i * 1024));
-            }
+            ask_q4k_tile((m ? p.W1 : W) + (size_t)r0 * row_bytes + (size_t)sbc * 144, row_bytes, last, lane, l0 + (uint32_t)(m * kRoundTile * 4));
         }
         const h8 *xa = reinterpret_cast<const h8 *>(p.Xp) + (size_t)sbc * 16 * 64 + lane;
         h8 a[16];
@@ -1634,11 +1657,13 @@ int launch_mul_mm(const ksh_kernel &k, const LaunchArgs &a, hipStream_t st)
         p.Xf = Xf; p.SxA = SxA;
         const dim3 sg((rows + 31) / 32);
         const int mt = batch <= 32 ? 1 : 2;
-        const size_t lds = (size_t)8 * mt * 16 * 64 * 4;
-        if (f32x && mt == 1) hipLaunchKernelGGL((q4k_mm_skinny_kernel<1, true>), sg, dim3(512), lds, st, p, Xf_lo, SxA_lo, 1.0f / 2048.0f);
-        else if (f32x) hipLaunchKernelGGL((q4k_mm_skinny_kernel<2, true>), sg, dim3(512), lds, st, p, Xf_lo, SxA_lo, 1.0f / 2048.0f);
-        else if (mt == 1) hipLaunchKernelGGL((q4k_mm_skinny_kernel<1, false>), sg, dim3(512), lds, st, p, Xf, SxA, 0.f);
-        else hipLaunchKernelGGL((q4k_mm_skinny_kernel<2, false>), sg, dim3(512), lds, st, p, Xf, SxA, 0.f);
+        const bool pieces = skinny_pieces(mt, f32x, (int)(cols / 256));
+        const size_t lds = (size_t)8 * skinny_wave(mt, pieces) * 4;
+        auto launch = [&](auto kernel) { hipLaunchKernelGGL(kernel, sg, dim3(512), lds, st, p, Xf_lo, SxA_lo, f32x ? 1.0f / 2048.0f : 0.f); };
+        if (f32x && mt == 2) launch(q4k_mm_skinny_kernel<2, true, false>);
+        else if (f32x) pieces ? launch(q4k_mm_skinny_kernel<1, true, true>) : launch(q4k_mm_skinny_kernel<1, true, false>);
+        else if (mt == 2) pieces ? launch(q4k_mm_skinny_kernel<2, false, true>) : launch(q4k_mm_skinny_kernel<2, false, false>);
+        else pieces ? launch(q4k_mm_skinny_kernel<1, false, true>) : launch(q4k_mm_skinny_kernel<1, false, false>);
         const hipError_t e2 = hipGetLastError();
         return e2 == hipSuccess ? 0 : hip_fail(e2, "mul_mm (small batch) launch");
     }
@@ -1797,7 +1822,8 @@ int bind_matvec_batch(ksh_kernel &k)
     k.variant = (want == 32 || (want == 0 && can_skinny && !long_rows)) ? 1 : 0;
     k.info.sched = k.desc.sched;
     if (k.variant == 1) {
-        set_launch(k, (uint32_t)((rows + 31) / 32), 1, 1, 512, (uint32_t)(8 * (batch <= 32 ? 1 : 2) * 16 * 64 * 4));
+        const int mt = batch <= 32 ? 1 : 2;
+        set_launch(k, (uint32_t)((rows + 31) / 32), 1, 1, 512, (uint32_t)(8 * skinny_wave(mt, skinny_pieces(mt, f32x, (int)(cols / 256))) * 4));
         k.info.sched.tg = 512; k.info.sched.nsg = 8; k.info.sched.nr0 = 32; k.info.sched.k_split = 8; k.info.sched.lds_tile = 16;
         set_name(k, "mul_mm_q4k_skinny_32xT%d%s", batch <= 32 ? 32 : 64, f32x ? "_f32x" : "");
         k.launch = launch_mul_mm;

@@ -390,6 +390,28 @@ def test_mul_mm_bf16_rows_at_the_edges_of_its_tiles(ctx, rows, batch, cols, ks, 
         assert float(rel_err(got[t], oracle.matvec_f64(oracle.Q4K, w, rows, cols, xs[t])).max()) <= 2e-5, t
 
 
+@pytest.mark.parametrize("xdt", [DType.F32, DType.BF16])
+@pytest.mark.parametrize("rows,batch,cols", [(1, 2, 1024), (31, 32, 1280), (33, 33, 2048), (65, 64, 2304), (300, 3, 6400), (97, 50, 4352)])
+def test_mul_mm_small_batch_edges(ctx, xdt, rows, batch, cols):
+    """The small-batch form on both sides of its rule for the weights' way in (4 and 5 superblocks; one and two parts; up to and
+    past 32 tokens), waves without a superblock, with one and with several, a row past a tile or short of it.  Against float64:
+    2e-5, as for the tiles."""
+    w = synth.q4k_blocks(rows * cols // 256, 735)
+    x = synth.normal_f32(batch * cols, 736)
+    xb = ctx.buffer_f32(x)
+    if xdt == DType.BF16:
+        x, raw = synth.bf16_round(x)
+        xb = ctx.buffer_bytes(raw)
+    k = ctx.compile(hip.make_desc(hip.Kind.MATVEC_BATCH, (rows, cols, batch), (DType.Q4K, xdt, DType.F32), (), dict(nr0=32)))
+    assert "skinny" in k.name
+    y = ctx.buffer_empty_f32(batch * rows)
+    ctx.encode_multi(k, [ctx.buffer_bytes(w), xb], [y])
+    ctx.synchronize()
+    got = ctx.read_f32(y, batch * rows).reshape(batch, rows)
+    for t in range(batch):
+        assert float(rel_err(got[t], oracle.matvec_f64(oracle.Q4K, w, rows, cols, x.reshape(batch, cols)[t])).max()) <= 2e-5, t
+
+
 @pytest.mark.parametrize("rows,batch,cols,ks,at,shape", [
     (1, 1, 256, 1, 0, "32x128"), (33, 31, 768, 3, 2, "32x128"), (129, 33, 2816, 7, 14, "32x128"), (127, 32, 256, 1, 6, "32x128"),
     (4095, 65, 2816, 1, 10, "32x128"), (4097, 63, 6144, 8, 8, "64x128"), (4130, 64, 7936, 5, 4, "64x128"), (4223, 193, 768, 1, 12, "32x128")])
