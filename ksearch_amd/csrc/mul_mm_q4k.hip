@@ -439,12 +439,16 @@ MmPlan mm_plan_bf16(bool q6, int row_tiles, int nsb, int64_t batch, int64_t rows
     return best;
 }
 
+// (the small-batch form's way of loading, see q4k_mm_skinny_kernel)
+constexpr bool skinny_pieces(int mt, bool lo, int nsb) { return mt == 1 ? nsb > 4 : !lo && nsb % 8 == 0; }
+
 // The small-batch form beside it (Q4_K, bf16), with its preparation: a workgroup of eight waves per 32 rows, superblocks dealt to
 // the waves (300 .. 12288 rows of 512 .. 6144 columns).
 float mm_skinny_us(int64_t rows, int nsb, int64_t batch)
 {
     const float turns = std::max(1.f, (float)((rows + 31) / 32) / 128.f - 1.f), each = (float)nsb / 8.f;
-    return batch <= 32 ? 5.4f + 2.f * each * turns : 6.2f + 4.3f * std::max(each, 0.45f) * turns;
+    if (batch <= 32) return 5.4f + 2.f * each * turns;
+    return skinny_pieces(2, false, nsb) ? 6.2f + 4.3f * each * turns : 6.4f + 5.f * std::max(each, 0.45f) * turns;
 }
 
 // Bf16 rows of Q6_K products as they are (the kernel's ROWS form): the conversion between the matrix instructions costs 0.42
@@ -856,15 +860,21 @@ __device__ __forceinline__ void ask_q4k_tile(const uint8_t *blk, uint32_t row_by
 // (each converted weight is used for both), so f32 activations cost one launch.
 //
 // PIECES: the weights come as pieces of 16 bytes by way of LDS, which costs a second round trip and saves most of the time in L1.
-// Measured (us, rows a lane -> pieces; 1536 rows, or as said): up to 32 tokens 2048 columns 8.4 -> 6.9, 6144 15.2 -> 11.0, 12288
-// rows of 2048 11.8 -> 9.1; 33 .. 64 tokens 10.6 -> 9.9, 21 -> 19, 17 -> 15.  Where two waves do everything (512 columns) it is
-// the round trip that counts, 5.8 -> 6.3 and 8.0 -> 8.5: rows a lane up to 4 superblocks.  So also for two parts of 64 tokens,
-// which have no registers left for it.
+// Measured (us, rows a lane -> pieces; 3045 rows, or as said): up to 32 tokens 1280 columns 6.9 -> 6.5, 2048 8.2 -> 6.7, 6144 15.2
+// -> 11.0, 12288 rows of 2048 11.8 -> 9.1; where four waves or fewer do everything it is the round trip that counts (512 columns
+// 5.8 -> 6.3).  33 .. 64 tokens: 2048 columns 10.2 -> 9.3, 4096 15.3 -> 13.7, 6144 20.7 -> 18.4, where all eight waves have the
+// same number of superblocks and L1 is busy throughout; else even or slower (1280 8.4 -> 8.7, 1792 9.1 -> 9.2, 2304 11.6 -> 12.1,
+// 3072 12.4 -> 12.9, 5120 17.3 -> 17.3).  Two parts of 64 tokens have no registers left for it.
 constexpr int skinny_wave(int mt, bool pieces) { return pieces && mt == 1 ? kRoundTile : mt * 16 * 64; }      // floats of LDS
-constexpr bool skinny_pieces(int mt, bool lo, int nsb) { return nsb > 4 && !(mt == 2 && lo); }
+struct SkinnyParams {      // (its own: arguments are copied at every launch, and two launches of 3 us are what such a call is)
+    const uint8_t *W;
+    const _Float16 *Xf, *SxA, *Xf_lo, *SxA_lo;
+    float *Y;
+    int rows, cols, batch;
+    float lo_scale;
+};
 template <int MT, bool HAS_LO, bool PIECES>
-__global__ __launch_bounds__(512) void q4k_mm_skinny_kernel(MmParams p, const _Float16 *__restrict__ Xf_lo, const _Float16 *__restrict__ SxA_lo,
-                                                             float lo_scale)
+__global__ __launch_bounds__(512) void q4k_mm_skinny_kernel(SkinnyParams p)
 {
     extern __shared__ __attribute__((aligned(16))) float red[];   // [8][WAVE]: a wave's weight rows, then its [MT][16][64]
     constexpr int WAVE = skinny_wave(MT, PIECES);
@@ -882,10 +892,10 @@ __global__ __launch_bounds__(512) void q4k_mm_skinny_kernel(MmParams p, const _F
     for (int mt = 0; mt < MT; mt++) {
         const size_t frag0 = (size_t)min(mt, ntt - 1) * (p.cols / 16) * 64 + lane;
         xa[mt] = reinterpret_cast<const h8 *>(p.Xf) + frag0;
-        xl[mt] = reinterpret_cast<const h8 *>(HAS_LO ? Xf_lo : p.Xf) + frag0;
+        xl[mt] = reinterpret_cast<const h8 *>(HAS_LO ? p.Xf_lo : p.Xf) + frag0;
         const size_t so = (size_t)min(mt * 32 + n, p.batch - 1) * nsb * 32 + 8 * h;   // + sb * 32 + 16 * ks
         sxa[mt] = p.SxA + so;
-        sxl[mt] = (HAS_LO ? SxA_lo : p.SxA) + so;
+        sxl[mt] = (HAS_LO ? p.SxA_lo : p.SxA) + so;
     }
     f16v F[MT], Fl[MT];
     const f16v kZero16 = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
@@ -982,7 +992,7 @@ __global__ __launch_bounds__(512) void q4k_mm_skinny_kernel(MmParams p, const _F
     for (int mt = 0; mt < MT; mt++)
 #pragma unroll
         for (int i = 0; i < 16; i++)
-            red[wave * WAVE + (mt * 16 + i) * 64 + lane] = HAS_LO ? fmaf(lo_scale, Fl[mt][i], F[mt][i]) : F[mt][i];
+            red[wave * WAVE + (mt * 16 + i) * 64 + lane] = HAS_LO ? fmaf(p.lo_scale, Fl[mt][i], F[mt][i]) : F[mt][i];
     __syncthreads();
     for (int o = tid; o < MT * 16 * 64; o += 512) {
         float sum = 0.f;
@@ -1643,6 +1653,21 @@ int launch_mul_mm(const ksh_kernel &k, const LaunchArgs &a, hipStream_t st)
         if (tile) hipLaunchKernelGGL(mm_prep_x_kernel<true>, xg, dim3(256), 0, st, (const uint16_t *)a.in[1], Xf, SxA, batch, cols);
         else hipLaunchKernelGGL(mm_prep_x_kernel<false>, xg, dim3(256), 0, st, (const uint16_t *)a.in[1], Xf, SxA, batch, cols);
     }
+    if (k.variant == 1) {
+        // the small-batch form: one launch, the low parts riding along
+        const SkinnyParams sp{(const uint8_t *)a.in[0], Xf, SxA, Xf_lo, SxA_lo, (float *)a.out[0], rows, cols, batch, 1.0f / 2048.0f};
+        const dim3 sg((rows + 31) / 32);
+        const int mt = batch <= 32 ? 1 : 2;
+        const bool pieces = skinny_pieces(mt, f32x, cols / 256);
+        const size_t lds = (size_t)8 * skinny_wave(mt, pieces) * 4;
+        auto launch = [&](auto kernel) { hipLaunchKernelGGL(kernel, sg, dim3(512), lds, st, sp); };
+        if (f32x && mt == 2) launch(q4k_mm_skinny_kernel<2, true, false>);
+        else if (f32x) pieces ? launch(q4k_mm_skinny_kernel<1, true, true>) : launch(q4k_mm_skinny_kernel<1, true, false>);
+        else if (mt == 2) pieces ? launch(q4k_mm_skinny_kernel<2, false, true>) : launch(q4k_mm_skinny_kernel<2, false, false>);
+        else pieces ? launch(q4k_mm_skinny_kernel<1, false, true>) : launch(q4k_mm_skinny_kernel<1, false, false>);
+        const hipError_t e2 = hipGetLastError();
+        return e2 == hipSuccess ? 0 : hip_fail(e2, "mul_mm (small batch) launch");
+    }
     MmParams p;
     p.W = (const uint8_t *)a.in[0];
     p.Y = (float *)a.out[0];
@@ -1652,21 +1677,6 @@ int launch_mul_mm(const ksh_kernel &k, const LaunchArgs &a, hipStream_t st)
     p.W1 = rows1 ? (const uint8_t *)a.in[2] : p.W; p.W2 = rows2 ? (const uint8_t *)a.in[3] : p.W;
     const bool unfolded_out = k.desc.dims[6] == 1, pair = k.desc.dims[6] == 3;
     p.Y1 = rows1 && !unfolded_out && !pair ? (float *)a.out[1] : p.Y; p.Y2 = rows2 && !unfolded_out ? (float *)a.out[2] : p.Y;
-    if (k.variant == 1) {
-        // the small-batch form: one launch, the low parts riding along
-        p.Xf = Xf; p.SxA = SxA;
-        const dim3 sg((rows + 31) / 32);
-        const int mt = batch <= 32 ? 1 : 2;
-        const bool pieces = skinny_pieces(mt, f32x, (int)(cols / 256));
-        const size_t lds = (size_t)8 * skinny_wave(mt, pieces) * 4;
-        auto launch = [&](auto kernel) { hipLaunchKernelGGL(kernel, sg, dim3(512), lds, st, p, Xf_lo, SxA_lo, f32x ? 1.0f / 2048.0f : 0.f); };
-        if (f32x && mt == 2) launch(q4k_mm_skinny_kernel<2, true, false>);
-        else if (f32x) pieces ? launch(q4k_mm_skinny_kernel<1, true, true>) : launch(q4k_mm_skinny_kernel<1, true, false>);
-        else if (mt == 2) pieces ? launch(q4k_mm_skinny_kernel<2, false, true>) : launch(q4k_mm_skinny_kernel<2, false, false>);
-        else pieces ? launch(q4k_mm_skinny_kernel<1, false, true>) : launch(q4k_mm_skinny_kernel<1, false, false>);
-        const hipError_t e2 = hipGetLastError();
-        return e2 == hipSuccess ? 0 : hip_fail(e2, "mul_mm (small batch) launch");
-    }
     const bool cut = k.desc.dims[6] == 2;
     const dim3 grid(k.info.grid[0], k.info.grid[1], k.info.grid[2]);
     p.Xf = rows_direct ? (const _Float16 *)a.in[1] : Xf;
