@@ -852,7 +852,7 @@ __device__ __forceinline__ void ask_q4k_tile(const uint8_t *blk, uint32_t row_by
 // A prompt remainder or a round of decoding slots is a few dozen tokens: the 128 x 128 tile then leaves most of the
 // chip idle (rows / 128 workgroups) and half of every tile empty.  Here a workgroup owns 32 weight rows and all
 // tokens; its 8 waves split the row's superblocks between them (K-split inside the workgroup, folded through LDS at
-// the end, so the sum order is fixed) and every wave reads its weights straight from memory in the order the matrix
+// the end, so the sum order is fixed) and every wave reads its weights, from memory or LDS, in the order the matrix
 // instruction wants its B operand: lane (n, h) = (lane % 32, lane / 32) owns row n and, in every 16-column slice,
 // columns 8h .. 8h+7 -- per 64-column group the low and the high nibbles of bytes 8h .. 8h+7 and 16+8h .. 16+8h+7,
 // two 8-byte loads.  Conversion (sc*n as exact f16, biased by 1024), the per-superblock scale and the bias / min
@@ -861,7 +861,7 @@ __device__ __forceinline__ void ask_q4k_tile(const uint8_t *blk, uint32_t row_by
 //
 // PIECES: the weights come as pieces of 16 bytes by way of LDS, which costs a second round trip and saves most of the time in L1.
 // Measured (us, rows a lane -> pieces; 3045 rows, or as said): up to 32 tokens 1280 columns 6.9 -> 6.5, 2048 8.2 -> 6.7, 6144 15.2
-// -> 11.0, 12288 rows of 2048 11.8 -> 9.1; where four waves or fewer do everything it is the round trip that counts (512 columns
+// -> 11.0, 12288 rows of 2048 11.8 -> 9.1 (two parts 2048 9.5 -> 8.4, 6144 19.0 -> 16.3, 2560 12.4 -> 12.6); where four waves or fewer do everything it is the round trip that counts (512 columns
 // 5.8 -> 6.3).  33 .. 64 tokens: 2048 columns 10.2 -> 9.3, 4096 15.3 -> 13.7, 6144 20.7 -> 18.4, where all eight waves have the
 // same number of superblocks and L1 is busy throughout; else even or slower (1280 8.4 -> 8.7, 1792 9.1 -> 9.2, 2304 11.6 -> 12.1,
 // 3072 12.4 -> 12.9, 5120 17.3 -> 17.3).  Two parts of 64 tokens have no registers left for it.
