@@ -142,6 +142,39 @@ __device__ __forceinline__ void to_lds4(const uint8_t *base, uint32_t off, uint3
     asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dword %1, %2" ::"s"(dst), "v"(off), "s"(base) : "memory");
 }
 
+// Values of LDS asked for ahead of their use: ordinary loads, so that a copy or a spill of one on its way is waited for by the
+// compiler like any other use.  Their place is held by what stands around them (scheduling barriers, statements that clobber
+// memory); lds_left waits where the kernel wants it, once for several values, in a form that the compiler counts; arrived keeps a
+// value as it came and its uses behind that place.  (As reads in asm, which the compiler takes for done: 2048 tokens of heads of 512
+// 314 us or, so, 311, heads of 256 79 and 79; GEMM, 2048 tokens, 1536 x 12288 193 or 194, gate | up of 12288 x 1536 284 and 284.)
+template <int OFF, class V>
+__device__ __forceinline__ void lds_ask(V &v, uint32_t addr)
+{
+    v = *(const __attribute__((address_space(3))) V *)(uintptr_t)(addr + OFF);
+}
+// one or two bytes, widened by the load itself.  (The annotation, which is no instruction, keeps the widening where the load is: moved
+// behind a branch to where the value is used, it would be an instruction of its own.)
+template <int OFF, class N>
+__device__ __forceinline__ void lds_ask_wide(uint32_t &v, uint32_t addr)
+{
+    N n;
+    lds_ask<OFF>(n, addr);
+    v = __builtin_annotation((uint32_t)n, "widened by the load");
+}
+template <int N>
+__device__ __forceinline__ void lds_left()
+{
+    asm volatile("" ::: "memory");
+    __builtin_amdgcn_s_waitcnt(0xC07F | (N << 8));     // lgkmcnt(N) alone
+    asm volatile("" ::: "memory");
+    __builtin_amdgcn_sched_barrier(0);
+}
+template <class V>
+__device__ __forceinline__ void arrived(V &v)
+{
+    asm volatile("" : "+v"(v));
+}
+
 constexpr int kWave = 64;
 
 // A zero the compiler cannot see through, in a vector register.  Added to the index of a load whose address is the

@@ -50,20 +50,9 @@ struct MmRows {
     static_assert(WM * WN == 4 && TT * PARTS <= 4 && MT * PARTS >= 2 && NT <= 2, "a wave fetches TF fragments of a half step, from one part of one token tile");
 };
 
-// Memory operations that the compiler does not count: it would wait for all that is on its way into LDS in front of every read
-// of LDS.  Read values are used behind lds_wait and arrived only; what comes into LDS is waited for by the number of younger
-// operations, so every one of them is issued whatever the sizes (addresses are clamped instead).
-template <int OFF, class V>
-__device__ __forceinline__ void lds_ask(V &v, uint32_t addr)
-{
-    asm volatile("ds_read_b128 %0, %1 offset:%2" : "=v"(v) : "v"(addr), "n"(OFF));
-}
-__device__ __forceinline__ void lds_wait() { asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory"); }
-template <class V>
-__device__ __forceinline__ void arrived(V &v)
-{
-    asm volatile("" : "+v"(v));
-}
+// What comes from memory into LDS is not counted by the compiler, which would wait for all of it in front of every read of LDS: it
+// is waited for by the number of younger operations, so every one of them is issued whatever the sizes (addresses are clamped
+// instead).
 
 template <class S, bool CUT, bool PAIR>
 __global__ __launch_bounds__(S::kThreads, 2) void q4k_mm_rows_kernel(MmParams p)
@@ -278,7 +267,7 @@ __global__ __launch_bounds__(S::kThreads, 2) void q4k_mm_rows_kernel(MmParams p)
     read_group(n3);
     read_header();
     read_rows(n0, n0, a[0]);
-    lds_wait();
+    lds_left<0>();
     settle(q[0]); settle(q[1]); settle(q[2]); settle(q[3]); settle(hdr); settle(a[0]);
     scales();
 #pragma unroll
@@ -384,7 +373,7 @@ __global__ __launch_bounds__(S::kThreads, 2) void q4k_mm_rows_kernel(MmParams p)
             }
         }
         __builtin_amdgcn_sched_barrier(0);
-        lds_wait();
+        lds_left<0>();
         settle(a[set ^ 1]);
         if constexpr (take0) { settle(q[0]); settle(hdr); }
         if constexpr (take3) { settle(q[1]); settle(q[2]); settle(q[3]); }
@@ -431,10 +420,8 @@ __global__ __launch_bounds__(S::kThreads, 2) void q4k_mm_rows_kernel(MmParams p)
         f32x4_t inv[4];
         if (S::LO) {
 #pragma unroll
-            for (int i4 = 0; i4 < 4; i4++) asm volatile("ds_read_b128 %0, %1" : "=v"(inv[i4]) : "v"(l0 + kAtInv + 4u * (uint32_t)(tb - t0 + 8 * i4)));
-            lds_wait();
-#pragma unroll
-            for (int i4 = 0; i4 < 4; i4++) arrived(inv[i4]);
+            for (int i4 = 0; i4 < 4; i4++) lds_ask<0>(inv[i4], l0 + kAtInv + 4u * (uint32_t)(tb - t0 + 8 * i4));
+            lds_left<0>();
         }
 #pragma unroll
         for (int nt = 0; nt < NT; nt += PAIR ? 2 : 1) {

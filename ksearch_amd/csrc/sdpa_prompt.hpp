@@ -48,38 +48,6 @@ __device__ __forceinline__ uint32_t lds_base(uint32_t addr)
     return addr;
 }
 
-// Reads on their way while the last block's are worked on: the compiler, left to itself, asks for everything at once (and keeps
-// it in memory) or, held to a block at a time, for a block's operands when it needs them.  Used behind lds_left and arrived only.
-template <int OFF, class V>
-__device__ __forceinline__ void ask16(V &v, uint32_t addr)
-{
-    asm volatile("ds_read_b128 %0, %1 offset:%2" : "=v"(v) : "v"(addr), "n"(OFF));
-}
-template <int OFF>
-__device__ __forceinline__ void ask4(float &v, uint32_t addr)
-{
-    asm volatile("ds_read_b32 %0, %1 offset:%2" : "=v"(v) : "v"(addr), "n"(OFF));
-}
-template <int OFF>
-__device__ __forceinline__ void ask2(uint32_t &v, uint32_t addr)
-{
-    asm volatile("ds_read_u16 %0, %1 offset:%2" : "=v"(v) : "v"(addr), "n"(OFF));
-}
-template <int OFF>
-__device__ __forceinline__ void ask1(uint32_t &v, uint32_t addr)
-{
-    asm volatile("ds_read_u8 %0, %1 offset:%2" : "=v"(v) : "v"(addr), "n"(OFF));
-}
-template <int N>
-__device__ __forceinline__ void lds_left()
-{
-    asm volatile("s_waitcnt lgkmcnt(%0)" ::"n"(N) : "memory");
-}
-template <class V>
-__device__ __forceinline__ void arrived(V &v)
-{
-    asm volatile("" : "+v"(v));
-}
 template <int I, int N, class F>
 __device__ __forceinline__ void each(F &f)
 {
@@ -262,22 +230,24 @@ __global__ __launch_bounds__((SdpaPrompt<HD, T>::WAVES * 64), 2) void sdpa_promp
 #pragma unroll
                     for (int r = 0; r < 4; r++) acc[k][t][r] = 0.f;
             struct Operands { f4v dk[TRK / 16]; uint32_t lo[TRK / 16], hi[TRK / 16]; h8v q[T]; float q24[T]; } op[2];
-            constexpr int ASKS = 3 * (TRK / 16) + 2 * T;
+            // (a block's operands are on their way while the last block's are worked on: the compiler, left to itself, asks for
+            // everything at once and keeps it in memory or, held to a block at a time, for a block's operands when it needs them)
+            constexpr int ASKS = 3 * (TRK / 16) + T + 1;    // (q24 of two tokens is one operation)
             auto ask_block = [&](auto btag) __attribute__((always_inline)) {
                 constexpr int b = decltype(btag)::value;
                 Operands &o = op[b & 1];
                 auto half = [&](auto ttag) __attribute__((always_inline)) {
                     constexpr int t = decltype(ttag)::value;
-                    ask2<16 * t * S::KPITCH + 18 * b>(o.lo[t], kcode);
-                    ask2<16 * t * S::KPITCH + 18 * b + 2>(o.hi[t], kcode);
-                    ask16<(b * TRK + 16 * t) * 4>(o.dk[t], kscale);
+                    lds_ask_wide<16 * t * S::KPITCH + 18 * b, uint16_t>(o.lo[t], kcode);
+                    lds_ask_wide<16 * t * S::KPITCH + 18 * b + 2, uint16_t>(o.hi[t], kcode);
+                    lds_ask<(b * TRK + 16 * t) * 4>(o.dk[t], kscale);
                 };
                 each<0, TRK / 16>(half);
-                ask16<b * 1024>(o.q[0], qop_at);
-                ask4<b * 256>(o.q24[0], qsum_at);
+                lds_ask<b * 1024>(o.q[0], qop_at);
+                lds_ask<b * 256>(o.q24[0], qsum_at);
                 if constexpr (T == 2) {
-                    ask16<S::kQ + b * 1024>(o.q[T - 1], qop_at);
-                    ask4<S::kQ + b * 256>(o.q24[T - 1], qsum_at);
+                    lds_ask<S::kQ + b * 1024>(o.q[T - 1], qop_at);
+                    lds_ask<S::kQ + b * 256>(o.q24[T - 1], qsum_at);
                 }
             };
             ask_block(std::integral_constant<int, 0>{});
@@ -288,9 +258,7 @@ __global__ __launch_bounds__((SdpaPrompt<HD, T>::WAVES * 64), 2) void sdpa_promp
                 Operands &o = op[b & 1];
                 h8v codes[TRK / 16];
 #pragma unroll
-                for (int t = 0; t < TRK / 16; t++) {
-                    arrived(o.lo[t]); arrived(o.hi[t]); arrived(o.dk[t]);
-                }
+                for (int t = 0; t < TRK / 16; t++) arrived(o.dk[t]);
 #pragma unroll
                 for (int k = 0; k < T; k++) { arrived(o.q[k]); arrived(o.q24[k]); }
 #pragma unroll
@@ -375,12 +343,12 @@ __global__ __launch_bounds__((SdpaPrompt<HD, T>::WAVES * 64), 2) void sdpa_promp
                 Operands &o = op[b & 1];
                 auto rows2 = [&](auto itag) __attribute__((always_inline)) {
                     constexpr int i = decltype(itag)::value, at = (16 * ((2 * i) >> 2) + ((2 * i) & 3)) * S::ROWBV + 18 * b;
-                    ask1<at>(o.a[i], vcode);
-                    ask1<at + S::ROWBV>(o.b[i], vcode);
+                    lds_ask_wide<at, uint8_t>(o.a[i], vcode);
+                    lds_ask_wide<at + S::ROWBV, uint8_t>(o.b[i], vcode);
                 };
                 each<0, 4>(rows2);
-                ask16<b * 128>(o.d[0], vscale);
-                ask16<b * 128 + 64>(o.d[1], vscale);
+                lds_ask<b * 128>(o.d[0], vscale);
+                lds_ask<b * 128 + 64>(o.d[1], vscale);
             };
             ask_block(std::integral_constant<int, 0>{});
             auto block = [&](auto btag) __attribute__((always_inline)) {
@@ -389,8 +357,6 @@ __global__ __launch_bounds__((SdpaPrompt<HD, T>::WAVES * 64), 2) void sdpa_promp
                 lds_left<b + 1 < NBV ? ASKS : 0>();
                 Operands &o = op[b & 1];
                 arrived(o.d[0]); arrived(o.d[1]);
-#pragma unroll
-                for (int i = 0; i < 4; i++) { arrived(o.a[i]); arrived(o.b[i]); }
                 const float dv[8] = {o.d[0][0], o.d[0][1], o.d[0][2], o.d[0][3], o.d[1][0], o.d[1][1], o.d[1][2], o.d[1][3]};
                 uint32_t vlo[4], vhi[4];
 #pragma unroll
