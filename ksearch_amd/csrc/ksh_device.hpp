@@ -132,14 +132,15 @@ __device__ __forceinline__ void act_st(float *p, size_t i, float v)
 }
 
 // 16 (or 4) bytes a lane straight from memory into LDS: lane l's at dst + 16 l (4 l).  The compiler does not count these (it
-// answers them with a wait for all in front of every read of LDS): whoever asks waits by the number of younger operations.
+// answers them with a wait for all in front of every read of LDS): whoever asks waits by the number of younger operations.  The place
+// in LDS goes by m0, which the compiler writes.
 __device__ __forceinline__ void to_lds16(const uint8_t *base, uint32_t off, uint32_t dst)
 {
-    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(dst), "v"(off), "s"(base) : "memory");
+    asm volatile("s_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" ::"v"(off), "s"(base), "{m0}"(dst) : "memory");
 }
 __device__ __forceinline__ void to_lds4(const uint8_t *base, uint32_t off, uint32_t dst)
 {
-    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dword %1, %2" ::"s"(dst), "v"(off), "s"(base) : "memory");
+    asm volatile("s_nop 0\n\tglobal_load_lds_dword %0, %1" ::"v"(off), "s"(base), "{m0}"(dst) : "memory");
 }
 
 // Values of LDS asked for ahead of their use: ordinary loads, so that a copy or a spill of one on its way is waited for by the

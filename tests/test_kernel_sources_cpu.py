@@ -44,3 +44,17 @@ def test_no_asm_returns_a_value_that_is_on_its_way(file, template, rest):
     outputs = rest.split(":")[1] if ":" in rest else ""
     if LOADS.search(template):
         assert "=" not in outputs and "+" not in outputs, f"{file}: {template}"
+
+
+# Registers with a name of their own: the compiler has to know what a statement writes there, and what it reads (a request straight
+# into LDS reads its place there from m0).
+WRITES = re.compile(r"\b[sv]_\w+\s+(m0|vcc|exec|scc)\b")
+
+
+@pytest.mark.parametrize("file,template,rest", statements())
+def test_asm_names_the_registers_it_uses(file, template, rest):
+    parts = rest.split(":")
+    for reg in WRITES.findall(template):
+        assert len(parts) > 3 and f'"{reg}"' in parts[3], f"{file}: {reg} in {template}"
+    if re.search(r"_load_lds_|_load_\w+ .*\blds\b", template):
+        assert '"{m0}"' in rest, f"{file}: {template}"
