@@ -444,6 +444,12 @@ __global__ __launch_bounds__((SdpaPrompt<HD, T>::WAVES * 64), 2) void sdpa_promp
         }
         asm volatile("s_waitcnt vmcnt(0)" ::: "memory");         // (nothing is on its way into what the states are written over)
 
+        // (worked out again from nothing: kept through the loop, these would be in memory)
+        uint32_t all = ~0u;
+        asm volatile("" : "+s"(all));
+        const int elane = (int)__builtin_amdgcn_mbcnt_hi(all, __builtin_amdgcn_mbcnt_lo(all, 0u)), ecol = elane & 15, eq4 = elane >> 4;
+        const uint32_t eodd_mask = 0u - (uint32_t)(eq4 & 1);
+
         // ---- the waves' states meet in LDS, one head's dimension a thread folds them in the order of a workgroup of one token:
         // tile t of B is tile t + delta here
         __syncthreads();
@@ -453,29 +459,30 @@ __global__ __launch_bounds__((SdpaPrompt<HD, T>::WAVES * 64), 2) void sdpa_promp
             float *ow = reinterpret_cast<float *>(lds_raw + k * S::kState);   // [V half][NW][8][256]
             float *mlw = ow + WAVES * 8 * 256;                              // [NW][8][2]
             const float l_tot = xor32_sum(xor16_sum(l_run[k]));
-            const int odd = q4 >> 1;
+            const int odd = eq4 >> 1;
 #pragma unroll
             for (int b = 0; b < NBV; b++) {
                 const uint32_t tcol = as_u32(24.f * xor32_sum(xor16_sum(Tl[k][b])));
 #pragma unroll
                 for (int r = 0; r < 4; r++) {
                     const uint32_t t_lo = (uint32_t)__builtin_amdgcn_readlane((int)tcol, r), t_hi = (uint32_t)__builtin_amdgcn_readlane((int)tcol, 4 + r);
-                    const float t24 = as_f32((t_lo & ~odd_mask) | (t_hi & odd_mask));
+                    const float t24 = as_f32((t_lo & ~eodd_mask) | (t_hi & eodd_mask));
                     const auto sw = __builtin_amdgcn_permlane32_swap(as_u32(O[k][2 * b][r]), as_u32(O[k][2 * b + 1][r]), false, false);
-                    ow[((size_t)wave * 8 + 4 * (q4 & 1) + r) * 256 + col + 16 * odd + 32 * b] = (as_f32(sw[0]) - t24) + as_f32(sw[1]);
+                    ow[((size_t)wave * 8 + 4 * (eq4 & 1) + r) * 256 + ecol + 16 * odd + 32 * b] = (as_f32(sw[0]) - t24) + as_f32(sw[1]);
                 }
             }
-            if (lane < 8 && wave < NW) { mlw[(wave * 8 + lane) * 2] = m_run[k]; mlw[(wave * 8 + lane) * 2 + 1] = l_tot; }
+            if (elane < 8 && wave < NW) { mlw[(wave * 8 + elane) * 2] = m_run[k]; mlw[(wave * 8 + elane) * 2 + 1] = l_tot; }
         }
         __syncthreads();
 #pragma unroll
         for (int k = 0; k < T; k++) {
             if (k && !joint) break;
             const float *ow = reinterpret_cast<const float *>(lds_raw + k * S::kState), *mlw = ow + WAVES * 8 * 256;
-            const int turn = k ? delta : 0, tok = k ? B.tok : A.tok;
+            static_assert(NT == HD, "a thread has one dimension of every head");
+            const int turn = k ? delta : 0, tok = k ? B.tok : A.tok, d = wave * 64 + elane;
 #pragma unroll
-            for (int o = tid; o < 8 * HD; o += NT) {
-                const int h = o / HD, d = o % HD, hq = head0 + h;      // (h is the same for a whole wave)
+            for (int h = 0; h < 8; h++) {
+                const int hq = head0 + h;
                 if (h >= groups) break;
                 float M = -1.0e30f;
 #pragma unroll

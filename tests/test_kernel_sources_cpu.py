@@ -1,8 +1,12 @@
-"""What the kernels' inline assembly may say, read from the sources: the compiler has to know everything it could break."""
+"""What the kernels' inline assembly may say, read from the sources: the compiler has to know everything it could break.  And what
+the compiler made of the kernels that sit at the edge of the register file, read from the built library's metadata."""
 import os
 import re
+import struct
 
 import pytest
+
+from ksearch_amd import _build
 
 CSRC = os.path.join(os.path.dirname(__file__), "..", "ksearch_amd", "csrc")
 
@@ -58,3 +62,45 @@ def test_asm_names_the_registers_it_uses(file, template, rest):
         assert len(parts) > 3 and f'"{reg}"' in parts[3], f"{file}: {reg} in {template}"
     if re.search(r"_load_lds_|_load_\w+ .*\blds\b", template):
         assert '"{m0}"' in rest, f"{file}: {template}"
+
+
+def kernels():
+    """{kernel: its metadata} of every gfx950 code object in the built library."""
+    msgpack = pytest.importorskip("msgpack")
+    lib, magic, out, at = open(_build.LIB_PATH, "rb").read(), b"__CLANG_OFFLOAD_BUNDLE__", {}, 0
+    while (at := lib.find(magic, at)) >= 0:
+        n, = struct.unpack_from("<Q", lib, at + 24)
+        entry = at + 32
+        for _ in range(n):
+            offset, size, id_len = struct.unpack_from("<QQQ", lib, entry)
+            name = lib[entry + 24:entry + 24 + id_len]
+            entry += 24 + id_len
+            if not size or _build.ARCH.encode() not in name:
+                continue
+            elf = lib[at + offset:at + offset + size]
+            table, = struct.unpack_from("<Q", elf, 0x28)
+            each, sections = struct.unpack_from("<HH", elf, 0x3A)
+            for i in range(sections):
+                kind, place = struct.unpack_from("<4xI16xQ", elf, table + i * each)
+                if kind != 7:                                  # SHT_NOTE
+                    continue
+                owner, length, note = struct.unpack_from("<III", elf, place)
+                if note == 32:                                 # NT_AMDGPU_METADATA
+                    begin = place + 12 + (owner + 3) // 4 * 4
+                    for k in msgpack.unpackb(elf[begin:begin + length])["amdhsa.kernels"]:
+                        out[k[".name"]] = k
+        at += len(magic)
+    return out
+
+
+# Kernels that fill their registers to fit two (or four) workgroups on a compute unit, and wait by the number of their requests: what
+# goes to memory and back beside those makes every such wait longer.
+FULL = re.compile(r"q[46]k_mm_rows_kernel|sdpa_prompt_kernel|q4k_mm_round_kernel|q4k_mm_skinny_kernel")
+
+
+def test_full_kernels_keep_their_values_in_registers():
+    found = {name: k for name, k in kernels().items() if FULL.search(name)}
+    assert len(found) >= 18
+    spilled = {name: (k[".vgpr_spill_count"], k[".private_segment_fixed_size"]) for name, k in found.items()
+               if k[".vgpr_spill_count"] or k[".private_segment_fixed_size"]}
+    assert not spilled
