@@ -439,8 +439,12 @@ MmPlan mm_plan_bf16(bool q6, int row_tiles, int nsb, int64_t batch, int64_t rows
     return best;
 }
 
-// (the small-batch form's way of loading, see q4k_mm_skinny_kernel)
-constexpr bool skinny_pieces(int mt, bool lo, int nsb) { return mt == 1 ? nsb > 4 : !lo && nsb % 8 == 0; }
+// (the small-batch form's way of loading, see the figures at q4k_mm_skinny_kernel)
+constexpr bool skinny_pieces(int mt, bool lo, int nsb)
+{
+    if (mt == 1) return lo ? nsb % 8 == 0 || nsb > 12 : nsb > 4;
+    return !lo && nsb % 8 == 0;
+}
 
 // The small-batch form beside it (Q4_K, bf16), with its preparation: a workgroup of eight waves per 32 rows, superblocks dealt to
 // the waves (300 .. 12288 rows of 512 .. 6144 columns).
@@ -860,11 +864,15 @@ __device__ __forceinline__ void ask_q4k_tile(const uint8_t *blk, uint32_t row_by
 // (each converted weight is used for both), so f32 activations cost one launch.
 //
 // PIECES: the weights come as pieces of 16 bytes by way of LDS, which costs a second round trip and saves most of the time in L1.
-// Measured (us, rows a lane -> pieces; 3045 rows, or as said): up to 32 tokens 1280 columns 6.9 -> 6.5, 2048 8.2 -> 6.7, 6144 15.2
-// -> 11.0, 12288 rows of 2048 11.8 -> 9.1 (two parts 2048 9.5 -> 8.4, 6144 19.0 -> 16.3, 2560 12.4 -> 12.6); where four waves or fewer do everything it is the round trip that counts (512 columns
-// 5.8 -> 6.3).  33 .. 64 tokens: 2048 columns 10.2 -> 9.3, 4096 15.3 -> 13.7, 6144 20.7 -> 18.4, where all eight waves have the
-// same number of superblocks and L1 is busy throughout; else even or slower (1280 8.4 -> 8.7, 1792 9.1 -> 9.2, 2304 11.6 -> 12.1,
-// 3072 12.4 -> 12.9, 5120 17.3 -> 17.3).  Two parts of 64 tokens have no registers left for it.
+// Measured (us, rows a lane -> pieces, 3045 rows; 500 and 8192 rows are alike):
+// up to 32 tokens, one part: 1280 columns 7.0 -> 6.5, 2048 8.3 -> 6.8, 6144 15.3 -> 10.9; where four waves or fewer do everything
+// it is even within what runs differ by (512 5.8 -> 5.7 .. 6.1).  Two parts, whose matrix instructions are as many again and hide more
+// of L1: where all eight waves have the same number of superblocks (2048 9.8 -> 8.9, 4096 14.9 -> 13.2, 6144 20.1 -> 17.5) and on
+// longer rows (3584 13.2 -> 12.9, 5120 17.3 -> 16.8), not between (1280 8.2 -> 8.6, 1792 8.8 -> 8.9, 2304 11.3 -> 12.0, 2560 11.9 ->
+// 12.1, 3072 12.3 -> 12.6).
+// 33 .. 64 tokens, one part: the same number to every wave (40 tokens: 2048 10.2 -> 9.5, 4096 15.3 -> 13.8, 6144 20.6 -> 18.0), else
+// even or slower (512 7.5 -> 8.1, 1280 8.4 -> 8.7, 2304 11.7 -> 12.2, 3584 13.3 -> 13.3, 5120 17.5 -> 17.2).  Two parts of 64 tokens
+// have no registers left for it.
 constexpr int skinny_wave(int mt, bool pieces) { return pieces && mt == 1 ? kRoundTile : mt * 16 * 64; }      // floats of LDS
 struct SkinnyParams {      // (its own: arguments are copied at every launch, and two launches of 3 us are what such a call is)
     const uint8_t *W;

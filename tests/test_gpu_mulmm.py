@@ -412,6 +412,31 @@ def test_mul_mm_small_batch_edges(ctx, xdt, rows, batch, cols):
         assert float(rel_err(got[t], oracle.matvec_f64(oracle.Q4K, w, rows, cols, x.reshape(batch, cols)[t])).max()) <= 2e-5, t
 
 
+@pytest.mark.parametrize("xdt,cols,batch,pieces", [
+    (DType.BF16, 256, 1, False), (DType.BF16, 1024, 32, False), (DType.BF16, 1280, 32, True), (DType.BF16, 1792, 33, False), (DType.BF16, 2048, 33, True), (DType.BF16, 2304, 32, True),
+    (DType.F32, 1280, 32, False), (DType.F32, 2048, 5, True), (DType.F32, 2304, 31, False), (DType.F32, 2560, 3, False),
+    (DType.F32, 3072, 32, False), (DType.F32, 3328, 32, True), (DType.F32, 2048, 33, False)])
+def test_mul_mm_small_batch_way_in(ctx, xdt, cols, batch, pieces):
+    """Which way the weights of the small-batch form come in, by pieces through LDS or a row a lane, on both sides of every line
+    of its rule, and the result there against float64 (2e-5, as for the tiles)."""
+    rows = 45
+    w = synth.q4k_blocks(rows * cols // 256, 737)
+    x = synth.normal_f32(batch * cols, 738)
+    xb = ctx.buffer_f32(x)
+    if xdt == DType.BF16:
+        x, raw = synth.bf16_round(x)
+        xb = ctx.buffer_bytes(raw)
+    k = ctx.compile(hip.make_desc(hip.Kind.MATVEC_BATCH, (rows, cols, batch), (DType.Q4K, xdt, DType.F32), (), dict(nr0=32)))
+    wave = 64 * 16 * 4 if batch <= 32 else 2 * 64 * 16 * 4
+    assert k.info.lds_bytes == 8 * (max(wave, 32 * 144) if pieces else wave)
+    y = ctx.buffer_empty_f32(batch * rows)
+    ctx.encode_multi(k, [ctx.buffer_bytes(w), xb], [y])
+    ctx.synchronize()
+    got = ctx.read_f32(y, batch * rows).reshape(batch, rows)
+    for t in {0, batch // 2, batch - 1}:
+        assert float(rel_err(got[t], oracle.matvec_f64(oracle.Q4K, w, rows, cols, x.reshape(batch, cols)[t])).max()) <= 2e-5, t
+
+
 @pytest.mark.parametrize("rows,batch,cols,ks,at,shape", [
     (1, 1, 256, 1, 0, "32x128"), (33, 31, 768, 3, 2, "32x128"), (129, 33, 2816, 7, 14, "32x128"), (127, 32, 256, 1, 6, "32x128"),
     (4095, 65, 2816, 1, 10, "32x128"), (4097, 63, 6144, 8, 8, "64x128"), (4130, 64, 7936, 5, 4, "64x128"), (4223, 193, 768, 1, 12, "32x128")])
