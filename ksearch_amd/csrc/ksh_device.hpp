@@ -133,14 +133,16 @@ __device__ __forceinline__ void act_st(float *p, size_t i, float v)
 
 // 16 (or 4) bytes a lane straight from memory into LDS: lane l's at dst + 16 l (4 l).  The compiler does not count these (it
 // answers them with a wait for all in front of every read of LDS): whoever asks waits by the number of younger operations.  The place
-// in LDS goes by m0, which the compiler writes.
+// in LDS goes by m0, which the compiler writes.  The address is copied by a scalar instruction, which waits for a register that a
+// v_readfirstlane has just written (the request itself would not, and the compiler does not keep the five wait states in front of
+// a statement); the copy is the wait state behind the write of m0, too.
 __device__ __forceinline__ void to_lds16(const uint8_t *base, uint32_t off, uint32_t dst)
 {
-    asm volatile("s_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" ::"v"(off), "s"(base), "{m0}"(dst) : "memory");
+    asm volatile("s_mov_b64 vcc, %1\n\tglobal_load_lds_dwordx4 %0, vcc" ::"v"(off), "s"(base), "{m0}"(dst) : "vcc", "memory");
 }
 __device__ __forceinline__ void to_lds4(const uint8_t *base, uint32_t off, uint32_t dst)
 {
-    asm volatile("s_nop 0\n\tglobal_load_lds_dword %0, %1" ::"v"(off), "s"(base), "{m0}"(dst) : "memory");
+    asm volatile("s_mov_b64 vcc, %1\n\tglobal_load_lds_dword %0, vcc" ::"v"(off), "s"(base), "{m0}"(dst) : "vcc", "memory");
 }
 
 // Values of LDS asked for ahead of their use: ordinary loads, so that a copy or a spill of one on its way is waited for by the

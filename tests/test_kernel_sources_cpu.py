@@ -29,7 +29,8 @@ def statements():
                 at += 1
             body = text[m.end():at - 1]
             template = re.match(r'\s*((?:"(?:[^"\\]|\\.)*"\s*)+)', body).group(1)
-            out.append((f, template, body[len(template):] if body.startswith(template) else body.split(template, 1)[1]))
+            rest = body.split(template, 1)[1]
+            out.append((f, template.replace("\\n", "\n").replace("\\t", " "), rest))
     return out
 
 
@@ -62,6 +63,20 @@ def test_asm_names_the_registers_it_uses(file, template, rest):
         assert len(parts) > 3 and f'"{reg}"' in parts[3], f"{file}: {reg} in {template}"
     if re.search(r"_load_lds_|_load_\w+ .*\blds\b", template):
         assert '"{m0}"' in rest, f"{file}: {template}"
+
+
+# A scalar register that a vector instruction has written (the compiler may put a uniform address there by v_readfirstlane) must not
+# be read by a vector-memory instruction within five wait states, which the compiler does not count into a statement; scalar
+# instructions wait for such a register by themselves.  So an address in scalar registers goes through one in the statement.
+VECTOR_MEMORY = re.compile(r"\b(?:global|buffer|flat|scratch)_(?:load|store|atomic)[^\n]*")
+
+
+@pytest.mark.parametrize("file,template,rest", statements())
+def test_asm_requests_take_no_scalar_address_as_it_comes(file, template, rest):
+    operands = re.findall(r'"([^"]*)"\s*\(', rest)
+    for request in VECTOR_MEMORY.findall(template):
+        for n in re.findall(r"%(\d+)", request):
+            assert operands[int(n)].strip("=&+") != "s", f"{file}: {request}"
 
 
 def kernels():
