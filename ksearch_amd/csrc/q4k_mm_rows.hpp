@@ -48,6 +48,9 @@ struct MmRows {
     static constexpr int kInv = 256;                  // the tokens' 1 / s
     static constexpr int kLds = 4 * kStage + kSums + WM * WN * NT * kTile + kInv;
     static_assert(WM * WN == 4 && TT * PARTS <= 4 && MT * PARTS >= 2 && NT <= 2, "a wave fetches TF fragments of a half step, from one part of one token tile");
+    // (a half step has MT PARTS units; the second half of them ask for a superblock's sums, one each)
+    static_assert((MT * PARTS == 2 && SUMS == 1) || MT * PARTS == 4, "every request that the loop's waits count has its place");
+    static_assert(!LO || TM * 4 <= kInv, "the tokens' 1 / s have their place");
 };
 
 // What comes from memory into LDS is not counted by the compiler, which would wait for all of it in front of every read of LDS: it
@@ -195,6 +198,7 @@ __global__ __launch_bounds__(S::kThreads, 2) void q4k_mm_rows_kernel(MmParams p)
 
     // CUT: lane t % 32 keeps the superblocks per slice of the tile's row t and what is left of the current one; finished slices
     // add up in T
+    static_assert(!PAIR || (S::LO && NT == 2), "a gate tile beside an up tile, of f32 rows");
     static_assert(!CUT || MT == 1, "one token tile to a wave leaves registers for T");
     f16v T[NT];
     int cut_len = nsb, cut_left = nsb;

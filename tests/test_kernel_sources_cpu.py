@@ -2,7 +2,9 @@
 the compiler made of the kernels that sit at the edge of the register file, read from the built library's metadata."""
 import os
 import re
+import shutil
 import struct
+import subprocess
 
 import pytest
 
@@ -119,3 +121,16 @@ def test_full_kernels_keep_their_values_in_registers():
     spilled = {name: (k[".vgpr_spill_count"], k[".private_segment_fixed_size"]) for name, k in found.items()
                if k[".vgpr_spill_count"] or k[".private_segment_fixed_size"]}
     assert not spilled
+
+
+@pytest.mark.skipif(not shutil.which("hipcc"), reason="needs the compiler")
+@pytest.mark.parametrize("shape,taken", [("2, 2, 1, 4", True), ("1, 2, 1, 4", True), ("1, 1, 1, 4", True), ("4, 1, 1, 4, false", True), ("2, 1, 1, 4, false", True),
+                                         ("1, 1, 2, 2", True), ("2, 1, 2, 2, false", False), ("3, 1, 1, 4, false", False)])
+def test_prompt_gemm_takes_only_shapes_that_its_waits_count(shape, taken):
+    """q4k_mm_rows_kernel waits by the number of its requests, which its units issue at places fixed at compile time: a shape with
+    fewer places than requests would read LDS ahead of what it waits for, so it does not compile.  (Four token tiles, or three, to
+    waves that have two places for a superblock's sums.)"""
+    r = subprocess.run(["hipcc", "-x", "hip", "-std=c++17", f"--offload-arch={_build.ARCH}", "--offload-host-only", "-fsyntax-only", "-w", "-I" + CSRC, "-"],
+                       input=f'#include "mul_mm_q4k.hip"\nstatic_assert(ksh::MmRows<{shape}>::TM > 0, "");\n', capture_output=True, text=True)
+    assert (r.returncode == 0) == taken, r.stderr[-500:]
+    assert taken or "static assertion failed" in r.stderr
