@@ -1849,7 +1849,8 @@ int bind_matvec_batch(ksh_kernel &k)
     }
     // K slices: workgroups of one launch, every slice storing its partial sums, and a second launch that adds them
     // (mm_k_slices, mm_plan_bf16).  sched.k_split names the slice count (a divisor of cols / 256; 1 = none).  For bf16 rows
-    // the plan takes any count, and a schedule that a bound kernel has reported (it names the tile too) takes it again.
+    // the plan takes any count, and a schedule that a bound kernel has reported (it names the tile too) takes it again.  (512
+    // threads and 64 columns are what the tile of two roles reports; saved plans of Q4_K may hold them too, from when it was theirs.)
     const int64_t row_tiles = mm_row_tiles(k.desc), nsb = cols / 256;
     int64_t ks = cut ? 1 : k.desc.sched.k_split;
     const bool reported = !f32x && want == BN && ((k.desc.sched.tg == kThreadsMM && k.desc.sched.lds_tile == KS) || (k.desc.sched.tg == MmRowsBf::kThreads && k.desc.sched.lds_tile == (q6 ? KS : 32))) &&
@@ -1997,31 +1998,43 @@ int bind_matvec_round(ksh_kernel &k)
     return 0;
 }
 
-// schedules of the prefill GEMM beside the library's own, which a search times first: the 128 x 128 tile with K depth 64
-// (LDS-staged, one K range per workgroup) and, for Q4_K weights and up to 64 tokens, 32 weight rows per workgroup with the
-// K range split over its 8 waves.  (bf16 rows: the token tile follows from the slice count, and counts that do not divide a
-// row come from the library's own schedule only.)
+// Schedules of the prefill GEMM beside the library's own, which a search times first, as the bound kernels report them: whole
+// rows, for Q4_K weights and up to 64 tokens 32 weight rows per workgroup with the K range split over its 8 waves, and K slices
+// where half as many leave the chip short of workgroups.  (The shape of a workgroup follows from the sizes, for bf16 rows from the
+// slice count too; counts that do not divide a row come from the library's own schedule only.)
 int mul_mm_candidates(const ksh_kernel_desc &d, ksh_sched *out, int cap)
 {
     int n = 0;
-    if (n < cap) {
+    const bool q6 = d.dtypes[0] == KSH_Q6K, f32x = d.dtypes[1] == KSH_F32;
+    const int row_tiles = mm_row_tiles(d), nsb = (int)(d.dims[1] / 256);
+    if (nsb <= 0 || row_tiles <= 0 || d.dims[2] <= 0) return 0;
+    int tm = BM;                       // tokens a workgroup
+    auto tile = [&](uint32_t ks) {
+        if (!f32x) tm = mm_plan_bf16(q6, row_tiles, nsb, d.dims[2], d.dims[0] + d.dims[3] + d.dims[4], (int)ks).tm;
+        const bool two_roles = q6 && tm == BM;
         ksh_sched s{};
-        s.tg = kThreadsMM; s.nsg = kThreadsMM / 64; s.nr0 = BN; s.lds_tile = KS; s.unroll = 1; s.vec = 0; s.k_split = 1;
-        out[n++] = s;
+        s.tg = two_roles ? kThreadsMM : MmRowsBf::kThreads; s.nsg = s.tg / 64; s.nr0 = BN; s.lds_tile = q6 ? KS : 32; s.unroll = 1; s.vec = 0; s.k_split = ks;
+        return s;
+    };
+    if (n < cap) out[n++] = tile(1);
+    // workgroups of whole rows, and the number that fills the chip: one to a compute unit of the tile of two roles, two of the others
+    // (two tall ones share what the chip's power allows one, see mm_rows_tall)
+    int64_t wgs = (d.dims[2] + tm - 1) / tm * row_tiles;
+    int64_t full = q6 && tm == BM ? 256 : 512;
+    if (f32x && !q6) {
+        const bool tall = mm_rows_tall(d, false, 1);
+        const dim3 g = tall ? mm_rows_grid(d, MmRowsTall::TM, MmRowsTall::TN, false, 1) : mm_rows_grid(d, MmRowsSmall::TM, MmRowsSmall::TN, false, 1);
+        wgs = (int64_t)g.x * g.y;
+        if (tall) full = 256;
     }
-    if (n < cap && d.dtypes[0] == KSH_Q4K && d.dims[2] <= kSkinnyMaxBatch && !d.dims[3]) {
+    if (n < cap && !q6 && d.dims[2] <= kSkinnyMaxBatch && !d.dims[3]) {
         ksh_sched s{};
         s.tg = 512; s.nsg = 8; s.nr0 = 32; s.lds_tile = 16; s.unroll = 1; s.vec = 0; s.k_split = 8;
         out[n++] = s;
     }
-    // the 128 x 128 tile over K slices, where whole rows leave the grid short of one workgroup per compute unit
-    const int64_t tiles = ((d.dims[2] + BM - 1) / BM) * ((d.dims[0] + BN - 1) / BN + (d.dims[3] + BN - 1) / BN + (d.dims[4] + BN - 1) / BN) * (d.dtypes[1] == KSH_F32 ? 2 : 1),
-                  nsb = d.dims[1] / 256;
     for (uint32_t ks : {2u, 4u, 8u, 16u}) {
-        if (n >= cap || nsb % ks || tiles * (ks / 2) >= 256) continue;
-        ksh_sched s{};
-        s.tg = kThreadsMM; s.nsg = kThreadsMM / 64; s.nr0 = BN; s.lds_tile = KS; s.unroll = 1; s.vec = 0; s.k_split = ks;
-        out[n++] = s;
+        if (n >= cap || nsb % ks || wgs * (ks / 2) >= full) continue;
+        out[n++] = tile(ks);
     }
     return n;
 }

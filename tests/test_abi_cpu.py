@@ -163,6 +163,16 @@ def test_plan_kinds_and_candidates():
     assert mm(40, 2048, 1536, hip.DType.F32) == [(128, 1), (32, 8), (128, 2)]
 
 
+@pytest.mark.parametrize("wdt,xdt,batch,tile", [(hip.DType.Q4K, hip.DType.F32, 256, (256, 32)), (hip.DType.Q4K, hip.DType.BF16, 40, (256, 32)),
+                                                (hip.DType.Q6K, hip.DType.F32, 40, (512, 64)), (hip.DType.Q6K, hip.DType.BF16, 40, (256, 64)),
+                                                (hip.DType.Q6K, hip.DType.BF16, 2000, (512, 64))])
+def test_prompt_gemm_candidates_name_kernels_that_are_built(wdt, xdt, batch, tile):
+    """Threads and columns a step of the tile that a candidate's handle reports (a plan saved under other names would claim a
+    kernel that does not run)."""
+    c = [s for s in hip.beam_candidates(hip.make_desc(hip.Kind.MATVEC_BATCH, (2048, 2048, batch), (wdt, xdt, hip.DType.F32))) if s.nr0 == 128]
+    assert c and {(s.tg, s.lds_tile) for s in c} == {tile} and all(s.tg == 64 * s.nsg for s in c)
+
+
 def test_kernel_lookup_takes_any_sequence():
     """Eng._k with lists, arrays and tuples of the same numbers finds one handle."""
     import numpy as np

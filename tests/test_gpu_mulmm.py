@@ -570,3 +570,14 @@ def test_mul_mm_errors(ctx):
         ctx.compile(hip.make_desc(hip.Kind.MATVEC_BATCH, (64, 256, 16), (DType.Q40, DType.BF16, DType.F32)))
     with pytest.raises(hip.KshError, match="multiple of 256"):
         ctx.compile(hip.make_desc(hip.Kind.MATVEC_BATCH, (64, 100, 16), (DType.Q4K, DType.BF16, DType.F32)))
+
+
+@pytest.mark.parametrize("wdt", [DType.Q4K, DType.Q6K])
+@pytest.mark.parametrize("xdt", [DType.F32, DType.BF16])
+@pytest.mark.parametrize("rows,cols,batch", [(2048, 2048, 256), (300, 7936, 40), (1536, 6144, 333), (8192, 2048, 512), (256, 512, 2)])
+def test_mul_mm_candidates_are_what_their_handles_report(ctx, wdt, xdt, rows, cols, batch):
+    """A schedule from the search's list binds, and the bound kernel reports the same tile and slices."""
+    dims, dtypes = (rows, cols, batch), (wdt, xdt, DType.F32)
+    for s in hip.beam_candidates(hip.make_desc(hip.Kind.MATVEC_BATCH, dims, dtypes)):
+        got = ctx.compile(hip.make_desc(hip.Kind.MATVEC_BATCH, dims, dtypes, (), s.as_dict())).info.sched
+        assert all(getattr(got, f) == getattr(s, f) for f in ("tg", "nsg", "nr0", "lds_tile", "k_split")), (s.as_dict(), got.as_dict())
