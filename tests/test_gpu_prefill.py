@@ -133,6 +133,17 @@ def test_sdpa_batch_equals_the_serial_oracle(ctx, hd, n_q, n_kv, sched, t, pos0,
     del row
 
 
+def assert_prompt_form(k, hd, n_kv, t, one_prompt):
+    """The handle is that of the prompt kernel, of one token to a workgroup or of two (which have more LDS and whole pairs of 32
+    tokens): its own tiles, operands and states, not those of the kernel that takes caches at any address."""
+    two = one_prompt and t * n_kv >= (512 if hd == 512 else 896)
+    vh, nb, n = hd // 256, hd // 32, 2 if two else 1
+    front = 4 * vh * (2 * 5120 + 32 // vh * nb * 4 + 32 * 8 * 4) + n * nb * 64 * 20 + n * (vh - 1) * 8192
+    assert tuple(k.info.grid) == (1, n_kv, -(-t // 64) * 64 if two else t), k.name
+    assert k.info.lds_bytes == max(front, n * (vh * 4 * 8 * 256 * 4 + 256)), k.name
+    return two
+
+
 @pytest.mark.parametrize("hd,n_q,n_kv,t,pos0,window,slots", [
     (256, 8, 1, 17, 0, 4096, 0), (256, 5, 1, 70, 29, 33, 0), (256, 16, 2, 129, 100, 64, 0), (512, 8, 1, 45, 31, 4096, 0), (512, 6, 2, 33, 0, 1, 0),
     (256, 8, 1, 900, 0, 250, 0), (256, 6, 2, 451, 3, 4096, 0), (256, 7, 1, 961, 60, 31, 0), (512, 8, 1, 545, 5, 4096, 0), (512, 4, 2, 300, 90, 65, 0),
@@ -146,6 +157,7 @@ def test_prompt_attention_has_the_bits_of_the_form_of_several_partitions(ctx, hd
     kv = [synth.q40_blocks(max(1, slots) * rows, 713 + i) for i in range(2)]
     q = ctx.buffer_f32(synth.normal_f32(t * n_q * hd, 715))
     k = ctx.compile(hip.make_desc(Kind.SDPA_BATCH, (n_q, n_kv, hd, max_t, t, 1, slots), (DType.Q40, DType.F32), (scale,)))
+    assert_prompt_form(k, hd, n_kv, t, not slots)
     tmp = ctx.buffer_empty_f32(t * n_q * (hd + 2))
     if slots:
         n = np.arange(t) % (t // slots + 1) + 1                      # attended rows: prompts one after the other
@@ -157,12 +169,36 @@ def test_prompt_attention_has_the_bits_of_the_form_of_several_partitions(ctx, hd
     got = []
     for at in (0, 2):
         bufs = [ctx.buffer_bytes(np.concatenate([np.zeros(at, np.uint8), np.frombuffer(bytes(x), np.uint8)])) for x in kv]
+        assert all(b.device_ptr % 16 == 0 for b in bufs)          # (what decides is the address, at every launch)
         out = ctx.buffer_empty_f32(t * n_q * hd)
         ctx.encode_offsets_multi(k, [q] + bufs + more, [0, at, at] + [0] * len(more), [tmp, out], None)
         ctx.synchronize()
         got.append(ctx.read_f32(out, t * n_q * hd).reshape(t, -1))
     assert np.isfinite(got[1]).all() and np.abs(got[1]).max() > 0
     assert np.array_equal(got[0], got[1]), np.flatnonzero((got[0] != got[1]).any(axis=1))[:8]
+
+
+@pytest.mark.parametrize("hd,n_q,n_kv,t,pos0,window", [(512, 8, 1, 545, 5, 4096), (512, 4, 2, 300, 90, 65), (256, 8, 1, 900, 0, 250), (256, 7, 1, 961, 60, 31)])
+def test_two_tokens_to_a_workgroup_equal_the_serial_oracle(ctx, hd, n_q, n_kv, t, pos0, window):
+    """Pairs from the cache's start on, pairs whose windows begin 32 rows apart, and those in between, which part: the first and
+    last tokens, and those on both sides of where the window begins to move."""
+    max_t = 1100
+    scale = 1.0 / np.sqrt(hd)
+    kk, vv = synth.q40_blocks(max_t * n_kv * hd // 32, 717), synth.q40_blocks(max_t * n_kv * hd // 32, 718)
+    q = synth.normal_f32(t * n_q * hd, 719).reshape(t, -1)
+    k = ctx.compile(hip.make_desc(Kind.SDPA_BATCH, (n_q, n_kv, hd, max_t, t, 1), (DType.Q40, DType.F32), (scale,)))
+    assert assert_prompt_form(k, hd, n_kv, t, True)
+    bufs = [ctx.buffer_bytes(kk), ctx.buffer_bytes(vv)]
+    assert all(b.device_ptr % 16 == 0 for b in bufs)
+    tmp, out = ctx.buffer_empty_f32(t * n_q * (hd + 2)), ctx.buffer_empty_f32(t * n_q * hd)
+    ctx.encode_multi(k, [ctx.buffer_f32(q)] + bufs + [ctx.buffer_f32(np.array([pos0 + 1, 0, window, 0], np.float32))], [tmp, out])
+    ctx.synchronize()
+    got = ctx.read_f32(out, t * n_q * hd).reshape(t, -1)
+    moves = window - pos0                                            # the first token that does not attend the cache's first row
+    for i in sorted({0, 31, 32, 63, t // 2, t // 2 + 32, moves - 33, moves - 32, moves - 1, moves, moves + 31, moves + 32, t - 33, t - 1} & set(range(t))):
+        tlen = min(pos0 + 1 + i, window)
+        want = oracle.sdpa(q[i], kk, vv, n_q, n_kv, hd, tlen, pos0 + 1 + i - tlen, scale)
+        assert_close(got[i], want, 1e-3, f"{k.name} token {i}")
 
 
 @pytest.mark.parametrize("wdt,batch,sched", [(DType.Q4K, 45, None), (DType.Q6K, 45, None), (DType.Q4K, 5, None), (DType.Q4K, 32, None),
