@@ -380,7 +380,16 @@ struct MmParams {
     // q4k_mm_rows_kernel's numbering of the workgroups: how many there are, in x and in y, ceil(2^32 / gx) and ceil(2^32 / gy)
     // (exact quotients where wgs * gx and wgs * gy stay below 2^32; wgs = 0: as the launch numbers them)
     uint32_t wgs, gx, gy, per_gx, per_gy;
+    // bf16 rows: results go through the L2s as usual (mm_keeps)
+    int keep;
 };
+
+template <bool KEEP>
+__device__ __forceinline__ void mm_store(float *y, float v)
+{
+    if (KEEP) *y = v;
+    else __builtin_nontemporal_store(v, y);
+}
 
 // F32 activations: the tokens and weight rows (BN) of the tiles that the rule of the K slices counts.  How a row's sum is cut
 // decides its bits, so the rule stays when the tiles that do the work change (q4k_mm_rows_kernel's are others).
@@ -437,6 +446,20 @@ MmPlan mm_plan_bf16(bool q6, int row_tiles, int nsb, int64_t batch, int64_t rows
             if (us < best.us) best = MmPlan{c->tm, ks, us};
         }
     return best;
+}
+
+// Partial sums of bf16 rows that stay in the L2s for the fold.  Results go past them, since what the L2s hold of them at the kernel's end
+// is written out before the next kernel starts (figures at the kernels' ends).  Partial sums are read again at once, and the more
+// slices there are the longer the fold waits for each: 10 tokens of 297 x 7424 in 29 slices (0.3 MB) 10.9 us past the L2s or 9.9
+// kept, 39 of 580 x 5120 in 20 (1.8 MB) 11.8 or 11.1, 11 of 3832 x 3328 in 13 (2.2 MB) even, 153 of 495 x 7680 in 15 (4.5 MB) 16.4 or
+// 17.0, 36 of 3288 x 2304 in 9 (4.3 MB) 11.5 or 12.0; Q6_K alike.  A fold of few slices of large results is bound by what it moves
+// (two slices of Q6_K, 733 tokens of 2549 x 3072 34.6 or 31.9 us, 315 of 4905 x 2560 29.2 or 28.0; 4.9 MB a slice 27.1 or
+// 26.2, 3.7 even).  344 shapes with slices: the rule is on average 0.04 % over the better of the
+// two and 1.6 % at most, all past 3.0 % on average, all kept 1.2 %.
+bool mm_keeps(int ks, int64_t batch, int64_t rows_all)
+{
+    const int64_t slice = batch * rows_all * 4;
+    return ks * slice <= 1000000 + (int64_t)ks * 160000 || slice >= 3600000;
 }
 
 // (the small-batch form's way of loading, see the figures at q4k_mm_skinny_kernel)
@@ -816,18 +839,19 @@ __global__ __launch_bounds__(kThreadsMM, 1) void q6k_mul_mm_kernel(MmParams p)
 
     if (CUT) return;   // (the last slices' ends have stored everything)
     // accumulator layout of the 32x32 tile: column = lane % 32, row = 8*(i/4) + 4*(lane/32) + i%4
+    auto store = [&](auto keep) __attribute__((always_inline)) {
 #pragma unroll
-    for (int nt = 0; nt < NW_; nt++) {
-        const int r = r0 + nt * 32 + lm;
+        for (int nt = 0; nt < NW_; nt++) {
+            const int r = r0 + nt * 32 + lm;
 #pragma unroll
-        for (int i = 0; i < 16; i++) {
-            const int t = t0 + wm * 32 + 8 * (i / 4) + 4 * (lane >> 5) + (i & 3);
-            if (t < p.batch && r < p.rows) {
-                if (LO) p.Y[(size_t)t * ystride + r] = F[nt][i] * p.inv_s[t];
-                else __builtin_nontemporal_store(F[nt][i], &p.Y[(size_t)t * ystride + r]);
+            for (int i = 0; i < 16; i++) {
+                const int t = t0 + wm * 32 + 8 * (i / 4) + 4 * (lane >> 5) + (i & 3);
+                if (t < p.batch && r < p.rows) mm_store<decltype(keep)::value>(&p.Y[(size_t)t * ystride + r], LO ? F[nt][i] * p.inv_s[t] : F[nt][i]);
             }
         }
-    }
+    };
+    if (LO || p.keep) store(std::true_type{});
+    else store(std::false_type{});
 }
 
 }  // namespace
@@ -1689,7 +1713,7 @@ int launch_mul_mm(const ksh_kernel &k, const LaunchArgs &a, hipStream_t st)
     const dim3 grid(k.info.grid[0], k.info.grid[1], k.info.grid[2]);
     p.Xf = rows_direct ? (const _Float16 *)a.in[1] : Xf;
     p.SxA = SxA; p.Xf_lo = Xf_lo; p.inv_s = inv_s;
-    p.ksplit = 0; p.Y_parts = nullptr;
+    p.ksplit = 0; p.Y_parts = nullptr; p.keep = 0;
     p.cut_as = cut ? (const float *)a.in[k.info.n_inputs - 1] : nullptr;
     const bool q6 = k.desc.dtypes[0] == KSH_Q6K;
     const uint64_t wgs = (uint64_t)grid.x * grid.y * grid.z;
@@ -1726,6 +1750,7 @@ int launch_mul_mm(const ksh_kernel &k, const LaunchArgs &a, hipStream_t st)
         // few tiles: K slices as blockIdx.z of one launch, then the fold
         const int ks = slices;
         p.ksplit = ks;
+        p.keep = mm_keeps(ks, batch, rows + rows1 + rows2);
         const bool unfolded = k.desc.dims[6] == 1;                    // the partial sums are the result: the reader adds them
         p.Y_parts = unfolded ? (float *)a.out[0] : (float *)((f32x ? SxA_lo : SxA) + sx_halves);     // (else behind the prepared activations)
         launch_tile();

@@ -418,32 +418,33 @@ __global__ __launch_bounds__(S::kThreads, 2) void q4k_mm_rows_kernel(MmParams p)
     // (bf16 rows: stored past the L2s, since what those hold of it at the kernel's end is written out before the next kernel
     // starts; 512 tokens, 8192 x 2048 30.8 -> 29.5 us, 300 tokens, 12288 x 1536 24.1 -> 22.9.  In a prompt's chain of launches it is even,
     // 700 tokens 10.09 ms.)
+    auto store = [&](auto keep) __attribute__((always_inline)) {
 #pragma unroll
-    for (int mt = 0; mt < MT; mt++) {
-        const int tb = t0 + (wm * MT + mt) * 32 + 4 * h, left = p.batch - tb;
-        f32x4_t inv[4];
-        if (S::LO) {
+        for (int mt = 0; mt < MT; mt++) {
+            const int tb = t0 + (wm * MT + mt) * 32 + 4 * h, left = p.batch - tb;
+            f32x4_t inv[4];
+            if (S::LO) {
 #pragma unroll
-            for (int i4 = 0; i4 < 4; i4++) lds_ask<0>(inv[i4], l0 + kAtInv + 4u * (uint32_t)(tb - t0 + 8 * i4));
-            lds_left<0>();
-        }
+                for (int i4 = 0; i4 < 4; i4++) lds_ask<0>(inv[i4], l0 + kAtInv + 4u * (uint32_t)(tb - t0 + 8 * i4));
+                lds_left<0>();
+            }
 #pragma unroll
-        for (int nt = 0; nt < NT; nt += PAIR ? 2 : 1) {
-            const int r = r0 + (PAIR ? wn : wn * NT + nt) * 32 + lm;
-            if (r >= p.rows) continue;
-            float *y = p.Y + (size_t)tb * ystride + r;
+            for (int nt = 0; nt < NT; nt += PAIR ? 2 : 1) {
+                const int r = r0 + (PAIR ? wn : wn * NT + nt) * 32 + lm;
+                if (r >= p.rows) continue;
+                float *y = p.Y + (size_t)tb * ystride + r;
 #pragma unroll
-            for (int i = 0; i < 16; i++) {
-                const int t = 8 * (i / 4) + (i & 3);
-                float v = S::LO ? F[mt][nt][i] * inv[i / 4][i & 3] : F[mt][nt][i];
-                if constexpr (PAIR) v = gelu_mul_f32(pinned(v), pinned(F[mt][1][i] * inv[i / 4][i & 3]));
-                if (t < left) {
-                    if (S::LO) y[(size_t)t * ystride] = v;
-                    else __builtin_nontemporal_store(v, &y[(size_t)t * ystride]);
+                for (int i = 0; i < 16; i++) {
+                    const int t = 8 * (i / 4) + (i & 3);
+                    float v = S::LO ? F[mt][nt][i] * inv[i / 4][i & 3] : F[mt][nt][i];
+                    if constexpr (PAIR) v = gelu_mul_f32(pinned(v), pinned(F[mt][1][i] * inv[i / 4][i & 3]));
+                    if (t < left) mm_store<decltype(keep)::value>(&y[(size_t)t * ystride], v);
                 }
             }
         }
-    }
+    };
+    if (S::LO || p.keep) store(std::true_type{});
+    else store(std::false_type{});
 }
 
 }  // namespace

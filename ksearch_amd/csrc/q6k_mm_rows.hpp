@@ -152,16 +152,20 @@ __global__ __launch_bounds__(256, 2) void q6k_mm_rows_kernel(MmParams p)
     }
     const int r = r0 + lm;
     if (r >= p.rows) return;
+    auto store = [&](auto keep) __attribute__((always_inline)) {
 #pragma unroll
-    for (int mt = 0; mt < MT; mt++) {
-        const int tb = t0 + mt * 32 + 4 * h, left = p.batch - tb;
-        float *y = p.Y + (size_t)tb * ystride + r;
+        for (int mt = 0; mt < MT; mt++) {
+            const int tb = t0 + mt * 32 + 4 * h, left = p.batch - tb;
+            float *y = p.Y + (size_t)tb * ystride + r;
 #pragma unroll
-        for (int i = 0; i < 16; i++) {
-            const int t = 8 * (i / 4) + (i & 3);
-            if (t < left) __builtin_nontemporal_store((float)F[mt][i], &y[(size_t)t * ystride]);
+            for (int i = 0; i < 16; i++) {
+                const int t = 8 * (i / 4) + (i & 3);
+                if (t < left) mm_store<decltype(keep)::value>(&y[(size_t)t * ystride], (float)F[mt][i]);
+            }
         }
-    }
+    };
+    if (p.keep) store(std::true_type{});
+    else store(std::false_type{});
 }
 
 }  // namespace

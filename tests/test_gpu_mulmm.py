@@ -581,3 +581,24 @@ def test_mul_mm_candidates_are_what_their_handles_report(ctx, wdt, xdt, rows, co
     for s in hip.beam_candidates(hip.make_desc(hip.Kind.MATVEC_BATCH, dims, dtypes)):
         got = ctx.compile(hip.make_desc(hip.Kind.MATVEC_BATCH, dims, dtypes, (), s.as_dict())).info.sched
         assert all(getattr(got, f) == getattr(s, f) for f in ("tg", "nsg", "nr0", "lds_tile", "k_split")), (s.as_dict(), got.as_dict())
+
+
+@pytest.mark.parametrize("wdt,rows,batch,cols,ks,shape", [
+    (DType.Q4K, 297, 10, 7424, 29, "64x128"), (DType.Q4K, 2049, 100, 2048, 8, "64x128"), (DType.Q4K, 8193, 1025, 4096, 4, "128x128"),
+    (DType.Q6K, 502, 31, 3584, 14, "32x128"), (DType.Q6K, 3371, 65, 2304, 9, "128x128"), (DType.Q6K, 2549, 733, 3072, 2, "128x128"),
+    (DType.Q6K, 3000, 63, 2304, 8, "64x128")])
+def test_mul_mm_bf16_partial_sums_kept_and_past(ctx, wdt, rows, batch, cols, ks, shape):
+    """Partial sums of bf16 rows that stay in the L2s for the fold (small ones, and large results in few slices) and that go past them,
+    of every shape of workgroup.  Against float64: 2e-5, as for the tiles."""
+    w = (synth.q6k_blocks if wdt == DType.Q6K else synth.q4k_blocks)(rows * cols // 256, 745)
+    xf, xb = synth.bf16_round(synth.normal_f32(batch * cols, 746))
+    k = ctx.compile(hip.make_desc(hip.Kind.MATVEC_BATCH, (rows, cols, batch), (wdt, DType.BF16, DType.F32), (),
+                                  dict(nr0=128, tg=256, lds_tile=64 if wdt == DType.Q6K else 32, k_split=ks)))
+    assert f"_{shape}x" in k.name and k.info.sched.k_split == ks, k.name
+    y = ctx.buffer_empty_f32(batch * rows)
+    ctx.encode_multi(k, [ctx.buffer_bytes(w), ctx.buffer_bytes(xb)], [y])
+    ctx.synchronize()
+    got = ctx.read_f32(y, batch * rows).reshape(batch, rows)
+    fmt = oracle.Q6K if wdt == DType.Q6K else oracle.Q4K
+    for t in sorted({0, 1, batch // 2, batch - 1}):
+        assert float(rel_err(got[t], oracle.matvec_f64(fmt, w, rows, cols, xf.reshape(batch, cols)[t])).max()) <= 2e-5, t
