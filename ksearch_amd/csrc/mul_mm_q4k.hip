@@ -412,42 +412,6 @@ __host__ __device__ constexpr int mm_k_slices(bool q6, int row_tiles, int nsb, i
     return ks;
 }
 
-// Bf16 activations: token tile and K slices (of any number of superblocks) by what the launches are made of, in us, fitted to
-// 256 .. 12288 rows of 512 .. 8192 columns, 2 .. 2048 tokens, every slice count:
-//   preparation (Q4_K), launches, what rows and results cost; per round of workgroups over the compute units; per superblock of
-//   the slice in one round, in two, in more (each), more as the chip fills; the fold
-// The choice is on average within 1 % of the best (tile, slices) at those shapes, within 10 % at all.  Q4_K: 2048 tokens of 12288 x
-// 4096 262 us with 64 tokens a workgroup, 227 with 128; 300 tokens of 12288 x 1536 24.4 or 30.8; 65 tokens of 12288 x 8192 47 us in
-// two slices of 64 tokens, 40 in eight of 128.  Q6_K (32 or 64 tokens: q6k_mm_rows_kernel; 128: q6k_mul_mm_kernel): 8 tokens of 1536 x 6144
-// 10.7 / 11.9 / 13.2 us, 50 of 4096 x 6144 19.6 / 18.0 / 20.9, 333 of 1536 x 6144 38 / 29 / 26.
-struct MmPlan {
-    int tm, ks;
-    float us;
-};
-MmPlan mm_plan_bf16(bool q6, int row_tiles, int nsb, int64_t batch, int64_t rows_all, int ks_given)
-{
-    struct Cost {
-        int tm;
-        float launch, round, one, two, more, fill, out, fold, part;
-    };
-    constexpr Cost kQ4[] = {{64, 5.2f, 0.6f, 1.45f, 1.7f, 0.73f, 0.18f, 1.4f, 4.2f, 1.4f}, {128, 6.4f, 0.6f, 1.87f, 2.62f, 1.31f, 0.08f, 2.f, 4.6f, 1.4f}};
-    constexpr Cost kQ6[] = {{32, 2.65f, 0.75f, 2.2f, 3.3f, 1.36f, 0.084f, 1.44f, 2.35f, 0.9f}, {64, 2.8f, 1.1f, 2.5f, 3.65f, 1.6f, 0.124f, 1.23f, 2.4f, 1.16f},
-                            {128, 2.3f, 2.57f, 2.7f, 5.4f, 2.7f, 0.058f, 2.25f, 2.8f, 1.3f}};
-    MmPlan best{128, 1, 1e30f};
-    const int ks_max = std::min(nsb, 64);
-    const float m = (float)(batch * rows_all) * 1e-6f;
-    for (const Cost *c = q6 ? kQ6 : kQ4, *end = c + (q6 ? 3 : 2); c < end; c++)
-        for (int ks = ks_given ? ks_given : 1; ks <= (ks_given ? ks_given : ks_max); ks++) {
-            const int64_t wgs = (batch + c->tm - 1) / c->tm * row_tiles * ks;
-            const float sb = (float)((nsb + ks - 1) / ks), w = std::min((float)wgs / 256.f, 2.f), rounds = (float)((wgs + 255) / 256);
-            const float each = rounds <= 1.f ? c->one : rounds <= 2.f ? c->two : c->more * rounds;
-            const float us = c->launch + c->round * rounds + each * (1.f + c->fill * w) * sb + c->out * m + (q6 ? 0.f : (float)(batch * nsb) * 256e-6f) +
-                             (ks > 1 ? c->fold + c->part * (float)ks * m : 0.f);
-            if (us < best.us) best = MmPlan{c->tm, ks, us};
-        }
-    return best;
-}
-
 // Partial sums of bf16 rows that stay in the L2s for the fold.  Results go past them, since what the L2s hold of them at the kernel's end
 // is written out before the next kernel starts (figures at the kernels' ends).  Partial sums are read again at once, and the more
 // slices there are the longer the fold waits for each: 10 tokens of 297 x 7424 in 29 slices (0.3 MB) 10.9 us past the L2s or 9.9
@@ -462,6 +426,41 @@ bool mm_keeps(int ks, int64_t batch, int64_t rows_all)
     return ks * slice <= 1000000 + (int64_t)ks * 160000 || slice >= 3600000;
 }
 
+// Bf16 activations: token tile and K slices (of any number of superblocks) by what the launches are made of, in us:
+//   preparation (Q4_K), launches, what rows and results cost; per round of workgroups over the compute units; per superblock of
+//   the slice in one round, in two, in more (each), more as the chip fills; the fold, less where it finds the partial sums in L2
+// Against the best (tile, slices, or the small-batch form) of 391 shapes of 200 .. 16384 rows of 512 .. 8192 columns, 2 .. 2048 tokens,
+// up to 17 slice counts each, to which Q4_K's figures are fitted: 0.4 % over it on average, 2 % at 19 in 20, 20 % at most (1963
+// tokens of 5221 x 1536 63.0 us, with 128 tokens a workgroup 52.4; next 7 %).  Q6_K (fitted before its kernels' stores and conversion
+// changed): 0.7 %, 5 %, 15 % (390 tokens of 4183 x 3840 48.0 us in three slices, 41.9 in one).
+struct MmPlan {
+    int tm, ks;
+    float us;
+};
+MmPlan mm_plan_bf16(bool q6, int row_tiles, int nsb, int64_t batch, int64_t rows_all, int ks_given)
+{
+    struct Cost {
+        int tm;
+        float launch, round, one, two, more, fill, out, fold, part, kept;
+    };
+    constexpr Cost kQ4[] = {{64, 5.9f, 0.f, 1.466f, 1.611f, 0.981f, 0.2f, 1.207f, 1.755f, 2.138f, 0.196f}, {128, 7.5f, 0.f, 1.749f, 2.746f, 1.738f, 0.074f, 1.573f, 2.873f, 1.764f, 0.488f}};
+    constexpr Cost kQ6[] = {{32, 2.65f, 0.75f, 2.2f, 3.3f, 1.36f, 0.084f, 1.44f, 2.35f, 0.9f, 0.f}, {64, 2.8f, 1.1f, 2.5f, 3.65f, 1.6f, 0.124f, 1.23f, 2.4f, 1.16f, 0.f},
+                            {128, 2.3f, 2.57f, 2.7f, 5.4f, 2.7f, 0.058f, 2.25f, 2.8f, 1.3f, 0.f}};
+    MmPlan best{128, 1, 1e30f};
+    const int ks_max = std::min(nsb, 64);
+    const float m = (float)(batch * rows_all) * 1e-6f;
+    for (const Cost *c = q6 ? kQ6 : kQ4, *end = c + (q6 ? 3 : 2); c < end; c++)
+        for (int ks = ks_given ? ks_given : 1; ks <= (ks_given ? ks_given : ks_max); ks++) {
+            const int64_t wgs = (batch + c->tm - 1) / c->tm * row_tiles * ks;
+            const float sb = (float)((nsb + ks - 1) / ks), w = std::min((float)wgs / 256.f, 2.f), rounds = (float)((wgs + 255) / 256);
+            const float each = rounds <= 1.f ? c->one : rounds <= 2.f ? c->two : c->more * rounds;
+            const float us = c->launch + c->round * rounds + each * (1.f + c->fill * w) * sb + c->out * m + (q6 ? 0.f : (float)(batch * nsb) * 256e-6f) +
+                             (ks > 1 ? c->fold + c->part * (float)ks * m - (mm_keeps(ks, batch, rows_all) ? c->kept : 0.f) : 0.f);
+            if (us < best.us) best = MmPlan{c->tm, ks, us};
+        }
+    return best;
+}
+
 // (the small-batch form's way of loading, see the figures at q4k_mm_skinny_kernel)
 constexpr bool skinny_pieces(int mt, bool lo, int nsb)
 {
@@ -470,12 +469,16 @@ constexpr bool skinny_pieces(int mt, bool lo, int nsb)
 }
 
 // The small-batch form beside it (Q4_K, bf16), with its preparation: a workgroup of eight waves per 32 rows, superblocks dealt to
-// the waves (300 .. 12288 rows of 512 .. 6144 columns).
+// the waves, the fullest of which has `turns` (fitted to 233 of those shapes, 5 % off up to 32 tokens, 2 % beyond).  8 tokens of
+// 757 x 6400 10.9 us here, 9.7 in the tile, 36 of 8371 x 5632 33.5 and 20.9; 4 of 3157 x 6144 10.0 and 11.7, 40 of 1724 x 2304 11.7 and 10.4.
 float mm_skinny_us(int64_t rows, int nsb, int64_t batch)
 {
-    const float turns = std::max(1.f, (float)((rows + 31) / 32) / 128.f - 1.f), each = (float)nsb / 8.f;
-    if (batch <= 32) return 5.4f + 2.f * each * turns;
-    return skinny_pieces(2, false, nsb) ? 6.2f + 4.3f * each * turns : 6.4f + 5.f * std::max(each, 0.45f) * turns;
+    const int64_t wgs = (rows + 31) / 32;
+    const float turns = (float)((nsb + 7) / 8), each = (float)nsb / 8.f, x = (float)(batch * nsb) * 1e-3f, more = (float)((wgs + 255) / 256 - 1);
+    if (batch <= 32) return 4.82f + 0.71f * turns + each * (0.91f + 2.26f * more) + 2.57f * x;
+    const float fill = (float)std::min<int64_t>(wgs, 256) / 256.f;
+    if (skinny_pieces(2, false, nsb)) return 4.67f + each * (4.5f + 0.27f * fill + 4.5f * more) + 1.16f * x;
+    return 4.81f + 1.89f * turns + each * (1.93f + 0.42f * fill + 5.45f * more) + 3.06f * x;
 }
 
 // Bf16 rows of Q6_K products as they are (the kernel's ROWS form): the conversion between the matrix instructions costs 0.42
