@@ -412,18 +412,23 @@ __host__ __device__ constexpr int mm_k_slices(bool q6, int row_tiles, int nsb, i
     return ks;
 }
 
-// Partial sums of bf16 rows that stay in the L2s for the fold.  Results go past them, since what the L2s hold of them at the kernel's end
-// is written out before the next kernel starts (figures at the kernels' ends).  Partial sums are read again at once, and the more
-// slices there are the longer the fold waits for each: 10 tokens of 297 x 7424 in 29 slices (0.3 MB) 10.9 us past the L2s or 9.9
-// kept, 39 of 580 x 5120 in 20 (1.8 MB) 11.8 or 11.1, 11 of 3832 x 3328 in 13 (2.2 MB) even, 153 of 495 x 7680 in 15 (4.5 MB) 16.4 or
-// 17.0, 36 of 3288 x 2304 in 9 (4.3 MB) 11.5 or 12.0; Q6_K alike.  A fold of few slices of large results is bound by what it moves
-// (two slices of Q6_K, 733 tokens of 2549 x 3072 34.6 or 31.9 us, 315 of 4905 x 2560 29.2 or 28.0; 4.9 MB a slice 27.1 or
-// 26.2, 3.7 even).  344 shapes with slices: the rule is on average 0.04 % over the better of the
-// two and 1.6 % at most, all past 3.0 % on average, all kept 1.2 %.
-bool mm_keeps(int ks, int64_t batch, int64_t rows_all)
+// Results of bf16 rows go past the L2s, since what those hold of them at the kernel's end is written out before the next kernel starts
+// (figures at the kernels' ends).  Not so:
+// - Small partial sums, which the fold reads at once, and waits the longer for the more slices there are: 10 tokens of 297 x 7424 in 29
+//   slices (0.3 MB) 10.9 us past the L2s or 9.9 kept, 39 of 580 x 5120 in 20 (1.8 MB) 11.8 or 11.1, 11 of 3832 x 3328 in 13 (2.2
+//   MB) even, 153 of 495 x 7680 in 15 (4.5 MB) 16.4 or 17.0, 36 of 3288 x 2304 in 9 (4.3 MB) 11.5 or 12.0; Q6_K alike.  (Whole results
+//   of that size 1 % shorter.)
+// - Few slices of large results, whose fold is bound by what it moves (two slices of Q6_K, 733 tokens of 2549 x 3072 34.6 or 31.9 us, 315
+//   of 4905 x 2560 29.2 or 28.0; 4.9 MB a slice 27.1 or 26.2, 3.7 even).
+// - Results of the tile of two roles (one workgroup a compute unit, nobody works while it stores) whose rows are not whole pieces of 64
+//   bytes: 1785 tokens of 4311 x 1024 46.1 or 36.4 us, 573 of 11713 x 1024 45.7 or 39.6, 463 of 3272 x 768 14.3 or 14.0, 339 of 5959 x 2816
+//   even; in whole pieces 338 of 9616 x 1792 25.9 or 27.4, 512 of 8192 x 2048 30.8 or 32.8.  (The others' within 5 % either way.)
+// 344 shapes with slices: 0.04 % over the better of the two on average and 1.6 % at most, all past 3.0 % on average, all kept 1.2 %.
+bool mm_keeps(int ks, int64_t batch, int64_t rows_all, bool two_roles, int64_t rows, int64_t rows1, int64_t rows2)
 {
     const int64_t slice = batch * rows_all * 4;
-    return ks * slice <= 1000000 + (int64_t)ks * 160000 || slice >= 3600000;
+    if (ks * slice <= 1000000 + (int64_t)ks * 160000) return true;
+    return ks > 1 ? slice >= 3600000 : two_roles && ((rows | rows1 | rows2) & 15);
 }
 
 // Bf16 activations: token tile and K slices (of any number of superblocks) by what the launches are made of, in us:
@@ -455,7 +460,7 @@ MmPlan mm_plan_bf16(bool q6, int row_tiles, int nsb, int64_t batch, int64_t rows
             const float sb = (float)((nsb + ks - 1) / ks), w = std::min((float)wgs / 256.f, 2.f), rounds = (float)((wgs + 255) / 256);
             const float each = rounds <= 1.f ? c->one : rounds <= 2.f ? c->two : c->more * rounds;
             const float us = c->launch + c->round * rounds + each * (1.f + c->fill * w) * sb + c->out * m + (q6 ? 0.f : (float)(batch * nsb) * 256e-6f) +
-                             (ks > 1 ? c->fold + c->part * (float)ks * m - (mm_keeps(ks, batch, rows_all) ? c->kept : 0.f) : 0.f);
+                             (ks > 1 ? c->fold + c->part * (float)ks * m - (mm_keeps(ks, batch, rows_all, false, 0, 0, 0) ? c->kept : 0.f) : 0.f);
             if (us < best.us) best = MmPlan{c->tm, ks, us};
         }
     return best;
@@ -1716,9 +1721,10 @@ int launch_mul_mm(const ksh_kernel &k, const LaunchArgs &a, hipStream_t st)
     const dim3 grid(k.info.grid[0], k.info.grid[1], k.info.grid[2]);
     p.Xf = rows_direct ? (const _Float16 *)a.in[1] : Xf;
     p.SxA = SxA; p.Xf_lo = Xf_lo; p.inv_s = inv_s;
-    p.ksplit = 0; p.Y_parts = nullptr; p.keep = 0;
+    p.ksplit = 0; p.Y_parts = nullptr;
     p.cut_as = cut ? (const float *)a.in[k.info.n_inputs - 1] : nullptr;
     const bool q6 = k.desc.dtypes[0] == KSH_Q6K;
+    p.keep = mm_keeps(std::max(slices, 1), batch, rows + rows1 + rows2, q6 && !(k.variant & kRows6), rows, rows1, rows2);
     const uint64_t wgs = (uint64_t)grid.x * grid.y * grid.z;
     p.wgs = wgs * std::max(grid.x, grid.y) < (1ull << 32) && grid.x > 1 && grid.y > 1 ? (uint32_t)wgs : 0;
     p.gx = grid.x; p.gy = grid.y;
@@ -1753,7 +1759,6 @@ int launch_mul_mm(const ksh_kernel &k, const LaunchArgs &a, hipStream_t st)
         // few tiles: K slices as blockIdx.z of one launch, then the fold
         const int ks = slices;
         p.ksplit = ks;
-        p.keep = mm_keeps(ks, batch, rows + rows1 + rows2);
         const bool unfolded = k.desc.dims[6] == 1;                    // the partial sums are the result: the reader adds them
         p.Y_parts = unfolded ? (float *)a.out[0] : (float *)((f32x ? SxA_lo : SxA) + sx_halves);     // (else behind the prepared activations)
         launch_tile();

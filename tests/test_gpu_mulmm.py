@@ -584,12 +584,13 @@ def test_mul_mm_candidates_are_what_their_handles_report(ctx, wdt, xdt, rows, co
 
 
 @pytest.mark.parametrize("wdt,rows,batch,cols,ks,shape", [
+    (DType.Q6K, 4096, 1023, 512, 1, "128x128"), (DType.Q6K, 4097, 1023, 512, 1, "128x128"),
     (DType.Q4K, 297, 10, 7424, 29, "64x128"), (DType.Q4K, 2049, 100, 2048, 8, "64x128"), (DType.Q4K, 8193, 1025, 4096, 4, "128x128"),
     (DType.Q6K, 502, 31, 3584, 14, "32x128"), (DType.Q6K, 3371, 65, 2304, 9, "128x128"), (DType.Q6K, 2549, 733, 3072, 2, "128x128"),
     (DType.Q6K, 3000, 63, 2304, 8, "64x128")])
 def test_mul_mm_bf16_partial_sums_kept_and_past(ctx, wdt, rows, batch, cols, ks, shape):
     """Partial sums of bf16 rows that stay in the L2s for the fold (small ones, and large results in few slices) and that go past them,
-    of every shape of workgroup.  Against float64: 2e-5, as for the tiles."""
+    of every shape of workgroup, and whole results of the tile of two roles in whole pieces of 64 bytes and not.  Against float64: 2e-5, as for the tiles."""
     w = (synth.q6k_blocks if wdt == DType.Q6K else synth.q4k_blocks)(rows * cols // 256, 745)
     xf, xb = synth.bf16_round(synth.normal_f32(batch * cols, 746))
     k = ctx.compile(hip.make_desc(hip.Kind.MATVEC_BATCH, (rows, cols, batch), (wdt, DType.BF16, DType.F32), (),
