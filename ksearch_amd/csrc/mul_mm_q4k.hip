@@ -435,9 +435,8 @@ bool mm_keeps(int ks, int64_t batch, int64_t rows_all, bool two_roles, int64_t r
 //   preparation (Q4_K), launches, what rows and results cost; per round of workgroups over the compute units; per superblock of
 //   the slice in one round, in two, in more (each), more as the chip fills; the fold, less where it finds the partial sums in L2
 // Against the best (tile, slices, or the small-batch form) of 391 shapes of 200 .. 16384 rows of 512 .. 8192 columns, 2 .. 2048 tokens,
-// up to 17 slice counts each, to which Q4_K's figures are fitted: 0.4 % over it on average, 2 % at 19 in 20, 20 % at most (1963
-// tokens of 5221 x 1536 63.0 us, with 128 tokens a workgroup 52.4; next 7 %).  Q6_K (fitted before its kernels' stores and conversion
-// changed): 0.7 %, 5 %, 15 % (390 tokens of 4183 x 3840 48.0 us in three slices, 41.9 in one).
+// up to 17 slice counts each, to which the figures are fitted: Q4_K 0.4 % over it on average, 2 % at 19 in 20, 20 % at most (1963
+// tokens of 5221 x 1536 63.0 us, with 128 tokens a workgroup 52.4; next 7 %), Q6_K 0.2 %, 1.5 %, 6 % (before 0.9, 5.7, 19).
 struct MmPlan {
     int tm, ks;
     float us;
@@ -449,8 +448,8 @@ MmPlan mm_plan_bf16(bool q6, int row_tiles, int nsb, int64_t batch, int64_t rows
         float launch, round, one, two, more, fill, out, fold, part, kept;
     };
     constexpr Cost kQ4[] = {{64, 5.9f, 0.f, 1.466f, 1.611f, 0.981f, 0.2f, 1.207f, 1.755f, 2.138f, 0.196f}, {128, 7.5f, 0.f, 1.749f, 2.746f, 1.738f, 0.074f, 1.573f, 2.873f, 1.764f, 0.488f}};
-    constexpr Cost kQ6[] = {{32, 2.65f, 0.75f, 2.2f, 3.3f, 1.36f, 0.084f, 1.44f, 2.35f, 0.9f, 0.f}, {64, 2.8f, 1.1f, 2.5f, 3.65f, 1.6f, 0.124f, 1.23f, 2.4f, 1.16f, 0.f},
-                            {128, 2.3f, 2.57f, 2.7f, 5.4f, 2.7f, 0.058f, 2.25f, 2.8f, 1.3f, 0.f}};
+    constexpr Cost kQ6[] = {{32, 3.26f, 0.275f, 1.88f, 2.58f, 1.36f, 0.181f, 0.686f, 1.8f, 1.7f, 0.f}, {64, 4.38f, 0.123f, 2.11f, 2.81f, 1.69f, 0.144f, 0.505f, 1.78f, 1.78f, 0.f},
+                            {128, 2.88f, 0.281f, 2.35f, 4.67f, 2.28f, 0.012f, 1.76f, 3.1f, 1.77f, 0.f}};
     MmPlan best{128, 1, 1e30f};
     const int ks_max = std::min(nsb, 64);
     const float m = (float)(batch * rows_all) * 1e-6f;
@@ -486,12 +485,13 @@ float mm_skinny_us(int64_t rows, int nsb, int64_t batch)
     return 4.81f + 1.89f * turns + each * (1.93f + 0.42f * fill + 5.45f * more) + 3.06f * x;
 }
 
-// Bf16 rows of Q6_K products as they are (the kernel's ROWS form): the conversion between the matrix instructions costs 0.42
-// us per superblock and round, the preparation a launch (2.5 us) and its pass over X (12288 x 4096: 2048 tokens 337 us
-// against 308, 50 tokens 32.4 against 33.2; 2048 x 8192, 2048 tokens 107.9 against 116.6).
+// Bf16 rows of Q6_K products as they are (the kernel's ROWS form): the conversion between the matrix instructions costs 0.25
+// us per superblock and round, the preparation a launch (2.5 us) and its pass over X (316 tokens of 3005 x 2048 28.2 us prepared, 26.0
+// as they are, 1211 of 8949 x 1280 73.9 and 68.6, 677 of 12177 x 8192 247 and 263).  At those shapes and their slice counts 0.1 % over
+// the better of the two on average, 7 % at most.
 bool mm_rows_direct(int64_t workgroups, int sb_per_slice, int64_t batch, int64_t cols)
 {
-    return 0.42f * (float)((workgroups + 255) / 256 * sb_per_slice) < 2.5f + (float)(batch * cols) * 1.1e-6f;
+    return 0.25f * (float)((workgroups + 255) / 256 * sb_per_slice) < 2.5f + (float)(batch * cols) * 1.1e-6f;
 }
 
 __device__ __forceinline__ uint32_t pair_f16(uint32_t masked, uint32_t sc)

@@ -584,7 +584,7 @@ def test_mul_mm_candidates_are_what_their_handles_report(ctx, wdt, xdt, rows, co
 
 
 @pytest.mark.parametrize("wdt,rows,batch,cols,ks,shape", [
-    (DType.Q6K, 4096, 1023, 512, 1, "128x128"), (DType.Q6K, 4097, 1023, 512, 1, "128x128"),
+    (DType.Q6K, 4000, 1023, 4096, 1, "128x128"), (DType.Q6K, 3999, 1023, 4096, 1, "128x128"),
     (DType.Q4K, 297, 10, 7424, 29, "64x128"), (DType.Q4K, 2049, 100, 2048, 8, "64x128"), (DType.Q4K, 8193, 1025, 4096, 4, "128x128"),
     (DType.Q6K, 502, 31, 3584, 14, "32x128"), (DType.Q6K, 3371, 65, 2304, 9, "128x128"), (DType.Q6K, 2549, 733, 3072, 2, "128x128"),
     (DType.Q6K, 3000, 63, 2304, 8, "64x128")])
