@@ -433,10 +433,11 @@ bool mm_keeps(int ks, int64_t batch, int64_t rows_all, bool two_roles, int64_t r
 
 // Bf16 activations: token tile and K slices (of any number of superblocks) by what the launches are made of, in us:
 //   preparation (Q4_K), launches, what rows and results cost; per round of workgroups over the compute units; per superblock of
-//   the slice in one round, in two, in more (each), more as the chip fills; the fold, less where it finds the partial sums in L2
-// Against the best (tile, slices, or the small-batch form) of 391 shapes of 200 .. 16384 rows of 512 .. 8192 columns, 2 .. 2048 tokens,
-// up to 17 slice counts each, to which the figures are fitted: Q4_K 0.4 % over it on average, 2 % at 19 in 20, 20 % at most (1963
-// tokens of 5221 x 1536 63.0 us, with 128 tokens a workgroup 52.4; next 7 %), Q6_K 0.2 %, 1.5 %, 6 % (before 0.9, 5.7, 19).
+//   the slice in one round, in two, in more (each), more as the chip fills; the fold and its round trips, eight slices each
+// Fitted to 525 shapes of 200 .. 16384 rows of 512 .. 8192 columns, 2 .. 2048 tokens, with every slice count that shortens a slice,
+// called one after the other as a program calls them.  Against the best (tile, slices) of 420 others: Q4_K 0.8 % over it on average,
+// 5 % at 19 in 20, 17 % at most, Q6_K 0.2 %, 1 %, 10 % (the figures of the kernels before these 1.4, 9, 22 and 1.1, 8, 21).  224 tokens of
+// 1653 x 4608 20.3 us, with 64 tokens a workgroup 17.9; 512 of 8192 x 2048 27.7, so 28.5.
 struct MmPlan {
     int tm, ks;
     float us;
@@ -445,11 +446,13 @@ MmPlan mm_plan_bf16(bool q6, int row_tiles, int nsb, int64_t batch, int64_t rows
 {
     struct Cost {
         int tm;
-        float launch, round, one, two, more, fill, out, fold, part, kept;
+        float launch, round, one, two, more, fill, out, out_more, fold, trip, part;
     };
-    constexpr Cost kQ4[] = {{64, 5.9f, 0.f, 1.466f, 1.611f, 0.981f, 0.2f, 1.207f, 1.755f, 2.138f, 0.196f}, {128, 7.5f, 0.f, 1.749f, 2.746f, 1.738f, 0.074f, 1.573f, 2.873f, 1.764f, 0.488f}};
-    constexpr Cost kQ6[] = {{32, 3.26f, 0.275f, 1.88f, 2.58f, 1.36f, 0.181f, 0.686f, 1.8f, 1.7f, 0.f}, {64, 4.38f, 0.123f, 2.11f, 2.81f, 1.69f, 0.144f, 0.505f, 1.78f, 1.78f, 0.f},
-                            {128, 2.88f, 0.281f, 2.35f, 4.67f, 2.28f, 0.012f, 1.76f, 3.1f, 1.77f, 0.f}};
+    constexpr Cost kQ4[] = {{64, 5.765f, 0.035f, 1.236f, 1.626f, 0.812f, 0.156f, 1.178f, 1.056f, 1.674f, 0.501f, 1.744f},
+                            {128, 6.168f, 0.041f, 1.767f, 2.606f, 1.338f, 0.124f, 1.19f, 1.26f, 1.919f, 0.584f, 1.408f}};
+    constexpr Cost kQ6[] = {{32, 2.974f, 0.424f, 1.888f, 2.881f, 1.306f, 0.081f, 1.314f, 0.f, 1.712f, 0.479f, 1.474f},
+                            {64, 3.872f, 0.06f, 2.121f, 3.147f, 1.582f, 0.076f, 0.962f, 0.913f, 1.885f, 0.43f, 1.564f},
+                            {128, 2.364f, 1.164f, 2.378f, 4.471f, 2.11f, 0.074f, 1.241f, 1.701f, 1.968f, 0.515f, 1.813f}};
     MmPlan best{128, 1, 1e30f};
     const int ks_max = std::min(nsb, 64);
     const float m = (float)(batch * rows_all) * 1e-6f;
@@ -458,8 +461,8 @@ MmPlan mm_plan_bf16(bool q6, int row_tiles, int nsb, int64_t batch, int64_t rows
             const int64_t wgs = (batch + c->tm - 1) / c->tm * row_tiles * ks;
             const float sb = (float)((nsb + ks - 1) / ks), w = std::min((float)wgs / 256.f, 2.f), rounds = (float)((wgs + 255) / 256);
             const float each = rounds <= 1.f ? c->one : rounds <= 2.f ? c->two : c->more * rounds;
-            const float us = c->launch + c->round * rounds + each * (1.f + c->fill * w) * sb + c->out * m + (q6 ? 0.f : (float)(batch * nsb) * 256e-6f) +
-                             (ks > 1 ? c->fold + c->part * (float)ks * m - (mm_keeps(ks, batch, rows_all, false, 0, 0, 0) ? c->kept : 0.f) : 0.f);
+            const float us = c->launch + c->round * rounds + each * (1.f + c->fill * w) * sb + (rounds <= 2.f ? c->out : c->out_more) * m +
+                             (q6 ? 0.f : (float)(batch * nsb) * 256e-6f) + (ks > 1 ? c->fold + c->trip * (float)((ks + 6) / 8) + c->part * (float)ks * m : 0.f);
             if (us < best.us) best = MmPlan{c->tm, ks, us};
         }
     return best;
@@ -473,16 +476,14 @@ constexpr bool skinny_pieces(int mt, bool lo, int nsb)
 }
 
 // The small-batch form beside it (Q4_K, bf16), with its preparation: a workgroup of eight waves per 32 rows, superblocks dealt to
-// the waves, the fullest of which has `turns` (fitted to 233 of those shapes, 5 % off up to 32 tokens, 2 % beyond).  8 tokens of
-// 757 x 6400 10.9 us here, 9.7 in the tile, 36 of 8371 x 5632 33.5 and 20.9; 4 of 3157 x 6144 10.0 and 11.7, 40 of 1724 x 2304 11.7 and 10.4.
+// the waves, the fullest of which has `turns` (fitted to 230 of those shapes, 2 to 5 % off; where it is chosen 18 % over the best at most: 59
+// tokens of 9510 x 512 10.8 us, 9.2 in the tile).  50 tokens of 10158 x 4352 28.3 us here, 19.2 in the tile; 5 of 1442 x 6144 9.9 and 10.8.
 float mm_skinny_us(int64_t rows, int nsb, int64_t batch)
 {
-    const int64_t wgs = (rows + 31) / 32;
-    const float turns = (float)((nsb + 7) / 8), each = (float)nsb / 8.f, x = (float)(batch * nsb) * 1e-3f, more = (float)((wgs + 255) / 256 - 1);
-    if (batch <= 32) return 4.82f + 0.71f * turns + each * (0.91f + 2.26f * more) + 2.57f * x;
-    const float fill = (float)std::min<int64_t>(wgs, 256) / 256.f;
-    if (skinny_pieces(2, false, nsb)) return 4.67f + each * (4.5f + 0.27f * fill + 4.5f * more) + 1.16f * x;
-    return 4.81f + 1.89f * turns + each * (1.93f + 0.42f * fill + 5.45f * more) + 3.06f * x;
+    const float turns = (float)((nsb + 7) / 8), each = (float)nsb / 8.f, x = (float)(batch * nsb) * 1e-3f, more = (float)((rows + 8191) / 8192 - 1);
+    if (batch <= 32) return 4.99f + 0.84f * turns + each * (0.73f + 1.57f * more) + 1.99f * x;
+    if (skinny_pieces(2, false, nsb)) return 5.01f + each * (3.97f + 4.22f * more) + 1.67f * x;
+    return 4.75f + 2.13f * turns + each * (1.8f + 5.41f * more) + 2.42f * x;
 }
 
 // Bf16 rows of Q6_K products as they are (the kernel's ROWS form): the conversion between the matrix instructions costs 0.25
@@ -2050,15 +2051,15 @@ int mul_mm_candidates(const ksh_kernel_desc &d, ksh_sched *out, int cap)
         return s;
     };
     if (n < cap) out[n++] = tile(1);
-    // workgroups of whole rows, and the number that fills the chip: one to a compute unit of the tile of two roles, two of the others
-    // (two tall ones share what the chip's power allows one, see mm_rows_tall)
+    // workgroups of whole rows, and the number that fills the chip: one to a compute unit of 128 tokens, two of the others (two of the
+    // large ones take turns on what the chip's power allows, see mm_rows_tall)
     int64_t wgs = (d.dims[2] + tm - 1) / tm * row_tiles;
-    int64_t full = q6 && tm == BM ? 256 : 512;
+    int64_t full = tm == BM ? 256 : 512;
     if (f32x && !q6) {
         const bool tall = mm_rows_tall(d, false, 1);
         const dim3 g = tall ? mm_rows_grid(d, MmRowsTall::TM, MmRowsTall::TN, false, 1) : mm_rows_grid(d, MmRowsSmall::TM, MmRowsSmall::TN, false, 1);
         wgs = (int64_t)g.x * g.y;
-        if (tall) full = 256;
+        full = tall ? 256 : 512;
     }
     if (n < cap && !q6 && d.dims[2] <= kSkinnyMaxBatch && !d.dims[3]) {
         ksh_sched s{};
