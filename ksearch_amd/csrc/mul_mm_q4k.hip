@@ -1236,8 +1236,12 @@ struct RoundParams {
 };
 
 // NM = 2: the gate | up pair (W0, W1 of rows0 rows each; gelu(W0 x) * (W1 x) to Y0)
-template <int NM>
-__global__ __launch_bounds__(512, 4) void q4k_mm_round_kernel(RoundParams p)
+// PIECES: the weights come as pieces of 16 bytes, lane after lane along the rows, straight into LDS.  (A row a lane, an instruction is
+// 64 places of L1 instead of some 20, and L1's path was the busy unit; read back matrix by matrix they also leave registers for a
+// second workgroup on the compute unit.  16 rows: gate | up of 12288 x 1536 17.1 -> 14.3 us, 1536 x 12288 11.9 -> 9.7, 1536 x 2048
+// 5.6 -> 4.9.)  Else a row a lane, which saves the way through LDS where that path is not busy (round_pieces).
+template <int NM, bool PIECES>
+__global__ __launch_bounds__(512, PIECES ? 4 : 2) void q4k_mm_round_kernel(RoundParams p)
 {
     // a wave's weight rows per matrix, and over them its shares of the results, [8][64]: kRoundTile floats each
     extern __shared__ __attribute__((aligned(16))) float red[];   // [8][NM][kRoundTile]
@@ -1259,17 +1263,25 @@ __global__ __launch_bounds__(512, 4) void q4k_mm_round_kernel(RoundParams p)
     // (the other waves ask for nothing: a quarter of the requests were for a row's last superblock again, and the vector-memory
     // path is what the launch is busy with -- gate | up of 12288 x 1536 for 16 rows 18.8 -> 16.8 us)
     if (active) {
-        // ---- every load of the wave, up front: the weights as pieces of 16 bytes, lane after lane along the rows, straight into
-        // LDS.  (A row a lane, an instruction is 64 places of L1 instead of some 20, and L1's path was the busy unit; read back
-        // matrix by matrix they also leave registers for a second workgroup on the compute unit.  16 rows: gate | up of 12288 x
-        // 1536 17.1 -> 14.3 us, 1536 x 12288 11.9 -> 9.7, 1536 x 2048 5.6 -> 4.9; 6144 x 1536, one workgroup a unit, 9.7 -> 10.0.)
+        // ---- every load of the wave, up front
         float *mine = red + wave * NM * kRoundTile;
-        const uint32_t l0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) float *)mine;
         const int last = rows - 1 - r0;
         const uint32_t row_bytes = (uint32_t)nsb * 144u;
+        u32x4_t hdr[NM];
+        u32x2_t q[NM][4][2];
+        auto take = [&](int m, const uint8_t *blk) __attribute__((always_inline)) {
+            hdr[m] = *reinterpret_cast<const u32x4_t *>(blk);
+#pragma unroll
+            for (int g = 0; g < 4; g++) {
+                q[m][g][0] = *reinterpret_cast<const u32x2_t *>(blk + 16 + 32 * g + 8 * h);
+                q[m][g][1] = *reinterpret_cast<const u32x2_t *>(blk + 16 + 32 * g + 16 + 8 * h);
+            }
+        };
 #pragma unroll
         for (int m = 0; m < NM; m++) {
-            ask_q4k_tile((m ? p.W1 : W) + (size_t)r0 * row_bytes + (size_t)sbc * 144, row_bytes, last, lane, l0 + (uint32_t)(m * kRoundTile * 4));
+            const uint8_t *blk = (m ? p.W1 : W) + (size_t)r0 * row_bytes + (size_t)sbc * 144;
+            if constexpr (PIECES) ask_q4k_tile(blk, row_bytes, last, lane, (uint32_t)(uintptr_t)(__attribute__((address_space(3))) float *)mine + (uint32_t)(m * kRoundTile * 4));
+            else take(m, blk + (size_t)min(n, last) * row_bytes);
         }
         const h8 *xa = reinterpret_cast<const h8 *>(p.Xp) + (size_t)sbc * 16 * 64 + lane;
         h8 a[16];
@@ -1278,27 +1290,20 @@ __global__ __launch_bounds__(512, 4) void q4k_mm_round_kernel(RoundParams p)
         // sums of x: rows 0..15 the tokens' hi parts, rows 16..31 their lo parts
         const _Float16 *sx = p.Xp + round_xf_halves(p.cols) + (n >= 16 ? round_sx_halves(p.cols) : 0) + ((size_t)(n & 15) * nsb + sbc) * 32 + 8 * h;
         const h8 a2[2] = {*reinterpret_cast<const h8 *>(sx), *reinterpret_cast<const h8 *>(sx + 16)};
-        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+        if constexpr (PIECES) asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
 
         const f16v kZero16 = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
 #pragma unroll
         for (int m = 0; m < NM; m++) {
-            const uint8_t *blk = reinterpret_cast<const uint8_t *>(mine + m * kRoundTile) + 144 * n;
-            const u32x4_t hdr = *reinterpret_cast<const u32x4_t *>(blk);
-            u32x2_t q[4][2];
-#pragma unroll
-            for (int g = 0; g < 4; g++) {
-                q[g][0] = *reinterpret_cast<const u32x2_t *>(blk + 16 + 32 * g + 8 * h);
-                q[g][1] = *reinterpret_cast<const u32x2_t *>(blk + 16 + 32 * g + 16 + 8 * h);
-            }
+            if constexpr (PIECES) take(m, reinterpret_cast<const uint8_t *>(mine + m * kRoundTile) + 144 * n);
             f16v C = kZero16;
 #pragma unroll
             for (int g = 0; g < 4; g++) {
-                const uint4 s = q4k_group_scales(hdr.y, hdr.z, hdr.w, g);   // sc_lo, mn_lo, sc_hi, mn_hi
+                const uint4 s = q4k_group_scales(hdr[m].y, hdr[m].z, hdr[m].w, g);   // sc_lo, mn_lo, sc_hi, mn_hi
 #pragma unroll
                 for (int j = 0; j < 4; j++) {
                     // slice j: bytes (j & 1 ? 16 + 8h : 8h) .. +7, low nibbles for j < 2, high nibbles after
-                    const u32x2_t qq = q[g][j & 1];
+                    const u32x2_t qq = q[m][g][j & 1];
                     const uint32_t sc = j < 2 ? s.x : s.z;
                     uint32_t o[4];
 #pragma unroll
@@ -1313,11 +1318,11 @@ __global__ __launch_bounds__(512, 4) void q4k_mm_round_kernel(RoundParams p)
             }
             // bias + mins of the superblock: the row's eight coefficients -(dmin*m_j + 1024*d) as f16 hi | lo, against the
             // sums of x (hi[8] hi[8] lo[8] 0[8] per row and superblock): hi*hi + hi*lo + lo*hi
-            const float d = half_bits_to_f32(hdr.x & 0xFFFFu), dmin = half_bits_to_f32(hdr.x >> 16);
+            const float d = half_bits_to_f32(hdr[m].x & 0xFFFFu), dmin = half_bits_to_f32(hdr[m].x >> 16);
             _Float16 chi[8], clo[8];
 #pragma unroll
             for (int g = 0; g < 4; g++) {
-                const uint4 s = q4k_group_scales(hdr.y, hdr.z, hdr.w, g);
+                const uint4 s = q4k_group_scales(hdr[m].y, hdr[m].z, hdr[m].w, g);
                 const float c0 = pinned(-(dmin * (float)s.y + 1024.f * d)), c1 = pinned(-(dmin * (float)s.w + 1024.f * d));
                 chi[2 * g] = (_Float16)c0; chi[2 * g + 1] = (_Float16)c1;
                 clo[2 * g] = (_Float16)(c0 - (float)chi[2 * g]); clo[2 * g + 1] = (_Float16)(c1 - (float)chi[2 * g + 1]);
@@ -1564,6 +1569,13 @@ int launch_round_prep(const ksh_kernel &k, const LaunchArgs &a, hipStream_t st)
     return e == hipSuccess ? 0 : hip_fail(e, "round_prep launch");
 }
 
+// The weights by pieces, or a row a lane: where all eight waves work, or two workgroups share a compute unit, the path of L1 is
+// busy; else the way through LDS is what counts.  16 rows, us, a row a lane | pieces: 1536 x 256 3.00 | 3.27, 4096 x 1024 3.65 | 4.00,
+// 2048 x 1536 with two of 256 rows 4.34 | 4.54, 8192 x 1792 5.37 | 5.58, 12288 x 768 4.92 | 5.20; 8448 x 1024 5.44 | 5.36, 8448 x
+// 1536 7.54 | 7.05, 256 x 2048 5.43 | 4.58, 8192 x 2048 6.53 | 5.82; gate | up 1024 x 256 3.67 | 4.08, 3072 x 768 4.33 | 4.46, 6144 x
+// 1536 even, 9000 x 512 6.32 | 5.82.
+bool round_pieces(bool pair, int nsb, int tiles) { return pair ? nsb >= 6 || tiles > 256 : nsb >= 8 || (nsb >= 4 && tiles > 256); }
+
 int launch_matvec_round(const ksh_kernel &k, const LaunchArgs &a, hipStream_t st)
 {
     const int64_t *d = k.desc.dims;
@@ -1597,8 +1609,9 @@ int launch_matvec_round(const ksh_kernel &k, const LaunchArgs &a, hipStream_t st
     if (d[6] == 1) { p.emit = (_Float16 *)a.out[0]; p.Y0 = p.Y1 = p.Y2 = nullptr; }
     if (d[6] == 2) p.part = (float *)a.out[0];     // the slices' partial sums are the result
     const dim3 grid(k.info.grid[0], k.info.grid[1]);
-    if (pair) hipLaunchKernelGGL(q4k_mm_round_kernel<2>, grid, dim3(512), k.info.lds_bytes, st, p);
-    else hipLaunchKernelGGL(q4k_mm_round_kernel<1>, grid, dim3(512), k.info.lds_bytes, st, p);
+    auto launch = [&](auto kernel) { hipLaunchKernelGGL(kernel, grid, dim3(512), k.info.lds_bytes, st, p); };
+    if (round_pieces(pair, p.cols / 256, (int)grid.x)) pair ? launch(q4k_mm_round_kernel<2, true>) : launch(q4k_mm_round_kernel<1, true>);
+    else pair ? launch(q4k_mm_round_kernel<2, false>) : launch(q4k_mm_round_kernel<1, false>);
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return hip_fail(e, "matvec_round launch");
     if (grid.y > 1 && d[6] != 2) {

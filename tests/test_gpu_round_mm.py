@@ -61,6 +61,26 @@ def test_matvec_round_vs_oracle(ctx, rows, cols, batch):
             assert err < 2e-5, err
 
 
+@pytest.mark.parametrize("rows,more,cols,pair", [(8192, 25, 1024, False), (8192, 25, 1536, False), (8192, 25, 768, False), (33, 8161, 1280, False),
+                                                  (8192, 25, 1280, True), (31, 8170, 256, True)])
+def test_matvec_round_weights_by_pieces_or_a_row_a_lane(ctx, rows, more, cols, pair):
+    """Weights come by pieces from 257 tiles on (of one matrix with four superblocks at least) and a row a lane up to 256: the same
+    rows alone and at the front of a longer matrix have the same bits, and the accuracy of the others (a pair's: see the ragged
+    tiles below)."""
+    batch = 16
+    ws = [np.frombuffer(bytes(synth.q4k_blocks((rows + more) * cols // 256, seed=930 + i)), np.uint8) for i in range(1 + pair)]
+    x = synth.normal_f32(batch * cols, 932).reshape(batch, cols) * 0.25
+    _, (alone,) = round_mm(ctx, [w[:rows * cols // 256 * 144] for w in ws], (rows,), cols, x, batch, pair)
+    _, (all_,) = round_mm(ctx, ws, (rows + more,), cols, x, batch, pair)
+    assert np.array_equal(alone, all_[:, :rows])
+    for t in (0, batch - 1):
+        want = [oracle.matvec_f64(oracle.Q4K, w, rows + more, cols, x[t]) for w in ws]
+        if pair:
+            g = np.clip(want[0], -20.0, 20.0)
+            want = [0.5 * g * (1.0 + np.tanh(0.7978845608 * (g + 0.044715 * g ** 3))) * want[1]]
+        assert np.max(np.abs(all_[t] - want[0]) / np.maximum(np.abs(want[0]), np.sqrt(np.mean(want[0] ** 2)))) < (3e-4 if pair else 2e-5)
+
+
 @pytest.mark.parametrize("rows,cols,batch", [(6144, 1536, 16), (12288, 1536, 3), (96, 2048, 9)])
 def test_matvec_round_gate_up_gelu(ctx, rows, cols, batch):
     wg, wu = synth.q4k_blocks(rows * cols // 256, seed=910), synth.q4k_blocks(rows * cols // 256, seed=911)
