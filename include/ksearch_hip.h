@@ -65,9 +65,8 @@ enum ksh_kind {
     KSH_MATVEC = 1,
     /* MatvecBatch: Y[t,r] = sum_c W[r,c] X[t,c].  dims: rows, cols, batch.
      * dtypes[0] = Q4K | Q6K (GGUF byte order, blocks at 2-byte alignment),
-     * dtypes[1] = BF16 (X) or F32 (X is then taken as hi + lo f16 parts, 22 bits: two passes, two sets of workgroups,
-     * or -- Q4_K with a grid of at least 256 tiles -- one workgroup walking both; the form the decode loops' prompt
-     * chunks use), output F32 token-major.
+     * dtypes[1] = BF16 (X) or F32 (X is then taken as hi + lo f16 parts, 22 bits, which meet a converted weight in
+     * the same workgroup; the form the decode loops' prompt chunks use), output F32 token-major.
      * in: W, X   out: Y[batch, rows]
      * dims[3], dims[4] (0 = none): rows of a second and a third matrix of the same dtype over the same X, taken in
      * the same launch (q | k | v of a prompt chunk: one preparation of X, one grid).  in: W, X, W1[, W2]
@@ -90,7 +89,9 @@ enum ksh_kind {
      *   fold's order, so a chain of GEMMs gives the same numbers with and without its folds.
      * F32 activations travel as hi + lo f16 parts.  The tile scales every row by its own power of two first (any
      * finite f32 row fits); the small-batch form does not: there |x| must stay below 65504.
-     * sched.nr0 = 32 | 128 picks the small-batch form (Q4_K, up to 64 tokens, one matrix) or the 128 x 128 tile;
+     * sched.nr0 = 32 | 128 picks the small-batch form (Q4_K, up to 64 tokens, one matrix) or the tiles, whose tokens
+     * and rows follow from the sizes (info.name has them; sched.tg and sched.lds_tile name the kernel that reports
+     * them: 256 and 32 Q4_K, 256 and 64 or 512 and 64 Q6_K);
      * sched.k_split = the tile's K slices (a divisor of cols / 256, or for bf16 rows the count of a reported schedule;
      * 1 = whole rows; 0 = enough to fill the chip). */
     KSH_MATVEC_BATCH = 2,

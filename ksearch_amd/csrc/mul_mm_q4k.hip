@@ -46,8 +46,8 @@ constexpr int PITCH = KS + 8;      // halves per LDS row of the main tiles (144 
 // X bf16 -> f16 (permuted) in the order the matrix instruction wants its A operand, plus the min-term
 // operand per (token, superblock): 32 halves = Sx_hi[8] | Sx_hi[8] | Sx_lo[8] | 0[8].
 // Xf[token / 32][k / 16][lane][8] with lane = token % 32 + 32 * ((k / 8) % 2): one 32 x 16 fragment is 1 KB,
-// lane after lane, so that a multiplying wave fetches it with a single 128-bit load per lane and the
-// activations never pass through LDS.
+// lane after lane: a whole kilobyte that goes straight into LDS (q4k_mm_rows.hpp) or, with a single 128-bit load
+// per lane, into a multiplying wave's registers (the others).
 // A wave takes 32 tokens x one 32-column sub-block: lane (token % 32, h) converts the 8-element runs h and 2 + h
 // of the sub-block and is lane token % 32 + 32 h of the sub-block's two fragments, so both leave as whole
 // kilobytes, lane after lane (with a thread per run in row order, the eight 16-byte pieces of a 128-byte line of
@@ -367,7 +367,7 @@ struct MmParams {
     // full K, results in Y).
     int ksplit;
     float *Y_parts;
-    // Up to three matrices that share the activations (q | k | v of a prompt chunk) in one launch of the 128 x 128
+    // Up to three matrices that share the activations (q | k | v of a prompt chunk) in one launch of the
     // tile: blockIdx.y counts the row tiles of W, then of W1, then of W2, each with its own result.
     const uint8_t *W1, *W2;
     float *Y1, *Y2;
@@ -886,7 +886,7 @@ __device__ __forceinline__ void ask_q4k_tile(const uint8_t *blk, uint32_t row_by
 }
 
 // ---- small batches (up to 64 tokens): a GEMV-shaped launch on the matrix cores ---------------------------------
-// A prompt remainder or a round of decoding slots is a few dozen tokens: the 128 x 128 tile then leaves most of the
+// A prompt remainder or a round of decoding slots is a few dozen tokens: the tiles then leave most of the
 // chip idle (rows / 128 workgroups) and half of every tile empty.  Here a workgroup owns 32 weight rows and all
 // tokens; its 8 waves split the row's superblocks between them (K-split inside the workgroup, folded through LDS at
 // the end, so the sum order is fixed) and every wave reads its weights, from memory or LDS, in the order the matrix
@@ -1436,7 +1436,7 @@ __global__ __launch_bounds__(256) void mm_parts_fold_kernel(const float *__restr
 // rows of up to 2048 columns).  The B operand is the 6-bit code minus 32 as an exact f16 integer (the code OR-ed into
 // the mantissa of 1024.0, minus 1056 with one packed subtraction per two weights); Q6_K has one int8 scale per 16
 // columns, which is the K depth of the matrix instruction, so the scale is applied in f32 to the instruction's
-// result: nothing is rounded (folded into the f16 operand as the 128 x 128 tile does it, sc * q above 2048 loses
+// result: nothing is rounded (folded into the f16 operand as the tile of two roles does it, sc * q above 2048 loses
 // its last bit).  A workgroup keeps the activations of the whole row in registers -- wave w the 16 fragments of
 // superblock w -- and walks tiles of 32 weight rows, the next tile's bytes in flight under the current one; the waves'
 // shares of a tile meet in LDS (two buffers, one barrier per tile).
@@ -1814,7 +1814,7 @@ int bind_matvec_batch(ksh_kernel &k)
     if (rows <= 0 || batch <= 0 || rows > (1 << 24) || batch > (1 << 20)) return set_error("matvec_batch: rows=%lld batch=%lld", (long long)rows, (long long)batch);
     if (cols <= 0 || cols % 256 || cols > (1 << 20)) return set_error("matvec_batch: cols=%lld is not a positive multiple of 256", (long long)cols);
     // dims[3], dims[4]: the rows of a second and a third matrix over the same activations (q | k | v of a prompt
-    // chunk), taken by the 128 x 128 tile in the same launch
+    // chunk), taken by the tiles in the same launch
     const int64_t rows1 = k.desc.dims[3], rows2 = k.desc.dims[4], rows_all = rows + rows1 + rows2;
     if (rows1 < 0 || rows2 < 0 || (rows2 && !rows1) || rows_all > (1 << 24)) return set_error("matvec_batch: rows of the further matrices %lld, %lld", (long long)rows1, (long long)rows2);
     const int n_mat = 1 + (rows1 > 0) + (rows2 > 0);
@@ -1874,7 +1874,7 @@ int bind_matvec_batch(ksh_kernel &k)
     const size_t batch32 = (size_t)((batch + 31) / 32 * 32);
     k.scratch_bytes = (batch32 * cols * 2 + batch32 * (cols / 256) * 64) * (f32x ? 2 : 1);
     // schedule: nr0 = weight rows per workgroup.  32 = the small-batch form (Q4_K, up to 64 tokens: the default
-    // there), 128 = the 128 x 128 tile.
+    // there), 128 = the tiles (their tokens and rows follow from the sizes).
     const uint32_t want = k.desc.sched.nr0;
     if (want && want != 32 && want != BN) return set_error("matvec_batch: unsupported schedule nr0=%u (32 or %d)", want, BN);
     const bool can_skinny = !q6 && batch <= kSkinnyMaxBatch && n_mat == 1 && !unfolded && !cut && !pair;

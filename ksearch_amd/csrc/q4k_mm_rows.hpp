@@ -2,8 +2,8 @@
 // part, mm_prep_x_kernel): every wave
 // converts its own weights in registers and multiplies them with fragments that the workgroup shares in LDS.
 //
-// What bounds it: the matrix pipe and the chip's power.  With two workgroups on every compute unit the pipe is busy 60 % of the
-// cycles, at 1.7 - 1.8 GHz; a launch of nothing but its matrix instructions holds 1.6 GHz.  In its place was a tile of four waves
+// What bounds it: the matrix pipe and the chip's power.  With two workgroups on every compute unit (gate | up of 12288 x 1536, 2048
+// tokens) the pipe is busy 60 % of the chip's cycles, at 1.7 GHz, and with one (1536 x 12288, 192 workgroups) 44 %; a launch of nothing but its matrix instructions holds 1.6 GHz.  In its place was a tile of four waves
 // that loaded and converted, handing weights to four that multiplied through LDS, and of fragments from memory to registers:
 // at 32 x 64 a wave the fragments alone keep the path from L1 busy for as long as the matrix instructions take, and the roles
 // waited for each other at every step (pipe busy 44 %).  Here a wave has 64 tokens x 64 rows (or 32 x 64, or 32 x 32), a
@@ -14,9 +14,10 @@
 //
 // With bf16 rows there are half as many matrix instructions to a converted weight, and a wave has 64 tokens x 32 rows, or 128 x
 // 32 where the chip is full: 2048 tokens, 12288 x 4096 257 -> 221 us, 300 tokens, 12288 x 1536 29.7 -> 24.1, 65 tokens, 12288 x
-// 8192 46 -> 40; 512 tokens, 8192 x 2048 30.8 -> 29.5, where the vector instructions (318 a superblock and wave) and the matrix
-// instructions fill a SIMD's time one after the other (20 and 18 thousand of 39 thousand cycles; neither fragments read two
-// units ahead nor eight half steps on their way change it).
+// 8192 46 -> 40; 512 tokens, 8192 x 2048 in 64 x 128 30.5 -> 30.2.  That launch takes 128 x 128 now (28.5 -> 27.7 with its
+// preparation), one wave to a SIMD, whose matrix pipe is busy for 36 % of the cycles and its vector ALU for 29; the wave waits for 18
+// %, the rest lies between its instructions.  (In 64 x 128, two waves to a SIMD, the two take 18 and 20 of 39 thousand cycles, yet neither
+// fragments read two units ahead, nor eight half steps on their way, nor a conversion of 11 % fewer instructions changed its time.)
 //
 // A product's order is fixed, so its bits do not depend on the shape that does it: per 16 columns the hi and the lo part against
 // the same weights into a superblock's own accumulator, then F = (bias and mins, two short products) + F and F = d * C + F.
@@ -415,9 +416,9 @@ __global__ __launch_bounds__(S::kThreads, 2) void q4k_mm_rows_kernel(MmParams p)
         for (int nt = 0; nt < NT; nt++) F[0][nt] = T[nt];
     }
     // accumulator layout of the 32x32 tile: column = lane % 32, row = 8*(i/4) + 4*(lane/32) + i%4
-    // (bf16 rows: stored past the L2s, since what those hold of it at the kernel's end is written out before the next kernel
-    // starts; 512 tokens, 8192 x 2048 30.8 -> 29.5 us, 300 tokens, 12288 x 1536 24.1 -> 22.9.  In a prompt's chain of launches it is even,
-    // 700 tokens 10.09 ms.)
+    // (bf16 rows: stored past the L2s where mm_keeps does not say otherwise, since what those hold of it at the kernel's end is
+    // written out before the next kernel starts; 512 tokens, 8192 x 2048 30.8 -> 29.5 us, 300 tokens, 12288 x 1536 24.1 -> 22.9.  In a
+    // prompt's chain of launches it is even, 700 tokens 10.09 ms.)
     auto store = [&](auto keep) __attribute__((always_inline)) {
 #pragma unroll
         for (int mt = 0; mt < MT; mt++) {

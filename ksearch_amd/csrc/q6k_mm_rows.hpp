@@ -5,10 +5,10 @@
 // What bounds it: the vector instructions (640 a superblock and wave for 64 tokens, 5.1 of some 7 thousand cycles with two waves a
 // SIMD; the matrix instructions 2).  What bounded the first form was the rate of L1: a row a lane, at the odd addresses of
 // blocks of 210 bytes, cost 186 cycles a load.  So a wave loads 16-byte pieces at 16-byte addresses, lane after lane along the
-// rows, and passes them through LDS.  2 tokens, 12288 x 6144 41.3 -> 25.8 us, 32 tokens 45.2 -> 30.0, 64 tokens 48.9 -> 39.6; 20
-// tokens, 4096 x 2048 12.0 -> 9.4; 77 tokens, 1000 x 3072 13.3 -> 11.0; 300 tokens, 12288 x 1536 47.7 -> 36.5.  Beyond (333
-// tokens, 1536 x 6144 25.9 or 28.8; 512, 8192 x 2048 36.5 or 44.4) converting for 64 tokens is the dearer way, and for 128
-// here (29 us, 43) one wave a SIMD is left.
+// rows, and passes them through LDS.  (The 128-token tile as it was -> this kernel now) 2 tokens, 12288 x 6144 41.0 -> 23.6 us, 32
+// tokens 45.3 -> 28.0, 64 tokens 47.1 -> 35.9; 20 tokens, 4096 x 2048 11.2 -> 8.7; 77 tokens, 1000 x 3072 13.0 -> 10.4; 300
+// tokens, 12288 x 1536 49.0 -> 34.3.  Beyond (512 tokens, 8192 x 2048 30.8 in that tile or 40.9 here) converting for 64 tokens is
+// the dearer way, and for 128 here one wave a SIMD is left.
 #pragma once
 #include "ksh_device.hpp"
 #include "ksh_internal.hpp"

@@ -1666,8 +1666,12 @@ bool prompt_rows(int64_t n_kv, int64_t hd, int64_t max_t, int nwg)
 bool prompt_rows_aligned(const LaneParams &p) { return (((uintptr_t)p.k | (uintptr_t)p.v | p.slot_stride) & 15) == 0; }
 
 // Two tokens to a workgroup, of one prompt and where half as many workgroups still fill the chip (two to a compute unit of
-// heads of 256, one of heads of 512): see the figures at sdpa_prompt_kernel; 1024 tokens of heads of 256 59 us with one token,
-// 61 with two, 699 40 and 46.
+// heads of 256, one of heads of 512).  Both ways go up in steps, with the rounds of their workgroups, and which step comes first hangs
+// on the rows attended, which the host does not know; the line is where chunks of 2048 and of 952 gain.  One token | two, us, from
+// an empty cache: heads of 256, 700 tokens 35.7 | 42.1, 800 43.6 | 42.4, 1024 52.1 | 54.1, 1200 71.7 | 78.4, 1300 83.1 | 79.3, 2048 152 |
+// 145, with a window of 512 1200 47.7 | 51.3, 2048 75.3 | 70.7, 952 behind 2048 41.9 | 37.9; heads of 512, 400 39.5 | 33.6, 600
+// 58.5 | 64.3, 800 93.7 | 77.9, 2048 359 | 311.  So a prompt of 1100 to 1200 tokens, or of 600 to 700 on heads of 512, pays up to
+// a tenth of a launch; the kernel before these two took 83.2 us where 78.4 stands.
 bool prompt_pairs(int64_t n_kv, int64_t hd, int64_t n_tok, bool one_prompt)
 {
     return one_prompt && n_tok * n_kv >= (hd == 512 ? 512 : 896);
