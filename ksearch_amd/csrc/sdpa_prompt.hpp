@@ -12,7 +12,7 @@
 // us, (one token in sdpa_mfma_kernel, T = 1, T = 2): heads of 512, 2048 tokens from an empty cache 452, 359, 311; 952 behind 2048
 // rows 485, 379, 309; 512 49, 40.5, 40.7; 63 behind 700 41.5, 33.7, 52.7; heads of 256, window of 512, 2048 tokens 87, 75, 71; 952
 // behind 2048 47, 42, 38; 699 from an empty cache 34, 30, 34.5.  The vector ALU is busy for 77 % of the cycles now (heads of 512, 2048
-// tokens; 83 with heads of 256, 67 with one token to a workgroup), the matrix pipe 8.
+// tokens; 83 with heads of 256, 67 with one token to a workgroup), the matrix pipe 10.
 #pragma once
 // (included by sdpa_q40_lanes.hip, behind sdpa_mfma_kernel)
 namespace ksh {
