@@ -16,7 +16,7 @@
 // 32 where the chip is full: 2048 tokens, 12288 x 4096 257 -> 221 us, 300 tokens, 12288 x 1536 29.7 -> 24.1, 65 tokens, 12288 x
 // 8192 46 -> 40; 512 tokens, 8192 x 2048 in 64 x 128 30.5 -> 30.2.  That launch takes 128 x 128 now (28.5 -> 27.7 with its
 // preparation), one wave to a SIMD, whose matrix pipe is busy for 36 % of the cycles and its vector ALU for 29; the wave waits for 18
-// %, the rest lies between its instructions.  (In 64 x 128, two waves to a SIMD, the two take 18 and 20 of 39 thousand cycles, yet neither
+// %, the rest lies between its instructions.  (In 64 x 128, two waves to a SIMD, the two take 18 and 23 of 45 thousand cycles, yet neither
 // fragments read two units ahead, nor eight half steps on their way, nor a conversion of 11 % fewer instructions changed its time.)
 //
 // A product's order is fixed, so its bits do not depend on the shape that does it: per 16 columns the hi and the lo part against

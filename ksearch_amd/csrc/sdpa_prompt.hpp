@@ -1,8 +1,8 @@
 // Attention of a prompt chunk's tokens (KSH_SDPA_BATCH, heads of 256 and 512, one partition): sdpa_mfma_kernel's workgroup of one
 // token, or of two, T -- the same products, scores and states in the same order, the same bits.
 //
-// What bounds it: the vector ALU (1208 instructions a tile of a 512-wide head and wave in that kernel, 57 % of the cycles; heads
-// of 256 1347, 68 %) and a wave's waits for its tile (45 and 32 % of its time).  Here K and V come straight into LDS, K of a
+// What bounds it: the vector ALU (1208 instructions a tile of a 512-wide head and wave in that kernel, 55 % of the cycles; heads
+// of 256 1336, 72 %) and a wave's waits for its tile (45 and 32 % of its time).  Here K and V come straight into LDS, K of a
 // wave's next tile under this one's softmax and products and V under the next one's scores, so that one set of buffers covers
 // both ways, and a block's operands are read from there while the last block is worked on.
 // T = 2: tokens t and t + 32 of one prompt attend the same tiles of 32 rows -- rows from the cache's start on, or windows that
