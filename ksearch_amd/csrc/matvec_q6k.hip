@@ -338,6 +338,7 @@ __global__ __launch_bounds__(NW * 64) void q6k_stream_kernel(Q6kParams p)
     };
 
     constexpr int KMAX = ((A + TAIL) * 512 + NW * 64 - 1) / (NW * 64);   // float4 of the vector per thread
+    static_assert(KMAX <= kStageP, "the norms' operands of the whole row in registers");
     StageRegs sr;
     stage_fetch<NW * 64, false, KMAX>(p.pro, cols, sr);
     // One group is asked for behind the vector, and the others behind the barrier: a compute unit takes a limited number of requests,
@@ -578,7 +579,8 @@ int bind_matvec_q6k(ksh_kernel &k)
     else if (cols > 2048 && G.R > 2) { G.rpw = G.rpw / G.R * 2; G.R = 2; }
     if (!((G.R == 1 || G.R == 2 || G.R == 4) && (G.NW == 2 || G.NW == 4 || G.NW == 8)) || G.rpw % G.R || G.rpw > 32767)
         return set_error("matvec_q6k: unsupported schedule nr0=%d nsg=%d unroll=%u", G.R, G.NW, k.desc.sched.unroll);
-    if (pro && cols > (int64_t)4 * G.NW * 64 * kStageP)
+    // (the streaming kernel holds the norms' operands of every length in registers, whatever the schedule that stands for it)
+    if (pro && !stream && cols > (int64_t)4 * G.NW * 64 * kStageP)
         return set_error("rmsnorm_matvec requires LOCAL staging of the vector (cols=%lld too large)", (long long)cols);
     k.info.n_inputs = pro ? (has_res ? 5 : 3) : 2;
     k.info.n_outputs = has_res ? 2 : 1;

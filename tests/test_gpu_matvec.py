@@ -417,6 +417,40 @@ def test_rmsnorm_matvec_q6k_lm_head_prologue(ctx, eng, has_res):
             assert_close(ctx.read_f32(xn, n), x_new, 1e-5, "x_new")
 
 
+@pytest.mark.parametrize("cols", [2304, 4096, 4352, 6144, 8192])
+@pytest.mark.parametrize("has_res", [False, True])
+def test_rmsnorm_matvec_q6k_long_rows(ctx, cols, has_res, tmp_path, monkeypatch):
+    """The norm in front of file-order Q6_K over every length that the streaming kernel takes: left open, by the schedule that its
+    handle reports, by the schedules of the regrouped rows' kernel and through a search, whose one candidate binds."""
+    monkeypatch.setenv("KSEARCH_BEAM_CACHE", str(tmp_path / "beam"))
+    rows, eps = 301, 1e-6
+    x, w_norm, w_post, res = (synth.normal_f32(cols, 820 + i) for i in range(4))
+    w_norm, w_post = 1.0 + 0.1 * w_norm, 1.0 + 0.1 * w_post
+    if has_res:
+        x_new, vec = oracle.rmsnorm_add_then_rmsnorm(x, w_post, res, w_norm, eps)
+    else:
+        x_new, vec = None, oracle.rmsnorm(x, w_norm, eps)
+    w = synth.q6k_blocks(rows * cols // 256, seed=cols)
+    want = oracle.matvec_f64(oracle.Q6K, w, rows, cols, vec)
+    ins = [ctx.buffer_bytes(w)] + [ctx.buffer_f32(a) for a in ([x, w_norm, w_post, res] if has_res else [x, w_norm])]
+    desc = lambda sched=None: hip.make_desc(hip.Kind.RMSNORM_MATVEC, (rows, cols, int(has_res)), (DType.Q6K, DType.F32), (eps,), sched)
+    k = ctx.compile(desc())
+    assert "stream" in k.name
+    scheds = [None, k.info.sched] + [dict(nsg=nsg, nr0=nr0, unroll=u) for nsg, nr0, u in ((8, 1, 2), (8, 4, 8), (4, 2, 2), (2, 1, 2))]
+    for s in scheds:
+        kk = ctx.compile(desc(s))
+        assert kk.name == k.name, s
+        y, xn = ctx.buffer_f32(np.full(rows + 64, 7.0, np.float32)), ctx.buffer_empty_f32(cols)
+        ctx.encode_multi(kk, ins, [y, xn] if has_res else [y])
+        got = ctx.read_f32(y, rows + 64)
+        assert_close(got[:rows], want, 1e-5, f"{cols} {s}")
+        assert np.all(got[rows:] == 7.0)
+        if has_res:
+            assert_close(ctx.read_f32(xn, cols), x_new, 1e-5, "x_new")
+    best, ms, cached = ctx.beam_search(desc(), ins, [y, xn] if has_res else [y], iters=2, force=True)
+    assert not cached and ms > 0 and ctx.compile(desc(best)).name == k.name
+
+
 def test_beam_search_on_device(ctx, eng, tmp_path, monkeypatch):
     """Eng::beam_matvec (ksearch_kernels/src/lib.rs:1985-2043): every candidate is timed on the device, the best one
     is saved as a plan under KSEARCH_BEAM_CACHE, a second search is served from the file, and a kernel compiled
