@@ -230,7 +230,8 @@ int bind_matvec_q4k_family(ksh_kernel &k)
     if (named) sched = ksh_sched{};
     const int64_t sized_by = s.nm == 2 ? s.rows[0] : total_rows;
     Q4kGeom G = pick_geom(sched, (int)sized_by, bpr);
-    G.stream = named || (sched_is_zero(sched) && s.prologue != kMergeParts && q4s_pays(s.n_mat, sized_by, bpr));
+    const int64_t half_wgs = (sized_by + G.rpw() * G.NW - 1) / (G.rpw() * G.NW);
+    G.stream = named || (sched_is_zero(sched) && s.prologue != kMergeParts && q4s_pays(s.n_mat, sized_by, bpr, half_wgs, G.NW));
     // QKV at one row per half-wave: one dot per lane does not pay for turning the vector into digit planes (3.86 vs 4.08 us)
     if (sched_is_zero(sched) && s.n_mat == 3 && G.half && G.R == 1) G.var = kXF32;
     if (s.prologue == kMergeParts) {

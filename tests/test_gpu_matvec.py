@@ -306,6 +306,27 @@ def test_matvec_q4k_stream_edges(ctx, bpr, rows, kv_rows):
             assert np.all(got[len(v):] == 7.0)
 
 
+@pytest.mark.parametrize("cols,rows,streams", [
+    (1536, 8192, False), (1536, 8193, True), (1536, 12272, True), (1536, 12273, True), (1536, 12287, True), (1536, 12288, False),
+    (1536, 12289, True), (1536, 15551, True), (1536, 15553, False), (1536, 16384, False), (1536, 16385, True), (1536, 20480, True),
+    (2048, 8192, False), (2048, 8193, True), (2048, 12288, True), (2048, 15551, True), (2048, 15585, False), (2048, 16384, False),
+    (2048, 16385, True), (2048, 24576, False), (2048, 24577, True)])
+def test_gate_up_form_follows_the_other_forms_turns(ctx, cols, rows, streams):
+    """gate | up of 1536 and 2048 columns left open: the half-wave form where its workgroups fill the compute units to the last turn, the
+    streaming form elsewhere; the result on either side of every line (bound as for the streaming kernel's edges)."""
+    k = ctx.compile(hip.make_desc(hip.Kind.MATVEC_GATE_UP_GELU, (rows, cols), (DType.Q4K, DType.F32)))
+    assert ("stream" in k.name) == streams, k.name
+    x = synth.normal_f32(cols, seed=rows)
+    ws = [synth.q4k_blocks(rows * cols // 256, seed=rows + i) for i in (1, 2)]
+    g, u = (oracle.matvec_f64(oracle.Q4K, w, rows, cols, x) for w in ws)
+    out = ctx.buffer_f32(np.full(rows + 64, 7.0, np.float32))
+    ctx.encode_multi(k, [ctx.buffer_bytes(w) for w in ws] + [ctx.buffer_f32(x)], [out])
+    got = ctx.read_f32(out, rows + 64)
+    most = 2.13 * 5e-6 * max(np.abs(g).max(), np.sqrt(cols)) * max(np.abs(u).max(), np.sqrt(cols))
+    assert np.abs(got[:rows] - oracle.gelu_mul(g.astype(np.float32), u.astype(np.float32))).max() <= most
+    assert np.all(got[rows:] == 7.0)
+
+
 def test_lm_head_cfg1_full_size_with_argmax(ctx, eng):
     rows, cols = 262144, 2048
     w, x = synth.cfg1_q6k_lm_head()
