@@ -479,9 +479,9 @@ int launch_q6k_stream(const Q6kParams &p, bool by_rows, unsigned grid, size_t ld
 // 155.5 and 134.9; 65536 x 2048 28.0 and 23.3, 32768 x 1536 14.9 and 12.0, 16384 x 2048 12.2 and 7.7, x 4096 28.1 and 12.9, 8192 x 2048 6.6
 // and 5.3, x 1536 6.2 and 5.1, 4096 x 2048 4.5 and 4.1, x 4096 7.7 and 6.2, x 1536 4.4 and 4.1, 3000 x 2048 4.4 and 3.9; below, where a
 // workgroup has few rows to stage the vector for, 2048 x 4096 4.5 and 4.9, x 1536 3.3 and 3.7, 1000 x 2048 3.15 and 3.4.  Rows of 1536 columns,
-// six of eight lane groups at work and requests of 2048 bytes for 1264, gain less the longer the stream: 65536 rows 25.0 and 23.2, 131072
-// 42.0 and 39.8, 262144 66.9 to 72.8 and 66.9 to 69.4.
-bool q6r_streams(int64_t rows, int bpr) { return rows >= 3000 && (bpr != 6 || rows <= 131072); }
+// six of eight lane groups at work and requests of 2048 bytes for 1264, gain less the longer the stream: 65536 rows 22.2 and 19.7, 131072
+// 34.0 and 31.7, 200000 51.6 and 46.6, 262144 62.4 and 60.8 (64.2 and 61.1 behind a norm).
+bool q6r_streams(int64_t rows) { return rows >= 3000; }
 
 struct Q6kGeom {
     int R, NW, rpw;
@@ -567,7 +567,7 @@ int bind_matvec_q6k(ksh_kernel &k)
     const bool named = sched.nsg == (uint32_t)form.NW && sched.nr0 == (uint32_t)form.G && sched.unroll == (uint32_t)form.NBUF;
     if (named) sched = ksh_sched{};
     Q6kGeom G = pick_geom6(sched, (int)rows);
-    const bool stream = !by_rows || named || (sched_is_zero(sched) && q6r_streams(rows, bpr));
+    const bool stream = !by_rows || named || (sched_is_zero(sched) && q6r_streams(rows));
     if (by_rows && sched_is_zero(sched)) {   // measured best on 262144 x 2048
         G.NW = 8;
         G.R = 1;
@@ -617,15 +617,15 @@ int bind_matvec_q6k(ksh_kernel &k)
 int matvec_q6k_candidates(const ksh_kernel_desc &d, ksh_sched *out, int cap)
 {
     int n = 0;
-    if (d.dtypes[0] == KSH_Q6K) {
-        const int64_t cols = d.dims[1];
-        if (cols <= 0 || cols % 256 || cols > 8192 || cap < 1) return 0;
+    const int64_t cols = d.dims[1];
+    // the streaming kernel: file order's one form, and one of regrouped rows'
+    if (n < cap && cols > 0 && cols % 256 == 0 && cols <= 8192) {
         const Q6sForm form = q6s_form((int)(cols / 256));
         ksh_sched s{};
         s.nsg = (uint32_t)form.NW; s.tg = 64ull * s.nsg; s.vec = 3; s.unroll = (uint32_t)form.NBUF; s.nr0 = (uint32_t)form.G; s.k_split = 1;
         out[n++] = s;
-        return n;
     }
+    if (d.dtypes[0] == KSH_Q6K) return n;
     for (uint32_t nsg : {2u, 4u, 8u})
         for (uint32_t nr0 : {1u, 2u, 4u})
             for (uint32_t unroll : {2u, 8u}) {

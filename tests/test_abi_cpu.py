@@ -173,6 +173,17 @@ def test_prompt_gemm_candidates_name_kernels_that_are_built(wdt, xdt, batch, til
     assert c and {(s.tg, s.lds_tile) for s in c} == {tile} and all(s.tg == 64 * s.nsg for s in c)
 
 
+@pytest.mark.parametrize("cols,stream", [(1536, (16, 1, 4)), (2048, (16, 2, 2)), (4096, (16, 1, 2))])
+@pytest.mark.parametrize("kind", [hip.Kind.MATVEC, hip.Kind.RMSNORM_MATVEC])
+def test_q6k_candidates_have_the_streaming_form(kind, cols, stream):
+    """A search over either byte order of Q6_K times the streaming form (waves, rows, groups on their way); regrouped rows' others beside
+    it, once each."""
+    of = lambda dt: [(s.nsg, s.nr0, s.unroll) for s in hip.beam_candidates(hip.make_desc(kind, (5000, cols, 0), (dt, hip.DType.F32)))]
+    assert of(hip.DType.Q6K) == [stream]
+    c = of(hip.DType.Q6K_ROWS)
+    assert c[0] == stream and len(c) == len(set(c)) == 19
+
+
 def test_kernel_lookup_takes_any_sequence():
     """Eng._k with lists, arrays and tuples of the same numbers finds one handle."""
     import numpy as np

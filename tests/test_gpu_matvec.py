@@ -193,7 +193,7 @@ def test_matvec_q6k_row_grouped(ctx, eng, rows, cols, sched):
 
 
 @pytest.mark.parametrize("cols,sched", [(1536, dict(nsg=16, nr0=1, unroll=4)), (2048, dict(nsg=16, nr0=2, unroll=2)), (4096, dict(nsg=16, nr0=1, unroll=2))])
-@pytest.mark.parametrize("rows", [1, 2, 37, 2999, 3000, 20001])
+@pytest.mark.parametrize("rows", [1, 2, 37, 2999, 3000, 20001, 131073])
 def test_matvec_q6k_row_grouped_streamed(ctx, eng, rows, cols, sched):
     """Regrouped rows in the streaming kernel: groups cut short by the last row, waves without rows and with several rounds of requests,
     by the schedule that its handles report and, from 3000 rows, left open.  Tolerance as for file order."""
