@@ -1873,9 +1873,14 @@ bool sdpa_lanes_supports(int64_t n_q, int64_t n_kv, int64_t hd)
 // 4000 rows attended 8.6 | 9.4 | 14.1 with one workgroup, 4.0 | 4.3 | 6.6 with eight; 8 over 4 5.5 | 5.9 | 8.6 and 4.2 | 4.3 | 6.5; 16 over 2,
 // 16384 rows, 64 partitions 8.9 | 10.8 | 14.4 (an eighth, half and all of them) and, four heads each, 6.4 | 7.1 | 9.1.  Three workgroups of
 // four heads and four waves share a compute unit: where two to a kv head are more than that, and one fits, one (400: 8.7 | 9.9 | 12.4 and
-// 10.2 | 11.3 | 13.4 with two; 320: 8.7 | 10.2 | 13.2 and 7.5 | 8.3 | 10.7).
+// 10.2 | 11.3 | 13.4 with two; 320: 8.7 | 10.2 | 13.2 and 7.5 | 8.3 | 10.7).  Up to four heads of partitions of 1024 rows and more stay
+// together where they would be 257 to 512 workgroups: eight waves of each are one workgroup too many for a compute unit, and four are
+// too few for the rows (32 over 8, 16 partitions, 1 | 512 | 2000 | 16384 rows attended 5.1 | 5.5 | 6.5 | 20.0 together, 5.9 | 6.2 | 6.7 |
+// 20.3 in eight waves each, 4.0 | 4.4 | 5.7 | 22.0 in four; 8 over 4, 64 partitions, 1 | 2000 | 65536 rows 4.8 | 5.3 | 20.5, 5.6 | 6.2 | 20.3
+// and 3.9 | 4.3 | 21.7).
 static int parts_head_split(int64_t launch, int64_t rows, int groups, int hd)
 {
+    if (hd == 128 && groups <= 4 && rows >= 1024 && launch * groups > 256 && launch * groups <= 512) return 1;
     if ((groups <= 2 && hd != 128) || launch * groups <= 512) return groups;
     if (hd == 512) return groups % 4 ? groups : groups / 4;
     if (hd == 256 && groups > 4 && launch > 128 && launch <= 256 && rows >= 256) return 1;
@@ -1886,16 +1891,20 @@ static int parts_head_split(int64_t launch, int64_t rows, int groups, int hd)
 }
 
 // ... and the waves of its workgroups: four of one head, eight where several heads leave at most 256 workgroups (two of
-// eight waves and several heads do not share a compute unit).  With more than 256 workgroups of one head, long partitions
+// eight waves and several heads do not share a compute unit).  With more than 256 workgroups of one head of 256, long partitions
 // keep the units busy to the end only with eight (32 heads over 8 kv heads, 16 partitions of 65536 rows: 152.6 us with
 // four, 129.6 with eight; of 4096 rows 14.0 and 13.3; a call that attends 200 rows of them: 4.6 and 6.1).  With at most 256, one to
-// a compute unit, eight from 512 rows a partition: a wave by itself has an instruction in flight only every eight cycles or so
-// (8 heads of 256 over one, 16 partitions, 512 | 2048 | 8192 rows attended 4.2 | 6.5 | 16.7 with four, 4.7 | 6.0 | 13.1 with eight).
+// a compute unit, eight would be the shorter ones for a call that attends a thousand rows and more and the longer ones below, whatever the
+// cache's length, which is all that is known here (8 heads of 256 over one, 16 partitions, 1 | 512 | 1000 | 2000 | 8000 rows attended
+// 3.3 | 3.8 | 4.8 | 6.6 | 17.6 with four, 3.85 | 4.4 | 4.6 | 5.75 | 12.9 with eight): heads of 256 take four, as every short conversation
+// wants it, and a schedule asks for eight (sched.nsg).  Heads of 128, which had eight with all heads in one workgroup, keep them from
+// 512 rows a partition on (8 over 4, 16 partitions, 1 | 2000 | 16384 rows 4.65 | 6.1 | 19.9 so, 4.2 | 4.9 | 12.8 with one head each).
 static int parts_waves(int64_t workgroups, int64_t rows, int heads, int hd)
 {
     if (hd == 512) return 8;
-    if (heads == 1) return workgroups <= 256 ? (rows >= 512 ? 8 : 4) : workgroups <= 512 && rows >= 1024 ? 8 : 4;
-    return workgroups <= 256 && rows >= 64 ? 8 : 4;
+    if (heads > 1) return workgroups <= 256 && rows >= 64 ? 8 : 4;
+    if (hd == 128) return workgroups <= 256 && rows >= 512 ? 8 : 4;
+    return workgroups > 256 && workgroups <= 512 && rows >= 1024 ? 8 : 4;
 }
 
 // KSH_SDPA_SLOTS with everything left open: partitions a slot (up to `most`, what the general rule gives: 512 workgroups, 64 rows

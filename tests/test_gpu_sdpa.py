@@ -221,6 +221,26 @@ def test_sdpa_slots_left_open(ctx, eng, n_q, n_kv, hd, max_t, n_slots, name):
         assert_close(got[s], oracle.sdpa(q[s], k[s], v[s], n_q, n_kv, hd, lens[s], 0, 0.0625, f64=True), TOL, f"slot {s} len {lens[s]}")
 
 
+@pytest.mark.parametrize("n_q,n_kv,hd,max_t,nwg,split,waves", [
+    (8, 1, 256, 8192, 16, 8, 4), (4, 1, 256, 8192, 16, 4, 4), (8, 2, 256, 16384, 32, 4, 4), (8, 1, 256, 4096, 16, 8, 4), (8, 1, 256, 34000, 33, 8, 8),
+    (8, 4, 128, 65536, 64, 1, 8), (32, 8, 128, 16384, 16, 1, 8), (32, 8, 128, 16383, 16, 4, 4), (16, 2, 128, 32768, 32, 8, 4),
+    (16, 2, 128, 8192, 16, 8, 8), (8, 4, 128, 8192, 16, 2, 8), (4, 4, 128, 8192, 16, 1, 8), (4, 4, 128, 66000, 65, 1, 4)])
+def test_split_kv_partials_by_cache_length(ctx, n_q, n_kv, hd, max_t, nwg, split, waves):
+    """How partials over long caches are split where the caller leaves it open: heads of 256 in four waves however long the cache is,
+    unless there are more workgroups than compute units.  Merged, a few rows of the cache attended and all of it, against the oracle."""
+    kk, vv = (synth.q40_blocks(max_t * n_kv * hd // 32, seed=21 + i) for i in (0, 1))
+    q = synth.normal_f32(n_q * hd, 23)
+    k = ctx.compile(hip.make_desc(hip.Kind.SDPA_MWG_PART, (n_q, n_kv, hd, max_t, nwg), (DType.Q40, DType.F32), (0.0625,)))
+    assert (int(k.info.sched.unroll), int(k.info.sched.nsg)) == (split, waves), k.name
+    red = ctx.compile(hip.make_desc(hip.Kind.SDPA_MWG_REDUCE, (n_q, hd, nwg)))
+    bq, bk, bv = ctx.buffer_f32(q), ctx.buffer_bytes(kk), ctx.buffer_bytes(vv)
+    tmp, o = ctx.buffer_empty_f32(n_q * nwg * (hd + 2)), ctx.buffer_empty_f32(n_q * hd)
+    for tlen, start in ((max_t, 0), (300, 7)):
+        ctx.encode_multi(k, [bq, bk, bv, ctx.buffer_f32(np.array([tlen, start, 0, 0], np.float32))], [tmp])
+        ctx.encode_multi(red, [tmp], [o])
+        assert_close(ctx.read_f32(o, n_q * hd), oracle.sdpa(q, kk, vv, n_q, n_kv, hd, tlen, start, 0.0625, f64=True), TOL, f"{tlen} rows")
+
+
 def test_sdpa_errors(ctx):
     with pytest.raises(hip.KshError, match="multiple of 32"):
         ctx.compile(hip.make_desc(hip.Kind.SDPA_NAIVE, (8, 1, 100, 64), (DType.Q40, DType.F32), (1.0,)))
