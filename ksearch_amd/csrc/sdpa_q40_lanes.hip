@@ -1918,7 +1918,13 @@ static int parts_waves(int64_t workgroups, int64_t rows, int heads, int hd)
 //   29.6, 16 of 16384 85.7 | 78.
 // - heads of 128: several slots four waves (the rule's eight for 256 rows and more leave one workgroup a compute unit: 8 heads
 //   over 4, 16 slots of 4000 22.1 | 17.8, 4 of 16384 22.8 | 18.4; 32 over 8, 8 of 16384 54.9 | 50.7).  A single slot's records are
-//   folded by its last workgroup, which wants few: 32 over 8, 4000 rows 16.6 with 63 partitions | 9.9 with 16.
+//   folded by its last workgroup, which wants few, and rows want many workgroups, up to one a compute unit: 16 partitions while a call
+//   that attends the whole cache is no longer for it, 32 beyond, and past 32 partitions of 468 rows, with up to four kv heads, the rule's 64.
+//   A tenth | half | all of the rows attended: 8 heads over 4, 4000 rows 11.0 | 11.5 | 11.8 by the rule, with 16 7.8 | 8.8 | 10.8; 8192
+//   rows 11.2 | 11.9 | 13.3, with 16 7.9 | 10.8 | 14.7, with 32 9.0 | 10.0 | 12.0; 14000 rows 11.5 | 13.1 | 15.7, with 32 9.1 | 11.6 |
+//   15.2; 16384 rows 11.2 | 12.5 | 14.6, with 32 9.1 | 12.1 | 16.0; 16 over 2, 8192 rows 16.8 | 18.0 | 20.0, with 16 11.5 | 16.5 | 23.2,
+//   with 32 12.4 | 14.5 | 17.9; 32 over 8, 4000 rows 15.0 | 16.3 | 16.8, with 16 8.8 | 10.1 | 12.0, 8192 19.8 | 21.2 | 22.6, with 16 9.0 |
+//   12.1 | 15.9, with 32 11.0 | 12.2 | 14.2.
 SlotsPlan slots_plan(int n_q, int n_kv, int hd, int64_t max_t, int64_t n_slots, int most)
 {
     SlotsPlan s;
@@ -1941,7 +1947,7 @@ SlotsPlan slots_plan(int n_q, int n_kv, int hd, int64_t max_t, int64_t n_slots, 
     } else if (n_slots > 1) {
         s = {parts(most), 4, 1};
     } else {
-        const int n = parts(std::max<int64_t>(16, max_t / 512));
+        const int n = parts(max_t < 4500 ? 16 : max_t >= 15000 && n_kv <= 4 ? most : std::max<int64_t>(32, max_t / 512));
         s = {n, max_t / n >= 100 ? 8 : 4, 1};
     }
     return s;

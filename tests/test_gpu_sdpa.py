@@ -221,6 +221,21 @@ def test_sdpa_slots_left_open(ctx, eng, n_q, n_kv, hd, max_t, n_slots, name):
         assert_close(got[s], oracle.sdpa(q[s], k[s], v[s], n_q, n_kv, hd, lens[s], 0, 0.0625, f64=True), TOL, f"slot {s} len {lens[s]}")
 
 
+@pytest.mark.parametrize("n_q,n_kv,max_t,parts", [(8, 4, 1023, 16), (8, 4, 4499, 16), (8, 4, 4500, 32), (16, 2, 8192, 32), (4, 1, 14999, 32),
+                                                  (8, 4, 15000, 64), (32, 8, 4499, 16), (32, 8, 8192, 32), (32, 8, 16384, 32), (32, 8, 20000, 39)])
+def test_sdpa_slots_one_slot_of_heads_of_128(ctx, eng, n_q, n_kv, max_t, parts):
+    """Partitions of a single slot left open, either side of the lines; all rows of the cache, and one, against float64."""
+    hd = 128
+    kk = ctx.compile(hip.make_desc(hip.Kind.SDPA_SLOTS, (n_q, n_kv, hd, max_t, 1, 0), (DType.Q40, DType.F32), (0.0625,)))
+    assert int(kk.info.sched.k_split) == parts, kk.name
+    k, v = kv(max_t, n_kv, hd, 31)
+    q = synth.normal_f32(n_q * hd, 33)
+    tmp, out = ctx.buffer_empty_f32(n_q * parts * (hd + 2)), ctx.buffer_empty_f32(n_q * hd)
+    for n in (max_t, 1):
+        eng.sdpa_slots(ctx, n_q, n_kv, hd, max_t, 1, ctx.buffer_f32(q), ctx.buffer_bytes(k), ctx.buffer_bytes(v), ctx.buffer_f32([n, 0, 0, 0]), tmp, out, 0.0625)
+        assert_close(ctx.read_f32(out, n_q * hd), oracle.sdpa(q, k, v, n_q, n_kv, hd, n, 0, 0.0625, f64=True), TOL, f"{n} rows")
+
+
 @pytest.mark.parametrize("n_q,n_kv,hd,max_t,nwg,split,waves", [
     (8, 1, 256, 8192, 16, 8, 4), (4, 1, 256, 8192, 16, 4, 4), (8, 2, 256, 16384, 32, 4, 4), (8, 1, 256, 4096, 16, 8, 4), (8, 1, 256, 34000, 33, 8, 8),
     (8, 4, 128, 65536, 64, 1, 8), (32, 8, 128, 16384, 16, 1, 8), (32, 8, 128, 16383, 16, 4, 4), (16, 2, 128, 32768, 32, 8, 4),
