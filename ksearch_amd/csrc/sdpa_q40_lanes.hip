@@ -209,7 +209,8 @@ __device__ __forceinline__ void unpack8(uint32_t d, float (&n)[8])
 
 // NR row steps: scores, one online-softmax update, P.V.  ALL: every step has rows.  With one or two heads a step is one chain of some 60
 // dependent instructions, and the branch around each kept the four chains of an update one behind the other; without it they
-// run side by side (8 heads of 256, 4000 rows, 16 partitions of four waves 10.3 -> 9.75 us).  The sums are the same.
+// run side by side (8 heads of 256, 4000 rows, 16 partitions of four waves 10.3 -> 9.75 us).  The sums are the same.  (Split-KV
+// partials of heads of 512 take their steps one by one: 64 partitions, 1000 | 2000 rows attended 5.7 | 6.1 us, with this beside 6.1 | 6.25.)
 template <int HD, int GP, int NR, bool ALL = false>
 __device__ __forceinline__ void process_rows(const RowRegs (&r)[NR], const bool (&valid)[NR], const bool (&live)[NR],
                                              const float (&qv)[GP][8], const float (&Sq)[GP], State<GP> &st, int c)
@@ -777,7 +778,7 @@ __global__ __launch_bounds__(NW * 64) void sdpa_lanes_kernel(LaneParams p_in)
                 live[t] = base + (t * NW + wave) * RPS < p1;
                 nxt[t] = load_row(min(row + TILE, p1 - 1));   // unconditional: keeps the wait counts exact
             }
-            if (GP <= 2 && live[kRT - 1]) process_rows<HD, GP, kRT, true>(cur, valid, live, qv, Sq, st, c);
+            if (GP <= 2 && HD < 512 && live[kRT - 1]) process_rows<HD, GP, kRT, true>(cur, valid, live, qv, Sq, st, c);
             else process_rows<HD, GP, kRT>(cur, valid, live, qv, Sq, st, c);
 #pragma unroll
             for (int t = 0; t < kRT; t++) cur[t] = nxt[t];
