@@ -61,7 +61,7 @@ int launch_q4k(const Q4kGeom &G, const MatvecParams &p, int total_waves, hipStre
 // where that still leaves ~150 workgroups, else fewer rows, else smaller
 // workgroups; int8 dot, except for rows longer than one 16-superblock step,
 // where the f32 form is the faster one.
-Q4kGeom pick_geom(const ksh_sched &s, int total_rows, int bpr)
+Q4kGeom pick_geom(const ksh_sched &s, int n_mat, int total_rows, int bpr)
 {
     Q4kGeom G;
     G.half = (bpr == 8 || bpr == 6);
@@ -79,11 +79,16 @@ Q4kGeom pick_geom(const ksh_sched &s, int total_rows, int bpr)
         return G;
     }
     // rows of more than one sweep: a wave's registers hold one of them and what follows it, and two in turn leave the last workgroups
-    // alone (r = 2 -> 1: 6000 x 8192 10.5 -> 8.8 us, 9000 x 5120 14.4 -> 11.6, 16384 x 8192 20.8 -> 19.2, gate | up 8192 x 5120, whose two
-    // rows of two matrices do not fit the registers, 178 -> 18.6)
+    // alone (r = 2 -> 1, the median of three in turn: 6000 x 4352 10.7 -> 8.6 us, x 8192 10.9 -> 9.8, 16384 x 5120 20.5 -> 18.8, q | k | v of
+    // 4096 + 2 x 1024 x 8192 11.7 -> 9.7, gate | up 8192 x 5120, whose two rows of two matrices do not fit the registers, 182 -> 21).  One
+    // matrix of 7680 columns and more is a little faster in two rows a wave where their workgroups are a turn over the compute units
+    // or fill the last one (r = 1 against 2: 1.01 to 1.06 at 2304 to 4096 rows of 7680 to 15360 columns, 1.02 to 1.035 at 8192, 12288,
+    // 16384 and 24576 x 8192).
+    const int64_t two = (total_rows + 15) / 16;
+    const bool pairs = n_mat == 1 && bpr >= 30 && (two <= 256 || full_turns(two));
     for (int nw : {8, 4})
         for (int r : {2, 1}) {
-            if (sched_is_zero(s) && bpr > 16 && r == 2) continue;
+            if (sched_is_zero(s) && bpr > 16 && r == 2 && !pairs) continue;
             if (s.nsg && (int)s.nsg != nw) continue;
             if (s.nr0 && (int)s.nr0 != r) continue;
             G.NW = nw;
@@ -229,7 +234,7 @@ int bind_matvec_q4k_family(ksh_kernel &k)
                        sched.unroll == (uint32_t)f.NBUF && sched.vec == kXI8;
     if (named) sched = ksh_sched{};
     const int64_t sized_by = s.nm == 2 ? s.rows[0] : total_rows;
-    Q4kGeom G = pick_geom(sched, (int)sized_by, bpr);
+    Q4kGeom G = pick_geom(sched, s.n_mat, (int)sized_by, bpr);
     const int64_t half_wgs = (sized_by + G.rpw() * G.NW - 1) / (G.rpw() * G.NW);
     G.stream = named || (sched_is_zero(sched) && s.prologue != kMergeParts && q4s_pays(s.n_mat, sized_by, bpr, half_wgs, G.NW));
     // QKV at one row per half-wave: one dot per lane does not pay for turning the vector into digit planes (3.86 vs 4.08 us)

@@ -327,6 +327,21 @@ def test_gate_up_form_follows_the_other_forms_turns(ctx, cols, rows, streams):
     assert np.all(got[rows:] == 7.0)
 
 
+@pytest.mark.parametrize("rows,cols,two", [(2303, 8192, False), (2304, 8192, True), (4096, 8192, True), (4097, 8192, False), (6000, 8192, False), (7776, 8192, False),
+                                           (7777, 8192, True), (8192, 8192, True), (8193, 8192, False), (2400, 7424, False), (2400, 7680, True), (4096, 4352, False),
+                                           (3000, 12288, True), (12288, 12288, True)])
+def test_matvec_q4k_long_rows_by_turns(ctx, eng, rows, cols, two):
+    """Rows of more than one sweep left open, either side of the lines between one and two rows a wave (f32 sums: 1e-5 of float64)."""
+    k = ctx.compile(hip.make_desc(hip.Kind.MATVEC, (rows, cols), (DType.Q4K, DType.F32)))
+    assert ("_r2_" in k.name) == two, k.name
+    w, x = synth.q4k_blocks(rows * cols // 256, seed=rows), synth.normal_f32(cols, seed=cols)
+    by = ctx.buffer_f32(np.full(rows + 64, 7.0, np.float32))
+    ctx.encode_multi(k, [ctx.buffer_bytes(w), ctx.buffer_f32(x)], [by])
+    got = ctx.read_f32(by, rows + 64)
+    assert_close(got[:rows], oracle.matvec_f64(oracle.Q4K, w, rows, cols, x), 1e-5, k.name)
+    assert np.all(got[rows:] == 7.0)
+
+
 def test_lm_head_cfg1_full_size_with_argmax(ctx, eng):
     rows, cols = 262144, 2048
     w, x = synth.cfg1_q6k_lm_head()
