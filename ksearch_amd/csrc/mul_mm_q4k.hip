@@ -498,10 +498,18 @@ float mm_skinny_us(int64_t rows, int nsb, int64_t batch)
 struct FewPlan {
     int rh, tokens;
     float us;
+    int64_t wgs;
 };
-// Whether a call that leaves the schedule open, and a search, may take it.  (Q4_K beyond 192 tokens, left open, stays the tile, whose handles
-// report its K slices; 300 rows of 1536 columns, 200 tokens: 11 us, 4 by schedule)
-bool mm_few_open(bool q6, int64_t batch) { return batch <= (q6 ? kFewMost : 192); }
+// Whether a call that leaves the schedule open may take it: where the estimate holds (of 405 further shapes inside the fit's range at which it is
+// taken the others are the shorter ones at 4, by 21 % at most).  Not rows of more than 8192 columns, where a wave has five superblocks and more one behind
+// the other (19 x 24576, 5 tokens 11.5 us and 15.2 so, 64 x 16384, 1000 tokens 16.8 and 24.8); more than 256 tokens of more than 4096
+// columns (128 x 8192, 1000 tokens 15.9 and 28.3, 512 13.0 and 14.2); Q4_K of 256 columns in more workgroups than compute units (65536 rows, 1
+// token 12.0 and 15.0, 14412, 21 tokens 6.7 and 8.6, 2048, 192 tokens 7.4 and 8.2).  Q4_K beyond 192 tokens, left open, stays the
+// tile, whose handles report its K slices (300 rows of 1536 columns, 200 tokens: 11 us, 4 in this form).
+bool mm_few_open(bool q6, int nsb, int64_t batch, const FewPlan &few)
+{
+    return nsb <= 32 && batch <= (q6 ? kFewMost : 192) && (nsb <= 16 || batch <= 256) && (q6 || nsb > 1 || few.wgs <= 256);
+}
 FewPlan mm_few_plan(bool q6, int64_t rows, int nsb, int64_t batch)
 {
     struct Cost {
@@ -509,7 +517,7 @@ FewPlan mm_few_plan(bool q6, int64_t rows, int nsb, int64_t batch)
     };
     constexpr Cost kCost[2][2] = {{{1.848f, 1.301f, 0.118f, 0.016f, -0.388f, 0.909f, 0.03f}, {1.495f, 0.944f, 0.583f, 0.362f, 0.f, 0.299f, 0.038f}},
                                   {{1.639f, 1.406f, 0.098f, 0.106f, -0.536f, 1.522f, 0.029f}, {1.302f, 0.114f, 0.254f, 1.71f, 0.f, 1.198f, 0.032f}}};
-    FewPlan best{1, 1, 1e30f};
+    FewPlan best{1, 1, 1e30f, 0};
     const float turns = (float)((nsb + 7) / 8), each = (float)nsb / 8.f;
     for (int most : {32, 16})
         for (int rh : {1, 2, 4}) {
@@ -517,10 +525,10 @@ FewPlan mm_few_plan(bool q6, int64_t rows, int nsb, int64_t batch)
             const int tokens = (int)((batch + groups - 1) / groups);
             if (!few_fits(q6, tokens, rh)) break;
             const Cost &c = kCost[q6][tokens > 16];
-            const int64_t load = ((rows + 16 * rh - 1) / (16 * rh) * groups + 255) / 256, fit = 163840 / few_lds(q6, tokens, rh);
+            const int64_t wgs = (rows + 16 * rh - 1) / (16 * rh) * groups, load = (wgs + 255) / 256, fit = 163840 / few_lds(q6, tokens, rh);
             const float us = c.launch + (float)((load + fit - 1) / fit) * (c.round + c.turn * turns) +
                              (float)load * (c.each + each * (c.tile + c.rows16 * (float)rh + c.token * (float)tokens));
-            if (us < best.us) best = FewPlan{rh, tokens, us};
+            if (us < best.us) best = FewPlan{rh, tokens, us, wgs};
         }
     return best;
 }
@@ -1951,7 +1959,7 @@ int bind_matvec_batch(ksh_kernel &k)
         const int nsb = (int)(cols / 256);
         const FewPlan few = mm_few_plan(q6, rows, nsb, batch);
         const float tiles = mm_plan_bf16(q6, mm_row_tiles(k.desc), nsb, batch, rows_all, 0).us;
-        if (want == 16 || (mm_few_open(q6, batch) && 1.04f * few.us < (q6 || batch > kSkinnyMaxBatch ? tiles : std::min(mm_skinny_us(rows, nsb, batch), tiles)))) {
+        if (want == 16 || (mm_few_open(q6, nsb, batch, few) && 1.04f * few.us < (q6 || batch > kSkinnyMaxBatch ? tiles : std::min(mm_skinny_us(rows, nsb, batch), tiles)))) {
             // (as a schedule names them, where they are a launch)
             const int u = (int)k.desc.sched.unroll, l = (int)std::min<uint32_t>(k.desc.sched.lds_tile, kFewTokens + 1);
             const int tokens = want == 16 && l >= 1 && l <= kFewTokens ? (int)std::min<int64_t>(l, batch) : few.tokens;
@@ -2126,8 +2134,8 @@ int bind_matvec_round(ksh_kernel &k)
 }
 
 // Schedules of the prefill GEMM beside the library's own, which a search times first, as the bound kernels report them: whole
-// rows, for bf16 tokens the form of one launch where an open call may take it, for Q4_K weights and up to 64 tokens 32 weight rows per
-// workgroup with the K range split over its 8 waves, and K slices where half as many leave the chip short of workgroups.  (The shape of a workgroup follows from the sizes, for bf16 rows from the
+// rows, for bf16 tokens the form of one launch (Q4_K: up to 192 tokens), for Q4_K weights and up to 64 tokens 32
+// weight rows per workgroup with the K range split over its 8 waves, and K slices where half as many leave the chip short of workgroups.  (The shape of a workgroup follows from the sizes, for bf16 rows from the
 // slice count too; counts that do not divide a row come from the library's own schedule only.)
 int mul_mm_candidates(const ksh_kernel_desc &d, ksh_sched *out, int cap)
 {
@@ -2154,10 +2162,12 @@ int mul_mm_candidates(const ksh_kernel_desc &d, ksh_sched *out, int cap)
         wgs = (int64_t)g.x * g.y;
         full = tall ? 256 : 512;
     }
-    if (!f32x && mm_few_open(q6, d.dims[2]) && !d.dims[3] && !d.dims[6]) {
-        const int tokens = mm_few_plan(q6, d.dims[0], nsb, d.dims[2]).tokens;
+    if (!f32x && d.dims[2] <= kFewMost && !d.dims[3] && !d.dims[6]) {
+        const FewPlan few = mm_few_plan(q6, d.dims[0], nsb, d.dims[2]);
+        const int tokens = few.tokens;
+        const bool timed = d.dims[2] <= (q6 ? kFewMost : 192);
         for (uint32_t rh : {1u, 2u, 4u}) {
-            if (n >= cap || !few_fits(q6, tokens, (int)rh)) break;
+            if (!timed || n >= cap || !few_fits(q6, tokens, (int)rh)) break;
             ksh_sched s{};
             s.tg = 512; s.nsg = 8; s.nr0 = 16; s.lds_tile = (uint32_t)tokens; s.unroll = rh; s.vec = 0; s.k_split = 8;
             out[n++] = s;

@@ -419,6 +419,24 @@ def test_mul_mm_few_tokens_refused(ctx, dims, xdt):
         ctx.compile(hip.make_desc(hip.Kind.MATVEC_BATCH, dims, (DType.Q4K, xdt, DType.F32), (), dict(nr0=16)))
 
 
+@pytest.mark.parametrize("wdt,rows,cols,batch,few", [
+    (DType.Q4K, 19, 24576, 5, False), (DType.Q6K, 64, 16384, 1000, False), (DType.Q4K, 300, 8448, 3, False), (DType.Q4K, 300, 8192, 3, True),
+    (DType.Q6K, 128, 8192, 512, False), (DType.Q6K, 128, 8192, 256, True), (DType.Q6K, 128, 4096, 512, True), (DType.Q4K, 65536, 256, 1, False),
+    (DType.Q4K, 14412, 256, 21, False), (DType.Q4K, 12300, 256, 9, True), (DType.Q6K, 10728, 256, 2, True)])
+def test_mul_mm_few_tokens_left_open(ctx, wdt, rows, cols, batch, few):
+    """Where an open call takes the form of one launch: not outside the sizes that its estimate holds for.  Either form against float64."""
+    k = ctx.compile(hip.make_desc(hip.Kind.MATVEC_BATCH, (rows, cols, batch), (wdt, DType.BF16, DType.F32)))
+    assert ("few" in k.name) == few, k.name
+    w = (synth.q4k_blocks if wdt == DType.Q4K else synth.q6k_blocks)(rows * cols // 256, 743)
+    x, raw = synth.bf16_round(synth.normal_f32(batch * cols, 744))
+    y = ctx.buffer_empty_f32(batch * rows)
+    ctx.encode_multi(k, [ctx.buffer_bytes(w), ctx.buffer_bytes(raw)], [y])
+    got = ctx.read_f32(y, batch * rows).reshape(batch, rows)
+    for t in sorted({0, batch // 2, batch - 1}):
+        want = oracle.matvec_f64(oracle.Q4K if wdt == DType.Q4K else oracle.Q6K, w, rows, cols, x.reshape(batch, cols)[t])
+        assert np.abs(got[t] - want).max() <= (2e-5 if wdt == DType.Q4K or few else 1e-3) * max(np.abs(want).max(), np.abs(x.reshape(batch, cols)[t]).max()), t
+
+
 @pytest.mark.parametrize("wdt,off", [(DType.Q4K, 0), (DType.Q6K, 0), (DType.Q6K, 14), (DType.Q6K, 6)])
 @pytest.mark.parametrize("rows,batch,cols,rh", [(1, 1, 256, 1), (15, 2, 1792, 1), (17, 15, 2048, 2), (33, 16, 2304, 4), (65, 17, 4096, 1), (129, 31, 768, 1), (200, 32, 6400, 1),
                                                 (63, 3, 8192, 4), (5000, 16, 512, 2), (12300, 9, 256, 4), (3000, 32, 2048, 0), (1000, 7, 2048, 0),
