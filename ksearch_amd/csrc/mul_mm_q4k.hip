@@ -2134,7 +2134,7 @@ int bind_matvec_round(ksh_kernel &k)
 }
 
 // Schedules of the prefill GEMM beside the library's own, which a search times first, as the bound kernels report them: whole
-// rows, for bf16 tokens the form of one launch (Q4_K: up to 192 tokens), for Q4_K weights and up to 64 tokens 32
+// rows, for bf16 tokens the form of one launch (Q4_K beyond 192 tokens: where it is estimated the shorter), for Q4_K weights and up to 64 tokens 32
 // weight rows per workgroup with the K range split over its 8 waves, and K slices where half as many leave the chip short of workgroups.  (The shape of a workgroup follows from the sizes, for bf16 rows from the
 // slice count too; counts that do not divide a row come from the library's own schedule only.)
 int mul_mm_candidates(const ksh_kernel_desc &d, ksh_sched *out, int cap)
@@ -2165,7 +2165,7 @@ int mul_mm_candidates(const ksh_kernel_desc &d, ksh_sched *out, int cap)
     if (!f32x && d.dims[2] <= kFewMost && !d.dims[3] && !d.dims[6]) {
         const FewPlan few = mm_few_plan(q6, d.dims[0], nsb, d.dims[2]);
         const int tokens = few.tokens;
-        const bool timed = d.dims[2] <= (q6 ? kFewMost : 192);
+        const bool timed = d.dims[2] <= (q6 ? kFewMost : 192) || few.us < mm_plan_bf16(q6, row_tiles, nsb, d.dims[2], d.dims[0], 0).us;
         for (uint32_t rh : {1u, 2u, 4u}) {
             if (!timed || n >= cap || !few_fits(q6, tokens, (int)rh)) break;
             ksh_sched s{};

@@ -184,6 +184,15 @@ def test_q6k_candidates_have_the_streaming_form(kind, cols, stream):
     assert c[0] == stream and len(c) == len(set(c)) == 19
 
 
+@pytest.mark.parametrize("wdt,rows,cols,batch,offered", [
+    (hip.DType.Q4K, 300, 1536, 192, True), (hip.DType.Q4K, 300, 1536, 200, True), (hip.DType.Q4K, 280, 1024, 1000, True), (hip.DType.Q4K, 280, 1024, 1025, False),
+    (hip.DType.Q4K, 8192, 2048, 200, False), (hip.DType.Q6K, 300, 1536, 1024, True), (hip.DType.Q6K, 19, 24576, 5, True)])
+def test_prompt_gemm_candidates_of_one_launch(wdt, rows, cols, batch, offered):
+    """The search times the GEMM of one launch beyond the tokens up to which an open call takes it, wherever it is estimated the shorter."""
+    c = hip.beam_candidates(hip.make_desc(hip.Kind.MATVEC_BATCH, (rows, cols, batch), (wdt, hip.DType.BF16, hip.DType.F32)))
+    assert any(s.nr0 == 16 for s in c) == offered
+
+
 def test_kernel_lookup_takes_any_sequence():
     """Eng._k with lists, arrays and tuples of the same numbers finds one handle."""
     import numpy as np
