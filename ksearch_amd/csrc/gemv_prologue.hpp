@@ -343,14 +343,18 @@ __device__ __forceinline__ void stage_finish(const Prologue &pr_in, uint8_t *lds
     }
     {
         const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+        // (of 16 waves some have no share of a short vector: zeros to add, nothing to do behind the barrier, and a SIMD's
+        // other waves waiting for what they would issue)
+        const bool share = NT < 1024 || wbase < n4;
 #pragma unroll
         for (int j = 0; j < 4; j++) {
             if (j == 0 || add) {
-                const float wsum = wave_sum(acc[j]);
+                const float wsum = share ? wave_sum(acc[j]) : 0.f;
                 if (lane == 0) red[wave * 4 + j] = wsum;
             }
         }
         __syncthreads();   // `red` has no earlier use in the kernel, so one barrier is enough
+        if (!share) return;
 #pragma unroll
         for (int j = 0; j < 4; j++) {
             acc[j] = 0.f;

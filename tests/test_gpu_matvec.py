@@ -453,10 +453,10 @@ def test_rmsnorm_matvec_q6k_lm_head_prologue(ctx, eng, has_res):
             assert_close(ctx.read_f32(xn, n), x_new, 1e-5, "x_new")
 
 
-@pytest.mark.parametrize("cols", [2304, 4096, 4352, 6144, 8192])
+@pytest.mark.parametrize("cols", [256, 1280, 2048, 2304, 4096, 4352, 6144, 8192])
 @pytest.mark.parametrize("has_res", [False, True])
-def test_rmsnorm_matvec_q6k_long_rows(ctx, cols, has_res, tmp_path, monkeypatch):
-    """The norm in front of file-order Q6_K over every length that the streaming kernel takes: left open, by the schedule that its
+def test_rmsnorm_matvec_q6k_row_lengths(ctx, cols, has_res, tmp_path, monkeypatch):
+    """The norm in front of file-order Q6_K, rows of which one wave to all sixteen have a share and the longest: left open, by the schedule that its
     handle reports, by the schedules of the regrouped rows' kernel and through a search, whose one candidate binds."""
     monkeypatch.setenv("KSEARCH_BEAM_CACHE", str(tmp_path / "beam"))
     rows, eps = 301, 1e-6
