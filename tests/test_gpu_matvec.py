@@ -168,9 +168,11 @@ SCHEDS_Q6K = [None, dict(tg=256, vec=0, unroll=2, nsg=4, nr0=1, k_split=1, lds_t
 @pytest.mark.parametrize("rows,cols", [(8, 2048), (1000, 2048), (4099, 2048), (300, 4096), (70, 256), (33, 512), (65, 1536), (40, 8192)])
 @pytest.mark.parametrize("sched", SCHEDS_Q6K)
 def test_matvec_q6k(ctx, eng, rows, cols, sched):
+    # (file order has one kernel a row length, which these schedules of the regrouped rows' kernel stand for too)
     w = synth.q6k_blocks(rows * cols // 256, seed=rows)
     x = synth.normal_f32(cols, seed=11)
     bw, bx, by = ctx.buffer_bytes(w), ctx.buffer_f32(x), ctx.buffer_empty_f32(rows)
+    assert "q6k_stream" in ctx.compile(hip.make_desc(hip.Kind.MATVEC, (rows, cols), (DType.Q6K, DType.F32), sched=sched)).name
     eng.matvec_wd(ctx, rows, cols, DType.Q6K, bw, bx, by, sched)
     assert_close(ctx.read_f32(by, rows), oracle.matvec(oracle.Q6K, w, rows, cols, x), TOL, f"q6k {rows}x{cols} {sched}")
 
@@ -304,6 +306,37 @@ def test_matvec_q4k_stream_edges(ctx, bpr, rows, kv_rows):
             got = ctx.read_f32(o, len(v) + 64)
             assert np.abs(got[:len(v)] - v).max() <= m, (kind, np.abs(got[:len(v)] - v).max(), m)
             assert np.all(got[len(v):] == 7.0)
+
+
+@pytest.mark.parametrize("kind,dtype,cols", [(hip.Kind.MATVEC, DType.Q4K, 256 * b) for b in (1, 2, 3, 4, 5, 7, 10, 14, 15)]
+                         + [(hip.Kind.MATVEC_GATE_UP_GELU, DType.Q4K, 256 * b) for b in (1, 2, 3, 4, 6, 8, 13, 16)]
+                         + [(hip.Kind.MATVEC, DType.Q6K, 256 * b) for b in (1, 2, 3, 4, 5, 7, 8, 9, 13, 17, 25, 32)]
+                         + [(hip.Kind.MATVEC, DType.Q6K_ROWS, c) for c in (1536, 2048, 4096)])
+def test_streamed_rows_keep_their_infinities_to_themselves(ctx, kind, dtype, cols):
+    """Streamed rows share a sweep, the step of their last superblocks and the registers of their results: a row whose scales are infinite
+    or no number (the first, some between, the last) is not finite, and every other has the bits that it has without it."""
+    rows, pair = 45, kind == hip.Kind.MATVEC_GATE_UP_GELU
+    size, at = (144, 0) if dtype == DType.Q4K else (210, 208)
+    bad = {0: 0x7E00, 7: 0x7C00, 8: 0x7E00, 21: 0xFC00, rows - 1: 0x7E00}
+    ws = [(synth.q4k_blocks if dtype == DType.Q4K else synth.q6k_blocks)(rows * cols // 256, seed=cols + i) for i in range(2 if pair else 1)]
+    hurt = [w.copy() for w in ws]
+    for j, (r, bits) in enumerate(bad.items()):
+        # (a gate is clamped in front of its GELU: a row is as finite as its up)
+        for w in hurt[(j % 2 if pair else 0):]:
+            w.reshape(rows, cols // 256, size)[r, (r * 5) % (cols // 256), at:at + 2] = np.array([bits], np.uint16).view(np.uint8)
+    x = synth.normal_f32(cols, seed=cols + 2)
+    big = ctx.compile(hip.make_desc(kind, (12000 if pair else 12300, cols), (dtype, DType.F32)))
+    k = ctx.compile(hip.make_desc(kind, (rows, cols), (dtype, DType.F32), sched=big.info.sched))
+    assert "stream" in k.name
+    got = []
+    for mats in (ws, hurt):
+        out = ctx.buffer_f32(np.zeros(rows, np.float32))
+        put = [ctx.buffer_bytes(q6k_rows(w, rows, cols) if dtype == DType.Q6K_ROWS else w) for w in mats]
+        ctx.encode_multi(k, put + [ctx.buffer_f32(x)], [out])
+        got.append(ctx.read_f32(out, rows))
+    others = [r for r in range(rows) if r not in bad]
+    assert np.all(np.isfinite(got[0])) and not np.any(np.isfinite(got[1][list(bad)]))
+    assert np.array_equal(got[0][others].view(np.uint32), got[1][others].view(np.uint32))
 
 
 @pytest.mark.parametrize("cols,rows,streams", [

@@ -419,6 +419,34 @@ def test_mul_mm_few_tokens_refused(ctx, dims, xdt):
         ctx.compile(hip.make_desc(hip.Kind.MATVEC_BATCH, dims, (DType.Q4K, xdt, DType.F32), (), dict(nr0=16)))
 
 
+@pytest.mark.parametrize("wdt", [DType.Q4K, DType.Q6K])
+@pytest.mark.parametrize("rows,batch,cols,rh", [(37, 5, 256, 1), (40, 16, 2304, 2), (70, 7, 1024, 4), (33, 29, 768, 1), (50, 75, 512, 1)])
+def test_mul_mm_few_tokens_keep_their_infinities(ctx, wdt, rows, batch, cols, rh):
+    """In the form of one launch a token with an infinity or no number is not finite, nor is a weight row with such a scale; every
+    other result has the bits that it has without them."""
+    size, at = (144, 0) if wdt == DType.Q4K else (210, 208)
+    w = (synth.q4k_blocks if wdt == DType.Q4K else synth.q6k_blocks)(rows * cols // 256, 747)
+    x, raw = synth.bf16_round(synth.normal_f32(batch * cols, 748))
+    hurt, hurt_x = w.copy(), np.asarray(raw).view(np.uint16).copy().reshape(batch, cols)
+    bad_rows, bad_tokens = {0: 0x7E00, 17: 0x7C00, rows - 1: 0xFC00}, {0: 0x7F80, batch // 2: 0x7FC0, batch - 1: 0xFF80}
+    for r, bits in bad_rows.items():
+        hurt.reshape(rows, cols // 256, size)[r, r % (cols // 256), at:at + 2] = np.array([bits], np.uint16).view(np.uint8)
+    for t, bits in bad_tokens.items():
+        hurt_x[t, (37 * t + 5) % cols] = bits
+    k = ctx.compile(hip.make_desc(hip.Kind.MATVEC_BATCH, (rows, cols, batch), (wdt, DType.BF16, DType.F32), (), dict(nr0=16, unroll=rh)))
+    assert "few" in k.name
+    got = []
+    for ww, xx in ((w, np.asarray(raw).view(np.uint16)), (hurt, hurt_x)):
+        y = ctx.buffer_f32(np.zeros(batch * rows, np.float32))
+        ctx.encode_multi(k, [ctx.buffer_bytes(ww), ctx.buffer_bytes(np.ascontiguousarray(xx).view(np.uint8))], [y])
+        got.append(ctx.read_f32(y, batch * rows).reshape(batch, rows))
+    touched = np.zeros((batch, rows), bool)
+    touched[list(bad_tokens)] = True
+    touched[:, list(bad_rows)] = True
+    assert np.all(np.isfinite(got[0])) and not np.any(np.isfinite(got[1][touched]))
+    assert np.array_equal(got[0][~touched].view(np.uint32), got[1][~touched].view(np.uint32))
+
+
 @pytest.mark.parametrize("wdt,rows,cols,batch,few", [
     (DType.Q4K, 19, 24576, 5, False), (DType.Q6K, 64, 16384, 1000, False), (DType.Q4K, 300, 8448, 3, False), (DType.Q4K, 300, 8192, 3, True),
     (DType.Q6K, 128, 8192, 512, False), (DType.Q6K, 128, 8192, 256, True), (DType.Q6K, 128, 4096, 512, True), (DType.Q4K, 65536, 256, 1, False),
