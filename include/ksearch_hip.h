@@ -61,7 +61,10 @@ enum ksh_dtype {
  * dtypes[2] = KSH_F16). */
 enum ksh_kind {
     /* Matvec{rows,cols,weight_dtype}: y = W x.  dims: rows, cols.
-     * dtypes[0] = Q4K | Q6K.  in: W, x   out: y[rows] */
+     * dtypes[0] = Q4K | Q6K | Q6K_ROWS.  in: W, x   out: y[rows]
+     * Q6K (file order, up to 8192 columns) has one kernel for a row length; info.name and info.sched name it.  A schedule of the
+     * kernel for Q6K_ROWS (nsg = 2 | 4 | 8 waves, nr0 = 1 | 2 | 4 rows, unroll: plans saved when file order had it too) is
+     * accepted and stands for that one kernel; any other is an error. */
     KSH_MATVEC = 1,
     /* MatvecBatch: Y[t,r] = sum_c W[r,c] X[t,c].  dims: rows, cols, batch.
      * dtypes[0] = Q4K | Q6K (GGUF byte order, blocks at 2-byte alignment),
@@ -90,9 +93,9 @@ enum ksh_kind {
      * F32 activations travel as hi + lo f16 parts.  The tile scales every row by its own power of two first (any
      * finite f32 row fits); the small-batch form does not: there |x| must stay below 65504.
      * sched.nr0 = 16 | 32 | 128 picks the form of one launch (bf16, one matrix, up to 1024 tokens; sched.unroll = 1, 2 or 4
-     * tiles of 16 weight rows and sched.lds_tile = up to 32 tokens to a workgroup), the small-batch form (Q4_K, up to 64 tokens, one matrix) or the tiles, whose tokens
-     * and rows follow from the sizes (info.name has them; sched.tg and sched.lds_tile name the kernel that reports
-     * them: 256 and 32 Q4_K, 256 and 64 or 512 and 64 Q6_K);
+     * tiles of 16 weight rows and sched.lds_tile = up to 32 tokens to a workgroup), the small-batch form (Q4_K, up to 64
+     * tokens, one matrix) or the tiles, whose tokens and rows follow from the sizes (info.name has them; sched.tg and
+     * sched.lds_tile name the kernel that reports them: 256 and 32 Q4_K, 256 and 64 or 512 and 64 Q6_K);
      * sched.k_split = the tile's K slices (a divisor of cols / 256, or for bf16 rows the count of a reported schedule;
      * 1 = whole rows; 0 = enough to fill the chip). */
     KSH_MATVEC_BATCH = 2,
@@ -285,8 +288,9 @@ typedef struct {
                         * planes, the activations to 2^-16 of their 32-element sub-block's largest magnitude.
                         * Attention: 1 = LDS-tile form, 3 = register (vector-ALU) form, 2 = matrix-core form of the
                         * row phase (heads of 256, up to 8 q heads per kv head.  KSH_SDPA_SLOTS with up to 16 slots:
-                        * the default there; lds_tile = 32 | 16 picks four waves with tiles of 32 rows or eight with
-                        * 16.  KSH_SDPA_BATCH: the default from 17 tokens on, every token's partitions workgroups of
+                        * the default there beyond some 5000 rows of caches times kv heads in all, 2000 of a single slot,
+                        * below which the register form is, and where entries name their pool slot; lds_tile = 32 | 16
+                        * picks four waves with tiles of 32 rows or eight with 16.  KSH_SDPA_BATCH: the default from 17 tokens on, every token's partitions workgroups of
                         * their own; vec = 2 with up to 64 tokens deals the partitions to the tokens by length) */
     uint32_t unroll;   /* superblocks in flight per lane */
     uint32_t nsg;      /* waves per workgroup */

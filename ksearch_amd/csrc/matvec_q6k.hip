@@ -204,7 +204,7 @@ __global__ __launch_bounds__(NW * 64) void q6r_gemv_kernel(Q6kParams p)
 
 // ---- Q6_K: blocks in file order (210 bytes, at 2-byte addresses) --------------
 // Streamed by way of LDS: a wave asks for G rows' bytes as whole 16-byte pieces at 16-byte addresses, NBUF such groups ahead,
-// and reads its lanes' fields from there.  What bounds it: the stream of the weights, 6.3 TB/s at 440 MB, which is what flat
+// and reads its lanes' fields from there.  What bounds it: the stream of the weights, 6.3 TB/s at 440 MB in a trace, which is what flat
 // 16-byte loads reach, with 85 vector instructions a step of eight superblocks (half of the stream's time) beside it.  Before,
 // lanes loaded their fields from memory: 80 cache lines touched a row instead of 14, a row of 1280 bytes or of 512 paid
 // for whole steps of eight superblocks, and the registers for a row's loads held rows of more than 4096 columns to one wave a

@@ -1940,8 +1940,8 @@ int bind_matvec_batch(ksh_kernel &k)
     k.scratch_bytes = (batch32 * cols * 2 + batch32 * (cols / 256) * 64) * (f32x ? 2 : 1);
     // schedule: nr0 = weight rows per workgroup.  32 = the small-batch form (Q4_K, up to 64 tokens: the default
     // there), 128 = the tiles (their tokens and rows follow from the sizes).
-    // 16: one launch of up to 32 bf16 tokens (sched.unroll: tiles of 16 weight rows a workgroup), the default where it is estimated
-    // the shortest.
+    // 16: one launch of bf16 tokens, up to 32 to a workgroup and kFewMost in all (sched.unroll: tiles of 16 weight rows a workgroup), the
+    // default where it is estimated the shortest (mm_few_open, mm_few_plan).
     const uint32_t want = k.desc.sched.nr0;
     if (want && want != 16 && want != 32 && want != BN) return set_error("matvec_batch: unsupported schedule nr0=%u (16, 32 or %d)", want, BN);
     const bool can_skinny = !q6 && batch <= kSkinnyMaxBatch && n_mat == 1 && !unfolded && !cut && !pair;

@@ -11,7 +11,7 @@
 // A workgroup is RH tiles of 16 weight rows and a group of the tokens; its eight waves deal a row's superblocks out and add their sums up through LDS
 // in their order.  Weights and tokens come as whole 16-byte pieces straight into LDS: from registers' loads, 16 rows an instruction at half a
 // line each, 16 tokens of 2048 x 2048 took 4.8 us, so 3.7.  What bounds it: up to some 256 workgroups the launch and one round trip (3.4
-// us), then the vector instructions, some 190 a tile and superblock (half of them the products with the scales), and, from 17 tokens on,
+// us), then the vector instructions, some 215 a tile and superblock (half of them the products with the scales), and, from 17 tokens on,
 // the LDS that lets one workgroup on a compute unit.  (Asking for the next superblock in front of the products: even.)
 #pragma once
 #include "ksh_device.hpp"

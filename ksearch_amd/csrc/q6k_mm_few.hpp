@@ -2,7 +2,7 @@
 // 16 columns: pieces from the 16-byte address in front of a block, the lane's words shifted as they leave LDS; 64 + q as bf16, from -96
 // sum(x) on.  Error 0.70 to 0.91e-7 of the result for 512 to 8192 columns, 0.71 to 1.04e-7 in the form with slices, whose products of
 // scale and weight are f16 (with scales of all eight bits 1.0e-7 and 1.4e-4).  2 tokens of 2048 x 2048
-// 7.5 -> 4.0 us, 16 of 4096 x 4096 11.8 -> 6.9, 2 of 12288 x 8192 29.7 -> 19.8; some 230 vector instructions a tile and superblock.
+// 7.5 -> 4.0 us, 16 of 4096 x 4096 11.8 -> 6.9, 2 of 12288 x 8192 29.7 -> 19.8; some 285 vector instructions a tile and superblock.
 #pragma once
 #include "q4k_mm_few.hpp"
 

@@ -1603,8 +1603,8 @@ int launch_inst(const LaneParams &p, int n_slots, hipStream_t st)
     return e == hipSuccess ? 0 : hip_fail(e, "sdpa (register form) launch");
 }
 
-// which launches take the instances for one or two q heads per workgroup: at heads of 256 and 512 the fused decode step,
-// and split-KV partials with one head per workgroup
+// which launches take the instances for one or two q heads per workgroup: at heads of 256 and 512 the fused decode step, and
+// partials with one head per workgroup at every head size (of one cache, or of slots whose partitions are dealt by length)
 bool lanes_few_heads(int fused, int mode, int groups, int hd)
 {
     return fused ? (hd == 256 || hd == 512) && groups <= 2 : mode == kModePart && groups == 1;
@@ -1612,7 +1612,7 @@ bool lanes_few_heads(int fused, int mode, int groups, int hd)
 
 int launch_lanes(const LaneParams &p, int hd, int nw, int n_slots, hipStream_t st)
 {
-    // the decode step with one or two q heads per workgroup (heads of 256): instances of their own
+    // one or two q heads per workgroup: instances of their own
     if (lanes_few_heads(p.fused, p.mode, p.groups, hd) && (nw == 4 || nw == 8)) {
         const dim3 grid(p.nwg, p.n_kv * p.hsplit, n_slots);
         if (!p.fused && hd == 128 && nw == 8) hipLaunchKernelGGL((sdpa_lanes_kernel<128, 1, 8, false>), grid, dim3(512), (lanes_lds_bytes<128, 1, 8>()), st, p);
@@ -1913,7 +1913,9 @@ static int parts_waves(int64_t workgroups, int64_t rows, int heads, int hd)
 // how much of it a call attends (the figures: half of it on average).  us, general rule | so:
 // - heads of 256, few rows in all: the matrix-core form's chain costs what it saves.  One head a workgroup of four waves, 512 of
 //   them; a single slot two heads and eight waves.  8 heads over one kv head, 2 slots of 300 rows 10.0 | 8.5, 4 of 600 10.1 | 8.4, 1 of
-//   1000 10.0 | 8.3; 16 of 300 10.6 | 9.7; beyond 5000 rows it turns (8 slots of 1000 10.2 | 10.8, 2 of 4000 10.3 | 10.8).
+//   1000 10.0 | 8.3; 16 of 300 10.6 | 9.7; beyond 5000 rows it turns (8 slots of 1000 10.2 | 10.8, 2 of 4000 10.3 | 10.8).  With all
+//   rows attended up to 256 workgroups are still the shorter form (9.6 | 8.7), more are not: 8 over one, 8 slots of 600 a tenth | half | all of
+//   the rows 8.4 | 9.6 | 9.65 by the rule, 7.6 | 8.7 | 10.35 so, 16 of 300 8.4 | 10.0 | 10.1 and 7.9 | 9.2 | 11.6.
 // - heads of 512: 256 workgroups of eight waves, one a compute unit (the general rule's 512 and more took turns): one head each while
 //   that leaves at most 130 rows, four beyond.  2 slots of 300 13.1 | 9.4, 4 of 4000 25.3 | 16.5, 8 of 8000 50.7 | 28.3, 16 of 4000 50.3 |
 //   29.6, 16 of 16384 85.7 | 78.
@@ -1963,7 +1965,7 @@ int bind_sdpa_lanes(ksh_kernel &k, int nwg, int n_slots, const SlotsPlan &plan)
     // sched.vec = 2: the matrix-core form of the row phase -- several slots' (or one slot's) split-KV partials for
     // heads of 256 and up to 8 q heads per kv head, merged by a second launch
     // It is the default wherever it fits (from one slot of a few thousand rows to sixteen long ones it takes 0.5 to
-    // 1.0 of the vector form's time); vec = 3 asks for the vector form by name.
+    // 1.0 of the vector form's time) but for few rows in all (slots_plan); vec = 3 asks for the vector form by name.
     // (a chunk of up to 64 prompt tokens over one cache is 64 slots that share it: a schedule of KSH_SDPA_BATCH, not its
     // default -- timed alone it takes 0.65 to 0.8 of the register form's time, inside a prompt chunk's pass its second
     // launch costs more than that saves at 63 tokens)
