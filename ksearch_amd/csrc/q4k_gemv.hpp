@@ -27,8 +27,8 @@ struct MatvecParams {
 };
 
 // ... as the launch passes them: a launch from a stream costs the host 2.7 us while its arguments take no more than 112 bytes, 3.4
-// beyond (4096 x 4096, a call after the other: 4.2 us with the 136 bytes of the fields one by one, so 3.8; median of four processes
-// each, in turn).  What follows from the rest is left out: the second and the third matrix have the same rows, and a matrix's waves
+// beyond, in a loop of launches that do nothing (4096 x 4096, a call after the other: 3.7 to 4.1 us by the process with the 136 bytes of the
+// fields one by one, so 3.6 to 3.9).  What follows from the rest is left out: the second and the third matrix have the same rows, and a matrix's waves
 // follow from its rows.
 struct MatvecArgs {
     const uint8_t *W0, *W1, *W2;
